@@ -1,4 +1,5 @@
-"""Builds libnntile_hip_sdpa.so (hand-written HIP for gfx950) in-tree.
+"""Builds libnntile_hip_sdpa.so (hand-written HIP for gfx950) and the native
+front-end of the Python binding (_front.so) in-tree.
 
     python -m nntile_amd.build [--force]
 """
@@ -16,6 +17,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wall", "-Wno-unused-function"]
+FRONT = os.path.join(HERE, "_front.so")
+ROCM = os.path.dirname(os.path.dirname(HIPCC)) if os.path.isabs(HIPCC) else "/opt/rocm"
 
 
 def _stale(obj, src):
@@ -26,6 +29,24 @@ def _stale(obj, src):
                     if f.endswith(".hpp")]
     deps.append(os.path.join(HERE, "..", "include", "nntile_hip_sdpa.h"))
     return any(os.path.getmtime(d) > t for d in deps)
+
+
+def _front_command():
+    """g++ on the binding's front-end: host code on torch's headers, linked
+    against the kernel library beside it."""
+    import sysconfig
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    inc = include_paths() + [os.path.join(ROCM, "include"), sysconfig.get_paths()["include"]]
+    lib = library_paths()
+    return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+             "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+             "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
+            + [x for d in inc for x in ("-isystem", d)]
+            + [os.path.join(CSRC, "front.cpp"), "-o", FRONT]
+            + ["-L" + d for d in lib] + ["-L" + HERE, "-lnntile_hip_sdpa", "-ltorch_python",
+                                         "-ltorch_cpu", "-lc10", "-lc10_hip",
+                                         "-Wl,-rpath,$ORIGIN"])
 
 
 def build(force=False, verbose=True):
@@ -55,6 +76,11 @@ def build(force=False, verbose=True):
         raise RuntimeError("hipcc failed")
     if force or procs or not os.path.exists(LIB):
         cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-o", LIB] + objs
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        subprocess.check_call(cmd)
+    if force or _stale(FRONT, os.path.join(CSRC, "front.cpp")):
+        cmd = _front_command()
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.check_call(cmd)

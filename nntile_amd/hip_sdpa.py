@@ -1,4 +1,8 @@
-"""ctypes binding of libnntile_hip_sdpa.so plus thin torch-tensor front-ends.
+"""Binding of libnntile_hip_sdpa.so plus thin torch-tensor front-ends.
+
+The per-call work - checks, argument block, stream, the call itself - is done
+by the native module _front (csrc/front.cpp); ctypes carries what is called
+rarely and the argument blocks of prepared calls.
 
 torch is used for device memory and streams only; every computation goes
 through the C ABI declared in include/nntile_hip_sdpa.h.  There is no fallback:
@@ -225,6 +229,23 @@ def lib():
     return _lib
 
 
+_front = None
+
+
+def _native():
+    """The native front-end; raises if it has not been built."""
+    global _front
+    if _front is None:
+        lib()
+        try:
+            from . import _front as module
+        except ImportError as e:
+            raise RuntimeError("the native front-end nntile_amd/_front.so cannot be loaded (%s): "
+                               "run `python -m nntile_amd.build`" % e)
+        _front = module
+    return _front
+
+
 class SdpaError(RuntimeError):
     def __init__(self, code, what):
         super().__init__("%s: %s (code %d)" % (what, _ERR.get(code, "error"), code))
@@ -267,13 +288,8 @@ def flash_sdpa_fwd(K, Q, mask, lse, V, A, scratch_lse=None, scratch_A=None, stre
     (execute_graph) with its argument order K, Q, mask, lse, V, A.
     scratch_lse ([batch, seq] fp32) and scratch_A (like A) are the reference's
     scratch tiles; the call may overwrite them."""
-    _dev(K, Q, mask, lse, V, A, scratch_lse, scratch_A)
-    batch, seq, head = Q.shape
-    if scratch_lse is not None and scratch_lse.numel() * scratch_lse.element_size() < 4 * batch * seq:
-        raise ValueError("scratch_lse is smaller than a logsumexp tile")
-    fn = getattr(lib(), "nntile_hip_flash_sdpa_fwd_" + dtype_name(Q))
-    _check(fn(_stream(stream), seq, head, batch, _ptr(K), _ptr(Q), _ptr(mask),
-              _ptr(scratch_lse), _ptr(V), _ptr(scratch_A), _ptr(lse), _ptr(A)), "flash_sdpa_fwd")
+    _check(_native().flash_fwd(K, Q, mask, lse, V, A, scratch_lse, scratch_A, stream),
+           "flash_sdpa_fwd")
 
 
 def _tile_args(K, Q, mask, lse, V, A, mask_mode, n_batch, kv_group, q_pos0,
@@ -295,23 +311,16 @@ def _tile_args(K, Q, mask, lse, V, A, mask_mode, n_batch, kv_group, q_pos0,
 
 def sdpa_fwd_tile(K, Q, mask, lse, V, A, mask_mode, n_batch=None, kv_group=1,
                   q_pos0=0, k_pos0=0, causal_offset=0, flags=0, stream=None):
-    _dev(K, Q, mask, lse, V, A)
-    a = _tile_args(K, Q, mask, lse, V, A, mask_mode, n_batch, kv_group, q_pos0,
-                   k_pos0, causal_offset, flags)
-    fn = getattr(lib(), "nntile_hip_sdpa_fwd_tile_" + dtype_name(Q))
-    _check(fn(_stream(stream), ctypes.byref(a)), "sdpa_fwd_tile")
+    _check(_native().fwd_tile(K, Q, mask, lse, V, A, mask_mode, n_batch, kv_group, q_pos0, k_pos0,
+                              causal_offset, flags, stream), "sdpa_fwd_tile")
 
 
 def flash_sdpa_bwd(K, Q, V, A, dA, mask, lse, scratch_dQ, dK, dQ, dV, stream=None):
     """One square tile with an additive mask: the reference's backward kernel
     call (execute_graph) with its argument order; the gradients are added to
     dK, dQ, dV.  scratch_dQ is the reference's scratch tile for dQ."""
-    _dev(K, Q, V, A, dA, mask, lse, scratch_dQ, dK, dQ, dV)
-    batch, seq, head = Q.shape
-    fn = getattr(lib(), "nntile_hip_flash_sdpa_bwd_" + dtype_name(Q))
-    _check(fn(_stream(stream), seq, head, batch, _ptr(K), _ptr(Q), _ptr(V), _ptr(A),
-              _ptr(dA), _ptr(mask), _ptr(lse), None, _ptr(scratch_dQ), None,
-              _ptr(dK), _ptr(dQ), _ptr(dV)), "flash_sdpa_bwd")
+    _check(_native().flash_bwd(K, Q, V, A, dA, mask, lse, scratch_dQ, dK, dQ, dV, stream),
+           "flash_sdpa_bwd")
 
 
 def sdpa_bwd_workspace_bytes(q_seq, k_seq, batch, mask_mode):
@@ -326,27 +335,12 @@ def sdpa_bwd_tile(K, Q, V, A, dA, mask, lse, dK, dQ, dV, mask_mode, n_batch=None
                   workspace=None, stream=None):
     """Backward of one (query tile, key tile) pair; the gradients are added to
     dK, dQ, dV (written with flags=OVERWRITE)."""
-    _dev(K, Q, V, A, dA, mask, lse, dK, dQ, dV, workspace)
-    batch, q_seq, head = Q.shape
-    k_seq = K.shape[1]
-    a = BwdArgs()
-    a.q_seq, a.k_seq, a.head, a.batch = q_seq, k_seq, head, batch
-    a.n_batch = batch if n_batch is None else n_batch
-    a.kv_group = kv_group
-    a.mask_mode = mask_mode
     if workspace is None:
-        need = lib().nntile_hip_sdpa_bwd_workspace_bytes(ctypes.byref(a))
+        need = sdpa_bwd_workspace_bytes(Q.shape[1], K.shape[1], Q.shape[0], mask_mode)
         workspace = torch.empty(need, dtype=torch.uint8, device=Q.device)
-    a.flags = flags
-    a.q_pos0, a.k_pos0, a.causal_offset = q_pos0, k_pos0, causal_offset
-    a.K, a.Q, a.V, a.A, a.dA = (t.data_ptr() for t in (K, Q, V, A, dA))
-    a.mask = None if mask is None else mask.data_ptr()
-    a.lse = lse.data_ptr()
-    a.dK, a.dQ, a.dV = dK.data_ptr(), dQ.data_ptr(), dV.data_ptr()
-    a.workspace = workspace.data_ptr()
-    a.workspace_bytes = workspace.numel() * workspace.element_size()
-    fn = getattr(lib(), "nntile_hip_sdpa_bwd_tile_" + dtype_name(Q))
-    _check(fn(_stream(stream), ctypes.byref(a)), "sdpa_bwd_tile")
+    _check(_native().bwd_tile(K, Q, V, A, dA, mask, lse, dK, dQ, dV, workspace, mask_mode, n_batch,
+                              kv_group, q_pos0, k_pos0, causal_offset, flags, stream),
+           "sdpa_bwd_tile")
 
 
 def _grid_args(K_tiles, Q_tiles, lse_tiles, V_tiles, A_tiles, q_seq, k_seq, q_tile, k_tile,
@@ -455,11 +449,14 @@ class Plan:
     its calls once; `launch` costs one foreign call."""
 
     def __init__(self, fn, args, what, extra=(), keep=()):
-        self._fn, self._args, self._what, self._extra = fn, args, what, extra
+        self._args, self._what = args, what
         self._keep = keep          # tensors whose memory the call refers to
+        values = tuple((e.value or 0) if isinstance(e, _vp) else int(e) for e in extra)
+        self._call = _native().Launch(ctypes.cast(fn, _vp).value, ctypes.addressof(args),
+                                      values).call
 
     def launch(self, stream=None):
-        rc = self._fn(_stream(stream), ctypes.byref(self._args), *self._extra)
+        rc = self._call(stream)
         if rc != OK:
             raise SdpaError(rc, self._what)
 
@@ -473,13 +470,12 @@ class FlashPlan:
         batch, seq, head = Q.shape
         if scratch_lse is not None and scratch_lse.numel() * scratch_lse.element_size() < 4 * batch * seq:
             raise ValueError("scratch_lse is smaller than a logsumexp tile")
-        self._fn = getattr(lib(), "nntile_hip_flash_sdpa_fwd_" + dtype_name(Q))
-        self._args = (seq, head, batch, _ptr(K), _ptr(Q), _ptr(mask), _ptr(scratch_lse), _ptr(V),
-                      _ptr(scratch_A), _ptr(lse), _ptr(A))
-        self._keep = (K, Q, mask, lse, V, A, scratch_lse, scratch_A)
+        dtype_name(Q)
+        self._call = _native().flash_fwd
+        self._tensors = (K, Q, mask, lse, V, A, scratch_lse, scratch_A)
 
     def launch(self, stream=None):
-        rc = self._fn(_stream(stream), *self._args)
+        rc = self._call(*self._tensors, stream)
         if rc != OK:
             raise SdpaError(rc, "flash_sdpa_fwd")
 
@@ -555,13 +551,8 @@ def sdpa_fwd_decode(K, Q, mask, lse, V, A, mask_mode, n_batch, kv_group,
     """K, V: [n_head_kv*n_batch, k_seq, head]; Q, A:
     [n_head_kv*kv_group*n_batch, q_seq, head]; workspace: a device byte
     tensor of at least decode_workspace_bytes()."""
-    _dev(K, Q, mask, lse, V, A, workspace)
-    a = _tile_args(K, Q, mask, lse, V, A, mask_mode, n_batch, kv_group, q_pos0,
-                   k_pos0, causal_offset, flags)
-    fn = getattr(lib(), "nntile_hip_sdpa_fwd_decode_" + dtype_name(Q))
-    nbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    _check(fn(_stream(stream), ctypes.byref(a), _ptr(workspace), nbytes),
-           "sdpa_fwd_decode")
+    _check(_native().fwd_decode(K, Q, mask, lse, V, A, mask_mode, n_batch, kv_group, q_pos0, k_pos0,
+                                causal_offset, flags, workspace, stream), "sdpa_fwd_decode")
 
 
 DECODE_STATIC_SCRATCH_BYTES = 16 << 20
@@ -582,14 +573,7 @@ def sdpa_fwd_decode_static(K, Q, mask, lse, V, A, mask_mode, n_batch, kv_group, 
 def kv_cache_append(k_new, v_new, k_cache, v_cache, filled, stream=None):
     """Write k_new, v_new ([entries, rows, head]) behind the `filled` rows of
     k_cache, v_cache ([entries, capacity, head])."""
-    _dev(k_new, v_new, k_cache, v_cache)
-    entries, rows, head = k_new.shape
-    if (tuple(v_new.shape) != (entries, rows, head) or k_cache.shape != v_cache.shape
-            or k_cache.shape[0] != entries or k_cache.shape[2] != head):
-        raise SdpaError(EINVAL, "kv_cache_append")
-    fn = getattr(lib(), "nntile_hip_kv_cache_append_" + dtype_name(k_cache))
-    _check(fn(_stream(stream), head, rows, entries, k_cache.shape[1], filled, _ptr(k_new),
-              _ptr(v_new), _ptr(k_cache), _ptr(v_cache)), "kv_cache_append")
+    _check(_native().kv_append(k_new, v_new, k_cache, v_cache, filled, stream), "kv_cache_append")
 
 
 def plan_kv_cache_append(k_new, v_new, k_cache, v_cache, filled):
@@ -600,17 +584,14 @@ def plan_kv_cache_append(k_new, v_new, k_cache, v_cache, filled):
     if (tuple(v_new.shape) != (entries, rows, head) or k_cache.shape != v_cache.shape
             or k_cache.shape[0] != entries or k_cache.shape[2] != head):
         raise SdpaError(EINVAL, "kv_cache_append")
-    fn = getattr(lib(), "nntile_hip_kv_cache_append_" + dtype_name(k_cache))
-    args = (head, rows, entries, k_cache.shape[1], filled, _ptr(k_new), _ptr(v_new),
-            _ptr(k_cache), _ptr(v_cache))
+    dtype_name(k_cache)
+    call = _native().kv_append
 
     class _Append:
         def launch(self, stream=None):
-            _check(fn(_stream(stream), *args), "kv_cache_append")
+            _check(call(k_new, v_new, k_cache, v_cache, filled, stream), "kv_cache_append")
 
-    plan = _Append()
-    plan._keep = (k_new, v_new, k_cache, v_cache)
-    return plan
+    return _Append()
 
 
 def _cache_args(K_cache, V_cache, k_seq, Q, mask, lse, A, mask_mode, n_batch, kv_group, q_pos0,
@@ -626,14 +607,8 @@ def sdpa_fwd_decode_cache(K_cache, V_cache, k_seq, Q, mask, lse, A, mask_mode, n
                           stream=None):
     """sdpa_fwd_decode over the first k_seq rows of every entry of the caches
     ([n_head_kv*n_batch, capacity, head]), read where they lie."""
-    _dev(K_cache, V_cache, Q, mask, lse, A, workspace)
-    if K_cache.shape != V_cache.shape:
-        raise SdpaError(EINVAL, "sdpa_fwd_decode_cache")
-    a = _cache_args(K_cache, V_cache, k_seq, Q, mask, lse, A, mask_mode, n_batch, kv_group,
-                    q_pos0, k_pos0, causal_offset, flags)
-    fn = getattr(lib(), "nntile_hip_sdpa_fwd_decode_cache_" + dtype_name(Q))
-    nbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-    _check(fn(_stream(stream), ctypes.byref(a), K_cache.shape[1], _ptr(workspace), nbytes),
+    _check(_native().fwd_decode_cache(K_cache, Q, mask, lse, V_cache, A, mask_mode, n_batch, kv_group,
+                                      q_pos0, k_pos0, causal_offset, flags, k_seq, workspace, stream),
            "sdpa_fwd_decode_cache")
 
 
@@ -642,13 +617,9 @@ def sdpa_fwd_tile_cache(K_cache, V_cache, k_seq, Q, mask, lse, A, mask_mode, n_b
     """sdpa_fwd_tile over the first k_seq rows of every entry of the caches
     ([entries, capacity, head]), read where they lie; any chunk length, fp32
     included."""
-    _dev(K_cache, V_cache, Q, mask, lse, A)
-    if K_cache.shape != V_cache.shape:
-        raise SdpaError(EINVAL, "sdpa_fwd_tile_cache")
-    a = _cache_args(K_cache, V_cache, k_seq, Q, mask, lse, A, mask_mode, n_batch, kv_group,
-                    q_pos0, k_pos0, causal_offset, flags)
-    fn = getattr(lib(), "nntile_hip_sdpa_fwd_tile_cache_" + dtype_name(Q))
-    _check(fn(_stream(stream), ctypes.byref(a), K_cache.shape[1]), "sdpa_fwd_tile_cache")
+    _check(_native().fwd_tile_cache(K_cache, Q, mask, lse, V_cache, A, mask_mode, n_batch, kv_group,
+                                    q_pos0, k_pos0, causal_offset, flags, k_seq, stream),
+           "sdpa_fwd_tile_cache")
 
 
 def plan_decode_cache(K_cache, V_cache, k_seq, Q, mask, lse, A, mask_mode, n_batch, kv_group,
@@ -685,10 +656,10 @@ def sdpa_fwd_decode_append_cache(k_new, v_new, K_cache, V_cache, k_seq, Q, mask,
     """kv_cache_append of k_new, v_new ([entries, rows, head]) behind the
     k_seq - rows filled rows of the caches and sdpa_fwd_decode_cache over the
     k_seq rows, in one launch."""
-    fn, a, extra = _append_cache_call(k_new, v_new, K_cache, V_cache, k_seq, Q, mask, lse, A,
-                                      mask_mode, n_batch, kv_group, workspace, q_pos0, k_pos0,
-                                      causal_offset, flags)
-    _check(fn(_stream(stream), ctypes.byref(a), *extra), "sdpa_fwd_decode_append_cache")
+    _check(_native().fwd_decode_append_cache(
+        K_cache, Q, mask, lse, V_cache, A, mask_mode, n_batch, kv_group, q_pos0, k_pos0,
+        causal_offset, flags, k_seq, k_new, v_new, workspace, stream),
+        "sdpa_fwd_decode_append_cache")
 
 
 def plan_decode_append_cache(k_new, v_new, K_cache, V_cache, k_seq, Q, mask, lse, A, mask_mode,
@@ -728,34 +699,20 @@ def mask_tile_class(mask, offset=0, workspace=None, stream=None):
 
 def accumulate_attn_output(src_lse, src_attn, dst_lse, dst_attn, stream=None):
     """dst <- merge(dst, src) row by row; attn tiles [batch, seq, head]."""
-    _dev(src_lse, src_attn, dst_lse, dst_attn)
-    batch, seq, head = dst_attn.shape
-    fn = getattr(lib(), "nntile_hip_accumulate_attn_output_" + dtype_name(dst_attn))
-    _check(fn(_stream(stream), head, seq, batch, _ptr(src_lse), _ptr(src_attn),
-              _ptr(dst_lse), _ptr(dst_attn)), "accumulate_attn_output")
+    _check(_native().accumulate(src_lse, src_attn, dst_lse, dst_attn, stream),
+           "accumulate_attn_output")
 
 
 def rope(sin, cos, src, dst, backward=False, stream=None):
     """Rotary embedding of src (memory order (2, m, n), m = sin.numel()) into
     dst; backward=True applies the transposed rotation (dy -> dx)."""
-    _dev(sin, cos, src, dst)
-    m = sin.numel()
-    if cos.numel() != m or src.numel() != dst.numel() or (m and src.numel() % (2 * m)):
-        raise SdpaError(EINVAL, "rope")
-    n = src.numel() // (2 * m) if m else 0
-    name = "nntile_hip_rope_backward_" if backward else "nntile_hip_rope_"
-    fn = getattr(lib(), name + dtype_name(src))
-    _check(fn(_stream(stream), m, n, _ptr(sin), _ptr(cos), _ptr(src), _ptr(dst)), "rope")
+    _check(_native().rope(sin, cos, src, dst, backward, stream), "rope")
 
 
 def transpose(alpha, src, dst, m, n, stream=None):
     """dst = alpha * src^T; src is m x n in Fortran order (memory order of a
     C-ordered [n, m] tensor), dst n x m in Fortran order."""
-    _dev(src, dst)
-    if src.numel() != m * n or dst.numel() != m * n:
-        raise SdpaError(EINVAL, "transpose")
-    fn = getattr(lib(), "nntile_hip_transpose_" + dtype_name(src))
-    _check(fn(_stream(stream), m, n, float(alpha), _ptr(src), _ptr(dst)), "transpose")
+    _check(_native().transpose(alpha, src, dst, m, n, stream), "transpose")
 
 
 def flash_sdpa_fwd_codelet(K, Q, mask, lse, V, A, scratch_lse=None, scratch_A=None,

@@ -69,6 +69,20 @@ class KVCache:
         decode kernels' shapes the two are ONE launch (the
         attention reads the new rows from k_partial / v_partial while other
         workgroups of the launch write them into the caches)."""
+        if mask is None and stream is None:
+            mode = hip_sdpa.MASK_CAUSAL if causal else hip_sdpa.MASK_NONE
+            step = hip_sdpa._native().cache_step
+            rc = step(self.k, self.v, k_partial, v_partial, Q, lse, A, self.k_cache_size,
+                      self.max_cache_size, n_batch, kv_group, mode, hip_sdpa.OVERWRITE,
+                      self._workspace, None)
+            if rc == hip_sdpa.OK:
+                self._mask_in_use = None
+                rows = k_partial.shape[1]
+                self.k_cache_size += rows
+                self.v_cache_size += rows
+                return
+            # (what is left - a first call, a larger workspace, other shapes,
+            # a call to be refused - takes the long way below)
         rows, q_seq = k_partial.shape[1], Q.shape[1]
         one_launch = (self.k is not None and v_partial.shape[1] == rows
                       and kv_group * q_seq <= 64 and Q.shape[2] in (64, 128)
