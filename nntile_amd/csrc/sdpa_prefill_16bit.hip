@@ -89,101 +89,117 @@ extern "C" int nntile_hip_debug_pf_trace(unsigned long long *host)
 // CU.  8 (analytic masks, head 64 and 128): one workgroup of 256 queries per
 // CU, whose eight wavefronts share every K/V step - a CU then brings each step
 // into LDS once where two workgroups of four bring it twice.
-// Scan of the mask rows of query block qb over key range sp of kMaskBitSplits:
-// the workgroup (THREADS threads) ORs what it finds in its range of 16-byte
-// chunks into bits[0] (bit s: some value of 64-key step s is not "open") and
-// bits[1] (not "hidden"); steps from 63 on share bit 63.  ES: bytes per mask
-// element; open / hidden: the 32-bit pattern of four (two) visible / hidden
-// elements.  bits is valid for every thread on return.
-template<int ES, int THREADS>
-__device__ __forceinline__ void mask_scan_range(const char *mask, int ld_bytes, int q_len,
-        int n_chunks, uint32_t open_word, uint32_t hidden_word, int qb, int sp,
-        unsigned long long *bits)
+// Scan of the mask rows of one query block over the key steps [s_lo, s_hi):
+// bit s of not_open: some value of 64-key step s is not "open", of not_hidden:
+// not "hidden" (steps from 63 on share bit 63).  NWAVES wavefronts; words:
+// 2 * NWAVES of LDS; the results are the same in every thread.  mask: the
+// block's first row; ES: bytes per element; open / hidden: the 32-bit pattern
+// of visible / hidden elements.
+//
+// A lane keeps to one step while it walks the rows, so that what it finds is
+// two words ORed together (four instructions a load) and a ballot at the end
+// says which steps; 16 loads of 16 bytes are in flight per lane.  Reads of a
+// row are contiguous whatever its length; rows and starts that are not
+// multiples of 16 bytes only cost some loads a second cache line.  The last
+// chunk of a row is moved back to end with the row: it then looks at elements
+// of the chunk before once more, which can only make the answer more careful.
+// (Before, a lane's loads fell on changing steps, each needing two 64-bit
+// shifts, and every lane added its words to LDS with atomics of its own: 7 us
+// for the 32 KiB of a 128 x 128 tile, and masks with rows of any other length
+// were not scanned at all.)
+template<int ES, int NWAVES>
+__device__ __forceinline__ void mask_scan_steps(const char *mask, uint32_t ld_bytes, int n_rows,
+        int row_bytes, int s_lo, int s_hi, uint32_t open_word, uint32_t hidden_word,
+        unsigned long long *words, unsigned long long &not_open_out,
+        unsigned long long &not_hidden_out)
 {
-    constexpr int CHUNKS_PER_STEP = kKeys * ES / 16;
-    const int tid = threadIdx.x;
-    if(tid == 0)
-    {
-        bits[0] = 0ull;
-        bits[1] = 0ull;
-    }
-    __syncthreads();
-    const int per_split = (n_chunks + kMaskBitSplits - 1) / kMaskBitSplits;
-    const int c_lo = min(sp * per_split, n_chunks);
-    const int n_loc = min(c_lo + per_split, n_chunks) - c_lo;
-    const int q_row0 = qb * kQRows;
-    const int n_rows = min(kQRows, q_len - q_row0);
+    constexpr int CPS = kKeys * ES / 16;        // chunks per step
+    constexpr int SPAN = 64 / CPS;              // steps that fit a wavefront's lanes
+    typedef u32x4 __attribute__((aligned(1))) u32x4_any;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     unsigned long long not_open = 0ull, not_hidden = 0ull;
-    if(n_loc > 0)
+    // lanes per row: the steps asked for, a power of two, at most all lanes
+    int steps_wide = SPAN;
+    while(steps_wide > 1 && steps_wide / 2 >= s_hi - s_lo)
     {
-        const int total = n_rows * n_loc;
-        const char *mbase = mask + (int64_t)q_row0 * ld_bytes + (int64_t)c_lo * 16;
-        // chunk tid, tid + THREADS, ... of the rows' pieces laid end to end
-        const int d_row = THREADS / n_loc, d_c = THREADS % n_loc;
-        int row = tid / n_loc, c = tid % n_loc;
-        for(int base = 0; base < total; base += 16 * THREADS)
+        steps_wide >>= 1;
+    }
+    const int lanes_row = steps_wide * CPS;
+    const int rows_pass = (64 / lanes_row) * NWAVES;    // rows one load of everybody covers
+    const int r0 = wave * (64 / lanes_row) + lane / lanes_row;
+    const int my_step = (lane % lanes_row) / CPS;
+    for(int s0 = s_lo; s0 < s_hi; s0 += steps_wide)
+    {
+        const bool mine = s0 + my_step < s_hi;
+        const int at = min((s0 + my_step) * kKeys * ES + (lane % CPS) * 16, row_bytes - 16);
+        uint32_t any_open = 0u, any_hidden = 0u;
+        for(int base = 0; base < n_rows; base += 16 * rows_pass)
         {
-            // (rows past the end re-read the last row: no branches, so that
-            // the 16 loads are in flight together)
             u32x4 v[16];
-            int st[16];
 #pragma unroll
             for(int u = 0; u < 16; ++u)
             {
-                const int r = min(row, n_rows - 1);
-                st[u] = min((c_lo + c) / CHUNKS_PER_STEP, 63);
-                v[u] = *reinterpret_cast<const u32x4 *>(
-                        mbase + (uint32_t)(r * ld_bytes + c * 16));
-                row += d_row;
-                c += d_c;
-                if(c >= n_loc)
+                // (rows past the end re-read the last one: no branches, so
+                // that the loads are in flight together)
+                const uint32_t row = (uint32_t)min(base + r0 + u * rows_pass, n_rows - 1);
+                v[u] = *reinterpret_cast<const u32x4_any *>(mask + row * ld_bytes + at);
+            }
+#pragma unroll
+            for(int u = 0; u < 16; ++u)
+            {
+#pragma unroll
+                for(int e = 0; e < 4; ++e)
                 {
-                    c -= n_loc;
-                    row += 1;
+                    any_open |= v[u][e] ^ open_word;
+                    any_hidden |= v[u][e] ^ hidden_word;
                 }
             }
-#pragma unroll
-            for(int u = 0; u < 16; ++u)
+        }
+        const unsigned long long b_open = __builtin_amdgcn_ballot_w64(mine && any_open != 0u);
+        const unsigned long long b_hidden = __builtin_amdgcn_ballot_w64(mine && any_hidden != 0u);
+        for(int l = 0; l < 64; l += CPS)
+        {
+            const unsigned long long bit = 1ull << min(s0 + (l % lanes_row) / CPS, 63);
+            if(((b_open >> l) & ((1ull << CPS) - 1ull)) != 0ull)
             {
-                const uint32_t any1 = v[u][0] | v[u][1] | v[u][2] | v[u][3];
-                const uint32_t all1 = v[u][0] & v[u][1] & v[u][2] & v[u][3];
-                const bool open = (any1 == open_word) & (all1 == open_word);
-                const bool hidden = (any1 == hidden_word) & (all1 == hidden_word);
-                not_open |= (unsigned long long)(!open) << st[u];
-                not_hidden |= (unsigned long long)(!hidden) << st[u];
+                not_open |= bit;
+            }
+            if(((b_hidden >> l) & ((1ull << CPS) - 1ull)) != 0ull)
+            {
+                not_hidden |= bit;
             }
         }
     }
-    // One LDS atomic per wavefront and word, not one per lane: the range
-    // covers few steps, and a ballot per step says whether any lane has its bit.
+    if(lane == 0)
     {
-        const int s_lo = min(c_lo / CHUNKS_PER_STEP, 63);
-        const int s_hi = min((c_lo + max(n_loc, 1) - 1) / CHUNKS_PER_STEP, 63);
-        unsigned long long w_open = 0ull, w_hidden = 0ull;
-        for(int st = s_lo; st <= s_hi; ++st)
-        {
-            if(__builtin_amdgcn_ballot_w64(((not_open >> st) & 1ull) != 0ull) != 0ull)
-            {
-                w_open |= 1ull << st;
-            }
-            if(__builtin_amdgcn_ballot_w64(((not_hidden >> st) & 1ull) != 0ull) != 0ull)
-            {
-                w_hidden |= 1ull << st;
-            }
-        }
-        if((tid & 63) == 0)
-        {
-            if(w_open != 0ull)
-            {
-                atomicOr(&bits[0], w_open);
-            }
-            if(w_hidden != 0ull)
-            {
-                atomicOr(&bits[1], w_hidden);
-            }
-        }
+        words[2 * wave] = not_open;
+        words[2 * wave + 1] = not_hidden;
     }
     __syncthreads();
+    not_open = not_hidden = 0ull;
+#pragma unroll
+    for(int w = 0; w < NWAVES; ++w)
+    {
+        not_open |= words[2 * w];
+        not_hidden |= words[2 * w + 1];
+    }
+    not_open_out = not_open;
+    not_hidden_out = not_hidden;
+}
+
+// Key range sp of kMaskBitSplits of query block qb, for the scan that is done
+// once for all batch entries.
+template<int ES, int NWAVES>
+__device__ __forceinline__ void mask_scan_range(const char *mask, uint32_t ld_bytes, int q_len,
+        int k_seq, uint32_t open_word, uint32_t hidden_word, int qb, int sp,
+        unsigned long long *words, unsigned long long &not_open, unsigned long long &not_hidden)
+{
+    const int n_steps = (k_seq + kKeys - 1) / kKeys;
+    const int per_split = (n_steps + kMaskBitSplits - 1) / kMaskBitSplits;
+    const int s_lo = min(sp * per_split, n_steps);
+    mask_scan_steps<ES, NWAVES>(mask + (int64_t)(qb * kQRows) * ld_bytes, ld_bytes,
+            min(kQRows, q_len - qb * kQRows), k_seq * ES, s_lo, min(s_lo + per_split, n_steps),
+            open_word, hidden_word, words, not_open, not_hidden);
 }
 
 template<typename T, int HEAD, int MODE, int WAVES = 4, int GROUPS = 1>
@@ -263,20 +279,21 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             if((int)blockIdx.x < p.n_scan_wgs)
             {
                 constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 2 : 1;
-                __shared__ unsigned long long pub_bits[2];
-                mask_scan_range<ES, kThreads>(static_cast<const char *>(p.mask),
-                        (int)(p.mask_ld * ES), (int)p.q_seq, (int)(p.k_seq * ES / 16),
+                __shared__ unsigned long long pub_words[2 * WAVES];
+                unsigned long long pub_open, pub_hidden;
+                mask_scan_range<ES, WAVES>(static_cast<const char *>(p.mask),
+                        (uint32_t)(p.mask_ld * ES), (int)p.q_seq, (int)p.k_seq,
                         (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0u : 0x01010101u,
                         (MODE == NNTILE_HIP_MASK_ADDITIVE) ? T::kNegInfPair : 0u,
                         (int)blockIdx.x / kMaskBitSplits, (int)blockIdx.x % kMaskBitSplits,
-                        pub_bits);
+                        pub_words, pub_open, pub_hidden);
                 if(tid == 0)
                 {
                     // written through to memory (device scope), acknowledged,
                     // then the flag: readers on any XCD find the words
                     unsigned long long *e = p.mask_bits + 3 * (int64_t)blockIdx.x;
-                    __hip_atomic_store(e, pub_bits[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(e + 1, pub_bits[1], __ATOMIC_RELAXED,
+                    __hip_atomic_store(e, pub_open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(e + 1, pub_hidden, __ATOMIC_RELAXED,
                             __HIP_MEMORY_SCOPE_AGENT);
                     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                     __hip_atomic_store(e + 2, p.mask_tag, __ATOMIC_RELAXED,
@@ -332,6 +349,10 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         + (int64_t)b * q_len * HEAD;
     const int my_q = q_row0 + wave * 32 + col;          // row within tile
     const bool q_ok = my_q < q_len;
+    // the stored logsumexp that the epilogue merges with: requested here, so
+    // that its latency passes beside the first loads
+    float *lse_ptr = p.lse[q_tile0 + qt] + (int64_t)b * q_len + (q_ok ? my_q : 0);
+    const float lse_stored = p.overwrite ? neg_inf() : *lse_ptr;
 
     // Q fragments, resident for the whole kernel.
     vec8 qf[KSTEPS];
@@ -564,10 +585,12 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // step ahead.  At the top of a step the wavefront classifies its 32 x 64
     // block from the raw bits: nothing hidden (the step runs as if there were
     // no mask), everything hidden (the step is skipped), or mixed (the values
-    // are applied).  Ragged steps and masks that are not aligned for the wide
-    // loads take the element-wise path.
+    // are applied).  The loads carry the alignment of one element; in a ragged
+    // last step a group that would reach past the row is moved back to end
+    // with it and shifted into place when it is used, and what lies past the
+    // end is made hidden.
     constexpr int MW = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 16 : 8;    // dwords per lane and step
-    enum { MASK_ZERO = 0, MASK_HIDDEN = 1, MASK_MIXED = 2, MASK_SLOW = 3 };
+    enum { MASK_ZERO = 0, MASK_HIDDEN = 1, MASK_MIXED = 2 };
     uint32_t mraw[MW];
 #pragma unroll
     for(int i = 0; i < MW; ++i)
@@ -575,38 +598,90 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         mraw[i] = 0;
     }
     const int64_t mask_row = (int64_t)(q_ok ? my_q : 0) * p.mask_ld;
-    // (every full step of any mask: the wide loads below carry the alignment
-    // of one element, and global memory takes unaligned accesses - a row
-    // length that is not a multiple of 4 costs some loads a second cache
-    // line, not a load per element)
-    const bool mask_wide = EXPLICIT;
-    // loads of the mask values of key step kb (a full step) into mraw
-    auto mask_fetch = [&](int kb)
+    // start of group i (keys key0 .. +3 of a step of `keys` keys) as loaded
+    auto group_key0 = [&](int i) -> int
     {
-        if(MODE == NNTILE_HIP_MASK_ADDITIVE)
+        return (i >> 2) * 32 + (i & 3) * 8 + 4 * half;
+    };
+    auto group_start = [&](int key0, int keys) -> int
+    {
+        return min(key0, keys == k_seq ? max(keys - 4, 0) : keys - 4);
+    };
+    // loads of the mask values of key step kb (of `keys` keys) into mraw
+    auto mask_fetch = [&](int kb, int keys)
+    {
+        typedef typename std::conditional<MODE == NNTILE_HIP_MASK_ADDITIVE, uint16_t,
+                uint8_t>::type M;
+        const M *mp = static_cast<const M *>(p.mask) + mask_row + kb * kKeys;
+        auto load_group = [&](int i, int at) __attribute__((always_inline))
         {
-            typedef u32x2 __attribute__((aligned(2))) u32x2_any;
-            const uint16_t *mp = static_cast<const uint16_t *>(p.mask) + mask_row
-                + kb * kKeys + 4 * half;
-#pragma unroll
-            for(int i = 0; i < 8; ++i)
+            if constexpr(MODE == NNTILE_HIP_MASK_ADDITIVE)
             {
-                const u32x2 v = *reinterpret_cast<const u32x2_any *>(
-                        mp + (i >> 2) * 32 + (i & 3) * 8);
+                typedef u32x2 __attribute__((aligned(2))) u32x2_any;
+                const u32x2 v = *reinterpret_cast<const u32x2_any *>(mp + at);
                 mraw[2 * i] = v[0];
                 mraw[2 * i + 1] = v[1];
             }
-        }
-        else if(MODE == NNTILE_HIP_MASK_BOOL)
+            else
+            {
+                typedef uint32_t __attribute__((aligned(1))) u32_any;
+                mraw[i] = *reinterpret_cast<const u32_any *>(mp + at);
+            }
+        };
+        if(keys >= kKeys)
         {
-            typedef uint32_t __attribute__((aligned(1))) u32_any;
-            const uint8_t *mp = static_cast<const uint8_t *>(p.mask) + mask_row
-                + kb * kKeys + 4 * half;
+            mp += 4 * half;
 #pragma unroll
             for(int i = 0; i < 8; ++i)
             {
-                mraw[i] = *reinterpret_cast<const u32_any *>(
-                        mp + (i >> 2) * 32 + (i & 3) * 8);
+                load_group(i, (i >> 2) * 32 + (i & 3) * 8);
+            }
+        }
+        else if(k_seq >= 4)
+        {
+#pragma unroll
+            for(int i = 0; i < 8; ++i)
+            {
+                load_group(i, group_start(group_key0(i), keys));
+            }
+        }
+        else
+        {
+            // (rows of less than one group)
+            const uint32_t e0 = mp[0], e1 = mp[min(1, k_seq - 1)], e2 = mp[k_seq - 1];
+            if constexpr(MODE == NNTILE_HIP_MASK_ADDITIVE)
+            {
+                mraw[0] = e0 | (e1 << 16);
+                mraw[1] = e2;
+            }
+            else
+            {
+                mraw[0] = e0 | (e1 << 8) | (e2 << 16);
+            }
+        }
+    };
+    // brings the groups of a ragged step of `keys` keys into place
+    auto mask_fix_ragged = [&](int keys)
+    {
+#pragma unroll
+        for(int i = 0; i < 8; ++i)
+        {
+            const int key0 = group_key0(i);
+            const int back = min(key0 - group_start(key0, keys), 4);
+            const int valid = min(max(keys - key0, 0), 4);
+            if constexpr(MODE == NNTILE_HIP_MASK_ADDITIVE)
+            {
+                const uint64_t raw = (uint64_t)mraw[2 * i] | ((uint64_t)mraw[2 * i + 1] << 32);
+                const uint64_t hidden = ((uint64_t)T::kNegInfPair << 32) | T::kNegInfPair;
+                const uint64_t keep = valid == 4 ? ~0ull : (1ull << (16 * valid)) - 1ull;
+                const uint64_t v = ((raw >> (16 * (back & 3))) & keep) | (hidden & ~keep);
+                mraw[2 * i] = (uint32_t)v;
+                mraw[2 * i + 1] = (uint32_t)(v >> 32);
+            }
+            else
+            {
+                const uint32_t keep = valid == 4 ? ~0u : (1u << (8 * valid)) - 1u;
+                mraw[i] = (mraw[i] >> (8 * (back & 3))) & keep;
             }
         }
     };
@@ -663,38 +738,44 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         advance_one(cur);       // the second group starts at step 1
     }
     StepCursor nxt = cur;                        // step being fetched
-    // Masks given as values: the first step's K and V are requested before the
+    // Masks given as values: what the loop most likely starts with - the first
+    // step's K and V and the K of the step behind it - is requested before the
     // mask is looked at (below: a wait for the scanning workgroups' flags, or a
     // scan of this workgroup's own rows).  What the mask then says may make
-    // the step unnecessary, which costs nothing but the request.
+    // any of it unnecessary, which costs nothing but the request.  (Not the
+    // first step's mask values: 16 loads that touch 32 rows each delay the
+    // scan more than they save, 6 % on 4 x 4 tiles of 355 keys.)
     bool first_requested = false;
     if(EXPLICIT)
     {
         const int own = GROUPS > 1 ? max(n_steps - grp + GROUPS - 1, 0) / GROUPS : n_steps;
         if(own > 0)
         {
-            fetch_k(nxt, lds_k0);
-            fetch_v(nxt, lds_v0);
+            fetch_k(cur, lds_k0);
+            fetch_v(cur, lds_v0);
+            if(own > 1)
+            {
+                advance(nxt);
+                fetch_k(nxt, lds_k1);
+                nxt = cur;
+            }
             first_requested = true;
         }
     }
     // Explicit masks: number of leading key steps in which the mask changes
     // nothing for any query of the workgroup (they run in the pipelined loop).
-    int n_open = 0;
+    int n_open = 0, n_skip = 0;
     if(EXPLICIT)
     {
-        // The workgroup's rows of the mask are scanned once, 16 bytes per
-        // thread and load, 16 loads in flight, beside the first step's loads.
-        // Per key step the scan records whether every value is "open" (+0 /
-        // true) and whether every value is "hidden" (-inf / false).  Hidden
-        // steps at the end are dropped - a tile pair above the diagonal of a
-        // causal mask given as values costs this scan instead of a pass over K
-        // and V - and the open steps at the start need no mask handling.
+        // The workgroup's rows of the mask are scanned once, beside the first
+        // step's loads.  Per key step the scan records whether every value is
+        // "open" (+0 / true) and whether every value is "hidden" (-inf /
+        // false).  Hidden steps at either end are dropped - a tile pair above
+        // the diagonal of a causal mask given as values costs this scan instead
+        // of a pass over K and V - and open steps in front need no mask handling.
         constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 2 : 1;
-        constexpr int CHUNKS_PER_STEP = kKeys * ES / 16;
         constexpr uint32_t OPEN = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0u : 0x01010101u;
         constexpr uint32_t HIDDEN = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? T::kNegInfPair : 0u;
-        const int64_t row_bytes = (int64_t)k_seq * ES;
         // bit s: some value of step s (steps >= 63 share bit 63) is not open / not hidden
         unsigned long long not_open = 0ull, not_hidden = 0ull;
         bool scanned = false;
@@ -760,73 +841,14 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 scanned = true;
             }
         }
-        // (rows whose length or start is not a multiple of 16 bytes are not
-        // scanned: with loads at the alignment of one element the scan cost
-        // what it saved - 49.6 against 48.1 us on 32 x 1001 x 128)
-        if(!scanned && n_steps > 0 && row_bytes % 16 == 0 && (p.mask_ld * ES) % 16 == 0
-                && reinterpret_cast<uintptr_t>(p.mask) % 16 == 0
+        if(!scanned && n_steps > 0 && k_seq * ES >= 16
                 && p.mask_ld * ES * kQRows < (int64_t)(1 << 30))
         {
-            __shared__ unsigned long long scan_bits[2];
-            if(tid == 0)
-            {
-                scan_bits[0] = 0ull;
-                scan_bits[1] = 0ull;
-            }
-            __syncthreads();
-            const int n_chunks = (int)(row_bytes / 16);
-            const int n_rows = min(kQRows, q_len - q_row0);
-            const int total = n_rows * n_chunks;
-            const char *mbase = static_cast<const char *>(p.mask)
-                + (int64_t)q_row0 * p.mask_ld * ES;
-            // chunk tid, tid + 256, ... of the rows laid end to end: (row, c)
-            // advances by 256 chunks per load without a division
-            const int d_row = kThreads / n_chunks, d_c = kThreads % n_chunks;
-            const int ld_bytes = (int)(p.mask_ld * ES);     // fits: checked above
-            int row = tid / n_chunks, c = tid % n_chunks;
-            for(int base = 0; base < total; base += 16 * kThreads)
-            {
-                // (rows past the end re-read the last row: no branches, so
-                // that the 16 loads are in flight together)
-                u32x4 v[16];
-                int st[16];
-#pragma unroll
-                for(int u = 0; u < 16; ++u)
-                {
-                    const int r = min(row, n_rows - 1);
-                    st[u] = min(c / CHUNKS_PER_STEP, 63);
-                    v[u] = *reinterpret_cast<const u32x4 *>(
-                            mbase + (uint32_t)(r * ld_bytes + c * 16));
-                    row += d_row;
-                    c += d_c;
-                    if(c >= n_chunks)
-                    {
-                        c -= n_chunks;
-                        row += 1;
-                    }
-                }
-#pragma unroll
-                for(int u = 0; u < 16; ++u)
-                {
-                    const uint32_t any1 = v[u][0] | v[u][1] | v[u][2] | v[u][3];
-                    const uint32_t all1 = v[u][0] & v[u][1] & v[u][2] & v[u][3];
-                    const bool open = (any1 == OPEN) & (all1 == OPEN);
-                    const bool hidden = (any1 == HIDDEN) & (all1 == HIDDEN);
-                    not_open |= (unsigned long long)(!open) << st[u];
-                    not_hidden |= (unsigned long long)(!hidden) << st[u];
-                }
-            }
-            if(not_open != 0ull)
-            {
-                atomicOr(&scan_bits[0], not_open);
-            }
-            if(not_hidden != 0ull)
-            {
-                atomicOr(&scan_bits[1], not_hidden);
-            }
-            __syncthreads();
-            not_open = scan_bits[0];
-            not_hidden = scan_bits[1];
+            __shared__ unsigned long long scan_words[2 * WAVES];
+            mask_scan_steps<ES, WAVES>(static_cast<const char *>(p.mask)
+                    + (int64_t)q_row0 * p.mask_ld * ES, (uint32_t)(p.mask_ld * ES),
+                    min(kQRows, q_len - q_row0), k_seq * ES, 0, (k_seq + kKeys - 1) / kKeys,
+                    OPEN, HIDDEN, scan_words, not_open, not_hidden);
             scanned = true;
         }
         if(scanned)
@@ -845,7 +867,26 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             {
                 n_steps = min(n_steps, 64 - __builtin_clzll(not_hidden));
             }
-            n_open = not_open == 0ull ? 63 : min(__builtin_ctzll(not_open), 63);
+            // hidden steps at the start are passed over
+            if(n_steps > 0)
+            {
+                n_skip = min(__builtin_ctzll(not_hidden), n_steps - 1);
+            }
+            not_open >>= n_skip;
+            n_open = not_open == 0ull ? 63 - n_skip : min(__builtin_ctzll(not_open), 63 - n_skip);
+            if(n_skip > 0)
+            {
+                // the step requested above is not wanted: its loads must have
+                // landed before the same buffers are asked for again
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                first_requested = false;
+                n_steps -= n_skip;
+                cur.kb += n_skip;
+                cur.rows_left -= n_skip * kKeys;
+                cur.Kp += (int64_t)n_skip * kKeys * RB;
+                cur.Vp += (int64_t)n_skip * kKeys * RB;
+                nxt = cur;
+            }
         }
     }
     // Leading steps that are complete (64 keys) and visible to every query of
@@ -855,7 +896,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     {
         const int n_full = (p.n_kv_tiles == 1 || k_tile % kKeys == 0)
             ? k_seq / kKeys : k_tile / kKeys;
-        n_fast = min(n_steps, n_full);
+        n_fast = min(n_steps, n_full - n_skip);
         n_spread = n_fast;
         if(MODE == NNTILE_HIP_MASK_CAUSAL)
         {
@@ -891,13 +932,13 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             fetch_v(nxt, lds_v0);
         }
         advance(nxt);
-        if(n_fast > 0)
+        if(n_fast > 0 && !first_requested)
         {
             fetch_k(nxt, lds_k1);       // the pipelined loop keeps K two steps ahead
         }
-        if(mask_wide && n_fast == 0 && cur.rows_left >= kKeys)
+        if(EXPLICIT && n_fast == 0)
         {
-            mask_fetch(cur.kb);
+            mask_fetch(cur.kb, cur.rows_left);
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -922,9 +963,13 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         const int keys_here = min(kKeys, cur.rows_left);
         // explicit mask: what this wavefront's block of the mask looks like
         // (the values were loaded during the previous step)
-        int mask_class = MASK_SLOW;
-        if(EXPLICIT && mask_wide && keys_here == kKeys)
+        int mask_class = MASK_MIXED;
+        if(EXPLICIT)
         {
+            if(keys_here < kKeys)
+            {
+                mask_fix_ragged(keys_here);
+            }
             mask_class = mask_classify();
         }
         // nothing of this step is visible to this wavefront, or the step is
@@ -998,46 +1043,6 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                                 {
                                     s[mb][r0 + e] = neg_inf();
                                 }
-                            }
-                        }
-                    }
-                }
-                else if(mask_class == MASK_SLOW)
-                {
-#pragma unroll
-                    for(int mb = 0; mb < 2; ++mb)
-                    {
-#pragma unroll
-                        for(int rg = 0; rg < 4; ++rg)
-                        {
-                            const int key0 = mb * 32 + 8 * rg + 4 * half;
-#pragma unroll
-                            for(int e = 0; e < 4; ++e)
-                            {
-                                // out-of-range keys of a ragged step are hidden;
-                                // their loads are clamped to the step's last key
-                                // instead of being branched around, so that the
-                                // 32 loads of a lane are independent and overlap
-                                const int64_t at = mask_row + k_row0
-                                    + max(min(key0 + e, keys_here - 1), 0);
-                                float add;
-                                if(MODE == NNTILE_HIP_MASK_ADDITIVE)
-                                {
-                                    add = T::to_float(static_cast<const uint16_t *>(
-                                                p.mask)[at]);
-                                }
-                                else
-                                {
-                                    add = static_cast<const uint8_t *>(
-                                            p.mask)[at] != 0
-                                        ? 0.0f : neg_inf();
-                                }
-                                if(key0 + e >= keys_here)
-                                {
-                                    add = neg_inf();
-                                }
-                                s[mb][4 * rg + e] = fmaf(add, inv_scale,
-                                        s[mb][4 * rg + e]);
                             }
                         }
                     }
@@ -1126,10 +1131,9 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             l_run += rs0 + rs1;
         }
         // mask values of the next step (this step's have been consumed)
-        if(EXPLICIT && mask_wide && g + 1 < n_steps
-                && cur.rows_left - GROUPS * kKeys >= kKeys)
+        if(EXPLICIT && g + 1 < n_steps)
         {
-            mask_fetch(cur.kb + GROUPS);
+            mask_fetch(cur.kb + GROUPS, cur.rows_left - GROUPS * kKeys);
         }
         NNTILE_PHASE(2)
 
@@ -1500,9 +1504,9 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         }
         g_first = n_fast;
         nxt = c1;
-        if(EXPLICIT && mask_wide && g_first < n_steps && cur.rows_left >= kKeys)
+        if(EXPLICIT && g_first < n_steps)
         {
-            mask_fetch(cur.kb);     // the general step finds its mask values loaded
+            mask_fetch(cur.kb, cur.rows_left);     // the general step finds its mask values loaded
         }
         // the general loop expects step g_first complete in its buffers
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1588,8 +1592,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     const bool live = q_ok && !(empty && !p.overwrite);
     const float to_ln = p.scale;
     const float lse_new = empty ? neg_inf() : m_run * to_ln + __logf(l_tot);
-    float *lse_ptr = p.lse[q_tile0 + qt] + (int64_t)b * q_len + (q_ok ? my_q : 0);
-    const float lse_old = (p.overwrite || !live) ? neg_inf() : *lse_ptr;
+    const float lse_old = live ? lse_stored : neg_inf();
     float w_old = 0.0f, w_new = 0.0f, lse_out = neg_inf();
     if(live && !empty)
     {
@@ -1602,78 +1605,67 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     const float w_o = (empty || !live) ? 0.0f : w_new / l_tot;
     // register r of block db holds head value  db*32 + 8*(r/4) + 4*half + r%4
 
-    if(__builtin_amdgcn_ballot_w64(live && w_old != 0.0f) == 0)
+    // The wavefront's 32 rows go through LDS (its own quarter of the K
+    // buffers, which nobody reads any more after the last barrier) so that they
+    // leave as whole rows, 16 bytes per lane, instead of 8-byte pieces 2*HEAD
+    // bytes apart - and, where the old A is merged in, come the same way: all
+    // its loads are in flight at once and a lane finds its pieces where it
+    // writes the sums.  (Loaded and stored in 8-byte pieces the merge of a
+    // 1024 x 1024 x 32 tile pair took 3 us more.)
+    // 16-byte chunk c of row r sits at chunk position c ^ (r % CPR).
+    // (two wavefronts per buffer: K0, K1, then V0, V1 for wavefronts 4 to 7)
+    // (two groups: wavefront w uses the end of array w, behind the triple
+    // it has just read - a neighbour may still be reading its own)
+    char *xch = GROUPS > 1
+        ? (wave == 0 ? lds_k0 : wave == 1 ? lds_k1 : wave == 2 ? lds_v0 : lds_v1)
+            + (K_BYTES * GROUPS - 32 * RB)
+        : ((wave >> 1) == 0 ? lds_k0 : (wave >> 1) == 1 ? lds_k1
+            : (wave >> 1) == 2 ? lds_v0 : lds_v1) + (wave & 1) * 32 * RB;
+    const uint64_t live_rows = __builtin_amdgcn_ballot_w64(live && half == 0);
+    constexpr int ROWS_PER_ST = 1024 / RB;      // rows one load or store instruction covers
+    constexpr int N_ST = 32 / ROWS_PER_ST;
+    const int st_row = lane / CPR, st_c = lane % CPR;
+    char *Abase = static_cast<char *>(p.A[q_tile0 + qt])
+        + ((int64_t)b * q_len + q_row0 + wave * 32) * RB;
+    const bool merge = __builtin_amdgcn_ballot_w64(live && w_old != 0.0f) != 0;
+    if(merge)
     {
-        // Nothing of the old A is needed by this wavefront: its 32 rows go
-        // through LDS (its own quarter of the K buffers, which nobody reads
-        // any more after the last barrier) so that they leave as whole rows,
-        // 16 bytes per lane, instead of 8-byte pieces 2*HEAD bytes apart.
-        // 16-byte chunk c of row r sits at chunk position c ^ (r % CPR).
-        // (two wavefronts per buffer: K0, K1, then V0, V1 for wavefronts 4 to 7)
-        // (two groups: wavefront w uses the end of array w, behind the triple
-        // it has just read - a neighbour may still be reading its own)
-        char *xch = GROUPS > 1
-            ? (wave == 0 ? lds_k0 : wave == 1 ? lds_k1 : wave == 2 ? lds_v0 : lds_v1)
-                + (K_BYTES * GROUPS - 32 * RB)
-            : ((wave >> 1) == 0 ? lds_k0 : (wave >> 1) == 1 ? lds_k1
-                : (wave >> 1) == 2 ? lds_v0 : lds_v1) + (wave & 1) * 32 * RB;
+        u32x4 old[N_ST];
 #pragma unroll
-        for(int db = 0; db < DBLOCKS; ++db)
+        for(int i = 0; i < N_ST; ++i)
         {
-#pragma unroll
-            for(int rg = 0; rg < 4; ++rg)
-            {
-                u32x2 out;
-                out[0] = T::pack2(o[db][4 * rg] * w_o, o[db][4 * rg + 1] * w_o);
-                out[1] = T::pack2(o[db][4 * rg + 2] * w_o, o[db][4 * rg + 3] * w_o);
-                const int cpos = (db * 4 + rg) ^ (col % CPR);
-                *reinterpret_cast<u32x2 *>(xch + col * RB + cpos * 16 + 8 * half) = out;
-            }
+            // (the rows of a tile end at q_len: rows past it re-read row 0)
+            const int r = i * ROWS_PER_ST + st_row;
+            const bool there = (live_rows >> r) & 1;
+            old[i] = *reinterpret_cast<const u32x4 *>(
+                    Abase + (there ? (int64_t)r * RB : -(int64_t)wave * 32 * RB) + st_c * 16);
         }
-        const uint64_t live_rows = __builtin_amdgcn_ballot_w64(live && half == 0);
-        constexpr int ROWS_PER_ST = 1024 / RB;      // rows one store instruction covers
-        char *Abase = static_cast<char *>(p.A[q_tile0 + qt])
-            + ((int64_t)b * q_len + q_row0 + wave * 32) * RB;
 #pragma unroll
-        for(int i = 0; i < 32 / ROWS_PER_ST; ++i)
+        for(int i = 0; i < N_ST; ++i)
         {
-            const int r = i * ROWS_PER_ST + lane / CPR;
-            const int c = lane % CPR;
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(
-                    xch + r * RB + (c ^ (r % CPR)) * 16);
-            if((live_rows >> r) & 1)
-            {
-                *reinterpret_cast<u32x4 *>(Abase + (int64_t)r * RB + c * 16) = v;
-            }
+            const int r = i * ROWS_PER_ST + st_row;
+            *reinterpret_cast<u32x4 *>(xch + r * RB + (st_c ^ (r % CPR)) * 16) = old[i];
         }
-#ifdef NNTILE_PF_TRACE
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        PF_STAMP(4);
-#endif
-        return;
     }
-    if(!live)
-    {
-        return;
-    }
-    uint16_t *Arow = static_cast<uint16_t *>(p.A[q_tile0 + qt])
-        + ((int64_t)b * q_len + my_q) * HEAD;
 #pragma unroll
     for(int db = 0; db < DBLOCKS; ++db)
     {
 #pragma unroll
         for(int rg = 0; rg < 4; ++rg)
         {
-            uint16_t *dst = Arow + db * 32 + 8 * rg + 4 * half;
+            const int cpos = (db * 4 + rg) ^ (col % CPR);
+            u32x2 *at = reinterpret_cast<u32x2 *>(xch + col * RB + cpos * 16 + 8 * half);
             float v[4];
 #pragma unroll
             for(int e = 0; e < 4; ++e)
             {
-                v[e] = empty ? 0.0f : o[db][4 * rg + e] * w_o;
+                v[e] = o[db][4 * rg + e] * w_o;
             }
-            if(w_old != 0.0f)
+            if(merge)
             {
-                const u32x2 old = *reinterpret_cast<const u32x2 *>(dst);
+                const u32x2 prev = *at;
+                // (a row that does not need its old A may hold anything)
+                const u32x2 old = w_old != 0.0f ? prev : u32x2{0, 0};
                 v[0] += w_old * T::to_float((uint16_t)(old[0] & 0xffffu));
                 v[1] += w_old * T::to_float((uint16_t)(old[0] >> 16));
                 v[2] += w_old * T::to_float((uint16_t)(old[1] & 0xffffu));
@@ -1682,9 +1674,24 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             u32x2 out;
             out[0] = T::pack2(v[0], v[1]);
             out[1] = T::pack2(v[2], v[3]);
-            *reinterpret_cast<u32x2 *>(dst) = out;
+            *at = out;
         }
     }
+#pragma unroll
+    for(int i = 0; i < N_ST; ++i)
+    {
+        const int r = i * ROWS_PER_ST + st_row;
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(
+                xch + r * RB + (st_c ^ (r % CPR)) * 16);
+        if((live_rows >> r) & 1)
+        {
+            *reinterpret_cast<u32x4 *>(Abase + (int64_t)r * RB + st_c * 16) = v;
+        }
+    }
+#ifdef NNTILE_PF_TRACE
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    PF_STAMP(4);
+#endif
 }
 
 template<typename T, int HEAD>
@@ -1774,22 +1781,26 @@ static int launch_mode(hipStream_t stream, const PrefillParams &p, int mode,
 // here; see PrefillParams::mask_bits).
 template<int ES>
 __global__ __launch_bounds__(kThreads)
-void mask_step_bits_kernel(const char *mask, int ld_bytes, int q_len, int n_chunks,
+void mask_step_bits_kernel(const char *mask, uint32_t ld_bytes, int q_len, int k_seq,
         uint32_t open_word, uint32_t hidden_word, unsigned long long *table)
 {
-    __shared__ unsigned long long bits[2];
-    mask_scan_range<ES, kThreads>(mask, ld_bytes, q_len, n_chunks, open_word, hidden_word,
-            (int)blockIdx.x / kMaskBitSplits, (int)blockIdx.x % kMaskBitSplits, bits);
+    __shared__ unsigned long long words[2 * kThreads / 64];
+    unsigned long long not_open, not_hidden;
+    mask_scan_range<ES, kThreads / 64>(mask, ld_bytes, q_len, k_seq, open_word, hidden_word,
+            (int)blockIdx.x / kMaskBitSplits, (int)blockIdx.x % kMaskBitSplits, words, not_open,
+            not_hidden);
     if(threadIdx.x == 0)
     {
-        table[3 * (int64_t)blockIdx.x] = bits[0];
-        table[3 * (int64_t)blockIdx.x + 1] = bits[1];
+        table[3 * (int64_t)blockIdx.x] = not_open;
+        table[3 * (int64_t)blockIdx.x + 1] = not_hidden;
     }
 }
 
 // Masks below this size are scanned by the attention kernel's workgroups
-// themselves: the launch of the scan would cost more than it saves.
-constexpr int64_t kMaskScanLaunchBytes = 1 << 20;
+// themselves, each its own rows: waiting for the shared scan costs a workgroup
+// about 2 us more than its first loads, scanning 128 rows of 400 values about
+// as much (7 x 355^2: 0.5 % slower shared, 10 x 621^2: 12 % faster).
+constexpr int64_t kMaskScanBytes = 3 << 17;
 
 // A value no earlier call of this process has used and that memory left
 // behind by anything else is unlikely to hold (never 0).
@@ -1826,12 +1837,10 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
     const int64_t es = additive ? 2 : 1;
     const int64_t row_bytes = p.k_seq * es;
     const int64_t table_bytes = (int64_t)p.q_blocks_per_tile * kMaskBitSplits * 24;
-    if(row_bytes % 16 != 0 || (p.mask_ld * es) % 16 != 0
-            || reinterpret_cast<uintptr_t>(p.mask) % 16 != 0
-            || p.mask_ld * es * kQRows >= (int64_t)(1 << 30)
+    if(row_bytes < 16 || p.mask_ld * es * kQRows >= (int64_t)(1 << 30)
             || reinterpret_cast<uintptr_t>(scratch) % 8 != 0
             || (int64_t)scratch_bytes < table_bytes
-            || p.q_seq * row_bytes < kMaskScanLaunchBytes || p.batch < 2)
+            || p.q_seq * row_bytes < kMaskScanBytes || p.batch < 2)
     {
         return NNTILE_HIP_OK;
     }
@@ -1854,14 +1863,14 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
     if(additive)
     {
         hipLaunchKernelGGL((mask_step_bits_kernel<2>), grid, dim3(kThreads), 0, stream,
-                static_cast<const char *>(p.mask), (int)(p.mask_ld * es), (int)p.q_seq,
-                (int)(row_bytes / 16), 0u, T::kNegInfPair, table);
+                static_cast<const char *>(p.mask), (uint32_t)(p.mask_ld * es), (int)p.q_seq,
+                (int)p.k_seq, 0u, T::kNegInfPair, table);
     }
     else
     {
         hipLaunchKernelGGL((mask_step_bits_kernel<1>), grid, dim3(kThreads), 0, stream,
-                static_cast<const char *>(p.mask), (int)(p.mask_ld * es), (int)p.q_seq,
-                (int)(row_bytes / 16), 0x01010101u, 0u, table);
+                static_cast<const char *>(p.mask), (uint32_t)(p.mask_ld * es), (int)p.q_seq,
+                (int)p.k_seq, 0x01010101u, 0u, table);
     }
     if(hipGetLastError() != hipSuccess)
     {
