@@ -9,7 +9,8 @@
 //
 // (include/nntile/kernel/flash_sdpa_bwd_cudnn/cuda.hh:44-68 is the interface
 // this replaces; tests/kernel/flash_sdpa_bwd_cudnn.cc:174-262 the arithmetic).
-// A small kernel writes D; then ONE launch computes the three gradients, each
+// A small launch writes D (and looks over a mask given as values); then ONE
+// launch computes the three gradients, each
 // by its own workgroups (no atomics, results independent of timing):
 //
 //  * sdpa_bwd_dq_body: a workgroup owns 128 queries (a wavefront 32, a lane
@@ -186,82 +187,174 @@ __device__ __forceinline__ int tile_row(int r, int half)
 }
 
 // ---------------------------------------------------------------------------------
-// Masks given as values: one pass writes the class of every 64 x 64 block of
-// the mask (the reference hands the kernel a materialised tile even where it is
-// causal, src/tile/flash_sdpa_bwd_cudnn.cc), so that the three kernels below skip
-// the steps whose blocks hide everything - without fetching them - and read no
-// mask values in the steps whose blocks mask nothing.
-constexpr int kMaskMixed = 0, kMaskOpen = 1, kMaskHidden = 2;
+// What the gradient launch needs first, in one launch of its own (the row dots
+// tile by tile and the classes of the mask blocks apart were up to nine
+// launches; each costs the stream 2 to 4 us):
+//
+//  * the row dots D[b][q] = dA[b][q][:] . A[b][q][:] in fp32: 16-byte loads,
+//    HEAD/8 lanes a row, kRowdotRows rows per lane in flight, summed across
+//    those lanes;
+//  * for a mask given as values the class of every 64 x 64 block (the
+//    reference hands the kernel a materialised tile even where it is causal,
+//    src/tile/flash_sdpa_bwd_cudnn.cc), so that the gradient bodies skip the
+//    steps whose blocks hide everything - without fetching them - and read mask
+//    values only where they must: not in blocks that mask nothing, and not in
+//    blocks that hold exactly what the rule `key <= query` (rows and columns
+//    of this tile) makes of them - the diagonal blocks of a causal tile.
+//
+// Class bits of a block: some value is visible; some value is not "open" (+0 /
+// true); some value is not what the rule says.
+constexpr int kMaskVisible = 1, kMaskMasked = 2, kMaskOffRule = 4;
+constexpr int kRowdotRows = 2;
+
+struct BwdPreludeParams
+{
+    int64_t q_seq, q_tile, mask_ld;
+    float *D;
+    const void *mask;
+    uint8_t *table;
+    int32_t k_seq, class_ld;        // (masks: one tile of each axis)
+    int32_t batch, n_q_tiles;       // slab s's tiles at [s*n_q_tiles + t] of the tables
+    int32_t n_class_wgs, wgs_per_tile;
+    const void *dA[kBwdMaxTiles];
+    const void *A[kBwdMaxTiles];
+};
 
 template<typename T, int MODE>
-__global__ __launch_bounds__(256)
-void sdpa_bwd_mask_classes_kernel(const void *mask, int64_t mask_ld, int q_seq, int k_seq,
-        uint8_t *table, int class_ld)
+__device__ __forceinline__ void bwd_mask_class(const BwdPreludeParams &p, int wg)
 {
-    const int qb = blockIdx.x / class_ld, kb = blockIdx.x % class_ld;
+    constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 2 : 1;
+    constexpr int PER_WORD = 4 / ES;
+    constexpr uint32_t OPEN = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0u : 0x01010101u;
+    constexpr uint32_t HIDDEN = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? T::kNegInfPair : 0u;
+    typedef u32x4 __attribute__((aligned(1))) u32x4_any;
+    const int qb = wg / p.class_ld, kb = wg % p.class_ld;
     const int row = qb * kBwdStep + (int)threadIdx.x / 4;
     const int col0 = kb * kBwdStep + ((int)threadIdx.x % 4) * 16;
-    bool any_visible = false, any_masked = false;
-    constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 2 : 1;
-    const bool wide = (mask_ld * ES) % 16 == 0 && reinterpret_cast<uintptr_t>(mask) % 16 == 0;
-    if(row < q_seq && col0 < k_seq)
+    uint32_t seen = 0u;
+    if(row < (int)p.q_seq && col0 < p.k_seq)
     {
-        const char *src = static_cast<const char *>(mask) + ((int64_t)row * mask_ld + col0) * ES;
-        if(wide && col0 + 16 <= k_seq)
+        const char *src = static_cast<const char *>(p.mask) + ((int64_t)row * p.mask_ld + col0) * ES;
+        const int n_vis = row - col0 + 1;       // columns of this thread that the rule shows
+        if(col0 + 16 <= p.k_seq)
         {
-            // the thread's 16 values as 16-byte loads
+            // the thread's 16 values as 16-byte loads of any alignment
+            u32x4 v[ES];
 #pragma unroll
             for(int i = 0; i < ES; ++i)
             {
-                const u32x4 v = *reinterpret_cast<const u32x4 *>(src + 16 * i);
-#pragma unroll
-                for(int w = 0; w < 4; ++w)
-                {
-                    if(MODE == NNTILE_HIP_MASK_ADDITIVE)
-                    {
-                        any_masked |= v[w] != 0u;
-                        any_visible |= v[w] != T::kNegInfPair;
-                    }
-                    else
-                    {
-                        any_masked |= v[w] != 0x01010101u;
-                        any_visible |= v[w] != 0u;
-                    }
-                }
+                v[i] = *reinterpret_cast<const u32x4_any *>(src + 16 * i);
             }
+            uint32_t masked = 0u, visible = 0u, off = 0u;
+#pragma unroll
+            for(int w = 0; w < 4 * ES; ++w)
+            {
+                const uint32_t x = v[w / 4][w % 4];
+                masked |= x ^ OPEN;
+                visible |= x ^ HIDDEN;
+                // elements PER_WORD*w ..: the first n of them are shown
+                const int n = min(max(n_vis - PER_WORD * w, 0), PER_WORD);
+                const uint32_t low = n == PER_WORD ? ~0u : (1u << (8 * ES * n)) - 1u;
+                off |= x ^ ((OPEN & low) | (HIDDEN & ~low));
+            }
+            seen = (visible != 0u ? kMaskVisible : 0) | (masked != 0u ? kMaskMasked : 0)
+                | (off != 0u ? kMaskOffRule : 0);
         }
         else
         {
-            for(int e = 0; e < 16 && col0 + e < k_seq; ++e)
+            for(int e = 0; e < p.k_seq - col0; ++e)
             {
+                bool open, hidden;
                 if(MODE == NNTILE_HIP_MASK_ADDITIVE)
                 {
-                    const uint16_t v = reinterpret_cast<const uint16_t *>(src)[e];
-                    any_visible |= (T::to_float(v) != neg_inf());
-                    any_masked |= (v != 0);         // anything but +0 changes the score
+                    const uint16_t x = reinterpret_cast<const uint16_t *>(src)[e];
+                    open = x == 0;              // anything but +0 changes the score
+                    hidden = x == (uint16_t)T::kNegInfPair;
                 }
                 else
                 {
-                    const bool vis = reinterpret_cast<const uint8_t *>(src)[e] != 0;
-                    any_visible |= vis;
-                    any_masked |= !vis;
+                    open = reinterpret_cast<const uint8_t *>(src)[e] == 1;
+                    hidden = reinterpret_cast<const uint8_t *>(src)[e] == 0;
                 }
+                seen |= (!hidden ? kMaskVisible : 0) | (!open ? kMaskMasked : 0)
+                    | ((e < n_vis ? !open : !hidden) ? kMaskOffRule : 0);
             }
         }
     }
-    const int vis = __syncthreads_or(any_visible ? 1 : 0);
-    const int msk = __syncthreads_or(any_masked ? 1 : 0);
+    uint32_t all = 0u;
+#pragma unroll
+    for(int b = 0; b < 3; ++b)
+    {
+        all |= __syncthreads_or((int)(seen & (1u << b))) != 0 ? (1u << b) : 0u;
+    }
     if(threadIdx.x == 0)
     {
-        table[blockIdx.x] = (uint8_t)(!msk ? kMaskOpen : (!vis ? kMaskHidden : kMaskMixed));
+        p.table[wg] = (uint8_t)all;
+    }
+}
+
+template<typename T, int HEAD, int MODE>
+__global__ __launch_bounds__(256)
+void sdpa_bwd_prelude_kernel(const BwdPreludeParams p)
+{
+    if constexpr(MODE == NNTILE_HIP_MASK_ADDITIVE || MODE == NNTILE_HIP_MASK_BOOL)
+    {
+        if((int)blockIdx.x < p.n_class_wgs)
+        {
+            bwd_mask_class<T, MODE>(p, (int)blockIdx.x);
+            return;
+        }
+    }
+    constexpr int LANES = HEAD / 8;             // lanes per row: 16, 8 or 4
+    constexpr int ROWS = 256 / LANES;           // rows one load of the workgroup covers
+    const int wg = (int)blockIdx.x - p.n_class_wgs;
+    const int tile = wg / p.wgs_per_tile;
+    const int64_t t0 = (int64_t)(tile % p.n_q_tiles) * p.q_tile;
+    const int64_t rows = (int64_t)p.batch * min(p.q_tile, p.q_seq - t0);
+    const int64_t row0 = (int64_t)(wg % p.wgs_per_tile) * (ROWS * kRowdotRows)
+        + (int)threadIdx.x / LANES;
+    const int part = (int)(threadIdx.x % LANES);
+    const uint16_t *dA = static_cast<const uint16_t *>(p.dA[tile]) + part * 8;
+    const uint16_t *A = static_cast<const uint16_t *>(p.A[tile]) + part * 8;
+    float *D = p.D + (int64_t)(tile / p.n_q_tiles) * p.q_seq * p.batch + (int64_t)p.batch * t0;
+    u32x4 g[kRowdotRows], a[kRowdotRows];
+#pragma unroll
+    for(int i = 0; i < kRowdotRows; ++i)
+    {
+        // (rows past the end read the last one)
+        const int64_t row = min(row0 + i * ROWS, rows - 1);
+        g[i] = *reinterpret_cast<const u32x4 *>(dA + row * HEAD);
+        a[i] = *reinterpret_cast<const u32x4 *>(A + row * HEAD);
+    }
+#pragma unroll
+    for(int i = 0; i < kRowdotRows; ++i)
+    {
+        float d = 0.0f;
+#pragma unroll
+        for(int e = 0; e < 4; ++e)
+        {
+            d += T::to_float((uint16_t)(g[i][e] & 0xffffu))
+                * T::to_float((uint16_t)(a[i][e] & 0xffffu));
+            d += T::to_float((uint16_t)(g[i][e] >> 16)) * T::to_float((uint16_t)(a[i][e] >> 16));
+        }
+#pragma unroll
+        for(int o = LANES / 2; o >= 1; o >>= 1)
+        {
+            d += __shfl_xor(d, o, 64);
+        }
+        if(row0 + i * ROWS < rows && part == 0)
+        {
+            D[row0 + i * ROWS] = d;
+        }
     }
 }
 
 // The steps a workgroup takes, as a bit set (up to 64 of them; longer walks
-// take every step), and the subset in which nothing is masked.
+// take every step), the subset in which nothing is masked and the subset in
+// which the mask is the rule `key <= query`.
 struct StepSet
 {
-    unsigned long long active, open;
+    unsigned long long active, open, rule;
     bool use_bits;
     int first, last;        // [first, last): the walk without the table
 
@@ -286,6 +379,10 @@ struct StepSet
     {
         return use_bits && ((open >> g) & 1ull) != 0ull;
     }
+    __device__ __forceinline__ bool is_rule(int g) const
+    {
+        return use_bits && ((rule >> g) & 1ull) != 0ull;
+    }
 };
 
 // Step set of a workgroup that owns the blocks [own0, own0 + n_own) of one axis
@@ -300,58 +397,95 @@ __device__ __forceinline__ StepSet make_step_set(const BwdParams &p, bool explic
     s.use_bits = explicit_mask && p.mask_class != nullptr && last <= 64;
     s.active = 0ull;
     s.open = 0ull;
+    s.rule = 0ull;
     if(s.use_bits)
     {
         // lane g looks at step g; the ballots make the two sets (every
         // wavefront computes the same)
         const int g = (int)(threadIdx.x & 63);
         const bool in_walk = g >= first && g < last;
-        bool hidden = true, open = true;
+        int c = 0;
         for(int o = 0; o < n_own; ++o)
         {
             const int idx = by_row ? (own0 + o) * p.class_ld + g : g * p.class_ld + own0 + o;
-            const int c = in_walk ? p.mask_class[idx] : kMaskHidden;
-            hidden = hidden && (c == kMaskHidden);
-            open = open && (c == kMaskOpen);
+            c |= in_walk ? p.mask_class[idx] : 0;
         }
-        s.active = __builtin_amdgcn_ballot_w64(in_walk && !hidden);
-        s.open = __builtin_amdgcn_ballot_w64(in_walk && open);
+        s.active = __builtin_amdgcn_ballot_w64(in_walk && (c & kMaskVisible) != 0);
+        s.open = __builtin_amdgcn_ballot_w64(in_walk && (c & kMaskMasked) == 0);
+        s.rule = __builtin_amdgcn_ballot_w64(in_walk && (c & kMaskOffRule) == 0);
     }
     return s;
 }
 
-// ---------------------------------------------------------------------------------
-// D[b][q] = dA[b][q][:] . A[b][q][:] in fp32, for the workgroups below: 16-byte
-// loads, HEAD/8 lanes a row, summed across those lanes.
+// A wavefront's 32 rows of a gradient (accumulators acc, transposed: register r
+// of block db is head value db*32 + tile_row(r, half) of row lane % 32), times
+// factor, to memory through LDS - so that they leave, and what they are added
+// to arrives, as whole rows, 16 bytes a lane, instead of 8-byte pieces 2*HEAD
+// bytes apart.  xch: 32 rows of LDS of the wavefront's own; base: the first
+// row; n_ok: rows that exist (may be none or more than 32).
 template<typename T, int HEAD>
-__global__ __launch_bounds__(256)
-void sdpa_bwd_rowdot_kernel(const void *dA, const void *A, float *D, int64_t rows)
+__device__ __forceinline__ void bwd_store_rows(char *xch, char *base, int n_ok,
+        const f32x16 (&acc)[HEAD / 32], float factor, bool add)
 {
-    constexpr int LANES = HEAD / 8;             // lanes per row: 16, 8 or 4
-    const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) / LANES;
-    const int part = (int)(threadIdx.x % LANES);
-    float d = 0.0f;
-    if(row < rows)
+    typedef BwdTile<HEAD> G;
+    constexpr int RB = G::RB, CPR = G::CPR, RPI = G::ROWS_PER_LOAD, N = 32 / RPI;
+    if(n_ok <= 0)
     {
-        const u32x4 g = *reinterpret_cast<const u32x4 *>(
-                static_cast<const uint16_t *>(dA) + row * HEAD + part * 8);
-        const u32x4 a = *reinterpret_cast<const u32x4 *>(
-                static_cast<const uint16_t *>(A) + row * HEAD + part * 8);
+        return;
+    }
+    const int lane = lane_index_again();
+    const int st_row = lane / CPR, st_c = lane % CPR;
+    if(add)
+    {
+        u32x4 old[N];
 #pragma unroll
-        for(int e = 0; e < 4; ++e)
+        for(int i = 0; i < N; ++i)
         {
-            d += T::to_float((uint16_t)(g[e] & 0xffffu)) * T::to_float((uint16_t)(a[e] & 0xffffu));
-            d += T::to_float((uint16_t)(g[e] >> 16)) * T::to_float((uint16_t)(a[e] >> 16));
+            old[i] = *reinterpret_cast<const u32x4 *>(base
+                    + (int64_t)min(i * RPI + st_row, n_ok - 1) * RB + st_c * 16);
+        }
+#pragma unroll
+        for(int i = 0; i < N; ++i)
+        {
+            const int r = i * RPI + st_row;
+            *reinterpret_cast<u32x4 *>(xch + r * RB + (st_c ^ (r % CPR)) * 16) = old[i];
+        }
+    }
+    const int col = lane & 31, half = lane >> 5;
+#pragma unroll
+    for(int db = 0; db < G::DBLOCKS; ++db)
+    {
+#pragma unroll
+        for(int rg = 0; rg < 4; ++rg)
+        {
+            u32x2 *at = reinterpret_cast<u32x2 *>(xch + col * RB
+                    + ((db * 4 + rg) ^ (col % CPR)) * 16 + 8 * half);
+            float v[4];
+#pragma unroll
+            for(int e = 0; e < 4; ++e)
+            {
+                v[e] = acc[db][4 * rg + e] * factor;
+            }
+            if(add)
+            {
+                const u32x2 old = *at;
+                v[0] += T::to_float((uint16_t)(old[0] & 0xffffu));
+                v[1] += T::to_float((uint16_t)(old[0] >> 16));
+                v[2] += T::to_float((uint16_t)(old[1] & 0xffffu));
+                v[3] += T::to_float((uint16_t)(old[1] >> 16));
+            }
+            *at = u32x2{T::pack2(v[0], v[1]), T::pack2(v[2], v[3])};
         }
     }
 #pragma unroll
-    for(int o = LANES / 2; o >= 1; o >>= 1)
+    for(int i = 0; i < N; ++i)
     {
-        d += __shfl_xor(d, o, 64);
-    }
-    if(row < rows && part == 0)
-    {
-        D[row] = d;
+        const int r = i * RPI + st_row;
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(xch + r * RB + (st_c ^ (r % CPR)) * 16);
+        if(r < n_ok)
+        {
+            *reinterpret_cast<u32x4 *>(base + (int64_t)r * RB + st_c * 16) = v;
+        }
     }
 }
 
@@ -463,7 +597,8 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
 
     // ---- which keys ---------------------------------------------------------------
     // key row kg is visible to query row q iff kg <= rel + q (causal)
-    int64_t rel64 = p.q_pos0 + p.causal_offset - p.k_pos0;
+    // (a mask given as values: the rule its blocks are compared with)
+    int64_t rel64 = EXPLICIT ? 0 : p.q_pos0 + p.causal_offset - p.k_pos0;
     rel64 = max((int64_t)-(1 << 30), min(rel64, (int64_t)(1 << 30)));
     const int rel = (int)rel64;
     int n_steps = (k_seq + kBwdStep - 1) / kBwdStep;
@@ -596,6 +731,8 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     const char *mask_wg = static_cast<const char *>(p.mask)
         + (int64_t)q_row0 * p.mask_ld * (int64_t)MASK_ES;
     const uint32_t mask_row_off = (uint32_t)(q_ok ? my_q - q_row0 : 0) * (uint32_t)p.mask_ld * MASK_ES;
+    // (at head 128 the groups of four cost registers that the body does not have)
+    constexpr bool MASK_GROUPS = HEAD <= 64;
     const uint32_t mask_off_wg = mask_row_off + (uint32_t)(4 * half) * MASK_ES;
 
     // the workgroup's two query blocks of 64 against the key blocks 0 .. n_steps-1
@@ -628,7 +765,9 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
         const int kg0 = g * kBwdStep;
         const int keys_here = min(kBwdStep, k_seq - kg0);
         const char *mask_step = mask_wg + (int64_t)kg0 * MASK_ES;
-        const uint32_t mask_off_last = mask_row_off + (uint32_t)(keys_here - 1) * MASK_ES;
+        // (the last place that a group of values, or a value, can start at)
+        const uint32_t mask_off_last = mask_row_off
+            + (uint32_t)max(keys_here - (MASK_GROUPS ? 4 : 1), 0) * MASK_ES;
         // (through an empty asm statement: the 32 offsets that a step adds
         // constants to are then made where the step uses them instead of once
         // before the loop and kept, which at head 128 means spilled)
@@ -642,7 +781,10 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
         // (one 32-key block at a time: half the accumulators live)
         // ---- P^T, dS^T: register r of block mb is key mb*32 + tile_row(r, half) ------------
         int lim = keys_here - 1;
-        if(MODE == NNTILE_HIP_MASK_CAUSAL)
+        // (the mask of this step is the rule `key <= query + rel`)
+        const bool ruled = MODE == NNTILE_HIP_MASK_CAUSAL
+            || (EXPLICIT && !use_mask && !steps.is_open(g));
+        if(ruled)
         {
             lim = min(lim, my_lim - kg0);
         }
@@ -650,8 +792,8 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
         // (wave-common: the last key of the step against the last key that
         // exists and the last key the workgroup's first query sees)
         const bool bounds = keys_here < kBwdStep
-            || (MODE == NNTILE_HIP_MASK_CAUSAL && kg0 + kBwdStep - 1 > rel + q_row0);
-        if constexpr(EXPLICIT || NNTILE_BWD_PIPE_DQ == 0)
+            || (ruled && kg0 + kBwdStep - 1 > rel + q_row0);
+        if constexpr(use_mask || NNTILE_BWD_PIPE_DQ == 0)
         {
 #pragma unroll
             for(int mb = 0; mb < 2; ++mb)
@@ -691,6 +833,44 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
                         sv[r] = mb * 32 + tile_row(r, 0) <= lim_less_half ? sv[r] : neg_inf();
                     }
                 }
+                // The values of four consecutive keys in one load of any
+                // alignment (2-byte loads, each touching 32 rows, took most of
+                // a masked step): wave-common address of the step's first key in
+                // the workgroup's first row + the lane's 32-bit offset.  A group
+                // that would reach past the row is moved back to end with it and
+                // shifted into place; keys past the end are hidden above.
+                uint64_t mval[4] = {0, 0, 0, 0};
+                if constexpr(use_mask && MASK_GROUPS)
+                {
+                    typedef std::conditional_t<MODE == NNTILE_HIP_MASK_ADDITIVE, uint64_t,
+                            uint32_t> group_t;
+                    typedef group_t __attribute__((aligned(1))) group_any;
+#pragma unroll
+                    for(int rg = 0; rg < 4; ++rg)
+                    {
+                        const uint32_t want = mask_off + (uint32_t)(mb * 32 + 8 * rg) * MASK_ES;
+                        const uint32_t at = min(want, mask_off_last);
+                        if(k_seq >= 4)
+                        {
+                            mval[rg] = (uint64_t)*reinterpret_cast<const group_any *>(
+                                    mask_step + at) >> (8u * min(want - at, 7u));
+                        }
+                        else
+                        {
+                            // (rows of less than one group: the lane's first)
+#pragma unroll
+                            for(int e = 0; mb == 0 && rg == 0 && e < 3; ++e)
+                            {
+                                const char *mp = mask_step + mask_row_off
+                                    + (uint32_t)min(e, k_seq - 1) * MASK_ES;
+                                const uint32_t x = (MODE == NNTILE_HIP_MASK_ADDITIVE)
+                                    ? *reinterpret_cast<const uint16_t *>(mp)
+                                    : *reinterpret_cast<const uint8_t *>(mp);
+                                mval[rg] |= (uint64_t)x << (8 * MASK_ES * e);
+                            }
+                        }
+                    }
+                }
                 float dsv[16];
 #pragma unroll
                 for(int r = 0; r < 16; ++r)
@@ -699,21 +879,29 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
                     bool visible = true;
                     if(use_mask)
                     {
-                        // wave-common address of the step's first key in the
-                        // workgroup's first row + the lane's 32-bit offset;
-                        // keys past the end read the last key, and are hidden
-                        const uint32_t key_off = (uint32_t)(mb * 32 + tile_row(r, 0)) * MASK_ES;
-                        const char *mp = mask_step + min(mask_off + key_off, mask_off_last);
+                        uint32_t x;
+                        if constexpr(MASK_GROUPS)
+                        {
+                            x = (uint32_t)(mval[r / 4] >> (8 * MASK_ES * (r % 4)))
+                                & (MODE == NNTILE_HIP_MASK_ADDITIVE ? 0xffffu : 0xffu);
+                        }
+                        else
+                        {
+                            const char *mp = mask_step + min(mask_off
+                                    + (uint32_t)(mb * 32 + tile_row(r, 0)) * MASK_ES, mask_off_last);
+                            x = (MODE == NNTILE_HIP_MASK_ADDITIVE)
+                                ? *reinterpret_cast<const uint16_t *>(mp)
+                                : *reinterpret_cast<const uint8_t *>(mp);
+                        }
                         if(MODE == NNTILE_HIP_MASK_ADDITIVE)
                         {
-                            const float add = T::to_float(*reinterpret_cast<const uint16_t *>(mp));
+                            const float add = T::to_float((uint16_t)x);
                             visible = visible && (add != neg_inf());
                             e = fmaf(add, kLog2e, e);
                         }
                         else
                         {
-                            const uint8_t shown = *reinterpret_cast<const uint8_t *>(mp);
-                            visible = visible && (shown != 0);
+                            visible = visible && (x != 0);
                         }
                     }
                     const float pr = use_mask ? (visible ? fast_exp2(e) : 0.0f) : fast_exp2(e);
@@ -916,7 +1104,7 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     };
     auto run = [&](int g, int g_next, auto buf_tag) __attribute__((always_inline))
     {
-        if(EXPLICIT && !steps.is_open(g))
+        if(EXPLICIT && !steps.is_open(g) && !steps.is_rule(g))
         {
             step(g, g_next, buf_tag, std::true_type{});
         }
@@ -942,43 +1130,12 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     // workgroup's LDS can be given away)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-    // ---- dQ (+)= scale acc: register r of block db is head value
-    // db*32 + tile_row(r, half); four consecutive ones per 8-byte store ----------------
-    if(!q_ok)
-    {
-        return;
-    }
-    const int lane_again = lane_index_again();
-    const int my_q_again = q_row0 + wave_u * 32 + (lane_again & 31);
-    const int half_again = lane_again >> 5;
-    uint16_t *dst = static_cast<uint16_t *>(dQ_own) + row_elem(my_q_again, true) * HEAD;
-#pragma unroll
-    for(int db = 0; db < DBLOCKS; ++db)
-    {
-#pragma unroll
-        for(int rg = 0; rg < 4; ++rg)
-        {
-            uint16_t *ptr = dst + db * 32 + 8 * rg + 4 * half_again;
-            float v[4];
-#pragma unroll
-            for(int e = 0; e < 4; ++e)
-            {
-                v[e] = acc[db][4 * rg + e] * p.scale;
-            }
-            if(!p.overwrite)
-            {
-                const u32x2 old = *reinterpret_cast<const u32x2 *>(ptr);
-                v[0] += T::to_float((uint16_t)(old[0] & 0xffffu));
-                v[1] += T::to_float((uint16_t)(old[0] >> 16));
-                v[2] += T::to_float((uint16_t)(old[1] & 0xffffu));
-                v[3] += T::to_float((uint16_t)(old[1] >> 16));
-            }
-            u32x2 out;
-            out[0] = T::pack2(v[0], v[1]);
-            out[1] = T::pack2(v[2], v[3]);
-            *reinterpret_cast<u32x2 *>(ptr) = out;
-        }
-    }
+    // ---- dQ (+)= scale acc (every wavefront is done with the tiles in LDS) -----------
+    __syncthreads();
+    const int row_first = q_row0 + wave_u * 32;
+    bwd_store_rows<T, HEAD>(wave_u == 0 ? lds_k0 : wave_u == 1 ? lds_k1 : wave_u == 2 ? lds_v0
+            : lds_v1, static_cast<char *>(dQ_own) + row_elem(row_first, true) * RB,
+            q_seq - row_first, acc, p.scale, !p.overwrite);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1116,7 +1273,8 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     }
 
     // key row kg is visible to query row q iff kg <= rel + q (causal)
-    int64_t rel64 = p.q_pos0 + p.causal_offset - p.k_pos0;
+    // (a mask given as values: the rule its blocks are compared with)
+    int64_t rel64 = EXPLICIT ? 0 : p.q_pos0 + p.causal_offset - p.k_pos0;
     rel64 = max((int64_t)-(1 << 30), min(rel64, (int64_t)(1 << 30)));
     const int rel = (int)rel64;
     const int n_steps = (q_seq + kBwdStep - 1) / kBwdStep;
@@ -1389,8 +1547,12 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
         const int rows_here = min(kBwdStep, q_seq - q0);
         // (wave-common: the workgroup's last key against the last key that
         // exists and the last key the step's first query sees)
+        // (ruled: the mask of this step is the rule `key <= query + rel`)
+        const bool ruled = MODE == NNTILE_HIP_MASK_CAUSAL
+            || (EXPLICIT && !use_mask && !steps.is_open(qs));
         const bool bounds = k_row0 + kDkvRows > k_seq
-            || (MODE == NNTILE_HIP_MASK_CAUSAL && k_row0 + kDkvRows - 1 > rel + q0);
+            || (ruled && k_row0 + kDkvRows - 1 > rel + q0);
+        const int vis_base = ruled ? rel + q0 : (1 << 30);
         // (the row stride through an empty asm statement: its multiples are
         // then computed where a step uses them - 32 scalar products - instead
         // of once before the loop and kept, which at head 128 means spilled)
@@ -1403,7 +1565,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
             + (int64_t)q0 * (int64_t)mask_row_bytes;
         const uint32_t mask_last_row = (uint32_t)(rows_here - 1) * mask_row_bytes;
 
-        if constexpr(!EXPLICIT && BOTH && HEAD > 64 && NNTILE_BWD_FUSED_ORDER == 1)
+        if constexpr(!use_mask && BOTH && HEAD > 64 && NNTILE_BWD_FUSED_ORDER == 1)
         {
             // Both gradients at head 128: 192 registers hold fragments and
             // accumulators, so a block goes product by product - S, P, dV, then
@@ -1445,9 +1607,9 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                         // (the lane's part on the left, the rest is wave-common)
                         const int qr = mb * 32 + tile_row(r, 0);
                         bool vis = k_ok;
-                        if(MODE == NNTILE_HIP_MASK_CAUSAL)
+                        if(MODE == NNTILE_HIP_MASK_CAUSAL || EXPLICIT)
                         {
-                            vis = vis && (my_k_less_half <= rel + q0 + qr);
+                            vis = vis && (my_k_less_half <= vis_base + qr);
                         }
                         sv[r] = vis ? sv[r] : neg_inf();
                     }
@@ -1530,7 +1692,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                 }
             }
         }
-        else if constexpr(EXPLICIT || NNTILE_BWD_PIPE == 0 || (BOTH && HEAD > 64))
+        else if constexpr(use_mask || NNTILE_BWD_PIPE == 0 || (BOTH && HEAD > 64))
         {
             // (one 32-query block at a time: half the accumulators live)
             // ---- S = Q K^T, dP = dA V^T: rows are queries, the lane's column its key;
@@ -1598,9 +1760,9 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                         // (the lane's part on the left, the rest is wave-common)
                         const int qr = mb * 32 + tile_row(r, 0);
                         bool vis = k_ok;
-                        if(MODE == NNTILE_HIP_MASK_CAUSAL)
+                        if(MODE == NNTILE_HIP_MASK_CAUSAL || EXPLICIT)
                         {
-                            vis = vis && (my_k_less_half <= rel + q0 + qr);
+                            vis = vis && (my_k_less_half <= vis_base + qr);
                         }
                         sv[r] = vis ? sv[r] : neg_inf();
                     }
@@ -1709,9 +1871,9 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                         // (the lane's part on the left, the rest is wave-common)
                         const int qr = mb * 32 + tile_row(r, 0);
                         bool vis = k_ok;
-                        if(MODE == NNTILE_HIP_MASK_CAUSAL)
+                        if(MODE == NNTILE_HIP_MASK_CAUSAL || EXPLICIT)
                         {
-                            vis = vis && (my_k_less_half <= rel + q0 + qr);
+                            vis = vis && (my_k_less_half <= vis_base + qr);
                         }
                         sv[mb][r] = vis ? sv[mb][r] : neg_inf();
                     }
@@ -1964,7 +2126,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     };
     auto run = [&](int i, int i_next, auto buf_tag) __attribute__((always_inline))
     {
-        if(EXPLICIT && !steps.is_open(i % kHeadStride))
+        if(EXPLICIT && !steps.is_open(i % kHeadStride) && !steps.is_rule(i % kHeadStride))
         {
             step(i, i_next, buf_tag, std::true_type{});
         }
@@ -1991,53 +2153,20 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     BWD_TRACE_FLUSH(PART);
-    // ---- dK (+)= scale dk, dV (+)= dv -------------------------------------------------
-    if(!k_ok)
-    {
-        return;
-    }
-    const int lane_again = lane_index_again();
-    const int my_k_again = k_row0 + wave_u * 32 + (lane_again & 31);
-    const int half_again = lane_again >> 5;
-    const int64_t k_off_again = row_elem(my_k_again, true) * HEAD;
-    auto store = [&](void *base, const f32x16 (&acc)[DBLOCKS], float factor)
-    {
-        uint16_t *dst = static_cast<uint16_t *>(base) + k_off_again;
-#pragma unroll
-        for(int db = 0; db < DBLOCKS; ++db)
-        {
-#pragma unroll
-            for(int rg = 0; rg < 4; ++rg)
-            {
-                uint16_t *ptr = dst + db * 32 + 8 * rg + 4 * half_again;
-                float v[4];
-#pragma unroll
-                for(int e = 0; e < 4; ++e)
-                {
-                    v[e] = acc[db][4 * rg + e] * factor;
-                }
-                if(!p.overwrite)
-                {
-                    const u32x2 old = *reinterpret_cast<const u32x2 *>(ptr);
-                    v[0] += T::to_float((uint16_t)(old[0] & 0xffffu));
-                    v[1] += T::to_float((uint16_t)(old[0] >> 16));
-                    v[2] += T::to_float((uint16_t)(old[1] & 0xffffu));
-                    v[3] += T::to_float((uint16_t)(old[1] >> 16));
-                }
-                u32x2 out;
-                out[0] = T::pack2(v[0], v[1]);
-                out[1] = T::pack2(v[2], v[3]);
-                *reinterpret_cast<u32x2 *>(ptr) = out;
-            }
-        }
-    };
+    // ---- dK (+)= scale dk, dV (+)= dv (every wavefront is done with the tiles in LDS) ---
+    __syncthreads();
+    const int row_first = k_row0 + wave_u * 32;
+    char *xch = wave_u == 0 ? lds_q0 : wave_u == 1 ? lds_q1 : wave_u == 2 ? lds_g0 : lds_g1;
+    const int64_t first_byte = row_elem(row_first, true) * RB;
     if(DO_DK)
     {
-        store(dK_own, dk, p.scale);
+        bwd_store_rows<T, HEAD>(xch, static_cast<char *>(dK_own) + first_byte, k_seq - row_first,
+                dk, p.scale, !p.overwrite);
     }
     if(DO_DV)
     {
-        store(dV_own, dv, 1.0f);
+        bwd_store_rows<T, HEAD>(xch, static_cast<char *>(dV_own) + first_byte, k_seq - row_first,
+                dv, 1.0f, !p.overwrite);
     }
 }
 
@@ -2096,6 +2225,37 @@ void sdpa_bwd_kernel(const std::conditional_t<GRID, BwdGridParams, BwdParams> p,
 #endif
 }
 
+static BwdPreludeParams prelude_params(const BwdParams &p, int64_t q_tile, int n_q_tiles)
+{
+    BwdPreludeParams pre = {};
+    pre.q_seq = p.q_seq;
+    pre.q_tile = q_tile;
+    pre.mask_ld = p.mask_ld;
+    pre.D = p.D;
+    pre.mask = p.mask;
+    pre.k_seq = (int32_t)p.k_seq;
+    pre.batch = p.batch;
+    pre.n_q_tiles = n_q_tiles;
+    return pre;
+}
+
+template<typename T, int HEAD, int MODE>
+static int launch_prelude(hipStream_t stream, BwdPreludeParams &pre, int n_tiles)
+{
+    constexpr int ROWS = 256 / (HEAD / 8) * kRowdotRows;
+    const int64_t rows = (int64_t)pre.batch * (pre.q_tile < pre.q_seq ? pre.q_tile : pre.q_seq);
+    const int64_t per_tile = (rows + ROWS - 1) / ROWS;
+    const int64_t n_wgs = pre.n_class_wgs + per_tile * n_tiles;
+    if(per_tile > 0x7fffffff || n_wgs > 0x7fffffff)
+    {
+        return NNTILE_HIP_EINVAL;
+    }
+    pre.wgs_per_tile = (int32_t)per_tile;
+    hipLaunchKernelGGL((sdpa_bwd_prelude_kernel<T, HEAD, MODE == NNTILE_HIP_MASK_CAUSAL
+                ? NNTILE_HIP_MASK_NONE : MODE>), dim3((unsigned)n_wgs), dim3(256), 0, stream, pre);
+    return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+}
+
 template<typename T, int HEAD, int MODE>
 static int launch_bwd_mode(hipStream_t stream, const BwdParams &p)
 {
@@ -2108,25 +2268,25 @@ static int launch_bwd_mode(hipStream_t stream, const BwdParams &p)
     {
         return NNTILE_HIP_EINVAL;
     }
+    BwdPreludeParams pre = prelude_params(p, p.q_seq, 1);
+    pre.dA[0] = p.dA;
+    pre.A[0] = p.A;
     if((MODE == NNTILE_HIP_MASK_ADDITIVE || MODE == NNTILE_HIP_MASK_BOOL)
             && p.mask_class != nullptr)
     {
+        pre.table = const_cast<uint8_t *>(p.mask_class);
+        pre.class_ld = p.class_ld;
         const int64_t n_cls = ((p.q_seq + kBwdStep - 1) / kBwdStep) * p.class_ld;
-        hipLaunchKernelGGL((sdpa_bwd_mask_classes_kernel<T, MODE>), dim3((unsigned)n_cls),
-                dim3(256), 0, stream, p.mask, p.mask_ld, (int)p.q_seq, (int)p.k_seq,
-                const_cast<uint8_t *>(p.mask_class), p.class_ld);
-        if(hipGetLastError() != hipSuccess)
+        if(n_cls > 0x3fffffff)
         {
-            return NNTILE_HIP_ELAUNCH;
+            return NNTILE_HIP_EINVAL;
         }
+        pre.n_class_wgs = (int32_t)n_cls;
     }
-    const int64_t rows = (int64_t)p.batch * p.q_seq;
-    hipLaunchKernelGGL((sdpa_bwd_rowdot_kernel<T, HEAD>),
-            dim3((unsigned)((rows * (HEAD / 8) + 255) / 256)), dim3(256), 0, stream, p.dA, p.A,
-            p.D, rows);
-    if(hipGetLastError() != hipSuccess)
+    const int pre_rc = launch_prelude<T, HEAD, MODE>(stream, pre, 1);
+    if(pre_rc != NNTILE_HIP_OK)
     {
-        return NNTILE_HIP_ELAUNCH;
+        return pre_rc;
     }
     if constexpr(kBwdFusedKeys<HEAD, MODE>)
     {
@@ -2163,22 +2323,16 @@ static int launch_bwd_grid_mode(hipStream_t stream, const BwdGridParams &p,
     {
         return NNTILE_HIP_EINVAL;
     }
-    for(int s = 0; s < p.n_slabs; ++s)
+    BwdPreludeParams pre = prelude_params(p, p.q_tile, n_q_tiles);
+    for(int t = 0; t < p.n_slabs * n_q_tiles; ++t)
     {
-        for(int t = 0; t < n_q_tiles; ++t)
-        {
-            const int64_t t0 = (int64_t)t * p.q_tile;
-            const int64_t rows = (int64_t)p.batch
-                * (p.q_tile < p.q_seq - t0 ? p.q_tile : p.q_seq - t0);
-            hipLaunchKernelGGL((sdpa_bwd_rowdot_kernel<T, HEAD>),
-                    dim3((unsigned)((rows * (HEAD / 8) + 255) / 256)), dim3(256), 0, stream,
-                    p.dAt[s * n_q_tiles + t], A_tiles[s * n_q_tiles + t],
-                    p.D + (int64_t)s * p.q_seq * p.batch + (int64_t)p.batch * t0, rows);
-            if(hipGetLastError() != hipSuccess)
-            {
-                return NNTILE_HIP_ELAUNCH;
-            }
-        }
+        pre.dA[t] = p.dAt[t];
+        pre.A[t] = A_tiles[t];
+    }
+    const int pre_rc = launch_prelude<T, HEAD, MODE>(stream, pre, p.n_slabs * n_q_tiles);
+    if(pre_rc != NNTILE_HIP_OK)
+    {
+        return pre_rc;
     }
     if constexpr(kBwdFusedKeys<HEAD, MODE>)
     {
