@@ -25,10 +25,11 @@ int launch_bwd_grid_16bit(hipStream_t stream, const BwdGridParams &p,
 size_t decode_workspace_bytes(int units, int n_splits, int rows, int head);
 size_t decode_partial_o_bytes(int units, int n_splits, int rows, int head);
 size_t decode_partial_ml_bytes(int units, int n_splits, int rows);
-int launch_decode_fp32(hipStream_t stream, const DecodeParams &p, int head, int mode);
+int launch_decode_fp32(hipStream_t stream, DecodeParams &p, int head, int mode);
 int decode_fp32_steps(int64_t k_seq);
-int decode_fp32_choose_splits(int units, int n_steps);
+int decode_fp32_choose_splits(int units, int n_steps, int head);
 size_t decode_fp32_workspace_bytes(int units, int n_splits, int rows, int head);
+size_t decode_fp32_partial_bytes(int units, int n_splits, int rows, int head);
 
 struct F32Store;
 struct Bf16Store;
@@ -555,14 +556,13 @@ static int decode_call(DType dt, void *stream, const nntile_hip_sdpa_tile_args *
         : launch_decode_16bit<Fp16>(s, p, (int)a->head, a->mask_mode);
 }
 
-// The fp32 twin: steps of 32 keys, partials in fp32, the merge always a second
-// launch.
+// The fp32 twin: steps of 32 keys, partials in fp32.
 static void decode_fp32_geometry(const nntile_hip_sdpa_tile_args *a, int &units,
         int &n_steps, int &splits, int &rows)
 {
     units = (int)(a->batch / a->kv_group);
     n_steps = decode_fp32_steps(a->k_seq);
-    splits = decode_fp32_choose_splits(units, n_steps);
+    splits = decode_fp32_choose_splits(units, n_steps, (int)a->head);
     rows = (int)(a->q_seq * a->kv_group);
 }
 
@@ -617,6 +617,10 @@ static int decode_fp32_call(void *stream, const nntile_hip_sdpa_tile_args *a,
     p.A = a->A;
     p.part_o = static_cast<float *>(workspace);
     p.part_ml = p.part_o + (size_t)units * splits * rows * a->head;
+    p.sync = reinterpret_cast<unsigned long long *>(static_cast<char *>(workspace)
+            + decode_fp32_partial_bytes(units, splits, rows, (int)a->head));
+    p.fused = (a->flags & NNTILE_HIP_SDPA_DECODE_SEPARATE_MERGE) ? 0 : 1;
+    p.fenced = (a->flags & NNTILE_HIP_SDPA_DECODE_FENCED) ? 1 : 0;
     p.n_batch = (int32_t)a->n_batch;
     p.kv_group = (int32_t)a->kv_group;
     p.n_head_kv = (int32_t)(units / a->n_batch);

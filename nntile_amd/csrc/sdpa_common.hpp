@@ -111,6 +111,7 @@ struct DecodeParams
     unsigned long long spin_limit;  // longest wait for a flag, in 100 MHz ticks
     int32_t fused, fenced;
     int32_t n_main, merge_blocks_per_unit, sync_stride;
+    int32_t units8;     // units rounded up to whole rounds of the XCDs
     // The append riding in the launch (n_new > 0): K and V are caches whose
     // rows [k_seq - n_new, k_seq) of every entry have not been written yet;
     // they are k_new / v_new ([entry][n_new][head]).  The main workgroups read

@@ -26,7 +26,7 @@
 #include <random>
 #include <type_traits>
 
-#include "sdpa_common.hpp"
+#include "sdpa_decode_merge.hpp"
 
 namespace nntile_hip
 {
@@ -37,7 +37,10 @@ namespace nntile_hip
 #endif
 
 constexpr int kDecThreads = 256;  // 4 wavefronts x 16 query rows
-constexpr int kDecodeCUs = 256;   // MI355X
+constexpr int kDecodeCUs = 256;   // MI355X, 8 XCDs
+// K and V bytes by which the XCDs' shares may differ, taken eight times, before
+// the units are spread over the XCDs regardless of where they are merged
+constexpr int64_t kDecodeUnevenBytes = 20 << 20;
 // Ring stages and workgroups per CU the kernel is built for
 #ifndef NNTILE_DEC_STAGES
 #define NNTILE_DEC_STAGES 2
@@ -111,36 +114,9 @@ template<int N> __device__ __forceinline__ void wait_vmcnt()
     asm volatile("" ::: "memory");
 }
 
-// Loads that are served by the L2 (never by a CU's own cache): what one
-// workgroup reads of memory another workgroup of the same launch has written.
-template<bool COH>
-__device__ __forceinline__ unsigned long long ld64(const void *ptr)
-{
-    if(COH)
-    {
-        return __hip_atomic_load(
-                const_cast<unsigned long long *>(static_cast<const unsigned long long *>(ptr)),
-                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    return *static_cast<const unsigned long long *>(ptr);
-}
-
-template<bool COH>
-__device__ __forceinline__ float ld32f(const float *ptr)
-{
-    if(COH)
-    {
-        return __hip_atomic_load(const_cast<float *>(ptr), __ATOMIC_RELAXED,
-                __HIP_MEMORY_SCOPE_AGENT);
-    }
-    return *ptr;
-}
-
-// The XCD this wavefront runs on (hardware register XCC_ID, bits 3:0).
-__device__ __forceinline__ int xcc_id()
-{
-    return (int)(__builtin_amdgcn_s_getreg((31 << 11) | 20) & 15u);
-}
+// The fp32 kernels' counters of the same two kinds (a device symbol belongs to
+// the file that defines it).
+long long decode_fp32_sync_count(bool misplaced);
 
 // Merge workgroups of the fused form that gave up waiting for a flag (they
 // leave their rows untouched); read with nntile_hip_debug_decode_sync_timeouts.
@@ -224,29 +200,92 @@ __device__ __forceinline__ void decode_merge_row(const DecodeParams &p, int unit
     }
     else
     {
-        for(int s0 = 0; s0 < p.n_splits; s0 += 8)
+        // More splits than that: the row's threads share out the maxima and
+        // sums, one or a few each, so that these take one round trip whatever
+        // their number, and the values follow 16 loads at a time, the first of
+        // them beside the maxima.  (Eight at a time for maxima and values in
+        // turn, 64 splits took 16 round trips; a step of one sequence over
+        // 4000 keys 13.0 us.)
+        constexpr int TPR = HEAD / 4;               // threads of the row, neighbours in a wavefront
+        constexpr int NC = 64 / TPR;                // splits per thread, at most 64 in all
+        const int t = d4 / 4;
+        f32x2 ml[NC];
+#pragma unroll
+        for(int i = 0; i < NC; ++i)
         {
-            float m[8];
+            ml[i] = __builtin_bit_cast(f32x2, ld64<COH>(p.part_ml
+                        + 2 * (base + (int64_t)min(t + i * TPR, last_split) * p.rows)));
+        }
+        float w[NC];
+        f32x4 v[16];
+        auto load16 = [&](int s0)
+        {
 #pragma unroll
-            for(int j = 0; j < 8; ++j)
+            for(int j = 0; j < 16; ++j)
             {
-                const int sidx = min(s0 + j, last_split);
-                m[j] = ld32f<COH>(p.part_ml + 2 * (base + (int64_t)sidx * p.rows));
+                const int64_t prow = base + (int64_t)min(s0 + j, last_split) * p.rows;
+#if NNTILE_DEC_PART16
+                const u32x2 raw = __builtin_bit_cast(u32x2, ld64<COH>(
+                        reinterpret_cast<const uint16_t *>(p.part_o) + prow * HEAD + d4));
+                v[j] = f32x4{T::to_float((uint16_t)(raw[0] & 0xffffu)),
+                    T::to_float((uint16_t)(raw[0] >> 16)), T::to_float((uint16_t)(raw[1] & 0xffffu)),
+                    T::to_float((uint16_t)(raw[1] >> 16))};
+#else
+                v[j] = *reinterpret_cast<const f32x4 *>(p.part_o + prow * HEAD + d4);
+#endif
             }
+        };
+        load16(0);
 #pragma unroll
-            for(int j = 0; j < 8; ++j)
-            {
-                top = fmaxf(top, m[j]);
-            }
+        for(int i = 0; i < NC; ++i)
+        {
+            ml[i][0] = t + i * TPR <= last_split ? ml[i][0] : neg_inf();
+            top = fmaxf(top, ml[i][0]);
+        }
+#pragma unroll
+        for(int o = TPR / 2; o >= 1; o >>= 1)
+        {
+            top = fmaxf(top, __shfl_xor(top, o, TPR));
         }
         if(top != neg_inf())
         {
-            for(int s0 = 0; s0 < p.n_splits; s0 += 8)
+#pragma unroll
+            for(int i = 0; i < NC; ++i)
             {
-                f32x2 ml[8];
-                f32x4 v[8];
-                load8(s0, ml, v);
-                add8(s0, ml, v);
+                const float e = ml[i][0] != neg_inf() ? __expf(ml[i][0] - top) : 0.0f;
+#if NNTILE_DEC_PART16
+                w[i] = e * ml[i][1];
+                l += w[i];
+#else
+                w[i] = e;
+                l += e * ml[i][1];
+#endif
+            }
+#pragma unroll
+            for(int o = TPR / 2; o >= 1; o >>= 1)
+            {
+                l += __shfl_xor(l, o, TPR);
+            }
+            for(int s0 = 0;;)
+            {
+                float ws = w[0];
+#pragma unroll
+                for(int i = 1; i < NC; ++i)
+                {
+                    ws = s0 / TPR == i ? w[i] : ws;
+                }
+#pragma unroll
+                for(int j = 0; j < 16; ++j)
+                {
+                    // (past the last split: weight 0, a value that exists)
+                    acc += __shfl(ws, s0 % TPR + j, TPR) * v[j];
+                }
+                s0 += 16;
+                if(s0 >= p.n_splits)
+                {
+                    break;
+                }
+                load16(s0);
             }
         }
     }
@@ -287,84 +326,6 @@ __device__ __forceinline__ void decode_merge_row(const DecodeParams &p, int unit
     if(d4 == 0)
     {
         p.lse[row] = lse_out;
-    }
-}
-
-// A merge workgroup of the fused form: block `idx` behind the main workgroups.
-// It is dispatched when main workgroups have left (the hardware starts the
-// workgroups of a launch in index order, and the main ones never wait for
-// anything), waits until every split of its unit has raised its flag, merges
-// its rows and lowers the flags again.
-//
-// Placement: the workgroups of one launch go round the 8 XCDs in index order,
-// so the main workgroups of a unit and its merge workgroups, whose indices
-// are equal modulo 8 by construction, share an XCD and its L2: partials
-// written by plain stores are there for plain loads once the writer's stores
-// are acknowledged, no cache has to be written back or invalidated.  Where
-// the round starts is not the launch's to say (XCD 0 on a fresh queue, another
-// one after a graph launch or on a second stream - but one start per launch,
-// also with several queues dispatching at once), so nothing here assumes a
-// particular XCD: every main workgroup puts the number of the XCD it ran on
-// (hardware register XCC_ID) into its flag and the merge workgroup compares
-// it with its own.  A difference - never seen - is counted and the rows are
-// left alone rather than merged from data that may not have arrived.  With
-// p.fenced both sides use device-scope fences instead and placement is not
-// looked at (for comparison: the fences write back and invalidate whole L2s).
-template<typename T, int HEAD>
-__device__ __forceinline__ void decode_merge_workgroup(const DecodeParams &p, int idx)
-{
-    constexpr int TPR = HEAD / 4;               // threads per row
-    constexpr int ROWS_PER_WG = 256 / TPR;
-    const int tid = threadIdx.x;
-    const int x = idx & 7, j = idx >> 3;
-    const int unit = (j / p.merge_blocks_per_unit) * 8 + x;
-    const int rb = j % p.merge_blocks_per_unit;
-    unsigned long long *flags = p.sync + (int64_t)unit * p.sync_stride + 1 + rb * p.n_splits;
-    int bad = 0;
-    if(tid < p.n_splits)
-    {
-        // (the tag's low four bits are clear: the flag carries the writer's XCD there)
-        const unsigned long long t0 = wall_clock64();
-        unsigned long long seen;
-        while(((seen = ld64<true>(flags + tid)) & ~15ull) != p.tag)
-        {
-            __builtin_amdgcn_s_sleep(4);
-            if(wall_clock64() - t0 > p.spin_limit)
-            {
-                bad = 1;
-                break;
-            }
-        }
-        if(!bad && !p.fenced && (int)(seen & 15ull) != xcc_id())
-        {
-            bad = 2;
-        }
-    }
-    bad = __syncthreads_or(bad);
-    if(bad)
-    {
-        if(tid == 0)
-        {
-            atomicAdd((bad & 1) ? &decode_sync_timeouts : &decode_sync_misplaced, 1u);
-        }
-        return;
-    }
-    if(p.fenced)
-    {
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    }
-    const int rr = rb * ROWS_PER_WG + tid / TPR;
-    if(rr < p.rows)
-    {
-        decode_merge_row<T, HEAD, true>(p, unit, rr, (tid % TPR) * 4);
-    }
-    // every partial of these rows has been read: the flags go down for the
-    // next call on this workspace (a replay of a captured graph has this
-    // call's tag again)
-    __syncthreads();
-    if(tid < p.n_splits)
-    {
-        __hip_atomic_store(flags + tid, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -414,7 +375,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
     // workgroups, then (append in the launch) one copying workgroup per unit.
     if((int)blockIdx.x >= p.n_main)
     {
-        const int n_merge = p.fused ? p.n_batch * p.n_head_kv * p.merge_blocks_per_unit : 0;
+        const int n_merge = p.fused ? p.units8 * p.merge_blocks_per_unit : 0;
         const int behind = (int)blockIdx.x - p.n_main;
         if(behind >= n_merge)
         {
@@ -439,7 +400,11 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
         if constexpr(!DIRECT)
         {
             DEC_STAMP(5);
-            decode_merge_workgroup<T, HEAD>(p, behind);
+            decode_merge_workgroup<HEAD>(p, behind, &decode_sync_timeouts, &decode_sync_misplaced,
+                    [&](int unit, int rr, int d4)
+                    {
+                        decode_merge_row<T, HEAD, true>(p, unit, rr, d4);
+                    });
 #ifdef NNTILE_DEC_TRACE
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             DEC_STAMP(6);
@@ -454,24 +419,10 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
     const int col = lane & 15;       // row (query) within the wavefront
     const int quad = lane >> 4;      // 0..3
 
-    // Workgroups are dealt round-robin to the 8 XCDs.  All key splits of a
-    // unit go to one XCD, and so do the workgroups of the merge kernel that
-    // read the unit's partials: the partials then stay within one L2
-    // (cfg4: 50.6 -> 50.0 us per step).
     int split, unit;
+    if(!decode_place(p, unit, split))
     {
-        const int units = p.n_batch * p.n_head_kv;
-        if(units % 8 == 0)
-        {
-            const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
-            unit = (j / p.n_splits) * 8 + x;
-            split = j % p.n_splits;
-        }
-        else
-        {
-            split = blockIdx.x % p.n_splits;
-            unit = blockIdx.x / p.n_splits;        // nb + n_batch*hkv
-        }
+        return;
     }
     const int nb = unit % p.n_batch;
     const int hkv = unit / p.n_batch;
@@ -620,7 +571,10 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
     // Each workgroup therefore starts at its own rotation of its range (the
     // online softmax does not care about the order of the steps).
     const int n_local = step_hi - step_lo;
-    const int rot = n_local > 0 ? (int)((blockIdx.x * 7u + (blockIdx.x >> 3)) % (unsigned)n_local) : 0;
+    // (from the place the units' layout in eights gives the workgroup, whichever
+    // layout this launch has: the order of the steps is part of the result)
+    const unsigned place = (unsigned)(((unit >> 3) * p.n_splits + split) * 8 + (unit & 7));
+    const int rot = n_local > 0 ? (int)((place * 7u + (place >> 3)) % (unsigned)n_local) : 0;
     auto actual = [&](int i) -> int
     {
         const int j = i + rot;
@@ -1017,21 +971,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
 #endif
     if(p.fused)
     {
-        // The partial is complete in this XCD's L2 once every wavefront's
-        // stores have been acknowledged (the barrier's release waits for
-        // them); then one flag per merge workgroup of the unit goes up, with
-        // the number of this XCD in its low bits.
-        __syncthreads();
-        if(p.fenced)
-        {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        }
-        if(tid < p.merge_blocks_per_unit)
-        {
-            __hip_atomic_store(p.sync + (int64_t)unit * p.sync_stride + 1 + tid * p.n_splits + split,
-                    p.tag | (unsigned long long)xcc_id(), __ATOMIC_RELAXED,
-                    __HIP_MEMORY_SCOPE_AGENT);
-        }
+        decode_raise_flags(p, unit, split);
     }
 }
 
@@ -1095,7 +1035,7 @@ int decode_sync_stride(int n_splits, int rows, int head)
 // behind by anything else is unlikely to hold: a random upper half fixed at
 // load time, a counter below it; the low four bits stay clear (a flag holds
 // the tag plus the number of the XCD that raised it).
-static unsigned long long next_decode_tag()
+unsigned long long next_decode_tag()
 {
     static const unsigned long long salt = []
     {
@@ -1111,6 +1051,11 @@ static unsigned long long next_decode_tag()
 // (2 s unless a test sets it).
 static std::atomic<unsigned long long> decode_spin_limit{200000000ull};
 
+unsigned long long decode_spin_limit_now()
+{
+    return decode_spin_limit.load(std::memory_order_relaxed);
+}
+
 extern "C" unsigned long long nntile_hip_debug_decode_spin_limit(unsigned long long ticks)
 {
     return decode_spin_limit.exchange(ticks);
@@ -1124,7 +1069,8 @@ extern "C" long long nntile_hip_debug_decode_sync_misplaced(void)
         (void)hipGetLastError();
         return -1;
     }
-    return (long long)n;
+    const long long more = decode_fp32_sync_count(true);
+    return more < 0 ? more : (long long)n + more;
 }
 
 extern "C" long long nntile_hip_debug_decode_sync_timeouts(void)
@@ -1134,7 +1080,8 @@ extern "C" long long nntile_hip_debug_decode_sync_timeouts(void)
     {
         return -1;
     }
-    return (long long)n;
+    const long long more = decode_fp32_sync_count(false);
+    return more < 0 ? more : (long long)n + more;
 }
 
 template<typename T, int HEAD, int MODE, int STAGES>
@@ -1156,20 +1103,26 @@ static int launch_decode_stages(hipStream_t stream, DecodeParams &p, int mode)
     const int units = p.n_batch * p.n_head_kv;
     constexpr int rows_per_wg = 256 / (HEAD / 4);
     const int merge_blocks = (p.rows + rows_per_wg - 1) / rows_per_wg;
-    // The merge rides in the main launch when the caller allows it, the unit
-    // has several splits and the units map onto the XCDs (8 at a time).
-    p.fused = (p.fused && p.n_splits > 1 && units % 8 == 0 && p.sync != nullptr
-            && NNTILE_DEC_PART16) ? 1 : 0;
-    p.n_main = units * p.n_splits;
+    // The merge rides in the main launch when the caller allows it and the
+    // unit has several splits.  The grid then gives the units out eight at a
+    // time so that a unit's workgroups share an XCD; units that are no multiple
+    // of eight leave places that end at once (12 units, 12 steps: 8.8 us with
+    // the merge as a second launch, 7.5 so) - and leave XCDs with less to do,
+    // which a second launch costs less than once the difference is worth more
+    // than 3 us of the stream (20 units of 15 000 keys: 31.9 against 39.7 us).
+    const int units8 = (units + 7) / 8 * 8;
+    p.fused = (p.fused && p.n_splits > 1 && !decode_uneven_units(units, p.k_seq, HEAD * 4) && p.sync != nullptr && NNTILE_DEC_PART16) ? 1 : 0;
+    p.units8 = (p.fused || units == units8) ? units8 : 0;
+    p.n_main = (p.units8 != 0 ? units8 : units) * p.n_splits;
     p.merge_blocks_per_unit = merge_blocks;
     p.sync_stride = decode_sync_stride(p.n_splits, p.rows, HEAD);
     if(p.fused)
     {
         p.tag = next_decode_tag();
-        p.spin_limit = decode_spin_limit.load(std::memory_order_relaxed);
+        p.spin_limit = decode_spin_limit_now();
     }
     p.n_append = p.n_new > 0 ? units : 0;
-    const dim3 grid((unsigned)(p.n_main + (p.fused ? units * merge_blocks : 0) + p.n_append));
+    const dim3 grid((unsigned)(p.n_main + (p.fused ? units8 * merge_blocks : 0) + p.n_append));
     switch(mode)
     {
         case NNTILE_HIP_MASK_ADDITIVE:
@@ -1209,14 +1162,38 @@ static int launch_decode_head(hipStream_t stream, DecodeParams &p, int mode)
     return launch_decode_stages<T, HEAD, NNTILE_DEC_STAGES>(stream, p, mode);
 }
 
+// places: workgroups that the chip holds at once.  Units go to the XCDs round robin, and no XCD gets more
+// workgroups than it has places for, or the last ones would run alone (36
+// units of 8000 keys as 15 splits each 35.6 us, as 12 splits 29).
+int decode_splits_by_units(int units, int places)
+{
+    return units > kDecodeCUs ? (places + units - 1) / units : places / 8 / ((units + 7) / 8);
+}
+
+bool decode_uneven_units(int units, int64_t k_seq, int64_t row_bytes)
+{
+    const int left = (units + 7) / 8 * 8 - units;
+    return left * k_seq * row_bytes > kDecodeUnevenBytes;
+}
+
 // Number of key splits per unit: two workgroups per CU when the units allow
 // it, never more than one split per key step.  Fewer splits mean fewer
-// partials to write and merge.
+// partials to write and merge: handing the partials over costs a launch 2 us,
+// a key step about 1 (while nothing but its own latency counts), so up to three
+// steps stay in one workgroup (two steps: 6.8 -> 5.6 us a call, three 6.9 ->
+// 6.5, four would be 6.6 -> 7.3), and from nine on a split takes two at least
+// (8 units of 63 steps: 64 splits 13.0 us, 32 splits 10.3).
 int decode_choose_splits(int units, int n_steps)
 {
-    int splits = (NNTILE_DEC_WGS_PER_CU * kDecodeCUs + units - 1) / units;
+    constexpr int kDirectSteps = 3, kSingleSteps = 8;
+    if(n_steps <= kDirectSteps)
+    {
+        return 1;
+    }
+    int splits = decode_splits_by_units(units, NNTILE_DEC_WGS_PER_CU * kDecodeCUs);
+    const int most = n_steps <= kSingleSteps ? n_steps : (n_steps + 1) / 2;
     splits = splits < 1 ? 1 : splits;
-    splits = splits > n_steps ? n_steps : splits;
+    splits = splits > most ? most : splits;
     splits = splits > 64 ? 64 : splits;
     return splits;
 }

@@ -16,9 +16,11 @@
 //    keys) is the B operand layout of the second product, so the
 //    probabilities never leave the registers;
 //  - partial (max, sum) and the normalised partial output of every split go to
-//    the workspace in fp32; a second small kernel merges the splits and folds
-//    the result into (lse, A) by the rule of accumulate_attn_output
-//    (src/kernel/accumulate_attn_output/cpu.cc:38-115).
+//    the workspace in fp32; merge workgroups at the end of the same grid (or,
+//    where the units' shares of the XCDs differ too much, a second small
+//    kernel) merge the splits and fold the result into (lse, A) by the rule of
+//    accumulate_attn_output (src/kernel/accumulate_attn_output/cpu.cc:38-115);
+//    a unit with a single split writes (lse, A) itself.
 //
 // Bound: at cfg4's shape in fp32 (541 MB, 17.2 GFLOP) the fp32 matrix rate
 // (157.3 TFLOP/s: 110 us) and the HBM stream (98 us at 5.5 TB/s) are about
@@ -27,7 +29,7 @@
 #include <stdint.h>
 #include <type_traits>
 #include "../../include/nntile_hip_sdpa.h"
-#include "sdpa_common.hpp"
+#include "sdpa_decode_merge.hpp"
 
 namespace nntile_hip
 {
@@ -53,7 +55,146 @@ __device__ __forceinline__ int64_t f32dec_row(const DecodeParams &p, int unit, i
     return qb * p.q_seq + tok;
 }
 
-template<int HEAD, int MODE>
+// Merge workgroups that gave up waiting for a flag, and that found a split of
+// their unit on another XCD (they leave their rows untouched).
+__device__ unsigned int decode_fp32_sync_timeouts;
+__device__ unsigned int decode_fp32_sync_misplaced;
+
+long long decode_fp32_sync_count(bool misplaced)
+{
+    unsigned int n = 0;
+    const hipError_t rc = misplaced
+        ? hipMemcpyFromSymbol(&n, HIP_SYMBOL(decode_fp32_sync_misplaced), sizeof(n))
+        : hipMemcpyFromSymbol(&n, HIP_SYMBOL(decode_fp32_sync_timeouts), sizeof(n));
+    if(rc != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return -1;
+    }
+    return (long long)n;
+}
+
+// Merge the split partials of row rr of a unit and fold the result into
+// (lse, A).  The calling thread handles head values d4 .. d4+3.  COH: the
+// partials were written by other workgroups of this launch.
+template<int HEAD, bool COH>
+__device__ __forceinline__ void f32dec_merge_row(const DecodeParams &p, int unit, int rr, int d4)
+{
+    const int64_t base = (int64_t)unit * p.n_splits * p.rows + rr;
+    const int64_t row = f32dec_row(p, unit, rr);
+    float *Adst = static_cast<float *>(p.A) + row * HEAD + d4;
+    typedef __attribute__((ext_vector_type(2))) float f32x2;
+    // The row's threads share out the maxima and sums, one or a few each, so
+    // that these take one round trip, and the values follow eight loads at a
+    // time, the first of them beside the maxima.
+    constexpr int TPR = HEAD / 4;               // threads of the row, neighbours in a wavefront
+    constexpr int NC = 64 / TPR;                // splits per thread, at most 64 in all
+    const int t = d4 / 4, last_split = p.n_splits - 1;
+    f32x2 ml[NC];
+#pragma unroll
+    for(int i = 0; i < NC; ++i)
+    {
+        ml[i] = __builtin_bit_cast(f32x2, ld64<COH>(p.part_ml
+                    + 2 * (base + (int64_t)min(t + i * TPR, last_split) * p.rows)));
+    }
+    f32x4 v8[8];
+    auto load8 = [&](int s0)
+    {
+#pragma unroll
+        for(int j = 0; j < 8; ++j)
+        {
+            // (splits past the last re-read the last one and get weight 0)
+            const float *src = p.part_o
+                + (base + (int64_t)min(s0 + j, last_split) * p.rows) * HEAD + d4;
+            const f32x2 lo = __builtin_bit_cast(f32x2, ld64<COH>(src)),
+                hi = __builtin_bit_cast(f32x2, ld64<COH>(src + 2));
+            v8[j] = f32x4{lo[0], lo[1], hi[0], hi[1]};
+        }
+    };
+    load8(0);
+    float top = neg_inf(), w[NC];
+#pragma unroll
+    for(int i = 0; i < NC; ++i)
+    {
+        const bool there = t + i * TPR <= last_split && ml[i][0] != neg_inf() && ml[i][1] > 0.0f;
+        w[i] = there ? ml[i][0] + __logf(ml[i][1]) : neg_inf();     // the split's logsumexp
+        top = fmaxf(top, w[i]);
+    }
+#pragma unroll
+    for(int o = TPR / 2; o >= 1; o >>= 1)
+    {
+        top = fmaxf(top, __shfl_xor(top, o, TPR));
+    }
+    float wsum = 0.0f;
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    if(top != neg_inf())
+    {
+#pragma unroll
+        for(int i = 0; i < NC; ++i)
+        {
+            w[i] = w[i] == neg_inf() ? 0.0f : __expf(w[i] - top);
+            wsum += w[i];
+        }
+#pragma unroll
+        for(int o = TPR / 2; o >= 1; o >>= 1)
+        {
+            wsum += __shfl_xor(wsum, o, TPR);
+        }
+        for(int s0 = 0;;)
+        {
+            float ws = w[0];
+#pragma unroll
+            for(int i = 1; i < NC; ++i)
+            {
+                ws = s0 / TPR == i ? w[i] : ws;
+            }
+#pragma unroll
+            for(int j = 0; j < 8; ++j)
+            {
+                acc += __shfl(ws, s0 % TPR + j, TPR) * v8[j];
+            }
+            s0 += 8;
+            if(s0 >= p.n_splits)
+            {
+                break;
+            }
+            load8(s0);
+        }
+    }
+    if(top == neg_inf())
+    {
+        // no visible key at all: leave lse and A untouched, or write the
+        // empty row when the running pair is being overwritten
+        if(p.overwrite)
+        {
+            *reinterpret_cast<f32x4 *>(Adst) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if(d4 == 0)
+            {
+                p.lse[row] = neg_inf();
+            }
+        }
+        return;
+    }
+    const float lse_new = top + __logf(wsum);
+    const float lse_old = p.overwrite ? neg_inf() : p.lse[row];
+    float w_old, w_new, lse_out;
+    merge_weights(lse_old, lse_new, w_old, w_new, lse_out);
+    f32x4 v = acc * (w_new / wsum);
+    if(w_old != 0.0f)
+    {
+        v += w_old * *reinterpret_cast<const f32x4 *>(Adst);
+    }
+    *reinterpret_cast<f32x4 *>(Adst) = v;
+    // The threads of a row sit in one wavefront (TPR <= 32 divides 64) and
+    // run in lock step: all of them have read lse_old by now.
+    if(d4 == 0)
+    {
+        p.lse[row] = lse_out;
+    }
+}
+
+// DIRECT: the unit has one key split: no partials, (lse, A) are written here.
+template<int HEAD, int MODE, bool DIRECT>
 __global__ __launch_bounds__(kDecF32Threads, 2)
 void sdpa_decode_fp32_kernel(const DecodeParams p)
 {
@@ -81,16 +222,29 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
     const int col = lane & 15;       // row (query) within the wavefront; key within a block for operand reads
     const int quad = lane >> 4;      // 0..3
 
-    // Behind the units x splits attention workgroups the grid holds, when rows
-    // are being appended to the caches by this call, one copying workgroup per
-    // unit: the new rows into the caches, 16 bytes a thread and piece.  Nobody
+    // Behind the attention workgroups the grid holds the merge workgroups (merge
+    // in the launch) and, when rows are being appended to the caches by this
+    // call, one copying workgroup per unit: the new rows into the caches, 16 bytes a thread and piece.  Nobody
     // in this launch reads them there (the attention takes them from k_new /
     // v_new), so there is nothing to wait for or to signal.
     {
-        const int n_main = p.n_batch * p.n_head_kv * p.n_splits;
-        if((int)blockIdx.x >= n_main)
+        if((int)blockIdx.x >= p.n_main)
         {
-            const int unit_a = (int)blockIdx.x - n_main;
+            const int n_merge = p.fused ? p.units8 * p.merge_blocks_per_unit : 0;
+            const int behind = (int)blockIdx.x - p.n_main;
+            if(behind < n_merge)
+            {
+                if constexpr(!DIRECT)
+                {
+                    decode_merge_workgroup<HEAD>(p, behind, &decode_fp32_sync_timeouts,
+                            &decode_fp32_sync_misplaced, [&](int unit, int rr, int d4)
+                            {
+                                f32dec_merge_row<HEAD, true>(p, unit, rr, d4);
+                            });
+                }
+                return;
+            }
+            const int unit_a = behind - n_merge;
             const int64_t filled = p.k_seq - p.n_new;
             const int n16 = p.n_new * (RB / 16);
             for(int t = tid; t < 2 * n16; t += kDecF32Threads)
@@ -107,23 +261,10 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
         }
     }
 
-    // Workgroups go round the 8 XCDs in index order: all key splits of a unit
-    // get indices that are equal modulo 8, i.e. one XCD and one L2 for the
-    // unit's K/V (the four wavefronts' query heads read them once).
     int split, unit;
+    if(!decode_place(p, unit, split))
     {
-        const int units = p.n_batch * p.n_head_kv;
-        if(units % 8 == 0)
-        {
-            const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
-            unit = (j / p.n_splits) * 8 + x;
-            split = j % p.n_splits;
-        }
-        else
-        {
-            split = blockIdx.x % p.n_splits;
-            unit = blockIdx.x / p.n_splits;
-        }
+        return;
     }
 
     const int rr = wave * 16 + col;
@@ -430,121 +571,81 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
     // ---- the partial: (max in natural-log units, sum) and the normalised output
     float l_tot = l_run + __shfl_xor(l_run, 16);
     l_tot = sum_across_halves(l_tot);
-    if(!row_ok)
+    const float to_ln = EXPLICIT ? 1.0f : p.scale;
+    const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+    // o[db][r] is head value 16*db + 4*quad + r of row rr
+    if constexpr(DIRECT)
     {
+        if(!row_ok)
+        {
+            return;
+        }
+        const int64_t row = f32dec_row(p, unit, rr);
+        float *dst = static_cast<float *>(p.A) + row * HEAD + 4 * quad;
+        // (no visible key at all: lse and A stay, or the empty row is written)
+        const bool empty = m_run == neg_inf() || !(l_tot > 0.0f);
+        if(empty && !p.overwrite)
+        {
+            return;
+        }
+        float w_old = 0.0f, w_new = 0.0f, lse_out = neg_inf();
+        if(!empty)
+        {
+            merge_weights(p.overwrite ? neg_inf() : p.lse[row], m_run * to_ln + __logf(l_tot), w_old,
+                    w_new, lse_out);
+        }
+#pragma unroll
+        for(int db = 0; db < DBLOCKS; ++db)
+        {
+            f32x4 v = empty ? f32x4{0.0f, 0.0f, 0.0f, 0.0f} : o[db] * (inv * w_new);
+            if(w_old != 0.0f)
+            {
+                v += w_old * *reinterpret_cast<const f32x4 *>(dst + 16 * db);
+            }
+            *reinterpret_cast<f32x4 *>(dst + 16 * db) = v;
+        }
+        // (the four lanes of a row sit in one wavefront and run in lock step:
+        // all of them have read the stored value by now)
+        if(quad == 0)
+        {
+            p.lse[row] = lse_out;
+        }
         return;
     }
-    const int64_t prow = ((int64_t)unit * p.n_splits + split) * p.rows + rr;
-    if(quad == 0)
+    if(row_ok)
     {
-        const float to_ln = EXPLICIT ? 1.0f : p.scale;
-        p.part_ml[2 * prow] = (m_run == neg_inf()) ? neg_inf() : m_run * to_ln;
-        p.part_ml[2 * prow + 1] = l_tot;
-    }
-    // o[db][r] is head value 16*db + 4*quad + r of row rr
-    const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    float *dst = p.part_o + prow * HEAD + 4 * quad;
+        const int64_t prow = ((int64_t)unit * p.n_splits + split) * p.rows + rr;
+        if(quad == 0)
+        {
+            p.part_ml[2 * prow] = (m_run == neg_inf()) ? neg_inf() : m_run * to_ln;
+            p.part_ml[2 * prow + 1] = l_tot;
+        }
+        float *dst = p.part_o + prow * HEAD + 4 * quad;
 #pragma unroll
-    for(int db = 0; db < DBLOCKS; ++db)
+        for(int db = 0; db < DBLOCKS; ++db)
+        {
+            *reinterpret_cast<f32x4 *>(dst + 16 * db) = o[db] * inv;
+        }
+    }
+    if(p.fused)
     {
-        *reinterpret_cast<f32x4 *>(dst + 16 * db) = o[db] * inv;
+        decode_raise_flags(p, unit, split);
     }
 }
 
-// Merge the split partials of each row and fold the result into (lse, A).  A
-// thread handles 4 head values of one row; a workgroup of 256 threads handles
-// 1024/HEAD rows.
+// The merge as a launch of its own: a thread handles 4 head values of one row,
+// a workgroup of 256 threads 1024/HEAD rows.
 template<int HEAD>
 __global__ __launch_bounds__(256)
 void sdpa_decode_fp32_reduce_kernel(const DecodeParams p)
 {
     constexpr int TPR = HEAD / 4;               // threads per row
     constexpr int ROWS_PER_WG = 256 / TPR;
-    const int tid = threadIdx.x;
-    const int64_t grow = (int64_t)blockIdx.x * ROWS_PER_WG + tid / TPR;
-    const int64_t total = (int64_t)p.n_batch * p.n_head_kv * p.rows;
-    if(grow >= total)
+    const int64_t grow = (int64_t)blockIdx.x * ROWS_PER_WG + threadIdx.x / TPR;
+    if(grow < (int64_t)p.n_batch * p.n_head_kv * p.rows)
     {
-        return;
-    }
-    const int unit = (int)(grow / p.rows), rr = (int)(grow % p.rows);
-    const int d4 = (tid % TPR) * 4;
-    const int64_t base = (int64_t)unit * p.n_splits * p.rows + rr;
-    // eight splits at a time, all their loads issued before anything is used
-    // (a loop of dependent trips to memory otherwise: 10.5 us for cfg4's shape)
-    const int64_t row = f32dec_row(p, unit, rr);
-    float *Adst = static_cast<float *>(p.A) + row * HEAD + d4;
-    typedef __attribute__((ext_vector_type(2))) float f32x2;
-    float top = neg_inf();
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    float wsum = 0.0f;
-    for(int s0 = 0; s0 < p.n_splits; s0 += 8)
-    {
-        f32x2 ml[8];
-        f32x4 v[8];
-#pragma unroll
-        for(int j = 0; j < 8; ++j)
-        {
-            // (splits past the last re-read the last one and get weight 0)
-            const int64_t prow = base + (int64_t)min(s0 + j, p.n_splits - 1) * p.rows;
-            ml[j] = *reinterpret_cast<const f32x2 *>(p.part_ml + 2 * prow);
-            v[j] = *reinterpret_cast<const f32x4 *>(p.part_o + prow * HEAD + d4);
-        }
-        float lse_s[8];
-        float top8 = top;
-#pragma unroll
-        for(int j = 0; j < 8; ++j)
-        {
-            const bool there = s0 + j < p.n_splits && ml[j][0] != neg_inf() && ml[j][1] > 0.0f;
-            lse_s[j] = there ? ml[j][0] + __logf(ml[j][1]) : neg_inf();
-            top8 = fmaxf(top8, lse_s[j]);
-        }
-        if(top8 == neg_inf())
-        {
-            continue;       // nothing visible so far
-        }
-        // what was accumulated against the old reference point
-        const float rescale = (top == neg_inf()) ? 0.0f : __expf(top - top8);
-        acc *= rescale;
-        wsum *= rescale;
-        top = top8;
-#pragma unroll
-        for(int j = 0; j < 8; ++j)
-        {
-            const float w = (lse_s[j] == neg_inf()) ? 0.0f : __expf(lse_s[j] - top);
-            wsum += w;
-            acc += w * v[j];
-        }
-    }
-    if(top == neg_inf())
-    {
-        // no visible key at all: leave lse and A untouched, or write the
-        // empty row when the running pair is being overwritten
-        if(p.overwrite)
-        {
-            *reinterpret_cast<f32x4 *>(Adst) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            if(d4 == 0)
-            {
-                p.lse[row] = neg_inf();
-            }
-        }
-        return;
-    }
-    const float lse_new = top + __logf(wsum);
-    const float lse_old = p.overwrite ? neg_inf() : p.lse[row];
-    float w_old, w_new, lse_out;
-    merge_weights(lse_old, lse_new, w_old, w_new, lse_out);
-    f32x4 v = acc * (w_new / wsum);
-    if(w_old != 0.0f)
-    {
-        v += w_old * *reinterpret_cast<const f32x4 *>(Adst);
-    }
-    *reinterpret_cast<f32x4 *>(Adst) = v;
-    // The threads of a row sit in one wavefront (TPR <= 32 divides 64) and
-    // run in lock step: all of them have read lse_old by now.
-    if(d4 == 0)
-    {
-        p.lse[row] = lse_out;
+        f32dec_merge_row<HEAD, false>(p, (int)(grow / p.rows), (int)(grow % p.rows),
+                (int)(threadIdx.x % TPR) * 4);
     }
 }
 
@@ -553,47 +654,85 @@ int decode_fp32_steps(int64_t k_seq)
     return (int)((k_seq + kDecF32Keys - 1) / kDecF32Keys);
 }
 
-// Key splits per unit: two workgroups per CU when the units allow it, never
-// more than one split per key step.
-int decode_fp32_choose_splits(int units, int n_steps)
+// Key splits per unit: two workgroups per CU when the units allow it - three at
+// head 64, whose ring is half as large and whose steps are bound by a
+// wavefront's own chain of MFMAs (36 units of 15 000 keys: 64.2 us with two, 50.6
+// with three, 53.3 with four) - never more than one split per key step; the limits for few steps are those of the
+// 16-bit kernel (handing partials over costs 2 us, a step about 1).
+int decode_fp32_choose_splits(int units, int n_steps, int head)
 {
-    int splits = (2 * kDecF32CUs + units - 1) / units;
-    splits = splits < 1 ? 1 : splits;
-    splits = splits > n_steps ? n_steps : splits;
+    constexpr int kDirectSteps = 3, kSingleSteps = 8;
+    if(n_steps <= kDirectSteps)
+    {
+        return 1;
+    }
+    const int by_units = decode_splits_by_units(units, (head <= 64 ? 3 : 2) * kDecF32CUs);
+    const int most = n_steps <= kSingleSteps ? n_steps : (n_steps + 1) / 2;
+    const int splits = by_units < most ? by_units : most;
     return splits > 64 ? 64 : splits;
 }
 
 // The workspace: the partial outputs [unit][split][rows][head] and the (max,
-// sum) pairs [unit][split][rows][2], both fp32
-size_t decode_fp32_workspace_bytes(int units, int n_splits, int rows, int head)
+// sum) pairs [unit][split][rows][2], both fp32, then the flags of the merge
+size_t decode_fp32_partial_bytes(int units, int n_splits, int rows, int head)
 {
     return (size_t)units * n_splits * rows * (head + 2) * sizeof(float);
 }
 
+size_t decode_fp32_workspace_bytes(int units, int n_splits, int rows, int head)
+{
+    return decode_fp32_partial_bytes(units, n_splits, rows, head)
+        + (size_t)units * decode_sync_stride(n_splits, rows, head) * sizeof(unsigned long long);
+}
+
+template<int HEAD, int MODE>
+static void launch_decode_fp32_mode(hipStream_t stream, const DecodeParams &p, dim3 grid)
+{
+    if(p.n_splits == 1)
+    {
+        hipLaunchKernelGGL((sdpa_decode_fp32_kernel<HEAD, MODE, true>), grid,
+                dim3(kDecF32Threads), 0, stream, p);
+    }
+    else
+    {
+        hipLaunchKernelGGL((sdpa_decode_fp32_kernel<HEAD, MODE, false>), grid,
+                dim3(kDecF32Threads), 0, stream, p);
+    }
+}
+
 template<int HEAD>
-static int launch_decode_fp32_head(hipStream_t stream, const DecodeParams &p, int mode)
+static int launch_decode_fp32_head(hipStream_t stream, DecodeParams &p, int mode)
 {
     const int units = p.n_batch * p.n_head_kv;
+    constexpr int rows_per_wg = 256 / (HEAD / 4);
+    // (the merge in the launch, and where not: as in the 16-bit launcher)
+    const int units8 = (units + 7) / 8 * 8;
+    p.merge_blocks_per_unit = (p.rows + rows_per_wg - 1) / rows_per_wg;
+    p.sync_stride = decode_sync_stride(p.n_splits, p.rows, HEAD);
+    p.fused = (p.fused && p.n_splits > 1 && !decode_uneven_units(units, p.k_seq, HEAD * 8)) ? 1 : 0;
+    p.units8 = (p.fused || units == units8) ? units8 : 0;
+    p.n_main = (p.units8 != 0 ? units8 : units) * p.n_splits;
+    if(p.fused)
+    {
+        p.tag = next_decode_tag();
+        p.spin_limit = decode_spin_limit_now();
+    }
     // (one more workgroup per unit when the call appends rows to the caches)
-    const dim3 grid((unsigned)(units * p.n_splits + (p.n_new > 0 ? units : 0))),
-        block(kDecF32Threads);
+    const dim3 grid((unsigned)(p.n_main + (p.fused ? units8 * p.merge_blocks_per_unit : 0)
+                + (p.n_new > 0 ? units : 0)));
     switch(mode)
     {
         case NNTILE_HIP_MASK_ADDITIVE:
-            hipLaunchKernelGGL((sdpa_decode_fp32_kernel<HEAD, NNTILE_HIP_MASK_ADDITIVE>), grid,
-                    block, 0, stream, p);
+            launch_decode_fp32_mode<HEAD, NNTILE_HIP_MASK_ADDITIVE>(stream, p, grid);
             break;
         case NNTILE_HIP_MASK_NONE:
-            hipLaunchKernelGGL((sdpa_decode_fp32_kernel<HEAD, NNTILE_HIP_MASK_NONE>), grid,
-                    block, 0, stream, p);
+            launch_decode_fp32_mode<HEAD, NNTILE_HIP_MASK_NONE>(stream, p, grid);
             break;
         case NNTILE_HIP_MASK_CAUSAL:
-            hipLaunchKernelGGL((sdpa_decode_fp32_kernel<HEAD, NNTILE_HIP_MASK_CAUSAL>), grid,
-                    block, 0, stream, p);
+            launch_decode_fp32_mode<HEAD, NNTILE_HIP_MASK_CAUSAL>(stream, p, grid);
             break;
         case NNTILE_HIP_MASK_BOOL:
-            hipLaunchKernelGGL((sdpa_decode_fp32_kernel<HEAD, NNTILE_HIP_MASK_BOOL>), grid,
-                    block, 0, stream, p);
+            launch_decode_fp32_mode<HEAD, NNTILE_HIP_MASK_BOOL>(stream, p, grid);
             break;
         default:
             return NNTILE_HIP_EINVAL;
@@ -602,17 +741,19 @@ static int launch_decode_fp32_head(hipStream_t stream, const DecodeParams &p, in
     {
         return NNTILE_HIP_ELAUNCH;
     }
-    constexpr int rows_per_wg = 256 / (HEAD / 4);
-    const int64_t total_rows = (int64_t)units * p.rows;
-    hipLaunchKernelGGL((sdpa_decode_fp32_reduce_kernel<HEAD>),
-            dim3((unsigned)((total_rows + rows_per_wg - 1) / rows_per_wg)), dim3(256), 0,
-            stream, p);
+    if(p.n_splits > 1 && !p.fused)
+    {
+        const int64_t total_rows = (int64_t)units * p.rows;
+        hipLaunchKernelGGL((sdpa_decode_fp32_reduce_kernel<HEAD>),
+                dim3((unsigned)((total_rows + rows_per_wg - 1) / rows_per_wg)), dim3(256), 0,
+                stream, p);
+    }
     return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
 }
 
-// p: fully filled but for nothing; part_o and part_ml point into the
-// workspace, n_splits / n_steps / steps_per_split from the functions above.
-int launch_decode_fp32(hipStream_t stream, const DecodeParams &p, int head, int mode)
+// p: filled but for the layout of the grid; part_o, part_ml and sync point into
+// the workspace, n_splits / n_steps / steps_per_split from the functions above.
+int launch_decode_fp32(hipStream_t stream, DecodeParams &p, int head, int mode)
 {
     switch(head)
     {
