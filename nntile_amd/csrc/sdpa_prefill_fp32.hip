@@ -29,7 +29,7 @@
 //     workgroups spread over the CUs.
 #include <type_traits>
 
-#include "sdpa_common.hpp"
+#include "sdpa_mask_scan.hpp"
 
 namespace nntile_hip
 {
@@ -319,6 +319,46 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         }
     }
 
+    // A mask given as values: the workgroup's rows of it are looked over once.
+    // Hidden steps at either end are not walked - a tile pair above the
+    // diagonal of a causal mask costs this look instead of a pass over K and V -
+    // and steps in which nothing is masked read no mask values.  (3 x 3 tasks of
+    // 800 x 800 x 2 under a window of 65 keys: 404 us without.)
+    int n_skip = 0;                             // key steps in front of the walk
+    unsigned long long not_open = ~0ull;        // bit s: step s reads its mask values
+    if constexpr(EXPLICIT)
+    {
+        constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 4 : 1;
+        if(n_steps > 0 && p.k_seq * ES >= 16 && p.mask_ld * ES * QROWS < (int64_t)(1 << 30))
+        {
+            __shared__ unsigned long long scan_words[2 * kThreads32 / 64];
+            unsigned long long not_hidden;
+            mask_scan_steps<ES, kThreads32 / 64, kKeys32>(static_cast<const char *>(p.mask)
+                    + q_row0 * p.mask_ld * ES, (uint32_t)(p.mask_ld * ES),
+                    (int)min((int64_t)QROWS, q_len - q_row0), (int)p.k_seq * ES, 0, n_steps,
+                    (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0u : 0x01010101u,
+                    (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0xff800000u : 0u, scan_words, not_open,
+                    not_hidden);
+            if(not_hidden == 0ull)
+            {
+                if(!p.overwrite)
+                {
+                    return;
+                }
+                n_steps = 0;        // the epilogue writes empty rows
+            }
+            else
+            {
+                if((not_hidden >> 63) == 0ull)
+                {
+                    n_steps = min(n_steps, 64 - __builtin_clzll(not_hidden));
+                }
+                n_skip = min(__builtin_ctzll(not_hidden), n_steps - 1);
+                n_steps -= n_skip;
+            }
+        }
+    }
+
     const float c = EXPLICIT ? kLog2e : p.scale * kLog2e;
 
     f32x16 o[DBLOCKS];
@@ -350,21 +390,28 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         // Explicit mask: the step's 16 values of this lane are loaded here,
         // ahead of the chain of MFMAs.  Register r holds key
         // 8*(r/4) + 4*half + r%4: four groups of four consecutive keys.  A full
-        // step of an aligned mask takes one 16-byte (additive) or 4-byte
-        // (boolean) load per group; lanes are queries, a mask row apart, so
-        // the cost of a load is the cache lines it touches, not its width.
-        // Otherwise element by element: keys past the end of a ragged step
-        // are hidden, and their loads are clamped to the step's last key
-        // instead of being branched around, so that the loads are independent.
+        // step takes one 16-byte (additive) or 4-byte (boolean) load per group,
+        // at the alignment of one element; lanes are queries, a mask row apart,
+        // so the cost of a load is the cache lines it touches, not its width.
+        // A ragged step goes element by element: keys past its end are hidden,
+        // and their loads are clamped to the step's last key instead of being
+        // branched around, so that the loads are independent.  A step in which
+        // nothing is masked loads nothing.
         float madd[EXPLICIT ? 16 : 1];
         if(EXPLICIT)
         {
             const int64_t mrow = (q_ok ? my_q : 0) * p.mask_ld + k_row0;
-            constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 4 : 1;
-            const bool wide = (p.mask_ld % 4 == 0) && (k_row0 % 4 == 0)
-                && (reinterpret_cast<uintptr_t>(p.mask) % (4 * ES) == 0)
-                && keys_here == kKeys32;
-            if(wide)
+            typedef f32x4 __attribute__((aligned(4))) f32x4_any;
+            typedef uint32_t __attribute__((aligned(1))) u32_any;
+            if(((not_open >> min(g, 63)) & 1ull) == 0ull && keys_here == kKeys32)
+            {
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    madd[r] = 0.0f;
+                }
+            }
+            else if(keys_here == kKeys32)
             {
 #pragma unroll
                 for(int rg = 0; rg < 4; ++rg)
@@ -372,7 +419,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
                     const int64_t at = mrow + 8 * rg + 4 * half;
                     if(MODE == NNTILE_HIP_MASK_ADDITIVE)
                     {
-                        const f32x4 v = *reinterpret_cast<const f32x4 *>(
+                        const f32x4 v = *reinterpret_cast<const f32x4_any *>(
                                 static_cast<const float *>(p.mask) + at);
 #pragma unroll
                         for(int e = 0; e < 4; ++e)
@@ -382,7 +429,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
                     }
                     else
                     {
-                        const uint32_t w = *reinterpret_cast<const uint32_t *>(
+                        const uint32_t w = *reinterpret_cast<const u32_any *>(
                                 static_cast<const uint8_t *>(p.mask) + at);
 #pragma unroll
                         for(int e = 0; e < 4; ++e)
@@ -612,12 +659,12 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         static_assert(LPW == QSTEPS && 16 * DBLOCKS == 4 * LPW, "one load instruction per four MFMAs");
         if(n_my > 0)
         {
-            const StepSource src0 = locate(wave_u);
+            const StepSource src0 = locate(n_skip + wave_u);
             fetch(src0.K, src0.rows_left, k_goff, lds_v0);         // K(0) into P
             StepSource src1 = {nullptr, nullptr, 0};
             if(n_my > 1)
             {
-                src1 = locate(wave_u + 4);
+                src1 = locate(n_skip + wave_u + 4);
                 fetch(src1.K, src1.rows_left, k_goff, lds_k0);     // K(1) into R
                 // K(0) has landed, K(1) may still be on its way.  (This also
                 // says that the Q values, ordinary loads, have arrived, with an
@@ -632,14 +679,14 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
             }
             F32_STAMP(1)
             f32x16 s_cur;
-            scores(wave_u, Pw, s_cur, nothing);
+            scores(n_skip + wave_u, Pw, s_cur, nothing);
             F32_STAMP(2)
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // P has been read
             StepSource cur = src0;      // step i: its V is still to be requested
             StepSource nxt = src1;      // step i+1: its K is in R or on its way there
             for(int i = 0; i < n_my; ++i)
             {
-                const int g = wave_u + 4 * i;
+                const int g = n_skip + wave_u + 4 * i;
                 const bool more = i + 1 < n_my;
                 const bool more2 = i + 2 < n_my;
                 StepSource nxt2 = {nullptr, nullptr, 0};
@@ -795,7 +842,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         // ---- the four wavefronts share every key step ------------------------------
         if(n_steps > 0)
         {
-            const StepSource src = locate(0);
+            const StepSource src = locate(n_skip);
             fetch(src.K, src.rows_left, k_goff, lds_k0);
             fetch(src.V, src.rows_left, v_goff, lds_v0);
         }
@@ -808,14 +855,14 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
             // passed the barrier that ended step g-1: nobody reads them)
             if(g + 1 < n_steps)
             {
-                const StepSource nxt = locate(g + 1);
+                const StepSource nxt = locate(n_skip + g + 1);
                 fetch(nxt.K, nxt.rows_left, k_goff, BUF ? lds_k0 : lds_k1);
                 fetch(nxt.V, nxt.rows_left, v_goff, BUF ? lds_v0 : lds_v1);
             }
             if(!hidden(g))
             {
                 f32x16 s;
-                scores(g, BUF ? lds_k1 : lds_k0, s, nothing);
+                scores(n_skip + g, BUF ? lds_k1 : lds_k0, s, nothing);
                 softmax(s);
                 output(BUF ? lds_v1 : lds_v0, s, nothing);
             }
