@@ -8,10 +8,15 @@
 //              dx[2i+1,j]  = cos[i] dy[2i+1,j] - sin[i] dy[2i,j]
 //
 // (the backward writes dx, it does not add to it).  Products and sums in fp32,
-// one rounding to the tile type.  Pure streaming: a thread takes four
-// neighbouring pairs - 16 bytes of a 16-bit tensor, 32 of an fp32 one - and
-// the four sines and cosines that go with them; m not a multiple of 4, or
-// addresses that are not aligned for that, take one pair per thread.
+// one rounding to the tile type.  Pure streaming, bound by HBM: a thread takes
+// four neighbouring pairs - 16 bytes of a 16-bit tensor, 32 of an fp32 one -
+// of COLS columns j and the four sines and cosines that go with them, which it
+// so reads once for all of them (read again for every column they are as many
+// bytes from L2 as the tensor has); the grid has one axis for i and one for j,
+// so that nothing is divided (a 64-bit remainder per thread before).  m not a
+// multiple of 4, or addresses that are not aligned for that, take one pair per
+// thread.  2 x 131072 x 32 bf16 (34.1 MB) 7.9 -> 6.6 us = 5.2 TB/s; two columns against
+// four: 6.6 and 7.1 us there, 14.9 and 15.6 on 2 x 524288 x 8 fp32.
 #include "sdpa_common.hpp"
 
 namespace nntile_hip
@@ -51,61 +56,75 @@ __device__ __forceinline__ void rotate(float c, float s, float a, float b, float
     }
 }
 
-template<typename S, bool BACKWARD>
+template<typename S, bool BACKWARD, int COLS>
 __global__ __launch_bounds__(256)
-void rope_vec_kernel(int64_t m, int64_t quads, const typename S::storage *sin,
+void rope_vec_kernel(int64_t m, int n, int row_blocks, const typename S::storage *sin,
         const typename S::storage *cos, const typename S::storage *src,
         typename S::storage *dst)
 {
     typedef typename S::storage E;
-    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if(t >= quads)
+    constexpr int NV = (int)sizeof(E) / 2;      // 16-byte pieces of four pairs
+    const int j0 = (int)(blockIdx.x / (unsigned)row_blocks) * COLS;
+    const int64_t i = 4 * ((int64_t)(blockIdx.x % (unsigned)row_blocks) * 256 + threadIdx.x);
+    if(i >= m)
     {
         return;
     }
-    const int64_t i = (4 * t) % m;              // m % 4 == 0: the four share a column j
-    __attribute__((aligned(16))) E in[8];
-    __attribute__((aligned(16))) E out[8];
     __attribute__((aligned(16))) E sv[4];
     __attribute__((aligned(16))) E cv[4];
     // src and dst pass through once (non-temporal); sin and cos are re-read
-    // by every column j and stay cached
+    // by the other columns and stay cached
     if constexpr(sizeof(E) == 2)
     {
-        *reinterpret_cast<u32x4 *>(in) = __builtin_nontemporal_load(
-                reinterpret_cast<const u32x4 *>(src + 8 * t));
         *reinterpret_cast<u32x2 *>(sv) = *reinterpret_cast<const u32x2 *>(sin + i);
         *reinterpret_cast<u32x2 *>(cv) = *reinterpret_cast<const u32x2 *>(cos + i);
     }
     else
     {
-        reinterpret_cast<u32x4 *>(in)[0] = __builtin_nontemporal_load(
-                reinterpret_cast<const u32x4 *>(src + 8 * t));
-        reinterpret_cast<u32x4 *>(in)[1] = __builtin_nontemporal_load(
-                reinterpret_cast<const u32x4 *>(src + 8 * t) + 1);
         *reinterpret_cast<u32x4 *>(sv) = *reinterpret_cast<const u32x4 *>(sin + i);
         *reinterpret_cast<u32x4 *>(cv) = *reinterpret_cast<const u32x4 *>(cos + i);
     }
+    u32x4 raw[COLS][NV];
 #pragma unroll
-    for(int k = 0; k < 4; ++k)
+    for(int c = 0; c < COLS; ++c)
     {
-        float x, y;
-        rotate<BACKWARD>(S::to_float(cv[k]), S::to_float(sv[k]), S::to_float(in[2 * k]),
-                S::to_float(in[2 * k + 1]), x, y);
-        out[2 * k] = S::from_float(x);
-        out[2 * k + 1] = S::from_float(y);
+        // (columns past the end re-read the last one)
+        const E *from = src + 2 * (i + m * min(j0 + c, n - 1));
+#pragma unroll
+        for(int v = 0; v < NV; ++v)
+        {
+            raw[c][v] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(from) + v);
+        }
     }
-    if constexpr(sizeof(E) == 2)
+#pragma unroll
+    for(int c = 0; c < COLS; ++c)
     {
-        __builtin_nontemporal_store(*reinterpret_cast<const u32x4 *>(out),
-                reinterpret_cast<u32x4 *>(dst + 8 * t));
-    }
-    else
-    {
-        __builtin_nontemporal_store(reinterpret_cast<const u32x4 *>(out)[0],
-                reinterpret_cast<u32x4 *>(dst + 8 * t));
-        __builtin_nontemporal_store(reinterpret_cast<const u32x4 *>(out)[1],
-                reinterpret_cast<u32x4 *>(dst + 8 * t) + 1);
+        __attribute__((aligned(16))) E in[8];
+        __attribute__((aligned(16))) E out[8];
+#pragma unroll
+        for(int v = 0; v < NV; ++v)
+        {
+            reinterpret_cast<u32x4 *>(in)[v] = raw[c][v];
+        }
+#pragma unroll
+        for(int k = 0; k < 4; ++k)
+        {
+            float x, y;
+            rotate<BACKWARD>(S::to_float(cv[k]), S::to_float(sv[k]), S::to_float(in[2 * k]),
+                    S::to_float(in[2 * k + 1]), x, y);
+            out[2 * k] = S::from_float(x);
+            out[2 * k + 1] = S::from_float(y);
+        }
+        if(j0 + c < n)
+        {
+            E *to = dst + 2 * (i + m * (j0 + c));
+#pragma unroll
+            for(int v = 0; v < NV; ++v)
+            {
+                __builtin_nontemporal_store(reinterpret_cast<const u32x4 *>(out)[v],
+                        reinterpret_cast<u32x4 *>(to) + v);
+            }
+        }
     }
 }
 
@@ -141,23 +160,41 @@ static int launch_rope_typed(hipStream_t stream, int64_t m, int64_t n, const voi
     {
         return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;
     };
-    const bool vec = m % 4 == 0 && aligned(src, 16) && aligned(dst, 16)
+    const bool vec = m % 4 == 0 && n <= 0x7fffffff && aligned(src, 16) && aligned(dst, 16)
         && aligned(sin, 4 * sizeof(E)) && aligned(cos, 4 * sizeof(E));
-    const int64_t threads = vec ? pairs / 4 : pairs;
-    const int64_t blocks = (threads + 255) / 256;
-    if(blocks > 0x7fffffff)
-    {
-        return NNTILE_HIP_EINVAL;
-    }
     if(vec)
     {
-        hipLaunchKernelGGL((rope_vec_kernel<S, BACKWARD>), dim3((unsigned)blocks), dim3(256), 0,
-                stream, m, threads, sin, cos, src, dst);
+        // two columns a thread once that leaves every CU eight workgroups,
+        // enough for its memory pipeline
+        constexpr int COLS = 2;
+        const int64_t rows = (m / 4 + 255) / 256;
+        const bool many = rows * ((n + COLS - 1) / COLS) >= 2048;
+        const int64_t cols = many ? (n + COLS - 1) / COLS : n;
+        if(rows > 0x7fffffff / cols)
+        {
+            return NNTILE_HIP_EINVAL;
+        }
+        const dim3 grid((unsigned)(rows * cols));
+        if(many)
+        {
+            hipLaunchKernelGGL((rope_vec_kernel<S, BACKWARD, COLS>), grid, dim3(256), 0, stream, m,
+                    (int)n, (int)rows, sin, cos, src, dst);
+        }
+        else
+        {
+            hipLaunchKernelGGL((rope_vec_kernel<S, BACKWARD, 1>), grid, dim3(256), 0, stream, m,
+                    (int)n, (int)rows, sin, cos, src, dst);
+        }
     }
     else
     {
+        const int64_t blocks = (pairs + 255) / 256;
+        if(blocks > 0x7fffffff)
+        {
+            return NNTILE_HIP_EINVAL;
+        }
         hipLaunchKernelGGL((rope_pair_kernel<S, BACKWARD>), dim3((unsigned)blocks), dim3(256), 0,
-                stream, m, threads, sin, cos, src, dst);
+                stream, m, pairs, sin, cos, src, dst);
     }
     return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
 }

@@ -148,15 +148,191 @@ void transpose16_kernel(int64_t m, int64_t n, int64_t tiles_m, float alpha,
     }
 }
 
+// Matrices with one short axis of 2 .. 64 (the heads of a layer: projections
+// into the attention layout and back).  A block of either kernel above fills
+// only as much of its own short side as the matrix has - 8 heads left three
+// threads in four idle, 12 heads went element by element - so here a
+// workgroup takes kTrShortBytes of the matrix whatever its short axis: `tl`
+// long indices, a flat contiguous piece on the side where the short axis is
+// the fast one, rows of tl elements on the other.  Both sides move 16 bytes per
+// thread; the elements cross over in LDS.
+//   SRC_SHORT: src is [long][short]; LDS rows are the short index, padded by 16
+//   bytes, and leave as they lie.
+//   otherwise: dst is [long][short]; LDS holds the flat piece of dst, with 4
+//   bytes of padding behind every 16 bytes x short, so that the lanes of a
+//   write, that far apart, fall on different banks.
+// Bound: HBM.  bf16, back to back: 8 x 262144 7.9 -> 3.6 us (a launch), 8 x 1163520
+// 27.8 -> 7.6 = 4.9 TB/s, 12 x 1163520 53.6 -> 11.3, 32 x 1163520 35.4 -> 26.0 =
+// 5.7 TB/s; fp32 16 x 1163520 92.5 -> 26.2.
+constexpr int kTrShortMax = 64, kTrShortBytes = 16384;
+
+template<typename S, bool SRC_SHORT>
+__global__ __launch_bounds__(256)
+void transpose_short_kernel(int n_short, int64_t n_long, int tile_long, float alpha,
+        const typename S::storage *src, typename S::storage *dst)
+{
+    typedef typename S::storage E;
+    constexpr int V = 16 / (int)sizeof(E);              // elements per access
+    constexpr int ELEMS = kTrShortBytes / (int)sizeof(E);
+    constexpr int ITERS = ELEMS / V / 256;
+    constexpr int WORD = 4 / (int)sizeof(E);
+    __shared__ __attribute__((aligned(16))) E lds[ELEMS
+        + (kTrShortMax * V > ELEMS / 8 ? kTrShortMax * V : ELEMS / 8)];
+    const int64_t l0 = (int64_t)blockIdx.x * tile_long;
+    const int tl = (int)min((int64_t)tile_long, n_long - l0);   // a multiple of V
+    const int row_vecs = tl / V, n_vecs = n_short * row_vecs;
+    const int pitch = tile_long + V;
+    // (quotients by the two wave-common divisors: exact below 2^16)
+    const uint32_t by_short = 0xffffffffu / (uint32_t)n_short + 1u;
+    const uint32_t by_row = 0xffffffffu / (uint32_t)row_vecs + 1u;
+    auto over = [](int x, uint32_t magic, int d) __attribute__((always_inline)) -> int
+    {
+        return d == 1 ? x : (int)__umulhi((uint32_t)x, magic);
+    };
+    const int tid = threadIdx.x;
+    const E *flat_src = src + l0 * n_short;
+    u32x4 raw[ITERS];
+#pragma unroll
+    for(int it = 0; it < ITERS; ++it)
+    {
+        const int v = min(tid + 256 * it, n_vecs - 1);
+        const int r = over(v, by_row, row_vecs);
+        raw[it] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(SRC_SHORT
+                    ? flat_src + v * V : src + r * n_long + l0 + (v - r * row_vecs) * V));
+    }
+#pragma unroll
+    for(int it = 0; it < ITERS; ++it)
+    {
+        const int v = tid + 256 * it;
+        if(v >= n_vecs)
+        {
+            break;
+        }
+        int at, step, i = 0;
+        if(SRC_SHORT)
+        {
+            const int j = over(v * V, by_short, n_short);
+            i = v * V - j * n_short;
+            at = i * pitch + j;
+            step = pitch;
+        }
+        else
+        {
+            const int j = over(v, by_row, row_vecs), c = v - j * row_vecs;
+            at = c * (V * n_short + WORD) + j;
+            step = n_short;
+        }
+#pragma unroll
+        for(int k = 0; k < V; ++k)
+        {
+            const uint32_t word = raw[it][k / WORD];
+            if constexpr(sizeof(E) == 2)
+            {
+                lds[at] = (E)(word >> (16 * (k % 2)));
+            }
+            else
+            {
+                lds[at] = __uint_as_float(word);
+            }
+            at += step;
+            if(SRC_SHORT && ++i == n_short)
+            {
+                i = 0;
+                at += 1 - n_short * pitch;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for(int it = 0; it < ITERS; ++it)
+    {
+        const int v = tid + 256 * it;
+        if(v >= n_vecs)
+        {
+            break;
+        }
+        uint32_t w[4];
+        E *to;
+        if(SRC_SHORT)
+        {
+            const int r = over(v, by_row, row_vecs), c = v - r * row_vecs;
+            const u32x4 x = *reinterpret_cast<const u32x4 *>(lds + r * pitch + c * V);
+#pragma unroll
+            for(int e = 0; e < 4; ++e)
+            {
+                w[e] = x[e];
+            }
+            to = dst + r * n_long + l0 + c * V;
+        }
+        else
+        {
+            const uint32_t *x = reinterpret_cast<const uint32_t *>(lds + v * V
+                    + over(v, by_short, n_short) * WORD);
+#pragma unroll
+            for(int e = 0; e < 4; ++e)
+            {
+                w[e] = x[e];
+            }
+            to = dst + l0 * n_short + v * V;
+        }
+        if(alpha != 1.0f)
+        {
+#pragma unroll
+            for(int e = 0; e < 4; ++e)
+            {
+                if constexpr(sizeof(E) == 2)
+                {
+                    const float lo = alpha * S::to_float((uint16_t)(w[e] & 0xffffu));
+                    const float hi = alpha * S::to_float((uint16_t)(w[e] >> 16));
+                    w[e] = (uint32_t)S::from_float(lo) | ((uint32_t)S::from_float(hi) << 16);
+                }
+                else
+                {
+                    w[e] = __float_as_uint(alpha * __uint_as_float(w[e]));
+                }
+            }
+        }
+        __builtin_nontemporal_store(u32x4{w[0], w[1], w[2], w[3]}, reinterpret_cast<u32x4 *>(to));
+    }
+}
+
 template<typename S>
 static int launch_transpose_typed(hipStream_t stream, int64_t m, int64_t n, float alpha,
         const void *src, void *dst)
 {
     typedef typename S::storage E;
+    const bool aligned = ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst))
+            & 15u) == 0;
+    {
+        // a short axis, and a long one of whole 16-byte pieces
+        constexpr int V = 16 / (int)sizeof(E);
+        const int64_t n_short = m < n ? m : n, n_long = m < n ? n : m;
+        if(aligned && n_short >= 2 && n_short <= kTrShortMax && n_long % V == 0 && n_long >= 64)
+        {
+            const int tile = kTrShortBytes / (int)sizeof(E) / (int)n_short / 32 * 32;
+            const int64_t wgs = (n_long + tile - 1) / tile;
+            if(wgs > 0x7fffffff)
+            {
+                return NNTILE_HIP_EINVAL;
+            }
+            if(m < n)
+            {
+                hipLaunchKernelGGL((transpose_short_kernel<S, true>), dim3((unsigned)wgs),
+                        dim3(256), 0, stream, (int)n_short, n_long, tile, alpha,
+                        static_cast<const E *>(src), static_cast<E *>(dst));
+            }
+            else
+            {
+                hipLaunchKernelGGL((transpose_short_kernel<S, false>), dim3((unsigned)wgs),
+                        dim3(256), 0, stream, (int)n_short, n_long, tile, alpha,
+                        static_cast<const E *>(src), static_cast<E *>(dst));
+            }
+            return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+        }
+    }
     if constexpr(sizeof(E) == 2)
     {
-        if(m % 8 == 0 && n % 8 == 0 && (reinterpret_cast<uintptr_t>(src) & 15u) == 0
-                && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0)
+        if(m % 8 == 0 && n % 8 == 0 && aligned)
         {
             const int64_t tm = (m + kTr16I - 1) / kTr16I, tn = (n + kTr16J - 1) / kTr16J;
             if(tm > 0x7fffffff / tn)

@@ -100,3 +100,25 @@ def test_errors():
     assert fn(None, 0, 7, None, None, None, None) == hip_sdpa.OK
     with pytest.raises(hip_sdpa.SdpaError):
         hip_sdpa.rope(s, s, x[:6], x[:6])       # 6 is not a multiple of 2 m = 4
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("m,n", [(4, 1), (1020, 3), (1024, 5), (262148, 9), (1048576, 4)])
+@pytest.mark.parametrize("backward", [False, True])
+def test_columns_per_thread(dtype, m, n, backward):
+    """One and two columns a thread, rows that end inside a workgroup, an odd
+    number of columns: against torch in fp32."""
+    print("case rope columns", dtype, m, n, backward, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    dt = H.TORCH_DT[dtype]
+    x = torch.randn(n, m, 2, generator=g, device="cuda").to(dt)
+    sin, cos = (torch.randn(m, generator=g, device="cuda").to(dt) for _ in range(2))
+    y = torch.full_like(x, float("nan"))
+    hip_sdpa.rope(sin, cos, x, y, backward=backward)
+    s, c = sin.float() * (-1 if backward else 1), cos.float()
+    a, b = x[..., 0].float(), x[..., 1].float()
+    want = torch.stack((c * a - s * b, s * a + c * b), dim=-1)
+    torch.cuda.synchronize()
+    bound = 2 * torch.finfo(dt).eps * (x.float().abs().sum(-1, keepdim=True)
+                                       * (s.abs() + c.abs())[None, :, None])
+    assert ((y.float() - want).abs() <= bound).all()

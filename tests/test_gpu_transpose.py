@@ -39,3 +39,20 @@ def test_errors():
     assert fn(None, 4, 4, 1.0, x.data_ptr(), x.data_ptr()) == hip_sdpa.EINVAL
     assert fn(None, 4, 4, 1.0, None, y.data_ptr()) == hip_sdpa.EINVAL
     assert fn(None, 0, 4, 1.0, None, None) == hip_sdpa.OK
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("short", [2, 3, 7, 12, 33, 63, 64])
+@pytest.mark.parametrize("long", [64, 104, 8192, 10000])
+@pytest.mark.parametrize("alpha", [1.0, 0.5])
+def test_short_axis(dtype, short, long, alpha):
+    """One axis of 2 to 64 elements: tiles that end inside the long axis,
+    either axis the short one."""
+    print("case transpose short", dtype, short, long, alpha, flush=True)
+    for m, n in ((short, long), (long, short)):
+        x = torch.randn(n, m, generator=torch.Generator(device="cuda").manual_seed(5),
+                        device="cuda").to(H.TORCH_DT[dtype])
+        y = torch.full_like(x, float("nan"))
+        hip_sdpa.transpose(alpha, x, y, m, n)
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(m, n), x.t() * alpha)
