@@ -560,6 +560,21 @@ int nntile_hip_sdpa_fwd_tile_cache_fp16(void *stream, const nntile_hip_sdpa_tile
 int nntile_hip_sdpa_fwd_tile_cache_fp32(void *stream, const nntile_hip_sdpa_tile_args *args,
         int64_t capacity);
 
+/* The same with device memory of the caller's, in which a chunk with fewer
+ * query blocks than the chip has places leaves the partial results of its key
+ * axis shared out over workgroups: nntile_hip_sdpa_fwd_tile_cache_workspace_bytes
+ * (16-bit tiles; ..._fp32) of it, 16-byte aligned, which later work on the same
+ * stream may reuse.  0 bytes: the call would not be shared out; with less
+ * memory, or none, it is not either. */
+size_t nntile_hip_sdpa_fwd_tile_cache_workspace_bytes(const nntile_hip_sdpa_tile_args *args);
+size_t nntile_hip_sdpa_fwd_tile_cache_workspace_bytes_fp32(const nntile_hip_sdpa_tile_args *args);
+int nntile_hip_sdpa_fwd_tile_cache_ws_bf16(void *stream, const nntile_hip_sdpa_tile_args *args,
+        int64_t capacity, void *workspace, size_t workspace_bytes);
+int nntile_hip_sdpa_fwd_tile_cache_ws_fp16(void *stream, const nntile_hip_sdpa_tile_args *args,
+        int64_t capacity, void *workspace, size_t workspace_bytes);
+int nntile_hip_sdpa_fwd_tile_cache_ws_fp32(void *stream, const nntile_hip_sdpa_tile_args *args,
+        int64_t capacity, void *workspace, size_t workspace_bytes);
+
 /* ---- 10. class of a mask tile -------------------------------------------------
  * For the layer that submits one task per (query tile, key tile) pair with
  * the pair's mask tile (src/tensor/flash_sdpa_fwd_cudnn.cc:246-274, which

@@ -12,7 +12,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libnntile_hip_sdpa.so")
 SOURCES = ["sdpa_prefill_16bit.hip", "sdpa_prefill_fp32.hip",
            "sdpa_decode_16bit.hip", "sdpa_decode_fp32.hip", "sdpa_bwd_16bit.hip", "rope.hip", "transpose.hip", "kv_cache.hip", "mask_classify.hip",
-           "accumulate_attn_output.hip", "capi.hip"]
+           "accumulate_attn_output.hip", "sdpa_parts_merge.hip", "capi.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

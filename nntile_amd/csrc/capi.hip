@@ -13,6 +13,11 @@ template<typename T>
 int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head, int mode,
         void *scan_scratch, size_t scan_scratch_bytes);
 int launch_prefill_fp32(hipStream_t stream, PrefillParams &p, int head, int mode);
+template<typename T>
+int launch_prefill_16bit_parts(hipStream_t stream, PrefillParams &p, int head, int mode);
+int launch_prefill_fp32_parts(hipStream_t stream, PrefillParams &p, int head, int mode);
+template<typename T>
+int launch_parts_merge(hipStream_t stream, const PrefillParams &p, int head);
 
 template<typename T>
 int launch_decode_16bit(hipStream_t stream, DecodeParams &p, int head, int mode);
@@ -98,10 +103,29 @@ static int dispatch_prefill(DType dt, hipStream_t stream, PrefillParams &p,
     }
 }
 
+// The two launches of a call whose keys are shared out in ranges.
+static int dispatch_parts(DType dt, hipStream_t stream, PrefillParams &p, int head, int mode)
+{
+    p.scale = 1.0f / sqrtf(static_cast<float>(head));
+    const int rc = dt == DType::bf16 ? launch_prefill_16bit_parts<Bf16>(stream, p, head, mode)
+        : dt == DType::fp16 ? launch_prefill_16bit_parts<Fp16>(stream, p, head, mode)
+        : launch_prefill_fp32_parts(stream, p, head, mode);
+    if(rc != NNTILE_HIP_OK)
+    {
+        return rc;
+    }
+    return dt == DType::bf16 ? launch_parts_merge<Bf16>(stream, p, head)
+        : dt == DType::fp16 ? launch_parts_merge<Fp16>(stream, p, head)
+        : launch_parts_merge<float>(stream, p, head);
+}
+
 // scan_scratch: device memory the call may overwrite (the reference's
-// scratch_logsumexp tile, scan_scratch_bytes of it), or null
+// scratch_logsumexp tile, scan_scratch_bytes of it), or null; parts_mem: memory
+// for the keys shared out in ranges (kv_rows given, prefill_parts says how
+// much), or null
 static int tile_call(DType dt, void *stream, const nntile_hip_sdpa_tile_args *a,
-        int64_t kv_rows = 0, void *scan_scratch = nullptr, size_t scan_scratch_bytes = 0)
+        int64_t kv_rows = 0, void *scan_scratch = nullptr, size_t scan_scratch_bytes = 0,
+        void *parts_mem = nullptr, size_t parts_bytes = 0)
 {
     if(a == nullptr || a->q_seq <= 0 || a->k_seq <= 0 || a->head <= 0
             || a->batch <= 0 || a->n_batch <= 0 || a->kv_group <= 0
@@ -146,6 +170,20 @@ static int tile_call(DType dt, void *stream, const nntile_hip_sdpa_tile_args *a,
     p.Q[0] = a->Q;
     p.lse[0] = a->lse;
     p.A[0] = a->A;
+    if(parts_mem != nullptr && kv_rows > 0 && !explicit_mask && p.form == 0)
+    {
+        const PrefillParts parts = prefill_parts(dt == DType::fp32, a->batch, a->q_seq, a->k_seq,
+                a->head);
+        if(parts.n > 1 && parts_bytes >= parts.bytes && aligned16(parts_mem))
+        {
+            p.n_parts = parts.n;
+            p.part_keys = parts.keys;
+            p.part_o = static_cast<float *>(parts_mem);
+            p.part_ml = p.part_o + (int64_t)parts.n * a->batch * a->q_seq * a->head;
+            return dispatch_parts(dt, static_cast<hipStream_t>(stream), p, (int)a->head,
+                    a->mask_mode);
+        }
+    }
     return dispatch_prefill(dt, static_cast<hipStream_t>(stream), p, a->head,
             a->mask_mode, scan_scratch, scan_scratch_bytes);
 }
@@ -1410,6 +1448,42 @@ int nntile_hip_sdpa_fwd_tile_cache_fp32(void *stream, const nntile_hip_sdpa_tile
     return args != nullptr && capacity < args->k_seq ? NNTILE_HIP_EINVAL
         : tile_call(DType::fp32, stream, args, capacity);
 }
+
+static size_t tile_cache_workspace(const nntile_hip_sdpa_tile_args *args, bool fp32)
+{
+    if(args == nullptr || args->batch <= 0 || args->q_seq <= 0 || args->k_seq <= 0
+            || args->batch > 0x7fffffff || args->q_seq > 0x7fffffff || args->k_seq > 0x7fffffff
+            || (args->mask_mode != NNTILE_HIP_MASK_NONE
+                && args->mask_mode != NNTILE_HIP_MASK_CAUSAL)
+            || prefill_form(args->flags) != 0)
+    {
+        return 0;
+    }
+    return prefill_parts(fp32, args->batch, args->q_seq, args->k_seq, args->head).bytes;
+}
+
+size_t nntile_hip_sdpa_fwd_tile_cache_workspace_bytes(const nntile_hip_sdpa_tile_args *args)
+{
+    return tile_cache_workspace(args, false);
+}
+
+size_t nntile_hip_sdpa_fwd_tile_cache_workspace_bytes_fp32(const nntile_hip_sdpa_tile_args *args)
+{
+    return tile_cache_workspace(args, true);
+}
+
+#define NNTILE_HIP_TILE_CACHE_WS(suffix, dt) \
+    int nntile_hip_sdpa_fwd_tile_cache_ws_##suffix(void *stream, \
+            const nntile_hip_sdpa_tile_args *args, int64_t capacity, void *workspace, \
+            size_t workspace_bytes) \
+    { \
+        return args != nullptr && capacity < args->k_seq ? NNTILE_HIP_EINVAL \
+            : tile_call(dt, stream, args, capacity, nullptr, 0, workspace, workspace_bytes); \
+    }
+NNTILE_HIP_TILE_CACHE_WS(bf16, DType::bf16)
+NNTILE_HIP_TILE_CACHE_WS(fp16, DType::fp16)
+NNTILE_HIP_TILE_CACHE_WS(fp32, DType::fp32)
+#undef NNTILE_HIP_TILE_CACHE_WS
 
 int nntile_hip_sdpa_fwd_decode_cache_bf16(void *stream, const nntile_hip_sdpa_tile_args *args,
         int64_t capacity, void *workspace, size_t workspace_bytes)

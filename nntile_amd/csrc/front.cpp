@@ -167,6 +167,8 @@ const tile_fn tile_fns[] = {nntile_hip_sdpa_fwd_tile_bf16, nntile_hip_sdpa_fwd_t
     nntile_hip_sdpa_fwd_tile_fp32};
 const tile_cache_fn tile_cache_fns[] = {nntile_hip_sdpa_fwd_tile_cache_bf16,
     nntile_hip_sdpa_fwd_tile_cache_fp16, nntile_hip_sdpa_fwd_tile_cache_fp32};
+const decode_cache_fn tile_cache_ws_fns[] = {nntile_hip_sdpa_fwd_tile_cache_ws_bf16,
+    nntile_hip_sdpa_fwd_tile_cache_ws_fp16, nntile_hip_sdpa_fwd_tile_cache_ws_fp32};
 const decode_fn decode_fns[] = {nntile_hip_sdpa_fwd_decode_bf16, nntile_hip_sdpa_fwd_decode_fp16,
     nntile_hip_sdpa_fwd_decode_fp32};
 const decode_cache_fn decode_cache_fns[] = {nntile_hip_sdpa_fwd_decode_cache_bf16,
@@ -258,6 +260,43 @@ PyObject *fwd_tile_cache(PyObject *, PyObject *const *v, Py_ssize_t n)
         }
         a.k_seq = integer(v[13]);
         return tile_cache_fns[ty](stream_of(v[14]), &a, capacity);
+    });
+}
+
+// ... + k_seq, workspace, stream: K, V are caches
+PyObject *fwd_tile_cache_ws(PyObject *, PyObject *const *v, Py_ssize_t n)
+{
+    return guarded(n, 16, [&]() -> int
+    {
+        nntile_hip_sdpa_tile_args a;
+        const at::Tensor *ws = maybe_tile(v[14]);
+        const Type ty = read_tile_call(a, v);
+        const int64_t capacity = a.k_seq;
+        if(tensor(v[0]).sizes() != tensor(v[4]).sizes())
+        {
+            return NNTILE_HIP_EINVAL;
+        }
+        a.k_seq = integer(v[13]);
+        return tile_cache_ws_fns[ty](stream_of(v[15]), &a, capacity, ptr(ws), nbytes(ws));
+    });
+}
+
+// (Q, k_seq, mask_mode) -> bytes
+PyObject *tile_cache_workspace(PyObject *, PyObject *const *v, Py_ssize_t n)
+{
+    return guarded(n, 3, [&]() -> long
+    {
+        const at::Tensor &Q = tensor(v[0]);
+        rank3(Q);
+        nntile_hip_sdpa_tile_args a = {};
+        a.batch = Q.size(0);
+        a.q_seq = Q.size(1);
+        a.head = Q.size(2);
+        a.k_seq = integer(v[1]);
+        a.mask_mode = (int32_t)integer(v[2]);
+        return (long)(type_of(v[0], Q) == FP32
+                ? nntile_hip_sdpa_fwd_tile_cache_workspace_bytes_fp32
+                : nntile_hip_sdpa_fwd_tile_cache_workspace_bytes)(&a);
     });
 }
 
@@ -674,7 +713,7 @@ PyTypeObject launch_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 #define FAST(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), \
     METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    FAST(fwd_tile), FAST(fwd_tile_cache), FAST(fwd_decode), FAST(fwd_decode_cache),
+    FAST(fwd_tile), FAST(fwd_tile_cache), FAST(fwd_tile_cache_ws), FAST(tile_cache_workspace), FAST(fwd_decode), FAST(fwd_decode_cache),
     FAST(fwd_decode_append_cache), FAST(cache_step), FAST(kv_append), FAST(flash_fwd),
     FAST(flash_bwd), FAST(bwd_tile), FAST(accumulate), FAST(rope), FAST(transpose),
     {nullptr, nullptr, 0, nullptr}};

@@ -104,7 +104,9 @@ __device__ __forceinline__ void mask_scan_range(const char *mask, uint32_t ld_by
             open_word, hidden_word, words, not_open, not_hidden);
 }
 
-template<typename T, int HEAD, int MODE, int WAVES = 4, int GROUPS = 1>
+// PARTS: the workgroup takes one of p.n_parts ranges of the keys and leaves
+// its triple in memory (PrefillParams::part_o), where launch_parts_merge finds it.
+template<typename T, int HEAD, int MODE, int WAVES = 4, int GROUPS = 1, bool PARTS = false>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1)
 void sdpa_prefill_16bit_kernel(const PrefillParams p)
 {
@@ -134,6 +136,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             && (LOADS_PER_WAVE == 1 || LOADS_PER_WAVE == 2 || LOADS_PER_WAVE == 4),
             "head size does not fit this tiling");
     static_assert(GROUPS == 1 || (GROUPS == 2 && WAVES == 8), "two groups of four wavefronts");
+    static_assert(!PARTS || (GROUPS == 2 && !EXPLICIT), "parts: analytic masks, two groups");
     static_assert(WAVES == 4 || (WAVES == 8 && (GROUPS == 2 || !EXPLICIT)),
             "eight wavefronts on 256 queries: analytic masks only");
 
@@ -214,6 +217,17 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             wg = ((3u * kCUsPerXCD - 1u - i) << 3) | (wg & 7u);
         }
     }
+    // (the parts of a query block have equal indices modulo 8 - one XCD - where
+    // the batch entries come in eights)
+    int part = 0;
+    if constexpr(PARTS)
+    {
+        const unsigned per_part = gridDim.x / (unsigned)p.n_parts;
+        part = (int)(wg / per_part);
+        wg -= (unsigned)part * per_part;
+    }
+    const int part_k0 = PARTS ? part * p.part_keys : 0;
+    const bool overwrite = PARTS || p.overwrite;
     int b, qblk;
     const int batch_all = p.batch * p.n_slabs;
     if(p.xcd_remap)
@@ -254,7 +268,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // the stored logsumexp that the epilogue merges with: requested here, so
     // that its latency passes beside the first loads
     float *lse_ptr = p.lse[q_tile0 + qt] + (int64_t)b * q_len + (q_ok ? my_q : 0);
-    const float lse_stored = p.overwrite ? neg_inf() : *lse_ptr;
+    const float lse_stored = overwrite ? neg_inf() : *lse_ptr;
 
     // Q fragments, resident for the whole kernel.
     vec8 qf[KSTEPS];
@@ -277,7 +291,8 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // row 0, plus the causal offset; key row kg is visible to query row
     // (q_row0 + r) iff kg <= rel0 + r.  Clamped so that the 32-bit arithmetic
     // below cannot overflow.
-    const int k_seq = (int)p.k_seq, k_tile = (int)p.k_tile;
+    const int k_seq = PARTS ? min(p.part_keys, (int)p.k_seq - part_k0) : (int)p.k_seq;
+    const int k_tile = PARTS ? k_seq : (int)p.k_tile;
     int rel0 = 0;
     const int last_k_len = k_seq - (p.n_kv_tiles - 1) * k_tile;
     int n_steps = (p.n_kv_tiles - 1) * p.k_blocks_per_tile
@@ -285,13 +300,13 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     if(MODE == NNTILE_HIP_MASK_CAUSAL)
     {
         int64_t rel = p.q_pos0 + (int64_t)qt * p.q_tile + q_row0
-            + p.causal_offset - p.k_pos0;
+            + p.causal_offset - p.k_pos0 - part_k0;
         rel = max((int64_t)-(1 << 30), min(rel, (int64_t)(1 << 30)));
         rel0 = (int)rel;
         const int hi = min(rel0 + min(kQRows, q_len - q_row0) - 1, k_seq - 1);
         if(hi < 0)
         {
-            if(!p.overwrite)
+            if(!overwrite)
             {
                 return;
             }
@@ -378,7 +393,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     auto slab = [&](int kt) -> int64_t
     {
         const int64_t rows = p.kv_rows > 0 ? p.kv_rows : (int64_t)tile_rows(kt);
-        return (int64_t)kvb * rows * HEAD * 2;
+        return ((int64_t)kvb * rows + part_k0) * (HEAD * 2);
     };
 
     // Global -> LDS loads of the K (or V) rows of one step.  Rows past the end
@@ -1490,6 +1505,38 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // ---- epilogue: normalise, merge into the running (lse, A) ----------------
     const float l_tot = sum_across_halves(l_run);
     const bool empty = !(l_tot > 0.0f);     // no visible key for this query
+    if constexpr(PARTS)
+    {
+        if(q_ok)
+        {
+            // (a sum that is no number stays one: the merged row is then empty,
+            // as it is without parts)
+            const bool none = l_tot == 0.0f;
+            const int64_t row = ((int64_t)part * p.batch + b) * p.q_seq + my_q;
+            if(half == 0)
+            {
+                p.part_ml[2 * row] = none ? neg_inf() : empty ? 0.0f : m_run * p.scale;
+                p.part_ml[2 * row + 1] = l_tot;
+            }
+            float *dst = p.part_o + row * HEAD + 4 * half;
+#pragma unroll
+            for(int db = 0; db < DBLOCKS; ++db)
+            {
+#pragma unroll
+                for(int rg = 0; rg < 4; ++rg)
+                {
+                    f32x4 v;
+#pragma unroll
+                    for(int e = 0; e < 4; ++e)
+                    {
+                        v[e] = none ? 0.0f : o[db][4 * rg + e];
+                    }
+                    *reinterpret_cast<f32x4 *>(dst + 32 * db + 8 * rg) = v;
+                }
+            }
+        }
+        return;
+    }
     // rows that are written; the others leave lse and A as they are
     const bool live = q_ok && !(empty && !p.overwrite);
     const float to_ln = p.scale;
@@ -1850,6 +1897,40 @@ int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head,
     }
 }
 
+// One tile against a long key axis, the keys in p.n_parts ranges (set by the
+// caller from prefill_parts, with p.part_*; p.kv_rows must be given).
+template<typename T>
+int launch_prefill_16bit_parts(hipStream_t stream, PrefillParams &p, int head, int mode)
+{
+    p.q_blocks_per_tile = (int)((p.q_tile + kQRows - 1) / kQRows);
+    p.k_blocks_per_tile = (int)((p.k_tile + kKeys - 1) / kKeys);
+    p.mask_bits = nullptr;
+    p.n_scan_wgs = 0;
+    p.xcd_remap = (p.batch % 8 == 0) ? 1 : 0;
+    const dim3 grid((unsigned)((int64_t)p.batch * p.q_blocks_per_tile * p.n_parts));
+    const bool causal = mode == NNTILE_HIP_MASK_CAUSAL;
+    auto launch = [&](auto kernel) -> int
+    {
+        hipLaunchKernelGGL(kernel, grid, dim3(512), 0, stream, p);
+        return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+    };
+    switch(head)
+    {
+        case 64:
+            return causal
+                ? launch(sdpa_prefill_16bit_kernel<T, 64, NNTILE_HIP_MASK_CAUSAL, 8, 2, true>)
+                : launch(sdpa_prefill_16bit_kernel<T, 64, NNTILE_HIP_MASK_NONE, 8, 2, true>);
+        case 128:
+            return causal
+                ? launch(sdpa_prefill_16bit_kernel<T, 128, NNTILE_HIP_MASK_CAUSAL, 8, 2, true>)
+                : launch(sdpa_prefill_16bit_kernel<T, 128, NNTILE_HIP_MASK_NONE, 8, 2, true>);
+        default:
+            return NNTILE_HIP_EUNSUPPORTED;
+    }
+}
+
+template int launch_prefill_16bit_parts<Bf16>(hipStream_t, PrefillParams &, int, int);
+template int launch_prefill_16bit_parts<Fp16>(hipStream_t, PrefillParams &, int, int);
 template int launch_prefill_16bit<Bf16>(hipStream_t, PrefillParams &, int, int, void *, size_t);
 template int launch_prefill_16bit<Fp16>(hipStream_t, PrefillParams &, int, int, void *, size_t);
 

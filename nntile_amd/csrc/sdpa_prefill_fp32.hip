@@ -83,7 +83,9 @@ template<int N> __device__ __forceinline__ void f32_wait_vmcnt()
     asm volatile("" ::: "memory");
 }
 
-template<int HEAD, int MODE, bool SPLIT>
+// PARTS: the workgroup takes one of p.n_parts ranges of the keys and leaves its
+// triple in memory (PrefillParams::part_o) for launch_parts_merge.
+template<int HEAD, int MODE, bool SPLIT, bool PARTS = false>
 __global__ __launch_bounds__(kThreads32, (SPLIT && HEAD == 128) ? 1 : 2)
 void sdpa_prefill_fp32_kernel(const PrefillParams p)
 {
@@ -101,6 +103,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     constexpr int BLOCK_BYTES = kKeys32 * RB;
     constexpr bool EXPLICIT = (MODE == NNTILE_HIP_MASK_ADDITIVE
             || MODE == NNTILE_HIP_MASK_BOOL);
+    static_assert(!PARTS || (SPLIT && !EXPLICIT), "parts: analytic masks, 32-query workgroups");
     static_assert(LPW >= 1, "head size does not fit this tiling");
 
     // SPLIT: lds_k0 / lds_v0 hold one step per wavefront (wavefront w owns
@@ -123,8 +126,26 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     const int q_blocks = p.n_q_tiles * p.q_blocks_per_tile;
     const int batch_all = p.batch * p.n_slabs;
     int wg = blockIdx.x;
+    int part = 0;
+    if constexpr(PARTS)
+    {
+        const int per_part = (int)gridDim.x / p.n_parts;
+        part = wg / per_part;
+        wg -= part * per_part;
+    }
+    const int64_t part_k0 = PARTS ? (int64_t)part * p.part_keys : 0;
+    const int64_t k_seq = PARTS ? min((int64_t)p.part_keys, p.k_seq - part_k0) : p.k_seq;
+    const int64_t k_tile = PARTS ? k_seq : p.k_tile;
+    const int64_t k_pos0 = p.k_pos0 + part_k0;
+    const bool overwrite = PARTS || p.overwrite;
     int b, qblk;
-    if(SPLIT)
+    if(PARTS)
+    {
+        // (all ranges alike: nothing to pair)
+        b = wg % batch_all;
+        qblk = q_blocks - 1 - wg / batch_all;
+    }
+    else if(SPLIT)
     {
         // A launch of this form fits the GPU at once, so where a workgroup
         // lands decides how evenly the CUs are loaded.  Workgroups are dealt
@@ -190,7 +211,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         }
     }
 
-    const int64_t last_k_len = p.k_seq - (int64_t)(p.n_kv_tiles - 1) * p.k_tile;
+    const int64_t last_k_len = k_seq - (int64_t)(p.n_kv_tiles - 1) * k_tile;
     int n_steps = (p.n_kv_tiles - 1) * p.k_blocks_per_tile
         + (int)((last_k_len + kKeys32 - 1) / kKeys32);
     const int64_t wg_qpos_hi = p.q_pos0 + (int64_t)qt * p.q_tile
@@ -246,11 +267,11 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         const char *K, *V;      // first row of the step
         int rows_left;          // rows of the tile from this step on
     };
-    const int64_t k_len0 = min(p.k_tile, p.k_seq);
+    const int64_t k_len0 = min(k_tile, k_seq);
     const bool one_tile = p.n_kv_tiles == 1;
     const int64_t entry_rows0 = p.kv_rows > 0 ? p.kv_rows : k_len0;
-    const char *K0 = static_cast<const char *>(p.K[k_tile0]) + ((int64_t)kvb * entry_rows0) * RB;
-    const char *V0 = static_cast<const char *>(p.V[k_tile0]) + ((int64_t)kvb * entry_rows0) * RB;
+    const char *K0 = static_cast<const char *>(p.K[k_tile0]) + ((int64_t)kvb * entry_rows0 + part_k0) * RB;
+    const char *V0 = static_cast<const char *>(p.V[k_tile0]) + ((int64_t)kvb * entry_rows0 + part_k0) * RB;
     auto locate = [&](int g) -> StepSource
     {
         StepSource src;
@@ -264,7 +285,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         {
             const int kt = g / p.k_blocks_per_tile;
             const int kb = g % p.k_blocks_per_tile;
-            const int64_t k_len = min(p.k_tile, p.k_seq - (int64_t)kt * p.k_tile);
+            const int64_t k_len = min(k_tile, k_seq - (int64_t)kt * k_tile);
             const int64_t off = ((int64_t)kvb * k_len + (int64_t)kb * kKeys32) * RB;
             src.K = static_cast<const char *>(p.K[k_tile0 + kt]) + off;
             src.V = static_cast<const char *>(p.V[k_tile0 + kt]) + off;
@@ -300,19 +321,19 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
 
     if(MODE == NNTILE_HIP_MASK_CAUSAL)
     {
-        const int64_t hi = wg_qpos_hi + p.causal_offset - p.k_pos0;
+        const int64_t hi = wg_qpos_hi + p.causal_offset - k_pos0;
         if(hi < 0)
         {
-            if(!p.overwrite)
+            if(!overwrite)
             {
                 return;
             }
             n_steps = 0;    // nothing visible: the epilogue writes empty rows
         }
-        const int64_t kt_hi = hi < 0 ? (int64_t)p.n_kv_tiles : hi / p.k_tile;
+        const int64_t kt_hi = hi < 0 ? (int64_t)p.n_kv_tiles : hi / k_tile;
         if(kt_hi < p.n_kv_tiles)
         {
-            const int64_t in_tile = hi - kt_hi * p.k_tile;
+            const int64_t in_tile = hi - kt_hi * k_tile;
             const int steps = (int)(kt_hi * p.k_blocks_per_tile
                     + in_tile / kKeys32 + 1);
             n_steps = min(n_steps, steps);
@@ -329,19 +350,19 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     if constexpr(EXPLICIT)
     {
         constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 4 : 1;
-        if(n_steps > 0 && p.k_seq * ES >= 16 && p.mask_ld * ES * QROWS < (int64_t)(1 << 30))
+        if(n_steps > 0 && k_seq * ES >= 16 && p.mask_ld * ES * QROWS < (int64_t)(1 << 30))
         {
             __shared__ unsigned long long scan_words[2 * kThreads32 / 64];
             unsigned long long not_hidden;
             mask_scan_steps<ES, kThreads32 / 64, kKeys32>(static_cast<const char *>(p.mask)
                     + q_row0 * p.mask_ld * ES, (uint32_t)(p.mask_ld * ES),
-                    (int)min((int64_t)QROWS, q_len - q_row0), (int)p.k_seq * ES, 0, n_steps,
+                    (int)min((int64_t)QROWS, q_len - q_row0), (int)k_seq * ES, 0, n_steps,
                     (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0u : 0x01010101u,
                     (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0xff800000u : 0u, scan_words, not_open,
                     not_hidden);
             if(not_hidden == 0ull)
             {
-                if(!p.overwrite)
+                if(!overwrite)
                 {
                     return;
                 }
@@ -383,9 +404,9 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     {
         const int kt = g / p.k_blocks_per_tile;
         const int kb = g % p.k_blocks_per_tile;
-        const int64_t k_len = min(p.k_tile, p.k_seq - (int64_t)kt * p.k_tile);
+        const int64_t k_len = min(k_tile, k_seq - (int64_t)kt * k_tile);
         const int64_t k_row0 = (int64_t)kb * kKeys32;
-        const int64_t k_pos_base = p.k_pos0 + (int64_t)kt * p.k_tile + k_row0;
+        const int64_t k_pos_base = k_pos0 + (int64_t)kt * k_tile + k_row0;
         const int keys_here = (int)min((int64_t)kKeys32, k_len - k_row0);
         // Explicit mask: the step's 16 values of this lane are loaded here,
         // ahead of the chain of MFMAs.  Register r holds key
@@ -630,7 +651,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         }
         const int kt = g / p.k_blocks_per_tile;
         const int kb = g % p.k_blocks_per_tile;
-        const int64_t k_pos_base = p.k_pos0 + (int64_t)kt * p.k_tile + (int64_t)kb * kKeys32;
+        const int64_t k_pos_base = k_pos0 + (int64_t)kt * k_tile + (int64_t)kb * kKeys32;
         return k_pos_base > wave_qpos_hi + p.causal_offset;
     };
 
@@ -937,14 +958,45 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     F32_STAMP(45)
     const float l_tot = l_run + __shfl_xor(l_run, 32);
     const bool empty = !(l_tot > 0.0f);     // no visible key for this query
-    if(!q_ok || (empty && !p.overwrite))
+    if constexpr(PARTS)
+    {
+        if(q_ok)
+        {
+            // (a sum that is no number stays one, as in the 16-bit kernel)
+            const bool none = l_tot == 0.0f;
+            const int64_t row = ((int64_t)part * p.batch + b) * p.q_seq + my_q;
+            if(half == 0)
+            {
+                p.part_ml[2 * row] = none ? neg_inf() : empty ? 0.0f : m_run * p.scale;
+                p.part_ml[2 * row + 1] = l_tot;
+            }
+            float *dst = p.part_o + row * HEAD + 4 * half;
+#pragma unroll
+            for(int db = 0; db < DBLOCKS; ++db)
+            {
+#pragma unroll
+                for(int rg = 0; rg < 4; ++rg)
+                {
+                    f32x4 v;
+#pragma unroll
+                    for(int e = 0; e < 4; ++e)
+                    {
+                        v[e] = none ? 0.0f : o[db][4 * rg + e];
+                    }
+                    *reinterpret_cast<f32x4 *>(dst + 32 * db + 8 * rg) = v;
+                }
+            }
+        }
+        return;
+    }
+    if(!q_ok || (empty && !overwrite))
     {
         return;     // leave lse and A as they are
     }
     const float to_ln = EXPLICIT ? 1.0f : p.scale;
     const float lse_new = empty ? neg_inf() : m_run * to_ln + __logf(l_tot);
     float *lse_ptr = p.lse[q_tile0 + qt] + (int64_t)b * q_len + my_q;
-    const float lse_old = p.overwrite ? neg_inf() : *lse_ptr;
+    const float lse_old = overwrite ? neg_inf() : *lse_ptr;
     float w_old = 0.0f, w_new = 0.0f, lse_out = neg_inf();
     if(!empty)
     {
@@ -1016,6 +1068,38 @@ static int launch_mode32(hipStream_t stream, const PrefillParams &p, int mode,
             return NNTILE_HIP_EINVAL;
     }
     return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+}
+
+// One tile against a long key axis, the keys in p.n_parts ranges (see
+// launch_prefill_16bit_parts).
+int launch_prefill_fp32_parts(hipStream_t stream, PrefillParams &p, int head, int mode)
+{
+    if(p.k_tile * head >= ((int64_t)1 << 31))
+    {
+        return NNTILE_HIP_EUNSUPPORTED;     // as without ranges
+    }
+    p.q_blocks_per_tile = (int)((p.q_tile + 31) / 32);
+    p.k_blocks_per_tile = (int)((p.k_tile + kKeys32 - 1) / kKeys32);
+    const dim3 grid((unsigned)((int64_t)p.batch * p.q_blocks_per_tile * p.n_parts));
+    const bool causal = mode == NNTILE_HIP_MASK_CAUSAL;
+    auto launch = [&](auto kernel) -> int
+    {
+        hipLaunchKernelGGL(kernel, grid, dim3(kThreads32), 0, stream, p);
+        return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+    };
+    switch(head)
+    {
+        case 64:
+            return causal
+                ? launch(sdpa_prefill_fp32_kernel<64, NNTILE_HIP_MASK_CAUSAL, true, true>)
+                : launch(sdpa_prefill_fp32_kernel<64, NNTILE_HIP_MASK_NONE, true, true>);
+        case 128:
+            return causal
+                ? launch(sdpa_prefill_fp32_kernel<128, NNTILE_HIP_MASK_CAUSAL, true, true>)
+                : launch(sdpa_prefill_fp32_kernel<128, NNTILE_HIP_MASK_NONE, true, true>);
+        default:
+            return NNTILE_HIP_EUNSUPPORTED;
+    }
 }
 
 int launch_prefill_fp32(hipStream_t stream, PrefillParams &p, int head, int mode)

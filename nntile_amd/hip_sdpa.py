@@ -134,6 +134,8 @@ EXPORTS = (
     + ["nntile_hip_sdpa_fwd_decode_cache_" + t for t in ("bf16", "fp16", "fp32")]
     + ["nntile_hip_sdpa_fwd_decode_append_cache_" + t for t in ("bf16", "fp16", "fp32")]
     + ["nntile_hip_sdpa_fwd_tile_cache_" + t for t in ("bf16", "fp16", "fp32")]
+    + ["nntile_hip_sdpa_fwd_tile_cache_ws_" + t for t in ("bf16", "fp16", "fp32")]
+    + ["nntile_hip_sdpa_fwd_tile_cache_workspace_bytes" + t for t in ("", "_fp32")]
     + ["nntile_hip_mask_tile_class_" + t for t in ("bf16", "fp16", "fp32", "bool")]
     + ["nntile_hip_sdpa_fwd_grid_codelet_" + t for t in ("bf16", "fp16", "fp32")]
     + ["nntile_hip_sdpa_bwd_grid_codelet_" + t for t in ("bf16", "fp16")]
@@ -204,6 +206,9 @@ def lib():
             f = getattr(L, "nntile_hip_sdpa_fwd_tile_cache_" + t)
             f.argtypes = [_vp, ctypes.POINTER(TileArgs), _i64]
             f.restype = ctypes.c_int
+            f = getattr(L, "nntile_hip_sdpa_fwd_tile_cache_ws_" + t)
+            f.argtypes = [_vp, ctypes.POINTER(TileArgs), _i64, _vp, ctypes.c_size_t]
+            f.restype = ctypes.c_int
             f = getattr(L, "nntile_hip_kv_cache_append_" + t)
             f.argtypes = [_vp] + [_i64] * 5 + [_vp] * 4
             f.restype = ctypes.c_int
@@ -219,6 +224,10 @@ def lib():
         L.nntile_hip_sdpa_fwd_decode_workspace_bytes.restype = ctypes.c_size_t
         L.nntile_hip_sdpa_fwd_decode_workspace_bytes_fp32.argtypes = [ctypes.POINTER(TileArgs)]
         L.nntile_hip_sdpa_fwd_decode_workspace_bytes_fp32.restype = ctypes.c_size_t
+        for t in ("", "_fp32"):
+            f = getattr(L, "nntile_hip_sdpa_fwd_tile_cache_workspace_bytes" + t)
+            f.argtypes = [ctypes.POINTER(TileArgs)]
+            f.restype = ctypes.c_size_t
         L.nntile_hip_sdpa_fwd_decode_static.argtypes = [_vp, ctypes.c_int32,
                                                         ctypes.POINTER(TileArgs)]
         L.nntile_hip_sdpa_fwd_decode_static.restype = ctypes.c_int
@@ -613,10 +622,17 @@ def sdpa_fwd_decode_cache(K_cache, V_cache, k_seq, Q, mask, lse, A, mask_mode, n
 
 
 def sdpa_fwd_tile_cache(K_cache, V_cache, k_seq, Q, mask, lse, A, mask_mode, n_batch=None,
-                        kv_group=1, q_pos0=0, k_pos0=0, causal_offset=0, flags=0, stream=None):
+                        kv_group=1, q_pos0=0, k_pos0=0, causal_offset=0, flags=0, stream=None,
+                        workspace=None):
     """sdpa_fwd_tile over the first k_seq rows of every entry of the caches
     ([entries, capacity, head]), read where they lie; any chunk length, fp32
-    included."""
+    included.  workspace: tile_cache_workspace_bytes of device memory, with
+    which a chunk too short to fill the chip shares its key axis out."""
+    if workspace is not None:
+        _check(_native().fwd_tile_cache_ws(K_cache, Q, mask, lse, V_cache, A, mask_mode, n_batch,
+                                           kv_group, q_pos0, k_pos0, causal_offset, flags, k_seq,
+                                           workspace, stream), "sdpa_fwd_tile_cache")
+        return
     _check(_native().fwd_tile_cache(K_cache, Q, mask, lse, V_cache, A, mask_mode, n_batch, kv_group,
                                     q_pos0, k_pos0, causal_offset, flags, k_seq, stream),
            "sdpa_fwd_tile_cache")
@@ -677,6 +693,12 @@ def decode_cache_workspace_bytes(k_seq, Q, n_batch, kv_group):
     a.batch, a.q_seq, a.head = Q.shape
     a.k_seq, a.n_batch, a.kv_group = k_seq, n_batch, kv_group
     return int(_decode_ws_fn(Q)(ctypes.byref(a)))
+
+
+def tile_cache_workspace_bytes(k_seq, Q, mask_mode):
+    """Bytes of workspace with which sdpa_fwd_tile_cache shares the key axis of
+    this call out; 0: it would not."""
+    return _native().tile_cache_workspace(Q, k_seq, mask_mode)
 
 
 def mask_tile_class(mask, offset=0, workspace=None, stream=None):

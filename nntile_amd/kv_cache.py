@@ -167,7 +167,9 @@ class KVCache:
         hidden) or a bool mask as for `mask_slice`, whose slice is then passed
         as values.  Few rows (kv_group * q_seq <= 64, head 64 or 128) take the
         split-key decode kernel of the tile type, everything else - longer
-        chunks, head 32 - the tile kernel; both read the caches in place."""
+        chunks, head 32 - the tile kernel, which shares its key axis out over
+        workgroups where the chunk's rows do not fill the chip; both read the
+        caches in place."""
         k_seq = len(self)
         q_seq = Q.shape[1]
         mode = hip_sdpa.MASK_CAUSAL if causal else hip_sdpa.MASK_NONE
@@ -187,9 +189,17 @@ class KVCache:
         self._mask_in_use = keep(sliced)
         decode = kv_group * q_seq <= 64 and Q.shape[2] in (64, 128)
         if not decode:
+            need = hip_sdpa.tile_cache_workspace_bytes(k_seq, Q, mode)
+            workspace = None
+            if need:
+                # (its own for each call, in the memory of the call's stream:
+                # calls on several streams may overlap)
+                with torch.cuda.stream(stream):
+                    workspace = torch.empty(need, dtype=torch.uint8, device=Q.device)
             hip_sdpa.sdpa_fwd_tile_cache(
                 self.k, self.v, k_seq, Q, sliced, lse, A, mode, n_batch, kv_group,
-                causal_offset=k_seq - q_seq, flags=hip_sdpa.OVERWRITE, stream=stream)
+                causal_offset=k_seq - q_seq, flags=hip_sdpa.OVERWRITE, stream=stream,
+                workspace=workspace)
             return
         workspace = self._decode_workspace(k_seq, Q, n_batch, kv_group, stream)
         hip_sdpa.sdpa_fwd_decode_cache(
