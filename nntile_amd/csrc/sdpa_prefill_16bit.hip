@@ -173,7 +173,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // work done.  The second group is therefore dealt in reverse: the longest
     // workgroup shares its CU with the shortest of the first 64.
     const int q_blocks = p.n_q_tiles * p.q_blocks_per_tile;
-    unsigned wg = blockIdx.x;
+    unsigned wg = blockIdx.x, n_att = gridDim.x;     // n_att: attention workgroups
     if constexpr(EXPLICIT)
     {
         // The first workgroups of the grid scan the mask for everybody (one
@@ -207,9 +207,12 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 return;
             }
             wg -= (unsigned)p.n_scan_wgs;
+            n_att -= (unsigned)p.n_scan_wgs;
         }
     }
-    if(WAVES == 4 && gridDim.x >= 8u * 2u * kCUsPerXCD)
+    // (only where the second group is complete: the places it is dealt to must
+    // all be attention workgroups' - those that scan a mask do not count)
+    if(WAVES == 4 && n_att >= 8u * 2u * kCUsPerXCD)
     {
         const unsigned i = wg >> 3;
         if(i >= kCUsPerXCD && i < 2u * kCUsPerXCD)

@@ -108,3 +108,31 @@ def test_a_scratch_smaller_than_a_logsumexp_tile_is_refused_or_left_alone():
     torch.cuda.synchronize()
     assert torch.isnan(tiny).all()            # left alone
     assert torch.equal(lse0, lse1) and torch.equal(A0.view(torch.int16), A1.view(torch.int16))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("seq,batch", [(640, 100), (1000, 63), (640, 102), (640, 103)])
+def test_every_block_where_the_scan_fills_the_second_round(dtype, seq, batch):
+    """The workgroups that scan the mask do not count where the second 256
+    attention workgroups are dealt in reverse: 500 + 40, 504 + 64 (not dealt so),
+    510 + 40 and 515 + 40 workgroups, each against the same mask as a rule."""
+    print("case", dtype, seq, batch, flush=True)
+    head = 64
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(seq + batch)
+    Q, K, V = (torch.randn(batch, seq, head, generator=gen, device="cuda").to(H.TORCH_DT[dtype])
+               for _ in range(3))
+    m = H.additive_mask(_mask("causal", seq), dtype).cuda()
+    lse = torch.full((batch, seq), float("-inf"), device="cuda")
+    A = torch.zeros_like(Q)
+    hip_sdpa.flash_sdpa_fwd(K, Q, m, lse, V, A, torch.empty_like(lse), torch.empty_like(Q))
+    lse2 = torch.full((batch, seq), float("-inf"), device="cuda")
+    A2 = torch.zeros_like(Q)
+    hip_sdpa.sdpa_fwd_tile(K, Q, None, lse2, V, A2, hip_sdpa.MASK_CAUSAL)
+    torch.cuda.synchronize()
+    # the same steps in the same order: probabilities and outputs rounded alike
+    # but for the scores' path through the mask addition (fp32, 2^-24 each)
+    assert H.rel_fro(H.to_np(lse), H.to_np(lse2)) < 1e-6
+    assert H.rel_fro(H.to_np(A), H.to_np(A2)) < H.TOL[dtype]
+    worst = (A.float() - A2.float()).norm(dim=-1) / A2.float().norm(dim=-1)
+    assert float(worst.max()) < H.ROW_TOL[dtype]
