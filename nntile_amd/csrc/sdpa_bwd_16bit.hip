@@ -764,14 +764,18 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
         constexpr bool use_mask = EXPLICIT && decltype(masked_tag)::value;
         const int kg0 = g * kBwdStep;
         const int keys_here = min(kBwdStep, k_seq - kg0);
-        const char *mask_step = mask_wg + (int64_t)kg0 * MASK_ES;
+        // (groups of four: offsets count from four keys in front of the step -
+        // where there are keys in front - as a step of fewer than four keys is
+        // read from there on)
+        const uint32_t lead = MASK_GROUPS && kg0 > 0 ? 4u * MASK_ES : 0u;
+        const char *mask_step = mask_wg + (int64_t)kg0 * MASK_ES - lead;
         // (the last place that a group of values, or a value, can start at)
-        const uint32_t mask_off_last = mask_row_off
-            + (uint32_t)max(keys_here - (MASK_GROUPS ? 4 : 1), 0) * MASK_ES;
+        const uint32_t mask_off_last = mask_row_off + lead
+            + (uint32_t)(keys_here - (MASK_GROUPS ? 4 : 1)) * MASK_ES;
         // (through an empty asm statement: the 32 offsets that a step adds
         // constants to are then made where the step uses them instead of once
         // before the loop and kept, which at head 128 means spilled)
-        uint32_t mask_off = mask_off_wg;
+        uint32_t mask_off = mask_off_wg + lead;
         if(use_mask)
         {
             asm volatile("" : "+v"(mask_off));

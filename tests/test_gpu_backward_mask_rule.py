@@ -15,7 +15,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("form", ["additive", "bool"])
 @pytest.mark.parametrize("head", [32, 64, 128])
-@pytest.mark.parametrize("q_seq,k_seq", [(64, 64), (128, 65), (197, 261), (3, 2), (130, 16)])
+@pytest.mark.parametrize("q_seq,k_seq", [(64, 64), (128, 65), (197, 261), (3, 2), (130, 16), (66, 194),
+                                          (130, 131)])
 @pytest.mark.parametrize("flip", [None, (1, 0), (64, 64), (63, 64), (128, 15), (196, 196)])
 def test_rule_blocks(form, head, q_seq, k_seq, flip, batch=2, dtype="fp16"):
     if flip is not None and (flip[0] >= q_seq or flip[1] >= k_seq):
