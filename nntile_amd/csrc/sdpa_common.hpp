@@ -72,13 +72,6 @@ struct PrefillParams
     int32_t xcd_remap;            // 1: regroup workgroups so a slab stays on one XCD
     int32_t overwrite;            // 1: ignore the running pair, write every row
     int32_t n_scan_wgs;
-    // The key axis of a one-tile call shared out over workgroups (n_parts > 1):
-    // part i takes the keys [i * part_keys, + part_keys) and leaves its
-    // unnormalised outputs in part_o [part][batch][q_seq][head] and its
-    // (maximum, sum) pairs in part_ml [part][batch][q_seq][2], in fp32, for
-    // launch_parts_merge.
-    int32_t n_parts, part_keys;
-    float *part_o, *part_ml;
     int32_t form;                 // fp32 launcher: 0 pick by size, 1 shared key steps, 2 split key steps
                                   // 16-bit launcher: 0 pick by size, 1 128-query workgroups, 2 the same with the key steps split over two groups of wavefronts, 8 256-query
     float scale;                  // 1/sqrt(head)
@@ -87,6 +80,13 @@ struct PrefillParams
     const void *Q[kMaxTiles];
     float *lse[kMaxTiles];
     void *A[kMaxTiles];
+    // The key axis of a one-tile call shared out over workgroups (n_parts > 1):
+    // part i takes the keys [i * part_keys, + part_keys) and leaves its
+    // unnormalised outputs in part_o [part][batch][q_seq][head] and its
+    // (maximum, sum) pairs in part_ml [part][batch][q_seq][2], in fp32, for
+    // launch_parts_merge.
+    int32_t n_parts, part_keys;
+    float *part_o, *part_ml;
 };
 
 // The ranges a one-tile call's keys are shared out in: their number (1: not

@@ -230,7 +230,9 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         wg -= (unsigned)part * per_part;
     }
     const int part_k0 = PARTS ? part * p.part_keys : 0;
-    const bool overwrite = PARTS || p.overwrite;
+    // (functions, here and below, so that kernels without ranges read their
+    // arguments where they use them, as if this were not there)
+    auto overwrite = [&]() __attribute__((always_inline)) { return PARTS || p.overwrite; };
     int b, qblk;
     const int batch_all = p.batch * p.n_slabs;
     if(p.xcd_remap)
@@ -271,7 +273,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // the stored logsumexp that the epilogue merges with: requested here, so
     // that its latency passes beside the first loads
     float *lse_ptr = p.lse[q_tile0 + qt] + (int64_t)b * q_len + (q_ok ? my_q : 0);
-    const float lse_stored = overwrite ? neg_inf() : *lse_ptr;
+    const float lse_stored = overwrite() ? neg_inf() : *lse_ptr;
 
     // Q fragments, resident for the whole kernel.
     vec8 qf[KSTEPS];
@@ -309,7 +311,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         const int hi = min(rel0 + min(kQRows, q_len - q_row0) - 1, k_seq - 1);
         if(hi < 0)
         {
-            if(!overwrite)
+            if(!overwrite())
             {
                 return;
             }
@@ -396,7 +398,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     auto slab = [&](int kt) -> int64_t
     {
         const int64_t rows = p.kv_rows > 0 ? p.kv_rows : (int64_t)tile_rows(kt);
-        return ((int64_t)kvb * rows + part_k0) * (HEAD * 2);
+        return (int64_t)kvb * rows * HEAD * 2 + (int64_t)part_k0 * (HEAD * 2);
     };
 
     // Global -> LDS loads of the K (or V) rows of one step.  Rows past the end

@@ -134,10 +134,18 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         wg -= part * per_part;
     }
     const int64_t part_k0 = PARTS ? (int64_t)part * p.part_keys : 0;
-    const int64_t k_seq = PARTS ? min((int64_t)p.part_keys, p.k_seq - part_k0) : p.k_seq;
-    const int64_t k_tile = PARTS ? k_seq : p.k_tile;
-    const int64_t k_pos0 = p.k_pos0 + part_k0;
-    const bool overwrite = PARTS || p.overwrite;
+    // (functions, so that kernels without ranges read their arguments where they
+    // use them, as if this were not there)
+    auto k_seq = [&]() __attribute__((always_inline)) -> int64_t
+    {
+        return PARTS ? min((int64_t)p.part_keys, p.k_seq - part_k0) : p.k_seq;
+    };
+    auto k_tile = [&]() __attribute__((always_inline)) -> int64_t
+    {
+        return PARTS ? k_seq() : p.k_tile;
+    };
+    auto k_pos0 = [&]() __attribute__((always_inline)) -> int64_t { return p.k_pos0 + part_k0; };
+    auto overwrite = [&]() __attribute__((always_inline)) { return PARTS || p.overwrite; };
     int b, qblk;
     if(PARTS)
     {
@@ -211,7 +219,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         }
     }
 
-    const int64_t last_k_len = k_seq - (int64_t)(p.n_kv_tiles - 1) * k_tile;
+    const int64_t last_k_len = k_seq() - (int64_t)(p.n_kv_tiles - 1) * k_tile();
     int n_steps = (p.n_kv_tiles - 1) * p.k_blocks_per_tile
         + (int)((last_k_len + kKeys32 - 1) / kKeys32);
     const int64_t wg_qpos_hi = p.q_pos0 + (int64_t)qt * p.q_tile
@@ -267,7 +275,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         const char *K, *V;      // first row of the step
         int rows_left;          // rows of the tile from this step on
     };
-    const int64_t k_len0 = min(k_tile, k_seq);
+    const int64_t k_len0 = min(k_tile(), k_seq());
     const bool one_tile = p.n_kv_tiles == 1;
     const int64_t entry_rows0 = p.kv_rows > 0 ? p.kv_rows : k_len0;
     const char *K0 = static_cast<const char *>(p.K[k_tile0]) + ((int64_t)kvb * entry_rows0 + part_k0) * RB;
@@ -285,7 +293,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         {
             const int kt = g / p.k_blocks_per_tile;
             const int kb = g % p.k_blocks_per_tile;
-            const int64_t k_len = min(k_tile, k_seq - (int64_t)kt * k_tile);
+            const int64_t k_len = min(k_tile(), k_seq() - (int64_t)kt * k_tile());
             const int64_t off = ((int64_t)kvb * k_len + (int64_t)kb * kKeys32) * RB;
             src.K = static_cast<const char *>(p.K[k_tile0 + kt]) + off;
             src.V = static_cast<const char *>(p.V[k_tile0 + kt]) + off;
@@ -321,19 +329,19 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
 
     if(MODE == NNTILE_HIP_MASK_CAUSAL)
     {
-        const int64_t hi = wg_qpos_hi + p.causal_offset - k_pos0;
+        const int64_t hi = wg_qpos_hi + p.causal_offset - k_pos0();
         if(hi < 0)
         {
-            if(!overwrite)
+            if(!overwrite())
             {
                 return;
             }
             n_steps = 0;    // nothing visible: the epilogue writes empty rows
         }
-        const int64_t kt_hi = hi < 0 ? (int64_t)p.n_kv_tiles : hi / k_tile;
+        const int64_t kt_hi = hi < 0 ? (int64_t)p.n_kv_tiles : hi / k_tile();
         if(kt_hi < p.n_kv_tiles)
         {
-            const int64_t in_tile = hi - kt_hi * k_tile;
+            const int64_t in_tile = hi - kt_hi * k_tile();
             const int steps = (int)(kt_hi * p.k_blocks_per_tile
                     + in_tile / kKeys32 + 1);
             n_steps = min(n_steps, steps);
@@ -350,19 +358,19 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     if constexpr(EXPLICIT)
     {
         constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 4 : 1;
-        if(n_steps > 0 && k_seq * ES >= 16 && p.mask_ld * ES * QROWS < (int64_t)(1 << 30))
+        if(n_steps > 0 && k_seq() * ES >= 16 && p.mask_ld * ES * QROWS < (int64_t)(1 << 30))
         {
             __shared__ unsigned long long scan_words[2 * kThreads32 / 64];
             unsigned long long not_hidden;
             mask_scan_steps<ES, kThreads32 / 64, kKeys32>(static_cast<const char *>(p.mask)
                     + q_row0 * p.mask_ld * ES, (uint32_t)(p.mask_ld * ES),
-                    (int)min((int64_t)QROWS, q_len - q_row0), (int)k_seq * ES, 0, n_steps,
+                    (int)min((int64_t)QROWS, q_len - q_row0), (int)k_seq() * ES, 0, n_steps,
                     (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0u : 0x01010101u,
                     (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0xff800000u : 0u, scan_words, not_open,
                     not_hidden);
             if(not_hidden == 0ull)
             {
-                if(!overwrite)
+                if(!overwrite())
                 {
                     return;
                 }
@@ -404,9 +412,9 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     {
         const int kt = g / p.k_blocks_per_tile;
         const int kb = g % p.k_blocks_per_tile;
-        const int64_t k_len = min(k_tile, k_seq - (int64_t)kt * k_tile);
+        const int64_t k_len = min(k_tile(), k_seq() - (int64_t)kt * k_tile());
         const int64_t k_row0 = (int64_t)kb * kKeys32;
-        const int64_t k_pos_base = k_pos0 + (int64_t)kt * k_tile + k_row0;
+        const int64_t k_pos_base = k_pos0() + (int64_t)kt * k_tile() + k_row0;
         const int keys_here = (int)min((int64_t)kKeys32, k_len - k_row0);
         // Explicit mask: the step's 16 values of this lane are loaded here,
         // ahead of the chain of MFMAs.  Register r holds key
@@ -651,7 +659,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         }
         const int kt = g / p.k_blocks_per_tile;
         const int kb = g % p.k_blocks_per_tile;
-        const int64_t k_pos_base = k_pos0 + (int64_t)kt * k_tile + (int64_t)kb * kKeys32;
+        const int64_t k_pos_base = k_pos0() + (int64_t)kt * k_tile() + (int64_t)kb * kKeys32;
         return k_pos_base > wave_qpos_hi + p.causal_offset;
     };
 
@@ -989,14 +997,14 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         }
         return;
     }
-    if(!q_ok || (empty && !overwrite))
+    if(!q_ok || (empty && !p.overwrite))
     {
         return;     // leave lse and A as they are
     }
     const float to_ln = EXPLICIT ? 1.0f : p.scale;
     const float lse_new = empty ? neg_inf() : m_run * to_ln + __logf(l_tot);
     float *lse_ptr = p.lse[q_tile0 + qt] + (int64_t)b * q_len + my_q;
-    const float lse_old = overwrite ? neg_inf() : *lse_ptr;
+    const float lse_old = p.overwrite ? neg_inf() : *lse_ptr;
     float w_old = 0.0f, w_new = 0.0f, lse_out = neg_inf();
     if(!empty)
     {
