@@ -61,16 +61,18 @@ __device__ __forceinline__ bool decode_place(const DecodeParams &p, int &unit, i
 }
 
 // The partial is complete in this XCD's L2 once every wavefront's stores have
-// been acknowledged (the barrier's release waits for them); then one flag per
-// merge workgroup of the unit goes up, with the number of this XCD in its low
-// bits.
+// been acknowledged.  Each wavefront waits for its own in front of the barrier:
+// the barrier itself waits for no memory operation, it is a bare s_barrier
+// within a workgroup.  Behind it one flag per merge workgroup of the unit goes
+// up, with the number of this XCD in its low bits.
 __device__ __forceinline__ void decode_raise_flags(const DecodeParams &p, int unit, int split)
 {
-    __syncthreads();
     if(p.fenced)
     {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
     const int tid = threadIdx.x;
     if(tid < p.merge_blocks_per_unit)
     {

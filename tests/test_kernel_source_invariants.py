@@ -132,3 +132,35 @@ def test_backward_kernels_use_no_scratch_memory_without_an_explicit_mask(assembl
         explicit = mode in (0, 3)           # NNTILE_HIP_MASK_ADDITIVE, NNTILE_HIP_MASK_BOOL
         assert size <= (112 if explicit and head == 128 else 0), (name, size)
     assert seen >= 48
+
+
+def test_decode_partials_have_arrived_before_their_flag_goes_up(assemblies):
+    """A merge workgroup reads another workgroup's partial as soon as it sees
+    the flag, which one wavefront stores for all four.  A workgroup barrier
+    waits for no memory operation on this target, so every wavefront has to
+    wait for its own stores in front of the barrier that precedes the flag: in
+    straight-line code (every wavefront passes it, whatever branch it came by)
+    and with no store in between."""
+    for name in ("sdpa_decode_16bit.hip", "sdpa_decode_fp32.hip"):
+        lines = [l.split(";")[0].strip() for l in assemblies[name].splitlines()]
+        lines = [l for l in lines if l and (not l.startswith(".") or l.startswith(".LBB"))]
+        raised = 0
+        for i, line in enumerate(lines):
+            # the flag: the first store behind the XCD's number that the L2 serves
+            if "HW_REG_XCC_ID" not in line:
+                continue
+            stores = [j for j in range(i, min(i + 30, len(lines)))
+                      if lines[j].startswith("global_store")]
+            if not stores:
+                continue                    # the merge workgroup compares the number
+            assert re.match(r"global_store_dwordx2 .* sc1$", lines[stores[0]]), (name, lines[stores[0]])
+            b = max(j for j in range(i) if lines[j] == "s_barrier")
+            assert not any("store" in l for l in lines[b:i]), (name, lines[b:i])
+            j = b - 1
+            while not lines[j].startswith(("global_", "flat_", "buffer_", "scratch_", "s_cbranch",
+                                           "s_branch", ".LBB", "s_waitcnt vmcnt(0)")):
+                j -= 1
+            assert lines[j].startswith("s_waitcnt vmcnt(0)"), (name, lines[j:b + 1])
+            raised += 1
+        kernels = re.findall(r"^(_ZN\S+_kernel\S+Lb0E\S*):", assemblies[name], re.M)
+        assert raised == len(kernels) > 0, (name, raised, len(kernels))
