@@ -43,7 +43,13 @@ extern "C" {
 /* The running pair is taken to be empty: lse and A are not read, every query
  * row of the call is written, rows without a visible key get lse = -inf and
  * A = 0.  Saves the fill of lse (wrappers/python/nntile/layer/sdpa.py:538-539)
- * and one read of A when the caller knows this is the first key tile. */
+ * and one read of A when the caller knows this is the first key tile.
+ *
+ * A query row with a NaN (or a score of +inf) among its visible scores becomes
+ * NaN in lse and A, whichever route the call takes.  Merging into a running
+ * pair, the decode entry points do the same; the tile and grid entry points
+ * leave the pair of such a row as it was, as the reference's merge does
+ * (src/kernel/accumulate_attn_output/cuda.cu:43-50). */
 #define NNTILE_HIP_SDPA_OVERWRITE 1
 /* Tile and grid calls, for tests and tuning: fix the workgroup shape instead
  * of letting the size of the launch pick it.  fp32: 128 queries sharing every

@@ -883,7 +883,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
         const int64_t qb = nb + (int64_t)p.n_batch * (g + (int64_t)p.kv_group * hkv);
         const int64_t row = qb * p.q_seq + tok;
         uint16_t *Adst = static_cast<uint16_t *>(p.A) + row * HEAD + 4 * quad;
-        if(m_run == neg_inf() || !(l_tot > 0.0f))
+        if(l_tot == 0.0f)
         {
             // no visible key at all: leave lse and A untouched, or write the
             // empty row when the running pair is being overwritten
@@ -937,9 +937,11 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
     const int64_t prow = ((int64_t)unit * p.n_splits + split) * p.rows + rr;
     if(quad == 0)
     {
-        // max in natural-log units so that the reduce kernel needs no mode
+        // max in natural-log units so that the reduce kernel needs no mode.  A
+        // row all of whose scores are NaN has no maximum, but a sum that is NaN:
+        // it is not one that sees no key, and its maximum goes out as 0.
         const float to_ln = EXPLICIT ? 1.0f : p.scale;
-        p.part_ml[2 * prow] = (m_run == neg_inf()) ? neg_inf() : m_run * to_ln;
+        p.part_ml[2 * prow] = l_tot == 0.0f ? neg_inf() : l_tot > 0.0f ? m_run * to_ln : 0.0f;
         p.part_ml[2 * prow + 1] = l_tot;
     }
     // o[db][r] is head value 16*db + 4*quad + r of row rr

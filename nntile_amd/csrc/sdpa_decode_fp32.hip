@@ -116,8 +116,11 @@ __device__ __forceinline__ void f32dec_merge_row(const DecodeParams &p, int unit
 #pragma unroll
     for(int i = 0; i < NC; ++i)
     {
-        const bool there = t + i * TPR <= last_split && ml[i][0] != neg_inf() && ml[i][1] > 0.0f;
-        w[i] = there ? ml[i][0] + __logf(ml[i][1]) : neg_inf();     // the split's logsumexp
+        // the split's logsumexp; one whose sum is NaN takes the top place, from
+        // where it makes the row's weights NaN (a maximum passes a NaN over)
+        const bool there = t + i * TPR <= last_split && ml[i][1] != 0.0f;
+        w[i] = !there ? neg_inf() : ml[i][1] > 0.0f ? ml[i][0] + __logf(ml[i][1])
+            : __builtin_huge_valf();
         top = fmaxf(top, w[i]);
     }
 #pragma unroll
@@ -583,7 +586,7 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
         const int64_t row = f32dec_row(p, unit, rr);
         float *dst = static_cast<float *>(p.A) + row * HEAD + 4 * quad;
         // (no visible key at all: lse and A stay, or the empty row is written)
-        const bool empty = m_run == neg_inf() || !(l_tot > 0.0f);
+        const bool empty = l_tot == 0.0f;
         if(empty && !p.overwrite)
         {
             return;
@@ -617,7 +620,7 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
         const int64_t prow = ((int64_t)unit * p.n_splits + split) * p.rows + rr;
         if(quad == 0)
         {
-            p.part_ml[2 * prow] = (m_run == neg_inf()) ? neg_inf() : m_run * to_ln;
+            p.part_ml[2 * prow] = l_tot == 0.0f ? neg_inf() : m_run * to_ln;
             p.part_ml[2 * prow + 1] = l_tot;
         }
         float *dst = p.part_o + prow * HEAD + 4 * quad;

@@ -130,9 +130,10 @@ void sdpa_parts_merge_kernel(const PrefillParams p)
         top = m_new;
     }
     auto *dst = static_cast<typename PartsOut<T>::elem *>(p.A[0]) + row * HEAD + d4;
-    if(!(l > 0.0f))
+    // (a row with a NaN among its scores: as the kernels without ranges do it)
+    if(l == 0.0f || (!(l > 0.0f) && !p.overwrite))
     {
-        // no visible key: as the kernels without ranges leave such a row
+        // no visible key
         if(p.overwrite)
         {
             PartsOut<T>::store(dst, f32x4{0.0f, 0.0f, 0.0f, 0.0f});

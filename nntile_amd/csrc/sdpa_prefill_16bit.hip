@@ -1509,18 +1509,19 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
 
     // ---- epilogue: normalise, merge into the running (lse, A) ----------------
     const float l_tot = sum_across_halves(l_run);
-    const bool empty = !(l_tot > 0.0f);     // no visible key for this query
+    // no visible key for this query.  A score that is NaN makes the sum NaN: such
+    // a row is NaN where (lse, A) are overwritten, and is not merged into a
+    // running pair (src/kernel/accumulate_attn_output/cuda.cu:43-50).
+    const bool empty = l_tot == 0.0f;
     if constexpr(PARTS)
     {
         if(q_ok)
         {
-            // (a sum that is no number stays one: the merged row is then empty,
-            // as it is without parts)
-            const bool none = l_tot == 0.0f;
+            // (a sum that is NaN goes out as it is, with some finite maximum)
             const int64_t row = ((int64_t)part * p.batch + b) * p.q_seq + my_q;
             if(half == 0)
             {
-                p.part_ml[2 * row] = none ? neg_inf() : empty ? 0.0f : m_run * p.scale;
+                p.part_ml[2 * row] = empty ? neg_inf() : l_tot > 0.0f ? m_run * p.scale : 0.0f;
                 p.part_ml[2 * row + 1] = l_tot;
             }
             float *dst = p.part_o + row * HEAD + 4 * half;
@@ -1534,7 +1535,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
 #pragma unroll
                     for(int e = 0; e < 4; ++e)
                     {
-                        v[e] = none ? 0.0f : o[db][4 * rg + e];
+                        v[e] = empty ? 0.0f : o[db][4 * rg + e];
                     }
                     *reinterpret_cast<f32x4 *>(dst + 32 * db + 8 * rg) = v;
                 }
@@ -1543,7 +1544,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         return;
     }
     // rows that are written; the others leave lse and A as they are
-    const bool live = q_ok && !(empty && !p.overwrite);
+    const bool live = q_ok && (l_tot > 0.0f || p.overwrite);
     const float to_ln = p.scale;
     const float lse_new = empty ? neg_inf() : m_run * to_ln + __logf(l_tot);
     const float lse_old = live ? lse_stored : neg_inf();

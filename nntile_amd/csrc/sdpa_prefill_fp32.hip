@@ -965,17 +965,17 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     // ---- epilogue --------------------------------------------------------------
     F32_STAMP(45)
     const float l_tot = l_run + __shfl_xor(l_run, 32);
-    const bool empty = !(l_tot > 0.0f);     // no visible key for this query
+    // no visible key for this query (a NaN among its scores: as in the 16-bit kernel)
+    const bool empty = l_tot == 0.0f;
     if constexpr(PARTS)
     {
         if(q_ok)
         {
-            // (a sum that is no number stays one, as in the 16-bit kernel)
-            const bool none = l_tot == 0.0f;
+            // (a sum that is NaN goes out as it is, with some finite maximum)
             const int64_t row = ((int64_t)part * p.batch + b) * p.q_seq + my_q;
             if(half == 0)
             {
-                p.part_ml[2 * row] = none ? neg_inf() : empty ? 0.0f : m_run * p.scale;
+                p.part_ml[2 * row] = empty ? neg_inf() : l_tot > 0.0f ? m_run * p.scale : 0.0f;
                 p.part_ml[2 * row + 1] = l_tot;
             }
             float *dst = p.part_o + row * HEAD + 4 * half;
@@ -989,7 +989,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
 #pragma unroll
                     for(int e = 0; e < 4; ++e)
                     {
-                        v[e] = none ? 0.0f : o[db][4 * rg + e];
+                        v[e] = empty ? 0.0f : o[db][4 * rg + e];
                     }
                     *reinterpret_cast<f32x4 *>(dst + 32 * db + 8 * rg) = v;
                 }
@@ -997,7 +997,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         }
         return;
     }
-    if(!q_ok || (empty && !p.overwrite))
+    if(!q_ok || !(l_tot > 0.0f || p.overwrite))
     {
         return;     // leave lse and A as they are
     }
