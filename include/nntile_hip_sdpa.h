@@ -313,7 +313,9 @@ int nntile_hip_sdpa_bwd_grid_fp16(void *stream, const nntile_hip_sdpa_bwd_grid_a
  * the accumulate_attn_output rule.  args->q_seq*kv_group must be <= 64.
  * workspace: device memory of at least
  * nntile_hip_sdpa_fwd_decode_workspace_bytes(args) bytes, private to the call
- * until the stream has passed it (a STARPU_SCRATCH buffer in NNTile terms). */
+ * until the stream has passed it (a STARPU_SCRATCH buffer in NNTile terms).
+ * The size never falls as k_seq grows: a workspace sized for the longest cache
+ * serves every shorter one. */
 size_t nntile_hip_sdpa_fwd_decode_workspace_bytes(const nntile_hip_sdpa_tile_args *args);
 int nntile_hip_sdpa_fwd_decode_bf16(void *stream, const nntile_hip_sdpa_tile_args *args,
         void *workspace, size_t workspace_bytes);

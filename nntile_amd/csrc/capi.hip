@@ -22,6 +22,7 @@ int launch_parts_merge(hipStream_t stream, const PrefillParams &p, int head);
 template<typename T>
 int launch_decode_16bit(hipStream_t stream, DecodeParams &p, int head, int mode);
 int decode_choose_splits(int units, int n_steps);
+int decode_most_splits(int units, int n_steps);
 template<typename T>
 int launch_bwd_16bit(hipStream_t stream, const BwdParams &p, int head, int mode);
 template<typename T>
@@ -33,6 +34,7 @@ size_t decode_partial_ml_bytes(int units, int n_splits, int rows);
 int launch_decode_fp32(hipStream_t stream, DecodeParams &p, int head, int mode);
 int decode_fp32_steps(int64_t k_seq);
 int decode_fp32_choose_splits(int units, int n_steps, int head);
+int decode_fp32_most_splits(int units, int n_steps, int head);
 size_t decode_fp32_workspace_bytes(int units, int n_splits, int rows, int head);
 size_t decode_fp32_partial_bytes(int units, int n_splits, int rows, int head);
 
@@ -1185,7 +1187,7 @@ size_t nntile_hip_sdpa_fwd_decode_workspace_bytes(const nntile_hip_sdpa_tile_arg
     }
     int units, n_steps, splits, rows;
     decode_geometry(args, units, n_steps, splits, rows);
-    return decode_workspace_bytes(units, splits, rows, (int)args->head);
+    return decode_workspace_bytes(units, decode_most_splits(units, n_steps), rows, (int)args->head);
 }
 
 int nntile_hip_sdpa_fwd_decode_bf16(void *stream, const nntile_hip_sdpa_tile_args *args,
@@ -1210,7 +1212,8 @@ size_t nntile_hip_sdpa_fwd_decode_workspace_bytes_fp32(const nntile_hip_sdpa_til
     }
     int units, n_steps, splits, rows;
     decode_fp32_geometry(args, units, n_steps, splits, rows);
-    return decode_fp32_workspace_bytes(units, splits, rows, (int)args->head);
+    return decode_fp32_workspace_bytes(units,
+            decode_fp32_most_splits(units, n_steps, (int)args->head), rows, (int)args->head);
 }
 
 int nntile_hip_sdpa_fwd_decode_fp32(void *stream, const nntile_hip_sdpa_tile_args *args,

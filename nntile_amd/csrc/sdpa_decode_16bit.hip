@@ -1187,17 +1187,26 @@ bool decode_uneven_units(int units, int64_t k_seq, int64_t row_bytes)
 // (8 units of 63 steps: 64 splits 13.0 us, 32 splits 10.3).
 int decode_choose_splits(int units, int n_steps)
 {
-    constexpr int kDirectSteps = 3, kSingleSteps = 8;
-    if(n_steps <= kDirectSteps)
+    if(n_steps <= kDecodeDirectSteps)
     {
         return 1;
     }
     int splits = decode_splits_by_units(units, NNTILE_DEC_WGS_PER_CU * kDecodeCUs);
-    const int most = n_steps <= kSingleSteps ? n_steps : (n_steps + 1) / 2;
+    const int most = n_steps <= kDecodeSingleSteps ? n_steps : (n_steps + 1) / 2;
     splits = splits < 1 ? 1 : splits;
     splits = splits > most ? most : splits;
     splits = splits > 64 ? 64 : splits;
     return splits;
+}
+
+// Most splits that a unit of at most n_steps steps takes: the workspace is sized
+// for these, so that one sized for the longest cache serves all shorter ones.
+int decode_most_splits(int units, int n_steps)
+{
+    const int here = decode_choose_splits(units, n_steps);
+    const int before = decode_choose_splits(units,
+            n_steps < kDecodeSingleSteps ? n_steps : kDecodeSingleSteps);
+    return here > before ? here : before;
 }
 
 // The workspace: the partial outputs [unit][split][rows][head], then the

@@ -664,15 +664,23 @@ int decode_fp32_steps(int64_t k_seq)
 // 16-bit kernel (handing partials over costs 2 us, a step about 1).
 int decode_fp32_choose_splits(int units, int n_steps, int head)
 {
-    constexpr int kDirectSteps = 3, kSingleSteps = 8;
-    if(n_steps <= kDirectSteps)
+    if(n_steps <= kDecodeDirectSteps)
     {
         return 1;
     }
     const int by_units = decode_splits_by_units(units, (head <= 64 ? 3 : 2) * kDecF32CUs);
-    const int most = n_steps <= kSingleSteps ? n_steps : (n_steps + 1) / 2;
+    const int most = n_steps <= kDecodeSingleSteps ? n_steps : (n_steps + 1) / 2;
     const int splits = by_units < most ? by_units : most;
     return splits > 64 ? 64 : splits;
+}
+
+// (see decode_most_splits)
+int decode_fp32_most_splits(int units, int n_steps, int head)
+{
+    const int here = decode_fp32_choose_splits(units, n_steps, head);
+    const int before = decode_fp32_choose_splits(units,
+            n_steps < kDecodeSingleSteps ? n_steps : kDecodeSingleSteps, head);
+    return here > before ? here : before;
 }
 
 // The workspace: the partial outputs [unit][split][rows][head] and the (max,

@@ -16,6 +16,10 @@ int decode_sync_stride(int n_splits, int rows, int head);
 // Key splits per unit of a launch of which the chip holds `places` workgroups
 // at once, before the limits that the number of key steps sets.
 int decode_splits_by_units(int units, int places);
+// Where the number of splits of a unit may fall as its key steps grow: up to
+// kDecodeDirectSteps one workgroup takes all, up to kDecodeSingleSteps a split
+// takes one step, beyond that at least two.
+constexpr int kDecodeDirectSteps = 3, kDecodeSingleSteps = 8;
 // Whether the units' shares of the XCDs differ too much for the merge to ride
 // in the launch; row_bytes: of K and V together.
 bool decode_uneven_units(int units, int64_t k_seq, int64_t row_bytes);
