@@ -155,6 +155,21 @@ PyObject *guarded(Py_ssize_t given, Py_ssize_t wanted, F body)
     }
 }
 
+// The C call itself, without the interpreter's lock: a launch into a full queue
+// blocks, and neither the other threads nor a host function ahead of it in the
+// stream that wants the lock may wait for it.
+// The arguments have been worked out by then, so nothing in here needs Python.
+template<typename F, typename... A>
+int unlocked(F fn, A... args)
+{
+    struct Released
+    {
+        PyThreadState *state = PyEval_SaveThread();
+        ~Released() { PyEval_RestoreThread(state); }
+    } released;
+    return fn(args...);
+}
+
 typedef int (*tile_fn)(void *, const nntile_hip_sdpa_tile_args *);
 typedef int (*tile_cache_fn)(void *, const nntile_hip_sdpa_tile_args *, int64_t);
 typedef int (*decode_fn)(void *, const nntile_hip_sdpa_tile_args *, void *, size_t);
@@ -181,12 +196,12 @@ int append_call(Type ty, void *s, const nntile_hip_sdpa_tile_args *a, int64_t ca
     const int64_t rows = k_new.size(1);
     if(ty == FP32)
     {
-        return nntile_hip_sdpa_fwd_decode_append_cache_fp32(s, a, capacity,
+        return unlocked(nntile_hip_sdpa_fwd_decode_append_cache_fp32, s, a, capacity,
                 static_cast<const float *>(k_new.data_ptr()),
                 static_cast<const float *>(v_new.data_ptr()), rows, ptr(ws), nbytes(ws));
     }
-    return (ty == BF16 ? nntile_hip_sdpa_fwd_decode_append_cache_bf16
-            : nntile_hip_sdpa_fwd_decode_append_cache_fp16)(s, a, capacity,
+    return unlocked(ty == BF16 ? nntile_hip_sdpa_fwd_decode_append_cache_bf16
+            : nntile_hip_sdpa_fwd_decode_append_cache_fp16, s, a, capacity,
                 static_cast<const uint16_t *>(k_new.data_ptr()),
                 static_cast<const uint16_t *>(v_new.data_ptr()), rows, ptr(ws), nbytes(ws));
 }
@@ -242,7 +257,7 @@ PyObject *fwd_tile(PyObject *, PyObject *const *v, Py_ssize_t n)
     {
         nntile_hip_sdpa_tile_args a;
         const Type ty = read_tile_call(a, v);
-        return tile_fns[ty](stream_of(v[13]), &a);
+        return unlocked(tile_fns[ty], stream_of(v[13]), &a);
     });
 }
 
@@ -259,7 +274,7 @@ PyObject *fwd_tile_cache(PyObject *, PyObject *const *v, Py_ssize_t n)
             return NNTILE_HIP_EINVAL;
         }
         a.k_seq = integer(v[13]);
-        return tile_cache_fns[ty](stream_of(v[14]), &a, capacity);
+        return unlocked(tile_cache_fns[ty], stream_of(v[14]), &a, capacity);
     });
 }
 
@@ -277,7 +292,7 @@ PyObject *fwd_tile_cache_ws(PyObject *, PyObject *const *v, Py_ssize_t n)
             return NNTILE_HIP_EINVAL;
         }
         a.k_seq = integer(v[13]);
-        return tile_cache_ws_fns[ty](stream_of(v[15]), &a, capacity, ptr(ws), nbytes(ws));
+        return unlocked(tile_cache_ws_fns[ty], stream_of(v[15]), &a, capacity, ptr(ws), nbytes(ws));
     });
 }
 
@@ -308,7 +323,7 @@ PyObject *fwd_decode(PyObject *, PyObject *const *v, Py_ssize_t n)
         nntile_hip_sdpa_tile_args a;
         const at::Tensor *ws = maybe_tile(v[13]);
         const Type ty = read_tile_call(a, v);
-        return decode_fns[ty](stream_of(v[14]), &a, ptr(ws), nbytes(ws));
+        return unlocked(decode_fns[ty], stream_of(v[14]), &a, ptr(ws), nbytes(ws));
     });
 }
 
@@ -326,7 +341,7 @@ PyObject *fwd_decode_cache(PyObject *, PyObject *const *v, Py_ssize_t n)
             return NNTILE_HIP_EINVAL;
         }
         a.k_seq = integer(v[13]);
-        return decode_cache_fns[ty](stream_of(v[15]), &a, capacity, ptr(ws), nbytes(ws));
+        return unlocked(decode_cache_fns[ty], stream_of(v[15]), &a, capacity, ptr(ws), nbytes(ws));
     });
 }
 
@@ -425,19 +440,19 @@ PyObject *kv_append(PyObject *, PyObject *const *v, Py_ssize_t n)
         switch(ty)
         {
             case BF16:
-                return nntile_hip_kv_cache_append_bf16(s, head, rows, entries, capacity, filled,
+                return unlocked(nntile_hip_kv_cache_append_bf16, s, head, rows, entries, capacity, filled,
                         static_cast<const uint16_t *>(k_new.data_ptr()),
                         static_cast<const uint16_t *>(v_new.data_ptr()),
                         static_cast<uint16_t *>(K.data_ptr()),
                         static_cast<uint16_t *>(V.data_ptr()));
             case FP16:
-                return nntile_hip_kv_cache_append_fp16(s, head, rows, entries, capacity, filled,
+                return unlocked(nntile_hip_kv_cache_append_fp16, s, head, rows, entries, capacity, filled,
                         static_cast<const uint16_t *>(k_new.data_ptr()),
                         static_cast<const uint16_t *>(v_new.data_ptr()),
                         static_cast<uint16_t *>(K.data_ptr()),
                         static_cast<uint16_t *>(V.data_ptr()));
             default:
-                return nntile_hip_kv_cache_append_fp32(s, head, rows, entries, capacity, filled,
+                return unlocked(nntile_hip_kv_cache_append_fp32, s, head, rows, entries, capacity, filled,
                         static_cast<const float *>(k_new.data_ptr()),
                         static_cast<const float *>(v_new.data_ptr()),
                         static_cast<float *>(K.data_ptr()), static_cast<float *>(V.data_ptr()));
@@ -466,14 +481,14 @@ PyObject *flash_fwd(PyObject *, PyObject *const *v, Py_ssize_t n)
         float *l = static_cast<float *>(lse.data_ptr()), *sl = static_cast<float *>(ptr(s_lse));
         if(ty == FP32)
         {
-            return nntile_hip_flash_sdpa_fwd_fp32(s, seq, head, batch,
+            return unlocked(nntile_hip_flash_sdpa_fwd_fp32, s, seq, head, batch,
                     static_cast<const float *>(K.data_ptr()),
                     static_cast<const float *>(Q.data_ptr()),
                     static_cast<const float *>(ptr(mask)), sl,
                     static_cast<const float *>(V.data_ptr()), static_cast<float *>(ptr(s_A)), l,
                     static_cast<float *>(A.data_ptr()));
         }
-        return (ty == BF16 ? nntile_hip_flash_sdpa_fwd_bf16 : nntile_hip_flash_sdpa_fwd_fp16)(
+        return unlocked(ty == BF16 ? nntile_hip_flash_sdpa_fwd_bf16 : nntile_hip_flash_sdpa_fwd_fp16,
                 s, seq, head, batch, static_cast<const uint16_t *>(K.data_ptr()),
                 static_cast<const uint16_t *>(Q.data_ptr()),
                 static_cast<const uint16_t *>(ptr(mask)), sl,
@@ -496,7 +511,7 @@ PyObject *flash_bwd(PyObject *, PyObject *const *v, Py_ssize_t n)
         rank3(Q);
         const Type ty = type_of(v[1], Q, false);
         auto p = [&](int i) { return static_cast<uint16_t *>(ptr(t[i])); };
-        return (ty == BF16 ? nntile_hip_flash_sdpa_bwd_bf16 : nntile_hip_flash_sdpa_bwd_fp16)(
+        return unlocked(ty == BF16 ? nntile_hip_flash_sdpa_bwd_bf16 : nntile_hip_flash_sdpa_bwd_fp16,
                 stream_of(v[11]), Q.size(1), Q.size(2), Q.size(0), p(0), p(1), p(2), p(3), p(4),
                 p(5), static_cast<const float *>(ptr(t[6])), nullptr, p(7), nullptr, p(8), p(9),
                 p(10));
@@ -541,7 +556,7 @@ PyObject *bwd_tile(PyObject *, PyObject *const *v, Py_ssize_t n)
         a.dV = ptr(t[9]);
         a.workspace = ptr(t[10]);
         a.workspace_bytes = nbytes(t[10]);
-        return bwd_fns[type_of(v[1], Q, false)](stream_of(v[18]), &a);
+        return unlocked(bwd_fns[type_of(v[1], Q, false)], stream_of(v[18]), &a);
     });
 }
 
@@ -559,12 +574,12 @@ PyObject *accumulate(PyObject *, PyObject *const *v, Py_ssize_t n)
         float *dst_lse = static_cast<float *>(dl.data_ptr());
         if(ty == FP32)
         {
-            return nntile_hip_accumulate_attn_output_fp32(s, head, seq, batch, src_lse,
+            return unlocked(nntile_hip_accumulate_attn_output_fp32, s, head, seq, batch, src_lse,
                     static_cast<const float *>(sa.data_ptr()), dst_lse,
                     static_cast<float *>(da.data_ptr()));
         }
-        return (ty == BF16 ? nntile_hip_accumulate_attn_output_bf16
-                : nntile_hip_accumulate_attn_output_fp16)(s, head, seq, batch, src_lse,
+        return unlocked(ty == BF16 ? nntile_hip_accumulate_attn_output_bf16
+                : nntile_hip_accumulate_attn_output_fp16, s, head, seq, batch, src_lse,
                     static_cast<const uint16_t *>(sa.data_ptr()), dst_lse,
                     static_cast<uint16_t *>(da.data_ptr()));
     });
@@ -593,7 +608,7 @@ PyObject *rope(PyObject *, PyObject *const *v, Py_ssize_t n_args)
         void *s = stream_of(v[5]);
         if(ty == FP32)
         {
-            return (backward ? nntile_hip_rope_backward_fp32 : nntile_hip_rope_fp32)(s, m, n,
+            return unlocked(backward ? nntile_hip_rope_backward_fp32 : nntile_hip_rope_fp32, s, m, n,
                     static_cast<const float *>(sin.data_ptr()),
                     static_cast<const float *>(cos.data_ptr()),
                     static_cast<const float *>(src.data_ptr()),
@@ -602,7 +617,7 @@ PyObject *rope(PyObject *, PyObject *const *v, Py_ssize_t n_args)
         const auto fn = ty == BF16
             ? (backward ? nntile_hip_rope_backward_bf16 : nntile_hip_rope_bf16)
             : (backward ? nntile_hip_rope_backward_fp16 : nntile_hip_rope_fp16);
-        return fn(s, m, n, static_cast<const uint16_t *>(sin.data_ptr()),
+        return unlocked(fn, s, m, n, static_cast<const uint16_t *>(sin.data_ptr()),
                 static_cast<const uint16_t *>(cos.data_ptr()),
                 static_cast<const uint16_t *>(src.data_ptr()),
                 static_cast<uint16_t *>(dst.data_ptr()));
@@ -629,11 +644,11 @@ PyObject *transpose(PyObject *, PyObject *const *v, Py_ssize_t n_args)
         void *s = stream_of(v[5]);
         if(ty == FP32)
         {
-            return nntile_hip_transpose_fp32(s, m, n, (float)alpha,
+            return unlocked(nntile_hip_transpose_fp32, s, m, n, (float)alpha,
                     static_cast<const float *>(src.data_ptr()),
                     static_cast<float *>(dst.data_ptr()));
         }
-        return (ty == BF16 ? nntile_hip_transpose_bf16 : nntile_hip_transpose_fp16)(s, m, n,
+        return unlocked(ty == BF16 ? nntile_hip_transpose_bf16 : nntile_hip_transpose_fp16, s, m, n,
                 (float)alpha, static_cast<const uint16_t *>(src.data_ptr()),
                 static_cast<uint16_t *>(dst.data_ptr()));
     });
@@ -691,14 +706,14 @@ PyObject *launch_call(PyObject *self_, PyObject *stream)
         {
             case 0:
                 // tile, grid and backward calls: (stream, block)
-                return reinterpret_cast<int (*)(void *, const void *)>(self->fn)(s, self->args);
+                return unlocked(reinterpret_cast<int (*)(void *, const void *)>(self->fn), s, self->args);
             case 2:
-                return reinterpret_cast<decode_fn>(self->fn)(s, ta, p(0), (size_t)self->extra[1]);
+                return unlocked(reinterpret_cast<decode_fn>(self->fn), s, ta, p(0), (size_t)self->extra[1]);
             case 3:
-                return reinterpret_cast<decode_cache_fn>(self->fn)(s, ta, self->extra[0], p(1),
+                return unlocked(reinterpret_cast<decode_cache_fn>(self->fn), s, ta, self->extra[0], p(1),
                         (size_t)self->extra[2]);
             default:
-                return reinterpret_cast<append_fn>(self->fn)(s, ta, self->extra[0], p(1), p(2),
+                return unlocked(reinterpret_cast<append_fn>(self->fn), s, ta, self->extra[0], p(1), p(2),
                         self->extra[3], p(4), (size_t)self->extra[5]);
         }
     });

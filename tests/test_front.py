@@ -1,8 +1,16 @@
 """The native front-end of the binding refuses what is not a device tile with
 the exceptions its Python wrappers document (no GPU needed)."""
+import ctypes
+import os
+import re
+import threading
+import time
+import types
+
 import pytest
 import torch
 
+from nntile_amd import build as B
 from nntile_amd import hip_sdpa as h
 from nntile_amd.kv_cache import KVCache
 
@@ -43,3 +51,37 @@ def test_a_step_into_a_cache_off_the_device_is_refused():
     with pytest.raises(ValueError, match="contiguous device tensors"):
         cache.append_attend(one, one, one, torch.zeros(2, 1), one, 2, 1)
     assert len(cache) == 0
+
+
+def test_the_interpreter_lock_is_released_during_the_c_call():
+    """A prepared call of sem_timedwait, given up by this thread while another
+    one is inside it: with the lock held, nobody could, and the wait would time
+    out.  (A launch into a full queue blocks just so.)"""
+    libc = ctypes.CDLL(None)
+    sem = ctypes.create_string_buffer(64)       # (larger than any sem_t)
+    assert libc.sem_init(sem, 0, 0) == 0
+    until = (ctypes.c_long * 2)(int(time.time()) + 10, 0)
+    call = h._native().Launch(ctypes.cast(libc.sem_timedwait, ctypes.c_void_p).value,
+                              ctypes.addressof(until), ()).call
+    inside, got = threading.Event(), []
+
+    def wait():
+        inside.set()
+        got.append(call(types.SimpleNamespace(cuda_stream=ctypes.addressof(sem))))
+
+    t = threading.Thread(target=wait)
+    t.start()
+    inside.wait()
+    time.sleep(0.2)         # (long enough for the thread to be in the call)
+    libc.sem_post(sem)
+    t.join()
+    assert got == [0]
+
+
+def test_every_launch_goes_through_the_form_that_releases_the_lock():
+    with open(os.path.join(B.CSRC, "front.cpp")) as f:
+        text = f.read()
+    called = set(re.findall(r"\b(nntile_hip_\w+)\(", text))
+    assert called == {"nntile_hip_sdpa_fwd_decode_workspace_bytes_fp32",
+                      "nntile_hip_sdpa_fwd_decode_workspace_bytes"}
+    assert not re.search(r"_fns\[[^]]*\]\(|\)\(s\b|fn\(s\b", text)
