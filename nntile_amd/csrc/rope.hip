@@ -12,11 +12,15 @@
 // four neighbouring pairs - 16 bytes of a 16-bit tensor, 32 of an fp32 one -
 // of COLS columns j and the four sines and cosines that go with them, which it
 // so reads once for all of them (read again for every column they are as many
-// bytes from L2 as the tensor has); the grid has one axis for i and one for j,
-// so that nothing is divided (a 64-bit remainder per thread before).  m not a
-// multiple of 4, or addresses that are not aligned for that, take one pair per
-// thread.  2 x 131072 x 32 bf16 (34.1 MB) 7.9 -> 6.6 us = 5.2 TB/s; two columns against
-// four: 6.6 and 7.1 us there, 14.9 and 15.6 on 2 x 524288 x 8 fp32.
+// bytes from L2 as the tensor has).  Threads are numbered through all columns,
+// whatever their length, so that none is left over at a column's end (with
+// workgroups that kept to one column, 2 x 64 x 65536 took 18.6 us, so 6.9; 2 x 4 x
+// 2^20 217, so 7.3; 2 x 1028 x 16320 33.2, so 23.8), and a thread's column is a
+// multiplication and a shift (a 64-bit remainder before).  m not a multiple of
+// 4, or addresses that are not aligned for that, take one pair per thread.
+// bf16, one and two columns a thread: 2 x 65536 x 64 (33.6 MB) 7.3 and 6.9 us =
+// 4.9 TB/s, 2 x 65536 x 256 24.0 and 22.3 = 6.0 TB/s; fp32 2 x 65536 x 256 55.1 and
+// 52.6.
 #include "sdpa_common.hpp"
 
 namespace nntile_hip
@@ -41,6 +45,26 @@ struct RopeFp16
     static __device__ __forceinline__ uint16_t from_float(float v) { return Fp16::from_float(v); }
 };
 
+// Quotients of numbers below 2^31 by a fixed divisor: a multiplication by
+// 2^32 (2^shift - by) / by + 1, rounded down, an addition and a shift, exact
+// for every such number (Granlund and Montgomery 1994, theorem 4.2 with N = 32).
+struct RopeDivide
+{
+    uint32_t by, factor, shift;
+    explicit RopeDivide(uint32_t d) : by(d), factor(0), shift(0)
+    {
+        while((1ull << shift) < d)
+        {
+            ++shift;
+        }
+        factor = (uint32_t)((((1ull << shift) - d) << 32) / d + 1);
+    }
+    __device__ __forceinline__ uint32_t quotient(uint32_t t) const
+    {
+        return (__umulhi(t, factor) + t) >> shift;
+    }
+};
+
 template<bool BACKWARD>
 __device__ __forceinline__ void rotate(float c, float s, float a, float b, float &x, float &y)
 {
@@ -58,15 +82,17 @@ __device__ __forceinline__ void rotate(float c, float s, float a, float b, float
 
 template<typename S, bool BACKWARD, int COLS>
 __global__ __launch_bounds__(256)
-void rope_vec_kernel(int64_t m, int n, int row_blocks, const typename S::storage *sin,
+void rope_vec_kernel(int64_t m, int n, RopeDivide per_col, const typename S::storage *sin,
         const typename S::storage *cos, const typename S::storage *src,
         typename S::storage *dst)
 {
     typedef typename S::storage E;
     constexpr int NV = (int)sizeof(E) / 2;      // 16-byte pieces of four pairs
-    const int j0 = (int)(blockIdx.x / (unsigned)row_blocks) * COLS;
-    const int64_t i = 4 * ((int64_t)(blockIdx.x % (unsigned)row_blocks) * 256 + threadIdx.x);
-    if(i >= m)
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t col = per_col.quotient(t);
+    const int j0 = (int)col * COLS;
+    const int64_t i = 4 * (int64_t)(t - col * per_col.by);
+    if(j0 >= n)
     {
         return;
     }
@@ -160,30 +186,30 @@ static int launch_rope_typed(hipStream_t stream, int64_t m, int64_t n, const voi
     {
         return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;
     };
-    const bool vec = m % 4 == 0 && n <= 0x7fffffff && aligned(src, 16) && aligned(dst, 16)
-        && aligned(sin, 4 * sizeof(E)) && aligned(cos, 4 * sizeof(E));
+    const int64_t per_col = m / 4;
+    // (a thread's number fits 31 bits)
+    const bool vec = m % 4 == 0 && n <= 0x7fffffff && pairs / 4 <= 0x7fffff00 && aligned(src, 16)
+        && aligned(dst, 16) && aligned(sin, 4 * sizeof(E)) && aligned(cos, 4 * sizeof(E));
     if(vec)
     {
         // two columns a thread once that leaves every CU eight workgroups,
-        // enough for its memory pipeline
-        constexpr int COLS = 2;
-        const int64_t rows = (m / 4 + 255) / 256;
-        const bool many = rows * ((n + COLS - 1) / COLS) >= 2048;
-        const int64_t cols = many ? (n + COLS - 1) / COLS : n;
-        if(rows > 0x7fffffff / cols)
-        {
-            return NNTILE_HIP_EINVAL;
-        }
-        const dim3 grid((unsigned)(rows * cols));
+        // enough for its memory pipeline, and where a column is whole cache
+        // lines, or each is touched by two loads far apart (bf16 2 x 4 x 2^20
+        // 7.3 us with one column, 10.2 with two; 2 x 1028 x 16320 23.5 and 24.1;
+        // 2 x 64 x 262144 23.5 and 22.1)
+        const bool many = (pairs / 4 + 511) / 512 >= 2048 && 2 * m * (int64_t)sizeof(E) % 128 == 0;
+        const int64_t threads = per_col * (many ? (n + 1) / 2 : n);
+        const dim3 grid((unsigned)((threads + 255) / 256));
+        const RopeDivide divide((uint32_t)per_col);
         if(many)
         {
-            hipLaunchKernelGGL((rope_vec_kernel<S, BACKWARD, COLS>), grid, dim3(256), 0, stream, m,
-                    (int)n, (int)rows, sin, cos, src, dst);
+            hipLaunchKernelGGL((rope_vec_kernel<S, BACKWARD, 2>), grid, dim3(256), 0, stream, m,
+                    (int)n, divide, sin, cos, src, dst);
         }
         else
         {
             hipLaunchKernelGGL((rope_vec_kernel<S, BACKWARD, 1>), grid, dim3(256), 0, stream, m,
-                    (int)n, (int)rows, sin, cos, src, dst);
+                    (int)n, divide, sin, cos, src, dst);
         }
     }
     else

@@ -122,3 +122,31 @@ def test_columns_per_thread(dtype, m, n, backward):
     bound = 2 * torch.finfo(dt).eps * (x.float().abs().sum(-1, keepdim=True)
                                        * (s.abs() + c.abs())[None, :, None])
     assert ((y.float() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "bf16"])
+@pytest.mark.parametrize("backward", [False, True])
+@pytest.mark.parametrize("m", [4, 8, 16, 64, 252, 1020, 1024, 1028, 4100])
+@pytest.mark.parametrize("n", [1, 3, 258, "many"])
+def test_columns_of_any_length_give_the_bits_of_the_pairwise_kernel(dtype, backward, m, n):
+    """Four pairs a thread, one column or two ("many": an odd number of them),
+    columns shorter and longer than a workgroup and no multiple of it, against
+    one pair a thread, which addresses off by one pair take."""
+    if n == "many":
+        n = (1 << 22) // m | 1
+    print("case rope columns", dtype, backward, m, n, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m * 1000 + n)
+    dt = H.TORCH_DT[dtype]
+    sin, cos = (torch.randn(m, generator=g, device="cuda").to(dt) for _ in range(2))
+    size = 2 * m * n
+    src = torch.randn(size + 2, generator=g, device="cuda").to(dt)
+    out = []
+    for shift in (0, 2):
+        x = src[shift:shift + size]
+        x.copy_(src[:size].clone())
+        y = torch.full((size + 18,), 7.0, dtype=dt, device="cuda")
+        hip_sdpa.rope(sin, cos, x, y[shift + 8:shift + 8 + size], backward=backward)
+        torch.cuda.synchronize()
+        assert (y[:shift + 8] == 7.0).all() and (y[shift + 8 + size:] == 7.0).all()
+        out.append(y[shift + 8:shift + 8 + size].clone())
+    assert torch.equal(out[0], out[1])
