@@ -31,6 +31,21 @@ def _stale(obj, src):
     return any(os.path.getmtime(d) > t for d in deps)
 
 
+def front_tag():
+    """What the front-end is compiled against: it reads torch's C++ objects and
+    the interpreter's, so it fits one build of each."""
+    import platform
+    import torch
+    return "torch %s, Python %s" % (torch.__version__, platform.python_version())
+
+
+def _front_stale():
+    if _stale(FRONT, os.path.join(CSRC, "front.cpp")):
+        return True
+    with open(FRONT, "rb") as f:
+        return ("nntile_front for %s;" % front_tag()).encode() not in f.read()
+
+
 def _front_command():
     """g++ on the binding's front-end: host code on torch's headers, linked
     against the kernel library beside it."""
@@ -41,6 +56,7 @@ def _front_command():
     lib = library_paths()
     return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
              "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+             '-DNNTILE_FRONT_TAG="%s"' % front_tag(),
              "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
             + [x for d in inc for x in ("-isystem", d)]
             + [os.path.join(CSRC, "front.cpp"), "-o", FRONT]
@@ -79,7 +95,7 @@ def build(force=False, verbose=True):
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.check_call(cmd)
-    if force or _stale(FRONT, os.path.join(CSRC, "front.cpp")):
+    if force or _front_stale():
         cmd = _front_command()
         if verbose:
             print(" ".join(cmd), flush=True)

@@ -758,5 +758,9 @@ PyMODINIT_FUNC PyInit__front()
     Py_INCREF(&launch_type);
     PyModule_AddObject(m, "Launch", reinterpret_cast<PyObject *>(&launch_type));
     PyModule_AddIntConstant(m, "OTHER_WAY", kOtherWay);
+    // the builds of torch and Python that this file was compiled against; the
+    // loader compares them, and the build looks for them in the file
+    static const char tag[] = "nntile_front for " NNTILE_FRONT_TAG ";";
+    PyModule_AddStringConstant(m, "TAG", tag);
     return m;
 }

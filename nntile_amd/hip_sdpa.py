@@ -246,11 +246,15 @@ def _native():
     global _front
     if _front is None:
         lib()
+        from .build import front_tag
         try:
             from . import _front as module
         except ImportError as e:
             raise RuntimeError("the native front-end nntile_amd/_front.so cannot be loaded (%s): "
                                "run `python -m nntile_amd.build`" % e)
+        if module.TAG != "nntile_front for %s;" % front_tag():
+            raise RuntimeError("the native front-end nntile_amd/_front.so is for another build of torch "
+                               "or Python (%s): run `python -m nntile_amd.build`" % module.TAG)
         _front = module
     return _front
 

@@ -85,3 +85,18 @@ def test_every_launch_goes_through_the_form_that_releases_the_lock():
     assert called == {"nntile_hip_sdpa_fwd_decode_workspace_bytes_fp32",
                       "nntile_hip_sdpa_fwd_decode_workspace_bytes"}
     assert not re.search(r"_fns\[[^]]*\]\(|\)\(s\b|fn\(s\b", text)
+
+
+def test_another_torch_makes_the_front_end_stale(monkeypatch):
+    """It reads torch's C++ objects: built against another torch it is built
+    again, and refused where that was not done."""
+    monkeypatch.setattr(B, "_stale", lambda obj, src: False)     # (no source is newer)
+    assert not B._front_stale()
+    monkeypatch.setattr(torch, "__version__", "1.2.3")
+    assert B._front_stale()
+    monkeypatch.setattr(h, "_front", None)
+    with pytest.raises(RuntimeError, match="another build of torch"):
+        h._native()
+    monkeypatch.undo()
+    monkeypatch.setattr(h, "_front", None)
+    assert h._native().TAG
