@@ -463,7 +463,7 @@ def bench_backward(cfg, steps, warmup):
     call over the whole sequence with the analytic causal mask: the row dots,
     then one launch for the three gradients.  FLOPs counted as 2.5 x the
     forward's (five products where the forward has two); the workgroups
-    execute eight, recomputing the scores for each gradient."""
+    execute seven, recomputing S and dP for dQ."""
     import torch
     from nntile_amd import hip_sdpa as h
     dt = {"bf16": torch.bfloat16, "fp16": torch.float16}[cfg.dtype]
@@ -495,12 +495,12 @@ def bench_backward(cfg, steps, warmup):
     return {"workload": cfg.name, "ms_per_step": round(wall, 4), "flops_per_step": fl,
             "what": "backward of %s in one call (row dots + one launch for dQ, dK, dV), analytic "
                     "causal mask, gradients written; 2.5 x the forward's causal-exact FLOPs" % cfg.name,
-            "roofline": roofline("mfma", "sdpa_bwd_rowdot_kernel + sdpa_bwd_kernel<bf16,128,causal>",
+            "roofline": roofline("mfma", "sdpa_bwd_prelude_kernel + sdpa_bwd_kernel<bf16,128,causal>",
                                  fl, dev, PEAK_BF16_TFLOPS, "TFLOP/s", TRAFFIC["cfg3_backward"]),
             "reference_tiling": {
                 "what": "the same over %d x %d separately allocated tiles of %d rows, gradients "
                         "added to the tiles: nntile_hip_sdpa_bwd_grid, one call for all tile pairs "
-                        "(row dots per query tile + one launch)" % (len(Qt), len(Kt), tile),
+                        "(row dots of all tiles + one launch)" % (len(Qt), len(Kt), tile),
                 "ms_per_step": round(wall_t, 4), "device_ms_per_step": round(dev_t, 4),
                 "frac_of_peak": round(fl / (dev_t * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, 4)}}
 

@@ -101,7 +101,7 @@ enum nntile_hip_mask_mode
  * The merge is fused into the kernel, so neither scratch tile is needed for
  * it and both may be null.  scratch_A is never touched.  scratch_lse (seq *
  * batch floats, as the reference registers it) may be overwritten: when the
- * mask is 1 MiB or larger the 16-bit variants scan it once per call - by the
+ * mask is 384 KiB or larger the 16-bit variants scan it once per call - by the
  * first workgroups of the attention launch, or, on a stream that is being
  * captured, by a small launch of their own - and keep what they found (24
  * bytes per 128 queries and key range) there, instead of letting the
@@ -325,7 +325,7 @@ int nntile_hip_sdpa_fwd_decode_fp16(void *stream, const nntile_hip_sdpa_tile_arg
  * wrappers/python/tests/model/test_llama_attention.py:296-345): the same
  * sharing of K/V among the query heads of a group and the same split of the
  * keys, with v_mfma_f32_16x16x4_f32; the partials are fp32, so the workspace
- * has a size function of its own, and the merge is always a second launch. */
+ * has a size function of its own. */
 size_t nntile_hip_sdpa_fwd_decode_workspace_bytes_fp32(const nntile_hip_sdpa_tile_args *args);
 int nntile_hip_sdpa_fwd_decode_fp32(void *stream, const nntile_hip_sdpa_tile_args *args,
         void *workspace, size_t workspace_bytes);
@@ -353,9 +353,11 @@ int nntile_hip_sdpa_fwd_decode_static(void *stream, int32_t dtype,
 
 /* ---- 4c. diagnostics of the decode entry points ------------------------------
  * No counterpart in the reference.  When a (batch entry, kv head) unit has
- * several key splits and the units come in multiples of 8, the merge of the
- * splits runs inside the main launch: merge workgroups behind the main ones
- * wait for flags in the workspace.  That wait is bounded (2 s of the 100 MHz
+ * several key splits, the merge of the splits runs inside the main launch, for
+ * every tile type - unless the units come in a number that would leave the
+ * XCDs' shares of K and V too different (then, and with
+ * NNTILE_HIP_SDPA_DECODE_SEPARATE_MERGE, it is a second launch): merge
+ * workgroups behind the main ones wait for flags in the workspace.  That wait is bounded (2 s of the 100 MHz
  * device clock unless set otherwise here; returns the previous bound); a merge
  * workgroup that gives up leaves its rows untouched and is counted.  The
  * count since the library was loaded (blocking; -1 on error): */

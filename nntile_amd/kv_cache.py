@@ -178,7 +178,7 @@ class KVCache:
             sliced, mode = self.mask_slice(mask, q_seq), hip_sdpa.MASK_BOOL
 
         def keep(t):
-            # The kernels are enqueued through ctypes; torch's allocator does
+            # The kernels are enqueued behind torch's back; its allocator does
             # not know they read t.  On a stream other than the current one the
             # allocator is told; in every case the tensor stays referenced
             # here until the next call.
