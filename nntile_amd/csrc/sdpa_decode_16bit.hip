@@ -1108,8 +1108,8 @@ static int launch_decode_stages(hipStream_t stream, DecodeParams &p, int mode)
     // The merge rides in the main launch when the caller allows it and the
     // unit has several splits.  The grid then gives the units out eight at a
     // time so that a unit's workgroups share an XCD; units that are no multiple
-    // of eight leave places that end at once (12 units, 12 steps: 8.8 us with
-    // the merge as a second launch, 7.5 so) - and leave XCDs with less to do,
+    // of eight leave places that end at once (12 units, 12 steps: 8.4 us with
+    // the merge as a second launch, 7.4 so) - and leave XCDs with less to do,
     // which a second launch costs less than once the difference is worth more
     // than 3 us of the stream (20 units of 15 000 keys: 31.9 against 39.7 us).
     const int units8 = (units + 7) / 8 * 8;
