@@ -953,10 +953,13 @@ def main():
             extras[name] = {
                 "ms_per_step": round(r["ms_per_step"], 4), "tflops": round(r["tflops"], 2),
                 "flops_causal_exact": c.flops(), "launches_per_step": r["launches_per_step"],
-                "roofline": roofline("mfma", "sdpa_prefill_fp32_kernel<%d,causal>" % c.head if fp32
-                                     else "sdpa_prefill_16bit_kernel<bf16,%d,causal>" % c.head,
+                # (fp32: eight workgroups on the fp32 units, or three fp16 products each)
+                "roofline": roofline("mfma", {"cfg1_single_head_fp32": "sdpa_prefill_fp32_kernel<%d,causal>",
+                                              "cfg2_gpt2_small_fp32": "sdpa_prefill_f16x2_kernel<%d,causal>",
+                                              }.get(name, "sdpa_prefill_16bit_kernel<bf16,%d,causal>") % c.head,
                                      c.flops(), r["device_ms_per_step"],
-                                     PEAK_FP32_TFLOPS if fp32 else PEAK_BF16_TFLOPS, "TFLOP/s",
+                                     PEAK_FP32_TFLOPS if c.calls == 1 and fp32
+                                     else PEAK_BF16_TFLOPS / 3 if fp32 else PEAK_BF16_TFLOPS, "TFLOP/s",
                                      TRAFFIC.get(name))}
             if c.calls > 1:
                 r1 = bench_prefill(c, few, 5, one_launch=False)

@@ -53,18 +53,21 @@ extern "C" {
 #define NNTILE_HIP_SDPA_OVERWRITE 1
 /* Tile and grid calls, for tests and tuning: fix the workgroup shape instead
  * of letting the size of the launch pick it.  fp32: 128 queries sharing every
- * key step (SHARED), or 32 queries whose four wavefronts split the key steps
- * (SPLIT).  16-bit: 128 queries and four wavefronts (SHARED), or the same 128
- * queries held by two groups of four wavefronts that take every second key
- * step each and merge through LDS (SPLIT; head 64 and 128; what a launch of
- * at most one workgroup per CU takes by itself).  Both set: ignored. */
+ * key step, on the fp16 matrix units (SHARED), or 32 queries whose four
+ * wavefronts split the key steps, on the fp32 ones (SPLIT).  16-bit: 128 queries
+ * and four wavefronts (SHARED), or the same 128 queries held by two groups of
+ * four wavefronts that take every second key step each and merge through LDS
+ * (SPLIT; head 64 and 128; what a launch of at most one workgroup per CU takes by
+ * itself).  Both set: ignored. */
 #define NNTILE_HIP_SDPA_FORM_SHARED 0x100
 #define NNTILE_HIP_SDPA_FORM_SPLIT  0x200
 /* 16-bit tile and grid calls with an analytic mask, head 64 or 128, for tests
  * and tuning: workgroups of 256 queries (eight wavefronts, one workgroup per
  * CU) instead of 128 (four, two per CU).  Without it a launch picks the form
  * from its size (256 queries at head 128 when every CU gets two workgroups);
- * NNTILE_HIP_SDPA_FORM_SHARED keeps such a call at 128 queries. */
+ * NNTILE_HIP_SDPA_FORM_SHARED keeps such a call at 128 queries.  fp32: the other
+ * shapes on the fp16 matrix units - 256 queries (WIDE), 128 queries and two key
+ * blocks (WIDE | SHARED), 64 queries and two key blocks (WIDE | SPLIT). */
 #define NNTILE_HIP_SDPA_FORM_WIDE   0x4000
 /* decode calls, for tests and tuning: merge the key splits in a second launch
  * instead of inside the main one (SEPARATE_MERGE); exchange the partials of

@@ -10,7 +10,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libnntile_hip_sdpa.so")
-SOURCES = ["sdpa_prefill_16bit.hip", "sdpa_prefill_fp32.hip",
+SOURCES = ["sdpa_prefill_16bit.hip", "sdpa_prefill_fp32.hip", "sdpa_prefill_f16x2.hip",
            "sdpa_decode_16bit.hip", "sdpa_decode_fp32.hip", "sdpa_bwd_16bit.hip", "rope.hip", "transpose.hip", "kv_cache.hip", "mask_classify.hip",
            "accumulate_attn_output.hip", "sdpa_parts_merge.hip", "capi.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

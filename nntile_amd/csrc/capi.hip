@@ -71,14 +71,14 @@ static bool mode_ok(int mode)
     return mode >= NNTILE_HIP_MASK_ADDITIVE && mode <= NNTILE_HIP_MASK_BOOL;
 }
 
-// the workgroup shape a caller asked for: 0 none, 1 shared, 2 split, 8 wide (16-bit kernels)
+// the workgroup shape a caller asked for: 0 none, 1 shared, 2 split, from 8 on wide
 static int prefill_form(int32_t flags)
 {
     const bool shared = (flags & NNTILE_HIP_SDPA_FORM_SHARED) != 0;
     const bool split = (flags & NNTILE_HIP_SDPA_FORM_SPLIT) != 0;
     if(flags & NNTILE_HIP_SDPA_FORM_WIDE)
     {
-        return 8;       // 16-bit kernels: 256-query workgroups
+        return 8 + (shared ? 1 : 0) + (split ? 2 : 0);      // 256-query workgroups; fp32: see launch_prefill_fp32
     }
     return shared == split ? 0 : (shared ? 1 : 2);
 }

@@ -72,8 +72,9 @@ struct PrefillParams
     int32_t xcd_remap;            // 1: regroup workgroups so a slab stays on one XCD
     int32_t overwrite;            // 1: ignore the running pair, write every row
     int32_t n_scan_wgs;
-    int32_t form;                 // fp32 launcher: 0 pick by size, 1 shared key steps, 2 split key steps
-                                  // 16-bit launcher: 0 pick by size, 1 128-query workgroups, 2 the same with the key steps split over two groups of wavefronts, 8 256-query
+    int32_t form;                 // 0 pick by size
+                                  // fp32 launcher: see launch_prefill_fp32
+                                  // 16-bit launcher: 1 128-query workgroups, 2 the same with the key steps split over two groups of wavefronts, from 8 on 256-query
     float scale;                  // 1/sqrt(head)
     const void *K[kMaxTiles];
     const void *V[kMaxTiles];
@@ -97,6 +98,12 @@ struct PrefillParts
     size_t bytes;
 };
 PrefillParts prefill_parts(bool fp32, int64_t batch, int64_t q_seq, int64_t k_seq, int64_t head);
+
+// Workgroup shapes of the fp32 forward on fp16 matrix units: query blocks of 32
+// times key blocks of 32 (none of them: the fp32 kernel's)
+constexpr int kF16x2None = 0, kF16x2Form22 = 1, kF16x2Form41 = 2, kF16x2Form42 = 3, kF16x2Form81 = 4;
+int prefill_f16x2_form(const PrefillParams &p, int head, int mode);
+int launch_prefill_f16x2(hipStream_t stream, PrefillParams &p, int head, int mode, int form);
 
 // Kernel arguments of the decode kernels.  K, V: [head, k_seq, n_batch,
 // n_head_kv]; Q, A: [head, q_seq, n_batch, kv_group, n_head_kv].

@@ -1843,7 +1843,7 @@ int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head,
         int mode, void *scan_scratch, size_t scan_scratch_bytes)
 {
     // 256-query workgroups (eight wavefronts, one workgroup a CU): when asked
-    // for (p.form == 8), and by themselves where they measured faster - head
+    // for (p.form from 8 on), and by themselves where they measured faster - head
     // 128, whole 256-query blocks, and enough of them that every CU gets two
     // under a causal mask (one workgroup a CU has nobody to share the CU with
     // while it starts and ends, and a causal launch of one round is set by its
@@ -1851,7 +1851,7 @@ int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head,
     // p.form == 1 keeps the 128-query form.
     const bool can_wide = (head == 64 || head == 128)
         && (mode == NNTILE_HIP_MASK_NONE || mode == NNTILE_HIP_MASK_CAUSAL);
-    bool wide = can_wide && p.form == 8;
+    bool wide = can_wide && p.form >= 8;
     if(can_wide && p.form == 0 && head == 128 && (p.q_tile % 256 == 0 || p.n_q_tiles == 1))
     {
         const int64_t n_w = (int64_t)p.batch * p.n_slabs * p.n_q_tiles * ((p.q_tile + 255) / 256);

@@ -1,0 +1,1426 @@
+// Prefill attention forward for fp32 tiles on the fp16 matrix units of gfx950.
+//
+// The fp32 matrix instructions run at 157 TFLOP/s, the fp16 ones at 2500.  A
+// float is, to 22 bits, the sum of two fp16 values: x = h + l with h = fp16(x),
+// l = fp16(x - h), what is left is at most 2^-23 of x.  Of the four products of
+// two such sums l.h, h.l and h.h are added up in fp32 by the matrix unit; l.l is
+// at most 2^-22 of the product, 2^-25 in the mean.  Three fp16 products cost
+// 3/16 of an fp32 one, so the ceiling moves from 157 to 833 TFLOP/s, and a sum
+// of head (or key) products is rounded a fifth as often.  (The method: Markidis
+// et al., "NVIDIA Tensor Core Programmability, Performance & Precision", 2018;
+// Ootomo and Yokota, "Recovering single precision accuracy from Tensor Cores
+// while surpassing the FP32 theoretical peak performance", 2022.)
+//
+// fp16 holds 22 bits of x in two values for 2^-3 <= |x| < 2^16, and 2^-25
+// absolutely below, so the values are moved there by powers of two, which are
+// exact: a row of Q so that its largest value is in [2^13, 2^14), K and V so that
+// the largest of a workgroup's first step is in [2^11, 2^12), the probabilities
+// (at most 1) by 2^14.  What that does not cover - infinities and NaN, later keys
+// 16 times larger than those of the first step, blocks of them 1000 times
+// smaller, rows of the output or of Q beyond 2^+-40 - is found by a test of the
+// blocks as they are split and of the results, and the workgroup then walks its
+// keys again with fp32 matrix instructions.
+//
+// S^T = K Q^T and O^T += V^T P^T with a lane owning one query, as in the other
+// prefill kernels.  A workgroup holds QW blocks of 32 queries; a key step is G
+// blocks of 32 keys, and wavefront (q, g) takes query block q against key block
+// g.  K and V are split once per workgroup on their way into LDS, where each
+// piece lies in the order in which a matrix operand is read (1 KB a fragment,
+// 16 bytes a lane: no bank conflicts, V transposed on the way in), Q once into
+// registers, the probabilities where they are.  A pass of the loop computes the
+// scores of step i+1 and the output of step i on the matrix unit; in slices
+// behind its instructions run the softmax of step i and the splitting of
+// K(i+2) and V(i+1), whose rows were requested into registers a pass before.
+// Two LDS buffers each for K and V: one barrier a pass.
+//
+// What bounds it: the vector port.  A matrix instruction takes it for 16 clocks
+// and every vector instruction for 4; a pass at head 64 is 24 of the first and
+// about 160 (8 x 1: 125) of the second for 32 x 32 scores, 1 100 clocks against 768
+// of the matrix unit; two wavefronts a SIMD come to 70 % of that.  (Three bf16
+// pieces, which need no powers of two: twice the products and 11 instead of 6
+// vector instructions for a pair of values, 50 us where this took 41 at 48 x 1024
+// x 64.)
+#include <cmath>
+#include <type_traits>
+
+#include "sdpa_mask_scan.hpp"
+
+namespace nntile_hip
+{
+
+constexpr int kX2Rows = 32;         // queries of a wavefront, keys of a wavefront's step
+// Probabilities are scaled by 2^4: their pieces are exact to 2^-29, and the
+// arguments of the exponentials that matter lie within 4 of zero, where a float
+// is finest (2^14: errors of A a fifth larger than with fp32 products, of lse 5 %).
+constexpr int kX2PExp = 4;
+
+// The two fp16 pieces of eight floats times a power of two, as matrix operands.
+struct Split8
+{
+    u32x4 h, l;
+    // (fma with an fp16 operand: no conversion back)
+    __device__ __forceinline__ void pair(int i, float a, float b, float scale)
+    {
+        h[i] = Fp16::pack2(a * scale, b * scale);
+        l[i] = Fp16::pack2(fmaf(a, scale, -lo_half(h[i])), fmaf(b, scale, -hi_half(h[i])));
+    }
+    // the same without a scale; one: 1.0f, unknown to the compiler, which would
+    // otherwise undo the fma
+    __device__ __forceinline__ void pair_unscaled(int i, float a, float b, float one)
+    {
+        h[i] = Fp16::pack2(a, b);
+        uint32_t low = Fp16::pack2(fmaf(a, one, -lo_half(h[i])), fmaf(b, one, -hi_half(h[i])));
+        asm volatile("" : "+v"(low));       // (here, not in front of its use)
+        l[i] = low;
+    }
+    static __device__ __forceinline__ float lo_half(uint32_t v)
+    {
+        return Fp16::to_float((uint16_t)(v & 0xffffu));
+    }
+    static __device__ __forceinline__ float hi_half(uint32_t v)
+    {
+        return Fp16::to_float((uint16_t)(v >> 16));
+    }
+};
+
+// acc += a.b; one of the three products, the smallest first
+__device__ __forceinline__ f32x16 product(int n, const Split8 &a, const Split8 &b, f32x16 acc)
+{
+    const u32x4 x = n == 0 ? a.l : a.h, y = n == 1 ? b.l : b.h;
+    return Fp16::mfma(__builtin_bit_cast(f16x8, x), __builtin_bit_cast(f16x8, y), acc);
+}
+
+// The power of two that moves `largest` into [2^(to-1), 2^to) and its inverse;
+// false when it is out of the range that is moved (then 1).  LEAST: what is below
+// 2^-40 is moved as if it were that (the factors of a score: times one below 2^40,
+// what the pieces then lose is below 2^-30).  Zeros: as if they were 2^(to-5).
+template<bool LEAST>
+__device__ __forceinline__ bool power_to(float largest, int to, float &scale, float &inverse)
+{
+    scale = inverse = 1.0f;
+    if(largest == 0.0f)
+    {
+        return true;
+    }
+    if(LEAST)
+    {
+        largest = fmaxf(largest, 0x1p-40f);
+    }
+    if(!(largest >= 0x1p-40f && largest < 0x1p40f))
+    {
+        return false;
+    }
+    const int e = __builtin_amdgcn_frexp_expf(largest);     // largest in [2^(e-1), 2^e)
+    scale = __uint_as_float((uint32_t)(127 + to - e) << 23);
+    inverse = __uint_as_float((uint32_t)(127 - to + e) << 23);
+    return true;
+}
+
+template<int HEAD, int MODE, int QW, int G, bool PARTS = false>
+__global__ __launch_bounds__(64 * QW * G, HEAD == 128 && QW == 2 ? 1 : 2)
+void sdpa_prefill_f16x2_kernel(const PrefillParams p)
+{
+    constexpr int THREADS = 64 * QW * G;
+    constexpr int QROWS = kX2Rows * QW;     // queries per workgroup
+    constexpr int KEYS = kX2Rows * G;       // keys per step of the workgroup
+    constexpr int CH = HEAD / 16;           // matrix instructions along the head (scores)
+    constexpr int DB = HEAD / 32;           // blocks of the head (output)
+    constexpr int HG = HEAD / 8;            // groups of 8 head values
+    constexpr int GB = 2 * kX2Rows * HEAD * 2;      // bytes of a key block's pieces
+    // pieces of 8 values that a thread splits per step of K, and of V
+    constexpr int UNITS = KEYS * HG;
+    constexpr int UPT = (UNITS + THREADS - 1) / THREADS;
+    constexpr int NS = 3 * CH, NP = 6 * DB;         // matrix instructions of scores and output
+    // Rows are requested into SETS sets of registers in turn, SETS passes before they
+    // are split (what a lane holds at head 128 leaves room for one).
+    constexpr int AHEAD_FR = HEAD == 64 ? 2 : 1;
+    constexpr int SETS = HEAD >= 128 ? 1 : 2;
+    constexpr bool EXPLICIT = (MODE == NNTILE_HIP_MASK_ADDITIVE
+            || MODE == NNTILE_HIP_MASK_BOOL);
+    static_assert(!PARTS || !EXPLICIT, "parts: analytic masks");
+
+    constexpr int BUF = G * GB;             // K(0) K(1) V(0) V(1)
+    __shared__ __attribute__((aligned(1024))) char lds[4 * BUF];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31;
+    const int half = lane >> 5;
+    const int qw = wave % QW, grp = wave / QW;
+
+    const int q_blocks = p.n_q_tiles * p.q_blocks_per_tile;
+    const int batch_all = p.batch * p.n_slabs;
+    int wg = blockIdx.x;
+    int part = 0;
+    if constexpr(PARTS)
+    {
+        const int per_part = (int)gridDim.x / p.n_parts;
+        part = wg / per_part;
+        wg -= part * per_part;
+    }
+    const int64_t part_k0 = PARTS ? (int64_t)part * p.part_keys : 0;
+    const int64_t k_seq = PARTS ? min((int64_t)p.part_keys, p.k_seq - part_k0) : p.k_seq;
+    const int64_t k_tile = PARTS ? k_seq : p.k_tile;
+    const int64_t k_pos0 = p.k_pos0 + part_k0;
+    const bool overwrite = PARTS || p.overwrite;
+    // Longest query blocks first, all batch entries of a block before the next
+    // block: CUs that become free take what is left in the order of its length,
+    // and a number of entries that is a multiple of 8 keeps an entry on one XCD.
+    int b = wg % batch_all;
+    const int qblk = q_blocks - 1 - wg / batch_all;
+    int q_tile0 = 0, k_tile0 = 0;
+    if(p.n_slabs > 1)
+    {
+        const int slab = b / p.batch;
+        b -= slab * p.batch;
+        q_tile0 = slab * p.n_q_tiles;
+        k_tile0 = slab * p.n_kv_tiles;
+    }
+    const int qt = qblk / p.q_blocks_per_tile;
+    const int qb = qblk % p.q_blocks_per_tile;
+    const int64_t q_len = min(p.q_tile, p.q_seq - (int64_t)qt * p.q_tile);
+    const int64_t q_row0 = (int64_t)qb * QROWS;
+    if(q_row0 >= q_len)
+    {
+        return;
+    }
+    const int kvb = kv_entry(b, p.n_batch, p.kv_group);
+    const float *Qt = static_cast<const float *>(p.Q[q_tile0 + qt]) + (int64_t)b * q_len * HEAD;
+    const int64_t wave_q = q_row0 + qw * kX2Rows;
+    const bool q_ok = wave_q + col < q_len;
+    // this lane's query row (the tile's first for a lane that has none)
+    auto my_row = [&]() __attribute__((always_inline)) -> int64_t
+    {
+        return q_ok ? wave_q + col : 0;
+    };
+
+    // ---- the steps to walk -----------------------------------------------------
+    const int64_t last_k_len = k_seq - (int64_t)(p.n_kv_tiles - 1) * k_tile;
+    int n_steps = (p.n_kv_tiles - 1) * p.k_blocks_per_tile
+        + (int)((last_k_len + KEYS - 1) / KEYS);
+    const int64_t wg_qpos_hi = p.q_pos0 + (int64_t)qt * p.q_tile + min(q_row0 + QROWS, q_len) - 1;
+    const int64_t wave_qpos_lo = p.q_pos0 + (int64_t)qt * p.q_tile + wave_q;
+    if(MODE == NNTILE_HIP_MASK_CAUSAL)
+    {
+        const int64_t hi = wg_qpos_hi + p.causal_offset - k_pos0;
+        if(hi < 0)
+        {
+            if(!overwrite)
+            {
+                return;
+            }
+            n_steps = 0;    // nothing visible: the epilogue writes empty rows
+        }
+        const int64_t kt_hi = hi < 0 ? (int64_t)p.n_kv_tiles : hi / k_tile;
+        if(kt_hi < p.n_kv_tiles)
+        {
+            const int64_t in_tile = hi - kt_hi * k_tile;
+            n_steps = min(n_steps, (int)(kt_hi * p.k_blocks_per_tile + in_tile / KEYS + 1));
+        }
+    }
+    // A mask given as values: the workgroup's rows of it are looked over once;
+    // hidden steps at either end are not walked, open ones read no mask values.
+    int n_skip = 0;
+    unsigned long long not_open = ~0ull;
+    if constexpr(EXPLICIT)
+    {
+        constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 4 : 1;
+        if(n_steps > 0 && k_seq * ES >= 16 && p.mask_ld * ES * QROWS < (int64_t)(1 << 30))
+        {
+            __shared__ unsigned long long scan_words[2 * THREADS / 64];
+            unsigned long long not_hidden;
+            mask_scan_steps<ES, THREADS / 64, KEYS>(static_cast<const char *>(p.mask)
+                    + q_row0 * p.mask_ld * ES, (uint32_t)(p.mask_ld * ES),
+                    (int)min((int64_t)QROWS, q_len - q_row0), (int)k_seq * ES, 0, n_steps,
+                    (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0u : 0x01010101u,
+                    (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0xff800000u : 0u, scan_words, not_open,
+                    not_hidden);
+            if(not_hidden == 0ull)
+            {
+                if(!overwrite)
+                {
+                    return;
+                }
+                n_steps = 0;        // the epilogue writes empty rows
+            }
+            else
+            {
+                if((not_hidden >> 63) == 0ull)
+                {
+                    n_steps = min(n_steps, 64 - __builtin_clzll(not_hidden));
+                }
+                n_skip = min(__builtin_ctzll(not_hidden), n_steps - 1);
+                n_steps -= n_skip;
+            }
+        }
+    }
+
+    // ---- where the rows of a step come from -------------------------------------
+    struct StepSource
+    {
+        const float *K, *V;     // first row of the step
+        int step, kt, rows_left;        // rows of the tile kt from this step on
+        int64_t k_row0, k_pos;  // the step's first key: in its tile, on the key axis
+    };
+    auto tile_of = [&](StepSource &src) __attribute__((always_inline))
+    {
+        const int64_t k_len = min(k_tile, k_seq - (int64_t)src.kt * k_tile);
+        const int64_t entry_rows = p.kv_rows > 0 ? p.kv_rows : k_len;   // (a cache is one tile)
+        const int64_t off = ((int64_t)kvb * entry_rows + part_k0 + src.k_row0) * HEAD;
+        src.K = static_cast<const float *>(p.K[k_tile0 + src.kt]) + off;
+        src.V = static_cast<const float *>(p.V[k_tile0 + src.kt]) + off;
+        src.rows_left = (int)(k_len - src.k_row0);
+        src.k_pos = k_pos0 + (int64_t)src.kt * k_tile + src.k_row0;
+    };
+    // (one division, in front of the walk; then from step to step)
+    auto first_step = [&]() __attribute__((always_inline)) -> StepSource
+    {
+        StepSource src;
+        src.step = 0;
+        src.kt = p.n_kv_tiles == 1 ? 0 : n_skip / p.k_blocks_per_tile;
+        src.k_row0 = (int64_t)(n_skip - src.kt * p.k_blocks_per_tile) * KEYS;
+        tile_of(src);
+        return src;
+    };
+    // (steps past the last are that one again: what is read there nobody uses)
+    auto advance = [&](StepSource &src) __attribute__((always_inline))
+    {
+        if(src.step + 1 < n_steps)
+        {
+            ++src.step;
+            src.K += KEYS * HEAD;
+            src.V += KEYS * HEAD;
+            src.rows_left -= KEYS;
+            src.k_row0 += KEYS;
+            src.k_pos += KEYS;
+            if(src.rows_left <= 0)
+            {
+                ++src.kt;
+                src.k_row0 = 0;
+                tile_of(src);
+            }
+        }
+    };
+
+    // ---- global memory -> registers -> pieces in LDS ------------------------------
+    // K unit u: key u / HG of the step, head values 8 * (u % HG) .. +7.  Its three
+    // pieces go to fragment (head group / 2) of the key's block; inside the 512
+    // bytes of a lane half the keys' places are permuted so that the 16 lanes of a
+    // write hit 16 different ones, and so do those of a read.
+    // V unit u: head value u % HEAD, keys of slot group u / HEAD - the eight keys
+    // that a lane half's score registers hold of 16 (4 * half .. +3 and 8 further).
+    // Rows past the end of the tile are its last row: their scores are masked, so
+    // their probabilities are exactly 0.
+    constexpr int KSW = 16 / HG;            // keys of a row of 16 lanes
+    auto k_place = [](int key, int hg) __attribute__((always_inline)) -> int
+    {
+        return key ^ hg ^ ((key & (KSW - 1)) * (HG % 16));
+    };
+    // Units i * THREADS + tid of a thread: a power of two of keys (of slot groups)
+    // apart, so what follows from i is an offset known when this is compiled.
+    constexpr int KSTRIDE = THREADS / HG, SSTRIDE = THREADS / HEAD;
+    static_assert(UPT == 1 || (KSTRIDE >= 16 && SSTRIDE >= 1), "units of a thread");
+    auto k_lds = [](int i) { return i * KSTRIDE / 32 * GB + i * KSTRIDE % 32 * 16; };
+    auto v_lds = [](int i)
+    {
+        const int slots = i * SSTRIDE;
+        return (slots >> 2) * GB + ((slots >> 1) & 1) * DB * 1024 + (slots & 1) * 512;
+    };
+    auto v_rows = [](int slots) { return (slots >> 1) * 16 + (slots & 1) * 4; };
+    StepSource k_src = {}, v_src = {}, s_src = {};      // the rows requested last, the scores
+    f32x4 k_raw[SETS][UPT][2];
+    float v_raw[SETS][UPT][8];
+    uint32_t k_goff, v_goff;
+    int k_at, v_at;
+    {
+        const int u = min(tid, UNITS - 1);
+        const int key = u / HG, hg = u % HG, d = u % HEAD, slots = u / HEAD;
+        k_goff = (uint32_t)(key * HEAD + hg * 8) * 4;
+        k_at = (key / kX2Rows) * GB + (hg / 2) * 1024 + (hg % 2) * 512
+            + k_place(key % kX2Rows, hg) * 16;
+        v_goff = (uint32_t)(v_rows(slots) * HEAD + d) * 4;
+        v_at = (slots >> 2) * GB + (((slots >> 1) & 1) * DB + d / 32) * 1024
+            + ((slots & 1) * 32 + d % 32) * 16;
+    }
+    // One load instruction of a step's rows: n of the 2 * UPT (K), of the 8 * UPT (V).
+    // (32-bit offsets on a base common to the wavefront.  The last rows of a tile go
+    // in one piece, load_k_tail / load_v_tail.)
+    auto load_k_piece = [&](int set, int n) __attribute__((always_inline))
+    {
+        const char *at = reinterpret_cast<const char *>(k_src.K) + n / 2 * KSTRIDE * HEAD * 4 + n % 2 * 16;
+        k_raw[set][n / 2][n % 2] = *reinterpret_cast<const f32x4 *>(at + k_goff);
+    };
+    auto load_v_piece = [&](int set, int n) __attribute__((always_inline))
+    {
+        const int e = n % 8;
+        const char *at = reinterpret_cast<const char *>(v_src.V)
+            + (v_rows(n / 8 * SSTRIDE) + (e < 4 ? e : e + 4)) * HEAD * 4;
+        v_raw[set][n / 8][e] = *reinterpret_cast<const float *>(at + v_goff);
+    };
+    auto load_k_tail = [&](int set) __attribute__((always_inline))
+    {
+#pragma unroll
+        for(int i = 0; i < UPT; ++i)
+        {
+            const int key = (int)(k_goff / (HEAD * 4)) + i * KSTRIDE;
+            const uint32_t off = k_goff + (uint32_t)(i * KSTRIDE * HEAD * 4)
+                - (uint32_t)(max(key - (k_src.rows_left - 1), 0) * HEAD * 4);
+            const char *at = reinterpret_cast<const char *>(k_src.K) + off;
+            k_raw[set][i][0] = *reinterpret_cast<const f32x4 *>(at);
+            k_raw[set][i][1] = *reinterpret_cast<const f32x4 *>(at + 16);
+            // (waits, and keeps the compiler from making one set of loads with
+            // 64-bit addresses out of the two forms)
+            asm volatile("" : "+v"(k_raw[set][i][0]), "+v"(k_raw[set][i][1]));
+        }
+    };
+    auto load_v_tail = [&](int set) __attribute__((always_inline))
+    {
+#pragma unroll
+        for(int i = 0; i < UPT; ++i)
+        {
+#pragma unroll
+            for(int e = 0; e < 8; ++e)
+            {
+                const int add = v_rows(i * SSTRIDE) + (e < 4 ? e : e + 4);
+                const int key = (int)(v_goff / (HEAD * 4)) + add;
+                const uint32_t off = v_goff + (uint32_t)(add * HEAD * 4)
+                    - (uint32_t)(max(key - (v_src.rows_left - 1), 0) * HEAD * 4);
+                v_raw[set][i][e] = *reinterpret_cast<const float *>(
+                        reinterpret_cast<const char *>(v_src.V) + off);
+            }
+#pragma unroll
+            for(int e = 0; e < 8; ++e)
+            {
+                asm volatile("" : "+v"(v_raw[set][i][e]));      // (as above)
+            }
+        }
+    };
+    auto load_k = [&](int set) __attribute__((always_inline))
+    {
+        if(k_src.rows_left >= KEYS)
+        {
+#pragma unroll
+            for(int n = 0; n < 2 * UPT; ++n)
+            {
+                load_k_piece(set, n);
+            }
+        }
+        else
+        {
+            load_k_tail(set);
+        }
+    };
+    auto load_v = [&](int set) __attribute__((always_inline))
+    {
+        if(v_src.rows_left >= KEYS)
+        {
+#pragma unroll
+            for(int n = 0; n < 8 * UPT; ++n)
+            {
+                load_v_piece(set, n);
+            }
+        }
+        else
+        {
+            load_v_tail(set);
+        }
+    };
+
+    // ---- this lane's operands and the powers of two --------------------------------
+    Split8 qf[CH];
+    float k_scale = 1.0f, v_scale = 1.0f, v_back = 1.0f;
+    float qk_back = 1.0f;       // scores / (what the matrix unit computes)
+    bool odd = false;           // something that the pieces cannot carry
+    __shared__ int any_odd;
+    if(n_steps > 0)
+    {
+        k_src = v_src = s_src = first_step();
+        __shared__ float first_max[2 * THREADS / 64];
+        if(tid == 0)
+        {
+            any_odd = 0;
+        }
+        load_k(0);
+        load_v(0);
+        const float *Qrow = Qt + my_row() * HEAD;
+        f32x4 raw[2 * CH];
+        float q_max = 0.0f;
+#pragma unroll
+        for(int j = 0; j < 2 * CH; ++j)
+        {
+            raw[j] = *reinterpret_cast<const f32x4 *>(Qrow + 16 * (j / 2) + 8 * half + 4 * (j % 2));
+            if(!q_ok)
+            {
+                raw[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+#pragma unroll
+            for(int e = 0; e < 4; ++e)
+            {
+                q_max = fmaxf(q_max, __builtin_fabsf(raw[j][e]));
+            }
+        }
+        float q_scale, q_back, k_back;
+        odd = !power_to<true>(max_across_halves(q_max), 14, q_scale, q_back);
+#pragma unroll
+        for(int j = 0; j < CH; ++j)
+        {
+#pragma unroll
+            for(int e = 0; e < 4; ++e)
+            {
+                qf[j].pair(e, raw[2 * j + e / 2][2 * (e % 2)], raw[2 * j + e / 2][2 * (e % 2) + 1],
+                        q_scale);
+            }
+        }
+        float k_max = 0.0f, v_max = 0.0f;
+#pragma unroll
+        for(int i = 0; i < UPT; ++i)
+        {
+#pragma unroll
+            for(int e = 0; e < 8; ++e)
+            {
+                k_max = fmaxf(k_max, __builtin_fabsf(k_raw[0][i][e / 4][e % 4]));
+                v_max = fmaxf(v_max, __builtin_fabsf(v_raw[0][i][e]));
+            }
+        }
+#pragma unroll
+        for(int d = 1; d < 64; d *= 2)
+        {
+            k_max = fmaxf(k_max, __shfl_xor(k_max, d));
+            v_max = fmaxf(v_max, __shfl_xor(v_max, d));
+        }
+        if(lane == 0)
+        {
+            first_max[2 * wave] = k_max;
+            first_max[2 * wave + 1] = v_max;
+        }
+        __syncthreads();
+#pragma unroll
+        for(int w = 0; w < THREADS / 64; ++w)
+        {
+            k_max = fmaxf(k_max, first_max[2 * w]);
+            v_max = fmaxf(v_max, first_max[2 * w + 1]);
+        }
+        // (the same in every lane; this makes the compiler see it)
+        k_max = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(k_max)));
+        v_max = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v_max)));
+        odd = !power_to<true>(k_max, 12, k_scale, k_back) || odd;
+        odd = !power_to<false>(v_max, 12, v_scale, v_back) || odd;
+        qk_back = q_back * k_back;
+    }
+    // item n of the 5 * UPT that split what was loaded: four pairs, then the store
+    Split8 staged;
+    auto store_pieces = [&](char *at, int piece_bytes, bool mine) __attribute__((always_inline))
+    {
+        if(UNITS % THREADS == 0 || mine)
+        {
+            *reinterpret_cast<u32x4 *>(at) = staged.h;
+            *reinterpret_cast<u32x4 *>(at + piece_bytes) = staged.l;
+        }
+    };
+    // A wavefront's share of a block (its pieces h) that is too small for them: scaled,
+    // all of it below 2 but not all zeros.  (Bit 14 of an fp16 value: 2 or more.)
+    int too_small = 0;
+    uint32_t staged_bits = 0;
+    auto look_at_staged = [&](int i) __attribute__((always_inline))
+    {
+        const uint32_t bits = staged.h[0] | staged.h[1] | staged.h[2] | staged.h[3];
+        staged_bits = i == 0 ? bits : staged_bits | bits;
+        if(i + 1 == UPT && __builtin_amdgcn_ballot_w64((staged_bits & 0x40004000u) != 0u) == 0)
+        {
+            too_small |= __builtin_amdgcn_ballot_w64((staged_bits & 0x7fff7fffu) != 0u) != 0;
+        }
+    };
+    auto split_k = [&](int set, int n, char *lds_k) __attribute__((always_inline))
+    {
+        const int i = n / 5, j = n % 5;
+        if(j < 4)
+        {
+            staged.pair(j, k_raw[set][i][j / 2][2 * (j % 2)], k_raw[set][i][j / 2][2 * (j % 2) + 1],
+                    k_scale);
+        }
+        else
+        {
+            store_pieces(lds_k + k_at + k_lds(i), CH * 1024, i * THREADS + tid < UNITS);
+            look_at_staged(i);
+        }
+    };
+    auto split_v = [&](int set, int n, char *lds_v) __attribute__((always_inline))
+    {
+        const int i = n / 5, j = n % 5;
+        if(j < 4)
+        {
+            staged.pair(j, v_raw[set][i][2 * j], v_raw[set][i][2 * j + 1], v_scale);
+        }
+        else
+        {
+            store_pieces(lds_v + v_at + v_lds(i), 2 * DB * 1024, i * THREADS + tid < UNITS);
+            look_at_staged(i);
+        }
+    };
+    // (chunk ch of a key is 32 * ch ^ the first one's place: bits below 512)
+    int k_base = grp * GB + half * 512 + k_place(col, half) * 16;
+    const int Vw = 2 * BUF + grp * GB + lane * 16;
+    // c: from what m_run and the scores are in to powers of two
+    // (1/sqrt(head) as two floats, and its product with log2(e) rounded once: what
+    // the factors are off by, every row's sum and logsumexp are)
+    constexpr double kScale = HEAD == 32 ? 0.17677669529663688 : HEAD == 64 ? 0.125 : 0.08838834764831845;
+    constexpr float kScaleHi = (float)kScale, kScaleLo = (float)(kScale - (double)kScaleHi);
+    constexpr float kScaleLog2e = (float)(kScale * 1.4426950408889634);
+    static_assert(HEAD == 32 || HEAD == 64 || HEAD == 128, "kScale");
+    float to_scores = kScaleHi * qk_back;
+    float c = EXPLICIT ? kLog2e : kScaleLog2e * qk_back;
+    float p_exp = (float)kX2PExp;       // the probabilities' power of two
+    float one = 1.0f;
+    asm volatile("" : "+s"(one));       // (keeps the product below an fma)
+
+    f32x16 o[DB];
+#pragma unroll
+    for(int db = 0; db < DB; ++db)
+    {
+#pragma unroll
+        for(int r = 0; r < 16; ++r)
+        {
+            o[db][r] = 0.0f;
+        }
+    }
+    float m_run = neg_inf(), l_run = 0.0f;
+
+    // The operand fragments of a pass, in turn those of K (CH) and of V (2 * DB), each
+    // read into one of two sets of registers while the other is in use.
+    constexpr int FR = AHEAD_FR == 2 ? 4 : 2;
+    Split8 fr[FR];
+    auto read_k = [&](int buf, int ch) __attribute__((always_inline))
+    {
+        const char *at = lds + buf * BUF + ch * 1024 + (k_base ^ (32 * ch));
+        fr[ch % FR].h = *reinterpret_cast<const u32x4 *>(at);
+        fr[ch % FR].l = *reinterpret_cast<const u32x4 *>(at + CH * 1024);
+    };
+    auto read_v = [&](int buf, int n) __attribute__((always_inline))
+    {
+        const char *at = lds + Vw + buf * BUF + n * 1024;   // n: 16 keys n / DB, head block n % DB
+        fr[(CH + n) % FR].h = *reinterpret_cast<const u32x4 *>(at);
+        fr[(CH + n) % FR].l = *reinterpret_cast<const u32x4 *>(at + 2 * DB * 1024);
+    };
+    static_assert((CH + 2 * DB) % FR == 0 && CH >= AHEAD_FR && 2 * DB >= AHEAD_FR, "fragments in turn");
+    // Scores of a step from K in buffer `buf`, its first fragment already read;
+    // `between(t)` is called behind matrix instruction t of the NS, `last()` where
+    // the first fragment of what follows can be read.
+    auto scores = [&](int buf, f32x16 &s, auto between, auto last) __attribute__((always_inline))
+    {
+#pragma unroll
+        for(int r = 0; r < 16; ++r)
+        {
+            s[r] = 0.0f;
+        }
+#pragma unroll
+        for(int ch = 0; ch < CH; ++ch)
+        {
+            if(ch + AHEAD_FR < CH)
+            {
+                read_k(buf, ch + AHEAD_FR);
+            }
+            else
+            {
+                last(ch + AHEAD_FR - CH);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for(int n = 0; n < 3; ++n)
+            {
+                s = product(n, fr[ch % FR], qf[ch], s);
+                between(3 * ch + n);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    Split8 pf[2];       // probabilities of 16 keys each
+    // O^T += V^T P^T from V in buffer `buf`, likewise; NP instructions
+    auto output = [&](int buf, auto between, auto last) __attribute__((always_inline))
+    {
+#pragma unroll
+        for(int n = 0; n < 2 * DB; ++n)
+        {
+            if(n + AHEAD_FR < 2 * DB)
+            {
+                read_v(buf, n + AHEAD_FR);
+            }
+            else
+            {
+                last(n + AHEAD_FR - 2 * DB);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for(int t = 0; t < 3; ++t)
+            {
+                o[n % DB] = product(t, fr[(CH + n) % FR], pf[n / DB], o[n % DB]);
+                between(3 * n + t);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    // What hides keys of a step from this lane's query; register r holds key
+    // 8 * (r / 4) + 4 * half + r % 4 of the wavefront's 32.
+    auto apply_mask = [&](const StepSource &src, f32x16 &s) __attribute__((always_inline))
+    {
+        const int keys_here = src.rows_left - grp * kX2Rows;    // may be below 1
+        if constexpr(EXPLICIT)
+        {
+            const int64_t mrow = my_row() * p.mask_ld + src.k_row0 + grp * kX2Rows;
+            typedef f32x4 __attribute__((aligned(4))) f32x4_any;
+            typedef uint32_t __attribute__((aligned(1))) u32_any;
+            if(((not_open >> min(src.step + n_skip, 63)) & 1ull) == 0ull && keys_here >= kX2Rows)
+            {
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    s[r] *= to_scores;
+                }
+            }
+            else if(keys_here >= kX2Rows)
+            {
+                float madd[16];
+#pragma unroll
+                for(int rg = 0; rg < 4; ++rg)
+                {
+                    const int64_t at = mrow + 8 * rg + 4 * half;
+                    if(MODE == NNTILE_HIP_MASK_ADDITIVE)
+                    {
+                        const f32x4 v = *reinterpret_cast<const f32x4_any *>(
+                                static_cast<const float *>(p.mask) + at);
+#pragma unroll
+                        for(int e = 0; e < 4; ++e)
+                        {
+                            madd[4 * rg + e] = v[e];
+                        }
+                    }
+                    else
+                    {
+                        const uint32_t w = *reinterpret_cast<const u32_any *>(
+                                static_cast<const uint8_t *>(p.mask) + at);
+#pragma unroll
+                        for(int e = 0; e < 4; ++e)
+                        {
+                            madd[4 * rg + e] = ((w >> (8 * e)) & 0xffu) != 0u ? 0.0f : neg_inf();
+                        }
+                    }
+                }
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    s[r] = madd[r] == neg_inf() ? neg_inf() : s[r] * to_scores + madd[r];
+                }
+            }
+            else
+            {
+                // a ragged step goes element by element: keys past its end are
+                // hidden, their reads clamped to the row's last value
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    const int key = 8 * (r >> 2) + 4 * half + (r & 3);
+                    const int64_t at = mrow + min(key, keys_here - 1);
+                    float add;
+                    if(MODE == NNTILE_HIP_MASK_ADDITIVE)
+                    {
+                        add = static_cast<const float *>(p.mask)[at];
+                    }
+                    else
+                    {
+                        add = static_cast<const uint8_t *>(p.mask)[at] != 0 ? 0.0f : neg_inf();
+                    }
+                    s[r] = (key >= keys_here || add == neg_inf()) ? neg_inf() : s[r] * to_scores + add;
+                }
+            }
+        }
+        else
+        {
+            const int64_t k_pos = src.k_pos + grp * kX2Rows;
+            const bool diagonal = MODE == NNTILE_HIP_MASK_CAUSAL
+                && k_pos + kX2Rows - 1 > wave_qpos_lo + p.causal_offset;
+            if(keys_here < kX2Rows || diagonal)
+            {
+                const int64_t vis = MODE == NNTILE_HIP_MASK_CAUSAL
+                    ? wave_qpos_lo + p.causal_offset - k_pos + col : (int64_t)kX2Rows;
+                const int lim = (int)max((int64_t)-1, min(vis, (int64_t)keys_here - 1));
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    if(8 * (r >> 2) + 4 * half + (r & 3) > lim)
+                    {
+                        s[r] = neg_inf();
+                    }
+                }
+            }
+        }
+    };
+    // Online softmax in pieces: the maximum and what follows from it, then the
+    // probabilities one by one.
+    // (l_run is summed with its rounding errors kept: a wavefront of these forms adds
+    // up to four times the steps that one of the fp32 kernel does)
+    float mc = 0.0f, rs = 0.0f, l_low = 0.0f;
+    auto softmax_head = [&](const f32x16 &s) __attribute__((always_inline))
+    {
+        float mx = neg_inf();
+#pragma unroll
+        for(int r = 0; r < 16; r += 2)
+        {
+            mx = max3(mx, s[r], s[r + 1]);
+        }
+        mx = max_across_halves(mx);
+        const float m_new = fmaxf(m_run, mx);
+        const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
+        mc = m_use * c - p_exp;
+        // the running maximum rarely moves after the first steps
+        if(__builtin_amdgcn_ballot_w64(m_new != m_run) != 0)
+        {
+            const float alpha = fast_exp2((m_run - m_use) * c);
+            l_run *= alpha;
+            l_low *= alpha;
+#pragma unroll
+            for(int db = 0; db < DB; ++db)
+            {
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    o[db][r] *= alpha;
+                }
+            }
+            m_run = m_new;
+        }
+        rs = 0.0f;
+        asm volatile("" : "+v"(mc));
+    };
+    auto softmax_one = [&](f32x16 &s, int r) __attribute__((always_inline))
+    {
+        float e = fast_exp2(fmaf(s[r], c, -mc));
+        // (keeps the exponential where it is written, beside the matrix
+        // instructions, instead of in front of its first use)
+        asm volatile("" : "+v"(e));
+        // (the one before: its exponential has arrived)
+        if(r > 0)
+        {
+            rs += s[r - 1];
+            asm volatile("" : "+v"(rs));
+        }
+        s[r] = e;
+        if(r == 15)
+        {
+            const float add = (rs + e) - l_low, sum = l_run + add;
+            l_low = (sum - l_run) - add;
+            l_run = sum;
+        }
+    };
+
+    // ---- the walk -------------------------------------------------------------------
+    if(n_steps > 0)
+    {
+        // (steps past the last are that one again: nobody reads them)
+        const int last_step = n_steps - 1;
+        f32x16 s_even, s_odd;
+#pragma unroll
+        for(int n = 0; n < 5 * UPT; ++n)
+        {
+            split_k(0, n, lds);
+        }
+#pragma unroll
+        for(int n = 0; n < 5 * UPT; ++n)
+        {
+            split_v(0, n, lds + 2 * BUF);
+        }
+        // K(1) and, with two sets, V(1) and K(2)
+        advance(k_src);
+        load_k(SETS - 1);
+        if(SETS == 2)
+        {
+            advance(v_src);
+            load_v(SETS - 1);
+            advance(k_src);
+            load_k(0);
+        }
+        __syncthreads();
+        for(int n = 0; n < AHEAD_FR; ++n)
+        {
+            read_k(0, n);
+        }
+        scores(0, s_even, [](int) {}, [](int) {});
+        apply_mask(s_src, s_even);
+#pragma unroll
+        for(int n = 0; n < 5 * UPT; ++n)
+        {
+            split_k(SETS - 1, n, lds + BUF);
+        }
+        advance(k_src);
+        load_k(SETS - 1);
+        __syncthreads();
+        for(int n = 0; n < AHEAD_FR; ++n)
+        {
+            read_k(1, n);
+        }
+        // One pass; step i's scores are in s, those of step i+1 go into s_nxt.  The
+        // barrier between the two parts: in front of it K(i+2) is written where K(i) was
+        // read before the barrier of the last pass, and read behind it; behind it
+        // V(i+1) is written where V(i-1) was read before it, and read behind the next.
+        // Beside the scores: V's next rows are requested, the softmax of step i, the
+        // pieces of its first 16 probabilities, K(i+2) into LDS.  Beside the output: K's
+        // next rows are requested, V(i+1) into LDS.
+        constexpr int NA = 1 + 16 + 4 + 5 * UPT;
+        constexpr int NB = 5 * UPT;
+        auto item_a = [&](int n, int buf, f32x16 &s) __attribute__((always_inline))
+        {
+            if(n == 0)
+            {
+                softmax_head(s);
+            }
+            else if(n < 17)
+            {
+                softmax_one(s, n - 1);
+            }
+            else if(n < 21)
+            {
+                const int j = n - 17;
+                pf[0].pair_unscaled(j, s[2 * j], s[2 * j + 1], one);
+            }
+            else
+            {
+                split_k(buf % SETS, n - 21, lds + buf * BUF);
+            }
+        };
+        // the pieces of the other 16 probabilities
+        auto pieces_b = [&](const f32x16 &s) __attribute__((always_inline))
+        {
+#pragma unroll
+            for(int n = 0; n < 4; ++n)
+            {
+                pf[1].pair_unscaled(n, s[8 + 2 * n], s[8 + 2 * n + 1], one);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto first_v = [&](int buf) __attribute__((always_inline))
+        {
+#pragma unroll
+            for(int n = 0; n < AHEAD_FR; ++n)
+            {
+                read_v(buf, n);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // INNER: the rows to be requested are whole steps of the tiles that the last ones
+        // requested are in: no branch, one instruction at a time behind the matrix
+        // instructions.  (With a branch around each, or all at once, the wavefront
+        // stands at its own loads: 32 x 4096, head 64, 264 and 241 us.)
+        auto pass = [&](auto inner_tag, auto buf_tag, f32x16 &s, f32x16 &s_nxt)
+            __attribute__((always_inline))
+        {
+            constexpr bool INNER = decltype(inner_tag)::value;
+            constexpr int buf = decltype(buf_tag)::value;
+            constexpr int v_set = SETS == 2 ? buf : 0, k_set = buf % SETS;
+            if(SETS == 1)
+            {
+                // (the places of the other chunks are worked out again in each pass)
+                asm volatile("" : "+v"(k_base));
+            }
+            // V(i+2) with two sets, V(i+1) with one
+            if(INNER)
+            {
+                v_src.V += KEYS * HEAD;
+            }
+            else
+            {
+                advance(v_src);
+                load_v(v_set);
+            }
+            scores(buf ^ 1, s_nxt, [&](int t) __attribute__((always_inline))
+            {
+#pragma unroll
+                for(int n = 0; n < 8 * UPT; ++n)
+                {
+                    if(INNER && n >= t * 8 * UPT / NS && n < (t + 1) * 8 * UPT / NS)
+                    {
+                        load_v_piece(v_set, n);
+                    }
+                }
+#pragma unroll
+                for(int n = 0; n < NA; ++n)
+                {
+                    if(n >= t * NA / NS && n < (t + 1) * NA / NS)
+                    {
+                        item_a(n, buf, s);
+                    }
+                }
+            }, [](int) {});
+            __syncthreads();
+            // (V(i) was written behind the last barrier: read behind this one, and
+            // behind the reads what needs no operand)
+            first_v(buf);
+            pieces_b(s);
+            // K(i+4) with two sets, K(i+3) with one
+            if(INNER)
+            {
+                k_src.K += KEYS * HEAD;
+            }
+            else
+            {
+                advance(k_src);
+                load_k(k_set);
+            }
+            output(buf, [&](int t) __attribute__((always_inline))
+            {
+#pragma unroll
+                for(int n = 0; n < 2 * UPT; ++n)
+                {
+                    if(INNER && n >= t * 2 * UPT / NP && n < (t + 1) * 2 * UPT / NP)
+                    {
+                        load_k_piece(k_set, n);
+                    }
+                }
+#pragma unroll
+                for(int n = 0; n < NB; ++n)
+                {
+                    if(n >= t * NB / NP && n < (t + 1) * NB / NP)
+                    {
+                        split_v((buf ^ 1) % SETS, n, lds + (2 + (buf ^ 1)) * BUF);
+                    }
+                }
+            }, [&](int n) __attribute__((always_inline)) { read_k(buf, n); });
+            advance(s_src);
+            apply_mask(s_src, s_nxt);
+        };
+        auto two_passes = [&](auto inner_tag) __attribute__((always_inline))
+        {
+            pass(inner_tag, std::integral_constant<int, 0>{}, s_even, s_odd);
+            pass(inner_tag, std::integral_constant<int, 1>{}, s_odd, s_even);
+        };
+        // passes whose two steps of either request lie inside a tile, in pairs
+        auto inner_pairs = [&](const StepSource &src) __attribute__((always_inline)) -> int
+        {
+            return (min(src.rows_left / KEYS, last_step - src.step + 1) - 1) / 2;
+        };
+        int pairs = last_step / 2;
+#pragma unroll 1
+        while(pairs > 0)
+        {
+            const int inner = min(pairs, min(inner_pairs(k_src), inner_pairs(v_src)));
+#pragma unroll 1
+            for(int n = 0; n < inner; ++n)
+            {
+                two_passes(std::integral_constant<bool, true>{});
+            }
+            auto inside = [&](StepSource &src) __attribute__((always_inline))
+            {
+                src.step += 2 * inner;
+                src.rows_left -= 2 * inner * KEYS;
+                src.k_row0 += 2 * inner * KEYS;
+                src.k_pos += 2 * inner * KEYS;
+            };
+            inside(k_src);
+            inside(v_src);
+            pairs -= inner;
+            if(pairs > 0)
+            {
+                two_passes(std::integral_constant<bool, false>{});
+                --pairs;
+            }
+        }
+        if(last_step & 1)
+        {
+            pass(std::integral_constant<bool, false>{}, std::integral_constant<int, 0>{}, s_even, s_odd);
+            s_even = s_odd;
+        }
+        __syncthreads();
+#pragma unroll
+        for(int n = 0; n < 21; ++n)
+        {
+            item_a(n, 0, s_even);
+        }
+        first_v(last_step & 1);
+        pieces_b(s_even);
+        output(last_step & 1, [](int) {}, [](int) {});
+    }
+
+    // ---- results that the pieces could not carry: once more in fp32 --------------------
+    // (A row whose output is far below the values of V it was taken from had its V
+    // in the last bits of the pieces.)
+    if(n_steps > 0)
+    {
+        float o_max = 0.0f, o_sum = 0.0f;
+#pragma unroll
+        for(int db = 0; db < DB; ++db)
+        {
+#pragma unroll
+            for(int r = 0; r < 16; ++r)
+            {
+                o_max = fmaxf(o_max, __builtin_fabsf(o[db][r]));
+                o_sum += o[db][r];
+            }
+        }
+        o_max = max_across_halves(o_max);
+        const float l_row = sum_across_halves(l_run);
+        // (a NaN or an infinity among the outputs is one in their sum)
+        odd = odd || !(l_row < __builtin_huge_valf())
+            || !(__builtin_fabsf(o_sum) < __builtin_huge_valf())
+            || (o_max > 0.0f && o_max < 0x1p-6f * l_row) || too_small != 0;
+        if(__builtin_amdgcn_ballot_w64(odd && q_ok) != 0 || too_small != 0)
+        {
+            any_odd = 1;
+        }
+        __syncthreads();
+        if(any_odd != 0)
+        {
+            qk_back = 1.0f;
+            to_scores = kScaleHi;
+            c = EXPLICIT ? kLog2e : kScaleLog2e;
+            v_back = 1.0f;
+            p_exp = 0.0f;
+            m_run = neg_inf();
+            l_run = l_low = 0.0f;
+#pragma unroll
+            for(int db = 0; db < DB; ++db)
+            {
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    o[db][r] = 0.0f;
+                }
+            }
+            const float *Qrow = Qt + my_row() * HEAD;
+#pragma unroll 1
+            for(StepSource src = first_step();; advance(src))
+            {
+                const int last = src.rows_left - 1;
+                f32x16 s;
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    s[r] = 0.0f;
+                }
+                const float *Krow = src.K + (int64_t)min(grp * kX2Rows + col, last) * HEAD;
+#pragma unroll 1
+                for(int j = half; j < HEAD; j += 2)
+                {
+                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(Krow[j], q_ok ? Qrow[j] : 0.0f, s, 0, 0, 0);
+                }
+                apply_mask(src, s);
+                softmax_head(s);
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    softmax_one(s, r);
+                }
+                l_low = 0.0f;       // (of an infinite sum: NaN)
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    const int key = grp * kX2Rows + 8 * (r >> 2) + 4 * half + (r & 3);
+                    const float *Vrow = src.V + (int64_t)min(key, last) * HEAD + col;
+#pragma unroll
+                    for(int db = 0; db < DB; ++db)
+                    {
+                        o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(Vrow[32 * db], s[r], o[db], 0, 0, 0);
+                    }
+                }
+                if(src.step + 1 == n_steps)
+                {
+                    break;
+                }
+            }
+        }
+        if(!EXPLICIT && m_run != neg_inf())
+        {
+            const float m = m_run * qk_back;
+            m_run = fmaf(m, kScaleHi, m * kScaleLo);        // the maximum of the scores
+        }
+        const float p_back = p_exp == 0.0f ? 1.0f : 0x1p-4f;
+        l_run *= p_back;
+        v_back *= p_back;
+#pragma unroll
+        for(int db = 0; db < DB; ++db)
+        {
+#pragma unroll
+            for(int r = 0; r < 16; ++r)
+            {
+                o[db][r] *= v_back;
+            }
+        }
+    }
+
+    // ---- the key blocks' results into those of the first ---------------------------------
+    if constexpr(G > 1)
+    {
+        // word w of lane l of wavefront (q, g > 0) sits at (((g-1)*QW + q)*NW + w)*64 + l
+        constexpr int NW = 2 + 16 * DB;
+        static_assert((G - 1) * QW * NW * 256 <= 4 * BUF, "exchange area does not fit");
+        float *area = reinterpret_cast<float *>(lds);
+        __syncthreads();        // everyone is done with the buffers
+        if(grp > 0)
+        {
+            float *dst = area + ((grp - 1) * QW + qw) * NW * 64 + lane;
+            dst[0] = m_run;
+            dst[64] = l_run;
+#pragma unroll
+            for(int db = 0; db < DB; ++db)
+            {
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    dst[(2 + 16 * db + r) * 64] = o[db][r];
+                }
+            }
+        }
+        __syncthreads();
+        if(grp > 0)
+        {
+            return;
+        }
+#pragma unroll
+        for(int v = 0; v < G - 1; ++v)
+        {
+            const float *src = area + (v * QW + qw) * NW * 64 + lane;
+            const float m_other = src[0];
+            const float m_new = fmaxf(m_run, m_other);
+            const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
+            const float a_mine = fast_exp2((m_run - m_use) * kLog2e);
+            const float a_other = fast_exp2((m_other - m_use) * kLog2e);
+            l_run = l_run * a_mine + src[64] * a_other;
+#pragma unroll
+            for(int db = 0; db < DB; ++db)
+            {
+#pragma unroll
+                for(int r = 0; r < 16; ++r)
+                {
+                    o[db][r] = o[db][r] * a_mine + src[(2 + 16 * db + r) * 64] * a_other;
+                }
+            }
+            m_run = m_new;
+        }
+    }
+
+    // ---- epilogue ---------------------------------------------------------------------
+    const float l_tot = l_run + __shfl_xor(l_run, 32);
+    // no visible key for this query (a NaN among its scores: as in the 16-bit kernel)
+    const bool empty = l_tot == 0.0f;
+    if constexpr(PARTS)
+    {
+        if(q_ok)
+        {
+            // (a sum that is NaN goes out as it is, with some finite maximum)
+            const int64_t row = ((int64_t)part * p.batch + b) * p.q_seq + my_row();
+            if(half == 0)
+            {
+                p.part_ml[2 * row] = empty ? neg_inf() : l_tot > 0.0f ? m_run : 0.0f;
+                p.part_ml[2 * row + 1] = l_tot;
+            }
+            float *dst = p.part_o + row * HEAD + 4 * half;
+#pragma unroll
+            for(int db = 0; db < DB; ++db)
+            {
+#pragma unroll
+                for(int rg = 0; rg < 4; ++rg)
+                {
+                    f32x4 v;
+#pragma unroll
+                    for(int e = 0; e < 4; ++e)
+                    {
+                        v[e] = empty ? 0.0f : o[db][4 * rg + e];
+                    }
+                    *reinterpret_cast<f32x4 *>(dst + 32 * db + 8 * rg) = v;
+                }
+            }
+        }
+        return;
+    }
+    if(!q_ok || !(l_tot > 0.0f || p.overwrite))
+    {
+        return;     // leave lse and A as they are
+    }
+    const float lse_new = empty ? neg_inf() : m_run + __logf(l_tot);
+    float *lse_ptr = p.lse[q_tile0 + qt] + (int64_t)b * q_len + my_row();
+    const float lse_old = p.overwrite ? neg_inf() : *lse_ptr;
+    float w_old = 0.0f, w_new = 0.0f, lse_out = neg_inf();
+    if(!empty)
+    {
+        merge_weights(lse_old, lse_new, w_old, w_new, lse_out);
+    }
+    if(half == 0)
+    {
+        *lse_ptr = lse_out;
+    }
+    const float w_o = empty ? 0.0f : w_new / l_tot;
+    float *Arow = static_cast<float *>(p.A[q_tile0 + qt]) + ((int64_t)b * q_len + my_row()) * HEAD;
+#pragma unroll
+    for(int db = 0; db < DB; ++db)
+    {
+#pragma unroll
+        for(int rg = 0; rg < 4; ++rg)
+        {
+            float *dst = Arow + db * 32 + 8 * rg + 4 * half;
+            f32x4 v;
+#pragma unroll
+            for(int e = 0; e < 4; ++e)
+            {
+                v[e] = empty ? 0.0f : o[db][4 * rg + e] * w_o;
+            }
+            if(w_old != 0.0f)
+            {
+                const f32x4 old = *reinterpret_cast<const f32x4 *>(dst);
+#pragma unroll
+                for(int e = 0; e < 4; ++e)
+                {
+                    v[e] += w_old * old[e];
+                }
+            }
+            *reinterpret_cast<f32x4 *>(dst) = v;
+        }
+    }
+}
+
+template<int HEAD, int QW, int G>
+static int launch_form(hipStream_t stream, PrefillParams &p, int mode)
+{
+    p.k_blocks_per_tile = (int)((p.k_tile + kX2Rows * G - 1) / (kX2Rows * G));
+    p.q_blocks_per_tile = (int)((p.q_tile + kX2Rows * QW - 1) / (kX2Rows * QW));
+    const int64_t n_wg = (int64_t)p.batch * p.n_slabs * p.n_q_tiles * p.q_blocks_per_tile;
+    if(n_wg <= 0 || n_wg > 0x7fffffff)
+    {
+        return NNTILE_HIP_EINVAL;
+    }
+    auto launch = [&](auto kernel) -> int
+    {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)n_wg), dim3(64 * QW * G), 0, stream, p);
+        return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+    };
+    if(mode == NNTILE_HIP_MASK_NONE)
+    {
+        return launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_NONE, QW, G>);
+    }
+    if(mode == NNTILE_HIP_MASK_CAUSAL)
+    {
+        return launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_CAUSAL, QW, G>);
+    }
+    if constexpr(QW * G == 4)       // (masks given as values)
+    {
+        return mode == NNTILE_HIP_MASK_ADDITIVE
+            ? launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_ADDITIVE, QW, G>)
+            : launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_BOOL, QW, G>);
+    }
+    return NNTILE_HIP_EINVAL;
+}
+
+template<int HEAD>
+static int launch_head(hipStream_t stream, PrefillParams &p, int mode, int form)
+{
+    if constexpr(HEAD > 32)
+    {
+        if(form == kF16x2Form42)
+        {
+            return launch_form<HEAD, 4, 2>(stream, p, mode);
+        }
+        if(form == kF16x2Form81)
+        {
+            return launch_form<HEAD, 8, 1>(stream, p, mode);
+        }
+    }
+    return form == kF16x2Form22 ? launch_form<HEAD, 2, 2>(stream, p, mode)
+        : launch_form<HEAD, 4, 1>(stream, p, mode);
+}
+
+// The form that is expected to be done first; kF16x2None: the fp32 kernel's
+// 32-query workgroups.
+//
+// A launch takes a fixed time (launch, prologue, epilogue), then the longer of two:
+// the longest workgroup's walk, at the time of a pass when it has the CU to
+// itself, and the passes that a CU gets, at the time a pass adds to a full one; a
+// second and third round of workgroups start anew.  The times are fitted to
+// launches of 1 to 200 heads of 64 to 8192 rows, causal and not, 4 to 8 % off in
+// the mean; what the rule picks is within 1 to 2.5 % of the fastest of the five in
+// the mean.  us, the fp32 kernel's 32 queries / 22 / 41 / 42 / 81 - head 64, causal:
+// 12 x 128 7.9 / 9.4 / 11.5 / 11.7 / 13.1; 12 x 1024 30 / 25 / 35 / 29 / 49; 48 x 1024
+// 75 / 40.3 / 40.1 / 38.3 / 51; 200 x 1024 293 / 144 / 117 / 145 / 138; 12 x 4096 251 /
+// 112 / 129 / 103 / 161; 32 x 4096 619 / 275 / 238 / 240 / 226.  Head 128, 48 x 1024: 177 /
+// 90 / 67 / 63 / 75; without a mask 290 / 134 / 96 / 110 / 84; 32 x 4096 1490 / 648 / 432 /
+// 444 / 386.
+int prefill_f16x2_form(const PrefillParams &p, int head, int mode)
+{
+    struct Cost
+    {
+        int form, rows, keys;
+        double fixed, alone, full, round;      // us: launch, pass, pass on a full CU, round
+    };
+    static const Cost costs[3][5] = {
+        {{kF16x2None, 32, 128, 4.5, 1.59, 1.25, 0.5}, {kF16x2Form22, 64, 64, 6.6, 0.76, 0.58, 1.5},
+            {kF16x2Form41, 128, 32, 6.6, 0.77, 0.56, 1.5}},
+        {{kF16x2None, 32, 128, 5.1, 2.74, 2.50, 1.2}, {kF16x2Form22, 64, 64, 7.7, 1.13, 1.00, 2.3},
+            {kF16x2Form41, 128, 32, 7.7, 0.90, 0.78, 2.6}, {kF16x2Form42, 128, 64, 8.8, 1.31, 1.50, 7.0},
+            {kF16x2Form81, 256, 32, 8.2, 1.30, 1.40, 9.0}},
+        {{kF16x2None, 32, 128, 7.2, 5.23, 5.50, 5.0}, {kF16x2Form22, 64, 64, 10.4, 2.17, 2.33, 8.7},
+            {kF16x2Form41, 128, 32, 9.4, 1.55, 1.31, 5.5}, {kF16x2Form42, 128, 64, 12.2, 2.30, 2.75, 11.0},
+            {kF16x2Form81, 256, 32, 10.3, 2.00, 2.85, 0.0}}};
+    const bool causal = mode == NNTILE_HIP_MASK_CAUSAL;
+    const bool values = mode == NNTILE_HIP_MASK_ADDITIVE || mode == NNTILE_HIP_MASK_BOOL;
+    int best = kF16x2None;
+    double least = 0.0;
+    for(const Cost &f : costs[head == 128 ? 2 : head == 64 ? 1 : 0])
+    {
+        // (head 32 and masks given as values: the small forms)
+        if(f.rows == 0 || (values && f.form > kF16x2Form41))
+        {
+            continue;
+        }
+        const int64_t blocks = (p.q_tile + f.rows - 1) / f.rows;
+        const double wgs = (double)p.batch * p.n_slabs * p.n_q_tiles * blocks / 256.0;    // per CU
+        const double rounds = ceil(wgs) - 1.0;
+        auto passes = [&](int64_t last_row)
+        {
+            const int64_t keys = causal
+                ? last_row + p.q_pos0 - p.k_pos0 + p.causal_offset + 1 : p.k_seq;
+            return ceil((double)(keys < 1 ? 1 : keys < p.k_seq ? keys : p.k_seq) / f.keys);
+        };
+        const double most = passes(p.q_seq - 1), first = passes((p.q_seq < f.rows ? p.q_seq : f.rows) - 1);
+        double t = f.fixed + f.round * rounds;
+        if(causal)
+        {
+            const double shared = 0.5 * (most + first) * wgs * f.full + (wgs > 1.0 ? 0.5 * first * f.full : 0.0);
+            t += most * f.alone > shared ? most * f.alone : shared;
+        }
+        else
+        {
+            t += wgs <= 1.0 ? most * f.alone : most * ceil(wgs) * f.full;
+        }
+        // (a close call stays with the fp32 kernel)
+        if(f.form == kF16x2None)
+        {
+            t *= 0.94;
+        }
+        if(f.form == kF16x2None || t < least)
+        {
+            best = f.form;
+            least = t;
+        }
+    }
+    return best;
+}
+
+int launch_prefill_f16x2(hipStream_t stream, PrefillParams &p, int head, int mode, int form)
+{
+    if(mode < NNTILE_HIP_MASK_ADDITIVE || mode > NNTILE_HIP_MASK_BOOL)
+    {
+        return NNTILE_HIP_EINVAL;
+    }
+    if(form > kF16x2Form41 && mode != NNTILE_HIP_MASK_NONE && mode != NNTILE_HIP_MASK_CAUSAL)
+    {
+        form = kF16x2Form41;
+    }
+    switch(head)
+    {
+        case 32:
+            return launch_head<32>(stream, p, mode, form);
+        case 64:
+            return launch_head<64>(stream, p, mode, form);
+        case 128:
+            return launch_head<128>(stream, p, mode, form);
+        default:
+            return NNTILE_HIP_EUNSUPPORTED;
+    }
+}
+
+} // namespace nntile_hip

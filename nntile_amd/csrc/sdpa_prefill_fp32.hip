@@ -15,18 +15,14 @@
 // unpadded and their 16-byte chunks XOR-swizzled by row against bank
 // conflicts, as in the 16-bit kernel.
 //
-// Two forms:
-//   * 128 queries per workgroup, four wavefronts of 32 queries sharing every
-//     key step: two LDS buffers per operand, the loads of step g+1 issued at
-//     the top of step g, one barrier per step;
-//   * SPLIT, for launches with fewer such workgroups than CUs: a workgroup is
-//     32 queries and its four wavefronts take every fourth key step each, each
-//     through its own LDS buffer - K of the next step is requested when the
-//     scores of this one are done, V when its output products are, and there
-//     is no barrier in the loop; at the end the four merge their (max, sum, O)
-//     through LDS.  The chain of dependent steps a wavefront walks, which
-//     bounds such a launch, is a quarter as long, and four times as many
-//     workgroups spread over the CUs.
+// A workgroup is 32 queries and its four wavefronts take every fourth key step
+// each, each through its own LDS buffer - K of the next step is requested when
+// the scores of this one are done, V when its output products are, and there is
+// no barrier in the loop; at the end the four merge their (max, sum, O) through
+// LDS.  The chain of dependent steps a wavefront walks, which bounds a small
+// launch, is a quarter as long, and four times as many workgroups spread over
+// the CUs.  Launches that fill the chip run on the fp16 matrix units instead
+// (sdpa_prefill_f16x2.hip, prefill_f16x2_form says which).
 #include <type_traits>
 
 #include "sdpa_mask_scan.hpp"
@@ -44,36 +40,14 @@ namespace nntile_hip
 #define F32_STAMP_DECL
 #define F32_STAMP_DUMP
 #endif
-// SPLIT form: the softmax of the previous step behind every score MFMA (1) or
+// The softmax of the previous step behind every score MFMA (1) or
 // behind the first of each group of four (0)
 #ifndef NNTILE_F32_FINE
 #define NNTILE_F32_FINE 0
 #endif
-// Launches with fewer 128-query workgroups than this take the SPLIT form.
-// Measured crossovers (fused launches of batch x seq x head, 100 launches
-// each): under a causal mask the 32-query workgroups, dealt longest first,
-// fill the triangle far better - head 64: 48 x 1024 81.7 us against 139.5,
-// 32 x 4096 619 against 771, 192 x 2048 1005 against 1087, and only at 384 x
-// 2048 (6144 such workgroups) 2301 against 2022; head 128: 96 x 1024 353
-// against 385, 64 x 2048 809 against 820, 96 x 2048 1227 against 1118.
-// Without a mask the shared key steps win earlier: head 64, 48 x 1024 122
-// against 139, 96 x 1024 243 against 202.
-static int split_below(int head, int mode)
-{
-#ifdef NNTILE_F32_SPLIT_BELOW
-    return NNTILE_F32_SPLIT_BELOW;
-#else
-    const bool causal = mode == NNTILE_HIP_MASK_CAUSAL;
-    if(head >= 128)
-    {
-        return causal ? 1025 : 256;
-    }
-    return causal ? 4096 : 512;
-#endif
-}
-constexpr int kQRows32 = 128;
+constexpr int kQRows32 = 32;
 constexpr int kKeys32 = 32;
-constexpr int kThreads32 = 256;          // 4 wavefronts in both forms
+constexpr int kThreads32 = 256;          // 4 wavefronts
 
 template<int N> __device__ __forceinline__ void f32_wait_vmcnt()
 {
@@ -85,12 +59,12 @@ template<int N> __device__ __forceinline__ void f32_wait_vmcnt()
 
 // PARTS: the workgroup takes one of p.n_parts ranges of the keys and leaves its
 // triple in memory (PrefillParams::part_o) for launch_parts_merge.
-template<int HEAD, int MODE, bool SPLIT, bool PARTS = false>
-__global__ __launch_bounds__(kThreads32, (SPLIT && HEAD == 128) ? 1 : 2)
+template<int HEAD, int MODE, bool PARTS = false>
+__global__ __launch_bounds__(kThreads32, HEAD == 128 ? 1 : 2)
 void sdpa_prefill_fp32_kernel(const PrefillParams p)
 {
-    constexpr int QROWS = SPLIT ? 32 : kQRows32;    // queries per workgroup
-    constexpr int NSUB = SPLIT ? 4 : 1;     // key steps in flight side by side (one per wavefront)
+    constexpr int QROWS = kQRows32;         // queries per workgroup
+    constexpr int NSUB = 4;                 // key steps in flight side by side (one per wavefront)
     constexpr int QSTEPS = HEAD / 8;        // 16-byte groups per lane half along head
     constexpr int DBLOCKS = HEAD / 32;
     constexpr int RB = HEAD * 4;            // bytes per K/V row
@@ -99,22 +73,18 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     constexpr int KSW = CPR >= 16 ? 16 : CPR;       // K: chunk c of row r at c ^ ((r / RPL) % KSW)
     constexpr int ROWS_PER_LOAD = 1024 / RB;        // rows one load instruction fills
     constexpr int LOADS = kKeys32 / ROWS_PER_LOAD;  // load instructions per K (or V) step
-    constexpr int LPW = SPLIT ? LOADS : LOADS / 4;  // ... of them issued by one wavefront
+    constexpr int LPW = LOADS;              // ... all of them issued by one wavefront
     constexpr int BLOCK_BYTES = kKeys32 * RB;
     constexpr bool EXPLICIT = (MODE == NNTILE_HIP_MASK_ADDITIVE
             || MODE == NNTILE_HIP_MASK_BOOL);
-    static_assert(!PARTS || (SPLIT && !EXPLICIT), "parts: analytic masks, 32-query workgroups");
+    static_assert(!PARTS || !EXPLICIT, "parts: analytic masks");
     static_assert(LPW >= 1, "head size does not fit this tiling");
 
-    // SPLIT: lds_k0 / lds_v0 hold one step per wavefront (wavefront w owns
-    // bytes [w * BLOCK_BYTES, +BLOCK_BYTES)); lds_k1 / lds_v1 are not used.
-    // Otherwise step g of the workgroup lives in lds_k[g % 2], lds_v[g % 2].
+    // One step per wavefront: wavefront w owns bytes [w * BLOCK_BYTES, +BLOCK_BYTES).
     // (Separate arrays: the compiler then knows that what streams into one
     // cannot alias the reads of another.)
     __shared__ __attribute__((aligned(1024))) char lds_k0[NSUB * BLOCK_BYTES];
     __shared__ __attribute__((aligned(1024))) char lds_v0[NSUB * BLOCK_BYTES];
-    __shared__ __attribute__((aligned(1024))) char lds_k1[SPLIT ? 16 : BLOCK_BYTES];
-    __shared__ __attribute__((aligned(1024))) char lds_v1[SPLIT ? 16 : BLOCK_BYTES];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -153,9 +123,9 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         b = wg % batch_all;
         qblk = q_blocks - 1 - wg / batch_all;
     }
-    else if(SPLIT)
+    else
     {
-        // A launch of this form fits the GPU at once, so where a workgroup
+        // A launch that fits the GPU at once: where a workgroup
         // lands decides how evenly the CUs are loaded.  Workgroups are dealt
         // round-robin to the 8 XCDs; each XCD puts its first 32 on its 32 CUs
         // and the next ones beside them, i + 32 next to i.  Query blocks go out
@@ -171,16 +141,6 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         const int k = (i << 3) | (wg & 7);
         b = k % batch_all;
         qblk = q_blocks - 1 - k / batch_all;
-    }
-    else
-    {
-        if(p.xcd_remap)
-        {
-            const int per_xcd = gridDim.x >> 3;
-            wg = (wg & 7) * per_xcd + (wg >> 3);
-        }
-        b = wg / q_blocks;
-        qblk = q_blocks - 1 - (wg % q_blocks);
     }
     // the slab of this entry: its tiles are allocations of their own
     int q_tile0 = 0, k_tile0 = 0;
@@ -203,7 +163,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
 
     const float *Qt = static_cast<const float *>(p.Q[q_tile0 + qt])
         + (int64_t)b * q_len * HEAD;
-    const int64_t my_q = q_row0 + (SPLIT ? 0 : wave * 32) + col;
+    const int64_t my_q = q_row0 + col;
     const bool q_ok = my_q < q_len;
     const int64_t my_qpos = p.q_pos0 + (int64_t)qt * p.q_tile + my_q;
 
@@ -224,9 +184,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         + (int)((last_k_len + kKeys32 - 1) / kKeys32);
     const int64_t wg_qpos_hi = p.q_pos0 + (int64_t)qt * p.q_tile
         + min(q_row0 + QROWS, q_len) - 1;
-    const int64_t wave_qpos_lo = p.q_pos0 + (int64_t)qt * p.q_tile + q_row0
-        + (SPLIT ? 0 : wave * 32);
-    const int64_t wave_qpos_hi = wave_qpos_lo + 31;
+    const int64_t wave_qpos_lo = p.q_pos0 + (int64_t)qt * p.q_tile + q_row0;
 
     // ---- LDS layout and the lane's fixed addresses ---------------------------
     // A step's K (and V) block is 32 rows of RB bytes, unpadded.  The 16-byte
@@ -245,8 +203,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
 #pragma unroll
     for(int i = 0; i < LPW; ++i)
     {
-        const int ld = SPLIT ? i : wave * LPW + i;
-        const int r = ld * ROWS_PER_LOAD + lane / CPR;
+        const int r = i * ROWS_PER_LOAD + lane / CPR;
         ld_row[i] = r;
         k_goff[i] = (uint32_t)(r * RB + (ld_cpos ^ ((r / RPL) % KSW)) * 16);
         v_goff[i] = (uint32_t)(r * RB + (ld_cpos ^ (VSW * ((r >> 2) & 1))) * 16);
@@ -306,7 +263,7 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     // keys are masked out of the scores, so their probabilities are exactly 0.
     auto fetch = [&](const char *src, int rows_left, const uint32_t (&goff)[LPW], char *dst_base)
     {
-        char *dst = dst_base + wave_u * (SPLIT ? BLOCK_BYTES : LPW * 1024);
+        char *dst = dst_base + wave_u * BLOCK_BYTES;
         if(rows_left >= kKeys32)
         {
 #pragma unroll
@@ -566,46 +523,6 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
         }
     };
 
-    // Online softmax of the scores (they become the probabilities) and the
-    // rescale of what has been accumulated.
-    auto softmax = [&](f32x16 &s) __attribute__((always_inline))
-    {
-        float mx = neg_inf();
-#pragma unroll
-        for(int r = 0; r < 16; ++r)
-        {
-            mx = fmaxf(mx, s[r]);
-        }
-        mx = max_across_halves(mx);
-        const float m_new = fmaxf(m_run, mx);
-        const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
-        const float mc = m_use * c;
-        // the running maximum rarely moves after the first steps
-        if(__builtin_amdgcn_ballot_w64(m_new != m_run) != 0)
-        {
-            const float alpha = fast_exp2((m_run - m_use) * c);
-            l_run *= alpha;
-#pragma unroll
-            for(int db = 0; db < DBLOCKS; ++db)
-            {
-#pragma unroll
-                for(int r = 0; r < 16; ++r)
-                {
-                    o[db][r] *= alpha;
-                }
-            }
-            m_run = m_new;
-        }
-        float rs = 0.0f;
-#pragma unroll
-        for(int r = 0; r < 16; ++r)
-        {
-            s[r] = fast_exp2(fmaf(s[r], c, -mc));
-            rs += s[r];
-        }
-        l_run += rs;
-    };
-
     // O^T += V^T P^T from the V block at Vw: MFMA n of the 16 * DBLOCKS takes
     // key n / DBLOCKS and output block n % DBLOCKS; its V operand is read from
     // LDS eight MFMAs ahead.  `between(n)` is called after MFMA n.
@@ -644,26 +561,12 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     auto fetch_piece = [&](const char *src, int rows_left, const uint32_t (&goff)[LPW],
             char *dst_base, int i) __attribute__((always_inline))
     {
-        char *dst = dst_base + wave_u * (SPLIT ? BLOCK_BYTES : LPW * 1024);
+        char *dst = dst_base + wave_u * BLOCK_BYTES;
         const int last = rows_left - 1;
         const uint32_t back = (uint32_t)(max(ld_row[i] - last, 0) * RB);
         load_to_lds16<0, false>(src, goff[i] - back, dst + i * 1024);
     };
 
-    // nothing of key step g is visible to this wavefront
-    auto hidden = [&](int g) -> bool
-    {
-        if(MODE != NNTILE_HIP_MASK_CAUSAL)
-        {
-            return false;
-        }
-        const int kt = g / p.k_blocks_per_tile;
-        const int kb = g % p.k_blocks_per_tile;
-        const int64_t k_pos_base = k_pos0() + (int64_t)kt * k_tile() + (int64_t)kb * kKeys32;
-        return k_pos_base > wave_qpos_hi + p.causal_offset;
-    };
-
-    if constexpr(SPLIT)
     {
         // ---- every wavefront walks its own key steps wave, wave + 4, ... ---------
         // through two buffers of its own and shares nothing with the others
@@ -866,50 +769,8 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
             f32_wait_vmcnt<0>();
         }
     }
-    else
-    {
-        // ---- the four wavefronts share every key step ------------------------------
-        if(n_steps > 0)
-        {
-            const StepSource src = locate(n_skip);
-            fetch(src.K, src.rows_left, k_goff, lds_k0);
-            fetch(src.V, src.rows_left, v_goff, lds_v0);
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        auto step = [&](int g, auto buf_tag) __attribute__((always_inline))
-        {
-            constexpr int BUF = decltype(buf_tag)::value;
-            // loads of the next step into the other buffers (every wavefront
-            // passed the barrier that ended step g-1: nobody reads them)
-            if(g + 1 < n_steps)
-            {
-                const StepSource nxt = locate(n_skip + g + 1);
-                fetch(nxt.K, nxt.rows_left, k_goff, BUF ? lds_k0 : lds_k1);
-                fetch(nxt.V, nxt.rows_left, v_goff, BUF ? lds_v0 : lds_v1);
-            }
-            if(!hidden(g))
-            {
-                f32x16 s;
-                scores(n_skip + g, BUF ? lds_k1 : lds_k0, s, nothing);
-                softmax(s);
-                output(BUF ? lds_v1 : lds_v0, s, nothing);
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-        };
-        for(int g = 0; g < n_steps; g += 2)
-        {
-            step(g, std::integral_constant<int, 0>{});
-            if(g + 1 < n_steps)
-            {
-                step(g + 1, std::integral_constant<int, 1>{});
-            }
-        }
-    }
 
-    // ---- SPLIT: merge the four wavefronts' results into wavefront 0 ----------------
-    if constexpr(SPLIT)
+    // ---- merge the four wavefronts' results into wavefront 0 ---------------------------
     {
         // word w of lane l of wavefront v (v = 1..3) sits at ((v-1)*NW + w)*64 + l
         constexpr int NW = 2 + 16 * DBLOCKS;
@@ -1046,36 +907,28 @@ void sdpa_prefill_fp32_kernel(const PrefillParams p)
     F32_STAMP_DUMP
 }
 
-template<int HEAD, bool SPLIT>
+template<int HEAD>
 static int launch_mode32(hipStream_t stream, const PrefillParams &p, int mode,
         dim3 grid)
 {
+    auto launch = [&](auto kernel) -> int
+    {
+        hipLaunchKernelGGL(kernel, grid, dim3(kThreads32), 0, stream, p);
+        return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+    };
     switch(mode)
     {
         case NNTILE_HIP_MASK_ADDITIVE:
-            hipLaunchKernelGGL((sdpa_prefill_fp32_kernel<HEAD,
-                        NNTILE_HIP_MASK_ADDITIVE, SPLIT>), grid, dim3(kThreads32), 0,
-                    stream, p);
-            break;
+            return launch(sdpa_prefill_fp32_kernel<HEAD, NNTILE_HIP_MASK_ADDITIVE>);
         case NNTILE_HIP_MASK_NONE:
-            hipLaunchKernelGGL((sdpa_prefill_fp32_kernel<HEAD,
-                        NNTILE_HIP_MASK_NONE, SPLIT>), grid, dim3(kThreads32), 0,
-                    stream, p);
-            break;
+            return launch(sdpa_prefill_fp32_kernel<HEAD, NNTILE_HIP_MASK_NONE>);
         case NNTILE_HIP_MASK_CAUSAL:
-            hipLaunchKernelGGL((sdpa_prefill_fp32_kernel<HEAD,
-                        NNTILE_HIP_MASK_CAUSAL, SPLIT>), grid, dim3(kThreads32), 0,
-                    stream, p);
-            break;
+            return launch(sdpa_prefill_fp32_kernel<HEAD, NNTILE_HIP_MASK_CAUSAL>);
         case NNTILE_HIP_MASK_BOOL:
-            hipLaunchKernelGGL((sdpa_prefill_fp32_kernel<HEAD,
-                        NNTILE_HIP_MASK_BOOL, SPLIT>), grid, dim3(kThreads32), 0,
-                    stream, p);
-            break;
+            return launch(sdpa_prefill_fp32_kernel<HEAD, NNTILE_HIP_MASK_BOOL>);
         default:
             return NNTILE_HIP_EINVAL;
     }
-    return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
 }
 
 // One tile against a long key axis, the keys in p.n_parts ranges (see
@@ -1099,54 +952,68 @@ int launch_prefill_fp32_parts(hipStream_t stream, PrefillParams &p, int head, in
     {
         case 64:
             return causal
-                ? launch(sdpa_prefill_fp32_kernel<64, NNTILE_HIP_MASK_CAUSAL, true, true>)
-                : launch(sdpa_prefill_fp32_kernel<64, NNTILE_HIP_MASK_NONE, true, true>);
+                ? launch(sdpa_prefill_fp32_kernel<64, NNTILE_HIP_MASK_CAUSAL, true>)
+                : launch(sdpa_prefill_fp32_kernel<64, NNTILE_HIP_MASK_NONE, true>);
         case 128:
             return causal
-                ? launch(sdpa_prefill_fp32_kernel<128, NNTILE_HIP_MASK_CAUSAL, true, true>)
-                : launch(sdpa_prefill_fp32_kernel<128, NNTILE_HIP_MASK_NONE, true, true>);
+                ? launch(sdpa_prefill_fp32_kernel<128, NNTILE_HIP_MASK_CAUSAL, true>)
+                : launch(sdpa_prefill_fp32_kernel<128, NNTILE_HIP_MASK_NONE, true>);
         default:
             return NNTILE_HIP_EUNSUPPORTED;
     }
 }
 
+// p.form: 0 what prefill_f16x2_form picks; 1 shared key steps (128 queries, fp16
+// pairs), 2 split key steps (32 queries, fp32 products); from 8 on the other forms
+// on fp16 pairs: 8 256 queries, 9 128 queries and two key blocks, 10 64 queries and
+// two key blocks (masks given as values: 8 and 9 as 1).
 int launch_prefill_fp32(hipStream_t stream, PrefillParams &p, int head, int mode)
 {
-    p.k_blocks_per_tile = (int)((p.k_tile + kKeys32 - 1) / kKeys32);
-    // the kernel addresses the rows of a key tile with 32-bit element offsets
+    // the kernels address the rows of a key tile with 32-bit element offsets
     if(p.k_tile * head >= ((int64_t)1 << 31))
     {
         return NNTILE_HIP_EUNSUPPORTED;
     }
-    // with fewer 128-query workgroups than CUs, or query tiles so short that
-    // half of such a workgroup's wavefronts would have no rows (the new tokens
-    // of a decode step), 32-query workgroups whose wavefronts share the keys
-    // instead
-    const int64_t batch_all = (int64_t)p.batch * p.n_slabs;
-    const int64_t n_wide = batch_all * p.n_q_tiles
-        * ((p.q_tile + kQRows32 - 1) / kQRows32);
-    const bool split = p.form != 0 ? p.form == 2
-        : (n_wide < split_below(head, mode) || p.q_tile <= 64);
-    const int q_rows = split ? 32 : kQRows32;
-    p.q_blocks_per_tile = (int)((p.q_tile + q_rows - 1) / q_rows);
-    const int64_t n_wg = batch_all * p.n_q_tiles * p.q_blocks_per_tile;
+    int form = kF16x2None;
+    switch(p.form)
+    {
+        case 0:
+            form = prefill_f16x2_form(p, head, mode);
+            break;
+        case 1:
+            form = kF16x2Form41;
+            break;
+        case 2:
+            break;
+        case 9:
+            form = kF16x2Form42;
+            break;
+        case 10:
+            form = kF16x2Form22;
+            break;
+        default:
+            form = kF16x2Form81;
+    }
+    if(form != kF16x2None)
+    {
+        return launch_prefill_f16x2(stream, p, head, mode, form);
+    }
+    p.k_blocks_per_tile = (int)((p.k_tile + kKeys32 - 1) / kKeys32);
+    p.q_blocks_per_tile = (int)((p.q_tile + kQRows32 - 1) / kQRows32);
+    const int64_t n_wg = (int64_t)p.batch * p.n_slabs * p.n_q_tiles * p.q_blocks_per_tile;
     if(n_wg <= 0 || n_wg > 0x7fffffff)
     {
         return NNTILE_HIP_EINVAL;
     }
-    p.xcd_remap = (n_wg % 8 == 0) ? 1 : 0;
     const dim3 grid((unsigned)n_wg);
     switch(head)
     {
         case 32:
-            return split ? launch_mode32<32, true>(stream, p, mode, grid)
-                : launch_mode32<32, false>(stream, p, mode, grid);
+            return launch_mode32<32>(stream, p, mode, grid);
         case 64:
-            return split ? launch_mode32<64, true>(stream, p, mode, grid)
-                : launch_mode32<64, false>(stream, p, mode, grid);
+            return launch_mode32<64>(stream, p, mode, grid);
         case 128:
-            return split ? launch_mode32<128, true>(stream, p, mode, grid)
-                : launch_mode32<128, false>(stream, p, mode, grid);
+            return launch_mode32<128>(stream, p, mode, grid);
         default:
             return NNTILE_HIP_EUNSUPPORTED;
     }

@@ -1,0 +1,202 @@
+"""fp32 tiles on the fp16 matrix units (sdpa_prefill_f16x2.hip): every workgroup
+shape against 64-bit arithmetic at the edges of its steps, and the values that
+two fp16 pieces cannot carry, which the kernel finds and takes in fp32."""
+import numpy as np
+import pytest
+import torch
+
+from nntile_amd import hip_sdpa
+from . import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+S, P, W = hip_sdpa.FORM_SHARED, hip_sdpa.FORM_SPLIT, hip_sdpa.FORM_WIDE
+# query blocks of 32 x key blocks of 32 of a workgroup
+FORMS = {"2x2": W | P, "4x1": S, "4x2": W | S, "8x1": W}
+FP32 = P        # the fp32 kernel
+
+
+def reference(Q, K, V, mask):
+    Q, K, V = (t.double() for t in (Q, K, V))
+    s = torch.matmul(Q, K.transpose(1, 2).contiguous()) / np.sqrt(Q.shape[2])
+    if mask is not None:
+        s = s.masked_fill(~mask, float("-inf"))
+    lse = torch.logsumexp(s, 2)
+    A = torch.matmul(torch.exp(s - lse[..., None]).nan_to_num(0.0), V)
+    return A, lse
+
+
+def call(Q, K, V, mode, flags, mask=None, offset=0):
+    lse = torch.full(Q.shape[:2], 1.5, device="cuda")
+    A = torch.full_like(Q, 0.25, device="cuda")
+    hip_sdpa.sdpa_fwd_tile(K.cuda(), Q.cuda(), mask, lse, V.cuda(), A, mode, causal_offset=offset,
+                           flags=flags | hip_sdpa.OVERWRITE)
+    torch.cuda.synchronize()
+    return A.cpu().double(), lse.cpu().double()
+
+
+def rel(a, b):
+    return float((a - b).norm() / b.norm())
+
+
+def draw(seed, batch, q_seq, k_seq, head):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(batch, n, head, generator=g) for n in (q_seq, k_seq, k_seq)]
+
+
+# one key; one and a half steps of either kind; whole steps; a last row of one
+# query; the pairs of passes of the inner loop, an odd and an even number of them
+SHAPES = [(1, 1), (33, 31), (70, 97), (129, 128), (257, 130), (96, 448), (65, 577), (200, 1000)]
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("head", [32, 64, 128])
+@pytest.mark.parametrize("mode", ["none", "causal", "additive", "bool"])
+def test_against_64_bits(form, head, mode):
+    worst = [0.0, 0.0]
+    for q_seq, k_seq in SHAPES:
+        print("case", form, head, mode, q_seq, k_seq, flush=True)
+        Q, K, V = draw(q_seq * 7 + k_seq, 3, q_seq, k_seq, head)
+        offset = k_seq - q_seq
+        q, k = torch.arange(q_seq)[:, None], torch.arange(k_seq)[None]
+        seen, m, mm = None, None, hip_sdpa.MASK_NONE
+        if mode == "causal":
+            seen, mm = k <= q + offset, hip_sdpa.MASK_CAUSAL
+        elif mode != "none":        # a window, and rows that see nothing
+            seen = ((k - q - offset).abs() <= 70) & (q % 17 != 3)
+            mm = hip_sdpa.MASK_ADDITIVE if mode == "additive" else hip_sdpa.MASK_BOOL
+            m = (H.additive_mask(seen.numpy(), "fp32") if mode == "additive" else seen.clone()).cuda()
+        A, lse = call(Q, K, V, mm, FORMS[form], m, offset)
+        wantA, want = reference(Q, K, V, seen)
+        hidden = torch.isinf(want)
+        assert torch.equal(torch.isinf(lse), hidden) and (A[hidden] == 0).all()
+        if bool(hidden.all()):
+            continue
+        # per product: pieces and the one left out, 6e-8 in the 2-norm; a row's
+        # exponentials: half an ulp of an argument up to 16, 2^-21; sums of a few
+        # hundred roundings of 2^-24
+        assert rel(A[~hidden], wantA[~hidden]) < 1e-6
+        assert float((lse[~hidden] - want[~hidden]).abs().max()) < 1e-6 * (1 + float(want[~hidden].abs().max()))
+
+
+def test_no_further_from_64_bits_than_fp32_products():
+    """2-norms over launches of the sizes that take these forms."""
+    for head, batch, seq in ((64, 4, 1024), (128, 4, 1024), (64, 2, 2000), (128, 3, 333)):
+        Q, K, V = draw(9, batch, seq, seq, head)
+        seen = torch.ones(seq, seq, dtype=torch.bool).tril()
+        for mode, mask in ((hip_sdpa.MASK_CAUSAL, seen), (hip_sdpa.MASK_NONE, None)):
+            wantA, want = reference(Q, K, V, mask)
+            fp32 = rel(call(Q, K, V, mode, FP32)[0], wantA)
+            for form in FORMS:
+                got = rel(call(Q, K, V, mode, FORMS[form])[0], wantA)
+                print(head, batch, seq, mode, form, "%.2e, fp32 %.2e" % (got, fp32), flush=True)
+                # (one rounding a product and pass: the longer a wavefront's walk,
+                # the more; the 32-query workgroups walk a quarter of the keys)
+                assert got < 1.2 * fp32
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("what", ["zeros first", "large later", "small later", "all tiny", "all huge",
+                                  "tiny rows", "tiny values", "zero keys", "one outlier", "tiny first row"])
+def test_ranges(form, head, what):
+    """Within twice the error of fp32 products whatever the powers of two: taken
+    again in fp32, a wavefront walks up to four times the keys that one of the
+    fp32 kernel does, and errors grow with the root of their number."""
+    print("case", form, head, what, flush=True)
+    q_seq, k_seq = 130, 700
+    Q, K, V = draw(3, 2, q_seq, k_seq, head)
+    mode = hip_sdpa.MASK_NONE
+    if what == "zeros first":
+        K[:, :64] = 0
+        V[:, :64] = 0
+    elif what == "large later":
+        V[:, 300:] *= 1e4       # past fp16 at the first step's power
+    elif what == "small later":
+        V[:, 64:] *= 1e-6
+        K[:, :64] = -Q[:, :1] * 30      # ... which the first query does not see
+    elif what == "all tiny":
+        V *= 1e-30
+        Q *= 1e-3
+        K *= 1e3
+    elif what == "all huge":
+        V *= 1e30
+        Q *= 1e13
+        K *= 1e-13
+    elif what == "tiny rows":
+        Q *= torch.logspace(-20, 0, q_seq)[None, :, None]
+    elif what == "tiny values":
+        V *= torch.logspace(-3, 0, head)
+    elif what == "zero keys":
+        K *= 0
+    elif what == "one outlier":
+        K[:, 5, 3] = 100.0
+        V[:, 5, 3] = 1000.0
+    elif what == "tiny first row":
+        V[:, 0] *= 1e-5
+        mode = hip_sdpa.MASK_CAUSAL
+    seen = None if mode == hip_sdpa.MASK_NONE else \
+        torch.arange(k_seq)[None] <= torch.arange(q_seq)[:, None]
+    wantA, want = reference(Q, K, V, seen)
+    A, lse = call(Q, K, V, mode, FORMS[form])
+    A32, lse32 = call(Q, K, V, mode, FP32)
+    # row by row: a row of small values counts as much as one of large ones
+    norm = wantA.norm(dim=2)
+    err, err32 = ((x - wantA).norm(dim=2) / norm for x in (A, A32))
+    assert float(err.mean()) < 2 * float(err32.mean())
+    assert float(err.max()) < 4 * float(err32.max())
+    # head by head likewise
+    col, col32 = ((x - wantA).norm(dim=1) / wantA.norm(dim=1) for x in (A, A32))
+    assert float(col.max()) < 4 * float(col32.max())
+    assert float((lse - want).abs().max()) < 2 * float((lse32 - want).abs().max()) + 1e-6
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 3.4e38])
+@pytest.mark.parametrize("where", ["query", "key", "value"])
+def test_what_is_not_finite(form, head, value, where):
+    """The same rows and elements are infinite, NaN or finite as with fp32
+    products, and the finite ones agree."""
+    print("case", form, head, value, where, flush=True)
+    q_seq, k_seq = 130, 400
+    Q, K, V = draw(4, 2, q_seq, k_seq, head)
+    {"query": Q, "key": K, "value": V}[where][1, 77, 5] = value
+    A, lse = call(Q, K, V, hip_sdpa.MASK_CAUSAL, FORMS[form], offset=k_seq - q_seq)
+    A32, lse32 = call(Q, K, V, hip_sdpa.MASK_CAUSAL, FP32, offset=k_seq - q_seq)
+    for got, want in ((A, A32), (lse, lse32)):
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(torch.isposinf(got), torch.isposinf(want))
+        assert torch.equal(torch.isneginf(got), torch.isneginf(want))
+        ok = torch.isfinite(want)
+        assert rel(got[ok], want[ok]) < 2e-6
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_tiles_of_any_length_and_the_running_pair(oracle, form):
+    """Tiles that end inside a step, several slabs, a second call that merges."""
+    head, batch, n_slabs, q_seq, q_tile = 64, 2, 2, 300, 150
+    for k_tile in (40, 100, 256, 330):
+        k_seq = 660
+        print("case", form, k_tile, flush=True)
+        tiles = lambda x, step: [x[:, i:i + step].contiguous().cuda() for i in range(0, x.shape[1], step)]
+        halves, Qt, want = [([], []), ([], [])], [], []
+        for s in range(n_slabs):
+            Q, K, V = draw(50 + s, batch, q_seq, k_seq, head)
+            want.append(reference(Q, K, V, torch.arange(k_seq)[None] <= torch.arange(q_seq)[:, None] + 200))
+            Qt += tiles(Q, q_tile)
+            for h in range(2):
+                half = slice(330 * h, 330 * (h + 1))
+                halves[h][0].extend(tiles(K[:, half], k_tile))
+                halves[h][1].extend(tiles(V[:, half], k_tile))
+        outs = [(torch.full(t.shape[:2], float("-inf"), device="cuda"), torch.zeros_like(t)) for t in Qt]
+        for h in range(2):
+            hip_sdpa.sdpa_fwd_grid(halves[h][0], Qt, [o[0] for o in outs], halves[h][1],
+                                   [o[1] for o in outs], q_seq, 330, q_tile, k_tile, hip_sdpa.MASK_CAUSAL,
+                                   causal_offset=200, k_pos0=330 * h, n_slabs=n_slabs, flags=FORMS[form])
+        torch.cuda.synchronize()
+        n_q = len(Qt) // n_slabs
+        for s in range(n_slabs):
+            A = torch.cat([o[1] for o in outs[s * n_q:(s + 1) * n_q]], 1).cpu().double()
+            lse = torch.cat([o[0] for o in outs[s * n_q:(s + 1) * n_q]], 1).cpu().double()
+            assert rel(A, want[s][0]) < 1e-6 and rel(lse, want[s][1]) < 1e-6
