@@ -2,6 +2,8 @@
 // walks the keys, shared by the 16-bit and the fp32 prefill kernels.
 #pragma once
 
+#include <type_traits>
+
 #include "sdpa_common.hpp"
 
 namespace nntile_hip
@@ -15,8 +17,8 @@ namespace nntile_hip
 // of visible / hidden elements.
 //
 // A lane keeps to one step while it walks the rows, so that what it finds is
-// two words ORed together (four instructions a load) and a ballot at the end
-// says which steps; 16 loads of 16 bytes are in flight per lane.  Reads of a
+// two words ORed and ANDed together (four instructions a load) and a ballot at the end
+// says which steps.  Reads of a
 // row are contiguous whatever its length; rows and starts that are not
 // multiples of 16 bytes only cost some loads a second cache line.  The last
 // chunk of a row is moved back to end with the row: it then looks at elements
@@ -50,29 +52,46 @@ __device__ __forceinline__ void mask_scan_steps(const char *mask, uint32_t ld_by
     {
         const bool mine = s0 + my_step < s_hi;
         const int at = min((s0 + my_step) * KEYS * ES + (lane % CPS) * 16, row_bytes - 16);
-        uint32_t any_open = 0u, any_hidden = 0u;
-        for(int base = 0; base < n_rows; base += 16 * rows_pass)
+        // (three-operand ors and ands, in two chains)
+        uint32_t all_or[2] = {0u, 0u}, all_and[2] = {~0u, ~0u};
+        // N loads in flight per lane: eight where they cover the rows (what a small
+        // tile's workgroup executes once costs its fetch: 128 x 128 10.8 us with 16
+        // and an exclusive or per word, 10.4 so), else 16
+        auto look = [&](auto n_tag) __attribute__((always_inline))
         {
-            u32x4 v[16];
-#pragma unroll
-            for(int u = 0; u < 16; ++u)
+            constexpr int N = decltype(n_tag)::value;
+            for(int base = 0; base < n_rows; base += N * rows_pass)
             {
-                // (rows past the end re-read the last one: no branches, so
-                // that the loads are in flight together)
-                const uint32_t row = (uint32_t)min(base + r0 + u * rows_pass, n_rows - 1);
-                v[u] = *reinterpret_cast<const u32x4_any *>(mask + row * ld_bytes + at);
-            }
+                u32x4 v[N];
 #pragma unroll
-            for(int u = 0; u < 16; ++u)
-            {
-#pragma unroll
-                for(int e = 0; e < 4; ++e)
+                for(int u = 0; u < N; ++u)
                 {
-                    any_open |= v[u][e] ^ open_word;
-                    any_hidden |= v[u][e] ^ hidden_word;
+                    // (rows past the end re-read the last one: no branches, so
+                    // that the loads are in flight together)
+                    const uint32_t row = (uint32_t)min(base + r0 + u * rows_pass, n_rows - 1);
+                    v[u] = *reinterpret_cast<const u32x4_any *>(mask + row * ld_bytes + at);
+                }
+#pragma unroll
+                for(int u = 0; u < N; ++u)
+                {
+                    all_or[0] |= v[u][0] | v[u][1];
+                    all_or[1] |= v[u][2] | v[u][3];
+                    all_and[0] &= v[u][0] & v[u][1];
+                    all_and[1] &= v[u][2] & v[u][3];
                 }
             }
+        };
+        if(n_rows <= 8 * rows_pass)
+        {
+            look(std::integral_constant<int, 8>{});
         }
+        else
+        {
+            look(std::integral_constant<int, 16>{});
+        }
+        const uint32_t or_all = all_or[0] | all_or[1], and_all = all_and[0] & all_and[1];
+        const uint32_t any_open = (or_all ^ open_word) | (and_all ^ open_word);
+        const uint32_t any_hidden = (or_all ^ hidden_word) | (and_all ^ hidden_word);
         const unsigned long long b_open = __builtin_amdgcn_ballot_w64(mine && any_open != 0u);
         const unsigned long long b_hidden = __builtin_amdgcn_ballot_w64(mine && any_hidden != 0u);
         for(int l = 0; l < 64; l += CPS)
