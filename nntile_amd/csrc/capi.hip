@@ -33,8 +33,8 @@ size_t decode_partial_o_bytes(int units, int n_splits, int rows, int head);
 size_t decode_partial_ml_bytes(int units, int n_splits, int rows);
 int launch_decode_fp32(hipStream_t stream, DecodeParams &p, int head, int mode);
 int decode_fp32_steps(int64_t k_seq);
-int decode_fp32_choose_splits(int units, int n_steps, int head);
-int decode_fp32_most_splits(int units, int n_steps, int head);
+int decode_fp32_choose_splits(int units, int n_steps, int head, int rows);
+int decode_fp32_most_splits(int units, int n_steps, int head, int rows);
 size_t decode_fp32_workspace_bytes(int units, int n_splits, int rows, int head);
 size_t decode_fp32_partial_bytes(int units, int n_splits, int rows, int head);
 
@@ -602,8 +602,8 @@ static void decode_fp32_geometry(const nntile_hip_sdpa_tile_args *a, int &units,
 {
     units = (int)(a->batch / a->kv_group);
     n_steps = decode_fp32_steps(a->k_seq);
-    splits = decode_fp32_choose_splits(units, n_steps, (int)a->head);
     rows = (int)(a->q_seq * a->kv_group);
+    splits = decode_fp32_choose_splits(units, n_steps, (int)a->head, rows);
 }
 
 static int decode_fp32_call(void *stream, const nntile_hip_sdpa_tile_args *a,
@@ -1213,7 +1213,8 @@ size_t nntile_hip_sdpa_fwd_decode_workspace_bytes_fp32(const nntile_hip_sdpa_til
     int units, n_steps, splits, rows;
     decode_fp32_geometry(args, units, n_steps, splits, rows);
     return decode_fp32_workspace_bytes(units,
-            decode_fp32_most_splits(units, n_steps, (int)args->head), rows, (int)args->head);
+            decode_fp32_most_splits(units, n_steps, (int)args->head, rows), rows,
+            (int)args->head);
 }
 
 int nntile_hip_sdpa_fwd_decode_fp32(void *stream, const nntile_hip_sdpa_tile_args *args,

@@ -197,13 +197,25 @@ __device__ __forceinline__ void f32dec_merge_row(const DecodeParams &p, int unit
 }
 
 // DIRECT: the unit has one key split: no partials, (lse, A) are written here.
-template<int HEAD, int MODE, bool DIRECT>
+//
+// ROW_WAVES: wavefronts with rows of their own, 4, or 1 for at most 16 rows (FEW
+// below).  Of four, one wavefront would have all of them and the others none,
+// and the workgroup would wait for its chain of matrix instructions, 64 a step at
+// head 64 (2 048 clocks of a step's 2 400).  Instead wavefront w takes the step's
+// key block w % 2 and, of the output, half w / 2 of the head: 24 instructions (two
+// wavefronts compute the same scores, which costs nothing and saves an exchange
+// inside the step).  The two key blocks keep maxima and sums of their own and are
+// merged through LDS at the end.  One row of head 64: 60 units of 778 keys 11.3 ->
+// 10.4 us, 12 of 101 7.3 -> 6.6; four of head 128: 8 units of 1 024 keys 10.8 -> 9.1,
+// 768 of 2 001 307 -> 282.
+template<int HEAD, int MODE, bool DIRECT, int ROW_WAVES>
 __global__ __launch_bounds__(kDecF32Threads, 2)
 void sdpa_decode_fp32_kernel(const DecodeParams p)
 {
+    constexpr bool FEW = ROW_WAVES == 1;
     constexpr int KT = HEAD / 16;           // 16-byte operand reads along head per 16-key block of S
-    constexpr int DBLOCKS = HEAD / 16;      // 16-row blocks of O^T
-    constexpr int KB = kDecF32Keys / 16;    // 16-key blocks of S^T per step
+    constexpr int DBLOCKS = HEAD / 16 / (FEW ? 2 : 1);      // 16-row blocks of O^T, of a wavefront
+    constexpr int KB = kDecF32Keys / 16 / (FEW ? 2 : 1);    // 16-key blocks of S^T per step, of a wavefront
     constexpr int RB = HEAD * 4;            // bytes per K/V row
     constexpr int CPR = RB / 16;            // 16-byte chunks per row
     constexpr int ROWS_PER_LOAD = 1024 / RB;
@@ -270,11 +282,14 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
         return;
     }
 
-    const int rr = wave * 16 + col;
+    const int rr = FEW ? col : wave * 16 + col;
     const bool row_ok = rr < p.rows;
+    // FEW: this wavefront's key block of a step and half of the head
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const int key_block = FEW ? wave_u & 1 : 0, head_half = FEW ? wave_u >> 1 : 0;
     // a wavefront none of whose 16 rows exists (one new token of a group of
     // four: three of the four) takes part in the loads and barriers only
-    const bool wave_idle = __builtin_amdgcn_readfirstlane(wave) * 16 >= p.rows;
+    const bool wave_idle = !FEW && wave_u * 16 >= p.rows;
     const int tok = row_ok ? rr % (int)p.q_seq : 0;
     const int64_t my_qpos = p.q_pos0 + tok;
 
@@ -304,7 +319,6 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
     // Load instruction `ld` fills rows [ld*ROWS_PER_LOAD, +ROWS_PER_LOAD): lane L
     // lands on row ld*ROWS_PER_LOAD + L/CPR at position L % CPR and fetches the
     // chunk that belongs there.
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     uint32_t k_goff[LOADS_PER_WAVE], v_goff[LOADS_PER_WAVE];
     int ld_row[LOADS_PER_WAVE];
 #pragma unroll
@@ -321,7 +335,7 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
 #pragma unroll
     for(int t = 0; t < KT; ++t)
     {
-        k_raddr[t] = (uint32_t)(col * RB + ((4 * t + quad) ^ col) * 16);
+        k_raddr[t] = (uint32_t)((16 * key_block + col) * RB + ((4 * t + quad) ^ col) * 16);
     }
     // PV operand: lane (col, quad) reads head value 16*db + col of key row
     // 16*kb + 4*quad + e; 16*kb + e goes into the immediate offset
@@ -329,8 +343,9 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
 #pragma unroll
     for(int db = 0; db < DBLOCKS; ++db)
     {
-        v_raddr[db] = (uint32_t)(K_BYTES + (4 * quad) * RB
-                + ((4 * db + (col >> 2)) ^ (4 * quad)) * 16 + (col & 3) * 4);
+        const int block = head_half * DBLOCKS + db;
+        v_raddr[db] = (uint32_t)(K_BYTES + (16 * key_block + 4 * quad) * RB
+                + ((4 * block + (col >> 2)) ^ (4 * quad)) * 16 + (col & 3) * 4);
     }
 
     // Loads of key step `step` into a ring slot; rows past the end of the
@@ -436,7 +451,7 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
             }
         }
 
-        // ---- mask: s[kb][e] is key 16*kb + 4*quad + e --------------------------
+        // ---- mask: s[kb][e] is key 16*(key_block + kb) + 4*quad + e ------------
         if(EXPLICIT)
         {
             // the mask is [k_seq, q_seq]: row index = token; keys past the end
@@ -446,7 +461,7 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
 #pragma unroll
             for(int kb = 0; kb < KB; ++kb)
             {
-                const int key0 = 16 * kb + 4 * quad;
+                const int key0 = 16 * (key_block + kb) + 4 * quad;
 #pragma unroll
                 for(int e = 0; e < 4; ++e)
                 {
@@ -486,7 +501,7 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
 #pragma unroll
                     for(int e = 0; e < 4; ++e)
                     {
-                        if(16 * kb + 4 * quad + e > lim)
+                        if(16 * (key_block + kb) + 4 * quad + e > lim)
                         {
                             s[kb][e] = neg_inf();
                         }
@@ -571,20 +586,73 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
         }
     }
 
+    // ---- FEW: the second key block's results into those of the first -------------
+    float lse_stored = neg_inf();
+    if constexpr(FEW)
+    {
+        // word w of lane l of half h sits at (h * NW + w) * 64 + l
+        constexpr int NW = 2 + 4 * DBLOCKS;
+        static_assert(2 * NW * 256 <= STAGE_BYTES, "exchange area does not fit");
+        float *xch = reinterpret_cast<float *>(ring0) + (head_half * NW * 64 + lane);
+        if(DIRECT && row_ok && !p.overwrite)
+        {
+            // (both halves read it, one writes it: in front of the barriers)
+            lse_stored = p.lse[f32dec_row(p, unit, rr)];
+        }
+        f32dec_wait_vmcnt<0>();
+        __syncthreads();        // everyone is done with the ring
+        if(key_block == 1)
+        {
+            xch[0] = m_run;
+            xch[64] = l_run;
+#pragma unroll
+            for(int db = 0; db < DBLOCKS; ++db)
+            {
+#pragma unroll
+                for(int e = 0; e < 4; ++e)
+                {
+                    xch[(2 + 4 * db + e) * 64] = o[db][e];
+                }
+            }
+        }
+        __syncthreads();
+        if(key_block == 0)
+        {
+            const float m_other = xch[0], m_new = fmaxf(m_run, m_other);
+            const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
+            const float a_mine = fast_exp2((m_run - m_use) * c);
+            const float a_other = fast_exp2((m_other - m_use) * c);
+            l_run = l_run * a_mine + xch[64] * a_other;
+#pragma unroll
+            for(int db = 0; db < DBLOCKS; ++db)
+            {
+#pragma unroll
+                for(int e = 0; e < 4; ++e)
+                {
+                    o[db][e] = o[db][e] * a_mine + xch[(2 + 4 * db + e) * 64] * a_other;
+                }
+            }
+            m_run = m_new;
+        }
+    }
+    // who leaves results, and which of them the row's (max, sum) or logsumexp
+    const bool leaves = row_ok && key_block == 0, leaves_row = quad == 0 && head_half == 0;
+
     // ---- the partial: (max in natural-log units, sum) and the normalised output
     float l_tot = l_run + __shfl_xor(l_run, 16);
     l_tot = sum_across_halves(l_tot);
     const float to_ln = EXPLICIT ? 1.0f : p.scale;
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    // o[db][r] is head value 16*db + 4*quad + r of row rr
+    // o[db][r] is head value 16*(head_half*DBLOCKS + db) + 4*quad + r of row rr
+    const int d0 = 16 * DBLOCKS * head_half + 4 * quad;
     if constexpr(DIRECT)
     {
-        if(!row_ok)
+        if(!leaves)
         {
             return;
         }
         const int64_t row = f32dec_row(p, unit, rr);
-        float *dst = static_cast<float *>(p.A) + row * HEAD + 4 * quad;
+        float *dst = static_cast<float *>(p.A) + row * HEAD + d0;
         // (no visible key at all: lse and A stay, or the empty row is written)
         const bool empty = l_tot == 0.0f;
         if(empty && !p.overwrite)
@@ -594,7 +662,7 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
         float w_old = 0.0f, w_new = 0.0f, lse_out = neg_inf();
         if(!empty)
         {
-            merge_weights(p.overwrite ? neg_inf() : p.lse[row], m_run * to_ln + __logf(l_tot), w_old,
+            merge_weights(FEW ? lse_stored : p.overwrite ? neg_inf() : p.lse[row], m_run * to_ln + __logf(l_tot), w_old,
                     w_new, lse_out);
         }
 #pragma unroll
@@ -609,21 +677,21 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
         }
         // (the four lanes of a row sit in one wavefront and run in lock step:
         // all of them have read the stored value by now)
-        if(quad == 0)
+        if(leaves_row)
         {
             p.lse[row] = lse_out;
         }
         return;
     }
-    if(row_ok)
+    if(leaves)
     {
         const int64_t prow = ((int64_t)unit * p.n_splits + split) * p.rows + rr;
-        if(quad == 0)
+        if(leaves_row)
         {
             p.part_ml[2 * prow] = l_tot == 0.0f ? neg_inf() : m_run * to_ln;
             p.part_ml[2 * prow + 1] = l_tot;
         }
-        float *dst = p.part_o + prow * HEAD + 4 * quad;
+        float *dst = p.part_o + prow * HEAD + d0;
 #pragma unroll
         for(int db = 0; db < DBLOCKS; ++db)
         {
@@ -658,13 +726,17 @@ int decode_fp32_steps(int64_t k_seq)
 }
 
 // Key splits per unit: two workgroups per CU when the units allow it - three at
-// head 64, whose ring is half as large and whose steps are bound by a
-// wavefront's own chain of MFMAs (36 units of 15 000 keys: 64.2 us with two, 50.6
-// with three, 53.3 with four) - never more than one split per key step; the limits for few steps are those of the
-// 16-bit kernel (handing partials over costs 2 us, a step about 1).
-int decode_fp32_choose_splits(int units, int n_steps, int head)
+// head 64, whose ring is half as large and whose steps, of more than 16 rows, are
+// bound by a wavefront's own chain of MFMAs (36 units of 15 000 keys: 64.2 us with
+// two, 50.6 with three, 53.3 with four) - never more than one split per key step;
+// the limits for few steps are those of the 16-bit kernel (handing partials over
+// costs 2 us, a step about 1).
+// At head 64 a step of up to 16 rows takes 0.8 us, and one workgroup takes a fourth:
+// 128 keys of 12 / 60 / 192 units 6.3 / 6.6 / 6.5 us, in four splits 6.7 / 6.8 / 8.3
+// (160 keys: 7.1 / 7.3 / 7.3 against 6.8 / 7.4 / 9.6 in five).
+int decode_fp32_choose_splits(int units, int n_steps, int head, int rows)
 {
-    if(n_steps <= kDecodeDirectSteps)
+    if(n_steps <= kDecodeDirectSteps + (head <= 64 && rows <= 16 ? 1 : 0))
     {
         return 1;
     }
@@ -675,11 +747,11 @@ int decode_fp32_choose_splits(int units, int n_steps, int head)
 }
 
 // (see decode_most_splits)
-int decode_fp32_most_splits(int units, int n_steps, int head)
+int decode_fp32_most_splits(int units, int n_steps, int head, int rows)
 {
-    const int here = decode_fp32_choose_splits(units, n_steps, head);
+    const int here = decode_fp32_choose_splits(units, n_steps, head, rows);
     const int before = decode_fp32_choose_splits(units,
-            n_steps < kDecodeSingleSteps ? n_steps : kDecodeSingleSteps, head);
+            n_steps < kDecodeSingleSteps ? n_steps : kDecodeSingleSteps, head, rows);
     return here > before ? here : before;
 }
 
@@ -699,15 +771,19 @@ size_t decode_fp32_workspace_bytes(int units, int n_splits, int rows, int head)
 template<int HEAD, int MODE>
 static void launch_decode_fp32_mode(hipStream_t stream, const DecodeParams &p, dim3 grid)
 {
-    if(p.n_splits == 1)
+    auto launch = [&](auto kernel)
     {
-        hipLaunchKernelGGL((sdpa_decode_fp32_kernel<HEAD, MODE, true>), grid,
-                dim3(kDecF32Threads), 0, stream, p);
+        hipLaunchKernelGGL(kernel, grid, dim3(kDecF32Threads), 0, stream, p);
+    };
+    if(p.rows <= 16)
+    {
+        launch(p.n_splits == 1 ? sdpa_decode_fp32_kernel<HEAD, MODE, true, 1>
+                : sdpa_decode_fp32_kernel<HEAD, MODE, false, 1>);
     }
     else
     {
-        hipLaunchKernelGGL((sdpa_decode_fp32_kernel<HEAD, MODE, false>), grid,
-                dim3(kDecF32Threads), 0, stream, p);
+        launch(p.n_splits == 1 ? sdpa_decode_fp32_kernel<HEAD, MODE, true, 4>
+                : sdpa_decode_fp32_kernel<HEAD, MODE, false, 4>);
     }
 }
 
