@@ -178,6 +178,7 @@ static int tile_call(DType dt, void *stream, const nntile_hip_sdpa_tile_args *a,
                 a->head);
         if(parts.n > 1 && parts_bytes >= parts.bytes && aligned16(parts_mem))
         {
+            p.form = parts.form;
             p.n_parts = parts.n;
             p.part_keys = parts.keys;
             p.part_o = static_cast<float *>(parts_mem);

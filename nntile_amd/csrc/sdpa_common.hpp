@@ -91,11 +91,13 @@ struct PrefillParams
 };
 
 // The ranges a one-tile call's keys are shared out in: their number (1: not
-// shared out), the keys of each but the last, the memory for what they leave.
+// shared out), the keys of each but the last, the memory for what they leave, and
+// in fp32 the kernel that takes them (PrefillParams::form: 2 or 10).
 struct PrefillParts
 {
     int n, keys;
     size_t bytes;
+    int form;
 };
 PrefillParts prefill_parts(bool fp32, int64_t batch, int64_t q_seq, int64_t k_seq, int64_t head);
 
@@ -104,6 +106,7 @@ PrefillParts prefill_parts(bool fp32, int64_t batch, int64_t q_seq, int64_t k_se
 constexpr int kF16x2None = 0, kF16x2Form22 = 1, kF16x2Form41 = 2, kF16x2Form42 = 3, kF16x2Form81 = 4;
 int prefill_f16x2_form(const PrefillParams &p, int head, int mode);
 int launch_prefill_f16x2(hipStream_t stream, PrefillParams &p, int head, int mode, int form);
+int launch_prefill_f16x2_parts(hipStream_t stream, PrefillParams &p, int head, int mode);
 
 // Kernel arguments of the decode kernels.  K, V: [head, k_seq, n_batch,
 // n_head_kv]; Q, A: [head, q_seq, n_batch, kv_group, n_head_kv].

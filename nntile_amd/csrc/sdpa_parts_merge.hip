@@ -9,39 +9,64 @@ namespace nntile_hip
 // kernels take, fewer query blocks than the chip has CUs - leave most CUs
 // idle while each workgroup walks the whole key axis.  The keys are shared out
 // over the idle ones, in the number of ranges that the measured times say is
-// best: a step of a workgroup alone on its CU takes kStep (64 keys x 128
-// queries of 16 bits, 32 keys x 32 queries of fp32; a second workgroup on a CU
-// gains little, so there are 256 places), writing and merging the ranges 3.5 us
-// plus 0.7 us for each 10^6 bytes they leave.  Where that is not 1 us faster the
-// keys stay together (32 heads, 400 rows, 1100 keys in two ranges: 21.3 -> 27.3
-// us).  32 heads over 8: 17 rows, 16000 keys 160 -> 35 us, 100 rows, 8000 keys
-// 86 -> 29; fp32, 12 heads, 100 rows, 4000 keys 96 -> 29.
+// best: a step of a workgroup alone on its CU takes the time given below (a second
+// workgroup on a CU gains little, so there are 256 places), writing and merging the
+// ranges 3.5 us plus 0.7 us for each 10^6 bytes they leave.  Where that is not 1 us
+// faster the keys stay together (32 heads, 400 rows, 1100 keys in two ranges: 21.3
+// -> 27.3 us).  32 heads over 8: 17 rows, 16000 keys 160 -> 35 us, 100 rows, 8000
+// keys 86 -> 29.
+//
+// In fp32 there are two kernels to take the ranges.  The one on fp16 pairs has twice
+// the rows, so twice the ranges fit, and is through its keys sooner, but is 4 us
+// behind from the start (its longer code and the splitting of the first rows).  us,
+// ranges with 32 queries of fp32 products / with 64 of fp16 pairs: 12 heads of 64,
+// 65 rows, 365 keys 15.2 / 16.3; 100 rows, 600 keys 15.6 / 17.4, 1100 17.2 / 19.1,
+// 4000 32.3 / 26.5; 256 rows, 2256 keys 37.6 / 26.1; 32 heads of 128 over 8, 33 rows,
+// 933 keys 24.4 / 21.6; 100 rows, 4100 keys 104.5 / 56.5.
 PrefillParts prefill_parts(bool fp32, int64_t batch, int64_t q_seq, int64_t k_seq, int64_t head)
 {
     constexpr int64_t kMost = 32, kPlaces = 256;
-    const int64_t rows = fp32 ? 32 : 128, keys = fp32 ? 32 : 64;    // of a workgroup, of a step
-    const int64_t groups = fp32 ? 4 : 2;    // sets of wavefronts that take steps in turn
-    const double kStep = fp32 ? (head == 64 ? 0.72 : 1.33) : (head == 64 ? 0.46 : 0.6);
-    const int64_t n_wg = batch * ((q_seq + rows - 1) / rows);
-    const int64_t steps = (k_seq + keys - 1) / keys;
-    const double part_bytes = 4.0 * (double)batch * (double)q_seq * (double)(head + 2);
-    PrefillParts best = {1, 0, 0};
+    struct Kernel
+    {
+        int form;
+        int64_t rows, keys;     // of a workgroup, of a step
+        int64_t groups;         // sets of wavefronts that take steps in turn
+        double step[2];         // us, head 64 and 128
+        double later;           // us behind the other from the start
+    };
+    static const Kernel kernels[] = {{0, 128, 64, 2, {0.46, 0.6}, 0.0},
+        {2, 32, 32, 4, {0.72, 1.33}, 0.0}, {10, 64, 64, 1, {1.13, 2.17}, 4.0}};
+    PrefillParts best = {1, 0, 0, 0};
     if(head != 64 && head != 128)
     {
         return best;
     }
-    double least = kStep * (double)steps - 1.0;
-    for(int64_t want = 2; want <= kMost && want * n_wg <= kPlaces; ++want)
+    const double part_bytes = 4.0 * (double)batch * (double)q_seq * (double)(head + 2);
+    const Kernel *first = fp32 ? kernels + 1 : kernels, *end = fp32 ? kernels + 3 : kernels + 1;
+    auto steps = [&](const Kernel &f) { return (k_seq + f.keys - 1) / f.keys; };
+    auto step_time = [&](const Kernel &f) { return f.step[head == 64 ? 0 : 1]; };
+    double least = 0.0;
+    for(const Kernel *f = first; f != end; ++f)
     {
-        // (whole rounds of the groups)
-        const int64_t each = ((steps + want - 1) / want + groups - 1) / groups * groups;
-        const int64_t n = (steps + each - 1) / each;
-        const double cost = kStep * (double)each + 3.5 + 0.7e-6 * (double)n * part_bytes;
-        if(n > 1 && cost < least)
+        const double together = step_time(*f) * (double)steps(*f) + f->later - 1.0;
+        least = f == first || together < least ? together : least;
+    }
+    for(const Kernel *f = first; f != end; ++f)
+    {
+        const int64_t n_wg = batch * ((q_seq + f->rows - 1) / f->rows);
+        for(int64_t want = 2; want <= kMost && want * n_wg <= kPlaces; ++want)
         {
-            least = cost;
-            best = {(int)n, (int)(each * keys),
-                (size_t)n * batch * q_seq * (head + 2) * sizeof(float)};
+            // (whole rounds of the groups)
+            const int64_t each = ((steps(*f) + want - 1) / want + f->groups - 1) / f->groups * f->groups;
+            const int64_t n = (steps(*f) + each - 1) / each;
+            const double cost = step_time(*f) * (double)each + f->later + 3.5
+                + 0.7e-6 * (double)n * part_bytes;
+            if(n > 1 && cost < least)
+            {
+                least = cost;
+                best = {(int)n, (int)(each * f->keys),
+                    (size_t)n * batch * q_seq * (head + 2) * sizeof(float), f->form};
+            }
         }
     }
     return best;

@@ -116,6 +116,8 @@ __device__ __forceinline__ bool power_to(float largest, int to, float &scale, fl
     return true;
 }
 
+// PARTS: the workgroup takes one of p.n_parts ranges of the keys and leaves its
+// triple in memory (PrefillParams::part_o) for launch_parts_merge.
 template<int HEAD, int MODE, int QW, int G, bool PARTS = false>
 __global__ __launch_bounds__(64 * QW * G, HEAD == 128 && QW == 2 ? 1 : 2)
 void sdpa_prefill_f16x2_kernel(const PrefillParams p)
@@ -1274,12 +1276,13 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     }
 }
 
-template<int HEAD, int QW, int G>
+template<int HEAD, int QW, int G, bool PARTS = false>
 static int launch_form(hipStream_t stream, PrefillParams &p, int mode)
 {
     p.k_blocks_per_tile = (int)((p.k_tile + kX2Rows * G - 1) / (kX2Rows * G));
     p.q_blocks_per_tile = (int)((p.q_tile + kX2Rows * QW - 1) / (kX2Rows * QW));
-    const int64_t n_wg = (int64_t)p.batch * p.n_slabs * p.n_q_tiles * p.q_blocks_per_tile;
+    const int64_t n_wg = (int64_t)p.batch * p.n_slabs * p.n_q_tiles * p.q_blocks_per_tile
+        * (PARTS ? p.n_parts : 1);
     if(n_wg <= 0 || n_wg > 0x7fffffff)
     {
         return NNTILE_HIP_EINVAL;
@@ -1291,13 +1294,13 @@ static int launch_form(hipStream_t stream, PrefillParams &p, int mode)
     };
     if(mode == NNTILE_HIP_MASK_NONE)
     {
-        return launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_NONE, QW, G>);
+        return launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_NONE, QW, G, PARTS>);
     }
     if(mode == NNTILE_HIP_MASK_CAUSAL)
     {
-        return launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_CAUSAL, QW, G>);
+        return launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_CAUSAL, QW, G, PARTS>);
     }
-    if constexpr(QW * G == 4)       // (masks given as values)
+    if constexpr(QW * G == 4 && !PARTS)     // (masks given as values)
     {
         return mode == NNTILE_HIP_MASK_ADDITIVE
             ? launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_ADDITIVE, QW, G>)
@@ -1398,6 +1401,12 @@ int prefill_f16x2_form(const PrefillParams &p, int head, int mode)
         }
     }
     return best;
+}
+
+int launch_prefill_f16x2_parts(hipStream_t stream, PrefillParams &p, int head, int mode)
+{
+    return head == 64 ? launch_form<64, 2, 2, true>(stream, p, mode)
+        : head == 128 ? launch_form<128, 2, 2, true>(stream, p, mode) : NNTILE_HIP_EUNSUPPORTED;
 }
 
 int launch_prefill_f16x2(hipStream_t stream, PrefillParams &p, int head, int mode, int form)

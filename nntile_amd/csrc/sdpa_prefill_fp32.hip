@@ -939,6 +939,10 @@ int launch_prefill_fp32_parts(hipStream_t stream, PrefillParams &p, int head, in
     {
         return NNTILE_HIP_EUNSUPPORTED;     // as without ranges
     }
+    if(p.form == 10)
+    {
+        return launch_prefill_f16x2_parts(stream, p, head, mode);
+    }
     p.q_blocks_per_tile = (int)((p.q_tile + 31) / 32);
     p.k_blocks_per_tile = (int)((p.k_tile + kKeys32 - 1) / kKeys32);
     const dim3 grid((unsigned)((int64_t)p.batch * p.q_blocks_per_tile * p.n_parts));

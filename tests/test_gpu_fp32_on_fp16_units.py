@@ -200,3 +200,51 @@ def test_tiles_of_any_length_and_the_running_pair(oracle, form):
             A = torch.cat([o[1] for o in outs[s * n_q:(s + 1) * n_q]], 1).cpu().double()
             lse = torch.cat([o[0] for o in outs[s * n_q:(s + 1) * n_q]], 1).cpu().double()
             assert rel(A, want[s][0]) < 1e-6 and rel(lse, want[s][1]) < 1e-6
+
+
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("what", ["plain", "huge range", "infinite value", "hidden ranges"])
+def test_key_ranges_of_a_cache(head, what):
+    """The keys of a chunk shared out in ranges, by both kernels that take them: last
+    ranges of one key and of one and a half steps, one block of queries and two,
+    rows of NaN behind the keys, a range that is taken again in fp32, ranges that no
+    query sees."""
+    heads, capacity = 3, 9000
+    K, V = (torch.full((heads, capacity, head), float("nan"), device="cuda") for _ in range(2))
+    for q_seq, k_seq in ((1, 700), (17, 1025), (33, 2049), (64, 4096), (65, 4193), (130, 8193), (200, 8191)):
+        print("case", head, what, q_seq, k_seq, flush=True)
+        Q, Kn, Vn = draw(k_seq, heads, q_seq, k_seq, head)
+        offset = k_seq - q_seq
+        if what == "huge range":
+            Vn[:, k_seq // 2:k_seq // 2 + 60, ::3] *= 1e30
+        elif what == "infinite value":
+            Vn[1, k_seq // 2, 5] = float("inf")
+        elif what == "hidden ranges":
+            offset = k_seq // 2 - q_seq     # the first rows may see no key at all
+        K[:, :k_seq], V[:, :k_seq] = Kn.cuda(), Vn.cuda()
+        K[:, k_seq:], V[:, k_seq:] = float("nan"), float("nan")
+        outs = []
+        need = hip_sdpa.tile_cache_workspace_bytes(k_seq, Q.cuda(), hip_sdpa.MASK_CAUSAL)
+        assert need > 0
+        for ws in (torch.full((need,), 0xff, dtype=torch.uint8, device="cuda"), None):
+            lse, A = torch.full((heads, q_seq), 0.5, device="cuda"), torch.full(Q.shape, 0.25, device="cuda")
+            hip_sdpa.sdpa_fwd_tile_cache(K, V, k_seq, Q.cuda(), None, lse, A, hip_sdpa.MASK_CAUSAL,
+                                         causal_offset=offset, workspace=ws)
+            torch.cuda.synchronize()
+            outs.append((A.cpu().double(), lse.cpu().double()))
+        (A, lse), (A1, lse1) = outs     # in ranges, and the keys together
+        for got, want in ((A, A1), (lse, lse1)):
+            assert torch.equal(torch.isnan(got), torch.isnan(want))
+            assert torch.equal(torch.isinf(got), torch.isinf(want))
+        ok = torch.isfinite(A1)
+        # (1e-6: as in test_against_64_bits, each of the two within half of it)
+        assert rel(A[ok], A1[ok]) < 1e-6 and float((lse - lse1).abs().max()) < 1e-5
+        if what == "infinite value":
+            assert not ok.all()
+            continue
+        seen = torch.arange(k_seq)[None] <= torch.arange(q_seq)[:, None] + offset
+        wantA, want = reference(Q, Kn, Vn, seen)
+        w = torch.sigmoid(0.5 - want)       # the pair that was there
+        wantA = wantA * (1 - w)[..., None] + 0.25 * w[..., None]
+        assert rel(A, wantA) < 1e-6
+        assert float((lse - torch.logaddexp(want, torch.tensor(0.5).double())).abs().max()) < 1e-5
