@@ -15,7 +15,7 @@
 // absolutely below, so the values are moved there by powers of two, which are
 // exact: a row of Q so that its largest value is in [2^13, 2^14), K and V so that
 // the largest of a workgroup's first step is in [2^11, 2^12), the probabilities
-// (at most 1) by 2^14.  What that does not cover - infinities and NaN, later keys
+// (at most 1) by 2^4.  What that does not cover - infinities and NaN, later keys
 // 16 times larger than those of the first step, blocks of them 1000 times
 // smaller, rows of the output or of Q beyond 2^+-40 - is found by a test of the
 // blocks as they are split and of the results, and the workgroup then walks its
