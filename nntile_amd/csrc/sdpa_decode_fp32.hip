@@ -7,7 +7,8 @@
 // split over workgroups.
 //
 //  - unit = one (batch entry, kv head): its kv_group*q_seq <= 64 query rows, 16
-//    per wavefront, share every K/V byte;
+//    per wavefront, share every K/V byte; up to 32 (one new token of every group)
+//    belong to two wavefronts or to all, which share the work of a step;
 //  - a workgroup (4 wavefronts) streams its range of 32-key steps HBM -> LDS
 //    through a ring of two buffers of 2 x 16 KiB (head 128): 64 KiB, two
 //    workgroups a CU;
@@ -198,23 +199,26 @@ __device__ __forceinline__ void f32dec_merge_row(const DecodeParams &p, int unit
 
 // DIRECT: the unit has one key split: no partials, (lse, A) are written here.
 //
-// ROW_WAVES: wavefronts with rows of their own, 4, or 1 for at most 16 rows (FEW
-// below).  Of four, one wavefront would have all of them and the others none,
-// and the workgroup would wait for its chain of matrix instructions, 64 a step at
-// head 64 (2 048 clocks of a step's 2 400).  Instead wavefront w takes the step's
-// key block w % 2 and, of the output, half w / 2 of the head: 24 instructions (two
-// wavefronts compute the same scores, which costs nothing and saves an exchange
-// inside the step).  The two key blocks keep maxima and sums of their own and are
-// merged through LDS at the end.  One row of head 64: 60 units of 778 keys 11.3 ->
-// 10.4 us, 12 of 101 7.3 -> 6.6; four of head 128: 8 units of 1 024 keys 10.8 -> 9.1,
-// 768 of 2 001 307 -> 282.
+// ROW_WAVES: sets of 16 rows, one wavefront each: 4; 1 for at most 16 rows and 2 for
+// at most 32 (FEW below).  Of four, one or two would have all of them and the others
+// none, and the workgroup would wait for a wavefront's chain of matrix instructions,
+// 64 a step at head 64 (2 048 clocks of a step's 2 400).  Instead wavefront w takes the
+// step's key block w % 2 and, of up to 32 rows, the 16 of w / 2: 32 instructions; of up
+// to 16, half w / 2 of the head of the output: 24 (two wavefronts compute the same
+// scores, which costs nothing and saves an exchange inside the step).  The two key
+// blocks keep maxima and sums of their own and are merged through LDS at the end.  One
+// row of head 64: 60 units of 778 keys 11.3 -> 10.4 us, 12 of 101 7.3 -> 6.6; four of
+// head 128: 8 units of 1 024 keys 10.8 -> 9.1, 768 of 2 001 307 -> 282.  20 rows, 60
+// units of 797 keys, head 64 15.1 -> 13.3; 32, 64 of 8 200, head 128 147 -> 104; 17, 768
+// of 2 017 416 -> 284.
 template<int HEAD, int MODE, bool DIRECT, int ROW_WAVES>
 __global__ __launch_bounds__(kDecF32Threads, 2)
 void sdpa_decode_fp32_kernel(const DecodeParams p)
 {
-    constexpr bool FEW = ROW_WAVES == 1;
+    constexpr bool FEW = ROW_WAVES < 4;
+    constexpr int HALVES = ROW_WAVES == 1 ? 2 : 1;      // of the head
     constexpr int KT = HEAD / 16;           // 16-byte operand reads along head per 16-key block of S
-    constexpr int DBLOCKS = HEAD / 16 / (FEW ? 2 : 1);      // 16-row blocks of O^T, of a wavefront
+    constexpr int DBLOCKS = HEAD / 16 / HALVES;      // 16-row blocks of O^T, of a wavefront
     constexpr int KB = kDecF32Keys / 16 / (FEW ? 2 : 1);    // 16-key blocks of S^T per step, of a wavefront
     constexpr int RB = HEAD * 4;            // bytes per K/V row
     constexpr int CPR = RB / 16;            // 16-byte chunks per row
@@ -282,13 +286,13 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
         return;
     }
 
-    const int rr = FEW ? col : wave * 16 + col;
-    const bool row_ok = rr < p.rows;
-    // FEW: this wavefront's key block of a step and half of the head
+    // FEW: this wavefront's key block of a step, and its half of the head or its rows
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    const int key_block = FEW ? wave_u & 1 : 0, head_half = FEW ? wave_u >> 1 : 0;
-    // a wavefront none of whose 16 rows exists (one new token of a group of
-    // four: three of the four) takes part in the loads and barriers only
+    const int key_block = FEW ? wave_u & 1 : 0, head_half = HALVES == 2 ? wave_u >> 1 : 0;
+    const int rr = (ROW_WAVES == 4 ? wave : ROW_WAVES == 2 ? wave >> 1 : 0) * 16 + col;
+    const bool row_ok = rr < p.rows;
+    // a wavefront none of whose 16 rows exists (33 rows: one of the
+    // four) takes part in the loads and barriers only
     const bool wave_idle = !FEW && wave_u * 16 >= p.rows;
     const int tok = row_ok ? rr % (int)p.q_seq : 0;
     const int64_t my_qpos = p.q_pos0 + tok;
@@ -590,13 +594,13 @@ void sdpa_decode_fp32_kernel(const DecodeParams p)
     float lse_stored = neg_inf();
     if constexpr(FEW)
     {
-        // word w of lane l of half h sits at (h * NW + w) * 64 + l
+        // word w of lane l of the wavefronts 2 h and 2 h + 1 sits at (h * NW + w) * 64 + l
         constexpr int NW = 2 + 4 * DBLOCKS;
         static_assert(2 * NW * 256 <= STAGE_BYTES, "exchange area does not fit");
-        float *xch = reinterpret_cast<float *>(ring0) + (head_half * NW * 64 + lane);
+        float *xch = reinterpret_cast<float *>(ring0) + ((wave_u >> 1) * NW * 64 + lane);
         if(DIRECT && row_ok && !p.overwrite)
         {
-            // (both halves read it, one writes it: in front of the barriers)
+            // (two wavefronts read it, one writes it: in front of the barriers)
             lse_stored = p.lse[f32dec_row(p, unit, rr)];
         }
         f32dec_wait_vmcnt<0>();
@@ -779,6 +783,11 @@ static void launch_decode_fp32_mode(hipStream_t stream, const DecodeParams &p, d
     {
         launch(p.n_splits == 1 ? sdpa_decode_fp32_kernel<HEAD, MODE, true, 1>
                 : sdpa_decode_fp32_kernel<HEAD, MODE, false, 1>);
+    }
+    else if(p.rows <= 32)
+    {
+        launch(p.n_splits == 1 ? sdpa_decode_fp32_kernel<HEAD, MODE, true, 2>
+                : sdpa_decode_fp32_kernel<HEAD, MODE, false, 2>);
     }
     else
     {

@@ -1,7 +1,7 @@
-"""The fp32 decode with at most 16 rows a unit, whose wavefronts share a step's two
-key blocks and the two halves of the head: against 64-bit arithmetic at the edges
-of a key block, of a step and of the direct form, with one key block hidden, and
-one row more than the form takes."""
+"""The fp32 decode with at most 16 or 32 rows a unit, whose wavefronts share a step's
+two key blocks and the two halves of the head or of the rows: against 64-bit
+arithmetic at the edges of a key block, of a step and of the direct form, with one
+key block hidden, and one row more than the forms take."""
 import numpy as np
 import pytest
 import torch
@@ -17,7 +17,7 @@ TOL = 1e-6
 
 
 @pytest.mark.parametrize("head", [64, 128])
-@pytest.mark.parametrize("group,q_seq", [(1, 1), (4, 1), (3, 5), (4, 4), (1, 17)])
+@pytest.mark.parametrize("group,q_seq", [(1, 1), (4, 1), (3, 5), (4, 4), (1, 17), (2, 16), (3, 11)])
 @pytest.mark.parametrize("mode", ["none", "causal", "first block", "second block", "running pair"])
 def test_against_64_bits(head, group, q_seq, mode):
     n_batch, n_kv = 2, 3
