@@ -18,7 +18,7 @@
 //    16 bytes per lane, 1 KB contiguous per instruction, no registers in
 //    between) through a ring of STAGES buffers, so that STAGES-1 steps of 32 KB
 //    are in flight per workgroup while one is consumed;
-//  * a wavefront owns 16 rows and uses v_mfma_f32_16x16x32 (S^T = K Q^T,
+//  * a wavefront owns 16 rows (few rows: shares them, see ROW_WAVES) and uses v_mfma_f32_16x16x32 (S^T = K Q^T,
 //    O^T += V^T P^T with P^T taken from the S^T accumulators); LDS rows are
 //    unpadded and XOR-swizzled by 16-byte chunks against bank conflicts, and
 //    the V operand is gathered with the transposing ds_read_b64_tr_b16.
@@ -331,14 +331,25 @@ __device__ __forceinline__ void decode_merge_row(const DecodeParams &p, int unit
 
 // DIRECT: the unit has one key split, so the partial is the result and is
 // folded into (lse, A) here; no partials are written and no merge kernel runs.
-template<typename T, int HEAD, int MODE, int STAGES, bool DIRECT = false>
+//
+// ROW_WAVES: sets of 16 rows, one wavefront each: 4, or 1 (FEW below) for at most 16
+// rows.  Of four, one would have them all and the others would read the same 32 KB of
+// a step from LDS for nothing (1 024 clocks of its 128 bytes a clock for a step whose
+// chain of matrix instructions takes about 700).  Instead wavefront w takes half w % 2
+// of the step's keys and, of the output, half w / 2 of the head, 48 KB in all; the two
+// halves of the keys keep maxima and sums of their own and are merged through LDS at
+// the end.  Four rows of head 128, us: 8 units of 1 024 keys 7.05 -> 6.79, of 101 5.29
+// -> 5.01; 128 of 191 6.89 -> 6.42; 512 of 1 001 39.8 -> 38.9.
+template<typename T, int HEAD, int MODE, int STAGES, bool DIRECT, int ROW_WAVES>
 __global__ __launch_bounds__(kDecThreads, NNTILE_DEC_WGS_PER_CU)
 void sdpa_decode_16bit_kernel(const DecodeParams p)
 {
     typedef typename T::vec8 vec8;
     constexpr int KSTEPS = HEAD / 32;       // MFMA steps along head for S
-    constexpr int DBLOCKS = HEAD / 16;      // 16-row blocks of O^T
-    constexpr int KB = kDecKeys / 16;       // 16-key blocks of S^T per step
+    constexpr bool FEW = ROW_WAVES == 1;
+    constexpr int DBLOCKS = HEAD / 16 / (FEW ? 2 : 1);  // 16-row blocks of O^T, of a wavefront
+    constexpr int KB = kDecKeys / 16 / (FEW ? 2 : 1);   // 16-key blocks of S^T per step, of a wavefront
+    static_assert(KB % 2 == 0, "a matrix instruction of the output takes 32 keys");
     constexpr int RB = HEAD * 2;            // bytes per K/V row
     constexpr int CPR = HEAD / 8;           // 16-byte chunks per row
     constexpr int RPL = 16 / CPR;           // rows per 256-byte line of LDS banks
@@ -428,7 +439,11 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
     const int hkv = unit / p.n_batch;
 
     // Row of this lane: rr = g*q_seq + tok.
-    const int rr = wave * 16 + col;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const int rr = FEW ? col : wave * 16 + col;
+    // FEW: this wavefront's half of a step's keys, and its half of the head
+    const int key0_wave = FEW ? (wave_u & 1) * (kDecKeys / 2) : 0;
+    const int head_half = FEW ? wave_u >> 1 : 0;
     const bool row_ok = rr < p.rows;
     const int g = row_ok ? rr / (int)p.q_seq : 0;
     const int tok = row_ok ? rr % (int)p.q_seq : 0;
@@ -459,7 +474,6 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
     //   V:  c ^ (2 * ((r / RPL) % (CPR/2)))  8 consecutive rows x 32 B -> 8 bank groups
     // Load instruction `ld` fills rows [ld*ROWS_PER_LOAD, +ROWS_PER_LOAD): lane L
     // lands on row ld*ROWS_PER_LOAD + L/CPR, chunk position L % CPR.
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     uint32_t k_goff[LOADS_PER_WAVE], v_goff[LOADS_PER_WAVE];
     int ld_row[LOADS_PER_WAVE];
     const int ld_cpos = lane % CPR;
@@ -478,7 +492,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
 #pragma unroll
     for(int ks = 0; ks < KSTEPS; ++ks)
     {
-        k_raddr[ks] = (uint32_t)(col * RB + ((4 * ks + quad) ^ ((col / RPL) % CPR)) * 16);
+        k_raddr[ks] = (uint32_t)((key0_wave + col) * RB + ((4 * ks + quad) ^ ((col / RPL) % CPR)) * 16);
     }
     // PV operand through the transposing read: a 16-lane block is one quad;
     // lane i addresses key j = i/4 and head values 4*(i%4)..+3 of the block's
@@ -493,8 +507,8 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
 #pragma unroll
         for(int db = 0; db < DBLOCKS; ++db)
         {
-            const int c = 2 * db + (r4 >> 1);
-            v_raddr[db] = (uint32_t)(K_BYTES + r * RB + (c ^ swz) * 16 + 8 * (r4 & 1));
+            const int c = 2 * (head_half * DBLOCKS + db) + (r4 >> 1);
+            v_raddr[db] = (uint32_t)(K_BYTES + (key0_wave + r) * RB + (c ^ swz) * 16 + 8 * (r4 & 1));
         }
     }
 
@@ -608,7 +622,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
             if(p.k_seq - kr >= kDecKeys)
             {
                 mnext_wide = true;
-                const int64_t at = (int64_t)tok * p.mask_ld + kr + 4 * quad;
+                const int64_t at = (int64_t)tok * p.mask_ld + kr + key0_wave + 4 * quad;
 #pragma unroll
                 for(int kb = 0; kb < KB; ++kb)
                 {
@@ -689,7 +703,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
         const int64_t k_pos_base = p.k_pos0 + k_row0;
         const int keys_here = (int)min((int64_t)kDecKeys, p.k_seq - k_row0);
 
-        // ---- S^T = K Q^T: 4 blocks of 16 keys ----------------------------------
+        // ---- S^T = K Q^T: KB blocks of 16 keys ---------------------------------
         acc4 s[KB];
 #pragma unroll
         for(int kb = 0; kb < KB; ++kb)
@@ -704,7 +718,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
             }
         }
 
-        // ---- mask: s[kb][r] is key 16*kb + 4*quad + r ----------------------------
+        // ---- mask: s[kb][r] is key key0_wave + 16*kb + 4*quad + r ------------------
         if(EXPLICIT)
         {
             // the mask is [k_seq, q_seq]: row index = token.  A full step of
@@ -716,7 +730,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
 #pragma unroll
             for(int kb = 0; kb < KB; ++kb)
             {
-                const int key0 = 16 * kb + 4 * quad;
+                const int key0 = key0_wave + 16 * kb + 4 * quad;
                 float add[4];
                 if(cur_wide)
                 {
@@ -782,7 +796,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
 #pragma unroll
                     for(int e = 0; e < 4; ++e)
                     {
-                        if(16 * kb + 4 * quad + e > lim)
+                        if(key0_wave + 16 * kb + 4 * quad + e > lim)
                         {
                             s[kb][e] = neg_inf();
                         }
@@ -835,7 +849,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
         }
         l_run += rs;
 
-        // ---- O^T += V^T P^T: 2 steps of 32 keys ----------------------------------
+        // ---- O^T += V^T P^T: KB / 2 steps of 32 keys -----------------------------
 #pragma unroll
         for(int t = 0; t < KB / 2; ++t)
         {
@@ -869,20 +883,73 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
         if(STAGES > 3 && it + 3 < n_local) { body(it + 3, std::integral_constant<int, 3>{}); }
     }
 
+    // ---- FEW: the second half's results into those of the first ------------------------
+    float lse_stored = neg_inf();
+    if constexpr(FEW)
+    {
+        // word w of lane l of the wavefronts 2 h and 2 h + 1 sits at (h * NW + w) * 64 + l
+        constexpr int NW = 2 + 4 * DBLOCKS;
+        static_assert(2 * NW * 256 <= STAGE_BYTES, "exchange area does not fit");
+        float *xch = reinterpret_cast<float *>(ring0) + ((wave_u >> 1) * NW * 64 + lane);
+        if(DIRECT && row_ok && !p.overwrite)
+        {
+            // (two wavefronts read it, one writes it: in front of the barriers)
+            lse_stored = p.lse[qb * p.q_seq + tok];
+        }
+        wait_vmcnt<0>();
+        __syncthreads();        // everyone is done with the ring
+        if(key0_wave != 0)
+        {
+            xch[0] = m_run;
+            xch[64] = l_run;
+#pragma unroll
+            for(int db = 0; db < DBLOCKS; ++db)
+            {
+#pragma unroll
+                for(int e = 0; e < 4; ++e)
+                {
+                    xch[(2 + 4 * db + e) * 64] = o[db][e];
+                }
+            }
+        }
+        __syncthreads();
+        if(key0_wave == 0)
+        {
+            const float m_other = xch[0], m_new = fmaxf(m_run, m_other);
+            const float m_use = (m_new == neg_inf()) ? 0.0f : m_new;
+            const float a_mine = fast_exp2((m_run - m_use) * c);
+            const float a_other = fast_exp2((m_other - m_use) * c);
+            l_run = l_run * a_mine + xch[64] * a_other;
+#pragma unroll
+            for(int db = 0; db < DBLOCKS; ++db)
+            {
+#pragma unroll
+                for(int e = 0; e < 4; ++e)
+                {
+                    o[db][e] = o[db][e] * a_mine + xch[(2 + 4 * db + e) * 64] * a_other;
+                }
+            }
+            m_run = m_new;
+        }
+    }
+    // who leaves results, and which of them the row's (max, sum) or logsumexp
+    const bool leaves = row_ok && key0_wave == 0, leaves_row = quad == 0 && head_half == 0;
+    const int d0 = 16 * DBLOCKS * head_half + 4 * quad;
+
     // ---- write the partial ---------------------------------------------------------
     DEC_STAMP(3);
     float l_tot = l_run + __shfl_xor(l_run, 16);
     l_tot = sum_across_halves(l_tot);
     if constexpr(DIRECT)
     {
-        if(!row_ok)
+        if(!leaves)
         {
             return;
         }
         const int g = rr / (int)p.q_seq, tok = rr % (int)p.q_seq;
         const int64_t qb = nb + (int64_t)p.n_batch * (g + (int64_t)p.kv_group * hkv);
         const int64_t row = qb * p.q_seq + tok;
-        uint16_t *Adst = static_cast<uint16_t *>(p.A) + row * HEAD + 4 * quad;
+        uint16_t *Adst = static_cast<uint16_t *>(p.A) + row * HEAD + d0;
         if(l_tot == 0.0f)
         {
             // no visible key at all: leave lse and A untouched, or write the
@@ -894,7 +961,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
                 {
                     *reinterpret_cast<u32x2 *>(Adst + 16 * db) = u32x2{0, 0};
                 }
-                if(quad == 0)
+                if(leaves_row)
                 {
                     p.lse[row] = neg_inf();
                 }
@@ -903,7 +970,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
         }
         const float to_ln = EXPLICIT ? 1.0f : p.scale;
         const float lse_new = m_run * to_ln + __logf(l_tot);
-        const float lse_old = p.overwrite ? neg_inf() : p.lse[row];
+        const float lse_old = FEW ? lse_stored : p.overwrite ? neg_inf() : p.lse[row];
         float w_old, w_new, lse_out;
         merge_weights(lse_old, lse_new, w_old, w_new, lse_out);
         const float sc = w_new / l_tot;
@@ -926,16 +993,16 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
         }
         // The four lanes of a row sit in one wavefront and run in lock step:
         // all of them have read lse_old by now.
-        if(quad == 0)
+        if(leaves_row)
         {
             p.lse[row] = lse_out;
         }
         return;
     }
-    if(row_ok)
+    if(leaves)
     {
     const int64_t prow = ((int64_t)unit * p.n_splits + split) * p.rows + rr;
-    if(quad == 0)
+    if(leaves_row)
     {
         // max in natural-log units so that the reduce kernel needs no mode.  A
         // row all of whose scores are NaN has no maximum, but a sum that is NaN:
@@ -944,12 +1011,12 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
         p.part_ml[2 * prow] = l_tot == 0.0f ? neg_inf() : l_tot > 0.0f ? m_run * to_ln : 0.0f;
         p.part_ml[2 * prow + 1] = l_tot;
     }
-    // o[db][r] is head value 16*db + 4*quad + r of row rr
+    // o[db][r] is head value d0 + 16*db + r of row rr
 #if NNTILE_DEC_PART16
     // the partial output, normalised, in the tile type: half the bytes of
     // fp32 partials (one more rounding, as the reference's scratch tile has)
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    uint16_t *dst = reinterpret_cast<uint16_t *>(p.part_o) + prow * HEAD + 4 * quad;
+    uint16_t *dst = reinterpret_cast<uint16_t *>(p.part_o) + prow * HEAD + d0;
 #pragma unroll
     for(int db = 0; db < DBLOCKS; ++db)
     {
@@ -959,7 +1026,7 @@ void sdpa_decode_16bit_kernel(const DecodeParams p)
         *reinterpret_cast<u32x2 *>(dst + 16 * db) = w;
     }
 #else
-    float *dst = p.part_o + prow * HEAD + 4 * quad;
+    float *dst = p.part_o + prow * HEAD + d0;
 #pragma unroll
     for(int db = 0; db < DBLOCKS; ++db)
     {
@@ -1086,17 +1153,34 @@ extern "C" long long nntile_hip_debug_decode_sync_timeouts(void)
     return more < 0 ? more : (long long)n + more;
 }
 
-template<typename T, int HEAD, int MODE, int STAGES>
-static void launch_decode_main(hipStream_t stream, const DecodeParams &p, dim3 grid)
+template<typename T, int HEAD, int MODE, int STAGES, int ROW_WAVES>
+static void launch_decode_rows(hipStream_t stream, const DecodeParams &p, dim3 grid)
 {
     if(p.n_splits == 1)
     {
-        auto kernel = sdpa_decode_16bit_kernel<T, HEAD, MODE, STAGES, true>;
+        auto kernel = sdpa_decode_16bit_kernel<T, HEAD, MODE, STAGES, true, ROW_WAVES>;
         hipLaunchKernelGGL(kernel, grid, dim3(kDecThreads), 0, stream, p);
         return;
     }
-    auto kernel = sdpa_decode_16bit_kernel<T, HEAD, MODE, STAGES>;
+    auto kernel = sdpa_decode_16bit_kernel<T, HEAD, MODE, STAGES, false, ROW_WAVES>;
     hipLaunchKernelGGL(kernel, grid, dim3(kDecThreads), 0, stream, p);
+}
+
+// (FEW at head 128 only: at 64 a step's chain is half as long, and the merge costs
+// what it saves: one row, 12 units of 778 keys 6.76 -> 6.88 us, of 101 4.45 -> 4.50.
+// Two wavefronts for each 16 of 17 to 32 rows: 8 units of 4 008 keys 10.0 -> 10.2.)
+template<typename T, int HEAD, int MODE, int STAGES>
+static void launch_decode_main(hipStream_t stream, const DecodeParams &p, dim3 grid)
+{
+    if constexpr(HEAD == 128)
+    {
+        if(p.rows <= 16)
+        {
+            launch_decode_rows<T, HEAD, MODE, STAGES, 1>(stream, p, grid);
+            return;
+        }
+    }
+    launch_decode_rows<T, HEAD, MODE, STAGES, 4>(stream, p, grid);
 }
 
 template<typename T, int HEAD, int STAGES>
