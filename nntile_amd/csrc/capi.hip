@@ -21,8 +21,8 @@ int launch_parts_merge(hipStream_t stream, const PrefillParams &p, int head);
 
 template<typename T>
 int launch_decode_16bit(hipStream_t stream, DecodeParams &p, int head, int mode);
-int decode_choose_splits(int units, int n_steps);
-int decode_most_splits(int units, int n_steps);
+int decode_choose_splits(int units, int n_steps, int head);
+int decode_most_splits(int units, int n_steps, int head);
 template<typename T>
 int launch_bwd_16bit(hipStream_t stream, const BwdParams &p, int head, int mode);
 template<typename T>
@@ -517,7 +517,7 @@ static void decode_geometry(const nntile_hip_sdpa_tile_args *a, int &units,
 {
     units = (int)(a->batch / a->kv_group);
     n_steps = (int)((a->k_seq + kDecKeys - 1) / kDecKeys);
-    splits = decode_choose_splits(units, n_steps);
+    splits = decode_choose_splits(units, n_steps, (int)a->head);
     rows = (int)(a->q_seq * a->kv_group);
 }
 
@@ -1188,7 +1188,8 @@ size_t nntile_hip_sdpa_fwd_decode_workspace_bytes(const nntile_hip_sdpa_tile_arg
     }
     int units, n_steps, splits, rows;
     decode_geometry(args, units, n_steps, splits, rows);
-    return decode_workspace_bytes(units, decode_most_splits(units, n_steps), rows, (int)args->head);
+    return decode_workspace_bytes(units, decode_most_splits(units, n_steps, (int)args->head), rows,
+            (int)args->head);
 }
 
 int nntile_hip_sdpa_fwd_decode_bf16(void *stream, const nntile_hip_sdpa_tile_args *args,

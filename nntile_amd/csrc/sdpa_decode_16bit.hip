@@ -18,7 +18,8 @@
 //    16 bytes per lane, 1 KB contiguous per instruction, no registers in
 //    between) through a ring of STAGES buffers, so that STAGES-1 steps of 32 KB
 //    are in flight per workgroup while one is consumed;
-//  * a wavefront owns 16 rows (few rows: shares them, see ROW_WAVES) and uses v_mfma_f32_16x16x32 (S^T = K Q^T,
+//  * a wavefront owns 16 rows (few rows: shares them, see ROW_WAVES) and uses
+//    v_mfma_f32_16x16x32 (S^T = K Q^T,
 //    O^T += V^T P^T with P^T taken from the S^T accumulators); LDS rows are
 //    unpadded and XOR-swizzled by 16-byte chunks against bank conflicts, and
 //    the V operand is gathered with the transposing ds_read_b64_tr_b16.
@@ -1269,9 +1270,18 @@ bool decode_uneven_units(int units, int64_t k_seq, int64_t row_bytes)
 // steps stay in one workgroup (two steps: 6.8 -> 5.6 us a call, three 6.9 ->
 // 6.5, four would be 6.6 -> 7.3), and from nine on a split takes two at least
 // (8 units of 63 steps: 64 splits 13.0 us, 32 splits 10.3).
-int decode_choose_splits(int units, int n_steps)
+//
+// Units of head 128 that are more than the CUs but fit the places as they are: two
+// splits would be more workgroups than places, and the last of them a round of their
+// own.  One split / two, 4 rows, us: 320 units of 256 keys 9.0 / 12.9, of 1 024 28.6 /
+// 34.0, of 4 001 103 / 118; 448 10.7 / 15.3, 37.3 / 39.8, 131 / 137; 64 rows, 320 units
+// 14.3 / 28.8, 34.8 / 45.0, 109 / 128.  (At head 64 a CU holds more than two: 320 units
+// of 1 024 keys 17.7 / 16.4.)
+int decode_choose_splits(int units, int n_steps, int head)
 {
-    if(n_steps <= kDecodeDirectSteps)
+    const bool one_round = head == 128 && units > kDecodeCUs
+        && units <= NNTILE_DEC_WGS_PER_CU * kDecodeCUs;
+    if(n_steps <= kDecodeDirectSteps || one_round)
     {
         return 1;
     }
@@ -1285,11 +1295,11 @@ int decode_choose_splits(int units, int n_steps)
 
 // Most splits that a unit of at most n_steps steps takes: the workspace is sized
 // for these, so that one sized for the longest cache serves all shorter ones.
-int decode_most_splits(int units, int n_steps)
+int decode_most_splits(int units, int n_steps, int head)
 {
-    const int here = decode_choose_splits(units, n_steps);
+    const int here = decode_choose_splits(units, n_steps, head);
     const int before = decode_choose_splits(units,
-            n_steps < kDecodeSingleSteps ? n_steps : kDecodeSingleSteps);
+            n_steps < kDecodeSingleSteps ? n_steps : kDecodeSingleSteps, head);
     return here > before ? here : before;
 }
 

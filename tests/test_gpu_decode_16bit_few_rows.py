@@ -63,3 +63,25 @@ def test_against_64_bits(dtype, group, q_seq, mode):
         if seen.any():      # (17 keys: the second half is beyond them)
             assert float((A.cpu().double() - want)[seen].norm() / want[seen].norm()) < ULP[dtype]
             assert float((lse.cpu().double() - want_lse)[seen].abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("q_seq", [1, 17])
+@pytest.mark.parametrize("units", [256, 257, 512, 513])
+def test_units_of_one_round(units, q_seq):
+    """More units than CUs that fit the chip's places without a key split, and one unit
+    on either side."""
+    k_seq, head = 300, 128
+    print("case", units, q_seq, flush=True)
+    g = torch.Generator().manual_seed(units)
+    Q, K, V = [torch.randn(units, s, head, generator=g).to(torch.bfloat16) for s in (q_seq, k_seq, k_seq)]
+    s = torch.matmul(Q.double(), K.double().transpose(1, 2).contiguous()) / np.sqrt(head)
+    s = s.masked_fill(torch.arange(k_seq) > torch.arange(q_seq)[:, None] + k_seq - q_seq, float("-inf"))
+    want_lse = torch.logsumexp(s, 2)
+    want = torch.matmul(torch.exp(s - want_lse[..., None]), V.double())
+    lse, A, Kd, Qd = torch.zeros(Q.shape[:2], device="cuda"), torch.zeros_like(Q).cuda(), K.cuda(), Q.cuda()
+    ws = torch.empty(hip_sdpa.decode_workspace_bytes(Kd, Qd, units, 1), dtype=torch.uint8, device="cuda")
+    hip_sdpa.sdpa_fwd_decode(Kd, Qd, None, lse, V.cuda(), A, hip_sdpa.MASK_CAUSAL, units, 1, ws,
+                             causal_offset=k_seq - q_seq, flags=hip_sdpa.OVERWRITE)
+    torch.cuda.synchronize()
+    assert float((A.cpu().double() - want).norm() / want.norm()) < ULP["bf16"]
+    assert float((lse.cpu().double() - want_lse).abs().max()) < 1e-5
