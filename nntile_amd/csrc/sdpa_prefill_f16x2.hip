@@ -16,10 +16,18 @@
 // exact: a row of Q so that its largest value is in [2^13, 2^14), K and V so that
 // the largest of a workgroup's first step is in [2^11, 2^12), the probabilities
 // (at most 1) by 2^4.  What that does not cover - infinities and NaN, later keys
-// 16 times larger than those of the first step, blocks of them 1000 times
-// smaller, rows of the output or of Q beyond 2^+-40 - is found by a test of the
-// blocks as they are split and of the results, and the workgroup then walks its
-// keys again with fp32 matrix instructions.
+// 16 times larger than those of the first step, blocks of V 1000 times smaller,
+// rows of the output or of Q beyond 2^+-40 - is found by a test of the blocks as
+// they are split and of the results, and the workgroup then walks its keys again
+// with fp32 matrix instructions.
+//
+// Scores: what a piece loses absolutely, 2^-25 of a scaled value, counts by what it
+// is multiplied with.  With q and k the largest values of a row of Q and of the first
+// keys that is up to q k 2^-37 in a score (rounding errors of random signs in every
+// channel), and where large channels of one meet small ones of the other the score
+// may be that and little else.  So rows with q k above 2^12 to 2^14 (the powers of
+// two say which, in front of the walk) go to fp32 from the start; below, the errors
+// of a score stay under 2^-23, or 2^-21 where all later keys are 16 times larger.
 //
 // S^T = K Q^T and O^T += V^T P^T with a lane owning one query, as in the other
 // prefill kernels.  A workgroup holds QW blocks of 32 queries; a key step is G
@@ -53,6 +61,9 @@ constexpr int kX2Rows = 32;         // queries of a wavefront, keys of a wavefro
 // arguments of the exponentials that matter lie within 4 of zero, where a float
 // is finest (2^14: errors of A a fifth larger than with fp32 products, of lse 5 %).
 constexpr int kX2PExp = 4;
+// The inverse of the product of a row's power of two and that of K up to which their
+// scores are taken from pieces: largest values of 2^12 to 2^14 as a product.
+constexpr float kX2Scores = 0x1p-12f;
 
 // The two fp16 pieces of eight floats times a power of two, as matrix operands.
 struct Split8
@@ -92,19 +103,19 @@ __device__ __forceinline__ f32x16 product(int n, const Split8 &a, const Split8 &
 
 // The power of two that moves `largest` into [2^(to-1), 2^to) and its inverse;
 // false when it is out of the range that is moved (then 1).  LEAST: what is below
-// 2^-40 is moved as if it were that (the factors of a score: times one below 2^40,
-// what the pieces then lose is below 2^-30).  Zeros: as if they were 2^(to-5).
+// 2^-40, zeros among them, is moved as if it were that (the factors of a score:
+// times one below 2^40, what the pieces then lose is below 2^-30).
 template<bool LEAST>
 __device__ __forceinline__ bool power_to(float largest, int to, float &scale, float &inverse)
 {
     scale = inverse = 1.0f;
-    if(largest == 0.0f)
-    {
-        return true;
-    }
     if(LEAST)
     {
         largest = fmaxf(largest, 0x1p-40f);
+    }
+    else if(largest == 0.0f)
+    {
+        return true;
     }
     if(!(largest >= 0x1p-40f && largest < 0x1p40f))
     {
@@ -506,9 +517,15 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         // (the same in every lane; this makes the compiler see it)
         k_max = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(k_max)));
         v_max = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v_max)));
-        odd = !power_to<true>(k_max, 12, k_scale, k_back) || odd;
+        // (a step of zeros: as if its largest were 8)
+        odd = !power_to<true>(k_max == 0.0f ? 8.0f : k_max, 12, k_scale, k_back) || odd;
         odd = !power_to<false>(v_max, 12, v_scale, v_back) || odd;
         qk_back = q_back * k_back;
+        odd = odd || !(qk_back <= kX2Scores);
+        if(__builtin_amdgcn_ballot_w64(odd && q_ok) != 0)
+        {
+            any_odd = 1;
+        }
     }
     // item n of the 5 * UPT that split what was loaded: four pairs, then the store
     Split8 staged;
@@ -520,8 +537,8 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             *reinterpret_cast<u32x4 *>(at + piece_bytes) = staged.l;
         }
     };
-    // A wavefront's share of a block (its pieces h) that is too small for them: scaled,
-    // all of it below 2 but not all zeros.  (Bit 14 of an fp16 value: 2 or more.)
+    // A wavefront's share of a block of V (its pieces h) that is too small for them:
+    // scaled, all of it below 2 but not all zeros.  (Bit 14 of an fp16 value: 2 or more.)
     int too_small = 0;
     uint32_t staged_bits = 0;
     auto look_at_staged = [&](int i) __attribute__((always_inline))
@@ -544,7 +561,6 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         else
         {
             store_pieces(lds_k + k_at + k_lds(i), CH * 1024, i * THREADS + tid < UNITS);
-            look_at_staged(i);
         }
     };
     auto split_v = [&](int set, int n, char *lds_v) __attribute__((always_inline))
@@ -817,9 +833,6 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     // ---- the walk -------------------------------------------------------------------
     if(n_steps > 0)
     {
-        // (steps past the last are that one again: nobody reads them)
-        const int last_step = n_steps - 1;
-        f32x16 s_even, s_odd;
 #pragma unroll
         for(int n = 0; n < 5 * UPT; ++n)
         {
@@ -841,6 +854,14 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             load_k(0);
         }
         __syncthreads();
+    }
+    // (one row that goes to fp32 from the start takes its workgroup with it; whoever
+    // sets any_odd behind the walk has passed a barrier since)
+    if(n_steps > 0 && __builtin_amdgcn_readfirstlane(any_odd) == 0)
+    {
+        // (steps past the last are that one again: nobody reads them)
+        const int last_step = n_steps - 1;
+        f32x16 s_even, s_odd;
         for(int n = 0; n < AHEAD_FR; ++n)
         {
             read_k(0, n);

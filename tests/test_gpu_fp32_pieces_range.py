@@ -1,0 +1,71 @@
+"""fp32 tiles on the fp16 matrix units: values that two fp16 pieces under a common
+power of two do not carry, in every place where they can hide."""
+import math
+
+import pytest
+import torch
+
+from nntile_amd import hip_sdpa
+
+pytestmark = pytest.mark.gpu
+
+S, P, W = hip_sdpa.FORM_SHARED, hip_sdpa.FORM_SPLIT, hip_sdpa.FORM_WIDE
+# query blocks of 32 x key blocks of 32 of a workgroup
+FORMS = {"2x2": W | P, "4x1": S, "4x2": W | S, "8x1": W}
+FP32 = P        # the fp32 kernel
+
+
+def draw(seed, batch, q_seq, k_seq, head):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(batch, n, head, generator=g) for n in (q_seq, k_seq, k_seq)]
+
+
+def call(Q, K, V, mode, flags):
+    lse = torch.zeros(Q.shape[:2], device="cuda")
+    A = torch.zeros_like(Q, device="cuda")
+    hip_sdpa.sdpa_fwd_tile(K.cuda(), Q.cuda(), None, lse, V.cuda(), A, mode, flags=flags | hip_sdpa.OVERWRITE)
+    torch.cuda.synchronize()
+    return A.cpu(), lse.cpu()
+
+
+def check(Q, K, V, form, mode=hip_sdpa.MASK_NONE):
+    """By rows and by channels, against 64 bits, and against what fp32 products are
+    off by: twice that in the mean, four times the largest (the bounds of the other
+    ranges' test: sums of up to four times the keys in one accumulator)."""
+    q, k, v = (t.double() for t in (Q, K, V))
+    s = torch.matmul(q, k.transpose(1, 2).contiguous()) / math.sqrt(Q.shape[2])
+    if mode == hip_sdpa.MASK_CAUSAL:
+        s = s.masked_fill(torch.ones(s.shape[1:], dtype=torch.bool).triu(1), float("-inf"))
+    want_lse = torch.logsumexp(s, 2)
+    want = torch.matmul(torch.exp(s - want_lse[..., None]), v)
+    (A, lse), (A32, lse32) = call(Q, K, V, mode, FORMS[form]), call(Q, K, V, mode, FP32)
+    for dim in (1, 2):
+        norm = want.norm(dim=dim).clamp_min(1e-300)
+        err, err32 = ((x.double() - want).norm(dim=dim) / norm for x in (A, A32))
+        print(form, dim, "mean %.2e, fp32 %.2e; largest %.2e, fp32 %.2e"
+              % (err.mean(), err32.mean(), err.max(), err32.max()), flush=True)
+        assert float(err.mean()) < 2 * float(err32.mean())
+        assert float(err.max()) < 4 * float(err32.max())
+    assert float((lse - want_lse).abs().max()) < 2 * float((lse32 - want_lse).abs().max()) + 1e-6
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("what", ["query 1e5", "query 1e7", "query 1e9", "half of the channels",
+                                  "key 1e5", "key -1e6", "key -1e9", "later key -1e7"])
+def test_scores_of_a_large_channel_against_a_small_one(form, head, what):
+    print("case", form, head, what, flush=True)
+    Q, K, V = draw(5, 2, 130, 700, head)
+    if what == "half of the channels":
+        Q[..., ::2] *= 1e5
+        K[..., ::2] *= 1e-8
+    elif what.startswith("query"):
+        Q[..., 3] = float(what.split()[1])
+        K[..., 3] = 0.0
+    else:       # hidden keys by a channel of their own
+        Q[..., 3] = 1.0
+        K[..., 3] = 0.0
+        K[:, (600 if "later" in what else 0)::4, 3] = float(what.split()[-1])
+        if what == "key 1e5":       # (nothing hidden: the channel counts for nothing)
+            Q[..., 3] = 0.0
+    check(Q, K, V, form)
