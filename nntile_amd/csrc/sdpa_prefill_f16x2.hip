@@ -323,8 +323,8 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     // write hit 16 different ones, and so do those of a read.
     // V unit u: head value u % HEAD, keys of slot group u / HEAD - the eight keys
     // that a lane half's score registers hold of 16 (4 * half .. +3 and 8 further).
-    // Rows past the end of the tile are its last row: their scores are masked, so
-    // their probabilities are exactly 0.
+    // Rows past the end of the tile are its last row (V: zeros, where all eight are past
+    // it): their scores are masked, so their probabilities are exactly 0.
     constexpr int KSW = 16 / HG;            // keys of a row of 16 lanes
     auto k_place = [](int key, int hg) __attribute__((always_inline)) -> int
     {
@@ -407,6 +407,14 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             {
                 asm volatile("" : "+v"(v_raw[set][i][e]));      // (as above)
             }
+            if((int)(v_goff / (HEAD * 4)) + v_rows(i * SSTRIDE) >= v_src.rows_left)
+            {
+#pragma unroll
+                for(int e = 0; e < 8; ++e)
+                {
+                    v_raw[set][i][e] = 0.0f;
+                }
+            }
         }
     };
     auto load_k = [&](int set) __attribute__((always_inline))
@@ -445,14 +453,14 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     float k_scale = 1.0f, v_scale = 1.0f, v_back = 1.0f;
     float qk_back = 1.0f;       // scores / (what the matrix unit computes)
     bool odd = false;           // something that the pieces cannot carry
-    __shared__ int any_odd;
+    __shared__ int any_odd, any_large;
     if(n_steps > 0)
     {
         k_src = v_src = s_src = first_step();
         __shared__ float first_max[2 * THREADS / 64];
         if(tid == 0)
         {
-            any_odd = 0;
+            any_odd = any_large = 0;
         }
         load_k(0);
         load_v(0);
@@ -514,12 +522,19 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             k_max = fmaxf(k_max, first_max[2 * w]);
             v_max = fmaxf(v_max, first_max[2 * w + 1]);
         }
-        // (the same in every lane; this makes the compiler see it)
-        k_max = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(k_max)));
-        v_max = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v_max)));
+        // (the same in every lane; this makes the compiler see it, here and below)
+        auto scalar = [](float x) __attribute__((always_inline)) -> float
+        {
+            return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x)));
+        };
+        k_max = scalar(k_max);
+        v_max = scalar(v_max);
         // (a step of zeros: as if its largest were 8)
         odd = !power_to<true>(k_max == 0.0f ? 8.0f : k_max, 12, k_scale, k_back) || odd;
         odd = !power_to<false>(v_max, 12, v_scale, v_back) || odd;
+        k_scale = scalar(k_scale);
+        v_scale = scalar(v_scale);
+        v_back = scalar(v_back);
         qk_back = q_back * k_back;
         odd = odd || !(qk_back <= kX2Scores);
         if(__builtin_amdgcn_ballot_w64(odd && q_ok) != 0)
@@ -537,18 +552,23 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             *reinterpret_cast<u32x4 *>(at + piece_bytes) = staged.l;
         }
     };
-    // A wavefront's share of a block of V (its pieces h) that is too small for them:
-    // scaled, all of it below 2 but not all zeros.  (Bit 14 of an fp16 value: 2 or more.)
-    int too_small = 0;
-    uint32_t staged_bits = 0;
-    auto look_at_staged = [&](int i) __attribute__((always_inline))
+    // Values of V that are too small for the pieces: the eight that a thread splits
+    // together are a channel's, and all of them below 2^-2 once scaled but not all zeros.
+    // (Otherwise what the pieces lose, 2^-25, is 2^-23 of the largest of the eight or
+    // less, whatever the other channels and keys hold.)  large: some value was moved
+    // to 2^13 or beyond.
+    bool too_small = false, large = false;
+    float unit_max = 0.0f;
+    const float v_least = 0x1p-2f * v_back, v_large = 0x1p13f * v_back;
+    auto look_at_pair = [&](int j, float a, float b) __attribute__((always_inline))
     {
-        const uint32_t bits = staged.h[0] | staged.h[1] | staged.h[2] | staged.h[3];
-        staged_bits = i == 0 ? bits : staged_bits | bits;
-        if(i + 1 == UPT && __builtin_amdgcn_ballot_w64((staged_bits & 0x40004000u) != 0u) == 0)
-        {
-            too_small |= __builtin_amdgcn_ballot_w64((staged_bits & 0x7fff7fffu) != 0u) != 0;
-        }
+        const float x = __builtin_fabsf(a), y = __builtin_fabsf(b);
+        unit_max = j == 0 ? fmaxf(x, y) : max3(unit_max, x, y);
+    };
+    auto look_at_unit = [&]() __attribute__((always_inline))
+    {
+        too_small |= __builtin_amdgcn_ballot_w64(unit_max < v_least && unit_max > 0.0f) != 0;
+        large |= __builtin_amdgcn_ballot_w64(unit_max >= v_large) != 0;
     };
     auto split_k = [&](int set, int n, char *lds_k) __attribute__((always_inline))
     {
@@ -569,11 +589,12 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         if(j < 4)
         {
             staged.pair(j, v_raw[set][i][2 * j], v_raw[set][i][2 * j + 1], v_scale);
+            look_at_pair(j, v_raw[set][i][2 * j], v_raw[set][i][2 * j + 1]);
         }
         else
         {
             store_pieces(lds_v + v_at + v_lds(i), 2 * DB * 1024, i * THREADS + tid < UNITS);
-            look_at_staged(i);
+            look_at_unit();
         }
     };
     // (chunk ch of a key is 32 * ch ^ the first one's place: bits below 512)
@@ -843,6 +864,10 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         {
             split_v(0, n, lds + 2 * BUF);
         }
+        if(too_small)
+        {
+            any_odd = 1;
+        }
         // K(1) and, with two sets, V(1) and K(2)
         advance(k_src);
         load_k(SETS - 1);
@@ -1050,6 +1075,10 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             pass(std::integral_constant<bool, false>{}, std::integral_constant<int, 0>{}, s_even, s_odd);
             s_even = s_odd;
         }
+        if(large)
+        {
+            any_large = 1;
+        }
         __syncthreads();
 #pragma unroll
         for(int n = 0; n < 21; ++n)
@@ -1062,8 +1091,9 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     }
 
     // ---- results that the pieces could not carry: once more in fp32 --------------------
-    // (A row whose output is far below the values of V it was taken from had its V
-    // in the last bits of the pieces.)
+    // (A row whose output, as a mean of scaled values, is below 2^-2 was taken from
+    // values or of probabilities in the last bits of the pieces; where values of V come
+    // up to 2^16, three bits above the others, the bound moves with them.)
     if(n_steps > 0)
     {
         float o_max = 0.0f, o_sum = 0.0f;
@@ -1079,11 +1109,12 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         }
         o_max = max_across_halves(o_max);
         const float l_row = sum_across_halves(l_run);
+        const float o_least = (any_large != 0 ? 0x1p1f : 0x1p-2f) * l_row;
         // (a NaN or an infinity among the outputs is one in their sum)
         odd = odd || !(l_row < __builtin_huge_valf())
             || !(__builtin_fabsf(o_sum) < __builtin_huge_valf())
-            || (o_max > 0.0f && o_max < 0x1p-6f * l_row) || too_small != 0;
-        if(__builtin_amdgcn_ballot_w64(odd && q_ok) != 0 || too_small != 0)
+            || (o_max > 0.0f && o_max < o_least);
+        if(__builtin_amdgcn_ballot_w64(odd && q_ok) != 0 || too_small)
         {
             any_odd = 1;
         }

@@ -69,3 +69,75 @@ def test_scores_of_a_large_channel_against_a_small_one(form, head, what):
         if what == "key 1e5":       # (nothing hidden: the channel counts for nothing)
             Q[..., 3] = 0.0
     check(Q, K, V, form)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("what", ["spread 1e5", "spread 1e7", "one channel 1e-9", "one channel 1e-13",
+                                  "one channel small later", "one key small", "last row small", "large later"])
+def test_values_of_any_size_in_any_channel(form, head, what):
+    """Small values among large ones, in a channel, in some keys of it, in the one
+    row of a ragged last step; values three bits above the first step's."""
+    print("case", form, head, what, flush=True)
+    Q, K, V = draw(6, 2, 130, 705 if "row" in what else 700, head)
+    mode = hip_sdpa.MASK_NONE
+    if what.startswith("spread"):
+        V *= torch.logspace(0, -round(math.log10(float(what.split()[1]))), head)
+    elif what == "one channel small later":
+        V[:, 200:, 7] *= 1e-8
+        K[:, :200] = -Q[:, :1] * 30         # ... which the first query does not see
+    elif what.startswith("one channel"):
+        V[..., 7] *= float(what.split()[-1])
+    elif what == "one key small":           # the first query's only key
+        V[:, 0] *= 1e-10
+        mode = hip_sdpa.MASK_CAUSAL
+    elif what == "last row small":
+        V[:, 704] *= 1e-12
+        K[:, 704] = Q[:, 0] * 30            # ... the first query's only key
+    elif what == "large later":
+        V[:, 40:] *= 8
+        K[:, 0] = Q[:, 0] * 30
+        V[:, 0] *= 1e-4
+    check(Q, K, V, form, mode)
+
+
+def walks_again(Q, K, V, form):
+    """Whether every workgroup takes its keys with fp32 instructions: with an
+    infinite value in channel 0, which makes all of them, the other channels have the
+    same bits.  (A workgroup that stays with the pieces does not: other sums.)"""
+    V1 = V.clone()
+    V1[:, 3, 0] = float("inf")
+    A, A1 = (call(Q, K, v, hip_sdpa.MASK_NONE, FORMS[form])[0] for v in (V, V1))
+    assert not torch.isfinite(A1[..., 0]).any()
+    return [torch.equal(a[:, 1:], a1[:, 1:]) for a, a1 in zip(A.flatten(0, 1).split(32), A1.flatten(0, 1).split(32))]
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("what", ["plain", "last channel small", "small spread", "small values",
+                                  "large values", "zero channel", "no value", "one more key"])
+def test_what_the_pieces_carry_is_not_taken_again(form, head, what):
+    print("case", form, head, what, flush=True)
+    Q, K, V = draw(7, 2, 128, 769 if "key" in what else 768, head)
+    if what == "last channel small":
+        V[..., head - 1] *= 1e-3
+    elif what == "small spread":
+        V *= torch.logspace(-2, 0, head)
+    elif what == "small values":
+        V *= 1e-9
+        K *= 1e-9
+    elif what == "large values":
+        V *= 1e9
+        K *= 20
+    elif what == "zero channel":
+        V[..., 1:4] = 0.0
+    elif what == "no value":
+        V[:, 32:64] = 0.0
+    assert not any(walks_again(Q, K, V, form))
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_what_is_taken_again_can_be_told(form):
+    Q, K, V = draw(8, 2, 128, 768, 64)
+    V[..., 7] *= 1e-9
+    assert all(walks_again(Q, K, V, form))
