@@ -15,7 +15,7 @@
 // absolutely below, so the values are moved there by powers of two, which are
 // exact: a row of Q so that its largest value is in [2^13, 2^14), K and V so that
 // the largest of a workgroup's first step is in [2^11, 2^12), the probabilities
-// (at most 1) by 2^4.  What that does not cover - infinities and NaN, later keys
+// (at most 1) by 2^15.  What that does not cover - infinities and NaN, later keys
 // 16 times larger than those of the first step, blocks of V 1000 times smaller,
 // rows of the output or of Q beyond 2^+-40 - is found by a test of the blocks as
 // they are split and of the results, and the workgroup then walks its keys again
@@ -57,10 +57,14 @@ namespace nntile_hip
 {
 
 constexpr int kX2Rows = 32;         // queries of a wavefront, keys of a wavefront's step
-// Probabilities are scaled by 2^4: their pieces are exact to 2^-29, and the
-// arguments of the exponentials that matter lie within 4 of zero, where a float
-// is finest (2^14: errors of A a fifth larger than with fp32 products, of lse 5 %).
+// Probabilities are scaled by 2^4 in the exponential - the arguments that matter lie
+// within 4 of zero, where a float is finest (2^14: errors of A a fifth larger than with
+// fp32 products, of lse 5 %) - and by 2^11 more as they are split: what their pieces
+// lose is below 2^-40.  (With 2^4 alone it was 2^-29, and rows that a first key with
+// little of a value takes most of were made of those errors: 13 above the others'
+// scores, 700 keys: 2.2e-5 where fp32 products have 4.0e-7.)
 constexpr int kX2PExp = 4;
+constexpr float kX2PPieces = 0x1p11f;
 // The inverse of the product of a row's power of two and that of K up to which their
 // scores are taken from pieces: largest values of 2^12 to 2^14 as a product.
 constexpr float kX2Scores = 0x1p-12f;
@@ -69,20 +73,12 @@ constexpr float kX2Scores = 0x1p-12f;
 struct Split8
 {
     u32x4 h, l;
-    // (fma with an fp16 operand: no conversion back)
+    // (fma with an fp16 operand: no conversion back.  Fmas with an fp16 result, four
+    // instructions instead of six, take 6 to 10 % longer in all.)
     __device__ __forceinline__ void pair(int i, float a, float b, float scale)
     {
         h[i] = Fp16::pack2(a * scale, b * scale);
         l[i] = Fp16::pack2(fmaf(a, scale, -lo_half(h[i])), fmaf(b, scale, -hi_half(h[i])));
-    }
-    // the same without a scale; one: 1.0f, unknown to the compiler, which would
-    // otherwise undo the fma
-    __device__ __forceinline__ void pair_unscaled(int i, float a, float b, float one)
-    {
-        h[i] = Fp16::pack2(a, b);
-        uint32_t low = Fp16::pack2(fmaf(a, one, -lo_half(h[i])), fmaf(b, one, -hi_half(h[i])));
-        asm volatile("" : "+v"(low));       // (here, not in front of its use)
-        l[i] = low;
     }
     static __device__ __forceinline__ float lo_half(uint32_t v)
     {
@@ -610,8 +606,6 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     float to_scores = kScaleHi * qk_back;
     float c = EXPLICIT ? kLog2e : kScaleLog2e * qk_back;
     float p_exp = (float)kX2PExp;       // the probabilities' power of two
-    float one = 1.0f;
-    asm volatile("" : "+s"(one));       // (keeps the product below an fma)
 
     f32x16 o[DB];
 #pragma unroll
@@ -927,7 +921,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             else if(n < 21)
             {
                 const int j = n - 17;
-                pf[0].pair_unscaled(j, s[2 * j], s[2 * j + 1], one);
+                pf[0].pair(j, s[2 * j], s[2 * j + 1], kX2PPieces);
             }
             else
             {
@@ -940,7 +934,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
 #pragma unroll
             for(int n = 0; n < 4; ++n)
             {
-                pf[1].pair_unscaled(n, s[8 + 2 * n], s[8 + 2 * n + 1], one);
+                pf[1].pair(n, s[8 + 2 * n], s[8 + 2 * n + 1], kX2PPieces);
             }
             __builtin_amdgcn_sched_barrier(0);
         };
@@ -1109,7 +1103,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         }
         o_max = max_across_halves(o_max);
         const float l_row = sum_across_halves(l_run);
-        const float o_least = (any_large != 0 ? 0x1p1f : 0x1p-2f) * l_row;
+        const float o_least = (any_large != 0 ? 0x1p1f : 0x1p-2f) * kX2PPieces * l_row;
         // (a NaN or an infinity among the outputs is one in their sum)
         odd = odd || !(l_row < __builtin_huge_valf())
             || !(__builtin_fabsf(o_sum) < __builtin_huge_valf())
@@ -1124,7 +1118,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             qk_back = 1.0f;
             to_scores = kScaleHi;
             c = EXPLICIT ? kLog2e : kScaleLog2e;
-            v_back = 1.0f;
+            v_back = kX2PPieces;        // (undone below)
             p_exp = 0.0f;
             m_run = neg_inf();
             l_run = l_low = 0.0f;
@@ -1186,7 +1180,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         }
         const float p_back = p_exp == 0.0f ? 1.0f : 0x1p-4f;
         l_run *= p_back;
-        v_back *= p_back;
+        v_back *= p_back / kX2PPieces;
 #pragma unroll
         for(int db = 0; db < DB; ++db)
         {

@@ -141,3 +141,22 @@ def test_what_is_taken_again_can_be_told(form):
     Q, K, V = draw(8, 2, 128, 768, 64)
     V[..., 7] *= 1e-9
     assert all(walks_again(Q, K, V, form))
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("gap", [6, 8, 10, 12])
+@pytest.mark.parametrize("value", [1e-3, 0.0, 1.0])
+def test_a_first_key_that_takes_most_of_every_row(form, head, gap, value):
+    """Scores of the first key `gap` above the others', and little in its values (as
+    in models that park what a row does not need at the first token): the output is
+    that of the others' probabilities, exp(-gap) and less."""
+    print("case", form, head, gap, value, flush=True)
+    Q, K, V = draw(9, 2, 130, 700, head)
+    Q[..., 0] = 1.0
+    K[..., 0] = 0.0
+    K[:, 0] = 0.0
+    K[:, 0, 0] = gap * math.sqrt(head)
+    V[:, 0] *= value
+    check(Q, K, V, form)
+    check(Q, K, V, form, hip_sdpa.MASK_CAUSAL)
