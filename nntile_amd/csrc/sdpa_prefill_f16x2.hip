@@ -109,10 +109,6 @@ __device__ __forceinline__ bool power_to(float largest, int to, float &scale, fl
     {
         largest = fmaxf(largest, 0x1p-40f);
     }
-    else if(largest == 0.0f)
-    {
-        return true;
-    }
     if(!(largest >= 0x1p-40f && largest < 0x1p40f))
     {
         return false;
@@ -313,7 +309,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     };
 
     // ---- global memory -> registers -> pieces in LDS ------------------------------
-    // K unit u: key u / HG of the step, head values 8 * (u % HG) .. +7.  Its three
+    // K unit u: key u / HG of the step, head values 8 * (u % HG) .. +7.  Its two
     // pieces go to fragment (head group / 2) of the key's block; inside the 512
     // bytes of a lane half the keys' places are permuted so that the 16 lanes of a
     // write hit 16 different ones, and so do those of a read.
@@ -525,9 +521,11 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         };
         k_max = scalar(k_max);
         v_max = scalar(v_max);
-        // (a step of zeros: as if its largest were 8)
+        // (a step of zeros, padding in front, says nothing of what follows: K's as if
+        // its largest were 8, which takes later keys up to 256; V's as if it were 2,
+        // which takes up to 64 and eight of a channel down to 2^-12)
         odd = !power_to<true>(k_max == 0.0f ? 8.0f : k_max, 12, k_scale, k_back) || odd;
-        odd = !power_to<false>(v_max, 12, v_scale, v_back) || odd;
+        odd = !power_to<false>(v_max == 0.0f ? 2.0f : v_max, 12, v_scale, v_back) || odd;
         k_scale = scalar(k_scale);
         v_scale = scalar(v_scale);
         v_back = scalar(v_back);

@@ -115,7 +115,8 @@ def walks_again(Q, K, V, form):
 @pytest.mark.parametrize("form", FORMS)
 @pytest.mark.parametrize("head", [64, 128])
 @pytest.mark.parametrize("what", ["plain", "last channel small", "small spread", "small values",
-                                  "large values", "zero channel", "no value", "one more key"])
+                                  "large values", "zero channel", "no value", "one more key",
+                                  "zeros first", "zeros first, small", "zeros first, large"])
 def test_what_the_pieces_carry_is_not_taken_again(form, head, what):
     print("case", form, head, what, flush=True)
     Q, K, V = draw(7, 2, 128, 769 if "key" in what else 768, head)
@@ -133,6 +134,10 @@ def test_what_the_pieces_carry_is_not_taken_again(form, head, what):
         V[..., 1:4] = 0.0
     elif what == "no value":
         V[:, 32:64] = 0.0
+    elif what.startswith("zeros first"):    # padding in front, a whole step of any form
+        V *= 0.01 if "small" in what else 6.0 if "large" in what else 0.4
+        K[:, :64] = 0.0
+        V[:, :64] = 0.0
     assert not any(walks_again(Q, K, V, form))
 
 
