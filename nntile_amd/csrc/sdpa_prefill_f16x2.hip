@@ -1129,22 +1129,72 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
                     o[db][r] = 0.0f;
                 }
             }
-            const float *Qrow = Qt + my_row() * HEAD;
-#pragma unroll 1
-            for(StepSource src = first_step();; advance(src))
+            // Operands come from the caches, four groups of eight head values (two
+            // halves of 16 bytes a lane) and eight keys ahead, the first of a step
+            // during the products of the step before.
+            constexpr int GROUPS = HEAD / 8, AHEAD = 4, KEYS_AHEAD = 8;
+            const char *Q_at = reinterpret_cast<const char *>(Qt + my_row() * HEAD + 4 * half);
+            f32x4 k_op[AHEAD], q_op[AHEAD];
+            float v_op[KEYS_AHEAD][DB];
+            auto read_kq = [&](const char *K_at, int g) __attribute__((always_inline))
             {
-                const int last = src.rows_left - 1;
+                k_op[g % AHEAD] = *reinterpret_cast<const f32x4 *>(K_at + 32 * g);
+                q_op[g % AHEAD] = *reinterpret_cast<const f32x4 *>(Q_at + 32 * g);
+            };
+            // (rows past the end of the tile are its last one)
+            auto keys_at = [&](const StepSource &src) __attribute__((always_inline)) -> const char *
+            {
+                return reinterpret_cast<const char *>(src.K)
+                    + (uint32_t)((min(grp * kX2Rows + col, src.rows_left - 1) * HEAD + 4 * half) * 4);
+            };
+            auto read_value = [&](const StepSource &src, int r) __attribute__((always_inline))
+            {
+                const int key = grp * kX2Rows + 8 * (r >> 2) + 4 * half + (r & 3);
+                const char *at = reinterpret_cast<const char *>(src.V)
+                    + (uint32_t)((min(key, src.rows_left - 1) * HEAD + col) * 4);
+#pragma unroll
+                for(int db = 0; db < DB; ++db)
+                {
+                    v_op[r % KEYS_AHEAD][db] = *reinterpret_cast<const float *>(at + 128 * db);
+                }
+            };
+            StepSource src = first_step();
+            const char *K_at = keys_at(src);
+#pragma unroll
+            for(int g = 0; g < AHEAD; ++g)
+            {
+                read_kq(K_at, g);
+            }
+            // (keys behind the last that this wavefront's queries see are not walked)
+#pragma unroll 1
+            while(MODE != NNTILE_HIP_MASK_CAUSAL
+                    || src.k_pos + grp * kX2Rows <= wave_qpos_lo + kX2Rows - 1 + p.causal_offset)
+            {
                 f32x16 s;
 #pragma unroll
                 for(int r = 0; r < 16; ++r)
                 {
                     s[r] = 0.0f;
                 }
-                const float *Krow = src.K + (int64_t)min(grp * kX2Rows + col, last) * HEAD;
-#pragma unroll 1
-                for(int j = half; j < HEAD; j += 2)
+#pragma unroll
+                for(int g = 0; g < GROUPS; ++g)
                 {
-                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(Krow[j], q_ok ? Qrow[j] : 0.0f, s, 0, 0, 0);
+                    const f32x4 k = k_op[g % AHEAD], q = q_op[g % AHEAD];
+#pragma unroll
+                    for(int e = 0; e < 4; ++e)
+                    {
+                        s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[e], q[e], s, 0, 0, 0);
+                    }
+                    if(g + AHEAD < GROUPS)
+                    {
+                        read_kq(K_at, g + AHEAD);
+                    }
+                    else
+                    {
+                        read_value(src, 2 * (g + AHEAD - GROUPS));
+                        read_value(src, 2 * (g + AHEAD - GROUPS) + 1);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 apply_mask(src, s);
                 softmax_head(s);
@@ -1154,21 +1204,32 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
                     softmax_one(s, r);
                 }
                 l_low = 0.0f;       // (of an infinite sum: NaN)
+                StepSource next = src;
+                advance(next);
+                K_at = keys_at(next);
 #pragma unroll
                 for(int r = 0; r < 16; ++r)
                 {
-                    const int key = grp * kX2Rows + 8 * (r >> 2) + 4 * half + (r & 3);
-                    const float *Vrow = src.V + (int64_t)min(key, last) * HEAD + col;
 #pragma unroll
                     for(int db = 0; db < DB; ++db)
                     {
-                        o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(Vrow[32 * db], s[r], o[db], 0, 0, 0);
+                        o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(v_op[r % KEYS_AHEAD][db], s[r], o[db], 0, 0, 0);
                     }
+                    if(r + KEYS_AHEAD < 16)
+                    {
+                        read_value(src, r + KEYS_AHEAD);
+                    }
+                    else if(r >= 16 - AHEAD)
+                    {
+                        read_kq(K_at, r + AHEAD - 16);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
                 if(src.step + 1 == n_steps)
                 {
                     break;
                 }
+                src = next;
             }
         }
         if(!EXPLICIT && m_run != neg_inf())

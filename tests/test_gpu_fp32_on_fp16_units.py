@@ -173,6 +173,45 @@ def test_what_is_not_finite(form, head, value, where):
 
 
 @pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("head", [32, 64, 128])
+@pytest.mark.parametrize("mode", ["none", "causal", "additive", "bool"])
+def test_the_walk_in_fp32_at_the_edges_of_its_steps(form, head, mode):
+    """A channel of V far below the others sends every workgroup to it; keys in one
+    tile and, where the mask is a rule, in tiles that end inside a step."""
+    for q_seq, k_seq in SHAPES:
+        print("case", form, head, mode, q_seq, k_seq, flush=True)
+        Q, K, V = draw(q_seq * 5 + k_seq, 3, q_seq, k_seq, head)
+        V[..., 7] *= 1e-9
+        offset = k_seq - q_seq
+        q, k = torch.arange(q_seq)[:, None], torch.arange(k_seq)[None]
+        seen, m, mm = None, None, hip_sdpa.MASK_NONE
+        if mode == "causal":
+            seen, mm = k <= q + offset, hip_sdpa.MASK_CAUSAL
+        elif mode != "none":
+            seen = ((k - q - offset).abs() <= 70) & (q % 17 != 3)
+            mm = hip_sdpa.MASK_ADDITIVE if mode == "additive" else hip_sdpa.MASK_BOOL
+            m = (H.additive_mask(seen.numpy(), "fp32") if mode == "additive" else seen.clone()).cuda()
+        wantA, want = reference(Q, K, V, seen)
+        hidden = torch.isinf(want)
+        outs = [call(Q, K, V, mm, FORMS[form], m, offset)]
+        if m is None:
+            tiles = [[x[:, i:i + 75].contiguous().cuda() for i in range(0, k_seq, 75)] for x in (K, V)]
+            lse, A = torch.full(Q.shape[:2], 1.5, device="cuda"), torch.full_like(Q, 0.25, device="cuda")
+            hip_sdpa.sdpa_fwd_grid(tiles[0], [Q.cuda()], [lse], tiles[1], [A], q_seq, k_seq, q_seq, min(75, k_seq),
+                                   mm, causal_offset=offset, flags=FORMS[form] | hip_sdpa.OVERWRITE)
+            torch.cuda.synchronize()
+            outs.append((A.cpu().double(), lse.cpu().double()))
+        for A, lse in outs:
+            assert torch.equal(torch.isinf(lse), hidden) and (A[hidden] == 0).all()
+            if bool(hidden.all()):
+                continue
+            # (the bounds of test_against_64_bits, for the small channel by itself too)
+            assert rel(A[~hidden], wantA[~hidden]) < 1e-6
+            assert rel(A[~hidden][..., 7], wantA[~hidden][..., 7]) < 1e-6
+            assert float((lse[~hidden] - want[~hidden]).abs().max()) < 1e-6 * (1 + float(want[~hidden].abs().max()))
+
+
+@pytest.mark.parametrize("form", FORMS)
 def test_tiles_of_any_length_and_the_running_pair(oracle, form):
     """Tiles that end inside a step, several slabs, a second call that merges."""
     head, batch, n_slabs, q_seq, q_tile = 64, 2, 2, 300, 150
