@@ -1447,23 +1447,33 @@ static int launch_head(hipStream_t stream, PrefillParams &p, int mode, int form)
 // 112 / 129 / 103 / 161; 32 x 4096 619 / 275 / 238 / 240 / 226.  Head 128, 48 x 1024: 177 /
 // 90 / 67 / 63 / 75; without a mask 290 / 134 / 96 / 110 / 84; 32 x 4096 1490 / 648 / 432 /
 // 444 / 386.
+//
+// Masks given as values: what they hide is not known in front of the launch.  A form is
+// taken for its sum over three masks: open, causal, and a window, of which a workgroup
+// walks its own rows and 64 keys more.  To look over more rows takes longer (scan).  us,
+// the fp32 kernel / 22 / 41, open, causal, window of 32 either side - head 64: 2 x 800
+// 30 29 12.5 / 30 28 18.5 / 40 40 23; 12 x 1000 54 38 18.7 / 39 38 23.4 / 53 53 27; 32 x
+// 1024 99 68 32 / 51 39 27 / 52 53 29; 64 x 1024 190 121 59 / 92 64 47 / 79 60 38; head
+// 128: 2 x 800 51 51 18 / 49 47 26 / 58 57 31; 32 x 1024 232 151 75 / 113 78 56 / 80 77 40.
+// (257 to 512 workgroups of the fp32 kernel at head 64: a window is slower with 22,
+// the others gain more.)
 int prefill_f16x2_form(const PrefillParams &p, int head, int mode)
 {
     struct Cost
     {
         int form, rows, keys;
         double fixed, alone, full, round;      // us: launch, pass, pass on a full CU, round
+        double scan;                            // us: a mask's rows beyond 32
     };
     static const Cost costs[3][5] = {
-        {{kF16x2None, 32, 128, 4.5, 1.59, 1.25, 0.5}, {kF16x2Form22, 64, 64, 6.6, 0.76, 0.58, 1.5},
-            {kF16x2Form41, 128, 32, 6.6, 0.77, 0.56, 1.5}},
-        {{kF16x2None, 32, 128, 5.1, 2.74, 2.50, 1.2}, {kF16x2Form22, 64, 64, 7.7, 1.13, 1.00, 2.3},
-            {kF16x2Form41, 128, 32, 7.7, 0.90, 0.78, 2.6}, {kF16x2Form42, 128, 64, 8.8, 1.31, 1.50, 7.0},
-            {kF16x2Form81, 256, 32, 8.2, 1.30, 1.40, 9.0}},
-        {{kF16x2None, 32, 128, 7.2, 5.23, 5.50, 5.0}, {kF16x2Form22, 64, 64, 10.4, 2.17, 2.33, 8.7},
-            {kF16x2Form41, 128, 32, 9.4, 1.55, 1.31, 5.5}, {kF16x2Form42, 128, 64, 12.2, 2.30, 2.75, 11.0},
-            {kF16x2Form81, 256, 32, 10.3, 2.00, 2.85, 0.0}}};
-    const bool causal = mode == NNTILE_HIP_MASK_CAUSAL;
+        {{kF16x2None, 32, 128, 4.5, 1.59, 1.25, 0.5, 0.0}, {kF16x2Form22, 64, 64, 6.6, 0.76, 0.58, 1.5, 1.5},
+            {kF16x2Form41, 128, 32, 6.6, 0.77, 0.56, 1.5, 3.3}},
+        {{kF16x2None, 32, 128, 5.1, 2.74, 2.50, 1.2, 0.0}, {kF16x2Form22, 64, 64, 7.7, 1.13, 1.00, 2.3, 1.5},
+            {kF16x2Form41, 128, 32, 7.7, 0.90, 0.78, 2.6, 3.3}, {kF16x2Form42, 128, 64, 8.8, 1.31, 1.50, 7.0, 0.0},
+            {kF16x2Form81, 256, 32, 8.2, 1.30, 1.40, 9.0, 0.0}},
+        {{kF16x2None, 32, 128, 7.2, 5.23, 5.50, 5.0, 0.0}, {kF16x2Form22, 64, 64, 10.4, 2.17, 2.33, 8.7, 3.5},
+            {kF16x2Form41, 128, 32, 9.4, 1.55, 1.31, 5.5, 4.5}, {kF16x2Form42, 128, 64, 12.2, 2.30, 2.75, 11.0, 0.0},
+            {kF16x2Form81, 256, 32, 10.3, 2.00, 2.85, 0.0, 0.0}}};
     const bool values = mode == NNTILE_HIP_MASK_ADDITIVE || mode == NNTILE_HIP_MASK_BOOL;
     int best = kF16x2None;
     double least = 0.0;
@@ -1476,24 +1486,27 @@ int prefill_f16x2_form(const PrefillParams &p, int head, int mode)
         }
         const int64_t blocks = (p.q_tile + f.rows - 1) / f.rows;
         const double wgs = (double)p.batch * p.n_slabs * p.n_q_tiles * blocks / 256.0;    // per CU
-        const double rounds = ceil(wgs) - 1.0;
-        auto passes = [&](int64_t last_row)
+        const double start = f.fixed + f.round * (ceil(wgs) - 1.0);
+        auto passes = [&](int64_t keys)
         {
-            const int64_t keys = causal
-                ? last_row + p.q_pos0 - p.k_pos0 + p.causal_offset + 1 : p.k_seq;
             return ceil((double)(keys < 1 ? 1 : keys < p.k_seq ? keys : p.k_seq) / f.keys);
         };
-        const double most = passes(p.q_seq - 1), first = passes((p.q_seq < f.rows ? p.q_seq : f.rows) - 1);
-        double t = f.fixed + f.round * rounds;
-        if(causal)
+        // every query block walks `keys`
+        auto alike = [&](int64_t keys)
         {
+            return start + passes(keys) * (wgs <= 1.0 ? f.alone : ceil(wgs) * f.full);
+        };
+        // row q walks `before` + q + 1
+        auto causal = [&](int64_t before)
+        {
+            const double most = passes(before + p.q_seq);
+            const double first = passes(before + (p.q_seq < f.rows ? p.q_seq : f.rows));
             const double shared = 0.5 * (most + first) * wgs * f.full + (wgs > 1.0 ? 0.5 * first * f.full : 0.0);
-            t += most * f.alone > shared ? most * f.alone : shared;
-        }
-        else
-        {
-            t += wgs <= 1.0 ? most * f.alone : most * ceil(wgs) * f.full;
-        }
+            return start + (most * f.alone > shared ? most * f.alone : shared);
+        };
+        double t = values ? alike(p.k_seq) + causal(0) + alike(f.rows + 64) + 3.0 * f.scan
+            : mode == NNTILE_HIP_MASK_CAUSAL ? causal(p.q_pos0 - p.k_pos0 + p.causal_offset)
+            : alike(p.k_seq);
         // (a close call stays with the fp32 kernel)
         if(f.form == kF16x2None)
         {

@@ -287,3 +287,17 @@ def test_key_ranges_of_a_cache(head, what):
         wantA = wantA * (1 - w)[..., None] + 0.25 * w[..., None]
         assert rel(A, wantA) < 1e-6
         assert float((lse - torch.logaddexp(want, torch.tensor(0.5).double())).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("head, batch, seq, fp32", [(64, 2, 800, True), (64, 12, 300, True), (64, 2, 2048, True),
+                                                    (128, 2, 800, True), (128, 12, 300, True), (128, 2, 2048, True),
+                                                    (64, 32, 1024, False), (128, 32, 500, False)])
+def test_masks_given_as_values_go_where_a_window_is_not_slower(head, batch, seq, fp32):
+    """Few workgroups of few steps: the 32-query kernel, whose bits the call then has."""
+    print("case", head, batch, seq, flush=True)
+    Q, K, V = draw(seq, batch, seq, seq, head)
+    seen = (torch.arange(seq)[None] - torch.arange(seq)[:, None]).abs() <= 32
+    for mode, m in ((hip_sdpa.MASK_ADDITIVE, H.additive_mask(seen.numpy(), "fp32")), (hip_sdpa.MASK_BOOL, seen)):
+        (A, lse), (A32, lse32) = (call(Q, K, V, mode, flags, m.cuda()) for flags in (0, FP32))
+        assert torch.equal(A, A32) == fp32
+        assert rel(A, A32) < 2e-6 and rel(lse, lse32) < 2e-6
