@@ -336,6 +336,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     StepSource k_src = {}, v_src = {}, s_src = {};      // the rows requested last, the scores
     f32x4 k_raw[SETS][UPT][2];
     float v_raw[SETS][UPT][8];
+    float k_scale = 1.0f, v_scale = 1.0f, v_back = 1.0f;
     uint32_t k_goff, v_goff;
     int k_at, v_at;
     {
@@ -379,6 +380,26 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             asm volatile("" : "+v"(k_raw[set][i][0]), "+v"(k_raw[set][i][1]));
         }
     };
+    // Units of the last one or two rows of a tile do not say how small a channel is: one
+    // value in 4000 of N(0, 1) is below what look_at_unit asks for, so one in 15 heads
+    // of 128 would walk its keys again for one of them (24 heads, 710 x 1781, head 128, 78 us
+    // or 330).  They hold that much in rows past the end, unless their values are below
+    // 2^-12 or nothing else speaks for the channel (a first step of one or two rows).
+    constexpr float LEAST = 0x1p-2f;
+    auto few_rows = [&](int set) __attribute__((always_inline))
+    {
+#pragma unroll
+        for(int i = 0; i < UPT; ++i)
+        {
+            const int rows = v_src.rows_left - (int)(v_goff / (HEAD * 4)) - v_rows(i * SSTRIDE);
+            const float largest = fmaxf(__builtin_fabsf(v_raw[set][i][0]), __builtin_fabsf(v_raw[set][i][1]));
+            const bool alone = v_src.step == 0 && v_src.rows_left <= 2;
+            if(rows <= 2 && !alone && largest >= 0x1p-10f * LEAST * v_back)
+            {
+                v_raw[set][i][7] = LEAST * v_back;
+            }
+        }
+    };
     auto load_v_tail = [&](int set) __attribute__((always_inline))
     {
 #pragma unroll
@@ -407,6 +428,10 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
                     v_raw[set][i][e] = 0.0f;
                 }
             }
+        }
+        if(v_src.step > 0)      // (the first step: once its power of two is known)
+        {
+            few_rows(set);
         }
     };
     auto load_k = [&](int set) __attribute__((always_inline))
@@ -442,7 +467,6 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
 
     // ---- this lane's operands and the powers of two --------------------------------
     Split8 qf[CH];
-    float k_scale = 1.0f, v_scale = 1.0f, v_back = 1.0f;
     float qk_back = 1.0f;       // scores / (what the matrix unit computes)
     bool odd = false;           // something that the pieces cannot carry
     __shared__ int any_odd, any_large;
@@ -529,6 +553,10 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         k_scale = scalar(k_scale);
         v_scale = scalar(v_scale);
         v_back = scalar(v_back);
+        if(v_src.rows_left < KEYS)
+        {
+            few_rows(0);
+        }
         qk_back = q_back * k_back;
         odd = odd || !(qk_back <= kX2Scores);
         if(__builtin_amdgcn_ballot_w64(odd && q_ok) != 0)
@@ -553,7 +581,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     // to 2^13 or beyond.
     bool too_small = false, large = false;
     float unit_max = 0.0f;
-    const float v_least = 0x1p-2f * v_back, v_large = 0x1p13f * v_back;
+    const float v_least = LEAST * v_back, v_large = 0x1p13f * v_back;
     auto look_at_pair = [&](int j, float a, float b) __attribute__((always_inline))
     {
         const float x = __builtin_fabsf(a), y = __builtin_fabsf(b);

@@ -165,3 +165,19 @@ def test_a_first_key_that_takes_most_of_every_row(form, head, gap, value):
     V[:, 0] *= value
     check(Q, K, V, form)
     check(Q, K, V, form, hip_sdpa.MASK_CAUSAL)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("k_seq", [769, 770, 773, 774, 33, 37])
+def test_a_few_small_values_in_the_last_rows_are_not_taken_again(form, head, k_seq):
+    """A last group of one or two rows (of a later step, of the first one) some of
+    whose channels are below 2^-2 at the power of two of the first step."""
+    print("case", form, head, k_seq, flush=True)
+    Q, K, V = draw(10, 2, 128, k_seq, head)
+    V[:, -1, ::9] = 1e-4
+    V[:, -2, ::9] *= 1e-4 if k_seq % 2 == 0 else 1.0
+    assert not any(walks_again(Q, K, V, form))
+    V[..., 7] *= 1e-9
+    assert all(walks_again(Q, K, V, form))
+    check(Q, K, V, form)
