@@ -1512,9 +1512,9 @@ int prefill_f16x2_form(const PrefillParams &p, int head, int mode)
         {
             continue;
         }
-        const int64_t blocks = (p.q_tile + f.rows - 1) / f.rows;
-        const double wgs = (double)p.batch * p.n_slabs * p.n_q_tiles * blocks / 256.0;    // per CU
-        const double start = f.fixed + f.round * (ceil(wgs) - 1.0);
+        const int64_t all = p.n_q_tiles * ((p.q_tile + f.rows - 1) / f.rows);     // query blocks
+        auto per_cu = [&](int64_t n) { return (double)p.batch * p.n_slabs * n / 256.0; };
+        auto start = [&](double wgs) { return f.fixed + f.round * (ceil(wgs) - 1.0); };
         auto passes = [&](int64_t keys)
         {
             return ceil((double)(keys < 1 ? 1 : keys < p.k_seq ? keys : p.k_seq) / f.keys);
@@ -1522,15 +1522,21 @@ int prefill_f16x2_form(const PrefillParams &p, int head, int mode)
         // every query block walks `keys`
         auto alike = [&](int64_t keys)
         {
-            return start + passes(keys) * (wgs <= 1.0 ? f.alone : ceil(wgs) * f.full);
+            const double wgs = per_cu(all);
+            return start(wgs) + passes(keys) * (wgs <= 1.0 ? f.alone : ceil(wgs) * f.full);
         };
-        // row q walks `before` + q + 1
+        // row q walks `before` + q + 1; the workgroups of rows that see no key end at once
+        // (32 heads, 984 x 209, causal from the last key, head 64: 15.1 us with 41, which
+        // was taken for their sake, 12.5 with the fp32 kernel)
         auto causal = [&](int64_t before)
         {
-            const double most = passes(before + p.q_seq);
-            const double first = passes(before + (p.q_seq < f.rows ? p.q_seq : f.rows));
+            const int64_t rows = before >= 0 ? p.q_seq : p.q_seq + before > 1 ? p.q_seq + before : 1;
+            const int64_t from = before > 0 ? before : 0, seen = (rows + f.rows - 1) / f.rows;
+            const double wgs = per_cu(before < 0 && seen < all ? seen : all);
+            const double most = passes(from + rows);
+            const double first = passes(from + (rows < f.rows ? rows : f.rows));
             const double shared = 0.5 * (most + first) * wgs * f.full + (wgs > 1.0 ? 0.5 * first * f.full : 0.0);
-            return start + (most * f.alone > shared ? most * f.alone : shared);
+            return start(wgs) + (most * f.alone > shared ? most * f.alone : shared);
         };
         double t = values ? alike(p.k_seq) + causal(0) + alike(f.rows + 64) + 3.0 * f.scan
             : mode == NNTILE_HIP_MASK_CAUSAL ? causal(p.q_pos0 - p.k_pos0 + p.causal_offset)

@@ -301,3 +301,39 @@ def test_masks_given_as_values_go_where_a_window_is_not_slower(head, batch, seq,
         (A, lse), (A32, lse32) = (call(Q, K, V, mode, flags, m.cuda()) for flags in (0, FP32))
         assert torch.equal(A, A32) == fp32
         assert rel(A, A32) < 2e-6 and rel(lse, lse32) < 2e-6
+
+
+@pytest.mark.parametrize("head, batch, q_seq, k_seq", [(64, 32, 984, 209), (64, 32, 362, 196)])
+def test_rows_that_see_no_key_do_not_pick_the_form(head, batch, q_seq, k_seq):
+    """Causal from the last key on: few workgroups walk at all, and the 32-query kernel
+    is done first."""
+    print("case", head, batch, q_seq, k_seq, flush=True)
+    Q, K, V = draw(q_seq, batch, q_seq, k_seq, head)
+    (A, lse), (A32, lse32) = (call(Q, K, V, hip_sdpa.MASK_CAUSAL, flags, offset=k_seq - q_seq) for flags in (0, FP32))
+    assert torch.equal(A, A32) and torch.equal(lse, lse32)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("head", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("mean", [0.0, 1.0])
+def test_long_walks(form, head, causal, mean):
+    """Roundings add up along a wavefront's keys.  Of n keys one of the fp32 kernel
+    adds n/4, two an instruction, n/8 roundings in each of four sums a fourth as large;
+    here it is n, 16 by three instructions (one key block; of two, half as many in sums
+    half as large).  With values of one sign the variances are as 1 to 6 (1.5): errors
+    as 1 to 2.45 (1.23), and less where signs change; a tenth on top for what else
+    rounds."""
+    print("case", form, head, causal, mean, flush=True)
+    q_seq, k_seq = 256, 8192
+    Q, K, V = draw(21, 2, q_seq, k_seq, head)
+    V += mean
+    offset = k_seq - q_seq
+    seen = torch.arange(k_seq)[None] <= torch.arange(q_seq)[:, None] + offset if causal else None
+    mode = hip_sdpa.MASK_CAUSAL if causal else hip_sdpa.MASK_NONE
+    wantA, want = reference(Q, K, V, seen)
+    (A, lse), (A32, lse32) = (call(Q, K, V, mode, f, offset=offset) for f in (FORMS[form], FP32))
+    got, fp32 = rel(A, wantA), rel(A32, wantA)
+    print("%.2e, fp32 %.2e; lse %.2e, %.2e" % (got, fp32, rel(lse, want), rel(lse32, want)), flush=True)
+    assert got < (2.45 if form in ("4x1", "8x1") else 1.23) * 1.1 * fp32
+    assert rel(lse, want) < 1.1 * rel(lse32, want)
