@@ -15,11 +15,15 @@
 // absolutely below, so the values are moved there by powers of two, which are
 // exact: a row of Q so that its largest value is in [2^13, 2^14), K and V so that
 // the largest of a workgroup's first step is in [2^11, 2^12), the probabilities
-// (at most 1) by 2^15.  What that does not cover - infinities and NaN, later keys
-// 16 times larger than those of the first step, blocks of V 1000 times smaller,
-// rows of the output or of Q beyond 2^+-40 - is found by a test of the blocks as
-// they are split and of the results, and the workgroup then walks its keys again
-// with fp32 matrix instructions.
+// (at most 1) by 2^15.  A workgroup takes its keys with fp32 matrix instructions
+// where that does not do.  From the start: rows whose scores the pieces may not carry
+// (below), Q, K or V beyond 2^40, V below 2^-40.  A second time, found on the way or in
+// the results: infinities and NaN, later keys or values more than 16 times larger
+// than those of the first step (an overflow makes them NaN), eight values of a channel
+// of V that are split together all 2^-13 times the first step's largest or less, rows
+// of the output that are as small.  What stays is, in a score, below 2^-21 of the
+// factors' largest product or less, and in the output 2^-23 of each probability times the
+// largest of the eight values of its channel that lie beside it.
 //
 // Scores: what a piece loses absolutely, 2^-25 of a scaled value, counts by what it
 // is multiplied with.  With q and k the largest values of a row of Q and of the first
@@ -870,6 +874,71 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             l_run = sum;
         }
     };
+    // A long walk's output is put by and begun anew every PUT_BY steps.  Three
+    // instructions a 16 keys round a sum that grows with the walk where a wavefront of
+    // the fp32 kernel, eight keys an instruction, adds up a fourth of it: without this,
+    // head 64, 16 x 2150 without a mask, A was off by 5.5e-7 against 5.2e-7 with fp32
+    // products, 16 x 8192 10.4e-7 / 8.7e-7, and 8.5e-7 / 3.4e-7 where values have a mean of
+    // 1; now 3.3e-7, 3.4e-7 and 1.0e-7.  In registers where they last, 16 steps (24 x 1750
+    // 84.5 -> 85.5 us, 32 x 2150 causal 87.6 -> 88.7); else in scratch memory, which a full
+    // chip writes and reads in 4 us, 64 steps (head 128, 16 x 4096 364 -> 370; with 16 steps
+    // 393; causal, 4 x 1, 32 x 4096 433 -> 446, others 0 to 1 %).  In registers there: spills
+    // in the loop, 48 x 1024 64 -> 73.  (Not carried in 64 steps: head 128, values of one
+    // sign, 600 to 4000 keys of a wavefront, up to 2.5e-7 where fp32 products have 1.3e-7.)
+    constexpr bool BY_MEMORY = HEAD == 128 || (HEAD == 64 && (QW == 2 || EXPLICIT));
+    constexpr int PUT_BY = BY_MEMORY ? 64 : 16, PUT_BY_FP32 = BY_MEMORY ? 32 : 16;
+    struct PutBy
+    {
+        f32x16 o[DB];
+        float m;
+    };
+    PutBy put;
+    float m_here = 0.0f;        // (of what is in memory, beside it where registers are short)
+    float &m_by = EXPLICIT ? put.m : m_here;
+    bool by = false;
+    // (whoever might look at it there: the compiler keeps it out of registers)
+    auto keep_in_memory = [&]() __attribute__((always_inline))
+    {
+        if(BY_MEMORY)
+        {
+            asm volatile("" : : "v"(&put) : "memory");
+        }
+    };
+    auto add_what_was_put_by = [&]() __attribute__((always_inline))
+    {
+        keep_in_memory();
+        const float m_use = (m_run == neg_inf()) ? 0.0f : m_run;
+        const float alpha = fast_exp2((m_by - m_use) * c);
+#pragma unroll
+        for(int db = 0; db < DB; ++db)
+        {
+#pragma unroll
+            for(int r = 0; r < 16; ++r)
+            {
+                o[db][r] = fmaf(put.o[db][r], alpha, o[db][r]);
+            }
+        }
+    };
+    auto put_by = [&]() __attribute__((always_inline))
+    {
+        if(by)
+        {
+            add_what_was_put_by();
+        }
+        by = true;
+        m_by = m_run;
+#pragma unroll
+        for(int db = 0; db < DB; ++db)
+        {
+            put.o[db] = o[db];
+#pragma unroll
+            for(int r = 0; r < 16; ++r)
+            {
+                o[db][r] = 0.0f;
+            }
+        }
+        keep_in_memory();
+    };
 
     // ---- the walk -------------------------------------------------------------------
     if(n_steps > 0)
@@ -1064,11 +1133,12 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         {
             return (min(src.rows_left / KEYS, last_step - src.step + 1) - 1) / 2;
         };
-        int pairs = last_step / 2;
+        int pairs = last_step / 2, since = 0;
 #pragma unroll 1
         while(pairs > 0)
         {
-            const int inner = min(pairs, min(inner_pairs(k_src), inner_pairs(v_src)));
+            const int inside_tile = min(inner_pairs(k_src), inner_pairs(v_src));
+            const int inner = min(min(pairs, PUT_BY / 2 - since), inside_tile);
 #pragma unroll 1
             for(int n = 0; n < inner; ++n)
             {
@@ -1084,10 +1154,17 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             inside(k_src);
             inside(v_src);
             pairs -= inner;
-            if(pairs > 0)
+            since += inner;
+            if(pairs > 0 && inner == inside_tile)
             {
                 two_passes(std::integral_constant<bool, false>{});
                 --pairs;
+                ++since;
+            }
+            if(pairs > 0 && since >= PUT_BY / 2)
+            {
+                put_by();
+                since = 0;
             }
         }
         if(last_step & 1)
@@ -1108,6 +1185,10 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         first_v(last_step & 1);
         pieces_b(s_even);
         output(last_step & 1, [](int) {}, [](int) {});
+        if(by)
+        {
+            add_what_was_put_by();
+        }
     }
 
     // ---- results that the pieces could not carry: once more in fp32 --------------------
@@ -1148,6 +1229,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             p_exp = 0.0f;
             m_run = neg_inf();
             l_run = l_low = 0.0f;
+            by = false;
 #pragma unroll
             for(int db = 0; db < DB; ++db)
             {
@@ -1257,7 +1339,15 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
                 {
                     break;
                 }
+                if(src.step % PUT_BY_FP32 == PUT_BY_FP32 - 1)
+                {
+                    put_by();
+                }
                 src = next;
+            }
+            if(by)
+            {
+                add_what_was_put_by();
             }
         }
         if(!EXPLICIT && m_run != neg_inf())
