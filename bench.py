@@ -34,7 +34,7 @@ PEAK_HBM_GBS = 8000.0         # MI355X HBM3E
 TRAFFIC = {
     "cfg3_llama_prefill_bf16": (177694720, "profiles/sdpa_prefill_16bit_kernel_cfg3_llama_prefill_bf16.txt"),
     "cfg4_gqa_decode_bf16": (288423936, "profiles/sdpa_decode_16bit_kernel_cfg4_gqa_decode_bf16.txt"),
-    "cfg2_gpt2_small_fp32": (55611392, "profiles/sdpa_prefill_f16x2_kernel_cfg2_gpt2_small_fp32.txt"),
+    "cfg2_gpt2_small_fp32": (52920320, "profiles/sdpa_prefill_f16x2_kernel_cfg2_gpt2_small_fp32.txt"),
     # row dots (64 MiB read, 0.5 MiB written) + the gradient launch (444.2 MiB read, 96.0 MiB written)
     "cfg3_backward": (634099712, "profiles/sdpa_bwd_kernels_cfg3_llama_prefill_bf16.txt"),
 }

@@ -21,9 +21,9 @@
 // the results: infinities and NaN, later keys or values more than 16 times larger
 // than those of the first step (an overflow makes them NaN), eight values of a channel
 // of V that are split together all 2^-13 times the first step's largest or less, rows
-// of the output that are as small.  What stays is, in a score, below 2^-21 of the
-// factors' largest product or less, and in the output 2^-23 of each probability times the
-// largest of the eight values of its channel that lie beside it.
+// of the output that are as small.  What stays is 2^-22 of a product and, absolutely,
+// 2^-23 of a score (below) and 2^-23 of a probability times the largest of the eight
+// values that are split together.
 //
 // Scores: what a piece loses absolutely, 2^-25 of a scaled value, counts by what it
 // is multiplied with.  With q and k the largest values of a row of Q and of the first
@@ -47,7 +47,7 @@
 //
 // What bounds it: the vector port.  A matrix instruction takes it for 16 clocks
 // and every vector instruction for 4; a pass at head 64 is 24 of the first and
-// about 160 (8 x 1: 125) of the second for 32 x 32 scores, 1 100 clocks against 768
+// about 175 (8 x 1: 120) of the second for 32 x 32 scores, 1 090 clocks against 768
 // of the matrix unit; two wavefronts a SIMD come to 70 % of that.  (Three bf16
 // pieces, which need no powers of two: twice the products and 11 instead of 6
 // vector instructions for a pair of values, 50 us where this took 41 at 48 x 1024
