@@ -128,7 +128,16 @@ int nntile_hip_flash_sdpa_fwd_fp16(void *stream, int64_t seq, int64_t head,
         uint16_t *scratch_A, float *lse, uint16_t *A);
 /* fp32 has no counterpart in the reference's flash pack
  * (include/nntile/starpu/flash_sdpa_fwd_cudnn.hh:149-153 lists bf16, fp16);
- * it is added so that fp32 models take the same path. */
+ * it is added so that fp32 models take the same path.
+ *
+ * Products of fp32 tiles here and in the tile, grid and key-range calls (not in
+ * decode): launches of more than a few workgroups take them on the fp16 matrix
+ * units, each value as two fp16 pieces (22 bits), three products, sums in fp32;
+ * values that two pieces do not carry are found and taken in fp32.  Against 64
+ * bits the results are no further off than with fp32 products on N(0, 1) values;
+ * where the values of V have a mean of 1, up to 2.1 times as far (1024 keys, head
+ * 128, no mask: 2.9e-7 in the 2-norm of A, to 1.4e-7).  Tile and grid calls with
+ * NNTILE_HIP_SDPA_FORM_SPLIT take fp32 products. */
 int nntile_hip_flash_sdpa_fwd_fp32(void *stream, int64_t seq, int64_t head,
         int64_t batch, const float *K, const float *Q, const float *mask,
         float *scratch_lse, const float *V, float *scratch_A, float *lse,
