@@ -882,14 +882,14 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     // 1; now 3.3e-7, 3.4e-7 and 1.0e-7.  In registers where they last, 16 steps (24 x 1750
     // 84.5 -> 85.5 us, 32 x 2150 causal 87.6 -> 88.7); else in scratch memory, which a full
     // chip writes and reads in 4 us: every 1024 keys of a wavefront where it walks all
-    // of them (head 128, G = 1; without a mask 16 x 4096 346 us without, 357 every 2048
+    // of them (G = 1; head 128 without a mask, 16 x 4096 346 us without, 357 every 2048
     // keys, 366 every 1024, 386 every 512; 16 x 2150 141, 145, 152, 165; A there 5.9e-7,
     // 4.6e-7, 3.8e-7, with fp32 products 5.9e-7; values with a mean of 1 4.3e-7, 2.2e-7,
     // 1.3e-7, fp32 1.9e-7), else 2048.  In registers there: spills in the loop, 48 x 1024
     // 64 -> 73.  (Not carried in 1024 keys: head 128, values of one sign, 400 to 1100 keys of
     // a wavefront, up to 2.9e-7 where fp32 products have 1.4e-7.)
     constexpr bool BY_MEMORY = HEAD == 128 || (HEAD == 64 && (QW == 2 || EXPLICIT));
-    constexpr int PUT_BY = !BY_MEMORY ? 16 : HEAD == 128 && G == 1 ? 32 : 64;
+    constexpr int PUT_BY = !BY_MEMORY ? 16 : G == 1 ? 32 : 64;
     constexpr int PUT_BY_FP32 = BY_MEMORY ? 32 : 16;
     struct PutBy
     {

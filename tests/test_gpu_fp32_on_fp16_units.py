@@ -382,14 +382,18 @@ def test_the_first_steps_of_a_long_walk_are_hidden():
                 assert float((lse[~hidden] - want[~hidden]).abs().max()) < 1e-5
 
 
-@pytest.mark.parametrize("form", ["4x1", "8x1"])
-def test_one_key_block_at_head_128_is_put_by_every_1024_keys(form):
+@pytest.mark.parametrize("form, head, mode", [("4x1", 128, "none"), ("8x1", 128, "none"),
+                                              ("4x1", 64, "additive"), ("4x1", 64, "bool")])
+def test_one_key_block_is_put_by_every_1024_keys(form, head, mode):
     """A wavefront that walks all keys, values of one sign: with f = 1024 the variance
     f^2/16n + n/3f is 31 S^2 at 2150 keys, the fp32 kernel's n/96 is 22 (test_long_walks):
     a ratio of 1.18 of the errors, 2.33 with f = 2048."""
-    Q, K, V = draw(23, 2, 2150, 2150, 128)
+    Q, K, V = draw(23, 2, 2150, 2150, head)
     V += 1.0
     wantA, want = reference(Q, K, V, None)
-    got, fp32 = (rel(call(Q, K, V, hip_sdpa.MASK_NONE, flags)[0], wantA) for flags in (FORMS[form], FP32))
-    print("case %s %.2e, fp32 %.2e" % (form, got, fp32), flush=True)
+    seen = torch.ones(2150, 2150, dtype=torch.bool)
+    m = {"none": None, "additive": torch.zeros(2150, 2150), "bool": seen}[mode]
+    mm = {"none": hip_sdpa.MASK_NONE, "additive": hip_sdpa.MASK_ADDITIVE, "bool": hip_sdpa.MASK_BOOL}[mode]
+    got, fp32 = (rel(call(Q, K, V, mm, flags, m if m is None else m.cuda())[0], wantA) for flags in (FORMS[form], FP32))
+    print("case %s %d %s %.2e, fp32 %.2e" % (form, head, mode, got, fp32), flush=True)
     assert got < 1.4 * fp32
