@@ -370,11 +370,14 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     };
     auto load_k_tail = [&](int set) __attribute__((always_inline))
     {
+        uint32_t goff = k_goff;
+        asm volatile("" : "+v"(goff));      // (worked out here, not kept in registers or
+                                            // scratch memory through the walk)
 #pragma unroll
         for(int i = 0; i < UPT; ++i)
         {
-            const int key = (int)(k_goff / (HEAD * 4)) + i * KSTRIDE;
-            const uint32_t off = k_goff + (uint32_t)(i * KSTRIDE * HEAD * 4)
+            const int key = (int)(goff / (HEAD * 4)) + i * KSTRIDE;
+            const uint32_t off = goff + (uint32_t)(i * KSTRIDE * HEAD * 4)
                 - (uint32_t)(max(key - (k_src.rows_left - 1), 0) * HEAD * 4);
             const char *at = reinterpret_cast<const char *>(k_src.K) + off;
             k_raw[set][i][0] = *reinterpret_cast<const f32x4 *>(at);
@@ -390,12 +393,12 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     // or 330).  They hold that much in rows past the end, unless their values are below
     // 2^-12 or nothing else speaks for the channel (a first step of one or two rows).
     constexpr float LEAST = 0x1p-2f;
-    auto few_rows = [&](int set) __attribute__((always_inline))
+    auto few_rows = [&](int set, uint32_t goff) __attribute__((always_inline))
     {
 #pragma unroll
         for(int i = 0; i < UPT; ++i)
         {
-            const int rows = v_src.rows_left - (int)(v_goff / (HEAD * 4)) - v_rows(i * SSTRIDE);
+            const int rows = v_src.rows_left - (int)(goff / (HEAD * 4)) - v_rows(i * SSTRIDE);
             const float largest = fmaxf(__builtin_fabsf(v_raw[set][i][0]), __builtin_fabsf(v_raw[set][i][1]));
             const bool alone = v_src.step == 0 && v_src.rows_left <= 2;
             if(rows <= 2 && !alone && largest >= 0x1p-10f * LEAST * v_back)
@@ -406,6 +409,8 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
     };
     auto load_v_tail = [&](int set) __attribute__((always_inline))
     {
+        uint32_t goff = v_goff;
+        asm volatile("" : "+v"(goff));      // (as above)
 #pragma unroll
         for(int i = 0; i < UPT; ++i)
         {
@@ -413,8 +418,8 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             for(int e = 0; e < 8; ++e)
             {
                 const int add = v_rows(i * SSTRIDE) + (e < 4 ? e : e + 4);
-                const int key = (int)(v_goff / (HEAD * 4)) + add;
-                const uint32_t off = v_goff + (uint32_t)(add * HEAD * 4)
+                const int key = (int)(goff / (HEAD * 4)) + add;
+                const uint32_t off = goff + (uint32_t)(add * HEAD * 4)
                     - (uint32_t)(max(key - (v_src.rows_left - 1), 0) * HEAD * 4);
                 v_raw[set][i][e] = *reinterpret_cast<const float *>(
                         reinterpret_cast<const char *>(v_src.V) + off);
@@ -424,7 +429,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
             {
                 asm volatile("" : "+v"(v_raw[set][i][e]));      // (as above)
             }
-            if((int)(v_goff / (HEAD * 4)) + v_rows(i * SSTRIDE) >= v_src.rows_left)
+            if((int)(goff / (HEAD * 4)) + v_rows(i * SSTRIDE) >= v_src.rows_left)
             {
 #pragma unroll
                 for(int e = 0; e < 8; ++e)
@@ -435,7 +440,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         }
         if(v_src.step > 0)      // (the first step: once its power of two is known)
         {
-            few_rows(set);
+            few_rows(set, goff);
         }
     };
     auto load_k = [&](int set) __attribute__((always_inline))
@@ -559,7 +564,7 @@ void sdpa_prefill_f16x2_kernel(const PrefillParams p)
         v_back = scalar(v_back);
         if(v_src.rows_left < KEYS)
         {
-            few_rows(0);
+            few_rows(0, v_goff);
         }
         qk_back = q_back * k_back;
         odd = odd || !(qk_back <= kX2Scores);
