@@ -29,6 +29,7 @@
 // (BwdTile::swz), which keeps both the row reads and the transposing reads
 // free of bank conflicts.
 #include <type_traits>
+#include <utility>
 
 #include "sdpa_common.hpp"
 
@@ -88,6 +89,9 @@ namespace nntile_hip
 #endif
 #ifndef NNTILE_BWD_AHEAD
 #define NNTILE_BWD_AHEAD 2          // LDS operands are read this many MFMAs early
+#endif
+#ifndef NNTILE_BWD_AHEAD_WIDE
+#define NNTILE_BWD_AHEAD_WIDE 2     // the same where a workgroup holds both gradients at head 128
 #endif
 #ifndef NNTILE_BWD_SPREAD
 #define NNTILE_BWD_SPREAD 2
@@ -179,6 +183,23 @@ __device__ __forceinline__ int lane_index_again()
     int l;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
     return l;
+}
+
+// base ^ BITS, in assembly text: the compiler would make all the places that
+// differ by a constant once, before the loop, and spill them.
+template<int BITS>
+__device__ __forceinline__ uint32_t flip_bits(uint32_t base)
+{
+    uint32_t r;
+    asm volatile("v_xor_b32 %0, %1, %2" : "=v"(r) : "n"(BITS), "v"(base));
+    return r;
+}
+
+// f(0), f(1), .. f(N-1), each index a compile-time constant
+template<typename F, int... I>
+__device__ __forceinline__ void each_slot(F f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
 }
 
 __device__ __forceinline__ int tile_row(int r, int half)
@@ -1152,16 +1173,9 @@ enum { BWD_PART_DK = 1, BWD_PART_DV = 2 };
 // Where one workgroup holds both gradients of its keys: at head sizes up to 64
 // under every mask mode; at head 128 (K and V fragments and the two
 // accumulators are 192 of a lane's 256 registers there) under the analytic
-// modes, with the blocks of a step one after the other and a few registers
-// spilled - 12 scratch accesses a step beside its 64 MFMAs.
+// modes, with the blocks of a step one after the other, product by product.
 #ifndef NNTILE_BWD_FUSED_KEYS_HEAD
 #define NNTILE_BWD_FUSED_KEYS_HEAD 64
-#endif
-#ifndef NNTILE_BWD_GOFF_IN_LDS
-#define NNTILE_BWD_GOFF_IN_LDS 1
-#endif
-#ifndef NNTILE_BWD_FUSED_ORDER
-#define NNTILE_BWD_FUSED_ORDER 1      // 1: product by product at head 128; 0: S with dP, then dV with dK
 #endif
 #ifndef NNTILE_BWD_FUSED_KEYS_HEAD_ANALYTIC
 #define NNTILE_BWD_FUSED_KEYS_HEAD_ANALYTIC 128
@@ -1178,7 +1192,7 @@ template<typename T, int HEAD, int MODE, int PART, bool GRID>
 __device__ __forceinline__ void sdpa_bwd_dkv_body(
         const std::conditional_t<GRID, BwdGridParams, BwdParams> &p, unsigned wg,
         char *lds_q0, char *lds_q1, char *lds_g0, char *lds_g1,
-        float (*lds_stat_arg)[2][kBwdStep])
+        float (*lds_stat)[2][kBwdStep])
 {
     constexpr bool DO_DK = (PART & BWD_PART_DK) != 0, DO_DV = (PART & BWD_PART_DV) != 0;
     constexpr bool BOTH = DO_DK && DO_DV;
@@ -1302,28 +1316,16 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
         ld_goff[i] = (uint32_t)(r * RB + (ld_cpos ^ G::swz(r)) * 16);
         ld_goff_end[i] = ld_goff[i] - (uint32_t)(max(r - (q_seq - 1) % kBwdStep, 0) * RB);
     }
-    // Both gradients at head 128 leave no registers for these tables, and a
-    // spilled entry is reloaded from scratch with a wait for every load in
-    // flight, the next step's tile loads included: they go to LDS, whose reads
-    // have a counter of their own.
-    constexpr bool GOFF_IN_LDS = BOTH && HEAD > 64 && NNTILE_BWD_GOFF_IN_LDS != 0;
-    // (the statistics of the two buffers behind them in the same array: one
-    // register, the thread's place in the array, then addresses all of it)
-    __shared__ __attribute__((aligned(16))) uint32_t lds_goff[GOFF_IN_LDS
-        ? (2 * LPW + 1) * kDkvThreads : 1];
-    static_assert(2 * 2 * kBwdStep <= kDkvThreads, "two buffers of statistics in one row of the table");
-    float (*lds_stat)[2][kBwdStep] = GOFF_IN_LDS
-        ? reinterpret_cast<float (*)[2][kBwdStep]>(lds_goff + 2 * LPW * kDkvThreads) : lds_stat_arg;
-    if constexpr(GOFF_IN_LDS)
-    {
-#pragma unroll
-        for(int i = 0; i < LPW; ++i)
-        {
-            lds_goff[i * kDkvThreads + tid] = ld_goff[i];
-            lds_goff[(LPW + i) * kDkvThreads + tid] = ld_goff_end[i];
-        }
-        // (each thread reads back what it wrote: no barrier needed)
-    }
+    // Both gradients at head 128 leave no registers for the tables of offsets
+    // here and below: one register stands for each table, an exclusive or with a
+    // constant makes the entry where it is used (the chunk index of a row's
+    // swizzled place is an exclusive or of the row's and the chunk's own bits).
+    constexpr bool WIDE = BOTH && HEAD > 64;
+    static_assert(!WIDE || (CPR == 16 && ROWS_PER_LOAD == 4 && LPW == 4 && LOADERS == kDkvWaves
+                && KSTEPS == 8 && DBLOCKS == 4), "the wide body's offsets are those of head 128");
+    // (a load's rows 4j + lane / 16 of the wavefront's 16 have the swizzle of
+    // lane / 16 with bits j)
+    const uint32_t wide_goff = ld_goff[0];
     // row operand: lane (col, half) reads row mb*32+col, logical chunk 2*ks+half;
     // 32 rows further on the swizzle is the same, so mb goes into the immediate
     uint32_t row_raddr[KSTEPS];
@@ -1360,7 +1362,8 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
             dv[db][r] = 0.0f;
         }
     }
-    const float c = p.scale * kLog2e;
+    const float c = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+                __builtin_bit_cast(int, p.scale * kLog2e)));
     // mask values: byte offsets of the lane's key within a row of the mask,
     // for the rows of the lower and of the upper half of the wave (the
     // launcher keeps 64 rows of the mask within 32 bits)
@@ -1431,41 +1434,49 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
         const char *Gp = static_cast<const char *>(at.dA) + at.elem * RB;
         char *qdst = qdst_base + wave_u * LPW * 1024;
         char *gdst = gdst_base + wave_u * LPW * 1024;
-        uint32_t goff;
-        if constexpr(GOFF_IN_LDS)
-        {
-            goff = lds_goff[((at_end ? LPW : 0) + j) * kDkvThreads + tid];
-        }
-        else
-        {
-            goff = at_end ? ld_goff_end[j] : ld_goff[j];
-        }
+        const uint32_t goff = at_end ? ld_goff_end[j] : ld_goff[j];
         load_to_lds16<0, false>(Qp, goff, qdst + j * 1024);
         load_to_lds16<0, false>(Gp, goff, gdst + j * 1024);
     };
+    // (the same where the offsets are not kept; last: the step's last row that
+    // exists, which the rows behind it read)
+    auto fetch_piece_wide = [&](const QueryRows &at, int last, char *qdst_base, char *gdst_base,
+            auto piece) __attribute__((always_inline))
+    {
+        constexpr int j = decltype(piece)::value;
+        const char *Qp = static_cast<const char *>(at.Q) + at.elem * RB;
+        const char *Gp = static_cast<const char *>(at.dA) + at.elem * RB;
+        // (row wide_goff / RB + 4 * j of the step, or its last one: the offset is
+        // not negative, the load widens it as unsigned)
+        const uint32_t place = flip_bits<16 * j>(wide_goff);
+        const int past = max((int)(place / (uint32_t)RB) + (4 * j - last), 0);
+        const uint32_t goff = place + (uint32_t)((4 * j - past) * RB);
+        load_to_lds16<0, false>(Qp, goff, qdst_base + wave_u * LPW * 1024 + j * 1024);
+        load_to_lds16<0, false>(Gp, goff, gdst_base + wave_u * LPW * 1024 + j * 1024);
+    };
     // The statistics of a step in two halves, so that the load's latency
     // passes behind the MFMAs of the step before: stat_load starts the read
-    // of the thread's value (threads 0..63 a logsumexp, 64..127 a row dot),
+    // of the lane's value (wavefront 0 a logsumexp, wavefront 1 a row dot),
     // stat_store turns it into what the step reads from LDS.
     auto stat_load = [&](const QueryRows &at, int last) __attribute__((always_inline)) -> float
     {
         float raw = 0.0f;
-        if(tid < 2 * kBwdStep)
+        // (in the wide body without a branch: the other wavefronts read along)
+        if(WIDE || wave_u < 2)
         {
-            const int which = tid / kBwdStep, r = tid % kBwdStep;
-            const float *src = which == 0 ? at.lse + at.elem : p.D + at.d_idx;
-            raw = src[min(r, last)];
+            const float *src = wave_u % 2 == 0 ? at.lse + at.elem : p.D + at.d_idx;
+            raw = src[min(WIDE ? lane_index_again() : lane, last)];
         }
         return raw;
     };
     auto stat_store = [&](float raw, int last, float (*stat)[kBwdStep])
         __attribute__((always_inline))
     {
-        if(tid < 2 * kBwdStep)
+        if(wave_u < 2)
         {
-            const int which = tid / kBwdStep, r = tid % kBwdStep;
+            const int r = WIDE ? lane_index_again() : lane;
             float v;
-            if(which == 0)
+            if(wave_u == 0)
             {
                 v = (r > last || raw == neg_inf()) ? __builtin_huge_valf() : raw * kLog2e;
             }
@@ -1473,7 +1484,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
             {
                 v = r > last ? 0.0f : -raw;
             }
-            (&stat[0][0])[tid] = v;        // = stat[which][r]
+            stat[wave_u][r] = v;
         }
     };
     auto fetch_stat = [&](const QueryRows &at, int last, float (*stat)[kBwdStep])
@@ -1490,7 +1501,14 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
         const int row0 = qs * kBwdStep;
         const int last = min(kBwdStep, q_seq - row0) - 1;
         const QueryRows at = query_rows(bq, row0);
-        if(LOADERS == kDkvWaves || wave_u < LOADERS)
+        if constexpr(WIDE)
+        {
+            each_slot([&](auto j) __attribute__((always_inline))
+            {
+                fetch_piece_wide(at, last, qdst_base, gdst_base, j);
+            }, std::make_integer_sequence<int, LPW>{});
+        }
+        else if(LOADERS == kDkvWaves || wave_u < LOADERS)
         {
 #pragma unroll
             for(int j = 0; j < LPW; ++j)
@@ -1531,7 +1549,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
         // only add their offsets)
         const QueryRows at_f = query_rows(bq_f, row0_f);
         float raw_next = 0.0f;
-        if(i_next >= 0)
+        if(!WIDE && i_next >= 0)
         {
             raw_next = stat_load(at_f, last_f);
             if(NNTILE_BWD_SPREAD == 0 && (LOADERS == kDkvWaves || wave_u < LOADERS))
@@ -1569,134 +1587,166 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
             + (int64_t)q0 * (int64_t)mask_row_bytes;
         const uint32_t mask_last_row = (uint32_t)(rows_here - 1) * mask_row_bytes;
 
-        if constexpr(!use_mask && BOTH && HEAD > 64 && NNTILE_BWD_FUSED_ORDER == 1)
+        if constexpr(WIDE)
         {
             // Both gradients at head 128: 192 registers hold fragments and
-            // accumulators, so a block goes product by product - S, P, dV, then
-            // dP, dS, dK - and the probabilities in fp32 are all that crosses
-            // from the first half to the second.
-#pragma unroll
-            for(int mb = 0; mb < 2; ++mb)
+            // accumulators.  The step's two 32-query blocks go product by product,
+            // S, dP, dV, dK, eight MFMAs each: 64 slots of one MFMA, the operand
+            // read of the slot AHEAD later - across the products' borders, the
+            // matrix unit does not wait for LDS anywhere in the step but at its
+            // start - and a slice of the vector work: P beside dP, dS beside dV.
+            // Bound: the matrix pipe, 64 x 32 clocks a step and wavefront, at the
+            // clock that the board's power leaves it (32 heads of 128, 4096 tokens,
+            // causal, the whole call: 439 to 445 us with every MFMA behind its own
+            // operand read, 435 to 437 so, on two boxes; the same bits).
+            static_assert(!use_mask, "masks given as values at head 128: dK and dV apart");
+            constexpr int AHEAD = NNTILE_BWD_AHEAD_WIDE;
+            constexpr int SLOTS = 64;
+            enum { PART_S, PART_DP, PART_DV, PART_DK };
+            f32x16 sv, dpv;
+            uint32_t p_pk[8], ds_pk[8];
+            vec8 ring[AHEAD + 1];
+            f32x4 lse4;
+            auto read = [&](auto slot) __attribute__((always_inline))
             {
-                f32x16 sv;
-#pragma unroll
-                for(int r = 0; r < 16; ++r)
+                constexpr int g = decltype(slot)::value;
+                constexpr int mb = g / 32, part = g % 32 / 8, k = g % 8;
+                if constexpr(g >= SLOTS)
                 {
-                    sv[r] = 0.0f;
+                    return;
                 }
-#pragma unroll
-                for(int ks = 0; ks < KSTEPS; ++ks)
+                else if constexpr(part == PART_S || part == PART_DP)
                 {
-                    const vec8 qa = *reinterpret_cast<const vec8 *>(Qs + row_raddr[ks]
-                            + mb * 32 * RB);
-                    sv = T::mfma(qa, kf[ks], sv);
-                    if(LOADERS == kDkvWaves || wave_u < LOADERS)
-                    {
+                    ring[g % (AHEAD + 1)] = *reinterpret_cast<const vec8 *>(
+                            (part == PART_S ? Qs : Gs) + mb * 32 * RB
+                            + flip_bits<32 * k>(row_raddr[0]));
+                }
+                else
+                {
+                    constexpr int db = k / 2, t = 2 * mb + k % 2;
+                    const char *src = (part == PART_DV ? Gs : Qs) + (16 * t) * RB;
+                    const u32x2 lo = bwd_lds_read_tr16(src
+                            + flip_bits<64 * db>(tr_raddr[0][0]));
+                    const u32x2 hi = bwd_lds_read_tr16(src + 8 * RB
+                            + flip_bits<64 * db + 32>(tr_raddr[0][0]));
+                    const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
+                    ring[g % (AHEAD + 1)] = __builtin_bit_cast(vec8, raw);
+                }
+            };
+            auto mfma = [&](auto slot) __attribute__((always_inline))
+            {
+                constexpr int g = decltype(slot)::value;
+                constexpr int part = g % 32 / 8, k = g % 8;
+                const vec8 a = ring[g % (AHEAD + 1)];
+                if constexpr(part == PART_S)
+                {
+                    sv = T::mfma(a, kf[k], k == 0 ? f32x16{} : sv);
+                }
+                else if constexpr(part == PART_DP)
+                {
+                    dpv = T::mfma(a, vf[k], dpv);
+                }
+                else
+                {
+                    constexpr int db = k / 2, tt = k % 2;
+                    const uint32_t (&pk)[8] = part == PART_DV ? p_pk : ds_pk;
+                    const u32x4 braw = {pk[4 * tt], pk[4 * tt + 1], pk[4 * tt + 2], pk[4 * tt + 3]};
+                    f32x16 &to = part == PART_DV ? dv[db] : dk[db];
+                    to = T::mfma(a, __builtin_bit_cast(vec8, braw), to);
+                }
+            };
+            // the vector work beside slot g: the sixteen values of the product in
+            // front, from the second slot on (the first is its last MFMA's time)
+            auto vector_work = [&](auto slot) __attribute__((always_inline))
+            {
+                constexpr int g = decltype(slot)::value;
+                constexpr int mb = g / 32, part = g % 32 / 8, k = g % 8;
+                if constexpr(part == PART_S && k < 4)
+                {
+                    // (dP - D: the accumulator starts at -D of its row)
+                    const f32x4 nd4 = *reinterpret_cast<const f32x4 *>(
+                            &stat[1][mb * 32 + 8 * k + 4 * half]);
 #pragma unroll
-                        for(int j = 0; j < LPW; ++j)
+                    for(int e = 0; e < 4; ++e)
+                    {
+                        dpv[4 * k + e] = nd4[e];
+                    }
+                }
+                // (values FIRST[k] .. FIRST[k + 1] beside slot k; of the logsumexps
+                // four at a time have registers, read a slot ahead)
+                constexpr int FIRST[9] = {0, 0, 2, 4, 6, 8, 12, 14, 16};
+                if constexpr(part == PART_DP)
+                {
+#pragma unroll
+                    for(int r = FIRST[k]; r < FIRST[k + 1]; ++r)
+                    {
+                        sv[r] = fast_exp2(fmaf(sv[r], c, -lse4[r % 4]));
+                        if(r % 2 == 1)
                         {
-                            if(NNTILE_BWD_SPREAD != 0 && mb * KSTEPS + ks == 1 + j * FETCH_STRIDE)
-                            {
-                                fetch_piece(at_f, at_end_f, BUF ? lds_q0 : lds_q1,
-                                        BUF ? lds_g0 : lds_g1, j);
-                            }
+                            p_pk[r / 2] = T::pack2(sv[r - 1], sv[r]);
+                            asm volatile("" : "+v"(p_pk[r / 2]));
+                        }
+                    }
+                    if constexpr(FIRST[k + 1] % 4 == 0 && k < 7)
+                    {
+                        lse4 = *reinterpret_cast<const f32x4 *>(
+                                &stat[0][mb * 32 + 2 * FIRST[k + 1] + 4 * half]);
+                    }
+                }
+                if constexpr(part == PART_DV)
+                {
+#pragma unroll
+                    for(int r = FIRST[k]; r < FIRST[k + 1]; ++r)
+                    {
+                        dpv[r] = sv[r] * dpv[r];
+                        if(r % 2 == 1)
+                        {
+                            ds_pk[r / 2] = T::pack2(dpv[r - 1], dpv[r]);
+                            asm volatile("" : "+v"(ds_pk[r / 2]));
                         }
                     }
                 }
-                if(bounds)
+            };
+            each_slot(read, std::make_integer_sequence<int, AHEAD>{});
+            __builtin_amdgcn_sched_barrier(0);
+            each_slot([&](auto slot) __attribute__((always_inline))
+            {
+                constexpr int g = decltype(slot)::value;
+                if(g % 32 == 8 && bounds)
                 {
+                    // keys past the end and pairs the causal mask hides
+                    float hidden = neg_inf();
+                    asm volatile("" : "+v"(hidden));
 #pragma unroll
                     for(int r = 0; r < 16; ++r)
                     {
                         // (the lane's part on the left, the rest is wave-common)
-                        const int qr = mb * 32 + tile_row(r, 0);
+                        const int qr = g / 32 * 32 + tile_row(r, 0);
                         bool vis = k_ok;
-                        if(MODE == NNTILE_HIP_MASK_CAUSAL || EXPLICIT)
+                        if(MODE == NNTILE_HIP_MASK_CAUSAL)
                         {
                             vis = vis && (my_k_less_half <= vis_base + qr);
                         }
-                        sv[r] = vis ? sv[r] : neg_inf();
+                        sv[r] = vis ? sv[r] : hidden;
                     }
                 }
-                // P in place of S
-                uint32_t pk[8];
-#pragma unroll
-                for(int rg = 0; rg < 4; ++rg)
+                read(std::integral_constant<int, g + AHEAD>{});
+                mfma(slot);
+                vector_work(slot);
+                // the next step's rows early in the step, its statistics half way
+                if constexpr(g % 8 == 2 && g / 8 < LPW)
                 {
-                    const f32x4 lse4 = *reinterpret_cast<const f32x4 *>(
-                            &stat[0][mb * 32 + 8 * rg + 4 * half]);
-#pragma unroll
-                    for(int e = 0; e < 4; ++e)
-                    {
-                        sv[4 * rg + e] = fast_exp2(fmaf(sv[4 * rg + e], c, -lse4[e]));
-                    }
+                    fetch_piece_wide(at_f, last_f, BUF ? lds_q0 : lds_q1, BUF ? lds_g0 : lds_g1,
+                            std::integral_constant<int, g / 8>{});
                 }
-#pragma unroll
-                for(int k = 0; k < 8; ++k)
+                if constexpr(g == SLOTS / 2)
                 {
-                    pk[k] = T::pack2(sv[2 * k], sv[2 * k + 1]);
+                    raw_next = stat_load(at_f, last_f);
                 }
-                // dV^T += dA^T P
-#pragma unroll
-                for(int tt = 0; tt < 2; ++tt)
-                {
-                    const int t = 2 * mb + tt;
-                    const u32x4 praw = {pk[4 * tt], pk[4 * tt + 1], pk[4 * tt + 2], pk[4 * tt + 3]};
-                    const vec8 pb = __builtin_bit_cast(vec8, praw);
-#pragma unroll
-                    for(int db = 0; db < DBLOCKS; ++db)
-                    {
-                        const u32x2 glo = bwd_lds_read_tr16(Gs + tr_raddr[0][db] + (16 * t) * RB);
-                        const u32x2 ghi = bwd_lds_read_tr16(Gs + tr_raddr[1][db] + (16 * t) * RB);
-                        const u32x4 graw = {glo[0], glo[1], ghi[0], ghi[1]};
-                        dv[db] = T::mfma(__builtin_bit_cast(vec8, graw), pb, dv[db]);
-                    }
-                }
-                // dP - D
-                f32x16 dpv;
-#pragma unroll
-                for(int rg = 0; rg < 4; ++rg)
-                {
-                    const f32x4 nd4 = *reinterpret_cast<const f32x4 *>(
-                            &stat[1][mb * 32 + 8 * rg + 4 * half]);
-#pragma unroll
-                    for(int e = 0; e < 4; ++e)
-                    {
-                        dpv[4 * rg + e] = nd4[e];
-                    }
-                }
-#pragma unroll
-                for(int ks = 0; ks < KSTEPS; ++ks)
-                {
-                    const vec8 ga = *reinterpret_cast<const vec8 *>(Gs + row_raddr[ks]
-                            + mb * 32 * RB);
-                    dpv = T::mfma(ga, vf[ks], dpv);
-                }
-                // dS, in the registers of the packed P
-#pragma unroll
-                for(int k = 0; k < 8; ++k)
-                {
-                    pk[k] = T::pack2(sv[2 * k] * dpv[2 * k], sv[2 * k + 1] * dpv[2 * k + 1]);
-                }
-                // dK^T += Q^T dS
-#pragma unroll
-                for(int tt = 0; tt < 2; ++tt)
-                {
-                    const int t = 2 * mb + tt;
-                    const u32x4 sraw = {pk[4 * tt], pk[4 * tt + 1], pk[4 * tt + 2], pk[4 * tt + 3]};
-                    const vec8 sb = __builtin_bit_cast(vec8, sraw);
-#pragma unroll
-                    for(int db = 0; db < DBLOCKS; ++db)
-                    {
-                        const u32x2 qlo = bwd_lds_read_tr16(Qs + tr_raddr[0][db] + (16 * t) * RB);
-                        const u32x2 qhi = bwd_lds_read_tr16(Qs + tr_raddr[1][db] + (16 * t) * RB);
-                        const u32x4 qraw = {qlo[0], qlo[1], qhi[0], qhi[1]};
-                        dk[db] = T::mfma(__builtin_bit_cast(vec8, qraw), sb, dk[db]);
-                    }
-                }
-            }
+                __builtin_amdgcn_sched_barrier(0);
+            }, std::make_integer_sequence<int, SLOTS>{});
         }
-        else if constexpr(use_mask || NNTILE_BWD_PIPE == 0 || (BOTH && HEAD > 64))
+        else if constexpr(use_mask || NNTILE_BWD_PIPE == 0)
         {
             // (one 32-query block at a time: half the accumulators live)
             // ---- S = Q K^T, dP = dA V^T: rows are queries, the lane's column its key;
