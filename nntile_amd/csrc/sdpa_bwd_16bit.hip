@@ -88,7 +88,10 @@ namespace nntile_hip
 #define NNTILE_BWD_PIPE_DQ 1        // the same in the dQ workgroups
 #endif
 #ifndef NNTILE_BWD_AHEAD
-#define NNTILE_BWD_AHEAD 2          // LDS operands are read this many MFMAs early
+#define NNTILE_BWD_AHEAD 2          // LDS operands are read this many MFMAs early, head 128
+#endif
+#ifndef NNTILE_BWD_AHEAD_NARROW
+#define NNTILE_BWD_AHEAD_NARROW 4   // and at head 32 and 64, whose bodies have the registers
 #endif
 #ifndef NNTILE_BWD_AHEAD_WIDE
 #define NNTILE_BWD_AHEAD_WIDE 2     // the same where a workgroup holds both gradients at head 128
@@ -102,6 +105,7 @@ namespace nntile_hip
 constexpr int kBwdRows = 128;       // queries (dQ workgroups) / keys (dK, dV workgroups) per workgroup
 constexpr int kBwdStep = 64;        // rows of the other axis per step
 constexpr int kBwdThreads = 256;
+template<int HEAD> constexpr int kBwdAhead = HEAD > 64 ? NNTILE_BWD_AHEAD : NNTILE_BWD_AHEAD_NARROW;
 
 __device__ __forceinline__ u32x2 bwd_lds_read_tr16(const char *lds_ptr)
 {
@@ -961,47 +965,65 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
         {
             // The step's two 32-key blocks in three phases each - A: the two
             // score products, B: dS on the vector ALU, C: dQ^T += K^T dS^T -
-            // issued as A0 | A1 with B0 | C0 with B1 | C1 (see the dK / dV body).
+            // issued as A0 | A1 with B0 | C0 with B1 | C1 (see the dK / dV body):
+            // slots of one MFMA, the operand read of the slot AHEAD later (across
+            // the phases' borders too) and a slice of the vector work, with a
+            // scheduling barrier after each.
             f32x16 sv[2], dpv[2];
             uint32_t ds_pk[2][8];
             constexpr int A_MFMAS = 2 * KSTEPS, C_MFMAS = 2 * DBLOCKS;
-            constexpr int AHEAD = NNTILE_BWD_AHEAD;
-            auto a_init = [&](int mb) __attribute__((always_inline))
+            constexpr int SLOTS = 2 * (A_MFMAS + C_MFMAS);
+            constexpr int AHEAD = kBwdAhead<HEAD>;
+            vec8 ring[AHEAD + 1];
+            auto read = [&](auto slot) __attribute__((always_inline))
             {
-#pragma unroll
-                for(int r = 0; r < 16; ++r)
+                constexpr int g = decltype(slot)::value;
+                if constexpr(g < 2 * A_MFMAS)
                 {
-                    sv[mb][r] = 0.0f;
-                    dpv[mb][r] = 0.0f;
+                    constexpr int mb = g / A_MFMAS, i = g % A_MFMAS;
+                    ring[g % (AHEAD + 1)] = *reinterpret_cast<const vec8 *>(((i & 1) ? Vs : Ks)
+                            + row_raddr[i / 2] + mb * 32 * RB);
+                }
+                else if constexpr(g < SLOTS)
+                {
+                    constexpr int i = g - 2 * A_MFMAS, t = i / DBLOCKS, db = i % DBLOCKS;
+                    const u32x2 lo = bwd_lds_read_tr16(Ks + tr_raddr[0][db] + (16 * t) * RB);
+                    const u32x2 hi = bwd_lds_read_tr16(Ks + tr_raddr[1][db] + (16 * t) * RB);
+                    const u32x4 araw = {lo[0], lo[1], hi[0], hi[1]};
+                    ring[g % (AHEAD + 1)] = __builtin_bit_cast(vec8, araw);
                 }
             };
-            auto a_read = [&](int mb, int i, vec8 (&ring)[AHEAD + 1]) __attribute__((always_inline))
+            auto mfma = [&](auto slot) __attribute__((always_inline))
             {
-                if(i >= A_MFMAS)
+                constexpr int g = decltype(slot)::value;
+                const vec8 a = ring[g % (AHEAD + 1)];
+                if constexpr(g < 2 * A_MFMAS)
                 {
-                    return;
-                }
-                ring[i % (AHEAD + 1)] = *reinterpret_cast<const vec8 *>(((i & 1) ? Vs : Ks)
-                        + row_raddr[i / 2] + mb * 32 * RB);
-            };
-            auto a_mfma = [&](int mb, int i, vec8 (&ring)[AHEAD + 1]) __attribute__((always_inline))
-            {
-                const int ks = i / 2;
-                if(i & 1)
-                {
-                    dpv[mb] = T::mfma(ring[i % (AHEAD + 1)], gf[ks], dpv[mb]);
-#pragma unroll
-                    for(int j = 0; j < LOADS_PER_WAVE; ++j)
+                    constexpr int mb = g / A_MFMAS, i = g % A_MFMAS, ks = i / 2;
+                    if constexpr((i & 1) == 0)
                     {
-                        if(NNTILE_BWD_SPREAD != 0 && mb * KSTEPS + ks == 1 + j * FETCH_STRIDE)
+                        sv[mb] = T::mfma(a, qf[ks], ks == 0 ? f32x16{} : sv[mb]);
+                    }
+                    else
+                    {
+                        dpv[mb] = T::mfma(a, gf[ks], ks == 0 ? f32x16{} : dpv[mb]);
+#pragma unroll
+                        for(int j = 0; j < LOADS_PER_WAVE; ++j)
                         {
-                            fetch_piece(at_f, BUF ? lds_k0 : lds_k1, BUF ? lds_v0 : lds_v1, j);
+                            if(NNTILE_BWD_SPREAD != 0 && mb * KSTEPS + ks == 1 + j * FETCH_STRIDE)
+                            {
+                                fetch_piece(at_f, BUF ? lds_k0 : lds_k1, BUF ? lds_v0 : lds_v1, j);
+                            }
                         }
                     }
                 }
                 else
                 {
-                    sv[mb] = T::mfma(ring[i % (AHEAD + 1)], qf[ks], sv[mb]);
+                    constexpr int i = g - 2 * A_MFMAS, mb = i / C_MFMAS;
+                    constexpr int tt = i % C_MFMAS / DBLOCKS, db = i % DBLOCKS;
+                    const u32x4 braw = {ds_pk[mb][4 * tt], ds_pk[mb][4 * tt + 1],
+                        ds_pk[mb][4 * tt + 2], ds_pk[mb][4 * tt + 3]};
+                    acc[db] = T::mfma(a, __builtin_bit_cast(vec8, braw), acc[db]);
                 }
             };
             // Keys past the end and keys the causal mask hides: their scores
@@ -1036,95 +1058,40 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
                     asm volatile("" : "+v"(ds_pk[mb][r / 2]));
                 }
             };
-            // the block's two sub-steps of 16 keys
-            auto c_read = [&](int mb, int i, vec8 (&ring)[AHEAD + 1]) __attribute__((always_inline))
+            each_slot(read, std::make_integer_sequence<int, AHEAD>{});
+            __builtin_amdgcn_sched_barrier(0);
+            each_slot([&](auto slot) __attribute__((always_inline))
             {
-                if(i >= C_MFMAS)
+                constexpr int g = decltype(slot)::value;
+                constexpr int i1 = g - A_MFMAS, i2 = g - 2 * A_MFMAS;
+                if constexpr(i1 == 0)
                 {
-                    return;
+                    hide(0);
                 }
-                const int t = 2 * mb + i / DBLOCKS, db = i % DBLOCKS;
-                const u32x2 lo = bwd_lds_read_tr16(Ks + tr_raddr[0][db] + (16 * t) * RB);
-                const u32x2 hi = bwd_lds_read_tr16(Ks + tr_raddr[1][db] + (16 * t) * RB);
-                const u32x4 araw = {lo[0], lo[1], hi[0], hi[1]};
-                ring[i % (AHEAD + 1)] = __builtin_bit_cast(vec8, araw);
-            };
-            auto c_mfma = [&](int mb, int i, vec8 (&ring)[AHEAD + 1]) __attribute__((always_inline))
-            {
-                const int tt = i / DBLOCKS, db = i % DBLOCKS;
-                const u32x4 braw = {ds_pk[mb][4 * tt], ds_pk[mb][4 * tt + 1], ds_pk[mb][4 * tt + 2],
-                    ds_pk[mb][4 * tt + 3]};
-                acc[db] = T::mfma(ring[i % (AHEAD + 1)], __builtin_bit_cast(vec8, braw), acc[db]);
-            };
-            {
-                vec8 ring[AHEAD + 1];
-                a_init(0);
-#pragma unroll
-                for(int i = 0; i < AHEAD; ++i)
+                if constexpr(i2 == 0)
                 {
-                    a_read(0, i, ring);
+                    hide(1);
                 }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for(int i = 0; i < A_MFMAS; ++i)
+                read(std::integral_constant<int, g + AHEAD>{});
+                mfma(slot);
+                if constexpr(i1 >= 0 && i1 < A_MFMAS)
                 {
-                    a_read(0, i + AHEAD, ring);
-                    a_mfma(0, i, ring);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                hide(0);
-                a_init(1);
 #pragma unroll
-                for(int i = 0; i < AHEAD; ++i)
-                {
-                    a_read(1, i, ring);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for(int i = 0; i < A_MFMAS; ++i)
-                {
-                    a_read(1, i + AHEAD, ring);
-                    a_mfma(1, i, ring);
-#pragma unroll
-                    for(int r = i * 16 / A_MFMAS; r < (i + 1) * 16 / A_MFMAS; ++r)
+                    for(int r = i1 * 16 / A_MFMAS; r < (i1 + 1) * 16 / A_MFMAS; ++r)
                     {
                         b_item(0, r);
                     }
-                    __builtin_amdgcn_sched_barrier(0);
                 }
-                hide(1);
-#pragma unroll
-                for(int i = 0; i < AHEAD; ++i)
+                if constexpr(i2 >= 0 && i2 < C_MFMAS)
                 {
-                    c_read(0, i, ring);
-                }
-                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for(int i = 0; i < C_MFMAS; ++i)
-                {
-                    c_read(0, i + AHEAD, ring);
-                    c_mfma(0, i, ring);
-#pragma unroll
-                    for(int r = i * 16 / C_MFMAS; r < (i + 1) * 16 / C_MFMAS; ++r)
+                    for(int r = i2 * 16 / C_MFMAS; r < (i2 + 1) * 16 / C_MFMAS; ++r)
                     {
                         b_item(1, r);
                     }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-#pragma unroll
-                for(int i = 0; i < AHEAD; ++i)
-                {
-                    c_read(1, i, ring);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for(int i = 0; i < C_MFMAS; ++i)
-                {
-                    c_read(1, i + AHEAD, ring);
-                    c_mfma(1, i, ring);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
+            }, std::make_integer_sequence<int, SLOTS>{});
         }
     };
     auto run = [&](int g, int g_next, auto buf_tag) __attribute__((always_inline))
@@ -1934,55 +1901,81 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                 }
             };
             // The overlapped order, written out slot by slot (one MFMA, the operand
-            // read of a later slot, a slice of the vector work) with a scheduling
-            // barrier after each, or the compiler regroups it into phases.
+            // read of the slot AHEAD later - of the next phase too -, a slice of the
+            // vector work) with a scheduling barrier after each, or the compiler
+            // regroups it into phases.
             constexpr int A_MFMAS = (DO_DK ? 2 : 1) * KSTEPS, C_MFMAS = (BOTH ? 2 : 1) * 2 * DBLOCKS;
-            constexpr int AHEAD = NNTILE_BWD_AHEAD;
-            auto a_read = [&](int mb, int i, vec8 (&ring)[AHEAD + 1]) __attribute__((always_inline))
+            constexpr int SLOTS = 2 * (A_MFMAS + C_MFMAS);
+            constexpr int AHEAD = kBwdAhead<HEAD>;
+            vec8 ring[AHEAD + 1];
+            auto read = [&](auto slot) __attribute__((always_inline))
             {
-                if(i >= A_MFMAS)
+                constexpr int g = decltype(slot)::value;
+                if constexpr(g < 2 * A_MFMAS)
                 {
-                    return;
+                    constexpr int mb = g / A_MFMAS, i = g % A_MFMAS, ks = DO_DK ? i / 2 : i;
+                    const char *src = (DO_DK && (i & 1)) ? Gs : Qs;
+                    ring[g % (AHEAD + 1)] = *reinterpret_cast<const vec8 *>(src + row_raddr[ks]
+                            + mb * 32 * RB);
                 }
-                const int ks = DO_DK ? i / 2 : i;
-                const char *src = (DO_DK && (i & 1)) ? Gs : Qs;
-                ring[i % (AHEAD + 1)] = *reinterpret_cast<const vec8 *>(src + row_raddr[ks]
-                        + mb * 32 * RB);
-            };
-            auto a_mfma = [&](int mb, int i, vec8 (&ring)[AHEAD + 1]) __attribute__((always_inline))
-            {
-                const int ks = DO_DK ? i / 2 : i;
-                if(DO_DK && (i & 1))
+                else if constexpr(g < SLOTS)
                 {
-                    dpv[mb] = T::mfma(ring[i % (AHEAD + 1)], vf[ks], dpv[mb]);
+                    // (both gradients: dV and dK products alternate)
+                    constexpr int i = (g - 2 * A_MFMAS) % C_MFMAS, mb = (g - 2 * A_MFMAS) / C_MFMAS;
+                    constexpr int j = BOTH ? i / 2 : i;
+                    constexpr bool for_dv = BOTH ? (i & 1) == 0 : DO_DV;
+                    constexpr int t = 2 * mb + j / DBLOCKS, db = j % DBLOCKS;
+                    const char *src = (for_dv ? Gs : Qs) + (16 * t) * RB;
+                    const u32x2 lo = bwd_lds_read_tr16(src + tr_raddr[0][db]);
+                    const u32x2 hi = bwd_lds_read_tr16(src + tr_raddr[1][db]);
+                    const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
+                    ring[g % (AHEAD + 1)] = __builtin_bit_cast(vec8, raw);
+                }
+            };
+            auto mfma = [&](auto slot) __attribute__((always_inline))
+            {
+                constexpr int g = decltype(slot)::value;
+                const vec8 a = ring[g % (AHEAD + 1)];
+                if constexpr(g < 2 * A_MFMAS)
+                {
+                    constexpr int mb = g / A_MFMAS, i = g % A_MFMAS, ks = DO_DK ? i / 2 : i;
+                    if constexpr(DO_DK && (i & 1))
+                    {
+                        dpv[mb] = T::mfma(a, vf[ks], dpv[mb]);
+                    }
+                    else
+                    {
+                        sv[mb] = T::mfma(a, kf[ks], ks == 0 ? f32x16{} : sv[mb]);
+                    }
+                    // the tile loads of the next step, spread over the products
+                    if((LOADERS == kDkvWaves || wave_u < LOADERS) && NNTILE_BWD_SPREAD != 0
+                            && (!DO_DK || (i & 1)))
+                    {
+#pragma unroll
+                        for(int j = 0; j < LPW; ++j)
+                        {
+                            if(mb * KSTEPS + ks == 1 + j * FETCH_STRIDE)
+                            {
+                                fetch_piece(at_f, at_end_f, BUF ? lds_q0 : lds_q1,
+                                        BUF ? lds_g0 : lds_g1, j);
+                            }
+                        }
+                    }
                 }
                 else
                 {
-                    sv[mb] = T::mfma(ring[i % (AHEAD + 1)], kf[ks], sv[mb]);
-                }
-                // the tile loads of the next step, spread over the products
-                if((LOADERS == kDkvWaves || wave_u < LOADERS) && NNTILE_BWD_SPREAD != 0
-                        && (!DO_DK || (i & 1)))
-                {
-#pragma unroll
-                    for(int j = 0; j < LPW; ++j)
-                    {
-                        if(mb * KSTEPS + ks == 1 + j * FETCH_STRIDE)
-                        {
-                            fetch_piece(at_f, at_end_f, BUF ? lds_q0 : lds_q1,
-                                    BUF ? lds_g0 : lds_g1, j);
-                        }
-                    }
+                    constexpr int i = (g - 2 * A_MFMAS) % C_MFMAS, mb = (g - 2 * A_MFMAS) / C_MFMAS;
+                    constexpr int j = BOTH ? i / 2 : i;
+                    constexpr bool for_dv = BOTH ? (i & 1) == 0 : DO_DV;
+                    constexpr int tt = j / DBLOCKS, db = j % DBLOCKS;
+                    const uint32_t (&pk)[8] = for_dv ? p_pk[mb] : ds_pk[mb];
+                    const u32x4 braw = {pk[4 * tt], pk[4 * tt + 1], pk[4 * tt + 2], pk[4 * tt + 3]};
+                    f32x16 &to = for_dv ? dv[db] : dk[db];
+                    to = T::mfma(a, __builtin_bit_cast(vec8, braw), to);
                 }
             };
             auto a_init = [&](int mb) __attribute__((always_inline))
             {
-#pragma unroll
-                for(int r = 0; r < 16; ++r)
-                {
-                    sv[mb][r] = 0.0f;
-                    dpv[mb][r] = 0.0f;
-                }
                 if(DO_DK)
                 {
 #pragma unroll
@@ -1996,38 +1989,6 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                             dpv[mb][4 * rg + e] = nd4[e];
                         }
                     }
-                }
-            };
-            auto c_read = [&](int mb, int i, vec8 (&ring)[AHEAD + 1]) __attribute__((always_inline))
-            {
-                if(i >= C_MFMAS)
-                {
-                    return;
-                }
-                // (both gradients: dV and dK products alternate)
-                const int j = BOTH ? i / 2 : i;
-                const bool for_dv = BOTH ? (i & 1) == 0 : DO_DV;
-                const int t = 2 * mb + j / DBLOCKS, db = j % DBLOCKS;
-                const char *src = (for_dv ? Gs : Qs) + (16 * t) * RB;
-                const u32x2 lo = bwd_lds_read_tr16(src + tr_raddr[0][db]);
-                const u32x2 hi = bwd_lds_read_tr16(src + tr_raddr[1][db]);
-                const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
-                ring[i % (AHEAD + 1)] = __builtin_bit_cast(vec8, raw);
-            };
-            auto c_mfma = [&](int mb, int i, vec8 (&ring)[AHEAD + 1]) __attribute__((always_inline))
-            {
-                const int j = BOTH ? i / 2 : i;
-                const bool for_dv = BOTH ? (i & 1) == 0 : DO_DV;
-                const int tt = j / DBLOCKS, db = j % DBLOCKS;
-                const uint32_t (&pk)[8] = for_dv ? p_pk[mb] : ds_pk[mb];
-                const u32x4 braw = {pk[4 * tt], pk[4 * tt + 1], pk[4 * tt + 2], pk[4 * tt + 3]};
-                if(for_dv)
-                {
-                    dv[db] = T::mfma(ring[i % (AHEAD + 1)], __builtin_bit_cast(vec8, braw), dv[db]);
-                }
-                else
-                {
-                    dk[db] = T::mfma(ring[i % (AHEAD + 1)], __builtin_bit_cast(vec8, braw), dk[db]);
                 }
             };
             // vector work of query r of block mb (statistics of four queries per
@@ -2089,84 +2050,55 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                 }
             };
             constexpr int B_TICKS = 18;
+            a_init(0);
+            each_slot(read, std::make_integer_sequence<int, AHEAD>{});
+            __builtin_amdgcn_sched_barrier(0);
+            each_slot([&](auto slot) __attribute__((always_inline))
             {
-                vec8 ring[AHEAD + 1];
-                // A0
-                a_init(0);
-#pragma unroll
-                for(int i = 0; i < AHEAD; ++i)
+                constexpr int g = decltype(slot)::value;
+                constexpr int i1 = g - A_MFMAS, i2 = g - 2 * A_MFMAS;
+                // (the second block's start and the first's statistics ahead of the
+                // phase that needs them)
+                if constexpr(g == A_MFMAS - 1)
                 {
-                    a_read(0, i, ring);
+                    a_init(1);
+                    b_begin(0);
                 }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for(int i = 0; i < A_MFMAS; ++i)
+                if constexpr(i1 == 0)
                 {
-                    a_read(0, i + AHEAD, ring);
-                    a_mfma(0, i, ring);
-                    __builtin_amdgcn_sched_barrier(0);
+                    BWD_TRACE_MARK(1);
+                    hide(0);
                 }
-                BWD_TRACE_MARK(1);
-                hide(0);
-                // A1 with B0
-                a_init(1);
-                b_begin(0);
-#pragma unroll
-                for(int i = 0; i < AHEAD; ++i)
+                if constexpr(i2 == 0)
                 {
-                    a_read(1, i, ring);
+                    BWD_TRACE_MARK(2);
+                    hide(1);
+                    b_begin(1);
                 }
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for(int i = 0; i < A_MFMAS; ++i)
+                if constexpr(i2 == C_MFMAS)
                 {
-                    a_read(1, i + AHEAD, ring);
-                    a_mfma(1, i, ring);
+                    BWD_TRACE_MARK(3);
+                }
+                read(std::integral_constant<int, g + AHEAD>{});
+                mfma(slot);
+                if constexpr(i1 >= 0 && i1 < A_MFMAS)
+                {
 #pragma unroll
-                    for(int t = i * B_TICKS / A_MFMAS; t < (i + 1) * B_TICKS / A_MFMAS; ++t)
+                    for(int t = i1 * B_TICKS / A_MFMAS; t < (i1 + 1) * B_TICKS / A_MFMAS; ++t)
                     {
                         b_tick(0, t);
                     }
-                    __builtin_amdgcn_sched_barrier(0);
                 }
-                BWD_TRACE_MARK(2);
-                hide(1);
-                // C0 with B1
-                b_begin(1);
-#pragma unroll
-                for(int i = 0; i < AHEAD; ++i)
+                if constexpr(i2 >= 0 && i2 < C_MFMAS)
                 {
-                    c_read(0, i, ring);
-                }
-                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for(int i = 0; i < C_MFMAS; ++i)
-                {
-                    c_read(0, i + AHEAD, ring);
-                    c_mfma(0, i, ring);
-#pragma unroll
-                    for(int t = i * B_TICKS / C_MFMAS; t < (i + 1) * B_TICKS / C_MFMAS; ++t)
+                    for(int t = i2 * B_TICKS / C_MFMAS; t < (i2 + 1) * B_TICKS / C_MFMAS; ++t)
                     {
                         b_tick(1, t);
                     }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                BWD_TRACE_MARK(3);
-                // C1
-#pragma unroll
-                for(int i = 0; i < AHEAD; ++i)
-                {
-                    c_read(1, i, ring);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for(int i = 0; i < C_MFMAS; ++i)
-                {
-                    c_read(1, i + AHEAD, ring);
-                    c_mfma(1, i, ring);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
+            }, std::make_integer_sequence<int, SLOTS>{});
         }
         BWD_TRACE_MARK(4);
         // (the other buffer's readers passed this step's barrier; the next
