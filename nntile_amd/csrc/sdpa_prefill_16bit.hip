@@ -104,6 +104,20 @@ __device__ __forceinline__ void mask_scan_range(const char *mask, uint32_t ld_by
             open_word, hidden_word, words, not_open, not_hidden);
 }
 
+// What a scan found about one (block, key range), as kMaskBitWords words: half of
+// one of its two words below, the call's tag above, by one thread each.
+__device__ __forceinline__ void mask_words_publish(unsigned long long *entry, int tid,
+        unsigned long long not_open, unsigned long long not_hidden, unsigned long long tag)
+{
+    if(tid < kMaskBitWords)
+    {
+        const unsigned long long w = (tid & 2) ? not_hidden : not_open;
+        const unsigned long long half = (tid & 1) ? w >> 32 : w & 0xffffffffull;
+        __hip_atomic_store(entry + tid, (tag << 32) | half, __ATOMIC_RELAXED,
+                __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
 // PARTS: the workgroup takes one of p.n_parts ranges of the keys and leaves
 // its triple in memory (PrefillParams::part_o), where launch_parts_merge finds it.
 template<typename T, int HEAD, int MODE, int WAVES = 4, int GROUPS = 1, bool PARTS = false>
@@ -192,18 +206,10 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                         (MODE == NNTILE_HIP_MASK_ADDITIVE) ? T::kNegInfPair : 0u,
                         (int)blockIdx.x / kMaskBitSplits, (int)blockIdx.x % kMaskBitSplits,
                         pub_words, pub_open, pub_hidden);
-                if(tid == 0)
-                {
-                    // written through to memory (device scope), acknowledged,
-                    // then the flag: readers on any XCD find the words
-                    unsigned long long *e = p.mask_bits + 3 * (int64_t)blockIdx.x;
-                    __hip_atomic_store(e, pub_open, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(e + 1, pub_hidden, __ATOMIC_RELAXED,
-                            __HIP_MEMORY_SCOPE_AGENT);
-                    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                    __hip_atomic_store(e + 2, p.mask_tag, __ATOMIC_RELAXED,
-                            __HIP_MEMORY_SCOPE_AGENT);
-                }
+                // written through to memory (device scope), where readers on any
+                // XCD find them; every word carries the tag, so none waits for another
+                mask_words_publish(p.mask_bits + kMaskBitWords * (int64_t)blockIdx.x, tid, pub_open,
+                        pub_hidden, p.mask_tag);
                 return;
             }
             wg -= (unsigned)p.n_scan_wgs;
@@ -704,37 +710,42 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         if(n_steps > 0 && p.mask_bits != nullptr && p.n_scan_wgs == 0)
         {
             // the scan was done once for all batch entries before the launch
-            const unsigned long long *w = p.mask_bits + (int64_t)qb * (3 * kMaskBitSplits);
+            const unsigned long long *w = p.mask_bits + (int64_t)qb * (kMaskBitWords * kMaskBitSplits);
 #pragma unroll
             for(int sp = 0; sp < kMaskBitSplits; ++sp)
             {
-                not_open |= w[3 * sp];
-                not_hidden |= w[3 * sp + 1];
+                const unsigned long long *e = w + kMaskBitWords * sp;
+                not_open |= (e[0] & 0xffffffffull) | (e[1] << 32);
+                not_hidden |= (e[2] & 0xffffffffull) | (e[3] << 32);
             }
             scanned = true;
         }
         else if(n_steps > 0 && p.mask_bits != nullptr)
         {
             // ... or is being done by the first workgroups of this launch: one
-            // thread per key range waits for that range's flag (bounded; the
+            // thread per word of the block's key ranges waits for it (bounded; the
             // Q fragments are on their way meanwhile), then everybody ORs
-            __shared__ unsigned long long got_bits[2];
+            static_assert(kMaskBitWords * kMaskBitSplits <= 64, "one wavefront reads them all");
+            __shared__ uint32_t got_bits[kMaskBitWords];
             __shared__ int got_all;
+            if(tid < kMaskBitWords)
+            {
+                got_bits[tid] = 0u;
+            }
             if(tid == 0)
             {
-                got_bits[0] = 0ull;
-                got_bits[1] = 0ull;
                 got_all = 1;
             }
             __syncthreads();
-            if(tid < kMaskBitSplits)
+            if(tid < kMaskBitWords * kMaskBitSplits)
             {
                 unsigned long long *e = p.mask_bits
-                    + 3 * ((int64_t)qb * kMaskBitSplits + tid);
+                    + (int64_t)qb * (kMaskBitWords * kMaskBitSplits) + tid;
                 const unsigned long long t0 = wall_clock64();
+                unsigned long long word;
                 bool ok = true;
-                while(__hip_atomic_load(e + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                        != p.mask_tag)
+                while(((word = __hip_atomic_load(e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                            >> 32) != (p.mask_tag & 0xffffffffull))
                 {
                     __builtin_amdgcn_s_sleep(2);
                     if(wall_clock64() - t0 > p.mask_spin_limit)
@@ -745,10 +756,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 }
                 if(ok)
                 {
-                    atomicOr(&got_bits[0], __hip_atomic_load(e, __ATOMIC_RELAXED,
-                                __HIP_MEMORY_SCOPE_AGENT));
-                    atomicOr(&got_bits[1], __hip_atomic_load(e + 1, __ATOMIC_RELAXED,
-                                __HIP_MEMORY_SCOPE_AGENT));
+                    atomicOr(&got_bits[tid % kMaskBitWords], (uint32_t)word);
                 }
                 else
                 {
@@ -758,8 +766,10 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             __syncthreads();
             if(got_all)
             {
-                not_open = got_bits[0];
-                not_hidden = got_bits[1];
+                not_open = (unsigned long long)got_bits[0]
+                    | ((unsigned long long)got_bits[1] << 32);
+                not_hidden = (unsigned long long)got_bits[2]
+                    | ((unsigned long long)got_bits[3] << 32);
                 scanned = true;
             }
         }
@@ -1731,9 +1741,8 @@ static int launch_mode(hipStream_t stream, const PrefillParams &p, int mode,
 // The scan of an explicit mask that every workgroup of the attention kernel
 // would do for its own 128 rows, done once for all batch entries, as a launch
 // of its own (calls under stream capture; otherwise the scan rides in the
-// attention launch): workgroup (query block, key range) writes its two words
-// to entry blockIdx.x of the table (three words an entry, the third unused
-// here; see PrefillParams::mask_bits).
+// attention launch): workgroup (query block, key range) writes what it finds
+// to entry blockIdx.x of the table (see PrefillParams::mask_bits), without a tag.
 template<int ES>
 __global__ __launch_bounds__(kThreads)
 void mask_step_bits_kernel(const char *mask, uint32_t ld_bytes, int q_len, int k_seq,
@@ -1744,11 +1753,8 @@ void mask_step_bits_kernel(const char *mask, uint32_t ld_bytes, int q_len, int k
     mask_scan_range<ES, kThreads / 64>(mask, ld_bytes, q_len, k_seq, open_word, hidden_word,
             (int)blockIdx.x / kMaskBitSplits, (int)blockIdx.x % kMaskBitSplits, words, not_open,
             not_hidden);
-    if(threadIdx.x == 0)
-    {
-        table[3 * (int64_t)blockIdx.x] = not_open;
-        table[3 * (int64_t)blockIdx.x + 1] = not_hidden;
-    }
+    mask_words_publish(table + kMaskBitWords * (int64_t)blockIdx.x, (int)threadIdx.x, not_open,
+            not_hidden, 0ull);
 }
 
 // Masks below this size are scanned by the attention kernel's workgroups
@@ -1757,18 +1763,19 @@ void mask_step_bits_kernel(const char *mask, uint32_t ld_bytes, int q_len, int k
 // as much (7 x 355^2: 0.5 % slower shared, 10 x 621^2: 12 % faster).
 constexpr int64_t kMaskScanBytes = 3 << 17;
 
-// A value no earlier call of this process has used and that memory left
-// behind by anything else is unlikely to hold (never 0).
+// A value that none of the last 2^32 calls of this process has used and that
+// memory left behind by anything else is unlikely to hold in the upper halves of
+// all words of a block's ranges (32 words; never 0).
 static unsigned long long next_scan_tag()
 {
-    static const unsigned long long salt = []
+    static const uint32_t salt = []
     {
         std::random_device rd;
-        return ((unsigned long long)rd() << 32) | 0x40000000ull;
+        return (uint32_t)rd();
     }();
-    static std::atomic<unsigned long long> counter{0};
-    const unsigned long long tag = salt + counter.fetch_add(1, std::memory_order_relaxed) + 1ull;
-    return tag == 0ull ? 1ull : tag;
+    static std::atomic<uint32_t> counter{0};
+    const uint32_t tag = salt + counter.fetch_add(1, std::memory_order_relaxed);
+    return tag == 0u ? next_scan_tag() : tag;
 }
 
 // One-tile calls with an explicit mask and a scratch buffer of the caller's
@@ -1791,7 +1798,8 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
     }
     const int64_t es = additive ? 2 : 1;
     const int64_t row_bytes = p.k_seq * es;
-    const int64_t table_bytes = (int64_t)p.q_blocks_per_tile * kMaskBitSplits * 24;
+    const int64_t table_bytes = (int64_t)p.q_blocks_per_tile * kMaskBitSplits
+        * (kMaskBitWords * (int64_t)sizeof(unsigned long long));
     if(row_bytes < 16 || p.mask_ld * es * kQRows >= (int64_t)(1 << 30)
             || reinterpret_cast<uintptr_t>(scratch) % 8 != 0
             || (int64_t)scratch_bytes < table_bytes
