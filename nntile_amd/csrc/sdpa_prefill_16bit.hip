@@ -507,16 +507,21 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     const float inv_scale = 1.0f / p.scale;
 
     // ---- explicit mask tiles ----------------------------------------------------
-    // The lane's 32 mask values of a key step (query my_q, keys
-    // mb*32 + 8*rg + 4*half + 0..3) are 8 groups of 4 consecutive elements:
-    // one 8-byte (additive) or 4-byte (boolean) load per group, issued one
-    // step ahead.  At the top of a step the wavefront classifies its 32 x 64
-    // block from the raw bits: nothing hidden (the step runs as if there were
-    // no mask), everything hidden (the step is skipped), or mixed (the values
-    // are applied).  The loads carry the alignment of one element; in a ragged
-    // last step a group that would reach past the row is moved back to end
-    // with it and shifted into place when it is used, and what lies past the
-    // end is made hidden.
+    // The wavefront's 32 x 64 mask values of a key step are loaded one step ahead
+    // as whole pieces of rows: load i brings rows 16*(i%2) + lane/4 and keys
+    // 32*(i/2) + 8*(lane%4) .. +7, 16 bytes a lane (boolean: 8).  At the top of the
+    // step the wavefront classifies its block from the raw bits: nothing hidden
+    // (the step runs as if there were no mask), everything hidden (the step is
+    // skipped), or mixed.  Mixed values go through LDS, 32 keys at a time, to the
+    // lanes that apply them: lane (col, half) has query my_q and keys
+    // mb*32 + 8*rg + 4*half + 0..3.  (Loaded from there directly - eight loads whose
+    // lanes lie in 32 rows each - a step took 1.0 to 1.3 us longer: the
+    // address path takes a lane a clock when neighbours share no line.  1024 x 1024
+    // x 32 of head 128: a window of 65 keys 20.7 -> 16.9 us, causal 26.3 -> 24.4,
+    // every step mixed 53.5 -> 38.9.)
+    // The loads carry the alignment of one element; in a ragged last step a piece
+    // that would reach past the row is moved back to end with it and shifted into
+    // place when it is used, and what lies past the end is made hidden.
     constexpr int MW = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 16 : 8;    // dwords per lane and step
     enum { MASK_ZERO = 0, MASK_HIDDEN = 1, MASK_MIXED = 2 };
     uint32_t mraw[MW];
@@ -525,92 +530,146 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     {
         mraw[i] = 0;
     }
-    const int64_t mask_row = (int64_t)(q_ok ? my_q : 0) * p.mask_ld;
-    // start of group i (keys key0 .. +3 of a step of `keys` keys) as loaded
-    auto group_key0 = [&](int i) -> int
+    constexpr int PW = MW / 4;                  // dwords of a piece of eight elements
+    constexpr int MASK_RB = 32 * 8 * PW / 16;   // bytes of 32 elements
+    constexpr int MASK_RPL = 256 / MASK_RB;     // such rows per 256-byte line of LDS banks
+    const int piece = lane & 3, piece_row = lane >> 2;
+    // first key of load i's piece within the step, as loaded and as meant
+    auto piece_key0 = [&](int i) -> int
     {
-        return (i >> 2) * 32 + (i & 3) * 8 + 4 * half;
+        return (i >> 1) * 32 + 8 * piece;
     };
-    auto group_start = [&](int key0, int keys) -> int
+    auto piece_start = [&](int key0, int keys) -> int
     {
-        return min(key0, keys == k_seq ? max(keys - 4, 0) : keys - 4);
+        // (a row of less than a piece is loaded from its start)
+        return max(min(key0, keys - 8), keys == k_seq ? 0 : -kKeys);
     };
     // loads of the mask values of key step kb (of `keys` keys) into mraw
     auto mask_fetch = [&](int kb, int keys)
     {
         typedef typename std::conditional<MODE == NNTILE_HIP_MASK_ADDITIVE, uint16_t,
                 uint8_t>::type M;
-        const M *mp = static_cast<const M *>(p.mask) + mask_row + kb * kKeys;
-        auto load_group = [&](int i, int at) __attribute__((always_inline))
-        {
-            if constexpr(MODE == NNTILE_HIP_MASK_ADDITIVE)
-            {
-                typedef u32x2 __attribute__((aligned(2))) u32x2_any;
-                const u32x2 v = *reinterpret_cast<const u32x2_any *>(mp + at);
-                mraw[2 * i] = v[0];
-                mraw[2 * i + 1] = v[1];
-            }
-            else
-            {
-                typedef uint32_t __attribute__((aligned(1))) u32_any;
-                mraw[i] = *reinterpret_cast<const u32_any *>(mp + at);
-            }
-        };
-        if(keys >= kKeys)
-        {
-            mp += 4 * half;
+        typedef typename std::conditional<MODE == NNTILE_HIP_MASK_ADDITIVE, u32x4, u32x2>::type V;
+        typedef V __attribute__((aligned(1))) V_any;
+        const M *mp[2];
 #pragma unroll
-            for(int i = 0; i < 8; ++i)
-            {
-                load_group(i, (i >> 2) * 32 + (i & 3) * 8);
-            }
+        for(int h = 0; h < 2; ++h)
+        {
+            // (rows past the end of the tile re-read its last one)
+            const int row = min(q_row0 + wave * 32 + 16 * h + piece_row, q_len - 1);
+            mp[h] = static_cast<const M *>(p.mask) + (int64_t)row * p.mask_ld + kb * kKeys;
         }
-        else if(k_seq >= 4)
+        if(k_seq >= 8)
         {
 #pragma unroll
-            for(int i = 0; i < 8; ++i)
+            for(int i = 0; i < 4; ++i)
             {
-                load_group(i, group_start(group_key0(i), keys));
+                const int at = keys >= kKeys ? piece_key0(i) : piece_start(piece_key0(i), keys);
+                const V v = *reinterpret_cast<const V_any *>(mp[i & 1] + at);
+#pragma unroll
+                for(int w = 0; w < PW; ++w)
+                {
+                    mraw[PW * i + w] = v[w];
+                }
             }
         }
         else
         {
-            // (rows of less than one group)
-            const uint32_t e0 = mp[0], e1 = mp[min(1, k_seq - 1)], e2 = mp[k_seq - 1];
-            if constexpr(MODE == NNTILE_HIP_MASK_ADDITIVE)
+            // (rows of less than one piece)
+#pragma unroll
+            for(int i = 0; i < 2; ++i)
             {
-                mraw[0] = e0 | (e1 << 16);
-                mraw[1] = e2;
-            }
-            else
-            {
-                mraw[0] = e0 | (e1 << 8) | (e2 << 16);
+#pragma unroll
+                for(int w = 0; w < PW; ++w)
+                {
+                    constexpr int EPW = 8 / PW;
+                    uint32_t x = 0u;
+#pragma unroll
+                    for(int e = 0; e < EPW; ++e)
+                    {
+                        x |= (uint32_t)mp[i][min(EPW * w + e, k_seq - 1)] << (32 / EPW * e);
+                    }
+                    mraw[PW * i + w] = x;
+                }
             }
         }
     };
-    // brings the groups of a ragged step of `keys` keys into place
+    // brings the pieces of a ragged step of `keys` keys into place
     auto mask_fix_ragged = [&](int keys)
     {
+        constexpr int EB = 32 * PW / 8;         // bits of an element
+        constexpr uint32_t HIDDEN = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? T::kNegInfPair : 0u;
 #pragma unroll
-        for(int i = 0; i < 8; ++i)
+        for(int i = 0; i < 4; ++i)
         {
-            const int key0 = group_key0(i);
-            const int back = min(key0 - group_start(key0, keys), 4);
-            const int valid = min(max(keys - key0, 0), 4);
-            if constexpr(MODE == NNTILE_HIP_MASK_ADDITIVE)
+            const int key0 = piece_key0(i);
+            const int back = key0 - piece_start(key0, keys);
+            const int valid = min(max(keys - key0, 0), 8);
+#pragma unroll
+            for(int w = 0; w < PW; ++w)
             {
-                const uint64_t raw = (uint64_t)mraw[2 * i] | ((uint64_t)mraw[2 * i + 1] << 32);
-                const uint64_t hidden = ((uint64_t)T::kNegInfPair << 32) | T::kNegInfPair;
-                const uint64_t keep = valid == 4 ? ~0ull : (1ull << (16 * valid)) - 1ull;
-                const uint64_t v = ((raw >> (16 * (back & 3))) & keep) | (hidden & ~keep);
-                mraw[2 * i] = (uint32_t)v;
-                mraw[2 * i + 1] = (uint32_t)(v >> 32);
+                // dword w of the piece moved down by `back` elements
+                const int bit = back * EB + 32 * w;
+                uint32_t lo = 0u, hi = 0u;
+#pragma unroll
+                for(int j = w; j < PW; ++j)
+                {
+                    lo = (bit >> 5) == j ? mraw[PW * i + j] : lo;
+                    hi = (bit >> 5) == j - 1 ? mraw[PW * i + j] : hi;
+                }
+                const uint32_t x = (uint32_t)((((uint64_t)hi << 32) | lo) >> (bit & 31));
+                // (its elements from `valid` on are past the end)
+                const int n = min(max(valid * EB - 32 * w, 0), 32);
+                const uint32_t keep = n == 32 ? ~0u : (1u << n) - 1u;
+                mraw[PW * i + w] = (x & keep) | (HIDDEN & ~keep);
             }
-            else
+        }
+    };
+    // hands the pieces to the lanes that apply them: group i (keys (i/4)*32 +
+    // 8*(i%4) + 4*half + 0..3 of query my_q) into dwords PW/2 * i .. of mraw.
+    // Chunk c of row r sits at chunk position c ^ (r / MASK_RPL) % 4 of its 32 keys:
+    // 256 bytes that are read together lie in different banks.
+    auto mask_transpose = [&]() __attribute__((always_inline))
+    {
+        typedef typename std::conditional<MODE == NNTILE_HIP_MASK_ADDITIVE, u32x4, u32x2>::type V;
+        __shared__ __attribute__((aligned(16))) char lds_mask[EXPLICIT ? WAVES * 32 * MASK_RB : 16];
+        char *mine = lds_mask + (tid >> 6) * (32 * MASK_RB);
+#pragma unroll
+        for(int mb = 0; mb < 2; ++mb)
+        {
+#pragma unroll
+            for(int h = 0; h < 2; ++h)
             {
-                const uint32_t keep = valid == 4 ? ~0u : (1u << (8 * valid)) - 1u;
-                mraw[i] = (mraw[i] >> (8 * (back & 3))) & keep;
+                const int r = 16 * h + piece_row;
+                V v;
+#pragma unroll
+                for(int w = 0; w < PW; ++w)
+                {
+                    v[w] = mraw[PW * (2 * mb + h) + w];
+                }
+                *reinterpret_cast<V *>(mine + r * MASK_RB
+                        + (piece ^ ((r / MASK_RPL) % 4)) * (4 * PW)) = v;
             }
+            // (the LDS accesses of a wavefront are carried out in order; this
+            // keeps the compiler to it)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for(int rg = 0; rg < 4; ++rg)
+            {
+                const char *at = mine + col * MASK_RB + (rg ^ ((col / MASK_RPL) % 4)) * (4 * PW)
+                    + half * (2 * PW);
+                if constexpr(MODE == NNTILE_HIP_MASK_ADDITIVE)
+                {
+                    const u32x2 v = *reinterpret_cast<const u32x2 *>(at);
+                    mraw[2 * (4 * mb + rg)] = v[0];
+                    mraw[2 * (4 * mb + rg) + 1] = v[1];
+                }
+                else
+                {
+                    mraw[4 * mb + rg] = *reinterpret_cast<const uint32_t *>(at);
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
     };
     auto mask_classify = [&]() -> int
@@ -903,6 +962,10 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 mask_fix_ragged(keys_here);
             }
             mask_class = mask_classify();
+            if(mask_class == MASK_MIXED)
+            {
+                mask_transpose();
+            }
         }
         // nothing of this step is visible to this wavefront, or the step is
         // the other group's last one and this group has none in this round
@@ -1425,6 +1488,10 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 fast_step(g + 1, std::integral_constant<int, 0>{}, No{});
             }
         }
+        if(EXPLICIT && n_fast < n_steps)
+        {
+            mask_fetch(cur.kb, cur.rows_left);     // the general step finds its mask values loaded
+        }
         // drain: the output of the last sub-block
         if((n_fast - 1) & 1)
         {
@@ -1436,10 +1503,6 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         }
         g_first = n_fast;
         nxt = c1;
-        if(EXPLICIT && g_first < n_steps)
-        {
-            mask_fetch(cur.kb, cur.rows_left);     // the general step finds its mask values loaded
-        }
         // the general loop expects step g_first complete in its buffers
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
