@@ -1906,6 +1906,10 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
     return NNTILE_HIP_OK;
 }
 
+// Key steps from which a head of 64 under a mask given as values is walked by two
+// groups of wavefronts (see below)
+constexpr int64_t kSplitSteps64 = 16;
+
 // Host launcher shared by the tile and grid entry points.  p must be fully
 // filled except for the block counts and the remap flag.  scan_scratch: device
 // memory the call may use for a scan of an explicit mask (may be null).
@@ -1940,17 +1944,23 @@ int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head,
     }
     // Two groups of four wavefronts per workgroup, each taking every second
     // key step (p.form == 2, or by itself): when the launch has at most one
-    // 128-query workgroup per CU, so that a CU would otherwise hold one
-    // wavefront per SIMD, and enough key steps to share (with a mask given as
-    // values a 1024-key tile measured no gain or a small loss - the scan of
-    // the mask rows and the mask loads weigh more there - 4096 keys 7-11 %;
-    // analytic masks: 3-8 % at 1024 keys and 256 workgroups, 12-20 % on
-    // longer rows or fewer workgroups).
+    // 128-query workgroup per CU, so that a CU would otherwise hold one wavefront
+    // per SIMD, and enough key steps to share.  Analytic masks: 3-8 % at 1024 keys and 256 workgroups,
+    // 12-20 % on longer rows or fewer workgroups.  Masks given as values, head 128:
+    // 1024 keys 21.5 us with four wavefronts, 22.6 with two groups (8 heads; hidden
+    // 3.9 / 5.0, causal 22.9 / 23.3), 4096 keys 7-11 % less; head 64: 500 keys 13.2 /
+    // 13.3 (12 heads), 777 17.5 / 17.5, 1024 17.2 / 16.1, causal 18.3 / 16.6, hidden 3.5
+    // / 3.9 (8 heads), 1500 24.2 / 21.4, causal 24.5 / 20.7.
     const bool can_split = (head == 64 || head == 128) && !wide;
     const bool explicit_mask = mode == NNTILE_HIP_MASK_ADDITIVE || mode == NNTILE_HIP_MASK_BOOL;
+    // (from 16 steps: the scanning workgroups counted, whether or not this call has
+    // any - what a call computes does not depend on its scratch)
+    const int64_t n_scan = p.n_q_tiles * (int64_t)p.q_blocks_per_tile * kMaskBitSplits;
+    const bool split_64 = head == 64 && p.k_seq >= kSplitSteps64 * kKeys
+        && n_wg + n_scan <= 8 * (int64_t)kCUsPerXCD;
     const bool key_split = can_split && (p.form == 2
             || (p.form == 0 && n_wg <= 8 * (int64_t)kCUsPerXCD
-                && p.k_seq >= (explicit_mask ? 32 : 4) * kKeys));
+                && (p.k_seq >= (explicit_mask ? 32 : 4) * kKeys || split_64)));
     p.mask_bits = nullptr;
     const int scan_rc = scan_mask_once<T>(stream, p, mode, scan_scratch, scan_scratch_bytes);
     if(scan_rc != NNTILE_HIP_OK)
