@@ -1821,9 +1821,10 @@ void mask_step_bits_kernel(const char *mask, uint32_t ld_bytes, int q_len, int k
 }
 
 // Masks below this size are scanned by the attention kernel's workgroups
-// themselves, each its own rows: waiting for the shared scan costs a workgroup
-// about 2 us more than its first loads, scanning 128 rows of 400 values about
-// as much (7 x 355^2: 0.5 % slower shared, 10 x 621^2: 12 % faster).
+// themselves, each its own rows, on a stream that is being captured: the shared scan
+// is a launch of its own there, 2 to 3 us.  (Elsewhere it is the faster one at every
+// size: 4 x 128^2 of head 64, causal, 9.1 -> 8.5 us, 30 x 256^2 of head 128 14.3 -> 13.4,
+// 40 x 355^2 of head 64 15.1 -> 12.9, 40 x 430^2 of head 128 16.7 -> 15.5.)
 constexpr int64_t kMaskScanBytes = 3 << 17;
 
 // A value that none of the last 2^32 calls of this process has used and that
@@ -1865,8 +1866,7 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
         * (kMaskBitWords * (int64_t)sizeof(unsigned long long));
     if(row_bytes < 16 || p.mask_ld * es * kQRows >= (int64_t)(1 << 30)
             || reinterpret_cast<uintptr_t>(scratch) % 8 != 0
-            || (int64_t)scratch_bytes < table_bytes
-            || p.q_seq * row_bytes < kMaskScanBytes || p.batch < 2)
+            || (int64_t)scratch_bytes < table_bytes)
     {
         return NNTILE_HIP_OK;
     }
@@ -1877,6 +1877,11 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
     {
         (void)hipGetLastError();
         capturing = hipStreamCaptureStatusActive;       // the careful form
+    }
+    if(capturing != hipStreamCaptureStatusNone
+            && (p.q_seq * row_bytes < kMaskScanBytes || p.batch < 2))
+    {
+        return NNTILE_HIP_OK;
     }
     if(capturing == hipStreamCaptureStatusNone)
     {
