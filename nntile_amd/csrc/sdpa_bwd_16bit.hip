@@ -514,10 +514,51 @@ __device__ __forceinline__ void bwd_store_rows(char *xch, char *base, int n_ok,
     }
 }
 
+// Two groups of wavefronts in a workgroup (GROUPS == 2): what the second has summed up
+// goes through LDS - its own tiles, which nobody reads any more - to the first, which
+// holds the same rows and adds it.  own: the group's array of the wavefront, 64 lanes x
+// 16 * N values; BYTES from the first group's to the second's.  False: nothing left to
+// do for this wavefront.
+template<int N, int BYTES>
+__device__ __forceinline__ bool bwd_add_groups(int grp, char *own, f32x16 (&acc)[N])
+{
+    static_assert(64 * 16 * N * 4 == BYTES, "a wavefront's sums fill its array");
+    float *at = reinterpret_cast<float *>(own + (grp == 0 ? BYTES : 0)) + lane_index_again();
+    if(grp == 1)
+    {
+#pragma unroll
+        for(int db = 0; db < N; ++db)
+        {
+#pragma unroll
+            for(int r = 0; r < 16; ++r)
+            {
+                at[(16 * db + r) * 64] = acc[db][r];
+            }
+        }
+    }
+    __syncthreads();
+    if(grp == 1)
+    {
+        return false;
+    }
+#pragma unroll
+    for(int db = 0; db < N; ++db)
+    {
+#pragma unroll
+        for(int r = 0; r < 16; ++r)
+        {
+            acc[db][r] += at[(16 * db + r) * 64];
+        }
+    }
+    return true;
+}
+
+// GROUPS: 2: the workgroup is two groups of four wavefronts on the same rows, which
+// take the steps of the walk in turn through tiles of their own (see the launcher).
 // GRID: the rows of both sequence axes live in separately allocated tiles
 // (BwdGridParams); a workgroup's own 128 rows lie in one tile and every 64-row
 // step of the other axis does too, because tile sizes are multiples of 128.
-template<typename T, int HEAD, int MODE, bool GRID>
+template<typename T, int HEAD, int MODE, bool GRID, int GROUPS>
 __device__ __forceinline__ void sdpa_bwd_dq_body(
         const std::conditional_t<GRID, BwdGridParams, BwdParams> &p, unsigned wg,
         char *lds_k0, char *lds_k1, char *lds_v0, char *lds_v1)
@@ -529,7 +570,10 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     constexpr bool EXPLICIT = (MODE == NNTILE_HIP_MASK_ADDITIVE
             || MODE == NNTILE_HIP_MASK_BOOL);
 
-    const int tid = threadIdx.x;
+    const int tid = (int)threadIdx.x % kBwdThreads;
+    const int grp = GROUPS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kBwdThreads) : 0;
+    // (the group's half of every array in LDS: part of the lanes' read addresses)
+    const int lds_grp = grp * G::BYTES;
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
@@ -663,7 +707,7 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
 #pragma unroll
     for(int ks = 0; ks < KSTEPS; ++ks)
     {
-        row_raddr[ks] = (uint32_t)(col * RB + ((2 * ks + half) ^ G::swz(col)) * 16);
+        row_raddr[ks] = (uint32_t)(lds_grp + col * RB + ((2 * ks + half) ^ G::swz(col)) * 16);
     }
     // transposed operand: within a 16-lane block lane i addresses row j = i/4 and
     // head values 4*(i%4)..+3 of the block's 16; lanes 16..31 take the upper 16
@@ -682,7 +726,7 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
             for(int db = 0; db < DBLOCKS; ++db)
             {
                 const int c = 4 * db + 2 * dblk + (r4 >> 1);
-                tr_raddr[a][db] = (uint32_t)(r * RB + (c ^ G::swz(r)) * 16 + 8 * (r4 & 1));
+                tr_raddr[a][db] = (uint32_t)(lds_grp + r * RB + (c ^ G::swz(r)) * 16 + 8 * (r4 & 1));
             }
         }
     }
@@ -719,8 +763,8 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     auto fetch_piece = [&](const KeyRows &at, char *kdst_base, char *vdst_base, int i)
         __attribute__((always_inline))
     {
-        char *kdst = kdst_base + wave_u * LOADS_PER_WAVE * 1024;
-        char *vdst = vdst_base + wave_u * LOADS_PER_WAVE * 1024;
+        char *kdst = kdst_base + lds_grp + wave_u * LOADS_PER_WAVE * 1024;
+        char *vdst = vdst_base + lds_grp + wave_u * LOADS_PER_WAVE * 1024;
         const uint32_t goff = at.at_end ? ld_goff_end[i] : ld_goff[i];
         load_to_lds16<0, false>(at.K, goff, kdst + i * 1024);
         load_to_lds16<0, false>(at.V, goff, vdst + i * 1024);
@@ -763,7 +807,18 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     // the workgroup's two query blocks of 64 against the key blocks 0 .. n_steps-1
     const StepSet steps = make_step_set(p, EXPLICIT, q_row0 / kBwdStep,
             min(2, (q_seq - q_row0 + kBwdStep - 1) / kBwdStep), 0, n_steps, true);
-    int g_cur = steps.begin();
+    // (the group's steps: every second of the walk)
+    auto next_own = [&](int g) __attribute__((always_inline)) -> int
+    {
+        const int n = steps.next(g);
+        return GROUPS == 1 || n < 0 ? n : steps.next(n);
+    };
+    int g_cur = steps.begin(), g_last = -1;
+    if(GROUPS > 1 && grp == 1 && g_cur >= 0)
+    {
+        g_last = -2;                        // (the first group has a step)
+        g_cur = steps.next(g_cur);
+    }
     if(g_cur >= 0)
     {
         fetch(g_cur, lds_k0, lds_v0);
@@ -1107,26 +1162,40 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     };
     while(g_cur >= 0)
     {
-        int g_next = steps.next(g_cur);
+        int g_next = next_own(g_cur);
         run(g_cur, g_next, std::integral_constant<int, 0>{});
+        g_last = g_cur;
         g_cur = g_next;
         if(g_cur < 0)
         {
             break;
         }
-        g_next = steps.next(g_cur);
+        g_next = next_own(g_cur);
         run(g_cur, g_next, std::integral_constant<int, 1>{});
+        g_last = g_cur;
         g_cur = g_next;
     }
     // (the last step's spare loads into LDS must have landed before the
     // workgroup's LDS can be given away)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // (one barrier a step: the second group meets that of a last step it has not)
+    if(GROUPS > 1 && grp == 1 && (g_last == -2 || (g_last >= 0 && steps.next(g_last) >= 0)))
+    {
+        __syncthreads();
+    }
 
     // ---- dQ (+)= scale acc (every wavefront is done with the tiles in LDS) -----------
     __syncthreads();
     const int row_first = q_row0 + wave_u * 32;
-    bwd_store_rows<T, HEAD>(wave_u == 0 ? lds_k0 : wave_u == 1 ? lds_k1 : wave_u == 2 ? lds_v0
-            : lds_v1, static_cast<char *>(dQ_own) + row_elem(row_first, true) * RB,
+    char *xch = (wave_u == 0 ? lds_k0 : wave_u == 1 ? lds_k1 : wave_u == 2 ? lds_v0 : lds_v1) + lds_grp;
+    if constexpr(GROUPS > 1)
+    {
+        if(!bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, acc))
+        {
+            return;
+        }
+    }
+    bwd_store_rows<T, HEAD>(xch, static_cast<char *>(dQ_own) + row_elem(row_first, true) * RB,
             q_seq - row_first, acc, p.scale, !p.overwrite);
 }
 
@@ -1155,7 +1224,7 @@ constexpr int kDkvWaves = 4;
 constexpr int kDkvThreads = kDkvWaves * 64;
 constexpr int kDkvRows = kDkvWaves * 32;        // keys per workgroup
 
-template<typename T, int HEAD, int MODE, int PART, bool GRID>
+template<typename T, int HEAD, int MODE, int PART, bool GRID, int GROUPS>
 __device__ __forceinline__ void sdpa_bwd_dkv_body(
         const std::conditional_t<GRID, BwdGridParams, BwdParams> &p, unsigned wg,
         char *lds_q0, char *lds_q1, char *lds_g0, char *lds_g1,
@@ -1173,7 +1242,10 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     constexpr bool EXPLICIT = (MODE == NNTILE_HIP_MASK_ADDITIVE
             || MODE == NNTILE_HIP_MASK_BOOL);
 
-    const int tid = threadIdx.x;
+    const int tid = (int)threadIdx.x % kDkvThreads;
+    const int grp = GROUPS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kDkvThreads) : 0;
+    // (the group's half of every array in LDS: part of the lanes' read addresses)
+    const int lds_grp = grp * G::BYTES;
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
@@ -1299,7 +1371,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
 #pragma unroll
     for(int ks = 0; ks < KSTEPS; ++ks)
     {
-        row_raddr[ks] = (uint32_t)(col * RB + ((2 * ks + half) ^ G::swz(col)) * 16);
+        row_raddr[ks] = (uint32_t)(lds_grp + col * RB + ((2 * ks + half) ^ G::swz(col)) * 16);
     }
     uint32_t tr_raddr[2][DBLOCKS];
     {
@@ -1313,7 +1385,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
             for(int db = 0; db < DBLOCKS; ++db)
             {
                 const int c = 4 * db + 2 * dblk + (r4 >> 1);
-                tr_raddr[a][db] = (uint32_t)(r * RB + (c ^ G::swz(r)) * 16 + 8 * (r4 & 1));
+                tr_raddr[a][db] = (uint32_t)(lds_grp + r * RB + (c ^ G::swz(r)) * 16 + 8 * (r4 & 1));
             }
         }
     }
@@ -1399,8 +1471,8 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     {
         const char *Qp = static_cast<const char *>(at.Q) + at.elem * RB;
         const char *Gp = static_cast<const char *>(at.dA) + at.elem * RB;
-        char *qdst = qdst_base + wave_u * LPW * 1024;
-        char *gdst = gdst_base + wave_u * LPW * 1024;
+        char *qdst = qdst_base + lds_grp + wave_u * LPW * 1024;
+        char *gdst = gdst_base + lds_grp + wave_u * LPW * 1024;
         const uint32_t goff = at_end ? ld_goff_end[j] : ld_goff[j];
         load_to_lds16<0, false>(Qp, goff, qdst + j * 1024);
         load_to_lds16<0, false>(Gp, goff, gdst + j * 1024);
@@ -1486,7 +1558,18 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
         fetch_stat(at, last, stat);
     };
 
-    int i_cur = walk_begin();
+    // (the group's steps: every second of the walk)
+    auto walk_own = [&](int i) __attribute__((always_inline)) -> int
+    {
+        const int n = walk_next(i);
+        return GROUPS == 1 || n < 0 ? n : walk_next(n);
+    };
+    int i_cur = walk_begin(), i_last = -1;
+    if(GROUPS > 1 && grp == 1 && i_cur >= 0)
+    {
+        i_last = -2;                        // (the first group has a step)
+        i_cur = walk_next(i_cur);
+    }
     if(i_cur >= 0)
     {
         fetch(i_cur, lds_q0, lds_g0, lds_stat[0]);
@@ -2123,26 +2206,41 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     };
     while(i_cur >= 0)
     {
-        int i_next = walk_next(i_cur);
+        int i_next = walk_own(i_cur);
         run(i_cur, i_next, std::integral_constant<int, 0>{});
+        i_last = i_cur;
         i_cur = i_next;
         if(i_cur < 0)
         {
             break;
         }
-        i_next = walk_next(i_cur);
+        i_next = walk_own(i_cur);
         run(i_cur, i_next, std::integral_constant<int, 1>{});
+        i_last = i_cur;
         i_cur = i_next;
     }
     // (the last step's spare loads into LDS must have landed before the
     // workgroup's LDS can be given away)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // (one barrier a step: the second group meets that of a last step it has not)
+    if(GROUPS > 1 && grp == 1 && (i_last == -2 || (i_last >= 0 && walk_next(i_last) >= 0)))
+    {
+        __syncthreads();
+    }
 
     BWD_TRACE_FLUSH(PART);
     // ---- dK (+)= scale dk, dV (+)= dv (every wavefront is done with the tiles in LDS) ---
     __syncthreads();
     const int row_first = k_row0 + wave_u * 32;
-    char *xch = wave_u == 0 ? lds_q0 : wave_u == 1 ? lds_q1 : wave_u == 2 ? lds_g0 : lds_g1;
+    char *xch = (wave_u == 0 ? lds_q0 : wave_u == 1 ? lds_q1 : wave_u == 2 ? lds_g0 : lds_g1) + lds_grp;
+    if constexpr(GROUPS > 1)
+    {
+        static_assert(!BOTH, "two groups: a gradient of its own each");
+        if(!bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, DO_DK ? dk : dv))
+        {
+            return;
+        }
+    }
     const int64_t first_byte = row_elem(row_first, true) * RB;
     if(DO_DK)
     {
@@ -2161,21 +2259,23 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
 // last n_dkv dV.  A tile-pair call has fewer workgroups per gradient than the
 // chip has places (two a CU); together they fill it, and a long call loses
 // the ends of two launches.
-template<typename T, int HEAD, int MODE, bool GRID, bool FUSED_KEYS = false>
-__global__ __launch_bounds__(kDkvThreads, 2)
+template<typename T, int HEAD, int MODE, bool GRID, bool FUSED_KEYS = false, int GROUPS = 1>
+__global__ __launch_bounds__(kDkvThreads * GROUPS, 2)
 void sdpa_bwd_kernel(const std::conditional_t<GRID, BwdGridParams, BwdParams> p, unsigned n_dkv,
         unsigned n_dq)
 {
     BWD_WALL(0, blockIdx.x < n_dkv ? 1 : (blockIdx.x < n_dkv + n_dq ? 0 : 2));
     typedef BwdTile<HEAD> G;
     static_assert(kDkvThreads == kBwdThreads, "one block size for the three parts");
-    __shared__ __attribute__((aligned(1024))) char lds_0[G::BYTES];
-    __shared__ __attribute__((aligned(1024))) char lds_1[G::BYTES];
-    __shared__ __attribute__((aligned(1024))) char lds_2[G::BYTES];
-    __shared__ __attribute__((aligned(1024))) char lds_3[G::BYTES];
+    __shared__ __attribute__((aligned(1024))) char lds_0[G::BYTES * GROUPS];
+    __shared__ __attribute__((aligned(1024))) char lds_1[G::BYTES * GROUPS];
+    __shared__ __attribute__((aligned(1024))) char lds_2[G::BYTES * GROUPS];
+    __shared__ __attribute__((aligned(1024))) char lds_3[G::BYTES * GROUPS];
     // dK, dV parts, per query of a step: logsumexp in log2 units (+inf for a
     // row that saw nothing) and minus the row dot D; rows past the end hold +inf / 0
-    __shared__ __attribute__((aligned(16))) float lds_stat[2][2][kBwdStep];
+    __shared__ __attribute__((aligned(16))) float lds_stat_all[GROUPS][2][2][kBwdStep];
+    const int grp = GROUPS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kDkvThreads) : 0;
+    float (*const lds_stat)[2][kBwdStep] = lds_stat_all[grp];
     if constexpr(FUSED_KEYS)
     {
         // (K and V fragments and both accumulators fit beside the rest: one
@@ -2183,26 +2283,26 @@ void sdpa_bwd_kernel(const std::conditional_t<GRID, BwdGridParams, BwdParams> p,
         // the scores, seven products a call instead of eight)
         if(blockIdx.x < n_dkv)
         {
-            sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK | BWD_PART_DV, GRID>(p, blockIdx.x, lds_0,
+            sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK | BWD_PART_DV, GRID, GROUPS>(p, blockIdx.x, lds_0,
                     lds_1, lds_2, lds_3, lds_stat);
         }
         else
         {
-            sdpa_bwd_dq_body<T, HEAD, MODE, GRID>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3);
+            sdpa_bwd_dq_body<T, HEAD, MODE, GRID, GROUPS>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3);
         }
     }
     else if(blockIdx.x < n_dkv)
     {
-        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK, GRID>(p, blockIdx.x, lds_0, lds_1, lds_2,
+        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK, GRID, GROUPS>(p, blockIdx.x, lds_0, lds_1, lds_2,
                 lds_3, lds_stat);
     }
     else if(blockIdx.x < n_dkv + n_dq)
     {
-        sdpa_bwd_dq_body<T, HEAD, MODE, GRID>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3);
+        sdpa_bwd_dq_body<T, HEAD, MODE, GRID, GROUPS>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3);
     }
     else
     {
-        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DV, GRID>(p, blockIdx.x - n_dkv - n_dq, lds_0,
+        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DV, GRID, GROUPS>(p, blockIdx.x - n_dkv - n_dq, lds_0,
                 lds_1, lds_2, lds_3, lds_stat);
     }
 #ifdef NNTILE_BWD_TRACE
@@ -2240,6 +2340,30 @@ static int launch_prelude(hipStream_t stream, BwdPreludeParams &pre, int n_tiles
     hipLaunchKernelGGL((sdpa_bwd_prelude_kernel<T, HEAD, MODE == NNTILE_HIP_MASK_CAUSAL
                 ? NNTILE_HIP_MASK_NONE : MODE>), dim3((unsigned)n_wgs), dim3(256), 0, stream, pre);
     return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+}
+
+// Workgroups of two groups of wavefronts (sdpa_bwd_kernel, GROUPS == 2): where every
+// workgroup has a CU to itself, which one group would leave with one wavefront on each
+// SIMD, waiting for its own operands, and where the longest walk has enough steps to
+// share: their sums meet in LDS at the end, 0.7 to 1.5 us.  One group / two, us, bf16:
+//   head 64, tiles with a causal mask as values, 12 x 500: 17.7 / 17.2, 8 x 1024 25.3 /
+//     23.1, without one 20.2 / 18.3, 25.3 / 23.5, a window 21.6 / 18.5, 21.6 / 18.3; as a
+//     rule, 8 x 260 (five steps) 12.6 / 12.3 and open 11.8 / 12.2, 8 x 400 14.5 / 13.6; two
+//     entries with groups of eight, 130 rows 37.0 / 27.6, 520 83 / 60;
+//   head 128, 8 x 400 17.6 / 18.8, 520 (nine steps) 20.1 / 20.9, 800 25.4 / 24.9, causal
+//     26.0 / 24.6, 1100 32.4 / 29.5; two entries with groups of eight, 130 rows 44.6 /
+//     37.2, 520 104 / 83.  (With mask values there it does not fit the registers.)
+// steps: of the longest walk, the queries of all heads of a group or the keys.
+static bool bwd_two_groups(int64_t n_wgs, int64_t steps, int head)
+{
+    return n_wgs <= kBwdCUs && steps >= (head == 64 ? 6 : 13);
+}
+
+static int64_t bwd_longest_walk(const BwdParams &p)
+{
+    const int64_t keys = (p.k_seq + kBwdStep - 1) / kBwdStep;
+    const int64_t queries = (p.q_seq + kBwdStep - 1) / kBwdStep * p.kv_group;
+    return keys > queries ? keys : queries;
 }
 
 template<typename T, int HEAD, int MODE>
@@ -2288,6 +2412,17 @@ static int launch_bwd_mode(hipStream_t stream, const BwdParams &p)
             return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
         }
     }
+    if constexpr(HEAD == 64 || (HEAD == 128
+                && (MODE == NNTILE_HIP_MASK_NONE || MODE == NNTILE_HIP_MASK_CAUSAL)))
+    {
+        if(bwd_two_groups(2 * n_dkv + n_dq, bwd_longest_walk(p), HEAD))
+        {
+            hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, false, false, 2>),
+                    dim3((unsigned)(2 * n_dkv + n_dq)), dim3(2 * kDkvThreads), 0, stream, p,
+                    (unsigned)n_dkv, (unsigned)n_dq);
+            return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+        }
+    }
     hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, false>),
             dim3((unsigned)(2 * n_dkv + n_dq)), dim3(kDkvThreads), 0, stream, p,
             (unsigned)n_dkv, (unsigned)n_dq);
@@ -2330,6 +2465,16 @@ static int launch_bwd_grid_mode(hipStream_t stream, const BwdGridParams &p,
         {
             hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, true, true>),
                     dim3((unsigned)(n_dkv + n_dq)), dim3(kDkvThreads), 0, stream, p,
+                    (unsigned)n_dkv, (unsigned)n_dq);
+            return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+        }
+    }
+    if constexpr(HEAD >= 64)
+    {
+        if(bwd_two_groups(2 * n_dkv + n_dq, bwd_longest_walk(p), HEAD))
+        {
+            hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, true, false, 2>),
+                    dim3((unsigned)(2 * n_dkv + n_dq)), dim3(2 * kDkvThreads), 0, stream, p,
                     (unsigned)n_dkv, (unsigned)n_dq);
             return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
         }
