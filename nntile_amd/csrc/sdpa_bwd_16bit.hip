@@ -517,10 +517,9 @@ __device__ __forceinline__ void bwd_store_rows(char *xch, char *base, int n_ok,
 // Two groups of wavefronts in a workgroup (GROUPS == 2): what the second has summed up
 // goes through LDS - its own tiles, which nobody reads any more - to the first, which
 // holds the same rows and adds it.  own: the group's array of the wavefront, 64 lanes x
-// 16 * N values; BYTES from the first group's to the second's.  False: nothing left to
-// do for this wavefront.
+// 16 * N values; BYTES from the first group's to the second's.
 template<int N, int BYTES>
-__device__ __forceinline__ bool bwd_add_groups(int grp, char *own, f32x16 (&acc)[N])
+__device__ __forceinline__ void bwd_add_groups(int grp, char *own, f32x16 (&acc)[N])
 {
     static_assert(64 * 16 * N * 4 == BYTES, "a wavefront's sums fill its array");
     float *at = reinterpret_cast<float *>(own + (grp == 0 ? BYTES : 0)) + lane_index_again();
@@ -537,20 +536,18 @@ __device__ __forceinline__ bool bwd_add_groups(int grp, char *own, f32x16 (&acc)
         }
     }
     __syncthreads();
-    if(grp == 1)
-    {
-        return false;
-    }
-#pragma unroll
-    for(int db = 0; db < N; ++db)
+    if(grp == 0)
     {
 #pragma unroll
-        for(int r = 0; r < 16; ++r)
+        for(int db = 0; db < N; ++db)
         {
-            acc[db][r] += at[(16 * db + r) * 64];
+#pragma unroll
+            for(int r = 0; r < 16; ++r)
+            {
+                acc[db][r] += at[(16 * db + r) * 64];
+            }
         }
     }
-    return true;
 }
 
 // GROUPS: 2: the workgroup is two groups of four wavefronts on the same rows, which
@@ -1190,7 +1187,8 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     char *xch = (wave_u == 0 ? lds_k0 : wave_u == 1 ? lds_k1 : wave_u == 2 ? lds_v0 : lds_v1) + lds_grp;
     if constexpr(GROUPS > 1)
     {
-        if(!bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, acc))
+        bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, acc);
+        if(grp == 1)
         {
             return;
         }
@@ -1490,8 +1488,8 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
         const uint32_t place = flip_bits<16 * j>(wide_goff);
         const int past = max((int)(place / (uint32_t)RB) + (4 * j - last), 0);
         const uint32_t goff = place + (uint32_t)((4 * j - past) * RB);
-        load_to_lds16<0, false>(Qp, goff, qdst_base + wave_u * LPW * 1024 + j * 1024);
-        load_to_lds16<0, false>(Gp, goff, gdst_base + wave_u * LPW * 1024 + j * 1024);
+        load_to_lds16<0, false>(Qp, goff, qdst_base + lds_grp + wave_u * LPW * 1024 + j * 1024);
+        load_to_lds16<0, false>(Gp, goff, gdst_base + lds_grp + wave_u * LPW * 1024 + j * 1024);
     };
     // The statistics of a step in two halves, so that the load's latency
     // passes behind the MFMAs of the step before: stat_load starts the read
@@ -2235,8 +2233,19 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     char *xch = (wave_u == 0 ? lds_q0 : wave_u == 1 ? lds_q1 : wave_u == 2 ? lds_g0 : lds_g1) + lds_grp;
     if constexpr(GROUPS > 1)
     {
-        static_assert(!BOTH, "two groups: a gradient of its own each");
-        if(!bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, DO_DK ? dk : dv))
+        if(DO_DK)
+        {
+            bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, dk);
+        }
+        if(BOTH)
+        {
+            __syncthreads();        // (the first sums have been read)
+        }
+        if(DO_DV)
+        {
+            bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, dv);
+        }
+        if(grp == 1)
         {
             return;
         }
@@ -2366,6 +2375,21 @@ static int64_t bwd_longest_walk(const BwdParams &p)
     return keys > queries ? keys : queries;
 }
 
+// The same where one workgroup computes dK and dV: the workgroups that own keys walk
+// every query of a group's heads, under a causal mask those of the first keys all of
+// them, and a launch that has not enough of them to fill the chip ends with their walks.
+// One group / two, us, bf16: head 128, causal, 64 query heads on 16, 800 rows 150 / 92, 2 500
+// 500 / 447, two groups of eight, 4 096 rows, 1 289 / 742; 32 heads, 800 rows 49 / 39, 8 heads, 4 096 rows 190 / 134; head 64 71 / 53, 240 / 230, 579 / 416, 26 / 24,
+// 96 / 77.  Without a mask every walk is as long: grouped 800 rows 156 / 98 (head 64 72 / 57),
+// 2 500 rows on 8 223 / 199, but one head a group 800 rows 53 / 57 (28 / 34), and from 208
+// workgroups of head 64 on 161 / 167.
+static bool bwd_two_groups_fused(int64_t n_dkv, const BwdParams &p, int mode)
+{
+    const bool few = mode == NNTILE_HIP_MASK_CAUSAL ? n_dkv <= kBwdCUs
+        : p.kv_group > 1 && n_dkv <= kBwdCUs * 3 / 4;
+    return few && bwd_longest_walk(p) >= 13;
+}
+
 template<typename T, int HEAD, int MODE>
 static int launch_bwd_mode(hipStream_t stream, const BwdParams &p)
 {
@@ -2406,6 +2430,16 @@ static int launch_bwd_mode(hipStream_t stream, const BwdParams &p)
         // the separate sets have the shorter ones.
         if(2 * n_dkv + n_dq > 2 * kBwdCUs)
         {
+            if constexpr(HEAD >= 64 && (MODE == NNTILE_HIP_MASK_NONE || MODE == NNTILE_HIP_MASK_CAUSAL))
+            {
+                if(bwd_two_groups_fused(n_dkv, p, MODE))
+                {
+                    hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, false, true, 2>),
+                            dim3((unsigned)(n_dkv + n_dq)), dim3(2 * kDkvThreads), 0, stream, p,
+                            (unsigned)n_dkv, (unsigned)n_dq);
+                    return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+                }
+            }
             hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, false, true>),
                     dim3((unsigned)(n_dkv + n_dq)), dim3(kDkvThreads), 0, stream, p,
                     (unsigned)n_dkv, (unsigned)n_dq);
@@ -2463,6 +2497,16 @@ static int launch_bwd_grid_mode(hipStream_t stream, const BwdGridParams &p,
         // the separate sets have the shorter ones.
         if(2 * n_dkv + n_dq > 2 * kBwdCUs)
         {
+            if constexpr(HEAD >= 64 && (MODE == NNTILE_HIP_MASK_NONE || MODE == NNTILE_HIP_MASK_CAUSAL))
+            {
+                if(bwd_two_groups_fused(n_dkv, p, MODE))
+                {
+                    hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, true, true, 2>),
+                            dim3((unsigned)(n_dkv + n_dq)), dim3(2 * kDkvThreads), 0, stream, p,
+                            (unsigned)n_dkv, (unsigned)n_dq);
+                    return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+                }
+            }
             hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, true, true>),
                     dim3((unsigned)(n_dkv + n_dq)), dim3(kDkvThreads), 0, stream, p,
                     (unsigned)n_dkv, (unsigned)n_dq);

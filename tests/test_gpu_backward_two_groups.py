@@ -51,3 +51,43 @@ def test_gradients_of_walks_shared_by_two_groups(dtype, mode, head, group, q_seq
     for name in want:
         err = H.rel_fro(H.to_np(out[name]), want[name].numpy())
         assert err < TOL[dtype], (name, err)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("mode", ["none", "causal"])
+@pytest.mark.parametrize("head,group,n_kv,q_seq,k_seq", [
+    (64, 4, 48, 200, 129), (64, 13, 33, 64, 70), (128, 4, 48, 200, 129), (128, 13, 33, 65, 128), (128, 5, 44, 140, 200),
+    (64, 1, 60, 830, 130), (128, 1, 60, 800, 257)])
+def test_both_gradients_by_two_groups(dtype, mode, head, group, n_kv, q_seq, k_seq):
+    """Launches of more workgroups, where one set of them computes dK and dV: the call
+    over all key-value heads against the same in small ones."""
+    print("case two groups fused", dtype, mode, head, group, n_kv, q_seq, k_seq, flush=True)
+    m = hip_sdpa.MASK_NONE if mode == "none" else hip_sdpa.MASK_CAUSAL
+    offset = max(k_seq - q_seq, 0)
+    kind = H.TORCH_DT[dtype]
+    torch.manual_seed(q_seq + k_seq)
+    K, V = (torch.randn(n_kv, k_seq, head, device="cuda").to(kind) for _ in range(2))
+    Q, G = (torch.randn(n_kv * group, q_seq, head, device="cuda").to(kind) for _ in range(2))
+    lse, A = H.fresh_outputs(n_kv * group, q_seq, head, dtype)
+    hip_sdpa.sdpa_fwd_tile(K, Q, None, lse, V, A, m, n_batch=1, kv_group=group, causal_offset=offset,
+                           flags=hip_sdpa.OVERWRITE)
+
+    def call(lo, hi):
+        q = slice(lo * group, hi * group)
+        args = [t.contiguous() for t in (K[lo:hi], Q[q], V[lo:hi], A[q], G[q])]
+        out = [torch.full_like(t, float("nan")) for t in args[:3]]
+        hip_sdpa.sdpa_bwd_tile(*args, None, lse[q].contiguous(), *out, m, n_batch=1, kv_group=group,
+                               causal_offset=offset, flags=hip_sdpa.OVERWRITE)
+        torch.cuda.synchronize()
+        return out
+
+    whole = call(0, n_kv)
+    parts = [call(i, min(i + 4, n_kv)) for i in range(0, n_kv, 4)]
+    # one rounding to the tile type each (2^-8 and 2^-11 of a value at most) of fp32 sums
+    # taken in another order
+    bound = {"bf16": 2.0 ** -8, "fp16": 2.0 ** -11}[dtype]
+    for i, name in enumerate(("dK", "dQ", "dV")):
+        want = torch.cat([p[i] for p in parts]).float()
+        assert torch.isfinite(want).all() and torch.isfinite(whole[i]).all(), name
+        err = float((whole[i].float() - want).norm() / want.norm())
+        assert err < bound, (name, err)
