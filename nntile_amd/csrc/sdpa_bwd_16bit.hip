@@ -2378,9 +2378,10 @@ static int64_t bwd_longest_walk(const BwdParams &p)
 // The same where one workgroup computes dK and dV: the workgroups that own keys walk
 // every query of a group's heads, under a causal mask those of the first keys all of
 // them, and a launch that has not enough of them to fill the chip ends with their walks.
-// One group / two, us, bf16: head 128, causal, 64 query heads on 16, 800 rows 150 / 92, 2 500
-// 500 / 447, two groups of eight, 4 096 rows, 1 289 / 742; 32 heads, 800 rows 49 / 39, 8 heads, 4 096 rows 190 / 134; head 64 71 / 53, 240 / 230, 579 / 416, 26 / 24,
-// 96 / 77.  Without a mask every walk is as long: grouped 800 rows 156 / 98 (head 64 72 / 57),
+// One group / two, us, bf16: head 128, causal, 64 query heads on 16, 800 rows 150 / 92,
+// 2 500 500 / 447, two groups of eight, 4 096 rows, 1 289 / 742; 32 heads, 800 rows 49 / 39,
+// 8 heads, 4 096 rows 190 / 134; head 64 71 / 53, 240 / 230, 579 / 416, 26 / 24, 96 / 77.
+// Without a mask every walk is as long: grouped 800 rows 156 / 98 (head 64 72 / 57),
 // 2 500 rows on 8 223 / 199, but one head a group 800 rows 53 / 57 (28 / 34), and from 208
 // workgroups of head 64 on 161 / 167.
 static bool bwd_two_groups_fused(int64_t n_dkv, const BwdParams &p, int mode)

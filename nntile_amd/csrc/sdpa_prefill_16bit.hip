@@ -1950,8 +1950,8 @@ int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head,
     // Two groups of four wavefronts per workgroup, each taking every second
     // key step (p.form == 2, or by itself): when the launch has at most one
     // 128-query workgroup per CU, so that a CU would otherwise hold one wavefront
-    // per SIMD, and enough key steps to share.  Analytic masks: 3-8 % at 1024 keys and 256 workgroups,
-    // 12-20 % on longer rows or fewer workgroups.  Masks given as values, head 128:
+    // per SIMD, and enough key steps to share.  Analytic masks: 3-8 % at 1024 keys and
+    // 256 workgroups, 12-20 % on longer rows or fewer workgroups.  Masks given as values, head 128:
     // 1024 keys 21.5 us with four wavefronts, 22.6 with two groups (8 heads; hidden
     // 3.9 / 5.0, causal 22.9 / 23.3), 4096 keys 7-11 % less; head 64: 500 keys 13.2 /
     // 13.3 (12 heads), 777 17.5 / 17.5, 1024 17.2 / 16.1, causal 18.3 / 16.6, hidden 3.5
