@@ -39,8 +39,8 @@ typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 // segment).  Query tile t holds rows [t*q_tile, min((t+1)*q_tile, q_seq)),
 // the same for key tiles.
 // Key ranges a mask is scanned in by mask_step_bits_kernel, and the 64-bit words
-// that say what a range holds
-constexpr int kMaskBitSplits = 8, kMaskBitWords = 4;
+// that say what a range holds (sdpa_mask_words.hpp)
+constexpr int kMaskBitSplits = 8, kMaskBitWords = 5;
 
 struct PrefillParams
 {
@@ -54,19 +54,18 @@ struct PrefillParams
     // 128-query block found - kMaskBitSplits entries per block, one per range of
     // keys, to be OR-ed.  Two bit sets: bit s of the first: some value of 64-key
     // step s is not "open", of the second: not "hidden" (steps from 63 on share
-    // bit 63).  An entry is kMaskBitWords words: the lower and upper half of the
-    // first set, then of the second, each below 32 bits of tag.  Null: every
+    // bit 63).  An entry is kMaskBitWords words (sdpa_mask_words.hpp).  Null: every
     // workgroup scans its own rows.
     unsigned long long *mask_bits;
     // The scan riding in the attention launch (n_scan_wgs > 0): the first
     // n_scan_wgs workgroups of the grid do the scan and publish the words of
-    // their (block, key range), mask_tag (unique to the call) above each; the
-    // attention workgroups wait until all words of their block carry it, at most
+    // their (block, key range) under mask_tag (unique to the call); the attention
+    // workgroups wait until every entry of their block is this call's, at most
     // mask_spin_limit ticks of the 100 MHz clock (then they scan their own rows).
-    // (A flag of its own behind the words cost a store acknowledged and a load
-    // more, one after the other: a pair that a mask hides, 1024 x 1024 x 32 of head
-    // 128, 5.5 -> 4.2 us, one that it leaves open 26.6 -> 25.3, 500 x 500 x 12 of
-    // head 64 under a causal mask 16.1 -> 14.3.)
+    // (A flag of its own, raised once the words were acknowledged, cost a store
+    // and a load more, one after the other: a pair that a mask hides, 1024 x 1024 x 32
+    // of head 128, 5.5 -> 4.2 us, one that it leaves open 26.6 -> 25.3, 500 x 500 x 12
+    // of head 64 under a causal mask 16.1 -> 14.3.)
     // Without (n_scan_wgs == 0) the words were written before the launch.
     unsigned long long mask_tag, mask_spin_limit;
     int32_t n_q_tiles, n_kv_tiles;

@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "sdpa_mask_scan.hpp"
+#include "sdpa_mask_words.hpp"
 
 #ifndef NNTILE_PF_AHEAD
 #define NNTILE_PF_AHEAD 3
@@ -104,18 +105,33 @@ __device__ __forceinline__ void mask_scan_range(const char *mask, uint32_t ld_by
             open_word, hidden_word, words, not_open, not_hidden);
 }
 
-// What a scan found about one (block, key range), as kMaskBitWords words: half of
-// one of its two words below, the call's tag above, by one thread each.
+// What a scan found about one (block, key range), as the words of its entry, by one
+// thread each.
 __device__ __forceinline__ void mask_words_publish(unsigned long long *entry, int tid,
         unsigned long long not_open, unsigned long long not_hidden, unsigned long long tag)
 {
+    static_assert(MaskWords::N == kMaskBitWords, "an entry holds its words");
     if(tid < kMaskBitWords)
     {
-        const unsigned long long w = (tid & 2) ? not_hidden : not_open;
-        const unsigned long long half = (tid & 1) ? w >> 32 : w & 0xffffffffull;
-        __hip_atomic_store(entry + tid, (tag << 32) | half, __ATOMIC_RELAXED,
-                __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(entry + tid,
+                (unsigned long long)MaskWords::word(tid, tag, not_open, not_hidden),
+                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+// Exclusive or of the values of every eight lanes that follow each other
+__device__ __forceinline__ uint64_t sum_of_eight(uint64_t x)
+{
+    uint32_t v[2] = {(uint32_t)x, (uint32_t)(x >> 32)};
+#pragma unroll
+    for(int w = 0; w < 2; ++w)
+    {
+        // the neighbour's, the other pair's, the other four's (lanes in reverse)
+        v[w] ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[w], 0xb1, 0xf, 0xf, true);
+        v[w] ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[w], 0x4e, 0xf, 0xf, true);
+        v[w] ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[w], 0x141, 0xf, 0xf, true);
+    }
+    return ((uint64_t)v[1] << 32) | v[0];
 }
 
 // PARTS: the workgroup takes one of p.n_parts ranges of the keys and leaves
@@ -192,7 +208,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     {
         // The first workgroups of the grid scan the mask for everybody (one
         // query tile, one key tile): they wait for nothing, so the attention
-        // workgroups behind them can wait for their flags.
+        // workgroups behind them can wait for their words.
         if(p.n_scan_wgs > 0)
         {
             if((int)blockIdx.x < p.n_scan_wgs)
@@ -207,7 +223,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                         (int)blockIdx.x / kMaskBitSplits, (int)blockIdx.x % kMaskBitSplits,
                         pub_words, pub_open, pub_hidden);
                 // written through to memory (device scope), where readers on any
-                // XCD find them; every word carries the tag, so none waits for another
+                // XCD find them; the tag says which are there, none waits for another
                 mask_words_publish(p.mask_bits + kMaskBitWords * (int64_t)blockIdx.x, tid, pub_open,
                         pub_hidden, p.mask_tag);
                 return;
@@ -773,39 +789,55 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
 #pragma unroll
             for(int sp = 0; sp < kMaskBitSplits; ++sp)
             {
-                const unsigned long long *e = w + kMaskBitWords * sp;
-                not_open |= (e[0] & 0xffffffffull) | (e[1] << 32);
-                not_hidden |= (e[2] & 0xffffffffull) | (e[3] << 32);
+                uint64_t e[MaskWords::N], open, hidden;
+#pragma unroll
+                for(int i = 0; i < MaskWords::N; ++i)
+                {
+                    e[i] = w[kMaskBitWords * sp + i];
+                }
+                (void)MaskWords::take(e, 0u, open, hidden);
+                not_open |= open;
+                not_hidden |= hidden;
             }
             scanned = true;
         }
         else if(n_steps > 0 && p.mask_bits != nullptr)
         {
-            // ... or is being done by the first workgroups of this launch: one
-            // thread per word of the block's key ranges waits for it (bounded; the
-            // Q fragments are on their way meanwhile), then everybody ORs
-            static_assert(kMaskBitWords * kMaskBitSplits <= 64, "one wavefront reads them all");
-            __shared__ uint32_t got_bits[kMaskBitWords];
+            // ... or is being done by the first workgroups of this launch: the
+            // first wavefront waits for the entries of the block's key ranges, eight
+            // lanes an entry, a word each (bounded; the Q fragments are on their way
+            // meanwhile), then everybody ORs.  (16 tasks of 4096 tokens, 32 heads, causal:
+            // 300.4 us; 297.5 with four words an entry that were taken one by one, which
+            // could be words from before; 4 % more with one lane an entry.)
+            static_assert(kMaskBitSplits == 8 && kMaskBitWords <= 8, "one wavefront reads them all");
+            __shared__ uint32_t got_bits[4];
             __shared__ int got_all;
-            if(tid < kMaskBitWords)
+            if(tid < 4)
             {
                 got_bits[tid] = 0u;
             }
-            if(tid == 0)
-            {
-                got_all = 1;
-            }
             __syncthreads();
-            if(tid < kMaskBitWords * kMaskBitSplits)
+            if(tid < 64)
             {
+                const int i = lane & 7;
+                const bool has_word = i < kMaskBitWords;
                 unsigned long long *e = p.mask_bits
-                    + (int64_t)qb * (kMaskBitWords * kMaskBitSplits) + tid;
+                    + ((int64_t)qb * kMaskBitSplits + (lane >> 3)) * kMaskBitWords
+                    + (has_word ? i : 0);
                 const unsigned long long t0 = wall_clock64();
                 unsigned long long word;
                 bool ok = true;
-                while(((word = __hip_atomic_load(e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                            >> 32) != (p.mask_tag & 0xffffffffull))
+                for(;;)
                 {
+                    word = __hip_atomic_load(e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    const uint64_t sum = sum_of_eight(
+                            has_word ? MaskWords::share(i, word, p.mask_tag) : 0u);
+                    const bool fits = !has_word
+                        || (MaskWords::tagged(i, word, p.mask_tag) && sum == 0u);
+                    if(__builtin_amdgcn_ballot_w64(!fits) == 0ull)
+                    {
+                        break;
+                    }
                     __builtin_amdgcn_s_sleep(2);
                     if(wall_clock64() - t0 > p.mask_spin_limit)
                     {
@@ -813,13 +845,13 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                         break;
                     }
                 }
-                if(ok)
+                if(i < 4)
                 {
-                    atomicOr(&got_bits[tid % kMaskBitWords], (uint32_t)word);
+                    atomicOr(&got_bits[i], (uint32_t)word);
                 }
-                else
+                if(lane == 0)
                 {
-                    got_all = 0;
+                    got_all = ok;
                 }
             }
             __syncthreads();
@@ -1827,26 +1859,23 @@ void mask_step_bits_kernel(const char *mask, uint32_t ld_bytes, int q_len, int k
 // 40 x 355^2 of head 64 15.1 -> 12.9, 40 x 430^2 of head 128 16.7 -> 15.5.)
 constexpr int64_t kMaskScanBytes = 3 << 17;
 
-// A value that none of the last 2^32 calls of this process has used and that
-// memory left behind by anything else is unlikely to hold in the upper halves of
-// all words of a block's ranges (32 words; never 0).
-static unsigned long long next_scan_tag()
+// A value that no earlier call of this process has used (see MaskWords).
+static uint64_t next_scan_tag()
 {
-    static const uint32_t salt = []
+    static const uint64_t start = []
     {
         std::random_device rd;
-        return (uint32_t)rd();
+        return ((uint64_t)rd() << 32) | rd();
     }();
-    static std::atomic<uint32_t> counter{0};
-    const uint32_t tag = salt + counter.fetch_add(1, std::memory_order_relaxed);
-    return tag == 0u ? next_scan_tag() : tag;
+    static std::atomic<uint64_t> counter{0};
+    return MaskWords::tag(start, counter.fetch_add(1, std::memory_order_relaxed));
 }
 
 // One-tile calls with an explicit mask and a scratch buffer of the caller's
 // (the reference's scratch_logsumexp tile): scan the mask once, into the
 // scratch, instead of once per batch entry - by the first workgroups of the
 // attention launch itself, or, on a stream that is being captured (a replay
-// would carry this call's tag again and find the flags of the replay before
+// would carry this call's tag again and find the words of the replay before
 // it), by a launch of its own.  Leaves p.mask_bits null when the conditions of
 // the kernel's own scan do not hold or the scratch is too small.
 template<typename T>
