@@ -103,13 +103,19 @@ enum nntile_hip_mask_mode
  * tile: seq queries against seq keys, additive mask [seq, seq] in T.
  * The merge is fused into the kernel, so neither scratch tile is needed for
  * it and both may be null.  scratch_A is never touched.  scratch_lse (seq *
- * batch floats, as the reference registers it) may be overwritten: when the
- * mask is 384 KiB or larger the 16-bit variants scan it once per call - by the
- * first workgroups of the attention launch, or, on a stream that is being
- * captured, by a small launch of their own - and keep what they found (24
- * bytes per 128 queries and key range) there, instead of letting the
- * workgroups of every batch entry scan the same rows.  Same result, bit for
- * bit.
+ * batch floats, as the reference registers it) may be overwritten: the 16-bit
+ * variants scan the mask once per call and keep what they found there (40 bytes
+ * for each of eight key ranges of every 128 queries, 320 together), instead of
+ * letting the workgroups of every batch entry scan the same rows.  The first
+ * workgroups of the attention launch do so for every mask of rows of 16 bytes
+ * and more; on a stream that is being captured a small launch of its own does,
+ * for masks of 384 KiB and more and two batch entries and more.  Where the buffer
+ * is too small for it, it is left alone.  Same result, bit for bit.
+ * The buffer's contents before the call do not matter.  Calls that may run at
+ * the same time, on different streams, should have a buffer each: where they
+ * share one the results are the same, but workgroups that find the other call's
+ * words wait, for 20 us and 10 ns a byte of a mask row, then scan for themselves;
+ * captured calls must not share one with calls that may run beside a replay.
  *
  * SIZE OF scratch_lse: the call has no argument for it and takes it to be
  * what the reference registers, seq * batch floats.  Pass NULL or a buffer of

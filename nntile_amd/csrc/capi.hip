@@ -404,8 +404,8 @@ static size_t tile_floats_bytes(int64_t seq, int64_t batch)
 
 // scratch_lse: the reference's scratch tile for the logsumexp of the pair
 // (seq * batch floats, src/starpu/flash_sdpa_fwd_cudnn.cc:128-136); the merge
-// is fused into the kernel, so the tile is free: a large mask is scanned once
-// into it instead of once per batch entry.  May be null.
+// is fused into the kernel, so the tile is free: the mask is scanned once into
+// it instead of once per batch entry.  May be null.
 static int flash_call(DType dt, void *stream, int64_t seq, int64_t head,
         int64_t batch, const void *K, const void *Q, const void *mask,
         const void *V, float *lse, void *A, float *scratch_lse,

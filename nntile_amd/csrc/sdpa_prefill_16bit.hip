@@ -1917,7 +1917,11 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
         p.mask_bits = table;
         p.n_scan_wgs = (int32_t)grid.x;
         p.mask_tag = next_scan_tag();
-        p.mask_spin_limit = 100000000ull;       // 1 s of the 100 MHz clock
+        // A scan takes 2 us, or what 128 rows of an eighth of the keys take a
+        // workgroup: well below a byte of a row a tick of the 100 MHz clock.  Words that
+        // are not there then were overwritten, by a call on another stream that
+        // was lent the same memory.
+        p.mask_spin_limit = 2000ull + (unsigned long long)row_bytes;
         return NNTILE_HIP_OK;
     }
     if(additive)

@@ -619,7 +619,7 @@ void flash_sdpa_fwd_cudnn_async(const Tile<T> &K, const Tile<T> &Q,
     const Index batch = K.shape[2] * K.shape[3] * K.shape[4];
     // The reference registers two scratch handles per call
     // (src/tile/flash_sdpa_fwd_cudnn.cc:176-195).  The HIP body fuses the
-    // merge and needs neither for it; it scans a large mask once into the
+    // merge and needs neither for it; it scans the mask once into the
     // first (seq * batch floats).  The second stays empty.
     starpu::VariableHandle scratch_logsumexp = starpu::worker_scratch(
             sizeof(float) * static_cast<std::size_t>(seq) * static_cast<std::size_t>(batch));

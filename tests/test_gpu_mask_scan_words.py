@@ -3,6 +3,8 @@
 the same bits, whatever that memory held before - words of earlier calls,
 constants, single words that carry the tag of the call to come - and at the
 edges of the sizes that are scanned so."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -128,3 +130,40 @@ def test_the_smallest_scratch_of_the_codelet_body(short):
     written = ~torch.isnan(memory)
     assert not bool(written[floats - short // 4:].any())
     assert bool(written.any()) == (short == 0)
+
+
+def test_two_streams_that_share_a_scratch():
+    """Calls that overwrite each other's words: workgroups that start late find those
+    of the other call and scan for themselves, after a wait of some 20 us, not one
+    that stalls the device."""
+    seq, head, batch, calls = 128, 64, 2048, 10
+    gen = torch.Generator(device="cuda").manual_seed(51)
+    Q, K, V = (torch.randn(batch, seq, head, generator=gen, device="cuda").bfloat16()
+               for _ in range(3))
+    masks = [H.additive_mask(_mask(kind, seq), "bf16").cuda() for kind in ("causal", "window")]
+    scratch = torch.zeros(batch, seq, device="cuda")
+
+    def outputs():
+        return torch.full((batch, seq), float("-inf"), device="cuda"), torch.zeros_like(Q)
+
+    want = []
+    for mask in masks:
+        want.append(outputs())
+        hip_sdpa.flash_sdpa_fwd(K, Q, mask, want[-1][0], V, want[-1][1])
+    got = [[outputs() for _ in range(calls)] for _ in masks]
+    streams = [torch.cuda.Stream() for _ in masks]
+    torch.cuda.synchronize()
+    t0 = time.monotonic()
+    for i in range(calls):
+        for mask, stream, outs in zip(masks, streams, got):
+            hip_sdpa.flash_sdpa_fwd(K, Q, mask, outs[i][0], V, outs[i][1], scratch_lse=scratch,
+                                    stream=stream)
+    torch.cuda.synchronize()
+    seconds = time.monotonic() - t0
+    print("%d calls in %.1f ms" % (2 * calls, 1e3 * seconds), flush=True)
+    for outs, (lse, A) in zip(got, want):
+        for l, a in outs:
+            assert torch.equal(l, lse) and torch.equal(a.view(torch.int16), A.view(torch.int16))
+    # 2048 workgroups, 512 at a time, 21 us of waiting each at the most: 0.1 ms a call
+    # beside its work; a call that waits out a second once is far above this
+    assert seconds < 0.5
