@@ -295,7 +295,11 @@ int nntile_hip_sdpa_fwd_grid_fp32(void *stream, const nntile_hip_sdpa_grid_args 
  * n_slabs*n_kv_tiles must not exceed NNTILE_HIP_SDPA_BWD_MAX_TILES.
  * workspace: n_slabs*q_seq*batch floats of device memory
  * (nntile_hip_sdpa_bwd_grid_workspace_bytes), 4-byte aligned, private to the
- * call until it has completed. */
+ * call until it has completed.
+ * The same call gives the same bits every time.  The order in which the sums of an
+ * entry's gradients are added in fp32 depends on the size of the launch (which form
+ * its kernel takes), so in their last bit they may differ between calls that put
+ * the entry beside others; the same holds for the tile calls. */
 #define NNTILE_HIP_SDPA_BWD_MAX_TILES 32
 
 typedef struct nntile_hip_sdpa_bwd_grid_args

@@ -214,7 +214,8 @@ def test_refusals():
 ])
 def test_slabs_in_one_call(dtype, head, mode, n_slabs, shape):
     """Several slabs of the batch grid in one call (n_slabs) give, bit for
-    bit, what one call per slab gives; the workspace grows with the slabs."""
+    bit, what one call per slab gives, at sizes where both launches share a walk
+    between as many groups of wavefronts; the workspace grows with the slabs."""
     q_seq, k_seq, q_tile, k_tile, n_batch, group, n_kv = shape
     print("case bwd slabs", dtype, head, mode, n_slabs, shape, flush=True)
     offset = max(k_seq - q_seq, 0)

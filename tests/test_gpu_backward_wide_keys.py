@@ -1,7 +1,7 @@
 """Key-owning workgroups that hold dK and dV at head 128 (a launch of more than
 512 workgroups under an analytic mask) against the same entries in launches that
-keep the two apart: the sums are the same, so the gradients agree bit for bit.
-Sizes at the edges of a step of 64 queries and of a workgroup's 128 keys."""
+keep the two apart: walks of less than 13 steps, which both take in one group of
+wavefronts, so the sums are the same and the gradients agree bit for bit.  Sizes at the edges of a step of 64 queries and of a workgroup's 128 keys."""
 import pytest
 import torch
 

@@ -1,5 +1,5 @@
-"""The reference-signature call with its scratch tile: a large additive mask
-is scanned once per call by a small kernel of its own (into the scratch
+"""The reference-signature call with its scratch tile: an additive mask is
+scanned once per call by the first workgroups of the launch (into the scratch
 logsumexp tile) instead of once per batch entry by the attention kernel's
 workgroups.  Both ways produce the same bits about the mask, so the results
 must be identical bit for bit, whatever the mask holds; and they must agree
