@@ -77,8 +77,6 @@ namespace nntile_hip
 #endif
 
 
-// Where the tile loads of the next step are issued: 0 = all at the start of
-// the step, 1 = between the MFMAs of the step's first half, 2 = of the whole
 // 1: a step's two query (key) blocks overlap - the matrix products of one
 // beside the vector work of the other; 0: one block after the other
 #ifndef NNTILE_BWD_PIPE
@@ -96,6 +94,8 @@ namespace nntile_hip
 #ifndef NNTILE_BWD_AHEAD_WIDE
 #define NNTILE_BWD_AHEAD_WIDE 2     // the same where a workgroup holds both gradients at head 128
 #endif
+// Where the tile loads of the next step are issued: 0 = all at the start of
+// the step, 1 = between the MFMAs of the step's first half, 2 = of the whole
 #ifndef NNTILE_BWD_SPREAD
 #define NNTILE_BWD_SPREAD 2
 #endif
@@ -1640,13 +1640,14 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
             // Both gradients at head 128: 192 registers hold fragments and
             // accumulators.  The step's two 32-query blocks go product by product,
             // S, dP, dV, dK, eight MFMAs each: 64 slots of one MFMA, the operand
-            // read of the slot AHEAD later - across the products' borders, the
-            // matrix unit does not wait for LDS anywhere in the step but at its
-            // start - and a slice of the vector work: P beside dP, dS beside dV.
+            // read of the slot AHEAD later - across the products' borders - and a
+            // slice of the vector work: P beside dP, dS beside dV.
             // Bound: the matrix pipe, 64 x 32 clocks a step and wavefront, at the
             // clock that the board's power leaves it (32 heads of 128, 4096 tokens,
             // causal, the whole call: 439 to 445 us with every MFMA behind its own
-            // operand read, 435 to 437 so, on two boxes; the same bits).
+            // operand read, 435 to 437 so, on two boxes; the same bits.  Waves stood
+            // at a wait or the barrier 43 % of their time, now 30 %, the matrix unit is
+            // busy 65 % of the clocks for 60, of which there are 1.68 GHz for 1.79).
             static_assert(!use_mask, "masks given as values at head 128: dK and dV apart");
             constexpr int AHEAD = NNTILE_BWD_AHEAD_WIDE;
             constexpr int SLOTS = 64;
@@ -2356,9 +2357,12 @@ static int launch_prelude(hipStream_t stream, BwdPreludeParams &pre, int n_tiles
 // SIMD, waiting for its own operands, and where the longest walk has enough steps to
 // share: their sums meet in LDS at the end, 0.7 to 1.5 us.  One group / two, us, bf16:
 //   head 64, tiles with a causal mask as values, 12 x 500: 17.7 / 17.2, 8 x 1024 25.3 /
-//     23.1, without one 20.2 / 18.3, 25.3 / 23.5, a window 21.6 / 18.5, 21.6 / 18.3; as a
-//     rule, 8 x 260 (five steps) 12.6 / 12.3 and open 11.8 / 12.2, 8 x 400 14.5 / 13.6; two
-//     entries with groups of eight, 130 rows 37.0 / 27.6, 520 83 / 60;
+//     23.1, without one 20.2 / 18.3, 25.3 / 23.5, a window 21.6 / 18.5, 21.6 / 18.3; six
+//     steps, 8 x 384: causal 15.5 / 15.4, a window 22.2 / 18.6, but open 14.7 / 15.0 (what the
+//     values hold is not known here), 8 x 330 16.2 / 16.1, 22.7 / 19.2, open 17.6 / 16.2; as a
+//     rule, 8 x 260 (five steps) 12.6 / 12.3 and open 11.8 / 12.2, 8 x 384 13.5 / 13.4 and
+//     open 12.9 / 13.1, 8 x 400 14.5 / 13.6; two entries with groups of eight, 130 rows 37.0 /
+//     27.6, 520 83 / 60;
 //   head 128, 8 x 400 17.6 / 18.8, 520 (nine steps) 20.1 / 20.9, 800 25.4 / 24.9, causal
 //     26.0 / 24.6, 1100 32.4 / 29.5; two entries with groups of eight, 130 rows 44.6 /
 //     37.2, 520 104 / 83.  (With mask values there it does not fit the registers.)
@@ -2378,17 +2382,58 @@ static int64_t bwd_longest_walk(const BwdParams &p)
 // The same where one workgroup computes dK and dV: the workgroups that own keys walk
 // every query of a group's heads, under a causal mask those of the first keys all of
 // them, and a launch that has not enough of them to fill the chip ends with their walks.
-// One group / two, us, bf16: head 128, causal, 64 query heads on 16, 800 rows 150 / 92,
-// 2 500 500 / 447, two groups of eight, 4 096 rows, 1 289 / 742; 32 heads, 800 rows 49 / 39,
-// 8 heads, 4 096 rows 190 / 134; head 64 71 / 53, 240 / 230, 579 / 416, 26 / 24, 96 / 77.
-// Without a mask every walk is as long: grouped 800 rows 156 / 98 (head 64 72 / 57),
-// 2 500 rows on 8 223 / 199, but one head a group 800 rows 53 / 57 (28 / 34), and from 208
-// workgroups of head 64 on 161 / 167.
+// One group (and operands not read ahead) / two, us, bf16, one box: head 128, causal, 64
+// query heads on 16, 800 rows 150 / 91, 2 500 503 / 457, two groups of eight, 4 096 rows,
+// 1 268 / 728; 32 heads, 800 rows 50 / 42, 8 heads, 4 096 rows 190 / 134; head 64 70 / 54,
+// 235 / 225, 546 / 405, 26.5 / 26.4, 95 / 77.  Without a mask every walk is as long:
+// grouped 800 rows 154 / 98 (head 64 72 / 59), two groups of eight, 4 096 rows, 1 305 / 787
+// (550 / 415), but one head a group 800 rows 53 / 57 (28 / 34), and from 208 workgroups of
+// head 64 on 161 / 167.
 static bool bwd_two_groups_fused(int64_t n_dkv, const BwdParams &p, int mode)
 {
     const bool few = mode == NNTILE_HIP_MASK_CAUSAL ? n_dkv <= kBwdCUs
         : p.kv_group > 1 && n_dkv <= kBwdCUs * 3 / 4;
     return few && bwd_longest_walk(p) >= 13;
+}
+
+// The gradient launch, the same for one allocation (GRID false) and for tiles.
+template<typename T, int HEAD, int MODE, bool GRID>
+static int launch_bwd_kernel(hipStream_t stream,
+        const std::conditional_t<GRID, BwdGridParams, BwdParams> &p, int64_t n_dkv, int64_t n_dq)
+{
+    constexpr bool ANALYTIC = MODE == NNTILE_HIP_MASK_NONE || MODE == NNTILE_HIP_MASK_CAUSAL;
+    auto launch = [&](auto kernel, int64_t n_wgs, int groups) -> int
+    {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)n_wgs), dim3(groups * kDkvThreads), 0, stream, p,
+                (unsigned)n_dkv, (unsigned)n_dq);
+        return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+    };
+    if constexpr(kBwdFusedKeys<HEAD, MODE>)
+    {
+        // One set of key-owning workgroups for both gradients (seven products
+        // instead of eight) once the three sets would not all be resident at
+        // the same time; below that the longest workgroup sets the time, and
+        // the separate sets have the shorter ones.
+        if(2 * n_dkv + n_dq > 2 * kBwdCUs)
+        {
+            if constexpr(HEAD >= 64 && ANALYTIC)
+            {
+                if(bwd_two_groups_fused(n_dkv, p, MODE))
+                {
+                    return launch(sdpa_bwd_kernel<T, HEAD, MODE, GRID, true, 2>, n_dkv + n_dq, 2);
+                }
+            }
+            return launch(sdpa_bwd_kernel<T, HEAD, MODE, GRID, true>, n_dkv + n_dq, 1);
+        }
+    }
+    if constexpr(HEAD == 64 || (HEAD == 128 && ANALYTIC))
+    {
+        if(bwd_two_groups(2 * n_dkv + n_dq, bwd_longest_walk(p), HEAD))
+        {
+            return launch(sdpa_bwd_kernel<T, HEAD, MODE, GRID, false, 2>, 2 * n_dkv + n_dq, 2);
+        }
+    }
+    return launch(sdpa_bwd_kernel<T, HEAD, MODE, GRID>, 2 * n_dkv + n_dq, 1);
 }
 
 template<typename T, int HEAD, int MODE>
@@ -2423,45 +2468,7 @@ static int launch_bwd_mode(hipStream_t stream, const BwdParams &p)
     {
         return pre_rc;
     }
-    if constexpr(kBwdFusedKeys<HEAD, MODE>)
-    {
-        // One set of key-owning workgroups for both gradients (seven products
-        // instead of eight) once the three sets would not all be resident at
-        // the same time; below that the longest workgroup sets the time, and
-        // the separate sets have the shorter ones.
-        if(2 * n_dkv + n_dq > 2 * kBwdCUs)
-        {
-            if constexpr(HEAD >= 64 && (MODE == NNTILE_HIP_MASK_NONE || MODE == NNTILE_HIP_MASK_CAUSAL))
-            {
-                if(bwd_two_groups_fused(n_dkv, p, MODE))
-                {
-                    hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, false, true, 2>),
-                            dim3((unsigned)(n_dkv + n_dq)), dim3(2 * kDkvThreads), 0, stream, p,
-                            (unsigned)n_dkv, (unsigned)n_dq);
-                    return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
-                }
-            }
-            hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, false, true>),
-                    dim3((unsigned)(n_dkv + n_dq)), dim3(kDkvThreads), 0, stream, p,
-                    (unsigned)n_dkv, (unsigned)n_dq);
-            return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
-        }
-    }
-    if constexpr(HEAD == 64 || (HEAD == 128
-                && (MODE == NNTILE_HIP_MASK_NONE || MODE == NNTILE_HIP_MASK_CAUSAL)))
-    {
-        if(bwd_two_groups(2 * n_dkv + n_dq, bwd_longest_walk(p), HEAD))
-        {
-            hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, false, false, 2>),
-                    dim3((unsigned)(2 * n_dkv + n_dq)), dim3(2 * kDkvThreads), 0, stream, p,
-                    (unsigned)n_dkv, (unsigned)n_dq);
-            return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
-        }
-    }
-    hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, false>),
-            dim3((unsigned)(2 * n_dkv + n_dq)), dim3(kDkvThreads), 0, stream, p,
-            (unsigned)n_dkv, (unsigned)n_dq);
-    return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+    return launch_bwd_kernel<T, HEAD, MODE, false>(stream, p, n_dkv, n_dq);
 }
 
 // The grid form: the row dots tile by tile (each tile's A and dA are one
@@ -2490,44 +2497,7 @@ static int launch_bwd_grid_mode(hipStream_t stream, const BwdGridParams &p,
     {
         return pre_rc;
     }
-    if constexpr(kBwdFusedKeys<HEAD, MODE>)
-    {
-        // One set of key-owning workgroups for both gradients (seven products
-        // instead of eight) once the three sets would not all be resident at
-        // the same time; below that the longest workgroup sets the time, and
-        // the separate sets have the shorter ones.
-        if(2 * n_dkv + n_dq > 2 * kBwdCUs)
-        {
-            if constexpr(HEAD >= 64 && (MODE == NNTILE_HIP_MASK_NONE || MODE == NNTILE_HIP_MASK_CAUSAL))
-            {
-                if(bwd_two_groups_fused(n_dkv, p, MODE))
-                {
-                    hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, true, true, 2>),
-                            dim3((unsigned)(n_dkv + n_dq)), dim3(2 * kDkvThreads), 0, stream, p,
-                            (unsigned)n_dkv, (unsigned)n_dq);
-                    return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
-                }
-            }
-            hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, true, true>),
-                    dim3((unsigned)(n_dkv + n_dq)), dim3(kDkvThreads), 0, stream, p,
-                    (unsigned)n_dkv, (unsigned)n_dq);
-            return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
-        }
-    }
-    if constexpr(HEAD >= 64)
-    {
-        if(bwd_two_groups(2 * n_dkv + n_dq, bwd_longest_walk(p), HEAD))
-        {
-            hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, true, false, 2>),
-                    dim3((unsigned)(2 * n_dkv + n_dq)), dim3(2 * kDkvThreads), 0, stream, p,
-                    (unsigned)n_dkv, (unsigned)n_dq);
-            return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
-        }
-    }
-    hipLaunchKernelGGL((sdpa_bwd_kernel<T, HEAD, MODE, true>),
-            dim3((unsigned)(2 * n_dkv + n_dq)), dim3(kDkvThreads), 0, stream, p,
-            (unsigned)n_dkv, (unsigned)n_dq);
-    return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+    return launch_bwd_kernel<T, HEAD, MODE, true>(stream, p, n_dkv, n_dq);
 }
 
 template<typename T, int HEAD>
