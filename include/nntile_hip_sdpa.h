@@ -57,8 +57,7 @@ extern "C" {
  * wavefronts split the key steps, on the fp32 ones (SPLIT).  16-bit: 128 queries
  * and four wavefronts (SHARED), or the same 128 queries held by two groups of
  * four wavefronts that take every second key step each and merge through LDS
- * (SPLIT; head 64 and 128; what a launch of at most one workgroup per CU takes by
- * itself).  Both set: ignored. */
+ * (SPLIT; head 64 and 128).  Both set: ignored. */
 #define NNTILE_HIP_SDPA_FORM_SHARED 0x100
 #define NNTILE_HIP_SDPA_FORM_SPLIT  0x200
 /* 16-bit tile and grid calls with an analytic mask, head 64 or 128, for tests
@@ -69,6 +68,11 @@ extern "C" {
  * shapes on the fp16 matrix units - 256 queries (WIDE), 128 queries and two key
  * blocks (WIDE | SHARED), 64 queries and two key blocks (WIDE | SPLIT). */
 #define NNTILE_HIP_SDPA_FORM_WIDE   0x4000
+/* 16-bit tile and grid calls, head 64 or 128, for tests and tuning: workgroups of 64
+ * queries whose four wavefronts take 32 keys of every step each (what most launches
+ * of at most one workgroup of 128 queries per CU take by themselves).  With another
+ * FORM flag and in fp32: ignored. */
+#define NNTILE_HIP_SDPA_FORM_HALVED 0x8000
 /* decode calls, for tests and tuning: merge the key splits in a second launch
  * instead of inside the main one (SEPARATE_MERGE); exchange the partials of
  * the in-launch merge through device-scope fences whatever XCD the

@@ -80,6 +80,10 @@ static int prefill_form(int32_t flags)
     {
         return 8 + (shared ? 1 : 0) + (split ? 2 : 0);      // 256-query workgroups; fp32: see launch_prefill_fp32
     }
+    if(flags & NNTILE_HIP_SDPA_FORM_HALVED)
+    {
+        return shared || split ? 0 : 3;
+    }
     return shared == split ? 0 : (shared ? 1 : 2);
 }
 

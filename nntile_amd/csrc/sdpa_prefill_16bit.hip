@@ -29,6 +29,7 @@
 // query tile; the epilogue merges the result into the (lse, A) pair in memory
 // (the hand-off between NNTile tasks), so one launch can stand for one task or
 // for a whole row of tasks.
+#include <algorithm>
 #include <atomic>
 #include <random>
 #include <type_traits>
@@ -136,7 +137,11 @@ __device__ __forceinline__ uint64_t sum_of_eight(uint64_t x)
 
 // PARTS: the workgroup takes one of p.n_parts ranges of the keys and leaves
 // its triple in memory (PrefillParams::part_o), where launch_parts_merge finds it.
-template<typename T, int HEAD, int MODE, int WAVES = 4, int GROUPS = 1, bool PARTS = false>
+// KH == 2: the workgroup's four wavefronts hold 64 queries, and every step's 64 keys
+// are shared by two wavefronts of the same 32 queries, 32 keys each; the two
+// (maximum, sum, output) triples are merged through LDS before the epilogue.
+template<typename T, int HEAD, int MODE, int WAVES = 4, int GROUPS = 1, bool PARTS = false,
+    int KH = 1>
 __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1)
 void sdpa_prefill_16bit_kernel(const PrefillParams p)
 {
@@ -148,8 +153,9 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // have no second workgroup to put on a CU: two wavefronts per SIMD (one's
     // softmax beside the other's MFMAs) and half the chain of dependent steps.
     constexpr int QW = WAVES / GROUPS;      // wavefronts that share a key step
-    constexpr int kQRows = QW * 32;
+    constexpr int kQRows = QW / KH * 32;
     constexpr int kThreads = WAVES * 64;
+    constexpr int NB = 2 / KH;              // 32-key blocks of a step that a wavefront takes
     typedef typename T::vec8 vec8;
     constexpr int KSTEPS = HEAD / 16;       // MFMA steps along head for S
     constexpr int DBLOCKS = HEAD / 32;      // 32-row blocks of O^T
@@ -160,6 +166,9 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     constexpr int LOADS = kKeys / ROWS_PER_LOAD;  // load instructions per K (or V) step
     constexpr int LOADS_PER_WAVE = LOADS / QW;
     constexpr int K_BYTES = kKeys * RB;
+    constexpr int NDB = DBLOCKS / KH;       // blocks of O^T a wavefront writes
+    constexpr int RBE = RB / KH;            // bytes of a row it writes
+    constexpr int CPRE = CPR / KH;
     constexpr bool EXPLICIT = (MODE == NNTILE_HIP_MASK_ADDITIVE
             || MODE == NNTILE_HIP_MASK_BOOL);
     static_assert(LOADS_PER_WAVE * QW == LOADS
@@ -169,6 +178,8 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     static_assert(!PARTS || (GROUPS == 2 && !EXPLICIT), "parts: analytic masks, two groups");
     static_assert(WAVES == 4 || (WAVES == 8 && (GROUPS == 2 || !EXPLICIT)),
             "eight wavefronts on 256 queries: analytic masks only");
+    static_assert(KH == 1 || (KH == 2 && WAVES == 4 && GROUPS == 1 && !PARTS && DBLOCKS % 2 == 0),
+            "halved steps: one group of four wavefronts, each left with half of the head");
 
     // Separate arrays, not one: the compiler then knows that the loads
     // streaming into one of them cannot alias the reads of the others and
@@ -186,6 +197,8 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     const int grp = GROUPS > 1 ? (tid >> 6) / QW : 0;      // which key steps
     const int wave = (tid >> 6) - grp * QW;                 // which 32 queries
     const int lds_grp_off = GROUPS > 1 ? __builtin_amdgcn_readfirstlane(grp) * K_BYTES : 0;
+    const int kh = KH > 1 ? __builtin_amdgcn_readfirstlane(wave >> 1) : 0;  // which 32 keys of a step
+    const int rb = KH > 1 ? wave & 1 : wave;                // which 32 of its group's queries
     const int col = lane & 31;      // query within the wavefront / row of a block
     const int half = lane >> 5;
 
@@ -234,7 +247,16 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     }
     // (only where the second group is complete: the places it is dealt to must
     // all be attention workgroups' - those that scan a mask do not count)
-    if(WAVES == 4 && n_att >= 8u * 2u * kCUsPerXCD)
+    if constexpr(KH > 1)
+    {
+        // (at most two workgroups a CU, the second group as long as it comes)
+        const unsigned i = wg >> 3, n = min(n_att >> 3, 2u * kCUsPerXCD);
+        if(i >= kCUsPerXCD && i < n)
+        {
+            wg = ((kCUsPerXCD + n - 1u - i) << 3) | (wg & 7u);
+        }
+    }
+    else if(WAVES == 4 && n_att >= 8u * 2u * kCUsPerXCD)
     {
         const unsigned i = wg >> 3;
         if(i >= kCUsPerXCD && i < 2u * kCUsPerXCD)
@@ -288,9 +310,54 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     }
     const int kvb = kv_entry(b, p.n_batch, p.kv_group);
 
+    // ---- keys and values into this XCD's L2 ----------------------------------------
+    // Workgroups of the same keys on one XCD walk them side by side, and what none of
+    // them has read yet comes from HBM at every step, later than the loop asks for it
+    // ahead.  So each touches a share of the lines first, four a thread at most.
+    constexpr int NT = KH > 1 ? 4 : 1;
+    uint32_t touched[NT];
+    auto touch_keys = [&]() __attribute__((always_inline))
+    {
+        if(p.touch_share > 0)
+        {
+            constexpr int LINES = kKeys * RB / 128;     // of a step's K, and of its V
+            const int order = q_blocks - 1 - qblk;
+            const int idx = p.touch_group > 1
+                ? (order / p.touch_period) * p.touch_group + (b / p.n_batch) % p.touch_group
+                : order / p.touch_period;
+            const int n_lines = idx < p.touch_share ? p.touch_steps * 2 * LINES : 0;
+#pragma unroll
+            for(int i = 0; i < NT; ++i)
+            {
+                const int line = (i * p.touch_share + idx) * kThreads + tid;
+                if(line < n_lines)
+                {
+                    const int st = line / (2 * LINES), in = line % (2 * LINES);
+                    const int kt = p.n_kv_tiles > 1 ? st / p.k_blocks_per_tile : 0;
+                    const int64_t rows = min(p.k_tile, p.k_seq - kt * p.k_tile);
+                    const int64_t at = min((int64_t)(st - kt * p.k_blocks_per_tile) * (kKeys * RB)
+                            + (in % LINES) * 128, rows * RB - 16)
+                        + (int64_t)kvb * (p.kv_rows > 0 ? p.kv_rows : rows) * RB;
+                    touched[i] = *reinterpret_cast<const volatile uint32_t *>(
+                            static_cast<const char *>(in < LINES ? p.K[k_tile0 + kt]
+                                : p.V[k_tile0 + kt]) + at);
+                }
+            }
+        }
+    };
+#pragma unroll
+    for(int i = 0; i < NT; ++i)
+    {
+        touched[i] = 0u;
+    }
+    if constexpr(KH > 1 && !EXPLICIT)
+    {
+        touch_keys();
+    }
+
     const uint16_t *Qt = static_cast<const uint16_t *>(p.Q[q_tile0 + qt])
         + (int64_t)b * q_len * HEAD;
-    const int my_q = q_row0 + wave * 32 + col;          // row within tile
+    const int my_q = q_row0 + rb * 32 + col;            // row within tile
     const bool q_ok = my_q < q_len;
     // the stored logsumexp that the epilogue merges with: requested here, so
     // that its latency passes beside the first loads
@@ -346,7 +413,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                     + (hi - kt_hi * k_tile) / kKeys + 1);
         }
     }
-    const int wave_rel_lo = rel0 + wave * 32;       // first query of the wavefront
+    const int wave_rel_lo = rel0 + rb * 32;         // first query of the wavefront
     const int my_rel = wave_rel_lo + col;
 
     // ---- LDS layout and the lane's fixed addresses ---------------------------
@@ -377,11 +444,12 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         }
     }
     // S operand: lane (col, half) reads row mb*32+col, logical chunk 2*ks+half.
-    uint32_t k_raddr[2][KSTEPS];
+    // (KH == 2: its one block is block kh of the step, and 32 rows change no swizzle)
+    uint32_t k_raddr[NB][KSTEPS];
 #pragma unroll
-    for(int mb = 0; mb < 2; ++mb)
+    for(int mb = 0; mb < NB; ++mb)
     {
-        const int r = mb * 32 + col;
+        const int r = (mb + kh) * 32 + col;
 #pragma unroll
         for(int ks = 0; ks < KSTEPS; ++ks)
         {
@@ -405,8 +473,10 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
 #pragma unroll
         for(int db = 0; db < DBLOCKS; ++db)
         {
-            const int c = 4 * db + 2 * dblk + (r4 >> 1);
-            v_raddr[db] = (uint32_t)(grp * K_BYTES + r * RB + (c ^ swz) * 16
+            // (KH == 2: a wavefront's blocks start with the half of the head that
+            // it is left with after the merge)
+            const int c = 4 * ((db + kh * (DBLOCKS / 2)) % DBLOCKS) + 2 * dblk + (r4 >> 1);
+            v_raddr[db] = (uint32_t)(grp * K_BYTES + (kh * 32 + r) * RB + (c ^ swz) * 16
                     + 8 * (r4 & 1));
         }
     }
@@ -538,7 +608,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // The loads carry the alignment of one element; in a ragged last step a piece
     // that would reach past the row is moved back to end with it and shifted into
     // place when it is used, and what lies past the end is made hidden.
-    constexpr int MW = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 16 : 8;    // dwords per lane and step
+    constexpr int MW = ((MODE == NNTILE_HIP_MASK_ADDITIVE) ? 16 : 8) / KH;     // dwords per lane and step
     enum { MASK_ZERO = 0, MASK_HIDDEN = 1, MASK_MIXED = 2 };
     uint32_t mraw[MW];
 #pragma unroll
@@ -546,14 +616,14 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     {
         mraw[i] = 0;
     }
-    constexpr int PW = MW / 4;                  // dwords of a piece of eight elements
+    constexpr int PW = MW / (2 * NB);           // dwords of a piece of eight elements
     constexpr int MASK_RB = 32 * 8 * PW / 16;   // bytes of 32 elements
     constexpr int MASK_RPL = 256 / MASK_RB;     // such rows per 256-byte line of LDS banks
     const int piece = lane & 3, piece_row = lane >> 2;
     // first key of load i's piece within the step, as loaded and as meant
     auto piece_key0 = [&](int i) -> int
     {
-        return (i >> 1) * 32 + 8 * piece;
+        return ((i >> 1) + kh) * 32 + 8 * piece;
     };
     auto piece_start = [&](int key0, int keys) -> int
     {
@@ -572,13 +642,13 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         for(int h = 0; h < 2; ++h)
         {
             // (rows past the end of the tile re-read its last one)
-            const int row = min(q_row0 + wave * 32 + 16 * h + piece_row, q_len - 1);
+            const int row = min(q_row0 + rb * 32 + 16 * h + piece_row, q_len - 1);
             mp[h] = static_cast<const M *>(p.mask) + (int64_t)row * p.mask_ld + kb * kKeys;
         }
         if(k_seq >= 8)
         {
 #pragma unroll
-            for(int i = 0; i < 4; ++i)
+            for(int i = 0; i < 2 * NB; ++i)
             {
                 const int at = keys >= kKeys ? piece_key0(i) : piece_start(piece_key0(i), keys);
                 const V v = *reinterpret_cast<const V_any *>(mp[i & 1] + at);
@@ -616,7 +686,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         constexpr int EB = 32 * PW / 8;         // bits of an element
         constexpr uint32_t HIDDEN = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? T::kNegInfPair : 0u;
 #pragma unroll
-        for(int i = 0; i < 4; ++i)
+        for(int i = 0; i < 2 * NB; ++i)
         {
             const int key0 = piece_key0(i);
             const int back = key0 - piece_start(key0, keys);
@@ -651,7 +721,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         __shared__ __attribute__((aligned(16))) char lds_mask[EXPLICIT ? WAVES * 32 * MASK_RB : 16];
         char *mine = lds_mask + (tid >> 6) * (32 * MASK_RB);
 #pragma unroll
-        for(int mb = 0; mb < 2; ++mb)
+        for(int mb = 0; mb < NB; ++mb)
         {
 #pragma unroll
             for(int h = 0; h < 2; ++h)
@@ -782,10 +852,12 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         // bit s: some value of step s (steps >= 63 share bit 63) is not open / not hidden
         unsigned long long not_open = 0ull, not_hidden = 0ull;
         bool scanned = false;
+        // the block of 128 rows that the words of a scan done for everybody are about
+        const int scan_blk = q_row0 / nntile_hip::kQRows;
         if(n_steps > 0 && p.mask_bits != nullptr && p.n_scan_wgs == 0)
         {
             // the scan was done once for all batch entries before the launch
-            const unsigned long long *w = p.mask_bits + (int64_t)qb * (kMaskBitWords * kMaskBitSplits);
+            const unsigned long long *w = p.mask_bits + (int64_t)scan_blk * (kMaskBitWords * kMaskBitSplits);
 #pragma unroll
             for(int sp = 0; sp < kMaskBitSplits; ++sp)
             {
@@ -822,7 +894,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 const int i = lane & 7;
                 const bool has_word = i < kMaskBitWords;
                 unsigned long long *e = p.mask_bits
-                    + ((int64_t)qb * kMaskBitSplits + (lane >> 3)) * kMaskBitWords
+                    + ((int64_t)scan_blk * kMaskBitSplits + (lane >> 3)) * kMaskBitWords
                     + (has_word ? i : 0);
                 const unsigned long long t0 = wall_clock64();
                 unsigned long long word;
@@ -868,9 +940,12 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 && p.mask_ld * ES * kQRows < (int64_t)(1 << 30))
         {
             __shared__ unsigned long long scan_words[2 * WAVES];
+            // (rows as in a scan done for everybody: a call's bits do not depend on which
+            // of the two it has)
+            const int scan_row0 = scan_blk * nntile_hip::kQRows;
             mask_scan_steps<ES, WAVES, kKeys>(static_cast<const char *>(p.mask)
-                    + (int64_t)q_row0 * p.mask_ld * ES, (uint32_t)(p.mask_ld * ES),
-                    min(kQRows, q_len - q_row0), k_seq * ES, 0, (k_seq + kKeys - 1) / kKeys,
+                    + (int64_t)scan_row0 * p.mask_ld * ES, (uint32_t)(p.mask_ld * ES),
+                    min(nntile_hip::kQRows, q_len - scan_row0), k_seq * ES, 0, (k_seq + kKeys - 1) / kKeys,
                     OPEN, HIDDEN, scan_words, not_open, not_hidden);
             scanned = true;
         }
@@ -964,7 +1039,16 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             mask_fetch(cur.kb, cur.rows_left);
         }
     }
+    if constexpr(KH > 1 && EXPLICIT)
+    {
+        touch_keys();       // (what the mask hides from everyone is not wanted)
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for(int i = 0; i < NT; ++i)
+    {
+        asm volatile("" :: "v"(touched[i]));
+    }
     __syncthreads();
     PF_STAMP(1);
 #ifdef NNTILE_PF_TRACE
@@ -1003,7 +1087,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         // the other group's last one and this group has none in this round
         const bool idle = (GROUPS > 1 && g >= n_steps)
             || (EXPLICIT ? (mask_class == MASK_HIDDEN)
-            : ((MODE == NNTILE_HIP_MASK_CAUSAL) && (kg0 > wave_rel_lo + 31)));
+            : ((MODE == NNTILE_HIP_MASK_CAUSAL) && (kg0 + kh * 32 > wave_rel_lo + 31)));
 
         // ---- loads of the next step into the other buffer ----------------------
         // (every wavefront passed the barrier that ended step g-1, so nobody
@@ -1016,13 +1100,13 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             advance(nxt);
         }
 
-        uint32_t pk[2][8];
+        uint32_t pk[NB][8];
         if(!idle)
         {
             // ---- S^T = K Q^T -------------------------------------------------
-            f32x16 s[2];
+            f32x16 s[NB];
 #pragma unroll
-            for(int mb = 0; mb < 2; ++mb)
+            for(int mb = 0; mb < NB; ++mb)
             {
 #pragma unroll
                 for(int r = 0; r < 16; ++r)
@@ -1040,13 +1124,13 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             NNTILE_PHASE(1)
 
             // ---- mask ---------------------------------------------------------
-            // register r of block mb holds key  mb*32 + 8*(r/4) + 4*half + r%4
+            // register r of block mb holds key  (mb + kh)*32 + 8*(r/4) + 4*half + r%4
             if(EXPLICIT)
             {
                 if(mask_class == MASK_MIXED)
                 {
 #pragma unroll
-                    for(int i = 0; i < 8; ++i)
+                    for(int i = 0; i < 4 * NB; ++i)
                     {
                         // group i: block i/4, registers 4*(i%4) .. +3
                         const int mb = i >> 2, r0 = 4 * (i & 3);
@@ -1079,7 +1163,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             {
                 const bool ragged = keys_here < kKeys;
                 const bool diagonal = (MODE == NNTILE_HIP_MASK_CAUSAL)
-                    && (kg0 + kKeys - 1 > wave_rel_lo);
+                    && (kg0 + (kh + NB) * 32 - 1 > wave_rel_lo);
                 if(ragged || diagonal)
                 {
                     // last visible key of this step for this lane's query
@@ -1088,8 +1172,9 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                     {
                         lim = min(lim, my_rel - kg0);
                     }
+                    lim -= kh * 32;
 #pragma unroll
-                    for(int mb = 0; mb < 2; ++mb)
+                    for(int mb = 0; mb < NB; ++mb)
                     {
 #pragma unroll
                         for(int r = 0; r < 16; ++r)
@@ -1108,7 +1193,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             // ---- online softmax -------------------------------------------------
             float mx = neg_inf();
 #pragma unroll
-            for(int mb = 0; mb < 2; ++mb)
+            for(int mb = 0; mb < NB; ++mb)
             {
 #pragma unroll
                 for(int r = 0; r < 16; ++r)
@@ -1143,7 +1228,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             // would sum a packed pair waits for the matrix unit)
             float rs0 = 0.0f, rs1 = 0.0f;
 #pragma unroll
-            for(int mb = 0; mb < 2; ++mb)
+            for(int mb = 0; mb < NB; ++mb)
             {
 #pragma unroll
                 for(int r = 0; r < 16; r += 2)
@@ -1168,7 +1253,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         if(!idle)
         {
 #pragma unroll
-            for(int t = 0; t < 4; ++t)
+            for(int t = 0; t < 2 * NB; ++t)
             {
                 const int mb = t >> 1, tt = t & 1;
                 const u32x4 praw = {pk[mb][4 * tt], pk[mb][4 * tt + 1],
@@ -1258,8 +1343,8 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             constexpr bool DO_S = decltype(do_s_tag)::value;
             constexpr bool DO_PV = decltype(do_pv_tag)::value;
             constexpr bool DO_SM = decltype(do_sm_tag)::value;
-            constexpr bool DO_FETCH = decltype(do_fetch_tag)::value;
-            static_assert(2 * LOADS_PER_WAVE <= NSLOT / 2, "one load every second slot");
+            constexpr int DO_FETCH = decltype(do_fetch_tag)::value;    // 0, or one load every DO_FETCH slots
+            static_assert(2 * LOADS_PER_WAVE * DO_FETCH <= NSLOT, "the loads fit the slots");
             auto fetch_piece = [&](int i) __attribute__((always_inline))
             {
                 if(i < LOADS_PER_WAVE)
@@ -1388,9 +1473,9 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                         item(it);
                     }
                 }
-                if(DO_FETCH && (sl & 1))
+                if(DO_FETCH > 0 && sl % max(DO_FETCH, 1) == DO_FETCH - 1)
                 {
-                    fetch_piece(sl >> 1);
+                    fetch_piece(sl / max(DO_FETCH, 1));
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -1440,6 +1525,8 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         };
         typedef std::integral_constant<bool, true> Yes;
         typedef std::integral_constant<bool, false> No;
+        typedef std::integral_constant<int, 0> NoFetch;
+        typedef std::integral_constant<int, (KH > 1 ? 1 : 2)> Spread;
 
         // scores of sub-block (0, 0)
 #pragma unroll
@@ -1479,7 +1566,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         auto fast_step = [&](int g, auto buf_tag, auto spread_tag) __attribute__((always_inline))
         {
             constexpr int BUF = decltype(buf_tag)::value;
-            body(Yes{}, Yes{}, Yes{}, No{}, BUF ? lds_k1 : lds_k0, 1, BUF ? lds_v0 : lds_v1, 1,
+            body(Yes{}, Yes{}, Yes{}, NoFetch{}, BUF ? lds_k1 : lds_k0, 1, BUF ? lds_v0 : lds_v1, 1,
                     sa, sb, no_dst, no_dst);
             if(decltype(spread_tag)::value)
             {
@@ -1487,7 +1574,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 __syncthreads();
                 char *kdst = (BUF ? lds_k1 : lds_k0) + lds_grp_off + wave_u * LOADS_PER_WAVE * 1024;
                 char *vdst = (BUF ? lds_v0 : lds_v1) + lds_grp_off + wave_u * LOADS_PER_WAVE * 1024;
-                body(Yes{}, Yes{}, Yes{}, Yes{}, BUF ? lds_k0 : lds_k1, 0,
+                body(Yes{}, Yes{}, Yes{}, Spread{}, BUF ? lds_k0 : lds_k1, 0,
                         BUF ? lds_v1 : lds_v0, 0, sb, sa, kdst, vdst);
                 c1 = c2;
                 advance(c2);
@@ -1495,29 +1582,103 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             else
             {
                 mid_step(g, buf_tag);
-                body(Yes{}, Yes{}, Yes{}, No{}, BUF ? lds_k0 : lds_k1, 0,
+                body(Yes{}, Yes{}, Yes{}, NoFetch{}, BUF ? lds_k0 : lds_k1, 0,
                         BUF ? lds_v1 : lds_v0, 0, sb, sa, no_dst, no_dst);
             }
             advance(cur);
         };
-        // step 0: there is no output yet in its first half
-        body(Yes{}, No{}, Yes{}, No{}, lds_k0, 1, lds_v1, 1, sa, sb, no_dst, no_dst);
-        mid_step(0, std::integral_constant<int, 0>{});
-        body(Yes{}, Yes{}, Yes{}, No{}, lds_k1, 0, lds_v0, 0, sb, sa, no_dst, no_dst);
-        advance(cur);
-        int g = 1;
-        for(; g + 1 < n_fast && g + 3 < n_spread; g += 2)
+        if constexpr(KH > 1)
         {
-            fast_step(g, std::integral_constant<int, 1>{}, Yes{});
-            fast_step(g + 1, std::integral_constant<int, 0>{}, Yes{});
-        }
-        // the last steps, whose successors may be incomplete or absent
-        for(; g < n_fast; g += 2)
-        {
-            fast_step(g, std::integral_constant<int, 1>{}, No{});
-            if(g + 1 < n_fast)
+            // A step is one sub-block of every wavefront: body g takes the softmax of
+            // step g, the scores of step g+1 and the output of step g-1.  K(g+2) takes
+            // the buffer of K(g), whose scores were taken a body ago, and V(g) the one
+            // of V(g-2); both are waited for at the end of the body.
+            auto end_body = [&]() __attribute__((always_inline))
             {
-                fast_step(g + 1, std::integral_constant<int, 0>{}, No{});
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();
+                advance(cur);
+            };
+            auto one_step = [&](int g, auto buf_tag, auto spread_tag) __attribute__((always_inline))
+            {
+                constexpr int BUF = decltype(buf_tag)::value;
+                char *kbuf = BUF ? lds_k1 : lds_k0, *vbuf = BUF ? lds_v1 : lds_v0;
+                const char *k_next = BUF ? lds_k0 : lds_k1, *v_prev = BUF ? lds_v0 : lds_v1;
+                f32x16 &s_cur = BUF ? sb : sa, &s_nxt = BUF ? sa : sb;
+                if(decltype(spread_tag)::value)
+                {
+                    const int at = wave_u * LOADS_PER_WAVE * 1024;
+                    c1 = cur;
+                    body(Yes{}, Yes{}, Yes{}, Spread{}, k_next, 0, v_prev, 0, s_cur, s_nxt,
+                            kbuf + at, vbuf + at);
+                    advance(c2);
+                }
+                else
+                {
+                    fetch_v(cur, vbuf);
+                    if(g + 2 <= n_fast && g + 2 < n_steps)
+                    {
+                        fetch_k(c2, kbuf);
+                        advance(c2);
+                    }
+                    body(Yes{}, Yes{}, Yes{}, NoFetch{}, k_next, 0, v_prev, 0, s_cur, s_nxt,
+                            no_dst, no_dst);
+                }
+                end_body();
+            };
+            // (every wavefront has taken the scores of step 0)
+            __syncthreads();
+            if(2 <= n_fast && 2 < n_steps)
+            {
+                fetch_k(c2, lds_k0);
+                advance(c2);
+            }
+            body(Yes{}, No{}, Yes{}, NoFetch{}, lds_k1, 0, lds_v0, 0, sa, sb, no_dst, no_dst);
+            end_body();
+            int g = 1;
+            for(; g + 3 <= n_fast && g + 3 < n_spread; g += 2)
+            {
+                one_step(g, std::integral_constant<int, 1>{}, Yes{});
+                one_step(g + 1, std::integral_constant<int, 0>{}, Yes{});
+            }
+            for(; g < n_fast; g += 2)
+            {
+                one_step(g, std::integral_constant<int, 1>{}, No{});
+                if(g + 1 < n_fast)
+                {
+                    one_step(g + 1, std::integral_constant<int, 0>{}, No{});
+                }
+            }
+            // cur is step n_fast now; its K is there where the general loop takes it
+            // up, its V takes the buffer of V(n_fast-2)
+            if(n_fast < n_steps)
+            {
+                fetch_v(cur, (n_fast & 1) ? lds_v1 : lds_v0);
+            }
+            c1 = cur;
+            advance(c1);
+        }
+        else
+        {
+            // step 0: there is no output yet in its first half
+            body(Yes{}, No{}, Yes{}, NoFetch{}, lds_k0, 1, lds_v1, 1, sa, sb, no_dst, no_dst);
+            mid_step(0, std::integral_constant<int, 0>{});
+            body(Yes{}, Yes{}, Yes{}, NoFetch{}, lds_k1, 0, lds_v0, 0, sb, sa, no_dst, no_dst);
+            advance(cur);
+            int g = 1;
+            for(; g + 1 < n_fast && g + 3 < n_spread; g += 2)
+            {
+                fast_step(g, std::integral_constant<int, 1>{}, Yes{});
+                fast_step(g + 1, std::integral_constant<int, 0>{}, Yes{});
+            }
+            // the last steps, whose successors may be incomplete or absent
+            for(; g < n_fast; g += 2)
+            {
+                fast_step(g, std::integral_constant<int, 1>{}, No{});
+                if(g + 1 < n_fast)
+                {
+                    fast_step(g + 1, std::integral_constant<int, 0>{}, No{});
+                }
             }
         }
         if(EXPLICIT && n_fast < n_steps)
@@ -1527,11 +1688,11 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         // drain: the output of the last sub-block
         if((n_fast - 1) & 1)
         {
-            body(No{}, Yes{}, No{}, No{}, lds_k0, 0, lds_v1, 1, sb, sa, no_dst, no_dst);
+            body(No{}, Yes{}, No{}, NoFetch{}, lds_k0, 0, lds_v1, NB - 1, sb, sa, no_dst, no_dst);
         }
         else
         {
-            body(No{}, Yes{}, No{}, No{}, lds_k0, 0, lds_v0, 1, sb, sa, no_dst, no_dst);
+            body(No{}, Yes{}, No{}, NoFetch{}, lds_k0, 0, lds_v0, NB - 1, sb, sa, no_dst, no_dst);
         }
         g_first = n_fast;
         nxt = c1;
@@ -1612,6 +1773,50 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         m_run = m_new;
     }
 
+    // ---- the two halves of a step's keys are put together ------------------------
+    // Wavefronts w and w + 2 hold the same queries: each writes the half of its output
+    // that the other is left with, and takes its own.
+    if constexpr(KH > 1)
+    {
+        static_assert((16 * NDB + 2) * 256 <= K_BYTES - 32 * RBE,
+                "the triple and the epilogue's staging rows share an array");
+        auto array = [&](int w) __attribute__((always_inline)) -> char *
+        {
+            return w == 0 ? lds_k0 : w == 1 ? lds_k1 : w == 2 ? lds_v0 : lds_v1;
+        };
+        float *mine = reinterpret_cast<float *>(array(wave)) + lane;
+        const float *theirs = reinterpret_cast<const float *>(array(wave ^ 2)) + lane;
+#pragma unroll
+        for(int db = 0; db < NDB; ++db)
+        {
+#pragma unroll
+            for(int r = 0; r < 16; ++r)
+            {
+                mine[(16 * db + r) * 64] = o[NDB + db][r];
+            }
+        }
+        mine[16 * NDB * 64] = m_run;
+        mine[(16 * NDB + 1) * 64] = l_run;
+        __syncthreads();
+        const float m_other = theirs[16 * NDB * 64];
+        const float l_other = theirs[(16 * NDB + 1) * 64];
+        const float m_new = fmaxf(m_run, m_other);
+        // (a half that saw no visible key has maximum -inf and weight 0)
+        const float a_mine = (m_run == neg_inf()) ? 0.0f : fast_exp2((m_run - m_new) * c);
+        const float a_other = (m_other == neg_inf()) ? 0.0f : fast_exp2((m_other - m_new) * c);
+#pragma unroll
+        for(int db = 0; db < NDB; ++db)
+        {
+#pragma unroll
+            for(int r = 0; r < 16; ++r)
+            {
+                o[db][r] = o[db][r] * a_mine + theirs[(16 * db + r) * 64] * a_other;
+            }
+        }
+        l_run = l_run * a_mine + l_other * a_other;
+        m_run = m_new;
+    }
+
     // ---- epilogue: normalise, merge into the running (lse, A) ----------------
     const float l_tot = sum_across_halves(l_run);
     // no visible key for this query.  A score that is NaN makes the sum NaN: such
@@ -1658,7 +1863,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     {
         merge_weights(lse_old, lse_new, w_old, w_new, lse_out);
     }
-    if(live && half == 0)
+    if(live && half == 0 && kh == 0)
     {
         *lse_ptr = lse_out;
     }
@@ -1679,14 +1884,16 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     char *xch = GROUPS > 1
         ? (wave == 0 ? lds_k0 : wave == 1 ? lds_k1 : wave == 2 ? lds_v0 : lds_v1)
             + (K_BYTES * GROUPS - 32 * RB)
+        : KH > 1 ? (wave == 0 ? lds_k0 : wave == 1 ? lds_k1 : wave == 2 ? lds_v0 : lds_v1)
+            + (K_BYTES - 32 * RBE)
         : ((wave >> 1) == 0 ? lds_k0 : (wave >> 1) == 1 ? lds_k1
             : (wave >> 1) == 2 ? lds_v0 : lds_v1) + (wave & 1) * 32 * RB;
     const uint64_t live_rows = __builtin_amdgcn_ballot_w64(live && half == 0);
-    constexpr int ROWS_PER_ST = 1024 / RB;      // rows one load or store instruction covers
+    constexpr int ROWS_PER_ST = 1024 / RBE;     // rows one load or store instruction covers
     constexpr int N_ST = 32 / ROWS_PER_ST;
-    const int st_row = lane / CPR, st_c = lane % CPR;
+    const int st_row = lane / CPRE, st_c = lane % CPRE;
     char *Abase = static_cast<char *>(p.A[q_tile0 + qt])
-        + ((int64_t)b * q_len + q_row0 + wave * 32) * RB;
+        + ((int64_t)b * q_len + q_row0 + rb * 32) * RB + kh * RBE;
     const bool merge = __builtin_amdgcn_ballot_w64(live && w_old != 0.0f) != 0;
     if(merge)
     {
@@ -1698,23 +1905,23 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             const int r = i * ROWS_PER_ST + st_row;
             const bool there = (live_rows >> r) & 1;
             old[i] = *reinterpret_cast<const u32x4 *>(
-                    Abase + (there ? (int64_t)r * RB : -(int64_t)wave * 32 * RB) + st_c * 16);
+                    Abase + (there ? (int64_t)r * RB : -(int64_t)rb * 32 * RB) + st_c * 16);
         }
 #pragma unroll
         for(int i = 0; i < N_ST; ++i)
         {
             const int r = i * ROWS_PER_ST + st_row;
-            *reinterpret_cast<u32x4 *>(xch + r * RB + (st_c ^ (r % CPR)) * 16) = old[i];
+            *reinterpret_cast<u32x4 *>(xch + r * RBE + (st_c ^ (r % CPRE)) * 16) = old[i];
         }
     }
 #pragma unroll
-    for(int db = 0; db < DBLOCKS; ++db)
+    for(int db = 0; db < NDB; ++db)
     {
 #pragma unroll
         for(int rg = 0; rg < 4; ++rg)
         {
-            const int cpos = (db * 4 + rg) ^ (col % CPR);
-            u32x2 *at = reinterpret_cast<u32x2 *>(xch + col * RB + cpos * 16 + 8 * half);
+            const int cpos = (db * 4 + rg) ^ (col % CPRE);
+            u32x2 *at = reinterpret_cast<u32x2 *>(xch + col * RBE + cpos * 16 + 8 * half);
             float v[4];
 #pragma unroll
             for(int e = 0; e < 4; ++e)
@@ -1742,7 +1949,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     {
         const int r = i * ROWS_PER_ST + st_row;
         const u32x4 v = *reinterpret_cast<const u32x4 *>(
-                xch + r * RB + (st_c ^ (r % CPR)) * 16);
+                xch + r * RBE + (st_c ^ (r % CPRE)) * 16);
         if((live_rows >> r) & 1)
         {
             *reinterpret_cast<u32x4 *>(Abase + (int64_t)r * RB + st_c * 16) = v;
@@ -1756,11 +1963,32 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
 
 template<typename T, int HEAD>
 static int launch_mode(hipStream_t stream, const PrefillParams &p, int mode,
-        dim3 grid, bool wide, bool key_split)
+        dim3 grid, bool wide, bool key_split, bool halved)
 {
     constexpr int kThreads = 256;
     if constexpr(HEAD >= 64)
     {
+        if(halved)
+        {
+            auto launch = [&](auto kernel) -> int
+            {
+                hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, p);
+                return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+            };
+            switch(mode)
+            {
+                case NNTILE_HIP_MASK_ADDITIVE:
+                    return launch(sdpa_prefill_16bit_kernel<T, HEAD, NNTILE_HIP_MASK_ADDITIVE, 4, 1, false, 2>);
+                case NNTILE_HIP_MASK_NONE:
+                    return launch(sdpa_prefill_16bit_kernel<T, HEAD, NNTILE_HIP_MASK_NONE, 4, 1, false, 2>);
+                case NNTILE_HIP_MASK_CAUSAL:
+                    return launch(sdpa_prefill_16bit_kernel<T, HEAD, NNTILE_HIP_MASK_CAUSAL, 4, 1, false, 2>);
+                case NNTILE_HIP_MASK_BOOL:
+                    return launch(sdpa_prefill_16bit_kernel<T, HEAD, NNTILE_HIP_MASK_BOOL, 4, 1, false, 2>);
+                default:
+                    return NNTILE_HIP_EINVAL;
+            }
+        }
         if(key_split)
         {
             switch(mode)
@@ -1891,7 +2119,8 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
     }
     const int64_t es = additive ? 2 : 1;
     const int64_t row_bytes = p.k_seq * es;
-    const int64_t table_bytes = (int64_t)p.q_blocks_per_tile * kMaskBitSplits
+    const int64_t scan_blocks = (p.q_seq + kQRows - 1) / kQRows;
+    const int64_t table_bytes = scan_blocks * kMaskBitSplits
         * (kMaskBitWords * (int64_t)sizeof(unsigned long long));
     if(row_bytes < 16 || p.mask_ld * es * kQRows >= (int64_t)(1 << 30)
             || reinterpret_cast<uintptr_t>(scratch) % 8 != 0
@@ -1900,7 +2129,7 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
         return NNTILE_HIP_OK;
     }
     auto *table = static_cast<unsigned long long *>(scratch);
-    const dim3 grid((unsigned)(p.q_blocks_per_tile * kMaskBitSplits));
+    const dim3 grid((unsigned)(scan_blocks * kMaskBitSplits));
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if(hipStreamIsCapturing(stream, &capturing) != hipSuccess)
     {
@@ -1944,9 +2173,113 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
     return NNTILE_HIP_OK;
 }
 
-// Key steps from which a head of 64 under a mask given as values is walked by two
-// groups of wavefronts (see below)
-constexpr int64_t kSplitSteps64 = 16;
+// How the keys of a launch lie on the XCDs: `steps` key steps an entry of the batch, of
+// which `fit` leading ones, of all entries that an XCD works on, have room in 3 of its
+// L2's 4 MiB; every `period`-th query block of an entry sits on the same XCD, and there
+// `group` heads share their keys.
+struct KeysOnXCD
+{
+    int64_t steps, fit;
+    int period, group;
+};
+
+static KeysOnXCD keys_on_xcd(const PrefillParams &p, int head)
+{
+    KeysOnXCD r;
+    const int64_t batch_all = (int64_t)p.batch * p.n_slabs;
+    const int64_t last_keys = p.k_seq - (p.n_kv_tiles - 1) * p.k_tile;
+    r.steps = (p.n_kv_tiles - 1) * ((p.k_tile + kKeys - 1) / kKeys) + (last_keys + kKeys - 1) / kKeys;
+    r.period = 8;
+    while(r.period > 1 && batch_all * (r.period / 2) % 8 == 0)
+    {
+        r.period /= 2;
+    }
+    // (an XCD has whole groups of heads where the entries come in eights: xcd_remap)
+    r.group = p.n_slabs == 1 && p.batch % (8 * (int64_t)p.n_batch * p.kv_group) == 0 ? p.kv_group : 1;
+    const int64_t entries = (batch_all * r.period + 7) / 8;
+    r.fit = ((int64_t)3 << 20) * r.group / (entries * (kKeys * 2 * 2) * head);
+    return r;
+}
+
+// From how many key steps on the first touch of the keys pays (us, touched / not, inputs
+// of other calls in between; bf16, head 128): 8 entries of 500 keys 11.2 / 11.0, of 1024
+// 14.9 / 15.7 (without a mask the same), of 2048 causal 23.1 / 28.8, 4 of 4096 37.9 / 50.6;
+// head 64, 8 of 1024 12.0 / 12.5, 4 of 4096 30.4 / 34.6.  128 queries a workgroup lose
+// by it: 32 x 1024 causal 24.2 / 21.8, 12 x 1500 27.5 / 26.0.
+constexpr int64_t kTouchSteps = 16;
+// ... with masks given as values and more than 256 workgroups at head 128: 24 x 1024
+// without a hidden key 26.7 / 25.4, 16 x 1500 under a causal mask 26.9 / 31.5
+constexpr int64_t kTouchStepsMask = 24;
+
+// Steps from which rectangular calls with an analytic mask may be halved (see below)
+constexpr int64_t kHalvedSteps = 8;
+
+// Workgroups of 64 queries whose wavefronts halve the key steps between them: launches
+// of at most 256 workgroups of 128 queries.  Twice the workgroups with half of the chain
+// each, on CUs that would stand empty (up to 256 of them), or two on a CU, long
+// beside short (causal); but each step comes into LDS twice as often for its MFMAs, and with
+// two such workgroups a CU and no mask that is what bounds the launch.  us before /
+// now, bf16, inputs of other calls in between:
+//   up to 256 workgroups, head 128: 8 x 128 causal 8.1 / 6.8, 4 x 300 11.7 / 9.0, 8 x 500
+//   15.1 / 11.0, 8 x 1024 19.9 / 14.9, 8 x 2048 30.8 / 23.1, open 31.1 / 25.2, 4 x 4096
+//   50.5 / 37.9, open 51.1 / 43.4; head 64: 8 x 500 10.6 / 8.9, 4 x 4096 37.0 / 30.4; masks
+//   as values: 4 x 128 11.4 / 9.5, 8 x 500 17.6 / 14.2, open 17.0 / 14.0, a window 15.6 / 12.5,
+//   hidden 4.2 / 4.2.  Not where the keys of an open launch outgrow the L2: 1 x 16384
+//   171.6 / 177.3.
+//   257 to 512, causal: 32 x 700 18.1 / 16.5, 32 x 1024 21.8 / 20.8, 8 x 4096 53.3 / 47.3;
+//   head 64 15.7 / 14.1, 38.1 / 33.2; 200 x 128 of head 128 10.0 / 9.3.  Open: 32 x 1024
+//   24.4 / 26.6.
+//   257 to 512, masks as values: what they hide is not known here.  Head 64, 36 x 500:
+//   causal 15.5 / 13.2, open 15.0 / 14.2, hidden 4.5 / 4.6; 32 x 1024 21.8 / 18.3, 20.8 / 20.1,
+//   4.5 / 5.1; 9 x 2048, whose keys outgrow the L2, 27.0 / 29.4, 27.8 / 30.0.  Head 128,
+//   32 x 1024: causal 27.6 / 24.1, open 27.3 / 30.0, hidden 5.0 / 6.4: not; 16 x 1500 34.7 / 26.9,
+//   34.5 / 34.9, 6.2 / 6.4, 16 x 2048 41.6 / 33.4, 45.4 / 46.9, 8.3 / 8.6; 20 x 1500, which outgrows
+//   the L2, 35.9 / 31.0, 36.2 / 40.1: not.
+static bool halved_is_faster(const PrefillParams &p, int head, int mode)
+{
+    const int64_t tiles = (int64_t)p.batch * p.n_slabs * p.n_q_tiles;
+    constexpr int64_t kCUs = 8 * kCUsPerXCD;
+    const int64_t n_wg = tiles * ((p.q_tile + kQRows / 2 - 1) / (kQRows / 2));
+    if(tiles * ((p.q_tile + kQRows - 1) / kQRows) > kCUs)
+    {
+        return false;
+    }
+    const KeysOnXCD keys = keys_on_xcd(p, head);
+    const bool rule = mode == NNTILE_HIP_MASK_CAUSAL || mode == NNTILE_HIP_MASK_NONE;
+    // Rectangular calls of few steps are left to the other forms, so that what one
+    // computes does not depend on how many entries share its launch.
+    if(rule && p.q_seq != p.k_seq && keys.steps < kHalvedSteps)
+    {
+        return false;
+    }
+    switch(mode)
+    {
+        case NNTILE_HIP_MASK_CAUSAL:
+            // (beyond 256 workgroups where the rule hides enough to make long and short
+            // ones: 64 heads, 333 queries behind 1500 keys 33.9 / 36.8)
+            return n_wg <= kCUs || p.q_pos0 + p.causal_offset - p.k_pos0 < p.k_seq / 2;
+        case NNTILE_HIP_MASK_NONE:
+            return n_wg <= kCUs && (keys.steps < 2 * kTouchSteps || 2 * keys.fit >= keys.steps);
+        default:
+            return n_wg <= kCUs || (keys.steps >= kTouchStepsMask ? keys.fit >= keys.steps : head == 64);
+    }
+}
+
+// Which lines of K and V the workgroups of a launch touch before they begin.
+static void set_touch(PrefillParams &p, int head, int mode, int64_t n_wg)
+{
+    const KeysOnXCD keys = keys_on_xcd(p, head);
+    const bool rule = mode == NNTILE_HIP_MASK_CAUSAL || mode == NNTILE_HIP_MASK_NONE;
+    const int64_t share = (int64_t)p.n_q_tiles * p.q_blocks_per_tile / keys.period * keys.group;
+    if(keys.steps >= (rule || head == 64 || n_wg <= 8 * kCUsPerXCD ? kTouchSteps : kTouchStepsMask)
+            && 3 * keys.fit >= keys.steps && share > 1)
+    {
+        p.touch_share = (int)share;
+        p.touch_period = keys.period;
+        p.touch_group = keys.group;
+        p.touch_steps = (int)std::min(keys.steps, keys.fit);
+    }
+}
 
 // Host launcher shared by the tile and grid entry points.  p must be fully
 // filled except for the block counts and the remap flag.  scan_scratch: device
@@ -1971,7 +2304,10 @@ int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head,
         wide = mode == NNTILE_HIP_MASK_CAUSAL ? n_w >= 512
             : (n_w >= 256 && (n_w % 256 == 0 || n_w >= 1024));
     }
-    const int q_rows = wide ? 256 : kQRows;
+    const bool can_halve = (head == 64 || head == 128) && !wide;
+    const bool halved = can_halve
+        && (p.form == 3 || (p.form == 0 && halved_is_faster(p, head, mode)));
+    const int q_rows = wide ? 256 : halved ? kQRows / 2 : kQRows;
     p.q_blocks_per_tile = (int)((p.q_tile + q_rows - 1) / q_rows);
     p.k_blocks_per_tile = (int)((p.k_tile + kKeys - 1) / kKeys);
     const int64_t batch_all = (int64_t)p.batch * p.n_slabs;
@@ -1983,22 +2319,23 @@ int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head,
     // Two groups of four wavefronts per workgroup, each taking every second
     // key step (p.form == 2, or by itself): when the launch has at most one
     // 128-query workgroup per CU, so that a CU would otherwise hold one wavefront
-    // per SIMD, and enough key steps to share.  Analytic masks: 3-8 % at 1024 keys and
-    // 256 workgroups, 12-20 % on longer rows or fewer workgroups.  Masks given as values, head 128:
-    // 1024 keys 21.5 us with four wavefronts, 22.6 with two groups (8 heads; hidden
-    // 3.9 / 5.0, causal 22.9 / 23.3), 4096 keys 7-11 % less; head 64: 500 keys 13.2 /
-    // 13.3 (12 heads), 777 17.5 / 17.5, 1024 17.2 / 16.1, causal 18.3 / 16.6, hidden 3.5
-    // / 3.9 (8 heads), 1500 24.2 / 21.4, causal 24.5 / 20.7.
-    const bool can_split = (head == 64 || head == 128) && !wide;
+    // per SIMD, is none of those that halve the steps, and has enough key steps to share.
+    // Without a mask: as fast at 1024 keys, 12-20 % less on longer rows (head 64: 3-8 % less at
+    // 1024 keys); shorter rows lose by it (head 128, 36 x 512 14.1 / 15.9, 4 x 300 11.0 / 12.6; head
+    // 64 10.7 / 11.2, 8.7 / 9.3).  Masks
+    // given as values, head 128: 1024 keys 25.3 us with four wavefronts, 28.6 with two
+    // groups (32 heads), 4096 keys 7-11 % less; head 64: 2048 keys 28.8 / 28.2 (16 heads).
+    const bool can_split = can_halve && !halved;
     const bool explicit_mask = mode == NNTILE_HIP_MASK_ADDITIVE || mode == NNTILE_HIP_MASK_BOOL;
-    // (from 16 steps: the scanning workgroups counted, whether or not this call has
-    // any - what a call computes does not depend on its scratch)
-    const int64_t n_scan = p.n_q_tiles * (int64_t)p.q_blocks_per_tile * kMaskBitSplits;
-    const bool split_64 = head == 64 && p.k_seq >= kSplitSteps64 * kKeys
-        && n_wg + n_scan <= 8 * (int64_t)kCUsPerXCD;
+    // (head 64 under such a mask comes here with 24 steps and more)
     const bool key_split = can_split && (p.form == 2
             || (p.form == 0 && n_wg <= 8 * (int64_t)kCUsPerXCD
-                && (p.k_seq >= (explicit_mask ? 32 : 4) * kKeys || split_64)));
+                && p.k_seq >= (explicit_mask ? (head == 64 ? 24 : 32) : head == 64 ? 12 : 16) * kKeys));
+    p.touch_share = 0;
+    if(halved)
+    {
+        set_touch(p, head, mode, n_wg);
+    }
     p.mask_bits = nullptr;
     const int scan_rc = scan_mask_once<T>(stream, p, mode, scan_scratch, scan_scratch_bytes);
     if(scan_rc != NNTILE_HIP_OK)
@@ -2012,11 +2349,11 @@ int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head,
     switch(head)
     {
         case 32:
-            return launch_mode<T, 32>(stream, p, mode, grid, false, false);
+            return launch_mode<T, 32>(stream, p, mode, grid, false, false, false);
         case 64:
-            return launch_mode<T, 64>(stream, p, mode, grid, wide, key_split);
+            return launch_mode<T, 64>(stream, p, mode, grid, wide, key_split, halved);
         case 128:
-            return launch_mode<T, 128>(stream, p, mode, grid, wide, key_split);
+            return launch_mode<T, 128>(stream, p, mode, grid, wide, key_split, halved);
         default:
             return NNTILE_HIP_EUNSUPPORTED;
     }
@@ -2031,6 +2368,7 @@ int launch_prefill_16bit_parts(hipStream_t stream, PrefillParams &p, int head, i
     p.k_blocks_per_tile = (int)((p.k_tile + kKeys - 1) / kKeys);
     p.mask_bits = nullptr;
     p.n_scan_wgs = 0;
+    p.touch_share = 0;
     p.xcd_remap = (p.batch % 8 == 0) ? 1 : 0;
     const dim3 grid((unsigned)((int64_t)p.batch * p.q_blocks_per_tile * p.n_parts));
     const bool causal = mode == NNTILE_HIP_MASK_CAUSAL;
