@@ -77,10 +77,9 @@ struct PrefillParams
     int32_t xcd_remap;            // 1: regroup workgroups so a slab stays on one XCD
     int32_t overwrite;            // 1: ignore the running pair, write every row
     int32_t n_scan_wgs;
-    // 16-bit: workgroups touch the lines of the first touch_steps key steps before they
-    // begin, each one of touch_share shares: those of every touch_period-th query block,
-    // and of the touch_group heads that have the same keys, are on one XCD.  0: none does.
-    int32_t touch_share, touch_period, touch_group, touch_steps;
+    // 16-bit: the workgroups that have the same keys on an XCD, of touch_group heads,
+    // touch the lines of the first touch_steps key steps between them before they begin
+    int32_t touch_steps, touch_group;
     int32_t form;                 // 0 pick by size
                                   // fp32 launcher: see launch_prefill_fp32
                                   // 16-bit launcher: 1 128-query workgroups, 2 the same with the key steps split over two groups of wavefronts, 3 64-query with each step halved, from 8 on 256-query

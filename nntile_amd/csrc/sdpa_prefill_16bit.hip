@@ -278,6 +278,8 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // arguments where they use them, as if this were not there)
     auto overwrite = [&]() __attribute__((always_inline)) { return PARTS || p.overwrite; };
     int b, qblk;
+    // this workgroup among those of its entry on its XCD
+    int my_place = 0, n_places = 0;
     const int batch_all = p.batch * p.n_slabs;
     if(p.xcd_remap)
     {
@@ -285,6 +287,27 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         const int i = (int)(wg >> 3);
         b = (int)(wg & 7) * b_per_xcd + i % b_per_xcd;
         qblk = q_blocks - 1 - i / b_per_xcd;
+        my_place = i / b_per_xcd;
+        n_places = q_blocks;
+    }
+    else if constexpr(KH > 1)
+    {
+        // Every XCD gets a run of the (entry, query block) pairs, so that it has few
+        // entries' keys in its L2.  An entry's blocks lie in the run as longest,
+        // shortest, second longest, ...: any piece of an entry is as much work as any
+        // other; of a run, the longer ones (even places) come first, then the others
+        // from long to short.
+        const int x = (int)(wg & 7), i = (int)(wg >> 3);
+        const int n = (int)n_att;
+        const int run0 = x * (n >> 3) + min(x, n & 7);
+        const int run = (n >> 3) + (x < (n & 7) ? 1 : 0), longer = (run + 1) >> 1;
+        const int at = run0 + (i < longer ? 2 * i : 2 * (run - 1 - i) + 1);
+        b = at / q_blocks;
+        const int place = at - b * q_blocks;
+        qblk = (place & 1) ? place >> 1 : q_blocks - 1 - (place >> 1);
+        const int first_place = max(run0 - b * q_blocks, 0);
+        my_place = place - first_place;
+        n_places = min(run0 + run - b * q_blocks, q_blocks) - first_place;
     }
     else
     {
@@ -318,18 +341,17 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     uint32_t touched[NT];
     auto touch_keys = [&]() __attribute__((always_inline))
     {
-        if(p.touch_share > 0)
+        if(p.touch_steps > 0)
         {
             constexpr int LINES = kKeys * RB / 128;     // of a step's K, and of its V
-            const int order = q_blocks - 1 - qblk;
+            const int share = n_places * p.touch_group;
             const int idx = p.touch_group > 1
-                ? (order / p.touch_period) * p.touch_group + (b / p.n_batch) % p.touch_group
-                : order / p.touch_period;
-            const int n_lines = idx < p.touch_share ? p.touch_steps * 2 * LINES : 0;
+                ? my_place * p.touch_group + (b / p.n_batch) % p.touch_group : my_place;
+            const int n_lines = p.touch_steps * 2 * LINES;
 #pragma unroll
             for(int i = 0; i < NT; ++i)
             {
-                const int line = (i * p.touch_share + idx) * kThreads + tid;
+                const int line = (i * share + idx) * kThreads + tid;
                 if(line < n_lines)
                 {
                     const int st = line / (2 * LINES), in = line % (2 * LINES);
@@ -2175,29 +2197,41 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
 
 // How the keys of a launch lie on the XCDs: `steps` key steps an entry of the batch, of
 // which `fit` leading ones, of all entries that an XCD works on, have room in 3 of its
-// L2's 4 MiB; every `period`-th query block of an entry sits on the same XCD, and there
-// `group` heads share their keys.
+// L2's 4 MiB; `group` heads of an XCD share their keys.
 struct KeysOnXCD
 {
     int64_t steps, fit;
-    int period, group;
+    int group;
 };
 
 static KeysOnXCD keys_on_xcd(const PrefillParams &p, int head)
 {
     KeysOnXCD r;
     const int64_t batch_all = (int64_t)p.batch * p.n_slabs;
+    const int64_t q_blocks = (p.q_tile + kQRows / 2 - 1) / (kQRows / 2) * p.n_q_tiles;
     const int64_t last_keys = p.k_seq - (p.n_kv_tiles - 1) * p.k_tile;
     r.steps = (p.n_kv_tiles - 1) * ((p.k_tile + kKeys - 1) / kKeys) + (last_keys + kKeys - 1) / kKeys;
-    r.period = 8;
-    while(r.period > 1 && batch_all * (r.period / 2) % 8 == 0)
+    int64_t entries = batch_all / 8;
+    r.group = 1;
+    if(batch_all % 8 == 0)
     {
-        r.period /= 2;
+        if(p.n_slabs == 1 && p.batch % (8 * (int64_t)p.n_batch * p.kv_group) == 0)
+        {
+            r.group = p.kv_group;
+        }
     }
-    // (an XCD has whole groups of heads where the entries come in eights: xcd_remap)
-    r.group = p.n_slabs == 1 && p.batch % (8 * (int64_t)p.n_batch * p.kv_group) == 0 ? p.kv_group : 1;
-    const int64_t entries = (batch_all * r.period + 7) / 8;
-    r.fit = ((int64_t)3 << 20) * r.group / (entries * (kKeys * 2 * 2) * head);
+    else
+    {
+        // (runs of the workgroups, as the kernel cuts them)
+        const int64_t n = batch_all * q_blocks;
+        for(int64_t x = 0; x < 8; ++x)
+        {
+            const int64_t lo = x * (n / 8) + std::min(x, n % 8);
+            const int64_t hi = lo + n / 8 + (x < n % 8 ? 1 : 0);
+            entries = hi > lo ? std::max(entries, (hi - 1) / q_blocks - lo / q_blocks + 1) : entries;
+        }
+    }
+    r.fit = ((int64_t)3 << 20) * r.group / (std::max<int64_t>(entries, 1) * (kKeys * 2 * 2) * head);
     return r;
 }
 
@@ -2227,14 +2261,14 @@ constexpr int64_t kHalvedSteps = 8;
 //   hidden 4.2 / 4.2.  Not where the keys of an open launch outgrow the L2: 1 x 16384
 //   171.6 / 177.3.
 //   257 to 512, causal: 32 x 700 18.1 / 16.5, 32 x 1024 21.8 / 20.8, 8 x 4096 53.3 / 47.3;
-//   head 64 15.7 / 14.1, 38.1 / 33.2; 200 x 128 of head 128 10.0 / 9.3.  Open: 32 x 1024
-//   24.4 / 26.6.
+//   head 64 15.7 / 14.1, 38.1 / 33.2; 12 x 2048 of head 128 31.0 / 26.1, 36 x 500 16.3 / 13.9, 200 x
+//   128 10.0 / 9.3; 4 x 8192, whose keys outgrow the L2, 94.7 / 96.5: not.  Open: 32 x 1024 24.4 /
+//   26.6.
 //   257 to 512, masks as values: what they hide is not known here.  Head 64, 36 x 500:
 //   causal 15.5 / 13.2, open 15.0 / 14.2, hidden 4.5 / 4.6; 32 x 1024 21.8 / 18.3, 20.8 / 20.1,
-//   4.5 / 5.1; 9 x 2048, whose keys outgrow the L2, 27.0 / 29.4, 27.8 / 30.0.  Head 128,
-//   32 x 1024: causal 27.6 / 24.1, open 27.3 / 30.0, hidden 5.0 / 6.4: not; 16 x 1500 34.7 / 26.9,
-//   34.5 / 34.9, 6.2 / 6.4, 16 x 2048 41.6 / 33.4, 45.4 / 46.9, 8.3 / 8.6; 20 x 1500, which outgrows
-//   the L2, 35.9 / 31.0, 36.2 / 40.1: not.
+//   4.5 / 5.1; 9 x 2048 26.4 / 24.3, 27.7 / 29.2.  Head 128, 32 x 1024: causal 27.6 / 24.1, open
+//   27.3 / 30.0, hidden 5.0 / 6.4: not; 16 x 1500 34.7 / 26.9, 34.5 / 34.9, 6.2 / 6.4, 16 x 2048 41.6 /
+//   33.4, 45.4 / 46.9, 8.3 / 8.6, 15 x 1622 35.5 / 32.0, 36.8 / 38.1; not where the keys outgrow the L2.
 static bool halved_is_faster(const PrefillParams &p, int head, int mode)
 {
     const int64_t tiles = (int64_t)p.batch * p.n_slabs * p.n_q_tiles;
@@ -2257,7 +2291,8 @@ static bool halved_is_faster(const PrefillParams &p, int head, int mode)
         case NNTILE_HIP_MASK_CAUSAL:
             // (beyond 256 workgroups where the rule hides enough to make long and short
             // ones: 64 heads, 333 queries behind 1500 keys 33.9 / 36.8)
-            return n_wg <= kCUs || p.q_pos0 + p.causal_offset - p.k_pos0 < p.k_seq / 2;
+            return n_wg <= kCUs || (keys.fit >= keys.steps
+                    && p.q_pos0 + p.causal_offset - p.k_pos0 < p.k_seq / 2);
         case NNTILE_HIP_MASK_NONE:
             return n_wg <= kCUs && (keys.steps < 2 * kTouchSteps || 2 * keys.fit >= keys.steps);
         default:
@@ -2270,12 +2305,9 @@ static void set_touch(PrefillParams &p, int head, int mode, int64_t n_wg)
 {
     const KeysOnXCD keys = keys_on_xcd(p, head);
     const bool rule = mode == NNTILE_HIP_MASK_CAUSAL || mode == NNTILE_HIP_MASK_NONE;
-    const int64_t share = (int64_t)p.n_q_tiles * p.q_blocks_per_tile / keys.period * keys.group;
     if(keys.steps >= (rule || head == 64 || n_wg <= 8 * kCUsPerXCD ? kTouchSteps : kTouchStepsMask)
-            && 3 * keys.fit >= keys.steps && share > 1)
+            && 3 * keys.fit >= keys.steps)
     {
-        p.touch_share = (int)share;
-        p.touch_period = keys.period;
         p.touch_group = keys.group;
         p.touch_steps = (int)std::min(keys.steps, keys.fit);
     }
@@ -2331,7 +2363,7 @@ int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head,
     const bool key_split = can_split && (p.form == 2
             || (p.form == 0 && n_wg <= 8 * (int64_t)kCUsPerXCD
                 && p.k_seq >= (explicit_mask ? (head == 64 ? 24 : 32) : head == 64 ? 12 : 16) * kKeys));
-    p.touch_share = 0;
+    p.touch_steps = 0;
     if(halved)
     {
         set_touch(p, head, mode, n_wg);
@@ -2368,7 +2400,7 @@ int launch_prefill_16bit_parts(hipStream_t stream, PrefillParams &p, int head, i
     p.k_blocks_per_tile = (int)((p.k_tile + kKeys - 1) / kKeys);
     p.mask_bits = nullptr;
     p.n_scan_wgs = 0;
-    p.touch_share = 0;
+    p.touch_steps = 0;
     p.xcd_remap = (p.batch % 8 == 0) ? 1 : 0;
     const dim3 grid((unsigned)((int64_t)p.batch * p.q_blocks_per_tile * p.n_parts));
     const bool causal = mode == NNTILE_HIP_MASK_CAUSAL;
