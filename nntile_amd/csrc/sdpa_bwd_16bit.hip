@@ -448,12 +448,13 @@ __device__ __forceinline__ StepSet make_step_set(const BwdParams &p, bool explic
 // to arrives, as whole rows, 16 bytes a lane, instead of 8-byte pieces 2*HEAD
 // bytes apart.  xch: 32 rows of LDS of the wavefront's own; base: the first
 // row; n_ok: rows that exist (may be none or more than 32).
-template<typename T, int HEAD>
+// KH == 2: half of each row, the blocks in front of acc; base: where that half begins.
+template<typename T, int HEAD, int KH = 1>
 __device__ __forceinline__ void bwd_store_rows(char *xch, char *base, int n_ok,
         const f32x16 (&acc)[HEAD / 32], float factor, bool add)
 {
     typedef BwdTile<HEAD> G;
-    constexpr int RB = G::RB, CPR = G::CPR, RPI = G::ROWS_PER_LOAD, N = 32 / RPI;
+    constexpr int STRIDE = G::RB, RB = G::RB / KH, CPR = G::CPR / KH, RPI = 1024 / RB, N = 32 / RPI;
     if(n_ok <= 0)
     {
         return;
@@ -467,7 +468,7 @@ __device__ __forceinline__ void bwd_store_rows(char *xch, char *base, int n_ok,
         for(int i = 0; i < N; ++i)
         {
             old[i] = *reinterpret_cast<const u32x4 *>(base
-                    + (int64_t)min(i * RPI + st_row, n_ok - 1) * RB + st_c * 16);
+                    + (int64_t)min(i * RPI + st_row, n_ok - 1) * STRIDE + st_c * 16);
         }
 #pragma unroll
         for(int i = 0; i < N; ++i)
@@ -478,7 +479,7 @@ __device__ __forceinline__ void bwd_store_rows(char *xch, char *base, int n_ok,
     }
     const int col = lane & 31, half = lane >> 5;
 #pragma unroll
-    for(int db = 0; db < G::DBLOCKS; ++db)
+    for(int db = 0; db < G::DBLOCKS / KH; ++db)
     {
 #pragma unroll
         for(int rg = 0; rg < 4; ++rg)
@@ -509,7 +510,7 @@ __device__ __forceinline__ void bwd_store_rows(char *xch, char *base, int n_ok,
         const u32x4 v = *reinterpret_cast<const u32x4 *>(xch + r * RB + (st_c ^ (r % CPR)) * 16);
         if(r < n_ok)
         {
-            *reinterpret_cast<u32x4 *>(base + (int64_t)r * RB + st_c * 16) = v;
+            *reinterpret_cast<u32x4 *>(base + (int64_t)r * STRIDE + st_c * 16) = v;
         }
     }
 }
@@ -550,12 +551,44 @@ __device__ __forceinline__ void bwd_add_groups(int grp, char *own, f32x16 (&acc)
     }
 }
 
+// Two wavefronts that halved the steps of the same 32 rows (KH == 2): each gives the
+// other the blocks of its sums that lie in the other's half of the head - those behind
+// N in acc - and adds what it gets to its own.  own, theirs: an array of LDS each.
+template<int N>
+__device__ __forceinline__ void bwd_add_halves(char *own, const char *theirs, f32x16 (&acc)[2 * N])
+{
+    const int lane = lane_index_again();
+    float *to = reinterpret_cast<float *>(own) + lane;
+    const float *from = reinterpret_cast<const float *>(theirs) + lane;
+#pragma unroll
+    for(int db = 0; db < N; ++db)
+    {
+#pragma unroll
+        for(int r = 0; r < 16; ++r)
+        {
+            to[(16 * db + r) * 64] = acc[N + db][r];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for(int db = 0; db < N; ++db)
+    {
+#pragma unroll
+        for(int r = 0; r < 16; ++r)
+        {
+            acc[db][r] += from[(16 * db + r) * 64];
+        }
+    }
+}
+
+// KH: 2: the workgroup has 64 rows, and each step's 64 are shared by two wavefronts of
+// the same 32 rows, 32 each (see the launcher).
 // GROUPS: 2: the workgroup is two groups of four wavefronts on the same rows, which
 // take the steps of the walk in turn through tiles of their own (see the launcher).
 // GRID: the rows of both sequence axes live in separately allocated tiles
 // (BwdGridParams); a workgroup's own 128 rows lie in one tile and every 64-row
 // step of the other axis does too, because tile sizes are multiples of 128.
-template<typename T, int HEAD, int MODE, bool GRID, int GROUPS>
+template<typename T, int HEAD, int MODE, bool GRID, int GROUPS, int KH>
 __device__ __forceinline__ void sdpa_bwd_dq_body(
         const std::conditional_t<GRID, BwdGridParams, BwdParams> &p, unsigned wg,
         char *lds_k0, char *lds_k1, char *lds_v0, char *lds_v1)
@@ -574,10 +607,14 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    constexpr int ROWS = kBwdRows / KH;     // queries of the workgroup
+    constexpr int NB = 2 / KH;              // 32-key blocks of a step that a wavefront takes
+    const int rows32 = KH > 1 ? wave_u & 1 : wave_u;    // which of the workgroup's queries
+    const int kh = KH > 1 ? wave_u >> 1 : 0;            // which 32 keys of a step
     const int col = lane & 31;
     const int half = lane >> 5;
 
-    const int q_blocks = (int)((p.q_seq + kBwdRows - 1) / kBwdRows);
+    const int q_blocks = (int)((p.q_seq + ROWS - 1) / ROWS);
     // the last query blocks see the most keys under a causal mask: first
     int b, q_block;
     // (the grid form: the slab of the entry, whose tiles are allocations of
@@ -600,10 +637,10 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     {
         map_workgroup(wg, p.batch, q_blocks, true, b, q_block);
     }
-    const int q_row0 = q_block * kBwdRows;
+    const int q_row0 = q_block * ROWS;
     const int kvb = kv_entry(b, p.n_batch, p.kv_group);
     const int q_seq = (int)p.q_seq, k_seq = (int)p.k_seq;
-    const int my_q = q_row0 + wave * 32 + col;
+    const int my_q = q_row0 + rows32 * 32 + col;
     const bool q_ok = my_q < q_seq;
     // the lane's query: its row within the allocation that holds it (of Q, dA,
     // dQ, and of lse without the head axis), and its place among the row dots
@@ -670,7 +707,7 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     int n_steps = (k_seq + kBwdStep - 1) / kBwdStep;
     if(MODE == NNTILE_HIP_MASK_CAUSAL)
     {
-        const int hi = min(rel + min(q_row0 + kBwdRows, q_seq) - 1, k_seq - 1);
+        const int hi = min(rel + min(q_row0 + ROWS, q_seq) - 1, k_seq - 1);
         n_steps = hi < 0 ? 0 : min(n_steps, hi / kBwdStep + 1);
     }
     const int my_lim = rel + my_q;          // last visible key of this lane's query
@@ -704,7 +741,7 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
 #pragma unroll
     for(int ks = 0; ks < KSTEPS; ++ks)
     {
-        row_raddr[ks] = (uint32_t)(lds_grp + col * RB + ((2 * ks + half) ^ G::swz(col)) * 16);
+        row_raddr[ks] = (uint32_t)(lds_grp + (kh * 32 + col) * RB + ((2 * ks + half) ^ G::swz(col)) * 16);
     }
     // transposed operand: within a 16-lane block lane i addresses row j = i/4 and
     // head values 4*(i%4)..+3 of the block's 16; lanes 16..31 take the upper 16
@@ -722,8 +759,9 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
 #pragma unroll
             for(int db = 0; db < DBLOCKS; ++db)
             {
-                const int c = 4 * db + 2 * dblk + (r4 >> 1);
-                tr_raddr[a][db] = (uint32_t)(lds_grp + r * RB + (c ^ G::swz(r)) * 16 + 8 * (r4 & 1));
+                // (KH == 2: the blocks that the wavefront is left with come first)
+                const int c = 4 * ((db + kh * (DBLOCKS / 2)) % DBLOCKS) + 2 * dblk + (r4 >> 1);
+                tr_raddr[a][db] = (uint32_t)(lds_grp + (kh * 32 + r) * RB + (c ^ G::swz(r)) * 16 + 8 * (r4 & 1));
             }
         }
     }
@@ -775,8 +813,8 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
             fetch_piece(at, kdst_base, vdst_base, i);
         }
     };
-    constexpr int FETCH_STRIDE = (NNTILE_BWD_SPREAD == 2 ? 2 : 1) * KSTEPS / LOADS_PER_WAVE;
-    static_assert(FETCH_STRIDE >= 1 && 1 + (LOADS_PER_WAVE - 1) * FETCH_STRIDE < 2 * KSTEPS,
+    constexpr int FETCH_STRIDE = (NNTILE_BWD_SPREAD == 2 ? NB : 1) * KSTEPS / LOADS_PER_WAVE;
+    static_assert(FETCH_STRIDE >= 1 && 1 + (LOADS_PER_WAVE - 1) * FETCH_STRIDE < NB * KSTEPS,
             "the pieces of a fetch must fit between the MFMAs of a step");
 
     f32x16 acc[DBLOCKS];
@@ -799,11 +837,11 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     const uint32_t mask_row_off = (uint32_t)(q_ok ? my_q - q_row0 : 0) * (uint32_t)p.mask_ld * MASK_ES;
     // (at head 128 the groups of four cost registers that the body does not have)
     constexpr bool MASK_GROUPS = HEAD <= 64;
-    const uint32_t mask_off_wg = mask_row_off + (uint32_t)(4 * half) * MASK_ES;
+    const uint32_t mask_off_wg = mask_row_off + (uint32_t)(kh * 32 + 4 * half) * MASK_ES;
 
     // the workgroup's two query blocks of 64 against the key blocks 0 .. n_steps-1
     const StepSet steps = make_step_set(p, EXPLICIT, q_row0 / kBwdStep,
-            min(2, (q_seq - q_row0 + kBwdStep - 1) / kBwdStep), 0, n_steps, true);
+            min(ROWS / kBwdStep, (q_seq - q_row0 + kBwdStep - 1) / kBwdStep), 0, n_steps, true);
     // (the group's steps: every second of the walk)
     auto next_own = [&](int g) __attribute__((always_inline)) -> int
     {
@@ -869,7 +907,7 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
         {
             lim = min(lim, my_lim - kg0);
         }
-        const int lim_less_half = lim - 4 * half;
+        const int lim_less_half = lim - 4 * half - kh * 32;
         // (wave-common: the last key of the step against the last key that
         // exists and the last key the workgroup's first query sees)
         const bool bounds = keys_here < kBwdStep
@@ -877,7 +915,7 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
         if constexpr(use_mask || NNTILE_BWD_PIPE_DQ == 0)
         {
 #pragma unroll
-            for(int mb = 0; mb < 2; ++mb)
+            for(int mb = 0; mb < NB; ++mb)
             {
                 f32x16 sv, dpv;
 #pragma unroll
@@ -1012,6 +1050,93 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
                     }
                 }
             }
+        }
+        else if constexpr(KH > 1)
+        {
+            // One block of 32 keys: S^T, dP^T with the exponentials beside it, dS^T, then
+            // dQ^T += K^T dS^T, in slots as below.
+            f32x16 sv, dpv;
+            uint32_t ds_pk[8];
+            constexpr int SLOTS = 2 * KSTEPS + 2 * DBLOCKS;
+            constexpr int AHEAD = kBwdAhead<HEAD>;
+            vec8 ring[AHEAD + 1];
+            auto read = [&](auto slot) __attribute__((always_inline))
+            {
+                constexpr int g = decltype(slot)::value;
+                if constexpr(g < 2 * KSTEPS)
+                {
+                    ring[g % (AHEAD + 1)] = *reinterpret_cast<const vec8 *>((g < KSTEPS ? Ks : Vs)
+                            + row_raddr[g % KSTEPS]);
+                }
+                else if constexpr(g < SLOTS)
+                {
+                    constexpr int i = g - 2 * KSTEPS, t = i / DBLOCKS, db = i % DBLOCKS;
+                    const u32x2 lo = bwd_lds_read_tr16(Ks + tr_raddr[0][db] + (16 * t) * RB);
+                    const u32x2 hi = bwd_lds_read_tr16(Ks + tr_raddr[1][db] + (16 * t) * RB);
+                    const u32x4 araw = {lo[0], lo[1], hi[0], hi[1]};
+                    ring[g % (AHEAD + 1)] = __builtin_bit_cast(vec8, araw);
+                }
+            };
+            each_slot(read, std::make_integer_sequence<int, AHEAD>{});
+            __builtin_amdgcn_sched_barrier(0);
+            each_slot([&](auto slot) __attribute__((always_inline))
+            {
+                constexpr int g = decltype(slot)::value;
+                if constexpr(g == KSTEPS)
+                {
+                    // (keys past the end and keys the rule hides: see below)
+                    if(bounds)
+                    {
+#pragma unroll
+                        for(int r = 0; r < 16; ++r)
+                        {
+                            sv[r] = tile_row(r, 0) <= lim_less_half ? sv[r] : neg_inf();
+                        }
+                    }
+                }
+                if constexpr(g == 2 * KSTEPS)
+                {
+#pragma unroll
+                    for(int k = 0; k < 8; ++k)
+                    {
+                        ds_pk[k] = T::pack2(sv[2 * k] * (dpv[2 * k] - d_row),
+                                sv[2 * k + 1] * (dpv[2 * k + 1] - d_row));
+                    }
+                }
+                read(std::integral_constant<int, g + AHEAD>{});
+                const vec8 a = ring[g % (AHEAD + 1)];
+                if constexpr(g < KSTEPS)
+                {
+                    sv = T::mfma(a, qf[g], g == 0 ? f32x16{} : sv);
+#pragma unroll
+                    for(int j = 0; j < LOADS_PER_WAVE; ++j)
+                    {
+                        if(NNTILE_BWD_SPREAD != 0 && g == 1 + j * FETCH_STRIDE)
+                        {
+                            fetch_piece(at_f, BUF ? lds_k0 : lds_k1, BUF ? lds_v0 : lds_v1, j);
+                        }
+                    }
+                }
+                else if constexpr(g < 2 * KSTEPS)
+                {
+                    constexpr int i = g - KSTEPS;
+                    dpv = T::mfma(a, gf[i], i == 0 ? f32x16{} : dpv);
+#pragma unroll
+                    for(int r = i * 16 / KSTEPS; r < (i + 1) * 16 / KSTEPS; ++r)
+                    {
+                        // (-inf: hidden, or a row that saw nothing)
+                        sv[r] = fast_exp2(fmaf(sv[r], c, -lse2));
+                    }
+                }
+                else
+                {
+                    constexpr int i = g - 2 * KSTEPS, t = i / DBLOCKS, db = i % DBLOCKS;
+                    const u32x4 braw = {ds_pk[4 * t], ds_pk[4 * t + 1], ds_pk[4 * t + 2],
+                        ds_pk[4 * t + 3]};
+                    acc[db] = T::mfma(a, __builtin_bit_cast(vec8, braw), acc[db]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }, std::make_integer_sequence<int, SLOTS>{});
         }
         else
         {
@@ -1183,7 +1308,7 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
 
     // ---- dQ (+)= scale acc (every wavefront is done with the tiles in LDS) -----------
     __syncthreads();
-    const int row_first = q_row0 + wave_u * 32;
+    const int row_first = q_row0 + rows32 * 32;
     char *xch = (wave_u == 0 ? lds_k0 : wave_u == 1 ? lds_k1 : wave_u == 2 ? lds_v0 : lds_v1) + lds_grp;
     if constexpr(GROUPS > 1)
     {
@@ -1193,8 +1318,14 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
             return;
         }
     }
-    bwd_store_rows<T, HEAD>(xch, static_cast<char *>(dQ_own) + row_elem(row_first, true) * RB,
-            q_seq - row_first, acc, p.scale, !p.overwrite);
+    if constexpr(KH > 1)
+    {
+        const char *other = wave_u == 0 ? lds_v0 : wave_u == 1 ? lds_v1 : wave_u == 2 ? lds_k0 : lds_k1;
+        bwd_add_halves<DBLOCKS / 2>(xch, other, acc);
+        xch += G::BYTES - 32 * (RB / 2);        // (behind what the other may still be reading)
+    }
+    bwd_store_rows<T, HEAD, KH>(xch, static_cast<char *>(dQ_own) + row_elem(row_first, true) * RB
+            + kh * (RB / 2), q_seq - row_first, acc, p.scale, !p.overwrite);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1222,7 +1353,7 @@ constexpr int kDkvWaves = 4;
 constexpr int kDkvThreads = kDkvWaves * 64;
 constexpr int kDkvRows = kDkvWaves * 32;        // keys per workgroup
 
-template<typename T, int HEAD, int MODE, int PART, bool GRID, int GROUPS>
+template<typename T, int HEAD, int MODE, int PART, bool GRID, int GROUPS, int KH>
 __device__ __forceinline__ void sdpa_bwd_dkv_body(
         const std::conditional_t<GRID, BwdGridParams, BwdParams> &p, unsigned wg,
         char *lds_q0, char *lds_q1, char *lds_g0, char *lds_g1,
@@ -1247,11 +1378,15 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    constexpr int ROWS = kDkvRows / KH;     // keys of the workgroup
+    constexpr int NB = 2 / KH;              // 32-query blocks of a step that a wavefront takes
+    const int rows32 = KH > 1 ? wave_u & 1 : wave_u;    // which of the workgroup's keys
+    const int kh = KH > 1 ? wave_u >> 1 : 0;            // which 32 queries of a step
     const int col = lane & 31;
     const int half = lane >> 5;
 
     const int q_seq = (int)p.q_seq, k_seq = (int)p.k_seq;
-    const int k_blocks = (k_seq + kDkvRows - 1) / kDkvRows;
+    const int k_blocks = (k_seq + ROWS - 1) / ROWS;
     // the first key blocks are seen by the most queries under a causal mask
     int kvb, k_block;                               // kvb = nb + n_batch*hkv
     int q_tile0 = 0, k_tile0 = 0;
@@ -1273,12 +1408,13 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     {
         map_workgroup(wg, p.batch / p.kv_group, k_blocks, false, kvb, k_block);
     }
-    const int k_row0 = k_block * kDkvRows;
+    const int k_row0 = k_block * ROWS;
     const int nb = kvb % p.n_batch, hkv = kvb / p.n_batch;
-    const int my_k = k_row0 + wave * 32 + col;
+    const int my_k = k_row0 + rows32 * 32 + col;
     const bool k_ok = my_k < k_seq;
     // key kg is visible to query q0 + qr + 4*half iff kg - 4*half <= rel + q0 + qr
-    const int my_k_less_half = my_k - 4 * half;
+    // (KH == 2: and q0 + 32 * kh)
+    const int my_k_less_half = my_k - 4 * half - kh * 32;
     // the lane's key: its row within the allocation that holds it (of K, V, dK, dV)
     // (a function of the row, so that the stores at the end can work it out
     // again instead of keeping it through the loop)
@@ -1357,7 +1493,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     // here and below: one register stands for each table, an exclusive or with a
     // constant makes the entry where it is used (the chunk index of a row's
     // swizzled place is an exclusive or of the row's and the chunk's own bits).
-    constexpr bool WIDE = BOTH && HEAD > 64;
+    constexpr bool WIDE = BOTH && HEAD > 64 && KH == 1;
     static_assert(!WIDE || (CPR == 16 && ROWS_PER_LOAD == 4 && LPW == 4 && LOADERS == kDkvWaves
                 && KSTEPS == 8 && DBLOCKS == 4), "the wide body's offsets are those of head 128");
     // (a load's rows 4j + lane / 16 of the wavefront's 16 have the swizzle of
@@ -1369,7 +1505,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
 #pragma unroll
     for(int ks = 0; ks < KSTEPS; ++ks)
     {
-        row_raddr[ks] = (uint32_t)(lds_grp + col * RB + ((2 * ks + half) ^ G::swz(col)) * 16);
+        row_raddr[ks] = (uint32_t)(lds_grp + (kh * 32 + col) * RB + ((2 * ks + half) ^ G::swz(col)) * 16);
     }
     uint32_t tr_raddr[2][DBLOCKS];
     {
@@ -1382,8 +1518,8 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
 #pragma unroll
             for(int db = 0; db < DBLOCKS; ++db)
             {
-                const int c = 4 * db + 2 * dblk + (r4 >> 1);
-                tr_raddr[a][db] = (uint32_t)(lds_grp + r * RB + (c ^ G::swz(r)) * 16 + 8 * (r4 & 1));
+                const int c = 4 * ((db + kh * (DBLOCKS / 2)) % DBLOCKS) + 2 * dblk + (r4 >> 1);
+                tr_raddr[a][db] = (uint32_t)(lds_grp + (kh * 32 + r) * RB + (c ^ G::swz(r)) * 16 + 8 * (r4 & 1));
             }
         }
     }
@@ -1412,7 +1548,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     // first_step .. n_steps-1, once per head of the group: walk position
     // i = head * 64K + query step
     const StepSet steps = make_step_set(p, EXPLICIT, k_row0 / kBwdStep,
-            min(kDkvRows / kBwdStep, (k_seq - k_row0 + kBwdStep - 1) / kBwdStep),
+            min(ROWS / kBwdStep, (k_seq - k_row0 + kBwdStep - 1) / kBwdStep),
             first_step, n_steps, false);
     constexpr int kHeadStride = 1 << 16;
     auto locate = [&](int i, int &bq, int &qs)
@@ -1528,8 +1664,8 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     {
         stat_store(stat_load(at, last), last, stat);
     };
-    constexpr int FETCH_STRIDE = (NNTILE_BWD_SPREAD == 2 ? 2 : 1) * KSTEPS / LPW;
-    static_assert(FETCH_STRIDE >= 1 && 1 + (LPW - 1) * FETCH_STRIDE < 2 * KSTEPS,
+    constexpr int FETCH_STRIDE = (NNTILE_BWD_SPREAD == 2 ? NB : 1) * KSTEPS / LPW;
+    static_assert(FETCH_STRIDE >= 1 && 1 + (LPW - 1) * FETCH_STRIDE < NB * KSTEPS,
             "the pieces of a fetch must fit between the MFMAs of a step");
     auto fetch = [&](int i, char *qdst_base, char *gdst_base, float (*stat)[kBwdStep])
     {
@@ -1620,8 +1756,8 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
         // (ruled: the mask of this step is the rule `key <= query + rel`)
         const bool ruled = MODE == NNTILE_HIP_MASK_CAUSAL
             || (EXPLICIT && !use_mask && !steps.is_open(qs));
-        const bool bounds = k_row0 + kDkvRows > k_seq
-            || (ruled && k_row0 + kDkvRows - 1 > rel + q0);
+        const bool bounds = k_row0 + ROWS > k_seq
+            || (ruled && k_row0 + ROWS - 1 > rel + q0);
         const int vis_base = ruled ? rel + q0 : (1 << 30);
         // (the row stride through an empty asm statement: its multiples are
         // then computed where a step uses them - 32 scalar products - instead
@@ -1801,7 +1937,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
             // ---- S = Q K^T, dP = dA V^T: rows are queries, the lane's column its key;
             // P, dS: register r of block mb is query q0 + mb*32 + tile_row(r, half) --------------
 #pragma unroll
-            for(int mb = 0; mb < 2; ++mb)
+            for(int mb = 0; mb < NB; ++mb)
             {
                 uint32_t p_pk[8], ds_pk[8];
                 f32x16 sv, dpv;
@@ -1819,7 +1955,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                     for(int rg = 0; rg < 4; ++rg)
                     {
                         const f32x4 nd4 = *reinterpret_cast<const f32x4 *>(
-                                &stat[1][mb * 32 + 8 * rg + 4 * half]);
+                                &stat[1][(mb + kh) * 32 + 8 * rg + 4 * half]);
 #pragma unroll
                         for(int e = 0; e < 4; ++e)
                         {
@@ -1875,7 +2011,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                 for(int rg = 0; rg < 4; ++rg)
                 {
                     // four consecutive queries: their statistics in one LDS read each
-                    const int qr0 = mb * 32 + 8 * rg + 4 * half;
+                    const int qr0 = (mb + kh) * 32 + 8 * rg + 4 * half;
                     const f32x4 lse4 = *reinterpret_cast<const f32x4 *>(&stat[0][qr0]);
 #pragma unroll
                     for(int e = 0; e < 4; ++e)
@@ -1890,7 +2026,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                             // four rows in the upper half, while those exist;
                             // rows past the end read a row that exists and are
                             // dropped by their logsumexp of +inf)
-                            const int rb = mb * 32 + 8 * rg + e;
+                            const int rb = (mb + kh) * 32 + 8 * rg + e;
                             const char *mrow = mask_step
                                 + min((uint32_t)rb * mask_row_bytes, mask_last_row);
                             const char *mp = mrow + (rb + 4 < rows_here ? mask_off_hi : mask_off_lo);
@@ -1948,6 +2084,157 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
                     }
                 }
             }
+        }
+        else if constexpr(KH > 1)
+        {
+            // One block of 32 queries: S, dP with P beside it, dV^T += dA^T P with dS
+            // beside it, dK^T += Q^T dS - those of them that this part has - in slots
+            // as below.
+            f32x16 sv, dpv;
+            uint32_t p_pk[8], ds_pk[8];
+            constexpr int N_DP = DO_DK ? KSTEPS : 0, N_DV = DO_DV ? 2 * DBLOCKS : 0;
+            constexpr int AT_DV = KSTEPS + N_DP, AT_DK = AT_DV + N_DV;
+            constexpr int SLOTS = AT_DK + (DO_DK ? 2 * DBLOCKS : 0);
+            constexpr int AHEAD = kBwdAhead<HEAD>;
+            vec8 ring[AHEAD + 1];
+            auto read = [&](auto slot) __attribute__((always_inline))
+            {
+                constexpr int g = decltype(slot)::value;
+                if constexpr(g < AT_DV)
+                {
+                    ring[g % (AHEAD + 1)] = *reinterpret_cast<const vec8 *>((g < KSTEPS ? Qs : Gs)
+                            + row_raddr[g % KSTEPS]);
+                }
+                else if constexpr(g < SLOTS)
+                {
+                    constexpr int i = g < AT_DK ? g - AT_DV : g - AT_DK;
+                    constexpr int t = i / DBLOCKS, db = i % DBLOCKS;
+                    const char *src = (g < AT_DK ? Gs : Qs) + (16 * t) * RB;
+                    const u32x2 lo = bwd_lds_read_tr16(src + tr_raddr[0][db]);
+                    const u32x2 hi = bwd_lds_read_tr16(src + tr_raddr[1][db]);
+                    const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
+                    ring[g % (AHEAD + 1)] = __builtin_bit_cast(vec8, raw);
+                }
+            };
+            auto four = [&](int which, int rg) __attribute__((always_inline)) -> f32x4
+            {
+                return *reinterpret_cast<const f32x4 *>(&stat[which][kh * 32 + 8 * rg + 4 * half]);
+            };
+            f32x4 lse4[4];
+            // probabilities [first, last) of the block
+            auto p_items = [&](int first, int last) __attribute__((always_inline))
+            {
+#pragma unroll
+                for(int r = first; r < last; ++r)
+                {
+                    sv[r] = fast_exp2(fmaf(sv[r], c, -lse4[r / 4][r % 4]));
+                    if(DO_DV && r % 2 == 1)
+                    {
+                        p_pk[r / 2] = T::pack2(sv[r - 1], sv[r]);
+                    }
+                }
+            };
+            auto ds_items = [&](int first, int last) __attribute__((always_inline))
+            {
+#pragma unroll
+                for(int r = first; r < last; ++r)
+                {
+                    dpv[r] = sv[r] * dpv[r];
+                    if(r % 2 == 1)
+                    {
+                        ds_pk[r / 2] = T::pack2(dpv[r - 1], dpv[r]);
+                    }
+                }
+            };
+            each_slot(read, std::make_integer_sequence<int, AHEAD>{});
+            __builtin_amdgcn_sched_barrier(0);
+            each_slot([&](auto slot) __attribute__((always_inline))
+            {
+                constexpr int g = decltype(slot)::value;
+                if constexpr(g == KSTEPS)
+                {
+                    // (keys past the end and pairs the rule hides: see below)
+                    if(bounds)
+                    {
+#pragma unroll
+                        for(int r = 0; r < 16; ++r)
+                        {
+                            bool vis = k_ok;
+                            if(MODE == NNTILE_HIP_MASK_CAUSAL || EXPLICIT)
+                            {
+                                vis = vis && (my_k_less_half <= vis_base + tile_row(r, 0));
+                            }
+                            sv[r] = vis ? sv[r] : neg_inf();
+                        }
+                    }
+                    if constexpr(!DO_DK)
+                    {
+                        p_items(0, 16);
+                    }
+                }
+                if constexpr(DO_DK && !DO_DV && g == AT_DK)
+                {
+                    ds_items(0, 16);
+                }
+                read(std::integral_constant<int, g + AHEAD>{});
+                const vec8 a = ring[g % (AHEAD + 1)];
+                if constexpr(g < KSTEPS)
+                {
+                    sv = T::mfma(a, kf[g], g == 0 ? f32x16{} : sv);
+                    if(LOADERS == kDkvWaves || wave_u < LOADERS)
+                    {
+#pragma unroll
+                        for(int j = 0; j < LPW; ++j)
+                        {
+                            if(NNTILE_BWD_SPREAD != 0 && g == 1 + j * FETCH_STRIDE)
+                            {
+                                fetch_piece(at_f, at_end_f, BUF ? lds_q0 : lds_q1,
+                                        BUF ? lds_g0 : lds_g1, j);
+                            }
+                        }
+                    }
+                    // the statistics of the rows, over the first slots
+#pragma unroll
+                    for(int rg = g * 4 / KSTEPS; rg < (g + 1) * 4 / KSTEPS; ++rg)
+                    {
+                        lse4[rg] = four(0, rg);
+                        if(DO_DK)
+                        {
+                            // dP - D: the accumulator starts at -D of its row
+                            const f32x4 nd4 = four(1, rg);
+#pragma unroll
+                            for(int e = 0; e < 4; ++e)
+                            {
+                                dpv[4 * rg + e] = nd4[e];
+                            }
+                        }
+                    }
+                }
+                else if constexpr(g < AT_DV)
+                {
+                    constexpr int i = g - KSTEPS;
+                    dpv = T::mfma(a, vf[i], dpv);
+                    p_items(i * 16 / KSTEPS, (i + 1) * 16 / KSTEPS);
+                }
+                else if constexpr(g < AT_DK)
+                {
+                    constexpr int i = g - AT_DV, t = i / DBLOCKS, db = i % DBLOCKS;
+                    const u32x4 braw = {p_pk[4 * t], p_pk[4 * t + 1], p_pk[4 * t + 2], p_pk[4 * t + 3]};
+                    dv[db] = T::mfma(a, __builtin_bit_cast(vec8, braw), dv[db]);
+                    if constexpr(BOTH)
+                    {
+                        ds_items(i * 16 / N_DV, (i + 1) * 16 / N_DV);
+                    }
+                }
+                else
+                {
+                    constexpr int i = g - AT_DK, t = i / DBLOCKS, db = i % DBLOCKS;
+                    const u32x4 braw = {ds_pk[4 * t], ds_pk[4 * t + 1], ds_pk[4 * t + 2],
+                        ds_pk[4 * t + 3]};
+                    dk[db] = T::mfma(a, __builtin_bit_cast(vec8, braw), dk[db]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }, std::make_integer_sequence<int, SLOTS>{});
         }
         else
         {
@@ -2230,7 +2517,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     BWD_TRACE_FLUSH(PART);
     // ---- dK (+)= scale dk, dV (+)= dv (every wavefront is done with the tiles in LDS) ---
     __syncthreads();
-    const int row_first = k_row0 + wave_u * 32;
+    const int row_first = k_row0 + rows32 * 32;
     char *xch = (wave_u == 0 ? lds_q0 : wave_u == 1 ? lds_q1 : wave_u == 2 ? lds_g0 : lds_g1) + lds_grp;
     if constexpr(GROUPS > 1)
     {
@@ -2251,15 +2538,29 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
             return;
         }
     }
-    const int64_t first_byte = row_elem(row_first, true) * RB;
+    const int64_t first_byte = row_elem(row_first, true) * RB + kh * (RB / 2);
+    const char *other = wave_u == 0 ? lds_g0 : wave_u == 1 ? lds_g1 : wave_u == 2 ? lds_q0 : lds_q1;
+    char *rows = KH > 1 ? xch + G::BYTES - 32 * (RB / 2) : xch;     // (behind the sums handed over)
+    if constexpr(KH > 1 && DO_DK)
+    {
+        bwd_add_halves<DBLOCKS / 2>(xch, other, dk);
+    }
     if(DO_DK)
     {
-        bwd_store_rows<T, HEAD>(xch, static_cast<char *>(dK_own) + first_byte, k_seq - row_first,
+        bwd_store_rows<T, HEAD, KH>(rows, static_cast<char *>(dK_own) + first_byte, k_seq - row_first,
                 dk, p.scale, !p.overwrite);
+    }
+    if constexpr(KH > 1 && DO_DV)
+    {
+        if(BOTH)
+        {
+            __syncthreads();        // (the first sums have been read)
+        }
+        bwd_add_halves<DBLOCKS / 2>(xch, other, dv);
     }
     if(DO_DV)
     {
-        bwd_store_rows<T, HEAD>(xch, static_cast<char *>(dV_own) + first_byte, k_seq - row_first,
+        bwd_store_rows<T, HEAD, KH>(rows, static_cast<char *>(dV_own) + first_byte, k_seq - row_first,
                 dv, 1.0f, !p.overwrite);
     }
 }
@@ -2269,7 +2570,7 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
 // last n_dkv dV.  A tile-pair call has fewer workgroups per gradient than the
 // chip has places (two a CU); together they fill it, and a long call loses
 // the ends of two launches.
-template<typename T, int HEAD, int MODE, bool GRID, bool FUSED_KEYS = false, int GROUPS = 1>
+template<typename T, int HEAD, int MODE, bool GRID, bool FUSED_KEYS = false, int GROUPS = 1, int KH = 1>
 __global__ __launch_bounds__(kDkvThreads * GROUPS, 2)
 void sdpa_bwd_kernel(const std::conditional_t<GRID, BwdGridParams, BwdParams> p, unsigned n_dkv,
         unsigned n_dq)
@@ -2293,26 +2594,26 @@ void sdpa_bwd_kernel(const std::conditional_t<GRID, BwdGridParams, BwdParams> p,
         // the scores, seven products a call instead of eight)
         if(blockIdx.x < n_dkv)
         {
-            sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK | BWD_PART_DV, GRID, GROUPS>(p, blockIdx.x, lds_0,
+            sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK | BWD_PART_DV, GRID, GROUPS, KH>(p, blockIdx.x, lds_0,
                     lds_1, lds_2, lds_3, lds_stat);
         }
         else
         {
-            sdpa_bwd_dq_body<T, HEAD, MODE, GRID, GROUPS>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3);
+            sdpa_bwd_dq_body<T, HEAD, MODE, GRID, GROUPS, KH>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3);
         }
     }
     else if(blockIdx.x < n_dkv)
     {
-        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK, GRID, GROUPS>(p, blockIdx.x, lds_0, lds_1, lds_2,
+        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK, GRID, GROUPS, KH>(p, blockIdx.x, lds_0, lds_1, lds_2,
                 lds_3, lds_stat);
     }
     else if(blockIdx.x < n_dkv + n_dq)
     {
-        sdpa_bwd_dq_body<T, HEAD, MODE, GRID, GROUPS>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3);
+        sdpa_bwd_dq_body<T, HEAD, MODE, GRID, GROUPS, KH>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3);
     }
     else
     {
-        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DV, GRID, GROUPS>(p, blockIdx.x - n_dkv - n_dq, lds_0,
+        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DV, GRID, GROUPS, KH>(p, blockIdx.x - n_dkv - n_dq, lds_0,
                 lds_1, lds_2, lds_3, lds_stat);
     }
 #ifdef NNTILE_BWD_TRACE
@@ -2352,26 +2653,9 @@ static int launch_prelude(hipStream_t stream, BwdPreludeParams &pre, int n_tiles
     return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
 }
 
-// Workgroups of two groups of wavefronts (sdpa_bwd_kernel, GROUPS == 2): where every
-// workgroup has a CU to itself, which one group would leave with one wavefront on each
-// SIMD, waiting for its own operands, and where the longest walk has enough steps to
-// share: their sums meet in LDS at the end, 0.7 to 1.5 us.  One group / two, us, bf16:
-//   head 64, tiles with a causal mask as values, 12 x 500: 17.7 / 17.2, 8 x 1024 25.3 /
-//     23.1, without one 20.2 / 18.3, 25.3 / 23.5, a window 21.6 / 18.5, 21.6 / 18.3; six
-//     steps, 8 x 384: causal 15.5 / 15.4, a window 22.2 / 18.6, but open 14.7 / 15.0 (what the
-//     values hold is not known here), 8 x 330 16.2 / 16.1, 22.7 / 19.2, open 17.6 / 16.2; as a
-//     rule, 8 x 260 (five steps) 12.6 / 12.3 and open 11.8 / 12.2, 8 x 384 13.5 / 13.4 and
-//     open 12.9 / 13.1, 8 x 400 14.5 / 13.6; two entries with groups of eight, 130 rows 37.0 /
-//     27.6, 520 83 / 60;
-//   head 128, 8 x 400 17.6 / 18.8, 520 (nine steps) 20.1 / 20.9, 800 25.4 / 24.9, causal
-//     26.0 / 24.6, 1100 32.4 / 29.5; two entries with groups of eight, 130 rows 44.6 /
-//     37.2, 520 104 / 83.  (With mask values there it does not fit the registers.)
-// steps: of the longest walk, the queries of all heads of a group or the keys.
-static bool bwd_two_groups(int64_t n_wgs, int64_t steps, int head)
-{
-    return n_wgs <= kBwdCUs && steps >= (head == 64 ? 6 : 13);
-}
-
+// Steps of the longest walk - the queries of all heads of a group, or the keys - from which
+// it is a long one
+constexpr int64_t kBwdLongWalk = 13;
 static int64_t bwd_longest_walk(const BwdParams &p)
 {
     const int64_t keys = (p.k_seq + kBwdStep - 1) / kBwdStep;
@@ -2379,7 +2663,66 @@ static int64_t bwd_longest_walk(const BwdParams &p)
     return keys > queries ? keys : queries;
 }
 
-// The same where one workgroup computes dK and dV: the workgroups that own keys walk
+// Workgroups of 64 rows whose wavefronts halve the steps of the walk between them
+// (sdpa_bwd_kernel, KH == 2): launches that leave CUs empty or with one wavefront on each
+// SIMD, waiting for its own operands, have twice the workgroups so with half of the chain
+// each, and skip blocks of a mask for 64 rows instead of 128; a launch that fills the chip
+// loses by it, as every step comes into LDS twice as often for its MFMAs (32 x 4096 of head
+// 128, causal, 463 / 594 us).  Whole calls, us, fp16, before / with dK and dV apart / with
+// both in one workgroup (head 64; at head 128 it does not fit the registers):
+//   masks as values, head 64: 2 x 128 10.9 / 8.9 / 10.3, 12 x 500 causal 18.1 / 14.8 / 16.7,
+//     open 18.7 / 18.2 / 18.0, a window 18.2 / 13.8 / 17.7; 8 x 1000 25.3 / 23.7 / 23.9, 27.3 /
+//     26.9 / 26.4, 19.0 / 14.7 / 18.9; 32 x 500 24.1 / 22.2 / 19.9, 26.1 / 24.4 / 21.9, 25.0 / 18.7 /
+//     21.5; 24 x 1000 36.0 / 34.8 / 30.8, 41.0 / 51.4 / 45.7, 43.5 / 27.1 / 32.2: not;
+//   head 128: 4 x 500 22.8 / 17.7, 25.0 / 19.0, 29.5 / 18.4; 8 x 1000 37.3 / 31.5, 42.0 / 36.8, 34.4 /
+//     24.5; 24 x 500 28.4 / 25.4, 32.2 / 34.8, 38.4 / 33.3: not;
+//   a rule, head 64: 4 x 1000 19.5 / 16.7 / 18.4, open 20.6 / 18.0 / 18.8, 8 x 1000 20.6 / 20.0 / 18.9,
+//     21.4 / 20.8 / 19.5; 16 x 1000 27.5 / 25.4 / 22.0, 29.8 / 29.0 / 25.0; 24 x 1000 28.6 / 30.3 / 26.2,
+//     34.8 / 42.8 / 40.2; 16 x 2000 47.3 / 55.4 / 45.7; 64 x 1000 47.8 / 59.8 / 53.4;
+//   head 128: 8 x 500 19.6 / 15.5, open 19.1 / 15.6, 8 x 1000 28.9 / 26.1, 29.9 / 29.1, 16 x 1000 38.6 /
+//     35.0, 44.3 / 48.0, 4 x 4000 113 / 87, 24 x 1000 43.5 / 45.1;
+//   grouped heads, whose longest chain is a key block's walk over all queries of its group:
+//     head 64, 32 on 8 x 1500 89.9 / 89.9 / 78.9, open 95.2 / 123 / 88.7, 64 on 16 x 800 54.5 / 56.4 /
+//     48.4, 59.6 / 76.3 / 54.0, x 2500 open 384 / 504 / 413; head 128, 32 on 8 x 800 80.7 / 55.6, 92.2 /
+//     66.6, x 1500 153 / 126, 169 / 180, 16 on 2 x 4000 728 / 526, 788 / 670; 32 on 16 x 900 57.3 /
+//     59.1.
+enum { BWD_WHOLE_STEPS, BWD_HALVED_APART, BWD_HALVED_BOTH };
+static int bwd_halved(const BwdParams &p, int head, int mode, int64_t entries, int64_t n_dkv,
+        int64_t n_dq)
+{
+    const int64_t apart = 2 * n_dkv + n_dq, both = n_dkv + n_dq;    // (workgroups of 64 rows)
+    const bool causal = mode == NNTILE_HIP_MASK_CAUSAL;
+    if(!causal && mode != NNTILE_HIP_MASK_NONE)
+    {
+        return apart <= 2 * kBwdCUs ? BWD_HALVED_APART
+            : head == 64 && both <= 2 * kBwdCUs ? BWD_HALVED_BOTH : BWD_WHOLE_STEPS;
+    }
+    // (beyond two workgroups a CU short walks of entries that do not come in eights, whose
+    // keys every XCD reads, are left in whole steps: a call then gives the bits that its
+    // entries have in a larger launch)
+    if(apart > 2 * kBwdCUs && entries % 8 != 0 && bwd_longest_walk(p) <= 16)
+    {
+        return BWD_WHOLE_STEPS;
+    }
+    if(head == 64)
+    {
+        const bool few = both <= (causal ? 4 : 2) * kBwdCUs
+            || (p.kv_group >= (causal ? 2 : 4) && n_dkv <= (causal ? 256 : 208));
+        return apart <= kBwdCUs ? BWD_HALVED_APART : few ? BWD_HALVED_BOTH : BWD_WHOLE_STEPS;
+    }
+    // (rectangular calls of short walks are taken in whole steps, so that what one
+    // computes does not depend on how many entries share its launch)
+    if(p.q_seq != p.k_seq && bwd_longest_walk(p) < kBwdLongWalk)
+    {
+        return BWD_WHOLE_STEPS;
+    }
+    const bool few = apart <= (causal ? 3 : 2) * kBwdCUs
+        || (p.kv_group >= 4 && n_dkv <= (causal ? 256 : 128));
+    return few ? BWD_HALVED_APART : BWD_WHOLE_STEPS;
+}
+
+// Workgroups of two groups of wavefronts (sdpa_bwd_kernel, GROUPS == 2), where one
+// computes dK and dV: the workgroups that own keys walk
 // every query of a group's heads, under a causal mask those of the first keys all of
 // them, and a launch that has not enough of them to fill the chip ends with their walks.
 // One group (and operands not read ahead) / two, us, bf16, one box: head 128, causal, 64
@@ -2393,7 +2736,7 @@ static bool bwd_two_groups_fused(int64_t n_dkv, const BwdParams &p, int mode)
 {
     const bool few = mode == NNTILE_HIP_MASK_CAUSAL ? n_dkv <= kBwdCUs
         : p.kv_group > 1 && n_dkv <= kBwdCUs * 3 / 4;
-    return few && bwd_longest_walk(p) >= 13;
+    return few && bwd_longest_walk(p) >= kBwdLongWalk;
 }
 
 // The gradient launch, the same for one allocation (GRID false) and for tiles.
@@ -2408,6 +2751,31 @@ static int launch_bwd_kernel(hipStream_t stream,
                 (unsigned)n_dkv, (unsigned)n_dq);
         return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
     };
+    if constexpr(HEAD >= 64)
+    {
+        // (workgroups of 64 rows for those of 128)
+        constexpr int kHalf = kDkvRows / 2;
+        const int64_t entries = n_dkv / ((p.k_seq + kDkvRows - 1) / kDkvRows);
+        const int64_t n_dkv64 = entries * ((p.k_seq + kHalf - 1) / kHalf);
+        const int64_t n_dq64 = n_dq / ((p.q_seq + kDkvRows - 1) / kDkvRows) * ((p.q_seq + kHalf - 1) / kHalf);
+        const int how = bwd_halved(p, HEAD, MODE, entries, n_dkv64, n_dq64);
+        if(how != BWD_WHOLE_STEPS)
+        {
+            n_dkv = n_dkv64;
+            n_dq = n_dq64;
+        }
+        if(how == BWD_HALVED_APART)
+        {
+            return launch(sdpa_bwd_kernel<T, HEAD, MODE, GRID, false, 1, 2>, 2 * n_dkv + n_dq, 1);
+        }
+        if constexpr(HEAD == 64)
+        {
+            if(how == BWD_HALVED_BOTH)
+            {
+                return launch(sdpa_bwd_kernel<T, HEAD, MODE, GRID, true, 1, 2>, n_dkv + n_dq, 1);
+            }
+        }
+    }
     if constexpr(kBwdFusedKeys<HEAD, MODE>)
     {
         // One set of key-owning workgroups for both gradients (seven products
@@ -2424,13 +2792,6 @@ static int launch_bwd_kernel(hipStream_t stream,
                 }
             }
             return launch(sdpa_bwd_kernel<T, HEAD, MODE, GRID, true>, n_dkv + n_dq, 1);
-        }
-    }
-    if constexpr(HEAD == 64 || (HEAD == 128 && ANALYTIC))
-    {
-        if(bwd_two_groups(2 * n_dkv + n_dq, bwd_longest_walk(p), HEAD))
-        {
-            return launch(sdpa_bwd_kernel<T, HEAD, MODE, GRID, false, 2>, 2 * n_dkv + n_dq, 2);
         }
     }
     return launch(sdpa_bwd_kernel<T, HEAD, MODE, GRID>, 2 * n_dkv + n_dq, 1);
