@@ -70,8 +70,9 @@ extern "C" {
 #define NNTILE_HIP_SDPA_FORM_WIDE   0x4000
 /* 16-bit tile and grid calls, head 64 or 128, for tests and tuning: workgroups of 64
  * queries whose four wavefronts take 32 keys of every step each (what most launches
- * of at most one workgroup of 128 queries per CU take by themselves).  With another
- * FORM flag and in fp32: ignored. */
+ * of at most one workgroup of 128 queries per CU take by themselves); fp32, head 64: 64
+ * queries and four key blocks.  With another FORM flag and in fp32 at other heads:
+ * ignored. */
 #define NNTILE_HIP_SDPA_FORM_HALVED 0x8000
 /* decode calls, for tests and tuning: merge the key splits in a second launch
  * instead of inside the main one (SEPARATE_MERGE); exchange the partials of

@@ -111,7 +111,8 @@ PrefillParts prefill_parts(bool fp32, int64_t batch, int64_t q_seq, int64_t k_se
 
 // Workgroup shapes of the fp32 forward on fp16 matrix units: query blocks of 32
 // times key blocks of 32 (none of them: the fp32 kernel's)
-constexpr int kF16x2None = 0, kF16x2Form22 = 1, kF16x2Form41 = 2, kF16x2Form42 = 3, kF16x2Form81 = 4;
+constexpr int kF16x2None = 0, kF16x2Form22 = 1, kF16x2Form41 = 2, kF16x2Form42 = 3, kF16x2Form81 = 4,
+    kF16x2Form24 = 5;
 int prefill_f16x2_form(const PrefillParams &p, int head, int mode);
 int launch_prefill_f16x2(hipStream_t stream, PrefillParams &p, int head, int mode, int form);
 int launch_prefill_f16x2_parts(hipStream_t stream, PrefillParams &p, int head, int mode);

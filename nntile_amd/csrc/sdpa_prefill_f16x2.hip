@@ -1532,7 +1532,7 @@ static int launch_form(hipStream_t stream, PrefillParams &p, int mode)
     {
         return launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_CAUSAL, QW, G, PARTS>);
     }
-    if constexpr(QW * G == 4 && !PARTS)     // (masks given as values)
+    if constexpr((QW * G == 4 || G == 4) && !PARTS)     // (masks given as values)
     {
         return mode == NNTILE_HIP_MASK_ADDITIVE
             ? launch(sdpa_prefill_f16x2_kernel<HEAD, NNTILE_HIP_MASK_ADDITIVE, QW, G>)
@@ -1544,6 +1544,13 @@ static int launch_form(hipStream_t stream, PrefillParams &p, int mode)
 template<int HEAD>
 static int launch_head(hipStream_t stream, PrefillParams &p, int mode, int form)
 {
+    if constexpr(HEAD == 64)
+    {
+        if(form == kF16x2Form24)
+        {
+            return launch_form<HEAD, 2, 4>(stream, p, mode);
+        }
+    }
     if constexpr(HEAD > 32)
     {
         if(form == kF16x2Form42)
@@ -1574,6 +1581,13 @@ static int launch_head(hipStream_t stream, PrefillParams &p, int mode, int form)
 // 112 / 129 / 103 / 161; 32 x 4096 619 / 275 / 238 / 240 / 226.  Head 128, 48 x 1024: 177 /
 // 90 / 67 / 63 / 75; without a mask 290 / 134 / 96 / 110 / 84; 32 x 4096 1490 / 648 / 432 /
 // 444 / 386.
+// Two query blocks and four key blocks (24, head 64: at 128 its pieces outgrow the LDS) are
+// for launches of at most one such workgroup a CU, which 22 leaves with one wavefront on a
+// SIMD: 22 / 24, causal, inputs of other calls in between, 12 x 1024 27.8 / 24.4, 6 x 2000 47.8 /
+// 39.4, 4 x 4096 85 / 65.5, 2 x 8192 161 / 119, open 27.3 / 24.3, 47.3 / 40.2, 84 / 73.5, 160 /
+// 136; two rounds of them, causal, 12 x 2000 50.7 / 42.1, 8 x 4096 94 / 82, but 32 x 1024 30.5 / 34.5.
+// Errors against 64 bits: a wavefront's sums are half as long (A, 2-norm, 6 x 2000 open
+// 4.0e-7 / 3.3e-7, values with a mean of 1 2.1e-7 / 1.2e-7; lse the same).
 //
 // Masks given as values: what they hide is not known in front of the launch.  A form is
 // taken for its sum over three masks: open, causal, and a window, of which a workgroup
@@ -1584,6 +1598,12 @@ static int launch_head(hipStream_t stream, PrefillParams &p, int mode, int form)
 // 128: 2 x 800 51 51 18 / 49 47 26 / 58 57 31; 32 x 1024 232 151 75 / 113 78 56 / 80 77 40.
 // (257 to 512 workgroups of the fp32 kernel at head 64: a window is slower with 22,
 // the others gain more.)
+// (the small forms, and head 64's two by four)
+static bool with_values(int form)
+{
+    return form <= kF16x2Form41 || form == kF16x2Form24;
+}
+
 int prefill_f16x2_form(const PrefillParams &p, int head, int mode)
 {
     struct Cost
@@ -1592,12 +1612,12 @@ int prefill_f16x2_form(const PrefillParams &p, int head, int mode)
         double fixed, alone, full, round;      // us: launch, pass, pass on a full CU, round
         double scan;                            // us: a mask's rows beyond 32
     };
-    static const Cost costs[3][5] = {
+    static const Cost costs[3][6] = {
         {{kF16x2None, 32, 128, 4.5, 1.59, 1.25, 0.5, 0.0}, {kF16x2Form22, 64, 64, 6.6, 0.76, 0.58, 1.5, 1.5},
             {kF16x2Form41, 128, 32, 6.6, 0.77, 0.56, 1.5, 3.3}},
         {{kF16x2None, 32, 128, 5.1, 2.74, 2.50, 1.2, 0.0}, {kF16x2Form22, 64, 64, 7.7, 1.13, 1.00, 2.3, 1.5},
             {kF16x2Form41, 128, 32, 7.7, 0.90, 0.78, 2.6, 3.3}, {kF16x2Form42, 128, 64, 8.8, 1.31, 1.50, 7.0, 0.0},
-            {kF16x2Form81, 256, 32, 8.2, 1.30, 1.40, 9.0, 0.0}},
+            {kF16x2Form81, 256, 32, 8.2, 1.30, 1.40, 9.0, 0.0}, {kF16x2Form24, 64, 128, 9.2, 1.95, 1.95, 5.0, 1.5}},
         {{kF16x2None, 32, 128, 7.2, 5.23, 5.50, 5.0, 0.0}, {kF16x2Form22, 64, 64, 10.4, 2.17, 2.33, 8.7, 3.5},
             {kF16x2Form41, 128, 32, 9.4, 1.55, 1.31, 5.5, 4.5}, {kF16x2Form42, 128, 64, 12.2, 2.30, 2.75, 11.0, 0.0},
             {kF16x2Form81, 256, 32, 10.3, 2.00, 2.85, 0.0, 0.0}}};
@@ -1606,8 +1626,10 @@ int prefill_f16x2_form(const PrefillParams &p, int head, int mode)
     double least = 0.0;
     for(const Cost &f : costs[head == 128 ? 2 : head == 64 ? 1 : 0])
     {
-        // (head 32 and masks given as values: the small forms)
-        if(f.rows == 0 || (values && f.form > kF16x2Form41))
+        // (masks given as values: the small forms; two by four, the last of them, where one
+        // of the other pieces' forms is faster than the fp32 kernel, which a window favours)
+        if(f.rows == 0 || (values && (!with_values(f.form)
+                        || (f.form == kF16x2Form24 && best == kF16x2None))))
         {
             continue;
         }
@@ -1666,7 +1688,7 @@ int launch_prefill_f16x2(hipStream_t stream, PrefillParams &p, int head, int mod
     {
         return NNTILE_HIP_EINVAL;
     }
-    if(form > kF16x2Form41 && mode != NNTILE_HIP_MASK_NONE && mode != NNTILE_HIP_MASK_CAUSAL)
+    if(!with_values(form) && mode != NNTILE_HIP_MASK_NONE && mode != NNTILE_HIP_MASK_CAUSAL)
     {
         form = kF16x2Form41;
     }

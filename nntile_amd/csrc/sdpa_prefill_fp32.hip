@@ -982,8 +982,10 @@ int launch_prefill_fp32(hipStream_t stream, PrefillParams &p, int head, int mode
     switch(p.form)
     {
         case 0:
-        case 3:     // (a form of the 16-bit kernels)
             form = prefill_f16x2_form(p, head, mode);
+            break;
+        case 3:
+            form = head == 64 ? kF16x2Form24 : prefill_f16x2_form(p, head, mode);
             break;
         case 1:
             form = kF16x2Form41;

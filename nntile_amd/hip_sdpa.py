@@ -26,7 +26,7 @@ BWD_MAX_TILES = 32
 OVERWRITE = 1
 FORM_SHARED, FORM_SPLIT = 0x100, 0x200     # fix the workgroup shape (tests, tuning); 16-bit SPLIT: two groups of four wavefronts
 FORM_WIDE = 0x4000                         # 256-query workgroups (16-bit: analytic masks); fp32: also with one of the above
-FORM_HALVED = 0x8000                       # 16-bit: 64-query workgroups, each key step halved between two pairs of wavefronts
+FORM_HALVED = 0x8000                       # 16-bit: 64-query workgroups, each key step halved between two pairs of wavefronts; fp32 head 64: four key blocks
 # decode calls (tests, tuning): merge the key splits in a second launch; exchange
 # the partials of the in-launch merge through device-scope fences
 DECODE_SEPARATE_MERGE, DECODE_FENCED = 0x400, 0x800
