@@ -245,23 +245,17 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             n_att -= (unsigned)p.n_scan_wgs;
         }
     }
-    // (only where the second group is complete: the places it is dealt to must
-    // all be attention workgroups' - those that scan a mask do not count)
-    if constexpr(KH > 1)
+    // (as far as it goes: the places it is dealt to must all be attention workgroups' -
+    // those that scan a mask do not count.  257 to 511 workgroups of 128 queries, causal,
+    // head 128, dealt in order / in reverse: 12 x 4096 71.2 / 67.7 us, 6 x 8192 131 / 124, 20 x 3000
+    // 59.2 / 56.5; a window given as values, 64 x 700, 20.8 / 22.6, so those only where the
+    // second group is complete)
+    if constexpr(WAVES == 4)
     {
-        // (at most two workgroups a CU, the second group as long as it comes)
         const unsigned i = wg >> 3, n = min(n_att >> 3, 2u * kCUsPerXCD);
-        if(i >= kCUsPerXCD && i < n)
+        if(i >= kCUsPerXCD && i < n && (KH > 1 || !EXPLICIT || n == 2u * kCUsPerXCD))
         {
             wg = ((kCUsPerXCD + n - 1u - i) << 3) | (wg & 7u);
-        }
-    }
-    else if(WAVES == 4 && n_att >= 8u * 2u * kCUsPerXCD)
-    {
-        const unsigned i = wg >> 3;
-        if(i >= kCUsPerXCD && i < 2u * kCUsPerXCD)
-        {
-            wg = ((3u * kCUsPerXCD - 1u - i) << 3) | (wg & 7u);
         }
     }
     // (the parts of a query block have equal indices modulo 8 - one XCD - where
@@ -2249,7 +2243,7 @@ constexpr int64_t kTouchStepsMask = 24;
 constexpr int64_t kHalvedSteps = 8;
 
 // Workgroups of 64 queries whose wavefronts halve the key steps between them: launches
-// of at most 256 workgroups of 128 queries.  Twice the workgroups with half of the chain
+// of at most 256 workgroups of 128 queries (head 64: see below).  Twice the workgroups with half of the chain
 // each, on CUs that would stand empty (up to 256 of them), or two on a CU, long
 // beside short (causal); but each step comes into LDS twice as often for its MFMAs, and with
 // two such workgroups a CU and no mask that is what bounds the launch.  us before /
@@ -2261,12 +2255,14 @@ constexpr int64_t kHalvedSteps = 8;
 //   hidden 4.2 / 4.2.  Not where the keys of an open launch outgrow the L2: 1 x 16384
 //   171.6 / 177.3.
 //   257 to 512, causal: 32 x 700 18.1 / 16.5, 32 x 1024 21.8 / 20.8, 8 x 4096 53.3 / 47.3;
-//   head 64 15.7 / 14.1, 38.1 / 33.2; 12 x 2048 of head 128 31.0 / 26.1, 36 x 500 16.3 / 13.9, 200 x
+//   head 64 15.7 / 14.1, 38.1 / 33.2, up to 768 40 x 1000 19.2 / 15.7, 24 x 2000 30.7 / 23.3, 12 x 4096
+//   51.4 / 41.1, 100 x 330 11.4 / 11.7 (not); 12 x 2048 of head 128 31.0 / 26.1, 36 x 500 16.3 / 13.9, 200 x
 //   128 10.0 / 9.3; 4 x 8192, whose keys outgrow the L2, 94.7 / 96.5: not.  Open: 32 x 1024 24.4 /
 //   26.6.
 //   257 to 512, masks as values: what they hide is not known here.  Head 64, 36 x 500:
 //   causal 15.5 / 13.2, open 15.0 / 14.2, hidden 4.5 / 4.6; 32 x 1024 21.8 / 18.3, 20.8 / 20.1,
-//   4.5 / 5.1; 9 x 2048 26.4 / 24.3, 27.7 / 29.2.  Head 128, 32 x 1024: causal 27.6 / 24.1, open
+//   4.5 / 5.1; 9 x 2048 26.4 / 24.3, 27.7 / 29.2; up to 768 24 x 2000 36.2 / 28.5, 43.9 / 42.0, 6.1 /
+//   7.5, 64 x 700 18.5 / 17.9, 22.7 / 21.1, 4.8 / 5.3.  Head 128, 32 x 1024: causal 27.6 / 24.1, open
 //   27.3 / 30.0, hidden 5.0 / 6.4: not; 16 x 1500 34.7 / 26.9, 34.5 / 34.9, 6.2 / 6.4, 16 x 2048 41.6 /
 //   33.4, 45.4 / 46.9, 8.3 / 8.6, 15 x 1622 35.5 / 32.0, 36.8 / 38.1; not where the keys outgrow the L2.
 static bool halved_is_faster(const PrefillParams &p, int head, int mode)
@@ -2274,7 +2270,11 @@ static bool halved_is_faster(const PrefillParams &p, int head, int mode)
     const int64_t tiles = (int64_t)p.batch * p.n_slabs * p.n_q_tiles;
     constexpr int64_t kCUs = 8 * kCUsPerXCD;
     const int64_t n_wg = tiles * ((p.q_tile + kQRows / 2 - 1) / (kQRows / 2));
-    if(tiles * ((p.q_tile + kQRows - 1) / kQRows) > kCUs)
+    // (head 64: three fit a CU; where entries do not come in eights the longest rows only:
+    // 33 x 1300 22.7 / 23.2)
+    const bool three = head == 64 && mode != NNTILE_HIP_MASK_NONE && n_wg <= 3 * kCUs
+        && (tiles % 8 == 0 || (mode == NNTILE_HIP_MASK_CAUSAL && p.k_seq >= 64 * kKeys));
+    if(!three && tiles * ((p.q_tile + kQRows - 1) / kQRows) > kCUs)
     {
         return false;
     }
@@ -2291,7 +2291,7 @@ static bool halved_is_faster(const PrefillParams &p, int head, int mode)
         case NNTILE_HIP_MASK_CAUSAL:
             // (beyond 256 workgroups where the rule hides enough to make long and short
             // ones: 64 heads, 333 queries behind 1500 keys 33.9 / 36.8)
-            return n_wg <= kCUs || (keys.fit >= keys.steps
+            return n_wg <= kCUs || ((head == 64 ? 2 : 1) * keys.fit >= keys.steps
                     && p.q_pos0 + p.causal_offset - p.k_pos0 < p.k_seq / 2);
         case NNTILE_HIP_MASK_NONE:
             return n_wg <= kCUs && (keys.steps < 2 * kTouchSteps || 2 * keys.fit >= keys.steps);
