@@ -245,23 +245,23 @@ struct BwdPreludeParams
     const void *A[kBwdMaxTiles];
 };
 
+// Class bits of the thread's 16 of a block's 64 x 64 values: row `row`, from column col0 on
+// (threads 4 * r + i: row r of the block, columns 16 * i ..; none past the end).
 template<typename T, int MODE>
-__device__ __forceinline__ void bwd_mask_class(const BwdPreludeParams &p, int wg)
+__device__ __forceinline__ uint32_t bwd_piece_class(const void *mask, int64_t mask_ld, int q_seq,
+        int k_seq, int row, int col0)
 {
     constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 2 : 1;
     constexpr int PER_WORD = 4 / ES;
     constexpr uint32_t OPEN = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0u : 0x01010101u;
     constexpr uint32_t HIDDEN = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? T::kNegInfPair : 0u;
     typedef u32x4 __attribute__((aligned(1))) u32x4_any;
-    const int qb = wg / p.class_ld, kb = wg % p.class_ld;
-    const int row = qb * kBwdStep + (int)threadIdx.x / 4;
-    const int col0 = kb * kBwdStep + ((int)threadIdx.x % 4) * 16;
     uint32_t seen = 0u;
-    if(row < (int)p.q_seq && col0 < p.k_seq)
+    if(row < q_seq && col0 < k_seq)
     {
-        const char *src = static_cast<const char *>(p.mask) + ((int64_t)row * p.mask_ld + col0) * ES;
+        const char *src = static_cast<const char *>(mask) + ((int64_t)row * mask_ld + col0) * ES;
         const int n_vis = row - col0 + 1;       // columns of this thread that the rule shows
-        if(col0 + 16 <= p.k_seq)
+        if(col0 + 16 <= k_seq)
         {
             // the thread's 16 values as 16-byte loads of any alignment
             u32x4 v[ES];
@@ -287,7 +287,7 @@ __device__ __forceinline__ void bwd_mask_class(const BwdPreludeParams &p, int wg
         }
         else
         {
-            for(int e = 0; e < p.k_seq - col0; ++e)
+            for(int e = 0; e < k_seq - col0; ++e)
             {
                 bool open, hidden;
                 if(MODE == NNTILE_HIP_MASK_ADDITIVE)
@@ -306,6 +306,15 @@ __device__ __forceinline__ void bwd_mask_class(const BwdPreludeParams &p, int wg
             }
         }
     }
+    return seen;
+}
+
+template<typename T, int MODE>
+__device__ __forceinline__ void bwd_mask_class(const BwdPreludeParams &p, int wg)
+{
+    const uint32_t seen = bwd_piece_class<T, MODE>(p.mask, p.mask_ld, (int)p.q_seq, p.k_seq,
+            wg / p.class_ld * kBwdStep + (int)threadIdx.x / 4,
+            wg % p.class_ld * kBwdStep + ((int)threadIdx.x % 4) * 16);
     uint32_t all = 0u;
 #pragma unroll
     for(int b = 0; b < 3; ++b)
@@ -316,6 +325,25 @@ __device__ __forceinline__ void bwd_mask_class(const BwdPreludeParams &p, int wg
     {
         p.table[wg] = (uint8_t)all;
     }
+}
+
+// Eight products of a row dot, one after the other.  (The products are exact in 32 bits.
+// Nothing may be contracted: in fp16 the compiler takes a two-way dot product where it finds
+// the pattern, which rounds otherwise, and the same row must give the same bits wherever
+// its dot is taken.)
+template<typename T>
+__device__ __forceinline__ float bwd_dot8(const u32x4 &g, const u32x4 &a)
+{
+#pragma clang fp contract(off)
+    float d = 0.0f;
+#pragma unroll
+    for(int e = 0; e < 4; ++e)
+    {
+        d = __builtin_fmaf(T::to_float((uint16_t)(g[e] & 0xffffu)),
+                T::to_float((uint16_t)(a[e] & 0xffffu)), d);
+        d = __builtin_fmaf(T::to_float((uint16_t)(g[e] >> 16)), T::to_float((uint16_t)(a[e] >> 16)), d);
+    }
+    return d;
 }
 
 template<typename T, int HEAD, int MODE>
@@ -354,14 +382,7 @@ void sdpa_bwd_prelude_kernel(const BwdPreludeParams p)
 #pragma unroll
     for(int i = 0; i < kRowdotRows; ++i)
     {
-        float d = 0.0f;
-#pragma unroll
-        for(int e = 0; e < 4; ++e)
-        {
-            d += T::to_float((uint16_t)(g[i][e] & 0xffffu))
-                * T::to_float((uint16_t)(a[i][e] & 0xffffu));
-            d += T::to_float((uint16_t)(g[i][e] >> 16)) * T::to_float((uint16_t)(a[i][e] >> 16));
-        }
+        float d = bwd_dot8<T>(g[i], a[i]);
 #pragma unroll
         for(int o = LANES / 2; o >= 1; o >>= 1)
         {
@@ -372,6 +393,88 @@ void sdpa_bwd_prelude_kernel(const BwdPreludeParams p)
             D[row0 + i * ROWS] = d;
         }
     }
+}
+
+// ---- without the launch in front ---------------------------------------------------
+// Walks of up to two blocks (OWN below): every workgroup finds out for itself what
+// it needs, with the arithmetic of the launch in front and so the same bits: the row dots of
+// its queries, the classes of the blocks that it meets.  A launch costs about 2.5 us before the
+// next one starts, the same work inside the workgroups the latency of one round of loads, and
+// more with each 128 rows that a key block's workgroup needs the dots of.  Measured (us, with the
+// launch / without): head 64, causal by rule, 4 x 64 7.2 / 5.3, 12 x 128 8.3 / 6.3, 64 x 128 10.0 / 7.6;
+// masks, 12 x 64 8.7 / 7.2, 40 x 128 10.0 / 9.0; head 128, causal by rule, 32 x 60 9.8 / 7.7, 64 x 128
+// 14.3 / 11.9; masks, 12 x 64 10.9 / 9.9, 4 x 128 11.6 / 11.7.  Longer walks lose (a variant that
+// took them, against its own form with the launch): masks, 8 x 200 of head 64 11.6 / 14.5, head
+// 128 14.9 / 19.0; by rule, 32 x 60 in groups of 4 10.4 / 11.7, 12 x 200 of head 128 12.9 / 14.1, and
+// of head 64 10.2 / 9.5 but 12 x 400 12.7 / 13.0.
+constexpr int kBwdOwnRows = 128;            // queries of a walk, all heads of a group
+constexpr int kBwdOwnSteps = kBwdOwnRows / kBwdStep;
+
+// Row dots of `rows` rows from dA, A on, by 256 threads, into out.
+template<typename T, int HEAD>
+__device__ __forceinline__ void bwd_own_row_dots(const uint16_t *dA, const uint16_t *A, int rows,
+        float *out)
+{
+    constexpr int LANES = HEAD / 8, ROWS = 256 / LANES, N = 4;
+    const int part = (int)threadIdx.x % LANES, row0 = (int)threadIdx.x / LANES;
+    for(int base = 0; base < rows; base += N * ROWS)
+    {
+        u32x4 g[N], a[N];
+#pragma unroll
+        for(int i = 0; i < N; ++i)
+        {
+            const int row = min(base + i * ROWS + row0, rows - 1);
+            g[i] = *reinterpret_cast<const u32x4 *>(dA + row * HEAD + part * 8);
+            a[i] = *reinterpret_cast<const u32x4 *>(A + row * HEAD + part * 8);
+        }
+#pragma unroll
+        for(int i = 0; i < N; ++i)
+        {
+            float d = bwd_dot8<T>(g[i], a[i]);
+#pragma unroll
+            for(int o = LANES / 2; o >= 1; o >>= 1)
+            {
+                d += __shfl_xor(d, o, 64);
+            }
+            if(base + i * ROWS + row0 < rows && part == 0)
+            {
+                out[base + i * ROWS + row0] = d;
+            }
+        }
+    }
+}
+
+// Classes of the blocks own0 x [first, last) (by_row: the owned block is one of queries),
+// three bits each, in the order of the walk.  word: one word of LDS, zero before.
+template<typename T, int MODE>
+__device__ __forceinline__ uint32_t bwd_own_classes(const BwdParams &p, int own0, int first, int last,
+        bool by_row, uint32_t *word)
+{
+    const int r = (int)threadIdx.x / 4, c = ((int)threadIdx.x % 4) * 16;
+    uint32_t seen[kBwdOwnSteps];
+#pragma unroll
+    for(int i = 0; i < kBwdOwnSteps; ++i)
+    {
+        const int g = first + i;
+        seen[i] = g < last ? bwd_piece_class<T, MODE>(p.mask, p.mask_ld, (int)p.q_seq, (int)p.k_seq,
+                (by_row ? own0 : g) * kBwdStep + r, (by_row ? g : own0) * kBwdStep + c) : 0u;
+    }
+    uint32_t all = 0u;
+#pragma unroll
+    for(int i = 0; i < kBwdOwnSteps; ++i)
+    {
+#pragma unroll
+        for(int b = 0; b < 3; ++b)
+        {
+            all |= __builtin_amdgcn_ballot_w64((seen[i] & (1u << b)) != 0u) != 0ull ? 1u << (3 * i + b) : 0u;
+        }
+    }
+    if(threadIdx.x % 64 == 0)
+    {
+        atomicOr(word, all);
+    }
+    __syncthreads();
+    return *word;
 }
 
 // The steps a workgroup takes, as a bit set (up to 64 of them; longer walks
@@ -414,12 +517,12 @@ struct StepSet
 // and walks the blocks [first, last) of the other.  by_row: the owned blocks
 // are query blocks (rows of the table).
 __device__ __forceinline__ StepSet make_step_set(const BwdParams &p, bool explicit_mask,
-        int own0, int n_own, int first, int last, bool by_row)
+        int own0, int n_own, int first, int last, bool by_row, bool own = false, uint32_t own_bits = 0u)
 {
     StepSet s;
     s.first = first;
     s.last = last;
-    s.use_bits = explicit_mask && p.mask_class != nullptr && last <= 64;
+    s.use_bits = explicit_mask && (own || p.mask_class != nullptr) && last <= 64;
     s.active = 0ull;
     s.open = 0ull;
     s.rule = 0ull;
@@ -430,7 +533,11 @@ __device__ __forceinline__ StepSet make_step_set(const BwdParams &p, bool explic
         const int g = (int)(threadIdx.x & 63);
         const bool in_walk = g >= first && g < last;
         int c = 0;
-        for(int o = 0; o < n_own; ++o)
+        if(own)
+        {
+            c = in_walk ? (int)(own_bits >> (3 * min(g - first, kBwdOwnSteps))) & 7 : 0;
+        }
+        for(int o = 0; !own && o < n_own; ++o)
         {
             const int idx = by_row ? (own0 + o) * p.class_ld + g : g * p.class_ld + own0 + o;
             c |= in_walk ? p.mask_class[idx] : 0;
@@ -588,10 +695,10 @@ __device__ __forceinline__ void bwd_add_halves(char *own, const char *theirs, f3
 // GRID: the rows of both sequence axes live in separately allocated tiles
 // (BwdGridParams); a workgroup's own 128 rows lie in one tile and every 64-row
 // step of the other axis does too, because tile sizes are multiples of 128.
-template<typename T, int HEAD, int MODE, bool GRID, int GROUPS, int KH>
+template<typename T, int HEAD, int MODE, bool GRID, int GROUPS, int KH, bool OWN>
 __device__ __forceinline__ void sdpa_bwd_dq_body(
         const std::conditional_t<GRID, BwdGridParams, BwdParams> &p, unsigned wg,
-        char *lds_k0, char *lds_k1, char *lds_v0, char *lds_v1)
+        char *lds_k0, char *lds_k1, char *lds_v0, char *lds_v1, uint32_t *lds_word)
 {
     typedef typename T::vec8 vec8;
     typedef BwdTile<HEAD> G;
@@ -693,7 +800,35 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
             gf[ks] = __builtin_bit_cast(vec8, g);
         }
     }
-    const float d_row = q_ok ? p.D[d_idx] : 0.0f;
+    float d_row;
+    if constexpr(OWN)
+    {
+        // (a lane's fragments are every second eight of its row: the sums in the order
+        // of the exchanges that add them up in the launch in front)
+        const uint16_t *as = static_cast<const uint16_t *>(p.A) + q_off + half * 8;
+        float part[KSTEPS];
+#pragma unroll
+        for(int ks = 0; ks < KSTEPS; ++ks)
+        {
+            part[ks] = bwd_dot8<T>(__builtin_bit_cast(u32x4, gf[ks]),
+                    *reinterpret_cast<const u32x4 *>(as + ks * 16));
+        }
+#pragma unroll
+        for(int o = KSTEPS / 2; o >= 1; o /= 2)
+        {
+#pragma unroll
+            for(int ks = 0; ks < o; ++ks)
+            {
+                part[ks] += part[ks + o];
+            }
+        }
+        d_row = part[0] + __shfl_xor(part[0], 32, 64);
+        d_row = q_ok ? d_row : 0.0f;
+    }
+    else
+    {
+        d_row = q_ok ? p.D[d_idx] : 0.0f;
+    }
     const float lse_q = q_ok ? lse_own[q_elem] : neg_inf();
     // exponent offset in log2 units; a row that saw nothing has P = 0
     const float lse2 = (lse_q == neg_inf()) ? __builtin_huge_valf() : lse_q * kLog2e;
@@ -840,8 +975,12 @@ __device__ __forceinline__ void sdpa_bwd_dq_body(
     const uint32_t mask_off_wg = mask_row_off + (uint32_t)(kh * 32 + 4 * half) * MASK_ES;
 
     // the workgroup's two query blocks of 64 against the key blocks 0 .. n_steps-1
+    constexpr bool OWN_CLASSES = OWN && EXPLICIT;
+    const uint32_t own_bits = OWN_CLASSES ? bwd_own_classes<T, MODE>(p, q_row0 / kBwdStep, 0, n_steps, true,
+            lds_word) : 0u;
     const StepSet steps = make_step_set(p, EXPLICIT, q_row0 / kBwdStep,
-            min(ROWS / kBwdStep, (q_seq - q_row0 + kBwdStep - 1) / kBwdStep), 0, n_steps, true);
+            min(ROWS / kBwdStep, (q_seq - q_row0 + kBwdStep - 1) / kBwdStep), 0, n_steps, true,
+            OWN_CLASSES, own_bits);
     // (the group's steps: every second of the walk)
     auto next_own = [&](int g) __attribute__((always_inline)) -> int
     {
@@ -1353,11 +1492,11 @@ constexpr int kDkvWaves = 4;
 constexpr int kDkvThreads = kDkvWaves * 64;
 constexpr int kDkvRows = kDkvWaves * 32;        // keys per workgroup
 
-template<typename T, int HEAD, int MODE, int PART, bool GRID, int GROUPS, int KH>
+template<typename T, int HEAD, int MODE, int PART, bool GRID, int GROUPS, int KH, bool OWN>
 __device__ __forceinline__ void sdpa_bwd_dkv_body(
         const std::conditional_t<GRID, BwdGridParams, BwdParams> &p, unsigned wg,
         char *lds_q0, char *lds_q1, char *lds_g0, char *lds_g1,
-        float (*lds_stat)[2][kBwdStep])
+        float (*lds_stat)[2][kBwdStep], uint32_t *lds_word, float *lds_own)
 {
     constexpr bool DO_DK = (PART & BWD_PART_DK) != 0, DO_DV = (PART & BWD_PART_DV) != 0;
     constexpr bool BOTH = DO_DK && DO_DV;
@@ -1547,9 +1686,12 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     // the workgroup's key blocks of 64 against the query blocks
     // first_step .. n_steps-1, once per head of the group: walk position
     // i = head * 64K + query step
+    constexpr bool OWN_CLASSES = OWN && EXPLICIT;
+    const uint32_t own_bits = OWN_CLASSES ? bwd_own_classes<T, MODE>(p, k_row0 / kBwdStep, first_step,
+            n_steps, false, lds_word) : 0u;
     const StepSet steps = make_step_set(p, EXPLICIT, k_row0 / kBwdStep,
             min(ROWS / kBwdStep, (k_seq - k_row0 + kBwdStep - 1) / kBwdStep),
-            first_step, n_steps, false);
+            first_step, n_steps, false, OWN_CLASSES, own_bits);
     constexpr int kHeadStride = 1 << 16;
     auto locate = [&](int i, int &bq, int &qs)
     {
@@ -1583,6 +1725,11 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
         const void *Q, *dA;
         const float *lse;
         int64_t elem, d_idx;
+        int own;                // place of the row among the workgroup's own row dots
+    };
+    auto own_row0 = [&](int bq) __attribute__((always_inline)) -> int
+    {
+        return OWN ? (bq / p.n_batch - p.kv_group * hkv) * q_seq : 0;
     };
     auto query_rows = [&](int bq, int row0) __attribute__((always_inline)) -> QueryRows
     {
@@ -1592,12 +1739,12 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
             const int tq = row0 / q_tile, t0 = tq * q_tile;
             const int64_t elem = (int64_t)bq * min(q_tile, q_seq - t0) + (row0 - t0);
             return QueryRows{p.Qt[q_tile0 + tq], p.dAt[q_tile0 + tq], p.lset[q_tile0 + tq], elem,
-                d_slab + (int64_t)p.batch * t0 + elem};
+                d_slab + (int64_t)p.batch * t0 + elem, own_row0(bq) + row0};
         }
         else
         {
             const int64_t elem = (int64_t)bq * q_seq + row0;
-            return QueryRows{p.Q, p.dA, p.lse, elem, elem};
+            return QueryRows{p.Q, p.dA, p.lse, elem, elem, own_row0(bq) + row0};
         }
     };
     auto fetch_piece = [&](const QueryRows &at, bool at_end, char *qdst_base, char *gdst_base,
@@ -1635,7 +1782,11 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     {
         float raw = 0.0f;
         // (in the wide body without a branch: the other wavefronts read along)
-        if(WIDE || wave_u < 2)
+        if(OWN && wave_u == 1)
+        {
+            raw = DO_DK ? lds_own[at.own + min(lane, last)] : 0.0f;
+        }
+        else if(WIDE || wave_u < 2)
         {
             const float *src = wave_u % 2 == 0 ? at.lse + at.elem : p.D + at.d_idx;
             raw = src[min(WIDE ? lane_index_again() : lane, last)];
@@ -1703,6 +1854,16 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     {
         i_last = -2;                        // (the first group has a step)
         i_cur = walk_next(i_cur);
+    }
+    if constexpr(OWN && DO_DK)
+    {
+        for(int g = 0; g < p.kv_group; ++g)
+        {
+            const QueryRows at = query_rows(nb + p.n_batch * (g + p.kv_group * hkv), 0);
+            bwd_own_row_dots<T, HEAD>(static_cast<const uint16_t *>(at.dA) + at.elem * HEAD,
+                    static_cast<const uint16_t *>(p.A) + at.elem * HEAD, q_seq, lds_own + g * q_seq);
+        }
+        __syncthreads();
     }
     if(i_cur >= 0)
     {
@@ -2570,7 +2731,8 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
 // last n_dkv dV.  A tile-pair call has fewer workgroups per gradient than the
 // chip has places (two a CU); together they fill it, and a long call loses
 // the ends of two launches.
-template<typename T, int HEAD, int MODE, bool GRID, bool FUSED_KEYS = false, int GROUPS = 1, int KH = 1>
+template<typename T, int HEAD, int MODE, bool GRID, bool FUSED_KEYS = false, int GROUPS = 1, int KH = 1,
+        bool OWN = false>
 __global__ __launch_bounds__(kDkvThreads * GROUPS, 2)
 void sdpa_bwd_kernel(const std::conditional_t<GRID, BwdGridParams, BwdParams> p, unsigned n_dkv,
         unsigned n_dq)
@@ -2585,6 +2747,13 @@ void sdpa_bwd_kernel(const std::conditional_t<GRID, BwdGridParams, BwdParams> p,
     // dK, dV parts, per query of a step: logsumexp in log2 units (+inf for a
     // row that saw nothing) and minus the row dot D; rows past the end hold +inf / 0
     __shared__ __attribute__((aligned(16))) float lds_stat_all[GROUPS][2][2][kBwdStep];
+    __shared__ float lds_own[OWN ? kBwdOwnRows : 1];
+    __shared__ uint32_t lds_word;
+    if constexpr(OWN)
+    {
+        lds_word = 0u;
+        __syncthreads();
+    }
     const int grp = GROUPS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kDkvThreads) : 0;
     float (*const lds_stat)[2][kBwdStep] = lds_stat_all[grp];
     if constexpr(FUSED_KEYS)
@@ -2594,27 +2763,27 @@ void sdpa_bwd_kernel(const std::conditional_t<GRID, BwdGridParams, BwdParams> p,
         // the scores, seven products a call instead of eight)
         if(blockIdx.x < n_dkv)
         {
-            sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK | BWD_PART_DV, GRID, GROUPS, KH>(p, blockIdx.x, lds_0,
-                    lds_1, lds_2, lds_3, lds_stat);
+            sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK | BWD_PART_DV, GRID, GROUPS, KH, OWN>(p, blockIdx.x, lds_0,
+                    lds_1, lds_2, lds_3, lds_stat, &lds_word, lds_own);
         }
         else
         {
-            sdpa_bwd_dq_body<T, HEAD, MODE, GRID, GROUPS, KH>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3);
+            sdpa_bwd_dq_body<T, HEAD, MODE, GRID, GROUPS, KH, OWN>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3, &lds_word);
         }
     }
     else if(blockIdx.x < n_dkv)
     {
-        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK, GRID, GROUPS, KH>(p, blockIdx.x, lds_0, lds_1, lds_2,
-                lds_3, lds_stat);
+        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DK, GRID, GROUPS, KH, OWN>(p, blockIdx.x, lds_0, lds_1, lds_2,
+                lds_3, lds_stat, &lds_word, lds_own);
     }
     else if(blockIdx.x < n_dkv + n_dq)
     {
-        sdpa_bwd_dq_body<T, HEAD, MODE, GRID, GROUPS, KH>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3);
+        sdpa_bwd_dq_body<T, HEAD, MODE, GRID, GROUPS, KH, OWN>(p, blockIdx.x - n_dkv, lds_0, lds_1, lds_2, lds_3, &lds_word);
     }
     else
     {
-        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DV, GRID, GROUPS, KH>(p, blockIdx.x - n_dkv - n_dq, lds_0,
-                lds_1, lds_2, lds_3, lds_stat);
+        sdpa_bwd_dkv_body<T, HEAD, MODE, BWD_PART_DV, GRID, GROUPS, KH, OWN>(p, blockIdx.x - n_dkv - n_dq, lds_0,
+                lds_1, lds_2, lds_3, lds_stat, &lds_word, lds_own);
     }
 #ifdef NNTILE_BWD_TRACE
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -2739,6 +2908,62 @@ static bool bwd_two_groups_fused(int64_t n_dkv, const BwdParams &p, int mode)
     return few && bwd_longest_walk(p) >= kBwdLongWalk;
 }
 
+// The same from the workgroups of 128 rows, which become those of 64 where it is halved.
+static int bwd_halved(const BwdParams &p, int head, int mode, int64_t &n_dkv, int64_t &n_dq)
+{
+    constexpr int kHalf = kDkvRows / 2;
+    const int64_t entries = n_dkv / ((p.k_seq + kDkvRows - 1) / kDkvRows);
+    const int64_t n_dkv64 = entries * ((p.k_seq + kHalf - 1) / kHalf);
+    const int64_t n_dq64 = n_dq / ((p.q_seq + kDkvRows - 1) / kDkvRows) * ((p.q_seq + kHalf - 1) / kHalf);
+    const int how = bwd_halved(p, head, mode, entries, n_dkv64, n_dq64);
+    if(how != BWD_WHOLE_STEPS)
+    {
+        n_dkv = n_dkv64;
+        n_dq = n_dq64;
+    }
+    return how;
+}
+
+template<typename Kernel, typename Params>
+static int launch_bwd_wgs(hipStream_t stream, Kernel kernel, const Params &p, int64_t n_wgs, int groups,
+        int64_t n_dkv, int64_t n_dq)
+{
+    hipLaunchKernelGGL(kernel, dim3((unsigned)n_wgs), dim3(groups * kDkvThreads), 0, stream, p,
+            (unsigned)n_dkv, (unsigned)n_dq);
+    return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+}
+
+// The form without the launch in front, where steps are halved and no workgroup needs more
+// than kBwdOwnRows (measured there); false: the call is for the other forms.
+template<typename T, int HEAD, int MODE>
+static bool launch_bwd_short(hipStream_t stream, const BwdParams &p, int64_t n_dkv, int64_t n_dq, int &rc)
+{
+    if constexpr(HEAD >= 64)
+    {
+        if(p.q_seq > kBwdOwnRows / p.kv_group || p.k_seq > kBwdOwnRows)
+        {
+            return false;
+        }
+        const int how = bwd_halved(p, HEAD, MODE, n_dkv, n_dq);
+        if(how == BWD_HALVED_APART)
+        {
+            rc = launch_bwd_wgs(stream, sdpa_bwd_kernel<T, HEAD, MODE, false, false, 1, 2, true>, p,
+                    2 * n_dkv + n_dq, 1, n_dkv, n_dq);
+            return true;
+        }
+        if constexpr(HEAD == 64)
+        {
+            if(how == BWD_HALVED_BOTH)
+            {
+                rc = launch_bwd_wgs(stream, sdpa_bwd_kernel<T, HEAD, MODE, false, true, 1, 2, true>, p,
+                        n_dkv + n_dq, 1, n_dkv, n_dq);
+                return true;
+            }
+        }
+    }
+    return false;
+}
+
 // The gradient launch, the same for one allocation (GRID false) and for tiles.
 template<typename T, int HEAD, int MODE, bool GRID>
 static int launch_bwd_kernel(hipStream_t stream,
@@ -2747,23 +2972,11 @@ static int launch_bwd_kernel(hipStream_t stream,
     constexpr bool ANALYTIC = MODE == NNTILE_HIP_MASK_NONE || MODE == NNTILE_HIP_MASK_CAUSAL;
     auto launch = [&](auto kernel, int64_t n_wgs, int groups) -> int
     {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)n_wgs), dim3(groups * kDkvThreads), 0, stream, p,
-                (unsigned)n_dkv, (unsigned)n_dq);
-        return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
+        return launch_bwd_wgs(stream, kernel, p, n_wgs, groups, n_dkv, n_dq);
     };
     if constexpr(HEAD >= 64)
     {
-        // (workgroups of 64 rows for those of 128)
-        constexpr int kHalf = kDkvRows / 2;
-        const int64_t entries = n_dkv / ((p.k_seq + kDkvRows - 1) / kDkvRows);
-        const int64_t n_dkv64 = entries * ((p.k_seq + kHalf - 1) / kHalf);
-        const int64_t n_dq64 = n_dq / ((p.q_seq + kDkvRows - 1) / kDkvRows) * ((p.q_seq + kHalf - 1) / kHalf);
-        const int how = bwd_halved(p, HEAD, MODE, entries, n_dkv64, n_dq64);
-        if(how != BWD_WHOLE_STEPS)
-        {
-            n_dkv = n_dkv64;
-            n_dq = n_dq64;
-        }
+        const int how = bwd_halved(p, HEAD, MODE, n_dkv, n_dq);
         if(how == BWD_HALVED_APART)
         {
             return launch(sdpa_bwd_kernel<T, HEAD, MODE, GRID, false, 1, 2>, 2 * n_dkv + n_dq, 1);
@@ -2809,6 +3022,11 @@ static int launch_bwd_mode(hipStream_t stream, const BwdParams &p)
     {
         return NNTILE_HIP_EINVAL;
     }
+    int rc;
+    if(launch_bwd_short<T, HEAD, MODE>(stream, p, n_dkv, n_dq, rc))
+    {
+        return rc;
+    }
     BwdPreludeParams pre = prelude_params(p, p.q_seq, 1);
     pre.dA[0] = p.dA;
     pre.A[0] = p.A;
@@ -2824,10 +3042,10 @@ static int launch_bwd_mode(hipStream_t stream, const BwdParams &p)
         }
         pre.n_class_wgs = (int32_t)n_cls;
     }
-    const int pre_rc = launch_prelude<T, HEAD, MODE>(stream, pre, 1);
-    if(pre_rc != NNTILE_HIP_OK)
+    rc = launch_prelude<T, HEAD, MODE>(stream, pre, 1);
+    if(rc != NNTILE_HIP_OK)
     {
-        return pre_rc;
+        return rc;
     }
     return launch_bwd_kernel<T, HEAD, MODE, false>(stream, p, n_dkv, n_dq);
 }
@@ -2846,6 +3064,25 @@ static int launch_bwd_grid_mode(hipStream_t stream, const BwdGridParams &p,
             || (int64_t)p.batch * p.q_tile * (HEAD / 8) / 256 > 0x7ffffffe)
     {
         return NNTILE_HIP_EINVAL;
+    }
+    if(p.n_slabs == 1 && n_q_tiles == 1 && p.n_kv_tiles == 1)
+    {
+        // (one tile an axis is one allocation)
+        BwdParams one = p;
+        one.Q = p.Qt[0];
+        one.K = p.Kt[0];
+        one.V = p.Vt[0];
+        one.A = A_tiles[0];
+        one.dA = p.dAt[0];
+        one.lse = p.lset[0];
+        one.dQ = p.dQt[0];
+        one.dK = p.dKt[0];
+        one.dV = p.dVt[0];
+        int rc;
+        if(launch_bwd_short<T, HEAD, MODE>(stream, one, n_dkv, n_dq, rc))
+        {
+            return rc;
+        }
     }
     BwdPreludeParams pre = prelude_params(p, p.q_tile, n_q_tiles);
     for(int t = 0; t < p.n_slabs * n_q_tiles; ++t)
