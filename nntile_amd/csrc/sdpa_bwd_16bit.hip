@@ -2933,6 +2933,21 @@ static int launch_bwd_wgs(hipStream_t stream, Kernel kernel, const Params &p, in
     return hipGetLastError() == hipSuccess ? NNTILE_HIP_OK : NNTILE_HIP_ELAUNCH;
 }
 
+// Whether a gradient lies in the memory of A.  The launch in front is done with A before
+// the first gradient is written, so such calls are right with it, and only with it.
+static bool bwd_writes_into_A(const BwdParams &p, int head)
+{
+    const int64_t q_bytes = (int64_t)p.batch * p.q_seq * head * 2;
+    const int64_t k_bytes = (int64_t)(p.batch / p.kv_group) * p.k_seq * head * 2;
+    const uintptr_t a = reinterpret_cast<uintptr_t>(p.A);
+    auto meets = [&](const void *out, int64_t bytes)
+    {
+        const uintptr_t o = reinterpret_cast<uintptr_t>(out);
+        return o < a + (uintptr_t)q_bytes && a < o + (uintptr_t)bytes;
+    };
+    return meets(p.dQ, q_bytes) || meets(p.dK, k_bytes) || meets(p.dV, k_bytes);
+}
+
 // The form without the launch in front, where steps are halved and no workgroup needs more
 // than kBwdOwnRows (measured there); false: the call is for the other forms.
 template<typename T, int HEAD, int MODE>
@@ -2940,7 +2955,7 @@ static bool launch_bwd_short(hipStream_t stream, const BwdParams &p, int64_t n_d
 {
     if constexpr(HEAD >= 64)
     {
-        if(p.q_seq > kBwdOwnRows / p.kv_group || p.k_seq > kBwdOwnRows)
+        if(p.q_seq > kBwdOwnRows / p.kv_group || p.k_seq > kBwdOwnRows || bwd_writes_into_A(p, HEAD))
         {
             return false;
         }

@@ -53,3 +53,32 @@ def test_same_bits_as_with_the_launch_in_front(dtype, mode, head, group, q_seq, 
         for s in range(2):
             assert not torch.isnan(want[s]).any(), (name, s)
             assert torch.equal(got[s].view(torch.int16), want[s].view(torch.int16)), (name, s)
+
+
+@pytest.mark.parametrize("name", ["dQ", "dK", "dV"])
+@pytest.mark.parametrize("grid", [False, True])
+@pytest.mark.parametrize("head,rows", [(64, 128), (128, 100)])
+def test_gradient_in_the_memory_of_A(head, rows, name, grid):
+    # A is read before a gradient is written: the same bits as with memory of its own
+    print("case bwd short into A", head, rows, name, grid, flush=True)
+    batch = 6
+    (Q, K, V), _ = H.make_qkv(41, batch, rows, rows, head, "bf16")
+    rng = np.random.default_rng(11)
+    A, G = (H.rounded(rng.standard_normal(tuple(Q.shape)), "bf16")[0] for _ in range(2))
+    lse = torch.from_numpy(np.log1p(rng.random((batch, rows))).astype(np.float32)) + 3.0
+    Q, K, V, A, G, lse = (x.cuda() for x in (Q, K, V, A, G, lse))
+
+    def run(shared):
+        a = A.clone()
+        outs = [a if n == shared else torch.empty_like(a) for n in ("dK", "dQ", "dV")]
+        if grid:
+            hip_sdpa.sdpa_bwd_grid(*([x] for x in (K, Q, V, a, G, lse)), *([x] for x in outs), rows, rows,
+                                   rows, rows, hip_sdpa.MASK_CAUSAL, flags=hip_sdpa.OVERWRITE)
+        else:
+            hip_sdpa.sdpa_bwd_tile(K, Q, V, a, G, None, lse, *outs, hip_sdpa.MASK_CAUSAL,
+                                   flags=hip_sdpa.OVERWRITE)
+        torch.cuda.synchronize()
+        return outs
+
+    for got, want in zip(run(name), run(None)):
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
