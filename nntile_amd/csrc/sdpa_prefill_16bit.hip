@@ -2189,12 +2189,20 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
     return NNTILE_HIP_OK;
 }
 
-// How the keys of a launch lie on the XCDs: `steps` key steps an entry of the batch, of
-// which `fit` leading ones, of all entries that an XCD works on, have room in 3 of its
-// L2's 4 MiB; `group` heads of an XCD share their keys.
+// Key steps an entry of the batch has.
+static int64_t key_steps(const PrefillParams &p)
+{
+    const int64_t last_keys = p.k_seq - (p.n_kv_tiles - 1) * p.k_tile;
+    return (p.n_kv_tiles - 1) * ((p.k_tile + kKeys - 1) / kKeys) + (last_keys + kKeys - 1) / kKeys;
+}
+
+// How the keys of a launch lie on the XCDs: `fit` leading key steps of all entries that an
+// XCD works on have room in 3 of its L2's 4 MiB; `group` heads of an XCD share their keys.
+// (Asked for only where the rules below need it: a call of a small tile is bound by
+// the host, which its dozens of divisions would keep.)
 struct KeysOnXCD
 {
-    int64_t steps, fit;
+    int64_t fit;
     int group;
 };
 
@@ -2203,8 +2211,6 @@ static KeysOnXCD keys_on_xcd(const PrefillParams &p, int head)
     KeysOnXCD r;
     const int64_t batch_all = (int64_t)p.batch * p.n_slabs;
     const int64_t q_blocks = (p.q_tile + kQRows / 2 - 1) / (kQRows / 2) * p.n_q_tiles;
-    const int64_t last_keys = p.k_seq - (p.n_kv_tiles - 1) * p.k_tile;
-    r.steps = (p.n_kv_tiles - 1) * ((p.k_tile + kKeys - 1) / kKeys) + (last_keys + kKeys - 1) / kKeys;
     int64_t entries = batch_all / 8;
     r.group = 1;
     if(batch_all % 8 == 0)
@@ -2278,11 +2284,11 @@ static bool halved_is_faster(const PrefillParams &p, int head, int mode)
     {
         return false;
     }
-    const KeysOnXCD keys = keys_on_xcd(p, head);
+    const int64_t steps = key_steps(p);
     const bool rule = mode == NNTILE_HIP_MASK_CAUSAL || mode == NNTILE_HIP_MASK_NONE;
     // Rectangular calls of few steps are left to the other forms, so that what one
     // computes does not depend on how many entries share its launch.
-    if(rule && p.q_seq != p.k_seq && keys.steps < kHalvedSteps)
+    if(rule && p.q_seq != p.k_seq && steps < kHalvedSteps)
     {
         return false;
     }
@@ -2291,25 +2297,29 @@ static bool halved_is_faster(const PrefillParams &p, int head, int mode)
         case NNTILE_HIP_MASK_CAUSAL:
             // (beyond 256 workgroups where the rule hides enough to make long and short
             // ones: 64 heads, 333 queries behind 1500 keys 33.9 / 36.8)
-            return n_wg <= kCUs || ((head == 64 ? 2 : 1) * keys.fit >= keys.steps
-                    && p.q_pos0 + p.causal_offset - p.k_pos0 < p.k_seq / 2);
+            return n_wg <= kCUs || (p.q_pos0 + p.causal_offset - p.k_pos0 < p.k_seq / 2
+                    && (head == 64 ? 2 : 1) * keys_on_xcd(p, head).fit >= steps);
         case NNTILE_HIP_MASK_NONE:
-            return n_wg <= kCUs && (keys.steps < 2 * kTouchSteps || 2 * keys.fit >= keys.steps);
+            return n_wg <= kCUs && (steps < 2 * kTouchSteps || 2 * keys_on_xcd(p, head).fit >= steps);
         default:
-            return n_wg <= kCUs || (keys.steps >= kTouchStepsMask ? keys.fit >= keys.steps : head == 64);
+            return n_wg <= kCUs || (steps >= kTouchStepsMask ? keys_on_xcd(p, head).fit >= steps : head == 64);
     }
 }
 
 // Which lines of K and V the workgroups of a launch touch before they begin.
 static void set_touch(PrefillParams &p, int head, int mode, int64_t n_wg)
 {
-    const KeysOnXCD keys = keys_on_xcd(p, head);
+    const int64_t steps = key_steps(p);
     const bool rule = mode == NNTILE_HIP_MASK_CAUSAL || mode == NNTILE_HIP_MASK_NONE;
-    if(keys.steps >= (rule || head == 64 || n_wg <= 8 * kCUsPerXCD ? kTouchSteps : kTouchStepsMask)
-            && 3 * keys.fit >= keys.steps)
+    if(steps < (rule || head == 64 || n_wg <= 8 * kCUsPerXCD ? kTouchSteps : kTouchStepsMask))
+    {
+        return;
+    }
+    const KeysOnXCD keys = keys_on_xcd(p, head);
+    if(3 * keys.fit >= steps)
     {
         p.touch_group = keys.group;
-        p.touch_steps = (int)std::min(keys.steps, keys.fit);
+        p.touch_steps = (int)std::min(steps, keys.fit);
     }
 }
 
