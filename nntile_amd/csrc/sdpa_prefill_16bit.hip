@@ -327,50 +327,6 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     }
     const int kvb = kv_entry(b, p.n_batch, p.kv_group);
 
-    // ---- keys and values into this XCD's L2 ----------------------------------------
-    // Workgroups of the same keys on one XCD walk them side by side, and what none of
-    // them has read yet comes from HBM at every step, later than the loop asks for it
-    // ahead.  So each touches a share of the lines first, four a thread at most.
-    constexpr int NT = KH > 1 ? 4 : 1;
-    uint32_t touched[NT];
-    auto touch_keys = [&]() __attribute__((always_inline))
-    {
-        if(p.touch_steps > 0)
-        {
-            constexpr int LINES = kKeys * RB / 128;     // of a step's K, and of its V
-            const int share = n_places * p.touch_group;
-            const int idx = p.touch_group > 1
-                ? my_place * p.touch_group + (b / p.n_batch) % p.touch_group : my_place;
-            const int n_lines = p.touch_steps * 2 * LINES;
-#pragma unroll
-            for(int i = 0; i < NT; ++i)
-            {
-                const int line = (i * share + idx) * kThreads + tid;
-                if(line < n_lines)
-                {
-                    const int st = line / (2 * LINES), in = line % (2 * LINES);
-                    const int kt = p.n_kv_tiles > 1 ? st / p.k_blocks_per_tile : 0;
-                    const int64_t rows = min(p.k_tile, p.k_seq - kt * p.k_tile);
-                    const int64_t at = min((int64_t)(st - kt * p.k_blocks_per_tile) * (kKeys * RB)
-                            + (in % LINES) * 128, rows * RB - 16)
-                        + (int64_t)kvb * (p.kv_rows > 0 ? p.kv_rows : rows) * RB;
-                    touched[i] = *reinterpret_cast<const volatile uint32_t *>(
-                            static_cast<const char *>(in < LINES ? p.K[k_tile0 + kt]
-                                : p.V[k_tile0 + kt]) + at);
-                }
-            }
-        }
-    };
-#pragma unroll
-    for(int i = 0; i < NT; ++i)
-    {
-        touched[i] = 0u;
-    }
-    if constexpr(KH > 1 && !EXPLICIT)
-    {
-        touch_keys();
-    }
-
     const uint16_t *Qt = static_cast<const uint16_t *>(p.Q[q_tile0 + qt])
         + (int64_t)b * q_len * HEAD;
     const int my_q = q_row0 + rb * 32 + col;            // row within tile
@@ -1055,16 +1011,54 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             mask_fetch(cur.kb, cur.rows_left);
         }
     }
-    if constexpr(KH > 1 && EXPLICIT)
+    // ---- keys and values into this XCD's L2 ----------------------------------------
+    // Workgroups of the same keys on one XCD walk them side by side, and what none of
+    // them has read yet comes from HBM at every step, later than the loop asks for it
+    // ahead.  So each touches a share of the lines first, four a thread at most, behind
+    // its own first step's loads and where it has a step to take.  A wavefront's 64 lines
+    // lie in one step of one of the two, so that where they are is scalar work and
+    // nothing stands between the loads.  (Through a volatile pointer each load was waited
+    // for before the next; so / now, causal, us: head 128, 25 x 1024 20.9 / 18.8, 32 x 1024 20.6 /
+    // 19.2, 8 x 4096 48.8 / 46.8, 8 x 1000 14.8 / 14.2; head 64, 40 x 1000 15.2 / 14.3; masks as
+    // values, head 64, 9 x 2048 25.1 / 24.0, open 30.2 / 29.2.)
+    if constexpr(KH > 1)
     {
-        touch_keys();       // (what the mask hides from everyone is not wanted)
+        if(p.touch_steps > 0 && n_steps > 0)
+        {
+            constexpr int NT = 4;
+            constexpr int LINES = kKeys * RB / 128;     // of a step's K, and of its V
+            static_assert(LINES % 64 == 0, "a wavefront's lines lie in one step's K or V");
+            const int share = n_places * p.touch_group;
+            const int idx = p.touch_group > 1
+                ? my_place * p.touch_group + (b / p.n_batch) % p.touch_group : my_place;
+            const int n_lines = p.touch_steps * 2 * LINES;
+            uint32_t touched[NT];
+#pragma unroll
+            for(int i = 0; i < NT; ++i)
+            {
+                const int line = __builtin_amdgcn_readfirstlane((i * share + idx) * kThreads + wave * 64);
+                touched[i] = 0u;
+                if(line < n_lines)
+                {
+                    const int st = line / (2 * LINES), in = line % (2 * LINES);
+                    const int kt = p.n_kv_tiles > 1 ? st / p.k_blocks_per_tile : 0;
+                    const int64_t rows = min(p.k_tile, p.k_seq - kt * p.k_tile);
+                    const int64_t at = min((int64_t)(st - kt * p.k_blocks_per_tile) * (kKeys * RB)
+                            + (in % LINES + lane) * 128, rows * RB - 16);
+                    const char *entry = static_cast<const char *>(in < LINES ? p.K[k_tile0 + kt]
+                            : p.V[k_tile0 + kt]) + (int64_t)kvb * (p.kv_rows > 0 ? p.kv_rows : rows) * RB;
+                    touched[i] = *(const __attribute__((address_space(1))) uint32_t *)(uintptr_t)(entry + at);
+                }
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+            for(int i = 0; i < NT; ++i)
+            {
+                asm volatile("" :: "v"(touched[i]));
+            }
+        }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-    for(int i = 0; i < NT; ++i)
-    {
-        asm volatile("" :: "v"(touched[i]));
-    }
     __syncthreads();
     PF_STAMP(1);
 #ifdef NNTILE_PF_TRACE

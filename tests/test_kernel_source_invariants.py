@@ -164,3 +164,12 @@ def test_decode_partials_have_arrived_before_their_flag_goes_up(assemblies):
             raised += 1
         kernels = re.findall(r"^(_ZN\S+_kernel\S+Lb0E\S*):", assemblies[name], re.M)
         assert raised == len(kernels) > 0, (name, raised, len(kernels))
+
+
+def test_nothing_is_read_past_the_caches(assemblies):
+    """A read through a volatile pointer bypasses the caches' scope and is waited for at
+    once, whatever else could be in flight beside it: the forward of halved steps
+    once touched its key lines so, four memory round trips one after the other."""
+    for name, text in assemblies.items():
+        for line in _instructions(text):
+            assert not re.match(r"(flat|global)_load_(dword|ushort|ubyte)\S* .*\bsc0 sc1$", line), (name, line)
