@@ -153,8 +153,8 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // have no second workgroup to put on a CU: two wavefronts per SIMD (one's
     // softmax beside the other's MFMAs) and half the chain of dependent steps.
     constexpr int QW = WAVES / GROUPS;      // wavefronts that share a key step
-    constexpr int kQRows = QW / KH * 32;
-    constexpr int kThreads = WAVES * 64;
+    constexpr int ROWS = QW / KH * 32;      // queries of the workgroup
+    constexpr int THREADS = WAVES * 64;
     constexpr int NB = 2 / KH;              // 32-key blocks of a step that a wavefront takes
     typedef typename T::vec8 vec8;
     constexpr int KSTEPS = HEAD / 16;       // MFMA steps along head for S
@@ -320,7 +320,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     const int qt = qblk / p.q_blocks_per_tile;
     const int qb = qblk % p.q_blocks_per_tile;
     const int q_len = (int)min(p.q_tile, p.q_seq - (int64_t)qt * p.q_tile);
-    const int q_row0 = qb * kQRows;                     // within the tile
+    const int q_row0 = qb * ROWS;                     // within the tile
     if(q_row0 >= q_len)
     {
         return;
@@ -369,7 +369,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             + p.causal_offset - p.k_pos0 - part_k0;
         rel = max((int64_t)-(1 << 30), min(rel, (int64_t)(1 << 30)));
         rel0 = (int)rel;
-        const int hi = min(rel0 + min(kQRows, q_len - q_row0) - 1, k_seq - 1);
+        const int hi = min(rel0 + min(ROWS, q_len - q_row0) - 1, k_seq - 1);
         if(hi < 0)
         {
             if(!overwrite())
@@ -825,7 +825,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         unsigned long long not_open = 0ull, not_hidden = 0ull;
         bool scanned = false;
         // the block of 128 rows that the words of a scan done for everybody are about
-        const int scan_blk = q_row0 / nntile_hip::kQRows;
+        const int scan_blk = q_row0 / kQRows;
         if(n_steps > 0 && p.mask_bits != nullptr && p.n_scan_wgs == 0)
         {
             // the scan was done once for all batch entries before the launch
@@ -914,10 +914,10 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
             __shared__ unsigned long long scan_words[2 * WAVES];
             // (rows as in a scan done for everybody: a call's bits do not depend on which
             // of the two it has)
-            const int scan_row0 = scan_blk * nntile_hip::kQRows;
+            const int scan_row0 = scan_blk * kQRows;
             mask_scan_steps<ES, WAVES, kKeys>(static_cast<const char *>(p.mask)
                     + (int64_t)scan_row0 * p.mask_ld * ES, (uint32_t)(p.mask_ld * ES),
-                    min(nntile_hip::kQRows, q_len - scan_row0), k_seq * ES, 0, (k_seq + kKeys - 1) / kKeys,
+                    min(kQRows, q_len - scan_row0), k_seq * ES, 0, (k_seq + kKeys - 1) / kKeys,
                     OPEN, HIDDEN, scan_words, not_open, not_hidden);
             scanned = true;
         }
@@ -1036,7 +1036,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
 #pragma unroll
             for(int i = 0; i < NT; ++i)
             {
-                const int line = __builtin_amdgcn_readfirstlane((i * share + idx) * kThreads + wave * 64);
+                const int line = __builtin_amdgcn_readfirstlane((i * share + idx) * THREADS + wave * 64);
                 touched[i] = 0u;
                 if(line < n_lines)
                 {
@@ -1975,7 +1975,6 @@ template<typename T, int HEAD>
 static int launch_mode(hipStream_t stream, const PrefillParams &p, int mode,
         dim3 grid, bool wide, bool key_split, bool halved)
 {
-    constexpr int kThreads = 256;
     if constexpr(HEAD >= 64)
     {
         if(halved)

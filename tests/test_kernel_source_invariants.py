@@ -173,3 +173,16 @@ def test_nothing_is_read_past_the_caches(assemblies):
     for name, text in assemblies.items():
         for line in _instructions(text):
             assert not re.match(r"(flat|global)_load_(dword|ushort|ubyte)\S* .*\bsc0 sc1$", line), (name, line)
+
+
+def test_no_constant_of_a_kernel_hides_one_of_its_file():
+    """The forward of halved steps has 64 rows a workgroup where the file's constant of
+    the same name said 128, and a bound on the scan of 128 mask rows was taken with 64."""
+    def constants(text, indent):
+        return set(re.findall(r"^%s(?:static )?constexpr \w+ (k[A-Z]\w*)" % indent, text, re.M))
+
+    common = open(os.path.join(B.CSRC, "sdpa_common.hpp")).read()
+    for name in B.SOURCES:
+        text = open(os.path.join(B.CSRC, name)).read()
+        hidden = constants(text, r"[ \t]+") & (constants(text, "") | constants(common, ""))
+        assert not hidden, (name, hidden)
