@@ -52,7 +52,8 @@ struct PrefillParams
     const void *mask;
     // explicit masks, one query tile: what a scan of the mask rows of every
     // 128-query block found - kMaskBitSplits entries per block, one per range of
-    // keys, to be OR-ed.  Two bit sets: bit s of the first: some value of 64-key
+    // keys, to be OR-ed (launches of 64-query workgroups: of every 64-query block, half as
+    // many).  Two bit sets: bit s of the first: some value of 64-key
     // step s is not "open", of the second: not "hidden" (steps from 63 on share
     // bit 63).  An entry is kMaskBitWords words (sdpa_mask_words.hpp).  Null: every
     // workgroup scans its own rows.

@@ -91,18 +91,23 @@ extern "C" int nntile_hip_debug_pf_trace(unsigned long long *host)
 // CU.  8 (analytic masks, head 64 and 128): one workgroup of 256 queries per
 // CU, whose eight wavefronts share every K/V step - a CU then brings each step
 // into LDS once where two workgroups of four bring it twice.
-// Key range sp of kMaskBitSplits of query block qb, for the scan that is done
-// once for all batch entries.
-template<int ES, int NWAVES>
+// The scan that is done once for all batch entries: blocks of as many rows as the
+// attention workgroups have, each in key ranges, so that a scanning workgroup reads as
+// much of blocks of 64 rows (four ranges) as of 128.
+template<int ROWS>
+constexpr int kScanSplits = ROWS < kQRows ? kMaskBitSplits * ROWS / kQRows : kMaskBitSplits;
+
+// Key range sp of kScanSplits<ROWS> of query block qb.
+template<int ES, int NWAVES, int ROWS>
 __device__ __forceinline__ void mask_scan_range(const char *mask, uint32_t ld_bytes, int q_len,
         int k_seq, uint32_t open_word, uint32_t hidden_word, int qb, int sp,
         unsigned long long *words, unsigned long long &not_open, unsigned long long &not_hidden)
 {
     const int n_steps = (k_seq + kKeys - 1) / kKeys;
-    const int per_split = (n_steps + kMaskBitSplits - 1) / kMaskBitSplits;
+    const int per_split = (n_steps + kScanSplits<ROWS> - 1) / kScanSplits<ROWS>;
     const int s_lo = min(sp * per_split, n_steps);
-    mask_scan_steps<ES, NWAVES, kKeys>(mask + (int64_t)(qb * kQRows) * ld_bytes, ld_bytes,
-            min(kQRows, q_len - qb * kQRows), k_seq * ES, s_lo, min(s_lo + per_split, n_steps),
+    mask_scan_steps<ES, NWAVES, kKeys>(mask + (int64_t)(qb * ROWS) * ld_bytes, ld_bytes,
+            min(ROWS, q_len - qb * ROWS), k_seq * ES, s_lo, min(s_lo + per_split, n_steps),
             open_word, hidden_word, words, not_open, not_hidden);
 }
 
@@ -155,6 +160,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     constexpr int QW = WAVES / GROUPS;      // wavefronts that share a key step
     constexpr int ROWS = QW / KH * 32;      // queries of the workgroup
     constexpr int THREADS = WAVES * 64;
+    constexpr int SCAN_SPLITS = kScanSplits<ROWS>;
     constexpr int NB = 2 / KH;              // 32-key blocks of a step that a wavefront takes
     typedef typename T::vec8 vec8;
     constexpr int KSTEPS = HEAD / 16;       // MFMA steps along head for S
@@ -229,12 +235,16 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 constexpr int ES = (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 2 : 1;
                 __shared__ unsigned long long pub_words[2 * WAVES];
                 unsigned long long pub_open, pub_hidden;
-                mask_scan_range<ES, WAVES>(static_cast<const char *>(p.mask),
+                const int scan_blk = (int)blockIdx.x / SCAN_SPLITS;
+                if(scan_blk * ROWS >= (int)p.q_seq)
+                {
+                    return;     // (there to make their number a multiple of 8)
+                }
+                mask_scan_range<ES, WAVES, ROWS>(static_cast<const char *>(p.mask),
                         (uint32_t)(p.mask_ld * ES), (int)p.q_seq, (int)p.k_seq,
                         (MODE == NNTILE_HIP_MASK_ADDITIVE) ? 0u : 0x01010101u,
                         (MODE == NNTILE_HIP_MASK_ADDITIVE) ? T::kNegInfPair : 0u,
-                        (int)blockIdx.x / kMaskBitSplits, (int)blockIdx.x % kMaskBitSplits,
-                        pub_words, pub_open, pub_hidden);
+                        scan_blk, (int)blockIdx.x % SCAN_SPLITS, pub_words, pub_open, pub_hidden);
                 // written through to memory (device scope), where readers on any
                 // XCD find them; the tag says which are there, none waits for another
                 mask_words_publish(p.mask_bits + kMaskBitWords * (int64_t)blockIdx.x, tid, pub_open,
@@ -824,14 +834,12 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         // bit s: some value of step s (steps >= 63 share bit 63) is not open / not hidden
         unsigned long long not_open = 0ull, not_hidden = 0ull;
         bool scanned = false;
-        // the block of 128 rows that the words of a scan done for everybody are about
-        const int scan_blk = q_row0 / kQRows;
         if(n_steps > 0 && p.mask_bits != nullptr && p.n_scan_wgs == 0)
         {
             // the scan was done once for all batch entries before the launch
-            const unsigned long long *w = p.mask_bits + (int64_t)scan_blk * (kMaskBitWords * kMaskBitSplits);
+            const unsigned long long *w = p.mask_bits + (int64_t)qb * (kMaskBitWords * SCAN_SPLITS);
 #pragma unroll
-            for(int sp = 0; sp < kMaskBitSplits; ++sp)
+            for(int sp = 0; sp < SCAN_SPLITS; ++sp)
             {
                 uint64_t e[MaskWords::N], open, hidden;
 #pragma unroll
@@ -849,11 +857,11 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
         {
             // ... or is being done by the first workgroups of this launch: the
             // first wavefront waits for the entries of the block's key ranges, eight
-            // lanes an entry, a word each (bounded; the Q fragments are on their way
-            // meanwhile), then everybody ORs.  (16 tasks of 4096 tokens, 32 heads, causal:
+            // lanes an entry, a word each (four entries: twice; bounded; the Q fragments are on
+            // their way meanwhile), then everybody ORs.  (16 tasks of 4096 tokens, 32 heads, causal:
             // 300.4 us; 297.5 with four words an entry that were taken one by one, which
             // could be words from before; 4 % more with one lane an entry.)
-            static_assert(kMaskBitSplits == 8 && kMaskBitWords <= 8, "one wavefront reads them all");
+            static_assert(8 % SCAN_SPLITS == 0 && kMaskBitWords <= 8, "one wavefront reads them all");
             __shared__ uint32_t got_bits[4];
             __shared__ int got_all;
             if(tid < 4)
@@ -866,7 +874,7 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 const int i = lane & 7;
                 const bool has_word = i < kMaskBitWords;
                 unsigned long long *e = p.mask_bits
-                    + ((int64_t)scan_blk * kMaskBitSplits + (lane >> 3)) * kMaskBitWords
+                    + ((int64_t)qb * SCAN_SPLITS + (lane >> 3) % SCAN_SPLITS) * kMaskBitWords
                     + (has_word ? i : 0);
                 const unsigned long long t0 = wall_clock64();
                 unsigned long long word;
@@ -908,16 +916,15 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
                 scanned = true;
             }
         }
+        // (the same rows and the same bounds as in a scan done for everybody: a call's bits
+        // do not depend on which of the two it has)
         if(!scanned && n_steps > 0 && k_seq * ES >= 16
                 && p.mask_ld * ES * kQRows < (int64_t)(1 << 30))
         {
             __shared__ unsigned long long scan_words[2 * WAVES];
-            // (rows as in a scan done for everybody: a call's bits do not depend on which
-            // of the two it has)
-            const int scan_row0 = scan_blk * kQRows;
             mask_scan_steps<ES, WAVES, kKeys>(static_cast<const char *>(p.mask)
-                    + (int64_t)scan_row0 * p.mask_ld * ES, (uint32_t)(p.mask_ld * ES),
-                    min(kQRows, q_len - scan_row0), k_seq * ES, 0, (k_seq + kKeys - 1) / kKeys,
+                    + (int64_t)q_row0 * p.mask_ld * ES, (uint32_t)(p.mask_ld * ES),
+                    min(ROWS, q_len - q_row0), k_seq * ES, 0, (k_seq + kKeys - 1) / kKeys,
                     OPEN, HIDDEN, scan_words, not_open, not_hidden);
             scanned = true;
         }
@@ -2071,19 +2078,19 @@ static int launch_mode(hipStream_t stream, const PrefillParams &p, int mode,
 }
 
 // The scan of an explicit mask that every workgroup of the attention kernel
-// would do for its own 128 rows, done once for all batch entries, as a launch
+// would do for its own rows, done once for all batch entries, as a launch
 // of its own (calls under stream capture; otherwise the scan rides in the
 // attention launch): workgroup (query block, key range) writes what it finds
 // to entry blockIdx.x of the table (see PrefillParams::mask_bits), without a tag.
-template<int ES>
+template<int ES, int ROWS>
 __global__ __launch_bounds__(kThreads)
 void mask_step_bits_kernel(const char *mask, uint32_t ld_bytes, int q_len, int k_seq,
         uint32_t open_word, uint32_t hidden_word, unsigned long long *table)
 {
     __shared__ unsigned long long words[2 * kThreads / 64];
     unsigned long long not_open, not_hidden;
-    mask_scan_range<ES, kThreads / 64>(mask, ld_bytes, q_len, k_seq, open_word, hidden_word,
-            (int)blockIdx.x / kMaskBitSplits, (int)blockIdx.x % kMaskBitSplits, words, not_open,
+    mask_scan_range<ES, kThreads / 64, ROWS>(mask, ld_bytes, q_len, k_seq, open_word, hidden_word,
+            (int)blockIdx.x / kScanSplits<ROWS>, (int)blockIdx.x % kScanSplits<ROWS>, words, not_open,
             not_hidden);
     mask_words_publish(table + kMaskBitWords * (int64_t)blockIdx.x, (int)threadIdx.x, not_open,
             not_hidden, 0ull);
@@ -2114,9 +2121,10 @@ static uint64_t next_scan_tag()
 // attention launch itself, or, on a stream that is being captured (a replay
 // would carry this call's tag again and find the words of the replay before
 // it), by a launch of its own.  Leaves p.mask_bits null when the conditions of
-// the kernel's own scan do not hold or the scratch is too small.
+// the kernel's own scan do not hold or the scratch is too small.  halved: the attention
+// workgroups have 64 rows, and so have the scan's blocks.
 template<typename T>
-static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
+static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode, bool halved,
         void *scratch, size_t scratch_bytes)
 {
     p.n_scan_wgs = 0;
@@ -2128,8 +2136,8 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
     }
     const int64_t es = additive ? 2 : 1;
     const int64_t row_bytes = p.k_seq * es;
-    const int64_t scan_blocks = (p.q_seq + kQRows - 1) / kQRows;
-    const int64_t table_bytes = scan_blocks * kMaskBitSplits
+    // (blocks of 64 rows take no more room: what a scratch is good for is one rule)
+    const int64_t table_bytes = (p.q_seq + kQRows - 1) / kQRows * kMaskBitSplits
         * (kMaskBitWords * (int64_t)sizeof(unsigned long long));
     if(row_bytes < 16 || p.mask_ld * es * kQRows >= (int64_t)(1 << 30)
             || reinterpret_cast<uintptr_t>(scratch) % 8 != 0
@@ -2138,7 +2146,9 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
         return NNTILE_HIP_OK;
     }
     auto *table = static_cast<unsigned long long *>(scratch);
-    const dim3 grid((unsigned)(scan_blocks * kMaskBitSplits));
+    constexpr int kHalf = kQRows / 2;
+    const int64_t n_scan = halved ? (p.q_seq + kHalf - 1) / kHalf * kScanSplits<kHalf>
+        : (p.q_seq + kQRows - 1) / kQRows * kScanSplits<kQRows>;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if(hipStreamIsCapturing(stream, &capturing) != hipSuccess)
     {
@@ -2153,26 +2163,30 @@ static int scan_mask_once(hipStream_t stream, PrefillParams &p, int mode,
     if(capturing == hipStreamCaptureStatusNone)
     {
         p.mask_bits = table;
-        p.n_scan_wgs = (int32_t)grid.x;
+        p.n_scan_wgs = (int32_t)((n_scan + 7) / 8 * 8);
         p.mask_tag = next_scan_tag();
-        // A scan takes 2 us, or what 128 rows of an eighth of the keys take a
-        // workgroup: well below a byte of a row a tick of the 100 MHz clock.  Words that
+        // A scan takes 2 us, or what 128 rows of an eighth of the keys (64 of a
+        // quarter) take a workgroup: well below a byte of a row a tick of the 100 MHz clock.  Words that
         // are not there then were overwritten, by a call on another stream that
         // was lent the same memory.
         p.mask_spin_limit = 2000ull + (unsigned long long)row_bytes;
         return NNTILE_HIP_OK;
     }
+    auto launch = [&](auto kernel, uint32_t open_word, uint32_t hidden_word)
+    {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)n_scan), dim3(kThreads), 0, stream,
+                static_cast<const char *>(p.mask), (uint32_t)(p.mask_ld * es), (int)p.q_seq,
+                (int)p.k_seq, open_word, hidden_word, table);
+    };
     if(additive)
     {
-        hipLaunchKernelGGL((mask_step_bits_kernel<2>), grid, dim3(kThreads), 0, stream,
-                static_cast<const char *>(p.mask), (uint32_t)(p.mask_ld * es), (int)p.q_seq,
-                (int)p.k_seq, 0u, T::kNegInfPair, table);
+        launch(halved ? mask_step_bits_kernel<2, kHalf> : mask_step_bits_kernel<2, kQRows>, 0u,
+                T::kNegInfPair);
     }
     else
     {
-        hipLaunchKernelGGL((mask_step_bits_kernel<1>), grid, dim3(kThreads), 0, stream,
-                static_cast<const char *>(p.mask), (uint32_t)(p.mask_ld * es), (int)p.q_seq,
-                (int)p.k_seq, 0x01010101u, 0u, table);
+        launch(halved ? mask_step_bits_kernel<1, kHalf> : mask_step_bits_kernel<1, kQRows>, 0x01010101u,
+                0u);
     }
     if(hipGetLastError() != hipSuccess)
     {
@@ -2372,7 +2386,7 @@ int launch_prefill_16bit(hipStream_t stream, PrefillParams &p, int head,
         set_touch(p, head, mode, n_wg);
     }
     p.mask_bits = nullptr;
-    const int scan_rc = scan_mask_once<T>(stream, p, mode, scan_scratch, scan_scratch_bytes);
+    const int scan_rc = scan_mask_once<T>(stream, p, mode, halved, scan_scratch, scan_scratch_bytes);
     if(scan_rc != NNTILE_HIP_OK)
     {
         return scan_rc;
