@@ -800,8 +800,18 @@ void sdpa_prefill_16bit_kernel(const PrefillParams p)
     // any of it unnecessary, which costs nothing but the request.  (Not the
     // first step's mask values: 16 loads that touch 32 rows each delay the
     // scan more than they save, 6 % on 4 x 4 tiles of 355 keys.)
+    // Workgroups of 64 queries are twice as many, and together their requests delay the
+    // scan: those that scan for themselves make none, nor do the others of a
+    // launch of about a workgroup a CU and more (two at head 64).  us, every workgroup's
+    // requests made / not, what a mask hides wholly: head 128, 32 x 500 4.7 / 4.3, 16 x 2048
+    // 8.8 / 7.6; head 64, 32 x 1024 5.0 / 4.5, 24 x 2000 7.3 / 6.9, 64 x 700 5.4 / 4.9; below
+    // that the others lose by it: 9 x 1700 of head 128, causal, 26.3 / 27.3, 4 x 2048 open 26.7 /
+    // 27.5, 16 x 1024 of head 64 open 15.3 / 15.9, 36 x 500 causal 12.1 / 12.6.  Without a
+    // shared scan, hidden: 16 x 1500 of head 128 14.9 / 14.2, 24 x 2000 of head 64 18.8 / 17.9, causal
+    // 34.7 / 35.1.
+    const bool early = KH == 1 || (p.mask_bits != nullptr && n_att * HEAD < 2u * 8u * kCUsPerXCD * 64u);
     bool first_requested = false;
-    if(EXPLICIT)
+    if(EXPLICIT && early)
     {
         const int own = GROUPS > 1 ? max(n_steps - grp + GROUPS - 1, 0) / GROUPS : n_steps;
         if(own > 0)
