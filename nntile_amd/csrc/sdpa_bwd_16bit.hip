@@ -410,10 +410,16 @@ void sdpa_bwd_prelude_kernel(const BwdPreludeParams p)
 constexpr int kBwdOwnRows = 128;            // queries of a walk, all heads of a group
 constexpr int kBwdOwnSteps = kBwdOwnRows / kBwdStep;
 
-// Row dots of `rows` rows from dA, A on, by 256 threads, into out.
+// Row dots of `rows` rows, q_seq of each head of a group, by 256 threads, into out.  dA, A:
+// the first; head_gap: elements between the rows of one head and those of the next.
+// (All heads in one run: a loop over the heads waits for memory once for each, and a
+// group of many heads has few rows of one.  With the launch in front / a loop / now, us, bf16, no
+// mask: head 64, 2 groups of 128 heads of a row 115 / 189 / 88, 4 of 32 x 4 30 / 50 / 24, 8 of 16 x 8
+// 18.7 / 27 / 14.7, 2 of 8 x 16 12.8 / 15.5 / 9.4, 16 of 4 x 32 10.0 / 10.1 / 7.3; head 128, 2 of 128 x
+// 1 151 / 231 / 116, 8 of 16 x 8 26 / 35 / 21.)
 template<typename T, int HEAD>
 __device__ __forceinline__ void bwd_own_row_dots(const uint16_t *dA, const uint16_t *A, int rows,
-        float *out)
+        int q_seq, int64_t head_gap, float *out)
 {
     constexpr int LANES = HEAD / 8, ROWS = 256 / LANES, N = 4;
     const int part = (int)threadIdx.x % LANES, row0 = (int)threadIdx.x / LANES;
@@ -424,8 +430,9 @@ __device__ __forceinline__ void bwd_own_row_dots(const uint16_t *dA, const uint1
         for(int i = 0; i < N; ++i)
         {
             const int row = min(base + i * ROWS + row0, rows - 1);
-            g[i] = *reinterpret_cast<const u32x4 *>(dA + row * HEAD + part * 8);
-            a[i] = *reinterpret_cast<const u32x4 *>(A + row * HEAD + part * 8);
+            const int64_t at = (rows > q_seq ? row / q_seq * head_gap : 0) + row * HEAD + part * 8;
+            g[i] = *reinterpret_cast<const u32x4 *>(dA + at);
+            a[i] = *reinterpret_cast<const u32x4 *>(A + at);
         }
 #pragma unroll
         for(int i = 0; i < N; ++i)
@@ -1857,13 +1864,14 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     }
     if constexpr(OWN && DO_DK)
     {
-        for(int g = 0; g < p.kv_group; ++g)
+        if(i_cur >= 0)
         {
-            const QueryRows at = query_rows(nb + p.n_batch * (g + p.kv_group * hkv), 0);
+            const QueryRows at = query_rows(nb + p.n_batch * (p.kv_group * hkv), 0);
             bwd_own_row_dots<T, HEAD>(static_cast<const uint16_t *>(at.dA) + at.elem * HEAD,
-                    static_cast<const uint16_t *>(p.A) + at.elem * HEAD, q_seq, lds_own + g * q_seq);
+                    static_cast<const uint16_t *>(p.A) + at.elem * HEAD, p.kv_group * q_seq, q_seq,
+                    (int64_t)(p.n_batch - 1) * q_seq * HEAD, lds_own);
+            __syncthreads();
         }
-        __syncthreads();
     }
     if(i_cur >= 0)
     {
