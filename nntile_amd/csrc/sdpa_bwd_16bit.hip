@@ -2690,18 +2690,10 @@ __device__ __forceinline__ void sdpa_bwd_dkv_body(
     char *xch = (wave_u == 0 ? lds_q0 : wave_u == 1 ? lds_q1 : wave_u == 2 ? lds_g0 : lds_g1) + lds_grp;
     if constexpr(GROUPS > 1)
     {
-        if(DO_DK)
-        {
-            bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, dk);
-        }
-        if(BOTH)
-        {
-            __syncthreads();        // (the first sums have been read)
-        }
-        if(DO_DV)
-        {
-            bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, dv);
-        }
+        static_assert(BOTH, "two groups: both gradients in one workgroup");
+        bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, dk);
+        __syncthreads();            // (the first sums have been read)
+        bwd_add_groups<DBLOCKS, G::BYTES>(grp, xch, dv);
         if(grp == 1)
         {
             return;
