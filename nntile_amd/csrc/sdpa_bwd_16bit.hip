@@ -2837,8 +2837,22 @@ static int64_t bwd_longest_walk(const BwdParams &p)
 // SIMD, waiting for its own operands, have twice the workgroups so with half of the chain
 // each, and skip blocks of a mask for 64 rows instead of 128; a launch that fills the chip
 // loses by it, as every step comes into LDS twice as often for its MFMAs (32 x 4096 of head
-// 128, causal, 463 / 594 us).  Whole calls, us, fp16, before / with dK and dV apart / with
-// both in one workgroup (head 64; at head 128 it does not fit the registers):
+// 128, causal, 463 / 594 us).
+//
+// The rule, in workgroups of 64 rows, dK and dV apart / together in one (head 64; at head
+// 128 that does not fit the registers):
+//   masks as values     apart up to two a CU, else together up to two
+//   a rule, head 64     apart up to one a CU, else together up to four (open: two), or where
+//                       a group's heads make the key blocks' walks the longest: 256 (208) of them
+//   a rule, head 128    apart up to three a CU (open: two), or 256 (128) of grouped heads
+// but for two lines that are not there for speed: launches on either side of them give
+// equal bits, which tests of this repository hold them to (the calls over slabs of 12
+// heads of 1024 rows in test_gpu_backward_grid.py, the rectangular ones of
+// test_gpu_backward_wide_keys.py), although a call's last bit may otherwise depend on
+// what shares its launch (head 64, causal, whole / halved: 12 x 1024 23.8 / -, beside it 16 x
+// 1000 26.5 / 20.8).
+//
+// Whole calls, us, fp16, before / apart / together:
 //   masks as values, head 64: 2 x 128 10.9 / 8.9 / 10.3, 12 x 500 causal 18.1 / 14.8 / 16.7,
 //     open 18.7 / 18.2 / 18.0, a window 18.2 / 13.8 / 17.7; 8 x 1000 25.3 / 23.7 / 23.9, 27.3 /
 //     26.9 / 26.4, 19.0 / 14.7 / 18.9; 32 x 500 24.1 / 22.2 / 19.9, 26.1 / 24.4 / 21.9, 25.0 / 18.7 /
@@ -2866,9 +2880,7 @@ static int bwd_halved(const BwdParams &p, int head, int mode, int64_t entries, i
         return apart <= 2 * kBwdCUs ? BWD_HALVED_APART
             : head == 64 && both <= 2 * kBwdCUs ? BWD_HALVED_BOTH : BWD_WHOLE_STEPS;
     }
-    // (beyond two workgroups a CU short walks of entries that do not come in eights, whose
-    // keys every XCD reads, are left in whole steps: a call then gives the bits that its
-    // entries have in a larger launch)
+    // (the first of those lines: short walks of entries that do not come in eights)
     if(apart > 2 * kBwdCUs && entries % 8 != 0 && bwd_longest_walk(p) <= 16)
     {
         return BWD_WHOLE_STEPS;
@@ -2879,8 +2891,7 @@ static int bwd_halved(const BwdParams &p, int head, int mode, int64_t entries, i
             || (p.kv_group >= (causal ? 2 : 4) && n_dkv <= (causal ? 256 : 208));
         return apart <= kBwdCUs ? BWD_HALVED_APART : few ? BWD_HALVED_BOTH : BWD_WHOLE_STEPS;
     }
-    // (rectangular calls of short walks are taken in whole steps, so that what one
-    // computes does not depend on how many entries share its launch)
+    // (the second: rectangular calls of short walks)
     if(p.q_seq != p.k_seq && bwd_longest_walk(p) < kBwdLongWalk)
     {
         return BWD_WHOLE_STEPS;

@@ -2253,48 +2253,62 @@ static KeysOnXCD keys_on_xcd(const PrefillParams &p, int head)
 }
 
 // From how many key steps on the first touch of the keys pays (us, touched / not, inputs
-// of other calls in between; bf16, head 128): 8 entries of 500 keys 11.2 / 11.0, of 1024
-// 14.9 / 15.7 (without a mask the same), of 2048 causal 23.1 / 28.8, 4 of 4096 37.9 / 50.6;
-// head 64, 8 of 1024 12.0 / 12.5, 4 of 4096 30.4 / 34.6.  128 queries a workgroup lose
-// by it: 32 x 1024 causal 24.2 / 21.8, 12 x 1500 27.5 / 26.0.
+// of other calls in between; bf16, causal): head 128, 8 entries of 1024 keys 14.6 / 15.3 (without
+// a mask 15.0 / 15.7), 8 x 2048 23.3 / 26.1, 4 x 4096 39.1 / 45.4, 16 x 2048 28.8 / 30.1; head 64, 24 x
+// 1300 16.3 / 17.0, 8 x 4096 34.5 / 37.1, its mask as values 40.5 / 51.5.  From fewer steps on some
+// lose: 12 x 300 of head 64 8.2 / 7.7, 12 x 800 12.1 / 11.5, head 128 30 x 900 20.8 / 19.6, 36 x 500
+// 13.6 / 13.0, 8 x 700 12.4 / 12.6.
 constexpr int64_t kTouchSteps = 16;
 // ... with masks given as values and more than 256 workgroups at head 128: 24 x 1024
-// without a hidden key 26.7 / 25.4, 16 x 1500 under a causal mask 26.9 / 31.5
+// without a hidden key 26.7 / 25.4, 16 x 1500 causal 25.2 / 26.6, open 33.9 / 32.7, a window 16.1 / 15.9,
+// 16 x 2048 32.0 / 32.6, 45.7 / 44.5, 19.1 / 18.3
 constexpr int64_t kTouchStepsMask = 24;
 
 // Steps from which rectangular calls with an analytic mask may be halved (see below)
 constexpr int64_t kHalvedSteps = 8;
 
-// Workgroups of 64 queries whose wavefronts halve the key steps between them: launches
-// of at most 256 workgroups of 128 queries (head 64: see below).  Twice the workgroups with half of the chain
-// each, on CUs that would stand empty (up to 256 of them), or two on a CU, long
-// beside short (causal); but each step comes into LDS twice as often for its MFMAs, and with
-// two such workgroups a CU and no mask that is what bounds the launch.  us before /
-// now, bf16, inputs of other calls in between:
-//   up to 256 workgroups, head 128: 8 x 128 causal 8.1 / 6.8, 4 x 300 11.7 / 9.0, 8 x 500
-//   15.1 / 11.0, 8 x 1024 19.9 / 14.9, 8 x 2048 30.8 / 23.1, open 31.1 / 25.2, 4 x 4096
-//   50.5 / 37.9, open 51.1 / 43.4; head 64: 8 x 500 10.6 / 8.9, 4 x 4096 37.0 / 30.4; masks
-//   as values: 4 x 128 11.4 / 9.5, 8 x 500 17.6 / 14.2, open 17.0 / 14.0, a window 15.6 / 12.5,
-//   hidden 4.2 / 4.2.  Not where the keys of an open launch outgrow the L2: 1 x 16384
-//   171.6 / 177.3.
-//   257 to 512, causal: 32 x 700 18.1 / 16.5, 32 x 1024 21.8 / 20.8, 8 x 4096 53.3 / 47.3;
-//   head 64 15.7 / 14.1, 38.1 / 33.2, up to 768 40 x 1000 19.2 / 15.7, 24 x 2000 30.7 / 23.3, 12 x 4096
-//   51.4 / 41.1, 100 x 330 11.4 / 11.7 (not); 12 x 2048 of head 128 31.0 / 26.1, 36 x 500 16.3 / 13.9, 200 x
-//   128 10.0 / 9.3; 4 x 8192, whose keys outgrow the L2, 94.7 / 96.5: not.  Open: 32 x 1024 24.4 /
-//   26.6.
-//   257 to 512, masks as values: what they hide is not known here.  Head 64, 36 x 500:
-//   causal 15.5 / 13.2, open 15.0 / 14.2, hidden 4.5 / 4.6; 32 x 1024 21.8 / 18.3, 20.8 / 20.1,
-//   4.5 / 5.1; 9 x 2048 26.4 / 24.3, 27.7 / 29.2; up to 768 24 x 2000 36.2 / 28.5, 43.9 / 42.0, 6.1 /
-//   7.5, 64 x 700 18.5 / 17.9, 22.7 / 21.1, 4.8 / 5.3.  Head 128, 32 x 1024: causal 27.6 / 24.1, open
-//   27.3 / 30.0, hidden 5.0 / 6.4: not; 16 x 1500 34.7 / 26.9, 34.5 / 34.9, 6.2 / 6.4, 16 x 2048 41.6 /
-//   33.4, 45.4 / 46.9, 8.3 / 8.6, 15 x 1622 35.5 / 32.0, 36.8 / 38.1; not where the keys outgrow the L2.
+// Workgroups of 64 queries whose wavefronts halve the key steps between them: twice the
+// workgroups with half of the chain each, on CUs that would stand empty, or two on a CU,
+// long beside short (causal); but each step comes into LDS twice as often for its MFMAs, and with
+// two such workgroups a CU and no mask that is what bounds the launch.
+//
+// The rule, in workgroups of 64 queries:
+//   up to 256         all launches, but long open ones whose keys outgrow the L2
+//   257 to about 512  (at most 256 of 128 queries) not without a mask; causal by rule where it hides
+//                     enough and the keys fit the L2; masks as values: head 64, and from
+//                     24 steps on, where the keys fit it, both heads
+//   to 768, head 64   three fit a CU: under a mask, entries in eights; other numbers of
+//                     entries only the longest causal rows
+// but for one line that is not there for speed: rectangular calls by rule of fewer than 8 steps
+// give equal bits whatever number of entries shares their launch, which a test of this
+// repository holds them to (test_gpu_backward_wide_keys.py, through the output that the
+// gradients start from), although a call's last bit may otherwise depend on that.
+//
+// us, 128-query forms / halved, bf16, inputs of other calls in between:
+//   up to 256, head 128: 8 x 128 causal 8.1 / 6.8, 4 x 300 11.7 / 9.0, 8 x 500 15.1 / 10.6, 8 x 1024 19.9 /
+//   14.6, 8 x 2048 30.8 / 23.3, open 31.1 / 24.9, 4 x 4096 50.5 / 38.6, open 51.3 / 44.3; head 64: 8 x 500
+//   10.6 / 8.9, 4 x 4096 37.0 / 30.4; masks as values, causal, open, window, hidden: head 128, 8 x 1024
+//   23.8 22.7 16.0 4.3 / 17.3 17.5 12.2 4.4, 8 x 2048 36.0 36.8 18.9 6.1 / 27.3 29.3 14.6 6.0, 32 x 500
+//   18.4 18.2 16.2 4.3 / 15.1 15.8 13.0 4.3; head 64, 12 x 1000 20.6 20.3 13.8 4.5 / 15.2 16.0 11.0
+//   4.4.  Not where the keys of an open launch outgrow the L2: 1 x 16384 171.6 / 177.3.
+//   257 to 512, causal: head 128, 32 x 700 17.0 / 14.6, 32 x 1024 22.2 / 19.2, 8 x 4096 54.3 / 46.8, 12 x 2048
+//   31.0 / 25.0, 25 x 1024 23.3 / 18.8, 36 x 500 16.0 / 12.7, 200 x 128 10.1 / 9.5; head 64, 20 x 1500
+//   19.5 / 16.5, 8 x 4096 38.3 / 32.9; up to 768 40 x 1000 18.0 / 14.3, 24 x 2000 29.2 / 23.5, 12 x 4096 50.0 /
+//   41.9, 96 x 330 10.9 / 9.5, 104 x 330 11.2 / 9.8, but 100 x 330 11.4 / 11.7 and 33 x 1300 22.7 / 23.2 before
+//   the touch was one batch.  4 x 8192 of head 128, whose keys outgrow the L2, 94.7 / 96.5: not.  Open:
+//   32 x 1024 24.4 / 26.6.
+//   257 to 512, masks as values (what they hide is not known here), causal, open, window,
+//   hidden: head 64, 36 x 500 15.5 15.2 13.6 4.5 / 12.1 14.0 10.9 4.3, 32 x 1024 20.8 20.5 14.3 4.5 / 16.8
+//   19.9 12.0 4.5, 9 x 2048 26.8 28.2 15.0 7.0 / 23.4 29.1 14.1 6.0, 16 x 2048 28.1 30.4 15.7 7.3 / 24.9
+//   31.1 13.4 6.0; up to 768 24 x 2000 35.5 46.0 18.3 6.3 / 28.0 43.1 16.7 6.8, 64 x 700 17.7 23.3 15.7
+//   4.9 / 15.8 21.6 13.8 4.8; head 128, 16 x 1500 33.1 35.5 18.9 6.3 / 25.9 34.9 16.4 5.6, 16 x 2048 39.6
+//   46.9 22.6 8.6 / 33.0 47.1 19.4 7.6, 15 x 1622 35.3 37.6 19.4 6.5 / 30.8 37.5 18.0 5.7; with fewer
+//   steps 32 x 1024 27.6 27.3 - 5.0 / 24.1 30.0 - 6.4: not; nor where the keys outgrow the L2.
 static bool halved_is_faster(const PrefillParams &p, int head, int mode)
 {
     const int64_t tiles = (int64_t)p.batch * p.n_slabs * p.n_q_tiles;
     constexpr int64_t kCUs = 8 * kCUsPerXCD;
     const int64_t n_wg = tiles * ((p.q_tile + kQRows / 2 - 1) / (kQRows / 2));
-    // (head 64: three fit a CU; where entries do not come in eights the longest rows only:
-    // 33 x 1300 22.7 / 23.2)
     const bool three = head == 64 && mode != NNTILE_HIP_MASK_NONE && n_wg <= 3 * kCUs
         && (tiles % 8 == 0 || (mode == NNTILE_HIP_MASK_CAUSAL && p.k_seq >= 64 * kKeys));
     if(!three && tiles * ((p.q_tile + kQRows - 1) / kQRows) > kCUs)
@@ -2303,8 +2317,6 @@ static bool halved_is_faster(const PrefillParams &p, int head, int mode)
     }
     const int64_t steps = key_steps(p);
     const bool rule = mode == NNTILE_HIP_MASK_CAUSAL || mode == NNTILE_HIP_MASK_NONE;
-    // Rectangular calls of few steps are left to the other forms, so that what one
-    // computes does not depend on how many entries share its launch.
     if(rule && p.q_seq != p.k_seq && steps < kHalvedSteps)
     {
         return false;

@@ -1566,6 +1566,12 @@ static int launch_head(hipStream_t stream, PrefillParams &p, int mode, int form)
         : launch_form<HEAD, 4, 1>(stream, p, mode);
 }
 
+// Forms that take masks given as values: the small ones, and head 64's two by four
+static bool with_values(int form)
+{
+    return form <= kF16x2Form41 || form == kF16x2Form24;
+}
+
 // The form that is expected to be done first; kF16x2None: the fp32 kernel's
 // 32-query workgroups.
 //
@@ -1574,8 +1580,8 @@ static int launch_head(hipStream_t stream, PrefillParams &p, int mode, int form)
 // itself, and the passes that a CU gets, at the time a pass adds to a full one; a
 // second and third round of workgroups start anew.  The times are fitted to
 // launches of 1 to 200 heads of 64 to 8192 rows, causal and not, 4 to 8 % off in
-// the mean; what the rule picks is within 1 to 2.5 % of the fastest of the five in
-// the mean.  us, the fp32 kernel's 32 queries / 22 / 41 / 42 / 81 - head 64, causal:
+// the mean; what the rule picks is within 1 to 2.5 % of the fastest of the first five
+// in the mean.  us, the fp32 kernel's 32 queries / 22 / 41 / 42 / 81 - head 64, causal:
 // 12 x 128 7.9 / 9.4 / 11.5 / 11.7 / 13.1; 12 x 1024 30 / 25 / 35 / 29 / 49; 48 x 1024
 // 75 / 40.3 / 40.1 / 38.3 / 51; 200 x 1024 293 / 144 / 117 / 145 / 138; 12 x 4096 251 /
 // 112 / 129 / 103 / 161; 32 x 4096 619 / 275 / 238 / 240 / 226.  Head 128, 48 x 1024: 177 /
@@ -1598,12 +1604,9 @@ static int launch_head(hipStream_t stream, PrefillParams &p, int mode, int form)
 // 128: 2 x 800 51 51 18 / 49 47 26 / 58 57 31; 32 x 1024 232 151 75 / 113 78 56 / 80 77 40.
 // (257 to 512 workgroups of the fp32 kernel at head 64: a window is slower with 22,
 // the others gain more.)
-// (the small forms, and head 64's two by four)
-static bool with_values(int form)
-{
-    return form <= kF16x2Form41 || form == kF16x2Form24;
-}
-
+// 22 / 24, in the same order: 12 x 1024 37.8 36.7 22.4 / 33.7 32.3 23.4; 6 x 2000 70.2 64.5 32.3 /
+// 60.8 58.6 34.4; 16 x 1000 41.8 39.5 25.0 / 37.6 36.2 25.4: a window loses a twentieth, the
+// others gain a tenth.
 int prefill_f16x2_form(const PrefillParams &p, int head, int mode)
 {
     struct Cost
