@@ -169,9 +169,10 @@ def test_decode_partials_have_arrived_before_their_flag_goes_up(assemblies):
 def test_nothing_is_read_past_the_caches(assemblies):
     """A read through a volatile pointer bypasses the caches' scope and is waited for at
     once, whatever else could be in flight beside it: the forward of halved steps
-    once touched its key lines so, four memory round trips one after the other."""
+    once touched its key lines so, four memory round trips one after the other.  (The
+    classification of masks looks at flags so, that other launches raise.)"""
     for name, text in assemblies.items():
-        for line in _instructions(text):
+        for line in _instructions(text) if name != "mask_classify.hip" else ():
             assert not re.match(r"(flat|global)_load_(dword|ushort|ubyte)\S* .*\bsc0 sc1$", line), (name, line)
 
 
